@@ -54,5 +54,7 @@ struct MatMulDirectArgs {
 
 int launch_conv_direct(const ConvDirectArgs& a, bool rne, hipStream_t s);
 int launch_matmul_direct(const MatMulDirectArgs& a, bool rne, hipStream_t s);
+// The same product on the matrix cores (gemm_i8.hip); EUNSUPPORTED, with nothing launched, for layouts it does not take.
+int launch_matmul_i8(const MatMulDirectArgs& a, bool rne, hipStream_t s);
 
 }  // namespace chx

@@ -1421,90 +1421,6 @@ extern "C" int chx_hip_conv_integer(
     return launch_conv_direct(a, false, s);
 }
 
-namespace chx {
-namespace {
-
-// A 2-D matrix product as a 1x1 convolution over M "pixels": a [M,K] is a channels-last
-// activation row per pixel, b [K,N] the weights of N output channels.
-int matmul_via_mfma(
-        const chx_hip_tensor& a, const chx_hip_tensor& b, chx_hip_tensor& y, const MatMulShape& ms, int32_t a_zp,
-        bool out_int32, bool rne, float b_scale, const int32_t* bias, const RequantParams& rq, hipStream_t s) {
-    const int nd = a.ndim;
-    if (ms.batch != 1 || b.dtype != CHX_HIP_INT8 || ms.M > INT32_MAX || ms.K > (1 << 20) || ms.N >= (1 << 24))
-        return CHX_HIP_EUNSUPPORTED;
-    if (stream_is_capturing(s)) return CHX_HIP_EUNSUPPORTED;  // b is packed into scratch memory per call: not inside a recorded run
-    chx_hip_tensor x4, w4, y4;
-    memset(&x4, 0, sizeof(x4));
-    memset(&w4, 0, sizeof(w4));
-    memset(&y4, 0, sizeof(y4));
-    x4.data = a.data; x4.dtype = a.dtype; x4.ndim = 4;
-    x4.shape[0] = 1; x4.shape[1] = ms.K; x4.shape[2] = 1; x4.shape[3] = ms.M;
-    x4.strides[0] = 0; x4.strides[1] = a.strides[nd - 1]; x4.strides[2] = 0; x4.strides[3] = a.strides[nd - 2];
-    w4.data = b.data; w4.dtype = b.dtype; w4.ndim = 4;
-    w4.shape[0] = ms.N; w4.shape[1] = ms.K; w4.shape[2] = 1; w4.shape[3] = 1;
-    w4.strides[0] = b.strides[nd - 1]; w4.strides[1] = b.strides[nd - 2]; w4.strides[2] = 0; w4.strides[3] = 0;
-    y4.data = y.data; y4.dtype = y.dtype; y4.ndim = 4;
-    y4.shape[0] = 1; y4.shape[1] = ms.N; y4.shape[2] = 1; y4.shape[3] = ms.M;
-    y4.strides[0] = 0; y4.strides[1] = y.strides[nd - 1]; y4.strides[2] = 0; y4.strides[3] = y.strides[nd - 2];
-    if (!weights_fit_mfma(w4, 1) || !x_is_mfma_ready(x4)) return CHX_HIP_EUNSUPPORTED;
-    int64_t px;
-    if (!y_is_pixel_major(y4, &px)) return CHX_HIP_EUNSUPPORTED;
-    chx_hip_conv_params p = {1, 1, 0, 0, 0, 0, 1};
-    ConvCall c;
-    memset(&c, 0, sizeof(c));
-    c.opt = read_launch_options();
-    c.x = &x4;
-    c.y = &y4;
-    c.p = &p;
-    c.cs.N = 1; c.cs.C = (int32_t)ms.K; c.cs.H = 1; c.cs.W = (int32_t)ms.M;
-    c.cs.OC = (int32_t)ms.N; c.cs.Cg = (int32_t)ms.K; c.cs.KH = 1; c.cs.KW = 1; c.cs.OH = 1; c.cs.OW = (int32_t)ms.M;
-    c.x_zp = a_zp;
-    c.out_int32 = out_int32;
-    c.rne = rne;
-    static const float kOne = 0.f;
-    (void)kOne;
-    c.w_scale = nullptr;
-    c.w_scale_len = 1;
-    c.bias = bias;
-    c.rq = rq;
-    PackedWeights pw;
-    CHX_PROPAGATE(make_packed(w4, false, s, &pw));
-    // the per-tensor b_scale is a host value; the kernel reads scales from device memory
-    void* scale_dev = nullptr;
-    int rc = CHX_HIP_OK;
-    if (!out_int32) {
-        rc = scratch_alloc(&scale_dev, sizeof(float), s);
-        if (rc == CHX_HIP_OK && hipMemcpyAsync(scale_dev, &b_scale, sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) {
-            set_error("hipMemcpyAsync of the weight scale failed");
-            rc = CHX_HIP_ERUNTIME;
-        }
-        c.w_scale = static_cast<const float*>(scale_dev);
-    }
-    if (rc == CHX_HIP_OK) rc = run_conv_mfma(c, pw, s);
-    scratch_free(scale_dev, s);
-    release_packed(&pw, false, s);
-    return rc;
-}
-
-// Scalar zero point held in a device array of one element (or absent): host value, via a
-// synchronizing read.  Returns false when the array is a per-axis vector.
-int scalar_zero_point(const chx_hip_tensor* zp, hipStream_t s, bool* is_scalar, int32_t* value) {
-    *is_scalar = true;
-    *value = 0;
-    if (!zp) return CHX_HIP_OK;
-    if (numel(*zp) != 1) {
-        *is_scalar = false;
-        return CHX_HIP_OK;
-    }
-    std::vector<uint8_t> v;
-    CHX_PROPAGATE(read_back(*zp, &v, s));
-    *value = zp->dtype == CHX_HIP_INT8 ? (int32_t)(int8_t)v[0] : (int32_t)v[0];
-    return CHX_HIP_OK;
-}
-
-}  // namespace
-}  // namespace chx
-
 extern "C" int chx_hip_matmul_integer(
         const chx_hip_tensor* a, const chx_hip_tensor* b, const chx_hip_tensor* a_zero_point,
         const chx_hip_tensor* b_zero_point, chx_hip_tensor* y, void* stream) {
@@ -1538,18 +1454,8 @@ extern "C" int chx_hip_matmul_integer(
         m.b_zp_signed = b_zero_point->dtype == CHX_HIP_INT8;
     }
     hipStream_t s = as_stream(stream);
-    if (ms.batch == 1 && b->dtype == CHX_HIP_INT8 && ms.M * ms.N * ms.K >= (int64_t(1) << 22) && !stream_is_capturing(s)) {
-        bool a_scalar, b_scalar;
-        int32_t az, bz;
-        CHX_PROPAGATE(scalar_zero_point(a_zero_point, s, &a_scalar, &az));
-        CHX_PROPAGATE(scalar_zero_point(b_zero_point, s, &b_scalar, &bz));
-        if (a_scalar && b_scalar && bz == 0) {
-            RequantParams rq;
-            memset(&rq, 0, sizeof(rq));
-            const int rc = matmul_via_mfma(*a, *b, *y, ms, az, true, false, 0.f, nullptr, rq, s);
-            if (rc != CHX_HIP_EUNSUPPORTED) return rc;
-        }
-    }
+    const int rc = launch_matmul_i8(m, false, s);
+    if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     return launch_matmul_direct(m, false, s);
 }
 
@@ -1574,10 +1480,8 @@ extern "C" int chx_hip_qlinear_matmul(
                                "QLinearMatMul", &m.rq, &m.bias));
     hipStream_t s = as_stream(stream);
     const bool rne = (flags & CHX_HIP_ROUND_ONNX_RNE) != 0;
-    if (b_zero_point == 0) {
-        const int rc = matmul_via_mfma(*a, *b, *y, ms, a_zero_point, false, rne, b_scale, m.bias, m.rq, s);
-        if (rc != CHX_HIP_EUNSUPPORTED) return rc;
-    }
+    const int rc = launch_matmul_i8(m, rne, s);
+    if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     return launch_matmul_direct(m, rne, s);
 }
 
