@@ -24,7 +24,7 @@ IDL_PATH = os.path.join(_HERE, "runtime", "chxvm_ops.idl")
 RUNTIME_EXPORTS = [
     "chxvm_last_error", "chxvm_num_ops", "chxvm_op_name", "chxvm_op_number", "chxvm_proto_roundtrip", "chxvm_free",
     "chxvm_program_create", "chxvm_program_destroy", "chxvm_program_num_instructions", "chxvm_program_num_inputs",
-    "chxvm_program_input_name", "chxvm_program_run", "chxvm_outputs_count", "chxvm_outputs_name", "chxvm_outputs_get",
+    "chxvm_program_input_name", "chxvm_program_run", "chxvm_program_run_to_host", "chxvm_outputs_host", "chxvm_outputs_count", "chxvm_outputs_name", "chxvm_outputs_get",
     "chxvm_outputs_destroy", "chxvm_backend_config_has", "chxvm_backend_config_name", "chxvm_set_option", "chxvm_counter",
     "chxvm_program_set_option", "chxvm_program_counter", "chxvm_program_capture", "chxvm_replay_launch", "chxvm_replay_synchronize",
     "chxvm_replay_outputs", "chxvm_replay_info", "chxvm_replay_destroy",
@@ -72,6 +72,9 @@ def runtime():
         rt.chxvm_program_input_name.restype = ctypes.c_char_p
         rt.chxvm_program_run.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(capi.Tensor),
                                          ctypes.c_int32, ctypes.c_int32, ctypes.POINTER(ctypes.c_void_p)]
+        rt.chxvm_program_run_to_host.argtypes = rt.chxvm_program_run.argtypes
+        rt.chxvm_outputs_host.argtypes = [ctypes.c_void_p, ctypes.c_int32]
+        rt.chxvm_outputs_host.restype = ctypes.c_void_p
         rt.chxvm_outputs_count.argtypes = [ctypes.c_void_p]
         rt.chxvm_outputs_name.argtypes = [ctypes.c_void_p, ctypes.c_int32]
         rt.chxvm_outputs_name.restype = ctypes.c_char_p
@@ -331,11 +334,16 @@ _NP_OF_CODE = {1: np.bool_, 2: np.int8, 3: np.int16, 4: np.int32, 5: np.int64, 6
                9: np.float64}
 
 
-def _to_numpy(desc):
-    """Host copy of the device array a descriptor names, with its shape and element order."""
+def _to_numpy(desc, host=None):
+    """Host copy of the device array a descriptor names, with its shape and element order.  host: where the runtime has
+    the dense elements in host memory already."""
     dt = np.dtype(_NP_OF_CODE[desc.dtype])
     nd = desc.ndim
-    shape = [desc.shape[i] for i in range(nd)]
+    shape = desc.shape[:nd]
+    if host:
+        a = np.empty(shape, dt)
+        ctypes.memmove(a.ctypes.data, host, a.nbytes)
+        return a
     strides = [desc.strides[i] for i in range(nd)]
     span = dt.itemsize + sum((s - 1) * st for s, st in zip(shape, strides)) if all(shape) else 0
     buf = np.empty(max(span, 1), dtype=np.uint8)
@@ -371,13 +379,13 @@ class Program:
         c_names = (ctypes.c_char_p * len(names))(*[n.encode() for n in names])
         descs = (capi.Tensor * len(names))(*[capi.desc(inputs[n]) for n in names])
         out = ctypes.c_void_p()
-        _check(rt.chxvm_program_run(self._h, c_names, descs, len(names), trace_level, ctypes.byref(out)))
+        _check(rt.chxvm_program_run_to_host(self._h, c_names, descs, len(names), trace_level, ctypes.byref(out)))
         try:
             result = {}
             for i in range(rt.chxvm_outputs_count(out)):
                 d = capi.Tensor()
                 _check(rt.chxvm_outputs_get(out, i, ctypes.byref(d)))
-                result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d)
+                result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d, rt.chxvm_outputs_host(out, i))
             return result
         finally:
             rt.chxvm_outputs_destroy(out)
@@ -438,7 +446,7 @@ class Replay:
         for i in range(rt.chxvm_outputs_count(out)):
             d = capi.Tensor()
             _check(rt.chxvm_outputs_get(out, i, ctypes.byref(d)))
-            result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d)
+            result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d, rt.chxvm_outputs_host(out, i))
         return result
 
     def info(self, name):

@@ -144,6 +144,8 @@ int launch_check(const char* kernel);
 // Stream-ordered scratch memory for one call.
 // device address of the scratch array of chx_hip_reduce_min_max_noalloc on the current device, looked up once (reduce_cast.hip)
 int prepare_noalloc_scratch();
+// copyout.hip: a copy of at most 512 KB to pageable memory, waited for; false when it is not one for that path
+bool small_copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s, int* rc);
 // whether work submitted to s is being recorded into a graph instead of executed
 bool stream_is_capturing(hipStream_t s);
 int scratch_alloc(void** p, size_t bytes, hipStream_t s);

@@ -174,6 +174,8 @@ int chx_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream) {
 int chx_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
     if (bytes == 0) return CHX_HIP_OK;
     CHX_REQUIRE(dst && src, "null pointer");
+    int rc = CHX_HIP_OK;
+    if (small_copy_to_host(dst, src, bytes, as_stream(stream), &rc)) return rc;
     CHX_HIP_CALL(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, as_stream(stream)));
     CHX_HIP_CALL(hipStreamSynchronize(as_stream(stream)));
     return CHX_HIP_OK;
@@ -188,6 +190,11 @@ int chx_hip_memset(void* dst, int value, size_t bytes, void* stream) {
 
 int chx_hip_stream_synchronize(void* stream) {
     CHX_HIP_CALL(hipStreamSynchronize(as_stream(stream)));
+    return CHX_HIP_OK;
+}
+
+int chx_hip_device_synchronize(void) {
+    CHX_HIP_CALL(hipDeviceSynchronize());
     return CHX_HIP_OK;
 }
 

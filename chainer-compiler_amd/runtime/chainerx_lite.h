@@ -340,8 +340,8 @@ inline Strides ContiguousStrides(const Shape& shape, int64_t item_size) {
     return s;
 }
 
-// Where the arrays of the calling thread come from and which stream its kernels go to.  The default is the
-// device runtime's allocator and the null stream, the counterpart of ChainerX's default device.  A run that is
+// Where the arrays of the calling thread come from and which stream its kernels go to.  The default is a cache
+// over the device runtime's allocator and the null stream, the counterpart of ChainerX's default device.  A run that is
 // to be captured into a graph installs a pool of its own (no allocation by the device runtime may happen while
 // a stream records) and the stream that records.
 class DeviceAllocator {
@@ -350,6 +350,8 @@ public:
     // memory of at least `bytes` bytes that stays valid until the returned handle is released
     virtual std::shared_ptr<void> Allocate(size_t bytes) = 0;
 };
+
+DeviceAllocator& DefaultDeviceAllocator();  // device_cache.cc
 
 struct DeviceContext {
     void* stream = nullptr;
@@ -386,14 +388,8 @@ private:
 inline Array Empty(const Shape& shape, Dtype dtype) {
     const int64_t bytes = shape.GetTotalSize() * GetItemSize(dtype);
     const size_t want = static_cast<size_t>(bytes > 0 ? bytes : 1);
-    std::shared_ptr<void> data;
-    if (DeviceAllocator* allocator = CurrentDeviceContext().allocator) {
-        data = allocator->Allocate(want);
-    } else {
-        void* p = nullptr;
-        CHXVM_HIP_CALL(chx_hip_malloc(&p, want));
-        data = std::shared_ptr<void>(p, [](void* q) { (void)chx_hip_free(q); });
-    }
+    DeviceAllocator* allocator = CurrentDeviceContext().allocator;
+    std::shared_ptr<void> data = (allocator ? *allocator : DefaultDeviceAllocator()).Allocate(want);
     return Array::MakeOwned(std::move(data), dtype, shape, ContiguousStrides(shape, GetItemSize(dtype)));
 }
 

@@ -7,6 +7,7 @@
 #include "chrome_tracing.h"
 #include "chxvm.h"
 #include "configs/backend_config.h"
+#include "device_cache.h"
 #include "replay.h"
 
 using chainer_compiler::BackendConfig;
@@ -43,15 +44,87 @@ void SetLastError(const std::string& message) {
 }  // namespace runtime
 }  // namespace chainer_compiler
 
+namespace {
+
+// Host copies of a run's results, when they are few bytes (chx_hip_copyout): queued behind the run, so that waiting for
+// the run and fetching its results is one wait.
+class HostResults {
+public:
+    HostResults() = default;
+    HostResults(const HostResults&) = delete;
+    HostResults& operator=(const HostResults&) = delete;
+    ~HostResults() {
+        chx_hip_copyout_destroy(copy_);
+    }
+    // false: these results are not for this path
+    bool Enqueue(const std::vector<chainerx::Array>& arrays, void* stream) {
+        stream_ = stream;
+        valid_ = false;
+        const void* src[8];
+        size_t bytes[8], total = 0;
+        if (arrays.empty() || arrays.size() > 8) return false;
+        for (size_t i = 0; i < arrays.size(); ++i) {
+            if (!arrays[i].IsContiguous()) return false;
+            src[i] = static_cast<char*>(arrays[i].raw_data()) + arrays[i].offset();
+            bytes[i] = static_cast<size_t>(arrays[i].GetNBytes());
+            total += bytes[i];
+        }
+        if (total > 512 * 1024) return false;
+        if (!copy_ || total > capacity_) {
+            chx_hip_copyout_destroy(copy_);
+            copy_ = nullptr;
+            if (chx_hip_copyout_create(total, &copy_) != 0) return false;
+            capacity_ = total;
+        }
+        CHXVM_HIP_CALL(chx_hip_copyout_enqueue(copy_, src, bytes, static_cast<int32_t>(arrays.size()), stream));
+        valid_ = true;
+        return true;
+    }
+    // whether the last launch's results are (or will be) in host memory, and the stream they were queued on
+    bool valid() const {
+        return valid_;
+    }
+    void* stream() const {
+        return stream_;
+    }
+    void Wait() {
+        CHXVM_HIP_CALL(chx_hip_copyout_wait(copy_));
+    }
+    const void* data(int32_t i) const {
+        return chx_hip_copyout_data(copy_, i);
+    }
+
+private:
+    chx_hip_copyout* copy_ = nullptr;
+    size_t capacity_ = 0;
+    void* stream_ = nullptr;
+    bool valid_ = false;
+};
+
+}  // namespace
+
 struct chxvm_program {
     std::unique_ptr<ChxVM> vm;
     int onnx_int32_bias = -1;  // -1: the process default at the time of a run
+    HostResults results;       // of chxvm_program_run_to_host
+
+    chxvm_program() {
+        DeviceCache::Get().AddProgram();
+    }
+    ~chxvm_program() {
+        // constants may be read by work of any stream still (a replay's)
+        (void)chx_hip_device_synchronize();
+        vm.reset();
+        DeviceCache::Get().RemoveProgram();
+    }
 };
 
 struct chxvm_outputs {
     std::vector<std::string> names;
     std::vector<chainerx::Array> arrays;
     InOuts keep_inputs;
+    std::vector<std::vector<char>> host;  // an eager run's host copies, where it made them
+    chxvm_replay* replay = nullptr;       // whose outputs these are
 };
 
 struct chxvm_replay {
@@ -59,6 +132,9 @@ struct chxvm_replay {
     void* stream = nullptr;
     chx_hip_graph* graph = nullptr;
     chxvm_outputs outputs;
+    // set once the host has asked for a launch's results: every launch then sends them along
+    bool host_reads = false;
+    HostResults results;
     int32_t warm_runs = 0;
     std::vector<chx_hip_qconv_plan*> pinned_plans;  // whose memory the graph's kernels address
 
@@ -148,13 +224,13 @@ const char* chxvm_program_input_name(const chxvm_program* program, int32_t i) {
     return program->vm->input_names()[static_cast<size_t>(i)].c_str();
 }
 
-int32_t chxvm_program_run(
-        chxvm_program* program,
-        const char* const* input_names,
-        const chx_hip_tensor* inputs,
-        int32_t num_inputs,
-        int32_t trace_level,
-        chxvm_outputs** out) {
+}  // extern "C"
+
+namespace {
+
+int32_t RunProgram(
+        chxvm_program* program, const char* const* input_names, const chx_hip_tensor* inputs, int32_t num_inputs, int32_t trace_level,
+        bool to_host, chxvm_outputs** out) {
     return Guard([&] {
         InOuts in = BorrowInputs(input_names, inputs, num_inputs);
         ChxVMOptions options;
@@ -178,9 +254,35 @@ int32_t chxvm_program_run(
             o->arrays.push_back(p.second->GetArray());
         }
         o->keep_inputs = in;
-        CHXVM_HIP_CALL(chx_hip_stream_synchronize(nullptr));  // device sync at the end of a run (tools/run_onnx.cc:462)
+        // the run ends with the device done (tools/run_onnx.cc:462)
+        HostResults* host = to_host ? &program->results : nullptr;
+        if (host && host->Enqueue(o->arrays, nullptr)) {
+            host->Wait();
+            for (size_t i = 0; i < o->arrays.size(); ++i) {
+                const char* p = static_cast<const char*>(host->data(static_cast<int32_t>(i)));
+                o->host.emplace_back(p, p + o->arrays[i].GetNBytes());
+            }
+        } else {
+            CHXVM_HIP_CALL(chx_hip_stream_synchronize(nullptr));
+        }
         *out = o.release();
     });
+}
+
+}  // namespace
+
+extern "C" {
+
+int32_t chxvm_program_run(
+        chxvm_program* program, const char* const* input_names, const chx_hip_tensor* inputs, int32_t num_inputs, int32_t trace_level,
+        chxvm_outputs** out) {
+    return RunProgram(program, input_names, inputs, num_inputs, trace_level, false, out);
+}
+
+int32_t chxvm_program_run_to_host(
+        chxvm_program* program, const char* const* input_names, const chx_hip_tensor* inputs, int32_t num_inputs, int32_t trace_level,
+        chxvm_outputs** out) {
+    return RunProgram(program, input_names, inputs, num_inputs, trace_level, true, out);
 }
 
 int32_t chxvm_program_capture(
@@ -228,6 +330,7 @@ int32_t chxvm_program_capture(
             r->outputs.arrays.push_back(p.second->GetArray());
         }
         r->outputs.keep_inputs = in;
+        r->outputs.replay = r.get();
         *out = r.release();
     });
 }
@@ -235,14 +338,18 @@ int32_t chxvm_program_capture(
 int32_t chxvm_replay_launch(chxvm_replay* replay, void* stream) {
     return Guard([&] {
         CHECK(replay != nullptr && replay->graph != nullptr) << "null replay";
-        CHXVM_HIP_CALL(chx_hip_graph_launch(replay->graph, stream ? stream : replay->stream));
+        void* on = stream ? stream : replay->stream;
+        CHXVM_HIP_CALL(chx_hip_graph_launch(replay->graph, on));
+        if (replay->host_reads) (void)replay->results.Enqueue(replay->outputs.arrays, on);
     });
 }
 
 int32_t chxvm_replay_synchronize(chxvm_replay* replay) {
     return Guard([&] {
         CHECK(replay != nullptr) << "null replay";
-        CHXVM_HIP_CALL(chx_hip_stream_synchronize(replay->stream));
+        // (the results are the last thing on the stream)
+        if (replay->results.valid() && replay->results.stream() == replay->stream) replay->results.Wait();
+        else CHXVM_HIP_CALL(chx_hip_stream_synchronize(replay->stream));
     });
 }
 
@@ -278,7 +385,26 @@ int32_t chxvm_outputs_get(const chxvm_outputs* outputs, int32_t i, chx_hip_tenso
     });
 }
 
+const void* chxvm_outputs_host(const chxvm_outputs* outputs, int32_t i) {
+    const void* p = nullptr;
+    (void)Guard([&] {
+        CHECK_LT(static_cast<size_t>(i), outputs->arrays.size());
+        if (chxvm_replay* replay = outputs->replay) {
+            replay->host_reads = true;
+            if (replay->results.valid()) {
+                replay->results.Wait();
+                p = replay->results.data(i);
+            }
+        } else if (static_cast<size_t>(i) < outputs->host.size()) {
+            p = outputs->host[static_cast<size_t>(i)].data();
+        }
+    });
+    return p;
+}
+
 void chxvm_outputs_destroy(chxvm_outputs* outputs) {
+    // the arrays' memory is handed out again: nothing may read it any more
+    if (outputs && !outputs->arrays.empty()) (void)chx_hip_device_synchronize();
     delete outputs;
 }
 

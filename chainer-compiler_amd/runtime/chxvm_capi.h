@@ -45,10 +45,21 @@ int32_t chxvm_program_run(
         int32_t num_inputs,
         int32_t trace_level,
         chxvm_outputs** out);
+/* The same, for a caller that reads the results on the host: those of few bytes travel with the end of the run. */
+int32_t chxvm_program_run_to_host(
+        chxvm_program* program,
+        const char* const* input_names,
+        const chx_hip_tensor* inputs,
+        int32_t num_inputs,
+        int32_t trace_level,
+        chxvm_outputs** out);
 int32_t chxvm_outputs_count(const chxvm_outputs* outputs);
 const char* chxvm_outputs_name(const chxvm_outputs* outputs, int32_t i);
 /* Descriptor of output i (device memory owned by `outputs`). */
 int32_t chxvm_outputs_get(const chxvm_outputs* outputs, int32_t i, chx_hip_tensor* out);
+/* Output i in host memory, dense, valid as long as `outputs` (a replay's: until its next launch), or null: copy it from
+ * the device then.  Of a replay this is the last launch's result; the first call makes later launches send theirs. */
+const void* chxvm_outputs_host(const chxvm_outputs* outputs, int32_t i);
 void chxvm_outputs_destroy(chxvm_outputs* outputs);
 
 /* One run of the program recorded into a device graph.  A program of the quantized-inference path does the

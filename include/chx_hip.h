@@ -133,8 +133,19 @@ int chx_hip_malloc(void** ptr, size_t bytes);
 int chx_hip_free(void* ptr);
 int chx_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream); /* synchronizes the stream */
 int chx_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream); /* synchronizes the stream */
+
+/* Small device results for the host: enqueue() queues the copy of up to 8 ranges (512 KB together) behind the work of
+ * `stream`, wait() returns when they are in host memory, data() is where range i of the last enqueue lies until the next
+ * one.  One object serves one copy at a time. */
+typedef struct chx_hip_copyout chx_hip_copyout;
+int chx_hip_copyout_create(size_t bytes, chx_hip_copyout** out);
+int chx_hip_copyout_enqueue(chx_hip_copyout* copyout, const void* const* src, const size_t* bytes, int32_t n, void* stream);
+int chx_hip_copyout_wait(chx_hip_copyout* copyout);
+const void* chx_hip_copyout_data(const chx_hip_copyout* copyout, int32_t i);
+void chx_hip_copyout_destroy(chx_hip_copyout* copyout);
 int chx_hip_memset(void* dst, int value, size_t bytes, void* stream);
 int chx_hip_stream_synchronize(void* stream);
+int chx_hip_device_synchronize(void);
 
 /* Streams and captured graphs, for hosts that replay a fixed instruction sequence (the ChxVM runtime
  * mirror captures one run of a program and replays it; nothing in the reference corresponds: its
