@@ -28,8 +28,7 @@
 // Float literals are decimal or 0x######## (the bit pattern of the float32).
 // The arithmetic type of a program is that of its floating-point ports (one type per program, as the reference's
 // `typedef ... T`, compiler/nvrtc_builder.cc:118-127): float32; float16, where every node computes in float32 and
-// rounds to float16 (what a half-precision operation is); or float64.  The 8-bit ops go with float32 only, and only
-// float32 programs have the vector kernel; the other two types run on the general kernel.
+// rounds to float16 (what a half-precision operation is); or float64.  The 8-bit ops go with float32 only.
 //
 // The CUDA C text that the reference's compiler emits for a group (BuildNvrtcProgram, nvrtc_builder.cc:91-206) is
 // accepted as well and turned into the same internal program: `typedef half|float|double T;`, the kernel's
@@ -45,9 +44,11 @@
 #include <mutex>
 #include <sstream>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "chx_internal.h"
+#include "conv_mfma.h"
 
 namespace chx {
 namespace {
@@ -606,14 +607,152 @@ const char* ctype_of(int32_t dt) {
            : dt == CHX_HIP_INT8 ? "signed char" : "unsigned char";
 }
 
+// What the general kernel is specialised for, beside the program: how each operand is addressed and the number of axes.
+//   F  dense in the order of the result: the flat index      S  one element
+//   C  innermost stride 1      Z  innermost stride 0      X  any strides
+struct GeneralForm {
+    std::string modes;
+    int ndim = 0;         // collapsed axes
+    int vec = 1;          // elements per thread: 16 bytes of the widest operand
+    bool wide = false;    // 2^31 elements or more: 64-bit indices
+    bool short_rows = false;  // the innermost axis is shorter than `vec`
+};
+
+// The general kernel: any strides, types and alignments.  A thread computes `vec` neighbouring elements of the result.
+// Where they lie in one row of the innermost axis (nearly always) each operand is one access of 16 bytes at whatever
+// alignment (F, C), one element (S, Z), or `vec` strided ones (X); a run that crosses the end of a row is read
+// element by element from two positions.  Divisions by the extents are multiplications with their reciprocals.
+// float16 chain over [8, 333, 1001] with two [1001] operands: 15.2 us with one element per thread and 64-bit divisions,
+// 7.0 this way.
+void emit_general(const Program& prog, const std::string& name, const GeneralForm& g, const std::string& VT, std::ostringstream& os) {
+    const size_t nin = prog.inputs.size(), nout = prog.outputs.size();
+    const int V = g.vec, ND = g.ndim > 0 ? g.ndim : 1;
+    const std::string last = std::to_string(ND - 1);
+    bool placed = false;  // an operand that needs the position of the run
+    for (char m : g.modes) placed = placed || m == 'C' || m == 'Z' || m == 'X';
+    const char* idx = g.wide ? "unsigned long long" : "unsigned int";
+    auto value_type = [&](const Port& p) { return is_float_dtype(p.dtype) ? VT : std::string("int"); };
+    auto vec_type = [&](int32_t dt) {
+        return std::string("V") + (dt == CHX_HIP_FLOAT32 ? "f" : dt == CHX_HIP_FLOAT16 ? "h" : dt == CHX_HIP_FLOAT64 ? "d" : "b");
+    };
+    os << "typedef " << idx << " gidx;\n";
+    os << "struct GenDesc { unsigned int mul[" << CHX_HIP_MAX_NDIM << "], shift[" << CHX_HIP_MAX_NDIM << "]; long long shape[" << CHX_HIP_MAX_NDIM
+       << "]; long long istr[" << nin << "][" << CHX_HIP_MAX_NDIM << "]; };\n";
+    os << "typedef float Vf __attribute__((ext_vector_type(" << V << "), aligned(4)));\n";
+    os << "typedef _Float16 Vh __attribute__((ext_vector_type(" << V << "), aligned(2)));\n";
+    os << "typedef double Vd __attribute__((ext_vector_type(" << V << "), aligned(8)));\n";
+    os << "typedef unsigned int Vb __attribute__((ext_vector_type(" << (V < 4 ? 1 : V / 4) << "), aligned(1)));\n";
+    os << "__device__ __forceinline__ gidx gdiv(gidx r, const GenDesc& d, int a) {\n";
+    if (g.wide) os << "  return r / (gidx)d.shape[a];\n}\n";
+    else os << "  return (__umulhi(r, d.mul[a]) + r) >> d.shift[a];\n}\n";
+    // element offsets of every placed operand at flat position r
+    os << "__device__ __forceinline__ void place(gidx r, const GenDesc& d, long long (&off)[" << nin << "], gidx& inner) {\n";
+    os << "  for (int i = 0; i < " << nin << "; ++i) off[i] = 0;\n  inner = 0;\n";
+    os << "#pragma unroll\n  for (int a = " << last << "; a >= 0; --a) {\n";
+    os << "    const gidx q = a ? gdiv(r, d, a) : 0, m = r - q * (gidx)d.shape[a];\n    r = q;\n    if (a == " << last << ") inner = m;\n";
+    for (size_t i = 0; i < nin; ++i)
+        if (g.modes[i] == 'C' || g.modes[i] == 'Z' || g.modes[i] == 'X') os << "    off[" << i << "] += (long long)m * d.istr[" << i << "][a];\n";
+    os << "  }\n}\n";
+
+    os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_gen(unsigned long long total";
+    for (size_t i = 0; i < nin; ++i) os << ", const " << ctype_of(prog.inputs[i].dtype) << "* __restrict__ i" << i;
+    for (size_t i = 0; i < nout; ++i) os << ", " << ctype_of(prog.outputs[i].dtype) << "* __restrict__ o" << i;
+    os << ", GenDesc d) {\n";
+    os << "  const gidx n = (gidx)total, base = ((gidx)blockIdx.x * 256u + threadIdx.x) * " << V << "u;\n";
+    os << "  if (base >= n) return;\n";
+    os << "  const int cnt = n - base < " << V << "u ? (int)(n - base) : " << V << ";\n";
+    os << "  long long off[" << nin << "]; gidx inner = 0;\n";
+    if (placed) {
+        os << "  place(base, d, off, inner);\n";
+        os << "  const gidx left = (gidx)d.shape[" << last << "] - inner;\n";
+        os << "  const bool straight = cnt == " << V << " && left >= " << V << "u;\n";
+    } else {
+        os << "  const bool straight = cnt == " << V << ";\n";
+    }
+    for (size_t i = 0; i < nin; ++i) os << "  " << value_type(prog.inputs[i]) << " x" << i << "[" << V << "];\n";
+    // a vector of 8-bit codes arrives as words
+    auto unpack = [&](size_t i, const std::string& from) {
+        const int32_t dt = prog.inputs[i].dtype;
+        if (is_float_dtype(dt)) {
+            os << "    for (int e = 0; e < " << V << "; ++e) x" << i << "[e] = (" << VT << ")" << from << "[e];\n";
+        } else {
+            for (int e = 0; e < V; ++e)
+                os << "    x" << i << "[" << e << "] = (int)" << (dt == CHX_HIP_INT8 ? "(signed char)" : "") << "((" << from << "[" << e / 4 << "] >> " << 8 * (e % 4)
+                   << ") & 0xffu);\n";
+        }
+    };
+    os << "  if (straight) {\n";
+    for (size_t i = 0; i < nin; ++i) {
+        const char m = g.modes[i];
+        if ((m == 'F' || m == 'C') && (is_float_dtype(prog.inputs[i].dtype) || V >= 4)) {
+            os << "    { const " << vec_type(prog.inputs[i].dtype) << " t = " << (m == 'F' ? "__builtin_nontemporal_load(" : "*(") << "(const "
+               << vec_type(prog.inputs[i].dtype) << "*)(i" << i << " + " << (m == 'F' ? "base" : "off[" + std::to_string(i) + "]") << "));\n";
+            unpack(i, "t");
+            os << "    }\n";
+        } else {
+            const std::string at = m == 'S' ? "0" : m == 'F' ? "base + e" : m == 'Z' ? "off[" + std::to_string(i) + "]"
+                                   : "off[" + std::to_string(i) + "] + e * d.istr[" + std::to_string(i) + "][" + last + "]";
+            os << "    for (int e = 0; e < " << V << "; ++e) x" << i << "[e] = (" << value_type(prog.inputs[i]) << ")i" << i << "[" << at << "];\n";
+        }
+    }
+    os << "  } else {\n";
+    if (placed && !g.short_rows) {
+        os << "    long long next[" << nin << "]; gidx zero;\n";
+        os << "    place(base + left < n ? base + left : base, d, next, zero);\n";
+    }
+    os << "#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) {\n      if (e < cnt) {\n";
+    if (placed && g.short_rows) os << "        place(base + e, d, off, inner);\n";
+    for (size_t i = 0; i < nin; ++i) {
+        const char m = g.modes[i];
+        const std::string k = std::to_string(i), step = m == 'C' ? "1" : m == 'Z' ? "0" : "d.istr[" + k + "][" + last + "]";
+        os << "        x" << i << "[e] = (" << value_type(prog.inputs[i]) << ")i" << i << "[";
+        if (m == 'S') os << "0";
+        else if (m == 'F') os << "base + e";
+        else if (g.short_rows) os << "off[" << k << "]";
+        else os << "(gidx)e < left ? off[" << k << "] + e * " << step << " : next[" << k << "] + (long long)(e - (int)left) * " << step;
+        os << "];\n";
+    }
+    os << "      } else {\n";
+    for (size_t i = 0; i < nin; ++i) os << "        x" << i << "[e] = 0;\n";
+    os << "      }\n    }\n  }\n";
+    for (size_t i = 0; i < nout; ++i) os << "  " << value_type(prog.outputs[i]) << " y" << i << "[" << V << "];\n";
+    os << "  bool rare = false;\n";
+    for (int fast = 1; fast >= 0; --fast) {
+        if (!fast) os << "  if (__builtin_expect(FM_ANY_LANE(rare), 0)) {\n";
+        os << "#pragma unroll\n  for (int e = 0; e < " << V << "; ++e) elem<" << (fast ? "true" : "false") << ">(";
+        for (size_t i = 0; i < nin; ++i) os << (i ? ", " : "") << "x" << i << "[e]";
+        for (size_t i = 0; i < nout; ++i) os << ", y" << i << "[e]";
+        os << ", rare);\n";
+        if (!fast) os << "  }\n";
+    }
+    os << "  if (cnt == " << V << ") {\n";
+    for (size_t i = 0; i < nout; ++i) {
+        const int32_t dt = prog.outputs[i].dtype;
+        if (is_float_dtype(dt)) {
+            os << "    { " << vec_type(dt) << " t; for (int e = 0; e < " << V << "; ++e) t[e] = (" << ctype_of(dt) << ")y" << i << "[e];\n";
+        } else if (V >= 4) {
+            os << "    { Vb t;\n";
+            for (int w = 0; w < V / 4; ++w) {
+                os << "      t[" << w << "] = ";
+                for (int k = 0; k < 4; ++k) os << (k ? " | " : "") << "(((unsigned int)y" << i << "[" << 4 * w + k << "] & 0xffu) << " << 8 * k << ")";
+                os << ";\n";
+            }
+        }
+        os << "      __builtin_nontemporal_store(t, (" << vec_type(dt) << "*)(o" << i << " + base)); }\n";
+    }
+    os << "  } else {\n#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) if (e < cnt) {\n";
+    for (size_t i = 0; i < nout; ++i) os << "      o" << i << "[base + e] = (" << ctype_of(prog.outputs[i].dtype) << ")y" << i << "[e];\n";
+    os << "    }\n  }\n}\n";
+}
+
 // Source of both kernels for one (program, operand modes) combination.
 //   <name>_vec : V elements per thread through 128-bit accesses; operands are full
 //                (same flat index as the output), scalar, or periodic (index modulo a
 //                period that is a multiple of V).
-//   <name>_gen : one element per thread, operands addressed through per-axis strides.
+//   <name>_gen : emit_general.
 int generate_source(
         const Program& prog, const std::string& name, const std::string& modes, const std::vector<uint32_t>& periods,
-        int vec, bool use_fma, std::string* out) {
+        int vec, const GeneralForm& gen, bool use_fma, std::string* out) {
     std::ostringstream os;
     os << "#pragma clang fp contract(off)\n";
     os << "#define FM_FN __device__ __forceinline__\n";
@@ -638,7 +777,7 @@ int generate_source(
     const int steps = 2;
     const std::string VT = prog.arith == CHX_HIP_FLOAT64 ? "double" : "float";  // what elem() takes and gives
     if (prog.arith != CHX_HIP_FLOAT32) {
-        // float16 and float64 programs run on the general kernel; this one is never launched
+        // float16 and float64 programs have the general kernel only; this one is never launched
         os << "extern \"C\" __global__ void " << name << "_vec(unsigned int n_vec) {}\n";
     } else {
     os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_vec(unsigned int n_vec";
@@ -731,34 +870,7 @@ int generate_source(
     }
 
     // ---- general kernel ----
-    os << "struct GenDesc { int ndim; int pad; long long shape[" << CHX_HIP_MAX_NDIM << "]; long long istr[" << nin << "]["
-       << CHX_HIP_MAX_NDIM << "]; };\n";
-    os << "extern \"C\" __global__ __launch_bounds__(256) void " << name
-       << "_gen(unsigned long long begin, unsigned long long n";
-    for (size_t i = 0; i < nin; ++i) os << ", const " << ctype_of(prog.inputs[i].dtype) << "* __restrict__ i" << i;
-    for (size_t i = 0; i < nout; ++i) os << ", " << ctype_of(prog.outputs[i].dtype) << "* __restrict__ o" << i;
-    os << ", GenDesc d) {\n";
-    os << "  const unsigned long long idx = begin + (unsigned long long)blockIdx.x * 256ull + threadIdx.x;\n";
-    os << "  if (idx >= n) return;\n";
-    os << "  long long off[" << nin << "];\n";
-    os << "  for (int i = 0; i < " << nin << "; ++i) off[i] = 0;\n";
-    os << "  unsigned long long rest = idx;\n";
-    os << "  for (int a = d.ndim - 1; a >= 0; --a) {\n";
-    os << "    const unsigned long long q = rest / (unsigned long long)d.shape[a];\n";
-    os << "    const long long r = (long long)(rest - q * (unsigned long long)d.shape[a]);\n";
-    os << "    for (int i = 0; i < " << nin << "; ++i) off[i] += r * d.istr[i][a];\n";
-    os << "    rest = q;\n  }\n";
-    for (size_t i = 0; i < nout; ++i)
-        os << "  " << (is_float_dtype(prog.outputs[i].dtype) ? VT : std::string("int")) << " r" << i << ";\n";
-    os << "  bool rare = false;\n  elem<false>(";
-    for (size_t i = 0; i < nin; ++i)
-        os << (i ? ", " : "") << "(" << (is_float_dtype(prog.inputs[i].dtype) ? VT : std::string("int")) << ")i" << i << "[off[" << i << "]]";
-    for (size_t i = 0; i < nout; ++i) os << ", r" << i;
-    os << ", rare);\n";
-    for (size_t i = 0; i < nout; ++i) {
-        os << "  o" << i << "[idx] = (" << ctype_of(prog.outputs[i].dtype) << ")r" << i << ";\n";
-    }
-    os << "}\n";
+    emit_general(prog, name, gen, VT, os);
     *out = os.str();
     return CHX_HIP_OK;
 }
@@ -805,6 +917,7 @@ struct Plan {
     int64_t shape[CHX_HIP_MAX_NDIM];
     std::vector<std::vector<int64_t>> istr;  // element strides per input, per collapsed axis
     std::vector<uint32_t> periods;
+    GeneralForm gen;
 };
 
 int make_plan(
@@ -907,7 +1020,7 @@ int make_plan(
     for (int a = 0; a < plan->ndim; ++a) plan->shape[a] = cshape[a];
     plan->istr = cstr;
 
-    bool any32 = false;
+    bool any32 = false;  // (an 8-bit operand beside a float32 one moves 4 bytes per access)
     for (const Port& p : prog.inputs) any32 = any32 || p.dtype == CHX_HIP_FLOAT32;
     for (const Port& p : prog.outputs) any32 = any32 || p.dtype == CHX_HIP_FLOAT32;
     plan->vec = any32 ? 4 : 16;
@@ -949,8 +1062,25 @@ int make_plan(
     for (int k = 0; k < n_outputs; ++k)
         if (!aligned(outputs[k]->data, 16)) ok = false;
     plan->vector_ok = ok && n >= plan->vec && prog.arith == CHX_HIP_FLOAT32;
+    GeneralForm& g = plan->gen;
+    g.ndim = plan->ndim;
+    g.vec = any32 ? 4 : prog.arith == CHX_HIP_FLOAT64 ? 2 : prog.arith == CHX_HIP_FLOAT16 ? 8 : 16;
+    g.wide = n >= (int64_t(1) << 31) - 4096;  // (indices run past the last element by less than a work-group's share)
+    g.short_rows = plan->ndim > 0 && cshape[plan->ndim - 1] < g.vec;
+    g.modes.assign(n_inputs, 'X');
+    for (int i = 0; i < n_inputs; ++i) {
+        bool flat = true, one = true;
+        for (int a = 0; a < plan->ndim; ++a) {
+            flat = flat && cstr[i][a] == dense[a];
+            one = one && cstr[i][a] == 0;
+        }
+        if (plan->ndim == 0 || one) g.modes[i] = 'S';
+        else if (flat) g.modes[i] = 'F';
+        else if (cstr[i][plan->ndim - 1] == 1) g.modes[i] = 'C';
+        else if (cstr[i][plan->ndim - 1] == 0) g.modes[i] = 'Z';
+    }
     if (!plan->vector_ok) {
-        // the general kernel ignores modes; use one canonical key
+        // the general kernel ignores these modes; use one canonical key
         plan->modes.assign(n_inputs, kFull);
         plan->periods.assign(n_inputs, 0);
     }
@@ -982,7 +1112,7 @@ int prepare(
     CHX_PROPAGATE(parse_program(code, prog));
     CHX_PROPAGATE(make_plan(*prog, inputs, n_inputs, outputs, n_outputs, plan));
     *name = "fusion" + std::to_string(fusion_id < 0 ? 0 : fusion_id);
-    CHX_PROPAGATE(generate_source(*prog, *name, plan->modes, plan->periods, plan->vec, host_libm_uses_fma(), src));
+    CHX_PROPAGATE(generate_source(*prog, *name, plan->modes, plan->periods, plan->vec, plan->gen, host_libm_uses_fma(), src));
     return CHX_HIP_OK;
 }
 
@@ -1026,10 +1156,25 @@ using namespace chx;
 
 extern "C" int chx_hip_elementwise_output_dtypes(const char* code, int32_t* dtypes, int32_t capacity, int32_t* count) {
     CHX_REQUIRE(count != nullptr && (dtypes != nullptr || capacity == 0), "elementwise_output_dtypes: null output");
-    Program prog;
-    CHX_PROPAGATE(parse_program(code, &prog));
-    *count = (int32_t)prog.outputs.size();
-    for (int32_t i = 0; i < *count && i < capacity; ++i) dtypes[i] = prog.outputs[(size_t)i].dtype;
+    CHX_REQUIRE(code != nullptr, "fusion program: null code");
+    static std::mutex mutex;
+    static std::unordered_map<std::string, std::vector<int32_t>> known;  // asked on every call of a group
+    std::vector<int32_t> found;
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        auto it = known.find(code);
+        if (it != known.end()) found = it->second;
+    }
+    if (found.empty()) {
+        Program prog;
+        CHX_PROPAGATE(parse_program(code, &prog));
+        for (const Port& p : prog.outputs) found.push_back(p.dtype);
+        std::lock_guard<std::mutex> lock(mutex);
+        if (known.size() >= 4096) known.clear();
+        known.emplace(code, found);
+    }
+    *count = (int32_t)found.size();
+    for (int32_t i = 0; i < *count && i < capacity; ++i) dtypes[i] = found[(size_t)i];
     return CHX_HIP_OK;
 }
 
@@ -1055,49 +1200,103 @@ extern "C" int chx_hip_elementwise_source(
     return CHX_HIP_OK;
 }
 
-extern "C" int chx_hip_elementwise(
-        const char* code, int32_t fusion_id, const chx_hip_tensor* const* inputs, int32_t n_inputs,
-        chx_hip_tensor* const* outputs, int32_t n_outputs, void* stream) {
+namespace chx {
+namespace {
+
+// What a call needs beyond its pointers, kept per (program text, operand layouts): parsing the text, planning and writing
+// out the kernel's source to look the compiled kernel up took 35 us of host time per call.
+struct PreparedCall {
+    std::shared_ptr<CompiledKernels> kernels;
+    bool vector = false;
+    int vec = 0;
+    int64_t n = 0;
+    unsigned grid = 0;
+    std::vector<char> desc;  // GenDesc of the general kernel
+};
+constexpr size_t kMostPrepared = 4096;  // (a few hundred bytes each; all are dropped when there are more)
+std::mutex g_prepared_mutex;
+std::unordered_map<std::string, std::shared_ptr<const PreparedCall>> g_prepared;
+
+void append_layout(const chx_hip_tensor* t, std::string* key) {
+    if (!t || t->ndim < 0 || t->ndim > CHX_HIP_MAX_NDIM) return;  // refused when the call is prepared
+    const int32_t head[3] = {t->dtype, t->ndim, aligned(t->data, 16) ? 1 : 0};
+    key->append(reinterpret_cast<const char*>(head), sizeof(head));
+    key->append(reinterpret_cast<const char*>(t->shape), sizeof(int64_t) * (size_t)t->ndim);
+    key->append(reinterpret_cast<const char*>(t->strides), sizeof(int64_t) * (size_t)t->ndim);
+}
+
+int prepare_call(
+        const char* code, int32_t fusion_id, const chx_hip_tensor* const* inputs, int32_t n_inputs, chx_hip_tensor* const* outputs,
+        int32_t n_outputs, PreparedCall* call) {
     Program prog;
     Plan plan;
     std::string name, src;
     CHX_PROPAGATE(prepare(code, fusion_id, inputs, n_inputs, outputs, n_outputs, &prog, &plan, &name, &src));
+    call->n = plan.n;
     if (plan.n == 0) return CHX_HIP_OK;
-    std::shared_ptr<CompiledKernels> ck;
-    CHX_PROPAGATE(get_compiled(src, name, &ck));
-    CHX_PROPAGATE(load_kernels(ck.get(), name));
-    hipStream_t s = as_stream(stream);
-
-    int64_t done = 0;
-    if (plan.vector_ok) {
-        const int64_t n_vec = plan.n / plan.vec;
-        ArgPacker a;
-        a.push((uint32_t)n_vec);
-        for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
-        for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
-        CHX_PROPAGATE(launch(ck->vec, (unsigned)((n_vec + 511) / 512), a, s));
-        done = n_vec * plan.vec;
+    CHX_REQUIRE(plan.n < (int64_t(1) << 39), "fusion: %lld elements is beyond what the general kernel covers", (long long)plan.n);
+    CHX_PROPAGATE(get_compiled(src, name, &call->kernels));
+    CHX_PROPAGATE(load_kernels(call->kernels.get(), name));
+    // (elements beyond whole vectors would be a launch of their own)
+    call->vector = plan.vector_ok && plan.n % plan.vec == 0;
+    call->vec = plan.vec;
+    if (call->vector) {
+        call->grid = (unsigned)((plan.n / plan.vec + 511) / 512);
+        return CHX_HIP_OK;
     }
-    if (done < plan.n) {
-        CHX_REQUIRE(plan.n - done < (int64_t(1) << 39), "fusion: %lld elements is beyond what the general kernel covers",
-                    (long long)(plan.n - done));
-        ArgPacker a;
-        a.push((unsigned long long)done);
-        a.push((unsigned long long)plan.n);
-        for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
-        for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
-        // GenDesc { int ndim; int pad; long long shape[MAX]; long long istr[nin][MAX]; }
-        std::vector<long long> d(1 + CHX_HIP_MAX_NDIM + (size_t)n_inputs * CHX_HIP_MAX_NDIM, 0);
-        int32_t head[2] = {plan.ndim, 0};
-        memcpy(&d[0], head, 8);
-        for (int k = 0; k < plan.ndim; ++k) d[1 + k] = plan.shape[k];
-        for (int k = plan.ndim; k < CHX_HIP_MAX_NDIM; ++k) d[1 + k] = 1;
-        for (int i = 0; i < n_inputs; ++i)
-            for (int k = 0; k < plan.ndim; ++k) d[1 + CHX_HIP_MAX_NDIM + (size_t)i * CHX_HIP_MAX_NDIM + k] = plan.istr[i][k];
-        a.push_bytes(d.data(), d.size() * sizeof(long long), 8);
-        CHX_PROPAGATE(launch(ck->gen, (unsigned)((plan.n - done + 255) / 256), a, s));
+    call->grid = (unsigned)((plan.n + 256 * plan.gen.vec - 1) / (256 * plan.gen.vec));
+    // GenDesc { unsigned mul[MAX], shift[MAX]; long long shape[MAX]; long long istr[nin][MAX]; }
+    const size_t M = CHX_HIP_MAX_NDIM;
+    call->desc.assign(2 * M * 4 + M * 8 + (size_t)n_inputs * M * 8, 0);
+    uint32_t* mul = reinterpret_cast<uint32_t*>(call->desc.data());
+    int64_t* shape = reinterpret_cast<int64_t*>(call->desc.data() + 2 * M * 4);
+    for (size_t a = 0; a < M; ++a) {
+        shape[a] = a < (size_t)plan.ndim ? plan.shape[a] : 1;
+        if (!plan.gen.wide) magic_divisor((uint32_t)shape[a], &mul[a], &mul[M + a]);
     }
+    for (int i = 0; i < n_inputs; ++i)
+        for (int a = 0; a < plan.ndim; ++a) shape[M * (size_t)(1 + i) + (size_t)a] = plan.istr[i][a];
     return CHX_HIP_OK;
+}
+
+}  // namespace
+}  // namespace chx
+
+extern "C" int chx_hip_elementwise(
+        const char* code, int32_t fusion_id, const chx_hip_tensor* const* inputs, int32_t n_inputs,
+        chx_hip_tensor* const* outputs, int32_t n_outputs, void* stream) {
+    CHX_REQUIRE(code != nullptr, "fusion program: null code");
+    CHX_REQUIRE(inputs != nullptr && n_inputs > 0, "fusion: no inputs");  // CHECK(!inputs.empty()), nvrtc.cc:93
+    CHX_REQUIRE(outputs != nullptr && n_outputs > 0, "fusion: no outputs");
+    for (int i = 0; i < n_inputs; ++i) CHX_PROPAGATE(check_tensor(inputs[i], "fusion input"));
+    for (int i = 0; i < n_outputs; ++i) CHX_PROPAGATE(check_tensor(outputs[i], "fusion output"));
+    std::string key(code);
+    const int32_t ids[3] = {fusion_id, n_inputs, n_outputs};
+    key.append(1, '\0').append(reinterpret_cast<const char*>(ids), sizeof(ids));
+    for (int i = 0; i < n_inputs; ++i) append_layout(inputs[i], &key);
+    for (int i = 0; i < n_outputs; ++i) append_layout(outputs[i], &key);
+    std::shared_ptr<const PreparedCall> call;
+    {
+        std::lock_guard<std::mutex> lock(g_prepared_mutex);
+        auto it = g_prepared.find(key);
+        if (it != g_prepared.end()) call = it->second;
+    }
+    if (!call) {
+        auto made = std::make_shared<PreparedCall>();
+        CHX_PROPAGATE(prepare_call(code, fusion_id, inputs, n_inputs, outputs, n_outputs, made.get()));
+        call = made;
+        std::lock_guard<std::mutex> lock(g_prepared_mutex);
+        if (g_prepared.size() >= kMostPrepared) g_prepared.clear();
+        g_prepared.emplace(std::move(key), call);
+    }
+    if (call->n == 0) return CHX_HIP_OK;
+    ArgPacker a;
+    if (call->vector) a.push((uint32_t)(call->n / call->vec));
+    else a.push((unsigned long long)call->n);
+    for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
+    for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
+    if (!call->vector) a.push_bytes(call->desc.data(), call->desc.size(), 8);
+    return launch(call->vector ? call->kernels->vec : call->kernels->gen, call->grid, a, as_stream(stream));
 }
 
 extern "C" int chx_hip_elementwise_match_residual_add(const char* code, int32_t* matches, chx_hip_residual_group* group) {
