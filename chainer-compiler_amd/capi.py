@@ -2,6 +2,7 @@
 current stream only; every computation goes through libchx_hip.so, and a missing
 library is an error (there is no fallback path)."""
 import ctypes
+import importlib.util
 import os
 
 import torch
@@ -9,6 +10,7 @@ import torch
 MAX_NDIM = 10
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libchx_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "lib", "_chx_torch_ops.so")
 
 # ChainerX dtype codes (compiler/dtype.h:14-25 of the reference tree)
 BOOL, INT8, INT16, INT32, INT64, UINT8, FLOAT16, FLOAT32, FLOAT64 = 1, 2, 3, 4, 5, 6, 7, 8, 9
@@ -91,6 +93,25 @@ def lib():
         _lib.chx_hip_version.restype = ctypes.c_char_p
         _lib.chx_hip_qconv_plan_destroy.restype = None
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The extension module with the ops' hot paths (binding/torch_ops.cc): tensors to descriptors, result allocation and
+    the call in one step."""
+    global _native
+    if _native is None:
+        lib()  # the in-tree build, which the extension is linked against
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError("%s is missing: build it with `make -C chainer-compiler_amd/binding`" % NATIVE_PATH)
+        spec = importlib.util.spec_from_file_location("_chx_torch_ops", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.init(ChxHipError)
+        _native = mod
+    return _native
 
 
 def check(rc):

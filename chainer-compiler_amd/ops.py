@@ -8,9 +8,11 @@ StrictScalar are Python numbers, with the zero point's dtype given explicitly
 because it selects the output dtype (runtime/ops/quantize.cc:17-25).
 
 All arithmetic happens in libchx_hip.so; these wrappers only infer output shapes
-and allocate, like the RunImpl bodies do.
+and allocate, like the RunImpl bodies do.  The ops of the quantized path do that in
+the native extension (capi.native()); the others through ctypes.
 """
 import ctypes
+import functools
 
 import torch
 
@@ -33,22 +35,12 @@ def _channels_last_empty(shape, dtype, device):
 def QuantizeLinear(x, y_scale, y_zero_point=None, zero_point_dtype=torch.uint8, flags=0, out=None):
     """QuantizeLinearOp::RunImpl, runtime/ops/quantize.cc:48-53.  An absent zero point
     means uint8 0."""
-    zp = 0 if y_zero_point is None else int(y_zero_point)
-    if out is None:
-        out = torch.empty_like(x, dtype=zero_point_dtype)
-    capi.check(capi.lib().chx_hip_quantize_linear(capi.ref(x), _f(y_scale), _i(zp), ctypes.c_uint32(flags),
-                                                  capi.ref(out), capi.stream_ptr()))
-    return out
+    return capi.native().quantize_linear(x, y_scale, 0 if y_zero_point is None else y_zero_point, zero_point_dtype, flags, out)
 
 
 def DequantizeLinear(x, x_scale, x_zero_point=None, out=None):
     """DequantizeLinearOp::RunImpl, runtime/ops/quantize.cc:55-60."""
-    zp = 0 if x_zero_point is None else int(x_zero_point)
-    if out is None:
-        out = torch.empty_like(x, dtype=torch.float32)
-    capi.check(capi.lib().chx_hip_dequantize_linear(capi.ref(x), _f(x_scale), _i(zp), capi.ref(out),
-                                                    capi.stream_ptr()))
-    return out
+    return capi.native().dequantize_linear(x, x_scale, 0 if x_zero_point is None else x_zero_point, out)
 
 
 _DTYPE_NAMES = {torch.float32: "float32", torch.float16: "float16", torch.float64: "float64", torch.uint8: "uint8", torch.int8: "int8"}
@@ -67,10 +59,12 @@ def fusion_program(inputs, statements, outputs):
     return "\n".join(lines) + "\n"
 
 
-def _program_output_dtypes(code):
-    """Result types of a fusion program: this library's program text or the CUDA C text the reference's compiler emits."""
+@functools.lru_cache(maxsize=1024)
+def _program_text(code):
+    """The text as bytes and the result types of a fusion program: this library's program text or the CUDA C text the
+    reference's compiler emits."""
     torch_of = {v: k for k, v in capi._TORCH_TO_CHX.items()}
-    return [torch_of[c] for c in capi.elementwise_output_dtypes(code)]
+    return code.encode(), tuple(torch_of[c] for c in capi.elementwise_output_dtypes(code))
 
 
 def ElementWiseNvrtc(inputs, num_outputs, code, fusion_id=0, outs=None):
@@ -78,23 +72,9 @@ def ElementWiseNvrtc(inputs, num_outputs, code, fusion_id=0, outs=None):
     broadcast of the input shapes; `num_outputs` arrays of that shape are allocated.
     When every full-shape input is channels-last the outputs are allocated
     channels-last too, so chains between convolutions never transpose."""
-    out_dtypes = _program_output_dtypes(code)
+    text, out_dtypes = _program_text(code)
     assert len(out_dtypes) == num_outputs
-    if outs is None:
-        shape = torch.broadcast_shapes(*[tuple(t.shape) for t in inputs])
-        full = [t for t in inputs if tuple(t.shape) == tuple(shape)]
-        cl = len(shape) == 4 and full and all(
-            t.permute(0, 2, 3, 1).is_contiguous() and not t.is_contiguous() for t in full)
-        if cl:
-            outs = [_channels_last_empty(shape, dt, inputs[0].device) for dt in out_dtypes]
-        else:
-            outs = [torch.empty(shape, dtype=dt, device=inputs[0].device) for dt in out_dtypes]
-    ins = capi.tensor_array([capi.desc(t) for t in inputs])
-    outp = capi.tensor_array([capi.desc(t) for t in outs])
-    capi.check(capi.lib().chx_hip_elementwise(code.encode(), ctypes.c_int32(fusion_id), ins,
-                                              ctypes.c_int32(len(inputs)), outp, ctypes.c_int32(len(outs)),
-                                              capi.stream_ptr()))
-    return outs
+    return capi.native().elementwise(inputs, text, fusion_id, out_dtypes, outs)
 
 
 # --- convolution attribute handling (runtime/chainerx_util.cc:180-200, 276-311) -----------------
@@ -135,6 +115,13 @@ def _conv_setup(x, w, strides, pads, group, auto_pad):
     return capi.conv_nd_params(strides, begin, end, group), (x.shape[0], w.shape[0]) + out
 
 
+def _plain_geometry(w, strides, pads, group):
+    """(strides, pads at the begin, at the end, group) of a 2-D convolution without auto_pad: independent of the input."""
+    strides, pads = _complement(strides, 2, 1), _complement(pads, 2, 0)
+    begin, end = (pads[:2], pads[2:]) if len(pads) == 4 else (pads, pads)
+    return tuple(int(v) for v in (*strides[:2], *begin[:2], *end[:2], group))
+
+
 def _alloc_like_input_layout(x, shape, dtype):
     if x.dim() == 4 and not x.is_contiguous() and x.permute(0, 2, 3, 1).is_contiguous():
         return _channels_last_empty(shape, dtype, x.device)
@@ -145,6 +132,9 @@ def QLinearConv(x, x_scale, x_zero_point, w, w_scale, w_zero_point, y_scale, y_z
                 pads=(), group=1, auto_pad="", zero_point_dtype=torch.uint8, flags=0, out=None):
     """QLinearConvOp::RunImpl, runtime/ops/quantize.cc:62-94.  The output dtype is the
     dtype of y_zero_point."""
+    if x.dim() == 4 and w.dim() == 4 and not auto_pad:
+        return capi.native().qlinear_conv(x, x_scale, x_zero_point, w, w_scale, w_zero_point, y_scale, y_zero_point, b,
+                                          _plain_geometry(w, strides, pads, group), zero_point_dtype, flags, out)
     params, shape = _conv_setup(x, w, strides, pads, group, auto_pad)
     if out is None:
         out = _alloc_like_input_layout(x, shape, zero_point_dtype)
@@ -158,6 +148,8 @@ def QLinearConv(x, x_scale, x_zero_point, w, w_scale, w_zero_point, y_scale, y_z
 
 def ConvInteger(x, w, x_zero_point=None, w_zero_point=None, strides=(), pads=(), group=1, auto_pad="", out=None):
     """ConvIntegerOp::RunImpl, runtime/ops/quantize.cc:116-146."""
+    if x.dim() == 4 and w.dim() == 4 and not auto_pad:
+        return capi.native().conv_integer(x, w, 0 if x_zero_point is None else x_zero_point, w_zero_point, _plain_geometry(w, strides, pads, group), out)
     params, shape = _conv_setup(x, w, strides, pads, group, auto_pad)
     if out is None:
         out = _alloc_like_input_layout(x, shape, torch.int32)
@@ -170,11 +162,7 @@ def ConvInteger(x, w, x_zero_point=None, w_zero_point=None, strides=(), pads=(),
 
 def MatMulInteger(a, b, a_zero_point=None, b_zero_point=None, out=None):
     """MatMulIntegerOp::RunImpl, runtime/ops/quantize.cc:96-114."""
-    if out is None:
-        out = torch.empty(tuple(a.shape[:-1]) + (b.shape[-1],), dtype=torch.int32, device=a.device)
-    capi.check(capi.lib().chx_hip_matmul_integer(capi.ref(a), capi.ref(b), capi.ref(a_zero_point),
-                                                 capi.ref(b_zero_point), capi.ref(out), capi.stream_ptr()))
-    return out
+    return capi.native().matmul_integer(a, b, a_zero_point, b_zero_point, out)
 
 
 def QLinearMatMul(a, a_scale, a_zero_point, b, b_scale, b_zero_point, y_scale, y_zero_point, bias=None,
@@ -182,12 +170,7 @@ def QLinearMatMul(a, a_scale, a_zero_point, b, b_scale, b_zero_point, y_scale, y
     """The DequantizeLinear, DequantizeLinear, MatMul, QuantizeLinear sequence that
     ReplaceQLinearMatMul (compiler/simplifier.cc:675-694) leaves for a QLinearMatMul
     node, as one call."""
-    if out is None:
-        out = torch.empty(tuple(a.shape[:-1]) + (b.shape[-1],), dtype=zero_point_dtype, device=a.device)
-    capi.check(capi.lib().chx_hip_qlinear_matmul(
-        capi.ref(a), _f(a_scale), _i(a_zero_point), capi.ref(b), _f(b_scale), _i(b_zero_point), _f(y_scale),
-        _i(y_zero_point), capi.ref(bias), ctypes.c_uint32(flags), capi.ref(out), capi.stream_ptr()))
-    return out
+    return capi.native().qlinear_matmul(a, a_scale, a_zero_point, b, b_scale, b_zero_point, y_scale, y_zero_point, bias, zero_point_dtype, flags, out)
 
 
 def BitShift(x, y, direction):
@@ -255,9 +238,13 @@ class QLinearConvPlan(object):
         self._keep = (w, w_scale, w_zero_point, b)
         self.w, self.strides, self.pads, self.group, self.auto_pad = w, strides, pads, group, auto_pad
         self._plans = {}
+        self._fixed = None  # (plan, (oc, kh, kw), geometry) of a plan whose geometry no input changes
 
     def _plan_for(self, x):
         params, shape = _conv_setup(x, self.w, self.strides, self.pads, self.group, self.auto_pad)
+        return self._plan_of(params), shape
+
+    def _plan_of(self, params):
         key = tuple(getattr(params, f) for f, _ in params._fields_)
         if key not in self._plans:
             handle = ctypes.c_void_p()
@@ -266,9 +253,15 @@ class QLinearConvPlan(object):
                 capi.ref(w), capi.ref(w_scale), capi.ref(w_zero_point), capi.ref(b), ctypes.byref(params),
                 capi.stream_ptr(), ctypes.byref(handle)))
             self._plans[key] = handle
-        return self._plans[key], shape
+        return self._plans[key]
 
     def run(self, x, x_scale, x_zero_point, y_scale, y_zero_point, zero_point_dtype=torch.uint8, flags=0, out=None):
+        if not self.auto_pad and self.w.dim() == 4 and x.dim() == 4:
+            if self._fixed is None:
+                geometry = _plain_geometry(self.w, self.strides, self.pads, self.group)
+                self._fixed = (self._plan_of(capi.ConvParams(*geometry)).value, (self.w.shape[0], self.w.shape[2], self.w.shape[3]), geometry)
+            plan, filters, geometry = self._fixed
+            return capi.native().plan_run(plan, x, filters, geometry, x_scale, x_zero_point, y_scale, y_zero_point, zero_point_dtype, flags, out)
         handle, shape = self._plan_for(x)
         if out is None:
             out = _alloc_like_input_layout(x, shape, zero_point_dtype)
@@ -321,6 +314,7 @@ class QLinearConvPlan(object):
         for handle in self._plans.values():
             capi.lib().chx_hip_qconv_plan_destroy(handle)
         self._plans = {}
+        self._fixed = None
 
     def __del__(self):
         try:
