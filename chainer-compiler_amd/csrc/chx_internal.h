@@ -151,6 +151,27 @@ bool stream_is_capturing(hipStream_t s);
 int scratch_alloc(void** p, size_t bytes, hipStream_t s);
 void scratch_free(void* p, hipStream_t s);
 
+// Scratch memory for one call, released when the object goes.  hipMallocAsync and hipFreeAsync take 9.4 us of host time
+// per buffer, so calls on the null stream share one block per device (they run in order; the object holds the block's
+// lock while its call enqueues): at most 256 MB, given back when calls have stopped needing it.  Other streams, and
+// larger requests, are stream-ordered allocations.
+class Scratch {
+public:
+    Scratch() = default;
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+    ~Scratch();
+    int acquire(size_t bytes, hipStream_t s);
+    void* ptr() const {
+        return ptr_;
+    }
+
+private:
+    void* ptr_ = nullptr;
+    hipStream_t stream_ = nullptr;
+    int shared_ = -1;  // device whose block this is
+};
+
 struct StridedDesc {
     int32_t ndim;
     int64_t shape[CHX_HIP_MAX_NDIM];

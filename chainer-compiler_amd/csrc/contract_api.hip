@@ -1393,8 +1393,16 @@ extern "C" int chx_hip_conv_integer(
         a.w_zp_stride = stride;
     }
     hipStream_t s = as_stream(stream);
-    // (a recorded run takes the kernel without scratch memory: the weights of this entry point are packed per call)
-    if (weights_fit_mfma(*w, params->group) && !stream_is_capturing(s)) {
+    // (a recorded run takes the kernel without scratch memory: the weights of this entry point arrive with the call)
+    const bool capturing = stream_is_capturing(s);
+    // The packed kernel multiplies faster but costs some 70 us of host time per call (read-back of the zero points,
+    // allocations, packing): the two meet at 8 G multiply-adds, and it takes channels-last results only.
+    const bool packed = weights_fit_mfma(*w, params->group) && (double)a.total * cs.Cg * cs.KH * cs.KW >= 0x1p33 && x_is_mfma_ready(*x);
+    if (!capturing && !packed) {
+        const int rc = run_conv_planar(a, s);
+        if (rc != CHX_HIP_EUNSUPPORTED) return rc;
+    }
+    if (weights_fit_mfma(*w, params->group) && !capturing) {
         bool zero = true;
         if (w_zero_point) {
             std::vector<uint8_t> zp;

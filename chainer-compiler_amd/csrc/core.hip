@@ -1,6 +1,7 @@
 // Library state, error reporting and the thin device-memory helpers of the C ABI.
 #include <cmath>
 #include <cstring>
+#include <mutex>
 
 #include "chx_internal.h"
 
@@ -101,6 +102,50 @@ int scratch_alloc(void** p, size_t bytes, hipStream_t s) {
 
 void scratch_free(void* p, hipStream_t s) {
     if (p) (void)hipFreeAsync(p, s);
+}
+
+namespace {
+constexpr int kMostDevices = 16;
+constexpr size_t kMostShared = size_t(256) << 20;
+struct SharedBlock {
+    std::mutex mutex;
+    void* ptr = nullptr;
+    size_t size = 0;
+    int small_uses = 0;  // calls in a row that needed less than a quarter of the block
+};
+SharedBlock& shared_block(int device) {
+    static SharedBlock* blocks = new SharedBlock[kMostDevices];  // never destroyed: calls may come from other destructors
+    return blocks[device];
+}
+}  // namespace
+
+int Scratch::acquire(size_t bytes, hipStream_t s) {
+    int device = 0;
+    if (s != nullptr || bytes > kMostShared || hipGetDevice(&device) != hipSuccess || device >= kMostDevices) {
+        stream_ = s;
+        return scratch_alloc(&ptr_, bytes, s);
+    }
+    SharedBlock& b = shared_block(device);
+    b.mutex.lock();
+    shared_ = device;
+    b.small_uses = bytes * 4 < b.size ? b.small_uses + 1 : 0;
+    if (bytes > b.size || b.small_uses > 256) {
+        size_t size = size_t(1) << 20;
+        while (size < bytes) size *= 2;
+        if (b.ptr) CHX_HIP_CALL(hipFree(b.ptr));  // (waits for the work that still uses it)
+        b.ptr = nullptr;
+        b.size = 0;
+        b.small_uses = 0;
+        CHX_HIP_CALL(hipMalloc(&b.ptr, size));
+        b.size = size;
+    }
+    ptr_ = b.ptr;
+    return CHX_HIP_OK;
+}
+
+Scratch::~Scratch() {
+    if (shared_ >= 0) shared_block(shared_).mutex.unlock();
+    else scratch_free(ptr_, stream_);
 }
 
 }  // namespace chx
