@@ -2,10 +2,14 @@
 // QLinearMatMul.  Validation and shape rules follow the reference's RunImpl bodies
 // (runtime/ops/quantize.cc:62-146) and GroupedConv (runtime/chainerx_util.cc:313-340);
 // the arithmetic is in the kernels.
+#include <algorithm>
+#include <array>
 #include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -248,13 +252,13 @@ LaunchOptions read_launch_options() {
 }
 
 // Tile shape: the largest tile that still gives every compute unit a work-group.
-void pick_tile(const LaunchOptions& opt, int OC, int64_t M, int bk, int* tile_oc, int* tile_px, int* max_wgs_per_cu, int* waves) {
+void pick_tile(const LaunchOptions& opt, const ConvMfmaArgs& a, bool out_int32, int* tile_oc, int* tile_px, int* max_wgs_per_cu, int* waves) {
     *waves = 4;
     if (opt.forced_tile) {
         const int toc = opt.tile_oc, tpx = opt.tile_px, wv = opt.waves;
         const bool four = wv == 4 && (toc == 64 || toc == 128) && (tpx == 64 || tpx == 128);
-        const bool eight = wv == 8 && ((toc == 128 && tpx == 128) || (bk == 128 && ((toc == 128 && tpx == 256) || (toc == 64 && tpx == 128))));
-        if (four || eight) {
+        const bool eight = wv == 8 && ((toc == 128 && tpx == 128) || (a.bk == 128 && ((toc == 128 && tpx == 256) || (toc == 64 && tpx == 128))));
+        if (four || eight || (conv_split_has(toc, tpx, wv) && conv_split_takes(a) && !out_int32)) {
             *tile_oc = toc;
             *tile_px = tpx;
             *max_wgs_per_cu = opt.max_wgs_per_cu;
@@ -266,8 +270,8 @@ void pick_tile(const LaunchOptions& opt, int OC, int64_t M, int bk, int* tile_oc
     const int64_t want = 256;
     for (int i = 0; i < 4; ++i) {
         int toc = cand[i][0], tpx = cand[i][1];
-        if (OC <= 64 && toc > 64) continue;
-        const int64_t blocks = (int64_t)((OC + toc - 1) / toc) * ((M + tpx - 1) / tpx);
+        if (a.OC <= 64 && toc > 64) continue;
+        const int64_t blocks = (int64_t)((a.OC + toc - 1) / toc) * ((a.M + tpx - 1) / tpx);
         *tile_oc = toc;
         *tile_px = tpx;
         if (blocks >= want) return;
@@ -275,13 +279,13 @@ void pick_tile(const LaunchOptions& opt, int OC, int64_t M, int bk, int* tile_oc
 }
 
 // Launch configurations measured for the input shapes a plan has seen: the first eager call on
-// a new shape times every tile shape and occupancy cap on the call's own operands (every
+// a new shape times the tile shapes and occupancy caps on the call's own operands (every
 // configuration writes the same bytes) and later calls reuse the fastest.
 struct TunedConfig {
     int64_t M;
     int32_t H, W, OH, OW;
     int tile_oc, tile_px, max_wgs_per_cu;
-    int waves;      // wavefronts per work-group: 4 or 8
+    int waves;      // wavefronts per work-group
     bool with_res;  // measured with a fused residual sum (an entry of its own: the epilogue differs)
     int32_t oc_split = 0;  // measured as two convolutions in one launch, split here (restricts the tiles)
 };
@@ -289,46 +293,99 @@ struct TuneCache {
     std::vector<TunedConfig> entries;
 };
 
-// Times every launch configuration on the call's operands and keeps the fastest in *best.
-int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hipStream_t s, TunedConfig* best) {
+struct Configuration {
+    int tile_oc, tile_px, max_wgs_per_cu, waves;
+};
+
+// What was measured for one plan holds for every other one of the same geometry: a network repeats most of its
+// convolutions, and a second program over the same shapes finds all of them measured.
+class MeasuredConfigurations {
+public:
+    using Key = std::array<int64_t, 24>;
+    static Key key(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne) {
+        int device = 0;
+        (void)hipGetDevice(&device);
+        const int64_t res = a.res.r ? 1 + a.res.affine : 0;
+        return {device, a.M, a.H, a.W, a.OH, a.OW, a.KH, a.KW, a.sh, a.sw, a.ph, a.pw, a.C16, a.KP, a.bk, a.OC, a.oc_split, a.x_n_stride,
+                a.x_w_stride, a.y_px_stride, a.y_vec_ok, res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
+    }
+    bool find(const Key& k, Configuration* c) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const auto it = known_.find(k);
+        if (it == known_.end()) return false;
+        *c = it->second;
+        return true;
+    }
+    void add(const Key& k, const Configuration& c) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (known_.size() >= 4096) known_.clear();  // bounded: a program of ever new shapes measures again
+        known_[k] = c;
+    }
+
+private:
+    std::mutex mutex_;
+    std::map<Key, Configuration> known_;
+};
+
+MeasuredConfigurations& measured_configurations() {
+    static MeasuredConfigurations* m = new MeasuredConfigurations;
+    return *m;
+}
+
+// Times the launch configurations on the call's operands and gives the fastest.
+int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hipStream_t s, Configuration* best) {
     // tile (output channels x pixels), wavefronts; the eight-wavefront kernels take the compute unit alone
     static const int tiles[7][3] = {{128, 128, 4}, {64, 128, 4}, {128, 64, 4}, {64, 64, 4}, {128, 128, 8}, {128, 256, 8}, {64, 128, 8}};
-    static const int caps[3] = {0, 2, 1};
+    struct Candidate {
+        Configuration c;
+        float ms;
+    };
+    std::vector<Candidate> all;
+    for (const auto& t : tiles) {
+        if (a.OC <= 64 && t[0] > 64) continue;
+        if (a.oc_split % t[0] != 0) continue;  // two outputs: a tile belongs to one of them whole
+        if (t[2] == 8 && (t[0] == 64 || t[1] == 256) && a.bk != 128) continue;
+        const int64_t tiles_all = (int64_t)((a.OC + t[0] - 1) / t[0]) * ((a.M + t[1] - 1) / t[1]);
+        all.push_back({{t[0], t[1], 0, t[2]}, 0.f});
+        // (a cap that the tiles do not reach is the launch without one)
+        if (t[2] == 4 && tiles_all > 512) all.push_back({{t[0], t[1], 2, t[2]}, 0.f});
+        if (t[2] == 4 && tiles_all > 256) all.push_back({{t[0], t[1], 1, t[2]}, 0.f});
+    }
+    // launches that the staged tiles fill (in tiles of 64 x 64, eight per compute unit) are not for the small tiles: they
+    // read their operands from L2 once per tile
+    if (!out_int32 && conv_split_takes(a) && (int64_t)((a.OC + 63) / 64) * ((a.M + 63) / 64) <= 2048)
+        for (const ConvSplitTile& t : kConvSplitTiles) all.push_back({{t.oc, t.px, 0, t.waves}, 0.f});
+
     hipEvent_t e0, e1;
     CHX_HIP_CALL(hipEventCreate(&e0));
     CHX_HIP_CALL(hipEventCreate(&e1));
-    float best_ms = -1.f;
     int rc = CHX_HIP_OK;
-    for (int t = 0; t < 7 && rc == CHX_HIP_OK; ++t) {
-        if (a.OC <= 64 && tiles[t][0] > 64) continue;
-        if (a.oc_split % tiles[t][0] != 0) continue;  // two outputs: a tile belongs to one of them whole
-        if (tiles[t][2] == 8 && (tiles[t][0] == 64 || tiles[t][1] == 256) && a.bk != 128) continue;
-        for (int c = 0; c < (tiles[t][2] == 8 ? 1 : 3) && rc == CHX_HIP_OK; ++c) {
-            const int reps = 3;
-            rc = launch_conv_mfma(a, tiles[t][0], tiles[t][1], caps[c], tiles[t][2], xu, out_int32, rne, s);  // warm
-            if (rc != CHX_HIP_OK) break;
-            if (hipEventRecord(e0, s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
-            for (int r = 0; r < reps && rc == CHX_HIP_OK; ++r)
-                rc = launch_conv_mfma(a, tiles[t][0], tiles[t][1], caps[c], tiles[t][2], xu, out_int32, rne, s);
-            if (rc != CHX_HIP_OK) break;
-            float ms = 0.f;
-            if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = CHX_HIP_ERUNTIME;
-                break;
+    auto measure = [&](const Configuration& c, int reps) {
+        float ms = 0.f;
+        rc = launch_conv_mfma(a, c.tile_oc, c.tile_px, c.max_wgs_per_cu, c.waves, xu, out_int32, rne, s);  // warm
+        if (rc != CHX_HIP_OK) return ms;
+        if (hipEventRecord(e0, s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+        for (int r = 0; r < reps && rc == CHX_HIP_OK; ++r) rc = launch_conv_mfma(a, c.tile_oc, c.tile_px, c.max_wgs_per_cu, c.waves, xu, out_int32, rne, s);
+        if (rc != CHX_HIP_OK) return ms;
+        if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+        return ms / reps;
+    };
+    // three launches each, then the best five again, in turn: single measurements of launches of a few microseconds differ
+    // by more than the configurations do
+    for (Candidate& c : all)
+        if (rc == CHX_HIP_OK) c.ms = measure(c.c, 3);
+    std::sort(all.begin(), all.end(), [](const Candidate& l, const Candidate& r) { return l.ms < r.ms; });
+    if (all.size() > 5) all.resize(5);
+    for (int round = 0; round < 3; ++round)
+        for (Candidate& c : all)
+            if (rc == CHX_HIP_OK && c.ms <= 1.3f * all[0].ms) {
+                const float ms = measure(c.c, 4);
+                c.ms = round == 0 ? ms : std::min(c.ms, ms);
             }
-            if (best_ms < 0.f || ms < best_ms) {
-                best_ms = ms;
-                best->tile_oc = tiles[t][0];
-                best->tile_px = tiles[t][1];
-                best->max_wgs_per_cu = caps[c];
-                best->waves = tiles[t][2];
-            }
-        }
-    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc != CHX_HIP_OK) CHX_FAIL(rc, "timing the convolution launch configurations failed: %s", chx_hip_last_error());
+    *best = std::min_element(all.begin(), all.end(), [](const Candidate& l, const Candidate& r) { return l.ms < r.ms; })->c;
     return CHX_HIP_OK;
 }
 
@@ -628,7 +685,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     if (c.res) a.res = *c.res;
     CHX_REQUIRE(a.M < (int64_t(1) << 31), "QLinearConv: too many output pixels for the MFMA kernel");
     int toc = 64, tpx = 64, cap = 0, waves = 4;
-    pick_tile(c.opt, cs.OC, a.M, a.bk, &toc, &tpx, &cap, &waves);
+    pick_tile(c.opt, a, c.out_int32, &toc, &tpx, &cap, &waves);
     if (a.oc_split % toc != 0) toc = 64, waves = 4, tpx = tpx > 128 ? 128 : tpx;  // (the split is a multiple of 64)
     int rc = CHX_HIP_OK;
     const TunedConfig* tuned = nullptr;
@@ -636,10 +693,14 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         for (const TunedConfig& t : c.tune->entries)
             if (t.M == a.M && t.H == a.H && t.W == a.W && t.OH == a.OH && t.OW == a.OW && t.with_res == (c.res != nullptr) && t.oc_split == a.oc_split) tuned = &t;
         if (!tuned && c.opt.autotune && !stream_is_capturing(s)) {
-            TunedConfig best = {a.M, a.H, a.W, a.OH, a.OW, toc, tpx, 0, waves, c.res != nullptr, a.oc_split};
-            rc = tune_conv_mfma(a, xu, c.out_int32, c.rne, s, &best);
+            const MeasuredConfigurations::Key key = MeasuredConfigurations::key(a, xu, c.out_int32, c.rne);
+            Configuration best;
+            if (!measured_configurations().find(key, &best)) {
+                rc = tune_conv_mfma(a, xu, c.out_int32, c.rne, s, &best);
+                if (rc == CHX_HIP_OK) measured_configurations().add(key, best);
+            }
             if (rc == CHX_HIP_OK) {
-                c.tune->entries.push_back(best);
+                c.tune->entries.push_back({a.M, a.H, a.W, a.OH, a.OW, best.tile_oc, best.tile_px, best.max_wgs_per_cu, best.waves, c.res != nullptr, a.oc_split});
                 tuned = &c.tune->entries.back();
             }
         }

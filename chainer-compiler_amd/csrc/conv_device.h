@@ -1,4 +1,4 @@
-// Device-side pieces shared by the matrix-core convolution kernels (conv_mfma.hip, conv_bs.hip).
+// Device-side pieces shared by the matrix-core convolution kernels.
 // Everything here has internal linkage: each translation unit gets its own copy.
 #pragma once
 
@@ -71,6 +71,32 @@ __device__ __forceinline__ void keep_scalar(int& v) { v = __builtin_amdgcn_readf
 // Per-lane byte offsets handed to buffer copies carry this bit when the lane must not fetch anything:
 // the offset then lies beyond any resource this library builds (at most 2^31 - 1 bytes).
 constexpr uint32_t kOutOfRange = 0x80000000u;
+
+// Touch every 64-byte line of the kernel arguments at once.  The argument block of a fresh launch
+// is not in any cache, and the compiler fetches the fields in several dependent batches that
+// each touch new lines: one round trip to memory per batch.  After this, one round trip.
+template <int BYTES>
+__device__ __forceinline__ void warm_kernel_arguments() {
+    const uint64_t ka = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LINES = (BYTES + 63) / 64;
+    static_assert(LINES >= 4 && LINES <= 8, "between four and eight lines are touched");
+    // offsets of the last lines, clamped into the block so that nothing outside it is read
+    constexpr int L4 = LINES > 4 ? 0x100 : 0xc0, L5 = LINES > 5 ? 0x140 : L4, L6 = LINES > 6 ? 0x180 : L5, L7 = LINES > 7 ? 0x1c0 : L6;
+    int t0, t1, t2, t3, t4, t5, t6, t7;
+    asm volatile(
+            "s_load_dword %0, %8, 0x0\n\t"
+            "s_load_dword %1, %8, 0x40\n\t"
+            "s_load_dword %2, %8, 0x80\n\t"
+            "s_load_dword %3, %8, 0xc0\n\t"
+            "s_load_dword %4, %8, %9\n\t"
+            "s_load_dword %5, %8, %10\n\t"
+            "s_load_dword %6, %8, %11\n\t"
+            "s_load_dword %7, %8, %12\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7)
+            : "s"(ka), "n"(L4), "n"(L5), "n"(L6), "n"(L7)
+            : "memory");
+}
 
 // Copies Q0 .. Q0+N-1 of a wave's group of up to four asynchronous 16-byte-per-lane copies through a buffer
 // resource into LDS, as one statement so that nothing can touch M0 between them.  Copy q reads byte offset

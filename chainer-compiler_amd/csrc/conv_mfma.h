@@ -177,6 +177,15 @@ CHX_CONV_MFMA_TILES(CHX_CONV_MFMA_DECLARE)
 int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_cu, int waves, bool x_unsigned, bool out_int32, bool rne,
                      hipStream_t s);
 
+// The kernels for launches with few tiles (conv_split.hip): tile and wavefronts.
+struct ConvSplitTile {
+    int oc, px, waves;
+};
+constexpr ConvSplitTile kConvSplitTiles[] = {{16, 32, 4}, {16, 32, 8}, {16, 32, 16}, {32, 32, 2}, {32, 32, 4}, {32, 32, 8}, {32, 64, 4}, {32, 64, 8}};
+bool conv_split_has(int tile_oc, int tile_px, int waves);
+inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
+int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s);
+
 // [N][C][HW] bytes -> [N][HW][pitch] bytes (lanes c >= C of a pixel are zero filled) and back
 int launch_nchw_to_nhwc_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);
 int launch_nhwc_to_nchw_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);

@@ -387,6 +387,10 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     a.row_unit = 0;
     if (a.KH * a.KW <= 32)
         for (int i = 0; i < a.KH; ++i) a.row_unit |= 1u << (i * a.KW);
+    if (tile_oc <= 32) {
+        if (out_int32) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the %dx%d tile has 8-bit results only", tile_oc, tile_px);
+        return launch_conv_split(a, tile_oc, tile_px, waves, x_unsigned, rne, s);
+    }
     if (waves == 8) {
         // eight wavefronts: the pixels of the tile are split four ways
         if (tile_oc == 128 && tile_px == 128) return a.bk == 128 ? launch_conv_mfma_2_1_128_4(a, x_unsigned, out_int32, rne, max_wgs_per_cu, s)

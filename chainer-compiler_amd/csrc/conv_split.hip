@@ -1,0 +1,300 @@
+// The packed-weight convolution for launches with few output tiles: small tiles whose K is shared out over the
+// wavefronts of a work-group.
+//
+// With one image (or a few) the tiles of conv_mfma_kernel occupy a fraction of the 256 compute units, each walking a K of
+// up to 4608 bytes through LDS stage by stage: 7 to 14 us per layer of ResNet-50 whatever the layer's size.  Here a
+// work-group owns R output channels x R*PN pixels (R = 16 or 32), and its W wavefronts take K apart: fragments come
+// straight from memory (16 bytes per lane: the packed weights and channels-last pixels have them contiguous), several
+// steps in flight, no barrier until the W partial sums meet in LDS.  Weights are read once per pixel tile and pixels once
+// per channel tile, from L2, so this is for launches bound by latency; which configuration runs is measured per shape
+// (tune_conv_mfma).  ResNet-50 on one image, all 55 launches replayed: 370 us with the staged tiles alone, 308 with these.
+//
+// Arguments, requantization, residual sums, pairs and storage are those of conv_mfma_kernel; filter taps outside the
+// image are replaced by the zero point on the fragment.
+#include <type_traits>
+
+#include "conv_mfma.h"
+#include "conv_device.h"
+
+namespace chx {
+namespace {
+
+// Four codes of the convolution and four of the residual -> four codes of the sum (affine_residual16).
+__device__ __forceinline__ uint32_t affine_residual4(uint32_t c, uint32_t r, const ResidualAdd& p) {
+    const uint32_t cw = c ^ p.c_flip, rw = r ^ p.r_flip;
+    float t[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        t[e] = __builtin_fmaf((float)((rw >> (8 * e)) & 0xffu), p.kr, p.k0);
+        t[e] = __builtin_fmaf((float)((cw >> (8 * e)) & 0xffu), p.kc, t[e]);
+        if (p.affine == 2) t[e] = __builtin_fmaxf(t[e], p.floor_pre);
+    }
+    return floor_sat_u8x4(t[0], t[1], t[2], t[3]);
+}
+
+template <int R, int PN, int W, bool kPad>
+__global__ __launch_bounds__(64 * W) void conv_split_kernel(ConvMfmaArgs a, uint32_t x_flip, int rne, int tiles_per_xcd) {
+    constexpr int kGroups = 64 / R, kStep = 16 * kGroups;  // K bytes per MFMA: 32 or 64
+    constexpr int kQuads = R * R / 256;                    // groups of four result registers: 4 or 1
+    constexpr int kUnits = PN * kQuads;
+    constexpr int kDepth = 4;                              // steps in flight
+    using acc_t = typename std::conditional<R == 32, v16i, v4i>::type;
+    __shared__ __attribute__((aligned(16))) v4i part[W > 1 ? W : 1][W > 1 ? kUnits : 1][64];
+
+    warm_kernel_arguments<sizeof(ConvMfmaArgs)>();
+    const int idx = (int)(blockIdx.x >> 3), tile = (int)(blockIdx.x & 7) * tiles_per_xcd + idx;
+    if (idx >= tiles_per_xcd || tile >= a.tiles_oc * a.tiles_px) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane % R, group = lane / R;
+    // an XCD's run of tiles: all pixels of a few channel tiles, so that their weights are fetched into one L2
+    const int oc_tile = tile / a.tiles_px, px_tile = tile - oc_tile * a.tiles_px;
+    const int oc0 = oc_tile * R, oc = oc0 + col;
+
+    // Every kernel of a network starts with cold caches (what the previous one wrote has to become visible to all XCDs),
+    // so a round trip to memory costs more than a microsecond here and the kernel is a chain of them.  The weights of the
+    // first steps are requested before the pixels' addresses are known, and the operands of the epilogue before the loop.
+    struct Step {
+        v4i w, x[PN];
+    };
+    const int steps = a.KP / kStep, per = (steps + W - 1) / W, lo = wave * per, hi = min(steps, lo + per), last = hi - 1;
+    const uint32_t w_off = (uint32_t)(oc >> 6) * (uint32_t)(64 * a.KP) + (uint32_t)((oc & 63) * a.bk + group * 16);
+    const uint32_t bk_shift = a.bk == 128 ? 7 : 6;
+    auto load_w = [&](int step, Step& s) {
+        // (past the wavefront's last step: that step again, see gemm_i8.hip)
+        const uint32_t k = (uint32_t)(min(step, last) * kStep);
+        s.w = *reinterpret_cast<const v4i*>(a.wp + (((k >> bk_shift) * 64u) << bk_shift) + (k & (uint32_t)(a.bk - 1)) + w_off);
+    };
+    Step ring[kDepth];
+    if (lo < hi) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) load_w(lo + d, ring[d]);
+    }
+    int32_t x_off[PN];
+    uint32_t taps[PN];  // inside the image
+#pragma unroll
+    for (int j = 0; j < PN; ++j) {
+        const int64_t m64 = (int64_t)(px_tile * PN + j) * R + col;
+        const uint32_t m = (uint32_t)(m64 < a.M ? m64 : a.M - 1);  // (pixels past the end are not stored)
+        if (a.px_linear) {
+            x_off[j] = (int32_t)(m * (uint32_t)a.x_w_stride);
+        } else {
+            const uint32_t r = fast_div(m, a.ow_mul, a.ow_shift), ow = m - r * (uint32_t)a.OW;
+            const uint32_t n = fast_div(r, a.oh_mul, a.oh_shift), oh = r - n * (uint32_t)a.OH;
+            const int ih0 = (int)oh * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
+            x_off[j] = (int32_t)n * (int32_t)a.x_n_stride + ih0 * (int32_t)a.x_h_stride + iw0 * (int32_t)a.x_w_stride;
+            if (kPad) {
+                const int c_lo = min(max(-iw0, 0), a.KW), c_hi = min(max(a.W - iw0, 0), a.KW);
+                const int r_lo = min(max(-ih0, 0), a.KH), r_hi = min(max(a.H - ih0, 0), a.KH);
+                // the column bits repeated in every filter row, the rows outside the image cut off
+                const uint32_t cols = c_hi > c_lo ? (uint32_t)(((uint64_t)1 << c_hi) - ((uint64_t)1 << c_lo)) : 0u;
+                const uint32_t rows = r_hi > r_lo ? (uint32_t)(((uint64_t)1 << (r_hi * a.KW)) - ((uint64_t)1 << (r_lo * a.KW))) : 0u;
+                taps[j] = (cols * a.row_unit) & rows;
+            }
+        }
+        x_off[j] += group * 16;
+    }
+    const int fill = (int)((uint32_t)(a.x_zp & 0xff) * 0x01010101u);
+
+    // the step whose pixels are loaded next: its place in its filter tap, the tap, and the offset into x
+    int k_in, tap, kw, at = lo;
+    uint32_t x_at;
+    {
+        const int k = lo * kStep;
+        tap = k / a.C64;
+        k_in = k - tap * a.C64;
+        kw = tap % a.KW;
+        x_at = (uint32_t)((tap / a.KW) * (int)a.x_h_stride + kw * (int)a.x_w_stride + k_in);
+    }
+    auto load_x = [&](Step& s) {
+        // channels past C16 have zero weights, and a tap outside the image becomes the zero point: both read anything inside x
+        const bool channels = k_in + group * 16 < a.C16;
+#pragma unroll
+        for (int j = 0; j < PN; ++j) {
+            const bool inside = channels && (!kPad || ((taps[j] >> tap) & 1));
+            const uint32_t off = inside ? (uint32_t)x_off[j] + x_at : 0u;
+            s.x[j] = *reinterpret_cast<const v4i*>(a.x + off);
+            if (kPad) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s.x[j][e] = inside ? s.x[j][e] : fill;
+            }
+        }
+        if (at < last) {
+            ++at;
+            k_in += kStep;
+            x_at += kStep;
+            if (k_in == a.C64) {
+                x_at -= (uint32_t)a.C64;
+                k_in = 0;
+                ++tap;
+                ++kw;
+                const bool row = kw == a.KW;
+                kw = row ? 0 : kw;
+                x_at += row ? (uint32_t)a.x_h_stride - (uint32_t)((a.KW - 1) * (int)a.x_w_stride) : (uint32_t)a.x_w_stride;
+            }
+        }
+    };
+    if (lo < hi) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) load_x(ring[d]);
+    }
+    // unit u of the result: four channels of one pixel per lane (u / kQuads: block of R pixels, u % kQuads: of 8 channels);
+    // this wavefront finishes units wave, wave + W, ...
+    constexpr int kMine = (kUnits + W - 1) / W;
+    struct Finish {
+        int64_t m;
+        int c0;
+        int32_t add[4];    // what the zero point and an int32 bias add to the sum
+        float scale[4], fbias[4];
+        uint32_t r;        // residual codes
+    };
+    const int OC = a.oc_split > 0 && oc0 < a.oc_split ? a.oc_split : a.OC;
+    auto prefetch = [&](int u, Finish& f) {
+        const int j = u / kQuads, q = u % kQuads;
+        f.m = (int64_t)(px_tile * PN + j) * R + col;
+        f.c0 = oc0 + q * 8 + group * 4;
+        const bool mine = f.m < a.M && f.c0 < OC;
+        f.r = 0;
+        if (a.res.r && mine) {
+            const char* src = a.res.r + f.m * a.res.r_px_stride + f.c0;
+            if (a.res.r_vec_ok && f.c0 + 4 <= OC) f.r = *reinterpret_cast<const uint32_t*>(src);
+            else
+                for (int e = 0; e < 4; ++e)
+                    if (f.c0 + e < OC) f.r |= (uint32_t)(uint8_t)src[e] << (8 * e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int ch = min(f.c0 + e, a.OC - 1);
+            f.add[e] = a.wsum[ch];
+            f.scale[e] = a.w_scale_len > 1 ? a.w_scale[ch] : a.w_scale[0];
+            f.fbias[e] = a.bias ? __builtin_bit_cast(float, a.bias[ch]) : 0.f;
+        }
+    };
+    Finish mine[kMine];
+#pragma unroll
+    for (int i = 0; i < kMine; ++i)
+        if (wave + i * W < kUnits) prefetch(wave + i * W, mine[i]);
+
+    acc_t acc[PN];
+#pragma unroll
+    for (int j = 0; j < PN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4 * kQuads; ++r) acc[j][r] = 0;
+    auto multiply = [&](const Step& s) {
+#pragma unroll
+        for (int j = 0; j < PN; ++j) {
+            v4i fx = s.x[j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fx[e] ^= (int)x_flip;
+            if constexpr (R == 32) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(s.w, fx, acc[j], 0, 0, 0);
+            else acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(s.w, fx, acc[j], 0, 0, 0);
+        }
+    };
+    if (lo < hi) {
+        int step = lo;
+        for (; step + kDepth < hi; step += kDepth) {
+#pragma unroll
+            for (int d = 0; d < kDepth; ++d) {
+                multiply(ring[d]);
+                load_w(step + d + kDepth, ring[d]);
+                load_x(ring[d]);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d)
+            if (step + d < hi) multiply(ring[d]);
+    }
+
+    // ---- the sums, requantized ----
+    if (a.oc_split > 0 && oc0 >= a.oc_split) {
+        a.y = a.y2 - a.oc_split;
+        a.y_px_stride = a.y2_px_stride;
+        a.y_vec_ok = a.y2_vec_ok;
+        a.y_flip = a.y2_flip;
+        a.rq.q = a.q2;
+        a.inv_y_scale = a.inv_y_scale2;
+        a.lo_folded = a.lo_folded2;
+    }
+    auto finish = [&](const Finish& f, v4i sum) {
+        if (f.m >= a.M || f.c0 >= OC) return;
+        int32_t code[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int32_t bias = __builtin_bit_cast(int32_t, f.fbias[e]);
+            int32_t v = sum[e] + a.corr_mult * f.add[e];
+            if (a.rq.bias_mode == kBiasOnnxInt32) v += bias;
+            float x = (float)v * (a.rq.x_scale * f.scale[e]);
+            if (a.rq.bias_mode == kBiasReferenceFloat) x = x + (float)bias;
+            code[e] = rne ? quantize_value_folded<true>(x, a.rq.q, a.inv_y_scale, a.lo_folded) : quantize_value_folded<false>(x, a.rq.q, a.inv_y_scale, a.lo_folded);
+        }
+        uint32_t word = pack4(code[0], code[1], code[2], code[3]);
+        if (a.res.r) {
+            if (a.res.affine) word = affine_residual4(word, f.r, a.res);
+            else word = (uint32_t)add_residual16_any(v4i{(int)word, 0, 0, 0}, v4i{(int)f.r, 0, 0, 0}, a.res)[0];
+        }
+        word ^= a.y_flip;
+        char* dst = a.y + f.m * a.y_px_stride + f.c0;
+        if (a.y_vec_ok && f.c0 + 4 <= OC) *reinterpret_cast<uint32_t*>(dst) = word;
+        else
+            for (int e = 0; e < 4; ++e)
+                if (f.c0 + e < OC) dst[e] = (char)(word >> (8 * e));
+    };
+    if constexpr (W > 1) {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            const int j = u / kQuads, q = u % kQuads;
+            part[wave][u][lane] = v4i{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+        const int u = wave + i * W;
+        if (u >= kUnits) break;
+        v4i sum;
+        if constexpr (W > 1) {
+            sum = part[0][u][lane];
+#pragma unroll
+            for (int w = 1; w < W; ++w) sum += part[w][u][lane];
+        } else {
+            const int j = i / kQuads, q = i % kQuads;
+            sum = v4i{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+        }
+        finish(mine[i], sum);
+    }
+}
+
+template <int R, int PN, int W>
+int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, bool pad, hipStream_t s) {
+    const int64_t tiles = (int64_t)a.tiles_oc * a.tiles_px;
+    const int per_xcd = (int)((tiles + 7) / 8);
+    if (pad) conv_split_kernel<R, PN, W, true><<<8 * per_xcd, 64 * W, 0, s>>>(a, flip, rne ? 1 : 0, per_xcd);
+    else conv_split_kernel<R, PN, W, false><<<8 * per_xcd, 64 * W, 0, s>>>(a, flip, rne ? 1 : 0, per_xcd);
+    return launch_check("conv_split_kernel");
+}
+
+}  // namespace
+
+bool conv_split_has(int tile_oc, int tile_px, int waves) {
+    for (const ConvSplitTile& t : kConvSplitTiles)
+        if (t.oc == tile_oc && t.px == tile_px && t.waves == waves) return true;
+    return false;
+}
+
+int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s) {
+    const bool pad = a.ph != 0 || a.pw != 0 || (int64_t)(a.OH - 1) * a.sh + a.KH > a.H || (int64_t)(a.OW - 1) * a.sw + a.KW > a.W;
+    const uint32_t flip = x_unsigned ? 0x80808080u : 0u;
+#define CHX_SPLIT(R, PN, W) \
+    if (tile_oc == R && tile_px == R * PN && waves == W) return launch<R, PN, W>(a, flip, rne, pad, s);
+    CHX_SPLIT(16, 2, 4)
+    CHX_SPLIT(16, 2, 8)
+    CHX_SPLIT(16, 2, 16)
+    CHX_SPLIT(32, 1, 2)
+    CHX_SPLIT(32, 1, 4)
+    CHX_SPLIT(32, 1, 8)
+    CHX_SPLIT(32, 2, 4)
+    CHX_SPLIT(32, 2, 8)
+#undef CHX_SPLIT
+    CHX_FAIL(CHX_HIP_EINVAL, "conv_split: no kernel for a %dx%d tile with %d wavefronts", tile_oc, tile_px, waves);
+}
+
+}  // namespace chx
