@@ -157,9 +157,10 @@ __global__ __launch_bounds__(256) void planes_channels_last_kernel(PlanarArgs a)
     }
 }
 
-// Tile of R filters x 4R pixels per work-group; W wavefronts share K out (see gemm_i8_split_kernel).
+// Tile of R filters x 4R pixels per work-group; W wavefronts share K out (see gemm_i8_split_kernel; for the launch
+// bounds conv_stem_kernel).
 template <int R, int W>
-__global__ __launch_bounds__(64 * W) void conv_planar_kernel(PlanarArgs g) {
+__global__ __launch_bounds__(64 * W, 2) void conv_planar_kernel(PlanarArgs g) {
     constexpr int kGroups = 64 / R, kStep = 16 * kGroups, kRegs = R * R / 64, kDepth = 2;
     using acc_t = typename std::conditional<R == 32, v16i, v4i>::type;
     // the offsets of K (rounded up to a step), later the partial sums [W][kRegs][64]; large sums as a static array, the

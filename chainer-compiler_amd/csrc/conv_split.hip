@@ -32,8 +32,9 @@ __device__ __forceinline__ uint32_t affine_residual4(uint32_t c, uint32_t r, con
     return floor_sat_u8x4(t[0], t[1], t[2], t[3]);
 }
 
+// (two wavefronts per SIMD promised, so that the sums stay out of the accumulation registers: see conv_stem_kernel)
 template <int R, int PN, int W, bool kPad>
-__global__ __launch_bounds__(64 * W) void conv_split_kernel(ConvMfmaArgs a, uint32_t x_flip, int rne, int tiles_per_xcd) {
+__global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, uint32_t x_flip, int rne, int tiles_per_xcd) {
     constexpr int kGroups = 64 / R, kStep = 16 * kGroups;  // K bytes per MFMA: 32 or 64
     constexpr int kQuads = R * R / 256;                    // groups of four result registers: 4 or 1
     constexpr int kUnits = PN * kQuads;

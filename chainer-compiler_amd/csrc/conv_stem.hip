@@ -74,8 +74,11 @@ __device__ __forceinline__ int small_div(int n, uint32_t m) {
     return (int)(((uint32_t)n * m) >> 20);
 }
 
+// (Two wavefronts per SIMD promised: the compiler then keeps the sums in the ordinary registers.  In the accumulation
+// registers every sum costs a move of its own before it can be requantized, and fewer work-groups fit: 3 -> 32 channels of
+// 128 images of 224 x 224 took 54 us, this way 43; 3 -> 64 with 7x7 filters, 64 images, 37 and 32.)
 template <int KWP, bool kRne>
-__global__ __launch_bounds__(256) void conv_stem_kernel(ConvStemArgs a) {
+__global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
     constexpr int GPL = 16 / KWP;  // groups per lane and K block
     extern __shared__ __attribute__((aligned(16))) char lds[];
     // LDS: weights [KB][2][64][16] | staging [4 waves][32 px][64 oc] | constants | patch

@@ -85,8 +85,9 @@ __device__ __forceinline__ int tile_of_block(const GemmI8Args& g) {
 // latency (a step costs about a microsecond when nothing hides it, so K is split and the loads run ahead) and, with many
 // tiles, by the vector instructions of the transposition.  One thread per result, K serial, took 160 us for
 // 197 x 770 x 1001; this 6.0.  1024 x 1024 x 4096: 14 us, against 22 us of packing and 18 us on the convolution kernel.
+// (Launch bounds: see conv_stem_kernel.)
 template <int R, int W, bool kBT, bool kNarrow>
-__global__ __launch_bounds__(64 * W) void gemm_i8_split_kernel(GemmI8Args g) {
+__global__ __launch_bounds__(64 * W, 2) void gemm_i8_split_kernel(GemmI8Args g) {
     constexpr int kGroups = 64 / R;         // groups of 16 k in a step
     constexpr int kStep = 16 * kGroups;     // 32 or 64
     constexpr int kRegs = R * R / 64;       // result registers of an MFMA
