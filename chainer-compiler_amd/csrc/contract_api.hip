@@ -258,7 +258,8 @@ void pick_tile(const LaunchOptions& opt, const ConvMfmaArgs& a, bool out_int32, 
         const int toc = opt.tile_oc, tpx = opt.tile_px, wv = opt.waves;
         const bool four = wv == 4 && (toc == 64 || toc == 128) && (tpx == 64 || tpx == 128);
         const bool eight = wv == 8 && ((toc == 128 && tpx == 128) || (a.bk == 128 && ((toc == 128 && tpx == 256) || (toc == 64 && tpx == 128))));
-        if (four || eight || (conv_split_has(toc, tpx, wv) && conv_split_takes(a) && !out_int32)) {
+        if (four || eight || (conv_split_has(toc, tpx, wv) && conv_split_takes(a) && !out_int32) ||
+            (toc == kConvPointTile.oc && tpx == kConvPointTile.px && wv == kConvPointTile.waves && conv_point_takes(a) && !out_int32)) {
             *tile_oc = toc;
             *tile_px = tpx;
             *max_wgs_per_cu = opt.max_wgs_per_cu;
@@ -355,6 +356,9 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
     // read their operands from L2 once per tile
     if (!out_int32 && conv_split_takes(a) && (int64_t)((a.OC + 63) / 64) * ((a.M + 63) / 64) <= 2048)
         for (const ConvSplitTile& t : kConvSplitTiles) all.push_back({{t.oc, t.px, 0, t.waves}, 0.f});
+
+    if (!out_int32 && conv_point_takes(a))
+        for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, 0.f});
 
     hipEvent_t e0, e1;
     CHX_HIP_CALL(hipEventCreate(&e0));

@@ -186,6 +186,19 @@ bool conv_split_has(int tile_oc, int tile_px, int waves);
 inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
 int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s);
 
+// 1x1, stride 1, no padding over a dense image: input pixel m is at x + m * x_w_stride
+inline bool conv_px_linear(const ConvMfmaArgs& a) {
+    return a.KH == 1 && a.KW == 1 && a.sh == 1 && a.sw == 1 && a.ph == 0 && a.pw == 0 && a.OH == a.H && a.OW == a.W &&
+                  a.x_h_stride == (int64_t)a.W * a.x_w_stride && a.x_n_stride == (int64_t)a.H * a.x_h_stride;
+}
+
+// The kernel for 1x1 filters over few channels and many pixels (conv_point.hip): 64 channels x 32 pixels per wavefront and
+// step.  K is held in registers, which 256 bytes fit; with fewer pixels than give every compute unit a wavefront the
+// weights' way into LDS is most of its time.
+constexpr ConvSplitTile kConvPointTile = {64, 32, 4};
+inline bool conv_point_takes(const ConvMfmaArgs& a) { return conv_px_linear(a) && a.KP <= 256 && a.M >= 32 * 256; }
+int launch_conv_point(const ConvMfmaArgs& a, int max_wgs_per_cu, bool x_unsigned, bool rne, hipStream_t s);
+
 // [N][C][HW] bytes -> [N][HW][pitch] bytes (lanes c >= C of a pixel are zero filled) and back
 int launch_nchw_to_nhwc_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);
 int launch_nhwc_to_nchw_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);

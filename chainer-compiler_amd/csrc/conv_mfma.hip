@@ -382,11 +382,14 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     a.tap_step_row = (uint32_t)(a.x_h_stride - (int64_t)(a.KW - 1) * a.x_w_stride - (a.C64 - a.bk));
     magic_divisor((uint32_t)a.OW, &a.ow_mul, &a.ow_shift);
     magic_divisor((uint32_t)a.OH, &a.oh_mul, &a.oh_shift);
-    a.px_linear = a.KH == 1 && a.KW == 1 && a.sh == 1 && a.sw == 1 && a.ph == 0 && a.pw == 0 && a.OH == a.H && a.OW == a.W &&
-                  a.x_h_stride == (int64_t)a.W * a.x_w_stride && a.x_n_stride == (int64_t)a.H * a.x_h_stride;
+    a.px_linear = conv_px_linear(a) ? 1 : 0;
     a.row_unit = 0;
     if (a.KH * a.KW <= 32)
         for (int i = 0; i < a.KH; ++i) a.row_unit |= 1u << (i * a.KW);
+    if (tile_oc == kConvPointTile.oc && tile_px == kConvPointTile.px && waves == kConvPointTile.waves) {
+        if (out_int32 || !conv_point_takes(a)) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the pixel-streaming kernel does not take this convolution");
+        return launch_conv_point(a, max_wgs_per_cu, x_unsigned, rne, s);
+    }
     if (tile_oc <= 32) {
         if (out_int32) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the %dx%d tile has 8-bit results only", tile_oc, tile_px);
         return launch_conv_split(a, tile_oc, tile_px, waves, x_unsigned, rne, s);
