@@ -643,6 +643,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         sa.rq = c.rq;
         sa.inv_y_scale = 1.0f / c.rq.q.scale;
         sa.lo_folded = fold_relu_floor(c.rq.q, c.rq.relu_floor, c.rne);
+        sa.qp = product_form(c.rq.q, sa.lo_folded, c.rne);
         int rc = launch_conv_stem(sa, c.rne, s);
         if (rc == CHX_HIP_OK && y_post) {
             rc = launch_nhwc_to_nchw_u8(static_cast<const char*>(y_scratch), static_cast<char*>(y.data), cs.N, cs.OC,
@@ -686,6 +687,14 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     a.rq = c.rq;
     a.inv_y_scale = c.out_int32 ? 0.f : 1.0f / c.rq.q.scale;
     a.lo_folded = fold_relu_floor(c.rq.q, c.rq.relu_floor, c.rne);
+    if (!c.out_int32) a.qp = product_form(c.rq.q, a.lo_folded, c.rne);
+    if (a.oc_split > 0) {
+        a.qp2 = product_form(c.rq2.q, a.lo_folded2, c.rne);
+        if ((a.qp.path == 3) != (a.qp2.path == 3)) {  // one form for both
+            a.qp = product_form(c.rq.q, a.lo_folded, c.rne, false);
+            a.qp2 = product_form(c.rq2.q, a.lo_folded2, c.rne, false);
+        }
+    }
     if (c.res) a.res = *c.res;
     CHX_REQUIRE(a.M < (int64_t(1) << 31), "QLinearConv: too many output pixels for the MFMA kernel");
     int toc = 64, tpx = 64, cap = 0, waves = 4;
@@ -942,6 +951,7 @@ int run_depthwise(const ConvCall& c, const DepthwiseState& st, hipStream_t s) {
     a.q = c.rq.q;
     a.inv_y_scale = 1.0f / c.rq.q.scale;
     a.lo_folded = fold_relu_floor(c.rq.q, c.rq.relu_floor, c.rne);
+    a.qp = product_form(c.rq.q, a.lo_folded, c.rne);
     a.y_flip = c.y_minus_128 ? 0x80808080u : 0u;  // (c.y is then the uint8 view of the caller's int8 array)
     return launch_depthwise3x3(a, c.rne, s);
 }

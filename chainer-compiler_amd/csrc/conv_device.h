@@ -79,22 +79,23 @@ template <int BYTES>
 __device__ __forceinline__ void warm_kernel_arguments() {
     const uint64_t ka = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
     constexpr int LINES = (BYTES + 63) / 64;
-    static_assert(LINES >= 4 && LINES <= 8, "between four and eight lines are touched");
+    static_assert(LINES >= 4 && LINES <= 9, "between four and nine lines are touched");
     // offsets of the last lines, clamped into the block so that nothing outside it is read
-    constexpr int L4 = LINES > 4 ? 0x100 : 0xc0, L5 = LINES > 5 ? 0x140 : L4, L6 = LINES > 6 ? 0x180 : L5, L7 = LINES > 7 ? 0x1c0 : L6;
-    int t0, t1, t2, t3, t4, t5, t6, t7;
+    constexpr int L4 = LINES > 4 ? 0x100 : 0xc0, L5 = LINES > 5 ? 0x140 : L4, L6 = LINES > 6 ? 0x180 : L5, L7 = LINES > 7 ? 0x1c0 : L6, L8 = LINES > 8 ? 0x200 : L7;
+    int t0, t1, t2, t3, t4, t5, t6, t7, t8;
     asm volatile(
-            "s_load_dword %0, %8, 0x0\n\t"
-            "s_load_dword %1, %8, 0x40\n\t"
-            "s_load_dword %2, %8, 0x80\n\t"
-            "s_load_dword %3, %8, 0xc0\n\t"
-            "s_load_dword %4, %8, %9\n\t"
-            "s_load_dword %5, %8, %10\n\t"
-            "s_load_dword %6, %8, %11\n\t"
-            "s_load_dword %7, %8, %12\n\t"
+            "s_load_dword %0, %9, 0x0\n\t"
+            "s_load_dword %1, %9, 0x40\n\t"
+            "s_load_dword %2, %9, 0x80\n\t"
+            "s_load_dword %3, %9, 0xc0\n\t"
+            "s_load_dword %4, %9, %10\n\t"
+            "s_load_dword %5, %9, %11\n\t"
+            "s_load_dword %6, %9, %12\n\t"
+            "s_load_dword %7, %9, %13\n\t"
+            "s_load_dword %8, %9, %14\n\t"
             "s_waitcnt lgkmcnt(0)"
-            : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7)
-            : "s"(ka), "n"(L4), "n"(L5), "n"(L6), "n"(L7)
+            : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8)
+            : "s"(ka), "n"(L4), "n"(L5), "n"(L6), "n"(L7), "n"(L8)
             : "memory");
 }
 

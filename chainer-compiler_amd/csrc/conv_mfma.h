@@ -78,6 +78,7 @@ struct ConvMfmaArgs {
     RequantParams rq;
     float inv_y_scale;           // 1 / y_scale, for the division-free requantization
     float lo_folded;             // lower clamp bound with the fused Relu folded in (fold_relu_floor)
+    QuantProduct qp;             // the same requantization as a product, where it is one
     int32_t tiles_oc, tiles_px;  // filled by the launcher
     uint32_t ow_mul, ow_shift, oh_mul, oh_shift;  // magic_divisor(OW), magic_divisor(OH), filled by the launcher
     uint32_t row_unit;           // bit i*KW set for every filter row i (when KH*KW <= 32), filled by the launcher
@@ -99,6 +100,7 @@ struct ConvMfmaArgs {
     QuantParams q2;
     float inv_y_scale2;
     float lo_folded2;
+    QuantProduct qp2;
 };
 
 // Direct convolution over planar activations with few channels (conv_stem.hip).
@@ -122,6 +124,7 @@ struct ConvStemArgs {
     RequantParams rq;
     float inv_y_scale;
     float lo_folded;
+    QuantProduct qp;
     // filled by the launcher
     int32_t KB, tiles_h, tiles_w, tiles;
     uint32_t m_ppw, m_ph, m_kh;

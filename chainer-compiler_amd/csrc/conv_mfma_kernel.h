@@ -486,6 +486,7 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
                 a.rq.q = a.q2;
                 a.inv_y_scale = a.inv_y_scale2;
                 a.lo_folded = a.lo_folded2;
+                a.qp = a.qp2;
             } else {
                 a.OC = a.oc_split;
             }
@@ -518,19 +519,17 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
             return;
         }
         // requantize: one instance of the element loop per bias mode and per conversion path (the
-        // branches are uniform).  kPath 0: any 8-bit type and rounding; 1: uint8 in the reference's
-        // rounding through floor_sat_u8x16; 2: the same with a lower bound above 0 (a folded Relu);
-        // 3: as 1 with a zero point of 0.
+        // branches are uniform).  kPath: QuantProduct::path.
         // the constants of the per-element arithmetic in vector registers (in_vector_register says why)
-        const QuantParams rq_q = in_vector_registers(a.rq.q);
-        const float inv_y_scale = in_vector_register(a.inv_y_scale);
-        const float lo_folded = in_vector_register(a.lo_folded);
         auto requantize_tile = [&](auto float_bias_tag, auto path_tag) {
             constexpr bool kFloatBias = decltype(float_bias_tag)::value;
             constexpr int kPath = decltype(path_tag)::value;
             // a block of 32 output channels that lies beyond OC altogether (OC = 96 in a 128-wide tile, say) is not
             // requantized: nobody reads its staged bytes (the test is the same for the whole wavefront)
             if constexpr (kPath == 0) {
+                const QuantParams rq_q = in_vector_registers(a.rq.q);
+                const float inv_y_scale = in_vector_register(a.inv_y_scale);
+                const float lo_folded = in_vector_register(a.lo_folded);
 #pragma unroll
                 for (int i = 0; i < FM; ++i) {
                     if (oc0 + wm * 32 * FM + i * 32 >= a.OC) continue;
@@ -557,6 +556,7 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
             } else {
                 // sixteen values (4 / FN row groups of the accumulator) per switch of the rounding mode
                 constexpr int G = 4 / FN;
+                const QuantProduct qp = in_vector_registers(a.qp);
 #pragma unroll
                 for (int i = 0; i < FM; ++i) {
                     if (oc0 + wm * 32 * FM + i * 32 >= a.OC) continue;
@@ -576,8 +576,7 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
                                 for (int e = 0; e < 4; ++e) {
                                     float v = (float)acc[i][j][g * 4 + e] * sc[e];
                                     if (kFloatBias) v = v + fb[e];
-                                    pre[(gl * FN + j) * 4 + e] =
-                                            quantize_prefloor_u8<kPath == 2, kPath != 3>(v, rq_q, inv_y_scale, lo_folded);
+                                    pre[(gl * FN + j) * 4 + e] = quantize_prefloor_u8<kPath>(v, qp);
                                 }
                         }
                         uint32_t word[4];
@@ -624,15 +623,14 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
             using P1 = std::integral_constant<int, 1>;
             using P2 = std::integral_constant<int, 2>;
             using P3 = std::integral_constant<int, 3>;
-            const bool u8_reference = !kRne && a.rq.q.lo == 0.f && a.rq.q.hi == 255.f;
             const bool float_bias = a.rq.bias_mode == kBiasReferenceFloat;
-            if (!u8_reference) {
+            if (kRne || a.qp.path == 0) {
                 if (float_bias) requantize_tile(std::true_type(), P0());
                 else requantize_tile(std::false_type(), P0());
-            } else if (a.lo_folded > 0.f) {
+            } else if (a.qp.path == 2) {
                 if (float_bias) requantize_tile(std::true_type(), P2());
                 else requantize_tile(std::false_type(), P2());
-            } else if (a.rq.q.zpf == 0.f) {
+            } else if (a.qp.path == 3) {
                 if (float_bias) requantize_tile(std::true_type(), P3());
                 else requantize_tile(std::false_type(), P3());
             } else {

@@ -56,8 +56,7 @@ __device__ __forceinline__ v4i load_part(const char* src, int n) {
     return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
-// kPath 0: any 8-bit type and rounding; 1: uint8 in the reference's rounding; 3: the same with a zero point of 0 and no
-// lower bound above 0 (quantize_prefloor_u8).
+// kPath: QuantProduct::path (2 also for a pair of which one is 1; both are 3 or none)
 template <int KS, int kPath, bool kFloatBias, bool kRes>
 __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs a, uint32_t x_flip_s, int rne, int chunks, int chunk_tiles) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -122,6 +121,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
             int64_t y_pitch = a.y_px_stride;
             QuantParams q = a.rq.q;
             float inv = a.inv_y_scale, lo = a.lo_folded;
+            QuantProduct qp = a.qp;
             uint32_t y_flip = a.y_flip;
             int OC = a.OC;
             if (a.oc_split > 0) {
@@ -131,6 +131,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
                     q = a.q2;
                     inv = a.inv_y_scale2;
                     lo = a.lo_folded2;
+                    qp = a.qp2;
                     y_flip = a.y2_flip;
                 } else {
                     OC = a.oc_split;
@@ -149,9 +150,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
                     else if (m < a.M && valid > 0) res[p] = load_part(src, valid);
                 }
             }
-            const QuantParams qv = in_vector_registers(q);
-            inv = in_vector_register(inv);
-            lo = in_vector_register(lo);
+            if (kPath == 0) {
+                q = in_vector_registers(q);
+                inv = in_vector_register(inv);
+                lo = in_vector_register(lo);
+            } else {
+                qp = in_vector_registers(qp);
+            }
             uint32_t word[2][4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -177,8 +182,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
                     for (int e = 0; e < 4; ++e) {
                         float v = (float)acc[p][e] * sc[e];
                         if (kFloatBias) v = v + fb[e];
-                        if (kPath == 0) code[p * 4 + e] = rne ? quantize_value_folded<true>(v, qv, inv, lo) : quantize_value_folded<false>(v, qv, inv, lo);
-                        else pre[p * 4 + e] = quantize_prefloor_u8<kPath == 1, kPath == 1>(v, qv, inv, lo);
+                        if (kPath == 0) code[p * 4 + e] = rne ? quantize_value_folded<true>(v, q, inv, lo) : quantize_value_folded<false>(v, q, inv, lo);
+                        else pre[p * 4 + e] = quantize_prefloor_u8<kPath>(v, qp);
                     }
                 if (kPath == 0) {
                     word[0][t] = pack4(code[0], code[1], code[2], code[3]);
@@ -226,16 +231,17 @@ int launch(const ConvMfmaArgs& a, int max_wgs_per_cu, uint32_t flip, bool rne, h
 
 template <int KS>
 int launch_steps(const ConvMfmaArgs& a, int max_wgs_per_cu, uint32_t flip, bool rne, hipStream_t s) {
-    auto u8 = [](const QuantParams& q) { return q.lo == 0.f && q.hi == 255.f; };
-    auto plain = [](const QuantParams& q, float lo_folded) { return q.zpf == 0.f && lo_folded <= 0.f; };
-    const bool fast = !rne && u8(a.rq.q) && (a.oc_split == 0 || u8(a.q2));
-    const bool lean = fast && plain(a.rq.q, a.lo_folded) && (a.oc_split == 0 || plain(a.q2, a.lo_folded2));
+    const bool product = a.qp.path != 0 && (a.oc_split == 0 || a.qp2.path != 0);
+    const bool two_fma = a.qp.path == 3;  // (of a pair, both)
+    const bool bound = a.qp.path == 2 || (a.oc_split > 0 && a.qp2.path == 2);
     const bool fb = a.rq.bias_mode == kBiasReferenceFloat, res = a.res.r != nullptr;
 #define CHX_POINT(PATH, FB) \
     return res ? launch<KS, PATH, FB, true>(a, max_wgs_per_cu, flip, rne, s) : launch<KS, PATH, FB, false>(a, max_wgs_per_cu, flip, rne, s)
-    if (!fast) CHX_POINT(0, true);
-    if (lean && fb) CHX_POINT(3, true);
-    if (lean) CHX_POINT(3, false);
+    if (!product) CHX_POINT(0, true);
+    if (two_fma && fb) CHX_POINT(3, true);
+    if (two_fma) CHX_POINT(3, false);
+    if (bound && fb) CHX_POINT(2, true);
+    if (bound) CHX_POINT(2, false);
     if (fb) CHX_POINT(1, true);
     CHX_POINT(1, false);
 #undef CHX_POINT

@@ -252,11 +252,12 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
         }
 
         // requantize into the wave's staging rows
-        // kPath 0: any 8-bit type and rounding; 1: uint8 in the reference's rounding through
-        // floor_sat_u8x4; 2: the same with a lower bound above 0 (a folded Relu)
+        // (kPath: QuantProduct::path)
         auto requantize_tile = [&](auto float_bias_tag, auto path_tag) {
             constexpr bool kFloatBias = decltype(float_bias_tag)::value;
             constexpr int kPath = decltype(path_tag)::value;
+            QuantProduct qp;
+            if (kPath != 0) qp = in_vector_registers(a.qp);
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 if (oc0 + i * 32 >= a.OC) break;
@@ -273,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
                         float v = (float)acc[i][g * 4 + e] * sc[e];
                         if (kFloatBias) v = v + fbs[e];
                         if (kPath == 0) code[e] = quantize_value_folded<kRne>(v, a.rq.q, a.inv_y_scale, a.lo_folded);
-                        else pre[e] = quantize_prefloor_u8<kPath == 2, kPath != 3>(v, a.rq.q, a.inv_y_scale, a.lo_folded);
+                        else pre[e] = quantize_prefloor_u8<kPath>(v, qp);
                     }
                     *reinterpret_cast<uint32_t*>(staged(p, ocl)) =
                             kPath == 0 ? pack4(code[0], code[1], code[2], code[3]) : floor_sat_u8x4(pre[0], pre[1], pre[2], pre[3]);
@@ -284,16 +285,15 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
             using P0 = std::integral_constant<int, 0>;
             using P1 = std::integral_constant<int, 1>;
             using P2 = std::integral_constant<int, 2>;
-            using P3 = std::integral_constant<int, 3>;  // as 1 with a zero point of 0
-            const bool u8_reference = !kRne && a.rq.q.lo == 0.f && a.rq.q.hi == 255.f;
+            using P3 = std::integral_constant<int, 3>;
             const bool float_bias = a.rq.bias_mode == kBiasReferenceFloat;
-            if (!u8_reference) {
+            if (kRne || a.qp.path == 0) {
                 if (float_bias) requantize_tile(std::true_type(), P0());
                 else requantize_tile(std::false_type(), P0());
-            } else if (a.lo_folded > 0.f) {
+            } else if (a.qp.path == 2) {
                 if (float_bias) requantize_tile(std::true_type(), P2());
                 else requantize_tile(std::false_type(), P2());
-            } else if (a.rq.q.zpf == 0.f) {
+            } else if (a.qp.path == 3) {
                 if (float_bias) requantize_tile(std::true_type(), P3());
                 else requantize_tile(std::false_type(), P3());
             } else {

@@ -4,8 +4,102 @@
 #include <mutex>
 
 #include "chx_internal.h"
+#include "quant_math.h"
 
 namespace chx {
+
+// Where the codes of one quantization begin: below[k] is the last float whose code is less than k, the float after it
+// (above(below[k], 1)) the first whose code is k or more.
+struct CodeBounds {
+    float below[256], from[256];
+};
+
+// n floats above v (which is that far from 0)
+static float above(float v, int n) {
+    int32_t bits;
+    memcpy(&bits, &v, 4);
+    bits += bits < 0 ? -n : n;
+    memcpy(&v, &bits, 4);
+    return v;
+}
+
+// The reference's QuantizeLinear in front of the conversion, which takes the floor and saturates.
+static float reference_form(float v, const QuantParams& q) {
+    const float s = v / q.scale, u = s + q.zpf;
+    return u + 0.5f;
+}
+
+static bool find_bounds(const QuantParams& q, CodeBounds* b) {
+    if (!(q.scale > 1e-30f && q.scale < 1e30f)) return false;
+    for (int k = 1; k <= 255; ++k) {
+        const float at = (float)k, v = (float)(((double)k - 0.5 - (double)q.zpf) * (double)q.scale);
+        int lo = -1024, hi = 1024;  // the additions round by at most 2^-16, which is 512 floats at 0.5
+        if (!(reference_form(above(v, lo), q) < at && reference_form(above(v, hi), q) >= at)) return false;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) / 2;
+            (reference_form(above(v, mid), q) < at ? lo : hi) = mid;
+        }
+        b->below[k] = above(v, lo);
+        b->from[k] = above(v, hi);
+    }
+    return true;
+}
+
+static float product_of(float v, const QuantProduct& p) {
+    return p.path == 3 ? std::fma(v, p.inv, std::fma(v, p.inv_low, p.half)) : std::fma(v, p.inv, v * p.inv_low) + p.half;
+}
+
+static bool same_codes(const CodeBounds& b, const QuantProduct& p) {
+    for (int k = 1; k <= 255; ++k)
+        if (!(product_of(b.below[k], p) < (float)k && product_of(b.from[k], p) >= (float)k)) return false;
+    // The inner sum of path 3 moves in steps of 2^-25 and against v where inv_low is negative.  From a quotient of 0.5 up
+    // the product grows by as much from one float to the next; from 0.25 up it does over two; below that no t reaches 1.
+    for (int n = 1; n <= 8; ++n)
+        if (!(product_of(above(b.below[1], -n), p) < 1.f && product_of(above(b.from[1], n), p) >= 1.f)) return false;
+    return true;
+}
+
+// inv moved by `ulps` and half by `half_ulps`
+static QuantProduct product_with(const QuantParams& q, int path, int ulps, int half_ulps) {
+    QuantProduct p = {};
+    p.path = path;
+    p.inv = above(1.0f / q.scale, ulps);
+    p.inv_low = (float)(1.0 / (double)q.scale - (double)p.inv);
+    p.half = above(q.zpf + 0.5f, half_ulps);
+    return p;
+}
+
+QuantProduct product_form(const QuantParams& q, float lo_folded, bool rne, bool two_fma) {
+    if (rne || q.lo != 0.f || q.hi != 255.f) return QuantProduct{};
+    // finding them takes about 25 us: a thread remembers them
+    struct Forms {
+        float scale, zpf;
+        QuantProduct plain, two_fma;  // path 0: there is none
+    };
+    static thread_local Forms seen[256] = {};
+    uint32_t bits;
+    memcpy(&bits, &q.scale, 4);
+    Forms& f = seen[((bits * 2654435761u) >> 24) ^ ((uint32_t)(int)q.zpf & 255u)];
+    if (f.scale != q.scale || f.zpf != q.zpf) {
+        f = Forms{q.scale, q.zpf, {}, {}};
+        CodeBounds b;
+        if (find_bounds(q, &b)) {
+            const QuantProduct p = product_with(q, 1, 0, 0);
+            if (same_codes(b, p)) f.plain = p;
+            // (99 of 100 scales have one in this range, most within a few steps)
+            for (int i = 0; q.zpf == 0.f && i < 129 * 7 && f.two_fma.path == 0; ++i) {
+                const int ring = (i / 7 + 1) / 2;
+                const QuantProduct t = product_with(q, 3, (i / 7) & 1 ? ring : -ring, i % 7 - 3);
+                if (same_codes(b, t)) f.two_fma = t;
+            }
+        }
+    }
+    const bool bound = lo_folded > 0.f;
+    QuantProduct p = two_fma && !bound && f.two_fma.path != 0 ? f.two_fma : f.plain;
+    if (p.path == 1 && bound) p.path = 2;
+    p.floor_half = lo_folded + 0.5f;
+    return p;
+}
 
 static thread_local std::string g_last_error;
 

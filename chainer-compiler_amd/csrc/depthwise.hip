@@ -123,6 +123,8 @@ __global__ __launch_bounds__(kDwThreads) void depthwise3x3_kernel(DepthwiseArgs 
             rp[e] = __builtin_amdgcn_perm(v[2], t, 0x0c000100u | ((4u + e) << 16));                               // [v0.e, v1.e, v2.e, 0]
         }
     };
+    QuantProduct qp;
+    if (kPath != 0) qp = in_vector_registers(a.qp);
     auto finish = [&](int oh, const uint32_t (&r0)[4], const uint32_t (&r1)[4], const uint32_t (&r2)[4]) {
         int32_t code[4];
         float pre[4];
@@ -137,9 +139,7 @@ __global__ __launch_bounds__(kDwThreads) void depthwise3x3_kernel(DepthwiseArgs 
             float v = (float)acc * sc[e];
             if (kFloatBias) v = v + fb[e];
             // uint8 in the reference's rounding: clamp, conversion and packing in floor_sat_u8x4
-            if (kPath == 2) pre[e] = quantize_prefloor_u8<true>(v, a.q, a.inv_y_scale, a.lo_folded);
-            else if (kPath == 1) pre[e] = quantize_prefloor_u8<false>(v, a.q, a.inv_y_scale, 0.f);
-            else if (kPath == 3) pre[e] = quantize_prefloor_u8<false, false>(v, a.q, a.inv_y_scale, 0.f);
+            if (kPath != 0) pre[e] = quantize_prefloor_u8<kPath>(v, qp);
             else code[e] = quantize_value_folded<kRne>(v, a.q, a.inv_y_scale, a.lo_folded);
         }
         const uint32_t o = kPath ? floor_sat_u8x4(pre[0], pre[1], pre[2], pre[3]) : pack4(code[0], code[1], code[2], code[3]);
@@ -234,8 +234,7 @@ int launch_depthwise3x3(DepthwiseArgs a, bool rne, hipStream_t s) {
     a.xcd_chunk = (uint32_t)((all_blocks + 7) / 8);
     const dim3 blocks(a.xcd_chunk * 8u);
     const bool fbias = a.bias != nullptr && a.float_bias != 0;
-    const bool u8_reference = !rne && a.q.lo == 0.f && a.q.hi == 255.f;
-    const int path = !u8_reference ? 0 : a.lo_folded > 0.f ? 2 : a.q.zpf == 0.f ? 3 : 1;
+    const int path = rne ? 0 : a.qp.path;
 #define CHX_DW_P(RN, FB, ST, TL)                                                                    \
     do {                                                                                            \
         if (path == 0) depthwise3x3_kernel<RN, FB, ST, 0, TL><<<blocks, kDwThreads, 0, s>>>(a);     \
