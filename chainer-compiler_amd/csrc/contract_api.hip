@@ -333,13 +333,20 @@ MeasuredConfigurations& measured_configurations() {
     return *m;
 }
 
+constexpr size_t kReadThrough = size_t(64) << 20;  // twice the L2 caches of the device's 8 XCDs
+
 // Times the launch configurations on the call's operands and gives the fastest.
 int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hipStream_t s, Configuration* best) {
     // tile (output channels x pixels), wavefronts; the eight-wavefront kernels take the compute unit alone
     static const int tiles[7][3] = {{128, 128, 4}, {64, 128, 4}, {128, 64, 4}, {64, 64, 4}, {128, 128, 8}, {128, 256, 8}, {64, 128, 8}};
     struct Candidate {
         Configuration c;
-        float ms;
+        std::vector<float> seen;
+        float ms() const {  // the median
+            std::vector<float> v = seen;
+            std::sort(v.begin(), v.end());
+            return v.empty() ? 1e30f : v[v.size() / 2];
+        }
     };
     std::vector<Candidate> all;
     for (const auto& t : tiles) {
@@ -347,49 +354,67 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
         if (a.oc_split % t[0] != 0) continue;  // two outputs: a tile belongs to one of them whole
         if (t[2] == 8 && (t[0] == 64 || t[1] == 256) && a.bk != 128) continue;
         const int64_t tiles_all = (int64_t)((a.OC + t[0] - 1) / t[0]) * ((a.M + t[1] - 1) / t[1]);
-        all.push_back({{t[0], t[1], 0, t[2]}, 0.f});
+        all.push_back({{t[0], t[1], 0, t[2]}, {}});
         // (a cap that the tiles do not reach is the launch without one)
-        if (t[2] == 4 && tiles_all > 512) all.push_back({{t[0], t[1], 2, t[2]}, 0.f});
-        if (t[2] == 4 && tiles_all > 256) all.push_back({{t[0], t[1], 1, t[2]}, 0.f});
+        if (t[2] == 4 && tiles_all > 512) all.push_back({{t[0], t[1], 2, t[2]}, {}});
+        if (t[2] == 4 && tiles_all > 256) all.push_back({{t[0], t[1], 1, t[2]}, {}});
     }
     // launches that the staged tiles fill (in tiles of 64 x 64, eight per compute unit) are not for the small tiles: they
     // read their operands from L2 once per tile
     if (!out_int32 && conv_split_takes(a) && (int64_t)((a.OC + 63) / 64) * ((a.M + 63) / 64) <= 2048)
-        for (const ConvSplitTile& t : kConvSplitTiles) all.push_back({{t.oc, t.px, 0, t.waves}, 0.f});
+        for (const ConvSplitTile& t : kConvSplitTiles)
+            if (t.waves * 512 / t.oc <= a.KP)  // (half a step and more for every wavefront)
+                all.push_back({{t.oc, t.px, 0, t.waves}, {}});
 
     if (!out_int32 && conv_point_takes(a))
-        for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, 0.f});
+        for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, {}});
 
-    hipEvent_t e0, e1;
-    CHX_HIP_CALL(hipEventCreate(&e0));
-    CHX_HIP_CALL(hipEventCreate(&e1));
+    std::vector<hipEvent_t> events(2 * all.size());
+    size_t created = 0;
     int rc = CHX_HIP_OK;
-    auto measure = [&](const Configuration& c, int reps) {
-        float ms = 0.f;
-        rc = launch_conv_mfma(a, c.tile_oc, c.tile_px, c.max_wgs_per_cu, c.waves, xu, out_int32, rne, s);  // warm
-        if (rc != CHX_HIP_OK) return ms;
-        if (hipEventRecord(e0, s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
-        for (int r = 0; r < reps && rc == CHX_HIP_OK; ++r) rc = launch_conv_mfma(a, c.tile_oc, c.tile_px, c.max_wgs_per_cu, c.waves, xu, out_int32, rne, s);
-        if (rc != CHX_HIP_OK) return ms;
-        if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) rc = CHX_HIP_ERUNTIME;
-        return ms / reps;
+    while (created < events.size() && hipEventCreate(&events[created]) == hipSuccess) ++created;
+    if (created < events.size()) rc = CHX_HIP_ERUNTIME;
+    void* other = nullptr;
+    if (rc == CHX_HIP_OK && hipMallocAsync(&other, kReadThrough, s) != hipSuccess) {
+        (void)hipGetLastError();
+        other = nullptr;  // (no memory to spare: the first look's verdict stands)
+    }
+    auto launch = [&](const Configuration& c) {
+        if (rc == CHX_HIP_OK) rc = launch_conv_mfma(a, c.tile_oc, c.tile_px, c.max_wgs_per_cu, c.waves, xu, out_int32, rne, s);
     };
-    // three launches each, then the best five again, in turn: single measurements of launches of a few microseconds differ
-    // by more than the configurations do
-    for (Candidate& c : all)
-        if (rc == CHX_HIP_OK) c.ms = measure(c.c, 3);
-    std::sort(all.begin(), all.end(), [](const Candidate& l, const Candidate& r) { return l.ms < r.ms; });
-    if (all.size() > 5) all.resize(5);
-    for (int round = 0; round < 3; ++round)
-        for (Candidate& c : all)
-            if (rc == CHX_HIP_OK && c.ms <= 1.3f * all[0].ms) {
-                const float ms = measure(c.c, 4);
-                c.ms = round == 0 ? ms : std::min(c.ms, ms);
-            }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    // every candidate once: `times` launches in a row after one that warms up, or one that finds the L2 caches full of
+    // something else; one wait for all of them
+    auto look = [&](int times, bool cold) {
+        for (size_t i = 0; i < all.size() && rc == CHX_HIP_OK; ++i) {
+            if (cold) rc = launch_read_through(other, kReadThrough, s);
+            else launch(all[i].c);
+            if (rc == CHX_HIP_OK && hipEventRecord(events[2 * i], s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+            for (int t = 0; t < times; ++t) launch(all[i].c);
+            if (rc == CHX_HIP_OK && hipEventRecord(events[2 * i + 1], s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+        }
+        if (rc == CHX_HIP_OK && hipStreamSynchronize(s) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+        for (size_t i = 0; i < all.size() && rc == CHX_HIP_OK; ++i) {
+            float ms = 0.f;
+            if (hipEventElapsedTime(&ms, events[2 * i], events[2 * i + 1]) != hipSuccess) rc = CHX_HIP_ERUNTIME;
+            all[i].seen.push_back(ms / times);
+        }
+    };
+    auto faster = [](const Candidate& l, const Candidate& r) { return l.ms() < r.ms(); };
+    // Two launches in a row each, to find the eight worth a closer look.  Those again, one launch at a time with cold
+    // caches: in a network a layer's weights and the previous layer's results come from memory, and a configuration that
+    // reads them in many places loses there what it wins in a loop (512 -> 128 channels of 8 images of 28 x 28: 12 us in the
+    // network with the tile that a loop prefers, 6 with another).
+    look(2, false);
+    std::sort(all.begin(), all.end(), faster);
+    if (all.size() > 8) all.resize(8);
+    if (other) {
+        for (Candidate& c : all) c.seen.clear();
+        for (int round = 0; round < 3; ++round) look(1, true);
+        (void)hipFreeAsync(other, s);
+    }
+    for (size_t i = 0; i < created; ++i) (void)hipEventDestroy(events[i]);
     if (rc != CHX_HIP_OK) CHX_FAIL(rc, "timing the convolution launch configurations failed: %s", chx_hip_last_error());
-    *best = std::min_element(all.begin(), all.end(), [](const Candidate& l, const Candidate& r) { return l.ms < r.ms; })->c;
+    *best = std::min_element(all.begin(), all.end(), faster)->c;
     return CHX_HIP_OK;
 }
 

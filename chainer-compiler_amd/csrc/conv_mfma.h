@@ -184,7 +184,7 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
 struct ConvSplitTile {
     int oc, px, waves;
 };
-constexpr ConvSplitTile kConvSplitTiles[] = {{16, 32, 4}, {16, 32, 8}, {16, 32, 16}, {32, 32, 2}, {32, 32, 4}, {32, 32, 8}, {32, 64, 4}, {32, 64, 8}};
+constexpr ConvSplitTile kConvSplitTiles[] = {{16, 16, 8}, {16, 16, 16}, {16, 32, 4}, {16, 32, 8}, {16, 32, 16}, {32, 32, 2}, {32, 32, 4}, {32, 32, 8}, {32, 64, 4}, {32, 64, 8}};
 bool conv_split_has(int tile_oc, int tile_px, int waves);
 inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
 int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s);
@@ -201,6 +201,9 @@ inline bool conv_px_linear(const ConvMfmaArgs& a) {
 constexpr ConvSplitTile kConvPointTile = {64, 32, 4};
 inline bool conv_point_takes(const ConvMfmaArgs& a) { return conv_px_linear(a) && a.KP <= 256 && a.M >= 32 * 256; }
 int launch_conv_point(const ConvMfmaArgs& a, int max_wgs_per_cu, bool x_unsigned, bool rne, hipStream_t s);
+
+// Reads `bytes` bytes (a multiple of 16): afterwards the L2 caches hold them and little else.
+int launch_read_through(const void* p, size_t bytes, hipStream_t s);
 
 // [N][C][HW] bytes -> [N][HW][pitch] bytes (lanes c >= C of a pixel are zero filled) and back
 int launch_nchw_to_nhwc_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);

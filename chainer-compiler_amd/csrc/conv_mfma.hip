@@ -363,6 +363,20 @@ int find_affine_residual(ResidualAdd* p, int32_t* scratch, hipStream_t s) {
     return CHX_HIP_OK;
 }
 
+__global__ __launch_bounds__(256) void read_through_kernel(const uint4* p, uint32_t n, uint32_t* never) {
+    uint32_t sum = 0;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const uint4 v = p[i];
+        sum ^= v.x ^ v.y ^ v.z ^ v.w;
+    }
+    if (never) *never = sum;  // (never is null: the loads are what it is for)
+}
+
+int launch_read_through(const void* p, size_t bytes, hipStream_t s) {
+    read_through_kernel<<<2048, 256, 0, s>>>(static_cast<const uint4*>(p), (uint32_t)(bytes / 16), nullptr);
+    return launch_check("read_through_kernel");
+}
+
 int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_cu, int waves, bool x_unsigned, bool out_int32, bool rne,
                      hipStream_t s) {
     a.tiles_oc = (a.OC + tile_oc - 1) / tile_oc;

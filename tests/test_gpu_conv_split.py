@@ -8,7 +8,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-TILES = [(16, 32, 4), (16, 32, 8), (16, 32, 16), (32, 32, 2), (32, 32, 4), (32, 32, 8), (32, 64, 4), (32, 64, 8)]
+TILES = [(16, 16, 8), (16, 16, 16), (16, 32, 4), (16, 32, 8), (16, 32, 16), (32, 32, 2), (32, 32, 4), (32, 32, 8), (32, 64, 4), (32, 64, 8)]
 
 
 @pytest.fixture(scope="module")
@@ -42,7 +42,7 @@ def codes(rng, shape, dt):
 
 # N, C, H, W, OC, k, stride, pad: one pixel, ragged channels and pixels, K from one step to many, padding wider than a row
 CASES = [(1, 16, 1, 1, 5, 1, 1, 0), (1, 64, 7, 7, 70, 1, 1, 0), (2, 24, 9, 5, 33, 3, 1, 1), (1, 128, 7, 7, 128, 3, 1, 1), (3, 96, 8, 8, 100, 1, 2, 0),
-         (1, 256, 5, 6, 64, 3, 2, 1), (1, 32, 6, 6, 40, 5, 1, 2), (5, 160, 4, 4, 24, 1, 1, 0)]
+         (1, 256, 5, 6, 64, 3, 2, 1), (1, 32, 6, 6, 40, 5, 1, 2), (5, 160, 4, 4, 24, 1, 1, 0), (1, 320, 5, 5, 48, 3, 1, 1)]
 
 
 @pytest.mark.parametrize("tile", TILES)
