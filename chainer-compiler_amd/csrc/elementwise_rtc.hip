@@ -395,6 +395,25 @@ int float_value(const std::string& tok, float* value) {
     return CHX_HIP_OK;
 }
 
+// tanh for a float16 argument whose result is rounded to float16: an odd rational function of degree 7 over 6 (minimax in
+// the relative error, 2^-25, up to 4.53, beyond which the result rounds to 1).  It is not the C library's float32 tanh, but
+// rounded to float16 it is for every one of the 65536 arguments (a test compares them all).  15 instructions instead of
+// about 60, which bound the float16 chains: two operands of [8, 333, 1001] and two of [1001] through Mul, Add, Tanh, Sigmoid,
+// Mul, Add and Relu 13.4 us, with this and the sigmoid below 7.5 (profiled).  NaN is left to the second evaluation.
+const char* const kTanhOfF16 = R"(
+__device__ __forceinline__ float chx_tanh_of_f16(float x, bool& rare) {
+  rare = rare || x != x;
+  const float v = __builtin_fminf(__builtin_fabsf(x), 0x1.21eb86p+2f), s = v * v;
+  float p = __builtin_fmaf(0x1.6ed3dep-18f, s, 0x1.4ea1ecp-9f);
+  p = __builtin_fmaf(p, s, 0x1.01e116p-3f);
+  p = __builtin_fmaf(p, s, 1.0f);
+  float q = __builtin_fmaf(0x1.6df1f6p-13f, s, 0x1.6d6cb6p-6f);
+  q = __builtin_fmaf(q, s, 0x1.d645cep-2f);
+  q = __builtin_fmaf(q, s, 1.0f);
+  return __builtin_copysignf((v * p) * __builtin_amdgcn_rcpf(q), x);
+}
+)";
+
 // Emits the per-element device function:  elem(in..., &out...).
 // Value kinds: 'f' floating-point value, 'q' 8-bit code held in an int.  A floating-point value is held as TY:
 // float for float32 and for float16 programs (in the latter every node's result goes through R(), the rounding
@@ -480,6 +499,7 @@ int emit_elem(const Program& prog, bool use_fma, std::ostringstream& os, bool* u
             CHX_PROPAGATE(need(1));
             CHX_PROPAGATE(val(0, 'f', &a));
             if (f64) os << decl << o << " = ::tanh(" << a << ");\n";
+            else if (f16) os << decl << o << " = chx_round_f16(kFast ? chx_tanh_of_f16(" << a << ", rare) : chx_fm::tanhf_faithful(" << a << "));\n";
             else os << decl << o << " = " << R0 << "chx_fm::tanhf_faithful(" << a << "));\n";
         } else if (s.op == "Exp") {
             CHX_PROPAGATE(need(1));
@@ -498,11 +518,12 @@ int emit_elem(const Program& prog, bool use_fma, std::ostringstream& os, bool* u
                 // 1 / (1 + exp(-x)), as the CPU path spells it
                 os << decl << o << " = 1.0 / (1.0 + ::exp(-" << a << "));\n";
             } else if (f16) {
-                // the same, every operation a float16 operation
-                os << decl << o << "_e = chx_round_f16(chx_fm::expf_faithful<" << fma << ">(-" << a << "));\n";
+                // the same, every operation a float16 operation.  Which exponential and which reciprocal give the
+                // float16 results of the C library's exp and of the division is a question of 65536 arguments, and a
+                // test asks it for all of them: the device's own instructions do.
+                os << decl << o << "_e = chx_round_f16(__builtin_amdgcn_exp2f(-0x1.715476p+0f * " << a << "));\n";
                 os << decl << o << "_d = chx_round_f16(1.0f + " << o << "_e);\n";
-                os << decl << o << " = chx_round_f16(1.0f / " << o << "_d);\n";
-                *uses_exp_table = true;
+                os << decl << o << " = chx_round_f16(__builtin_amdgcn_rcpf(" << o << "_d));\n";
             } else {
                 os << decl << o << " = kFast ? chx_fm::sigmoid_unless_rare<" << fma << ">(" << a
                    << ", rare) : chx_fm::sigmoid_faithful<" << fma << ">(" << a << ");\n";
@@ -623,7 +644,7 @@ struct GeneralForm {
 // alignment (F, C), one element (S, Z), or `vec` strided ones (X); a run that crosses the end of a row is read
 // element by element from two positions.  Divisions by the extents are multiplications with their reciprocals.
 // float16 chain over [8, 333, 1001] with two [1001] operands: 15.2 us with one element per thread and 64-bit divisions,
-// 7.0 this way.
+// 13.4 this way, and 7.5 once its functions cost less (kTanhOfF16).
 void emit_general(const Program& prog, const std::string& name, const GeneralForm& g, const std::string& VT, std::ostringstream& os) {
     const size_t nin = prog.inputs.size(), nout = prog.outputs.size();
     const int V = g.vec, ND = g.ndim > 0 ? g.ndim : 1;
@@ -764,6 +785,7 @@ int generate_source(
     CHX_PROPAGATE(emit_elem(prog, use_fma, body, &uses_table));
     os << kFaithfulMathText << "\n";
     os << "__device__ __forceinline__ float chx_round_f16(float x) { return (float)(_Float16)x; }\n";
+    if (prog.arith == CHX_HIP_FLOAT16) os << kTanhOfF16;
     os << "typedef float v4f __attribute__((ext_vector_type(4)));\n";
     os << "typedef unsigned int v4u __attribute__((ext_vector_type(4)));\n";
     os << "namespace {\n" << body.str() << "}\n";
