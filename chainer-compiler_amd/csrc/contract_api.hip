@@ -1499,7 +1499,8 @@ extern "C" int chx_hip_conv_integer(
     // allocations, packing): the two meet at 8 G multiply-adds, and it takes channels-last results only.
     const bool packed = weights_fit_mfma(*w, params->group) && (double)a.total * cs.Cg * cs.KH * cs.KW >= 0x1p33 && x_is_mfma_ready(*x);
     if (!capturing && !packed) {
-        const int rc = run_conv_planar(a, s);
+        int rc = run_conv_strip(a, s);
+        if (rc == CHX_HIP_EUNSUPPORTED) rc = run_conv_planar(a, s);
         if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     }
     if (weights_fit_mfma(*w, params->group) && !capturing) {
