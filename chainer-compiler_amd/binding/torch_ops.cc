@@ -14,8 +14,11 @@
 
 #include <algorithm>
 #include <cstring>
+#include <string>
 
 #include <chx_hip.h>
+
+#include "../runtime/chxvm_capi.h"
 
 namespace {
 
@@ -40,6 +43,15 @@ int32_t dtype_code(at::ScalarType t) {
         case at::kFloat: return CHX_HIP_FLOAT32;
         case at::kDouble: return CHX_HIP_FLOAT64;
         default: fail(PyExc_KeyError, "tensor of a type the library does not have");
+    }
+}
+
+int64_t element_size(int32_t code) {
+    switch (code) {
+        case CHX_HIP_INT16: case CHX_HIP_FLOAT16: return 2;
+        case CHX_HIP_INT32: case CHX_HIP_FLOAT32: return 4;
+        case CHX_HIP_INT64: case CHX_HIP_FLOAT64: return 8;
+        default: return 1;
     }
 }
 
@@ -412,6 +424,109 @@ PyObject* plan_run(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// ---- runs of the virtual machine (chxvm.py); its library is loaded by the caller, who hands the entry points over ----
+struct Machine {
+    decltype(&chxvm_program_run_to_host) run;
+    decltype(&chxvm_outputs_count) count;
+    decltype(&chxvm_outputs_name) name;
+    decltype(&chxvm_outputs_layout) layout;
+    decltype(&chxvm_outputs_host) host;
+    decltype(&chxvm_outputs_destroy) destroy;
+} g_machine;
+
+// vm_init(address of each, in the order above)
+PyObject* vm_init(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        need(n, 6);
+        void* at[6];
+        for (int i = 0; i < 6; ++i) at[i] = reinterpret_cast<void*>(integer(a[i]));
+        static_assert(sizeof(g_machine) == sizeof(at), "six addresses");
+        memcpy(&g_machine, at, sizeof(at));
+        Py_RETURN_NONE;
+    });
+}
+
+// [(name, dtype code, shape, bytearray with the dense elements)], or null, with no exception set, when the runtime has
+// no host copy of one of them
+PyObject* host_copies(const chxvm_outputs* out) {
+    const int32_t n = g_machine.count(out);
+    PyObject* list = PyList_New(n);
+    if (!list) throw PythonError();
+    for (int32_t i = 0; i < n; ++i) {
+        chx_hip_tensor d;
+        const void* p = nullptr;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = g_machine.layout(out, i, &d);
+        if (rc == 0) p = g_machine.host(out, i);
+        Py_END_ALLOW_THREADS
+        if (!p) {
+            Py_DECREF(list);
+            return nullptr;
+        }
+        int64_t bytes = element_size(d.dtype);
+        PyObject* shape = PyTuple_New(d.ndim);
+        for (int32_t k = 0; shape && k < d.ndim; ++k) {
+            bytes *= d.shape[k];
+            PyTuple_SET_ITEM(shape, k, PyLong_FromLongLong(d.shape[k]));
+        }
+        PyObject* item = shape ? Py_BuildValue("(siNN)", g_machine.name(out, i), static_cast<int>(d.dtype), shape,
+                                               PyByteArray_FromStringAndSize(static_cast<const char*>(p), static_cast<Py_ssize_t>(bytes)))
+                               : nullptr;
+        if (!item) {
+            Py_DECREF(list);
+            throw PythonError();
+        }
+        PyList_SET_ITEM(list, i, item);
+    }
+    return list;
+}
+
+// vm_outputs(outputs) -> the list above or None
+PyObject* vm_outputs(PyObject*, PyObject* o) {
+    return guarded([&]() -> PyObject* {
+        PyObject* list = host_copies(reinterpret_cast<const chxvm_outputs*>(integer(o)));
+        if (!list) Py_RETURN_NONE;
+        return list;
+    });
+}
+
+// vm_run(program, {name: tensor}, trace level) -> (code of the runtime, address of the outputs or 0, the list above or
+// None); with a list the outputs are gone already
+PyObject* vm_run(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        need(n, 3);
+        chxvm_program* program = reinterpret_cast<chxvm_program*>(integer(a[0]));
+        if (!PyDict_Check(a[1])) fail(PyExc_TypeError, "a dict of tensors is expected");
+        const int32_t trace = static_cast<int32_t>(integer(a[2]));
+        c10::SmallVector<std::string, 4> keys;
+        c10::SmallVector<const char*, 4> names;
+        c10::SmallVector<chx_hip_tensor, 4> descs;
+        Py_ssize_t at = 0;
+        PyObject *key, *value;
+        while (PyDict_Next(a[1], &at, &key, &value)) {
+            const char* name = PyUnicode_AsUTF8(key);
+            if (!name) throw PythonError();
+            keys.emplace_back(name);
+            descs.emplace_back();
+            describe(tensor(value), &descs.back());
+        }
+        for (const std::string& k : keys) names.push_back(k.c_str());
+        chxvm_outputs* out = nullptr;
+        int rc;
+        Py_BEGIN_ALLOW_THREADS
+        rc = g_machine.run(program, names.data(), descs.data(), static_cast<int32_t>(names.size()), trace, &out);
+        Py_END_ALLOW_THREADS
+        if (rc != 0) return Py_BuildValue("(iiO)", rc, 0, Py_None);
+        PyObject* list = host_copies(out);
+        if (!list) return Py_BuildValue("(iLO)", 0, static_cast<long long>(reinterpret_cast<intptr_t>(out)), Py_None);
+        Py_BEGIN_ALLOW_THREADS
+        g_machine.destroy(out);
+        Py_END_ALLOW_THREADS
+        return Py_BuildValue("(iiN)", 0, 0, list);
+    });
+}
+
 PyCFunction fast(PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t)) {
     return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f));
 }
@@ -427,6 +542,9 @@ PyMethodDef methods[] = {
         {"matmul_integer", fast(matmul_integer), METH_FASTCALL, nullptr},
         {"qlinear_matmul", fast(qlinear_matmul), METH_FASTCALL, nullptr},
         {"plan_run", fast(plan_run), METH_FASTCALL, nullptr},
+        {"vm_init", fast(vm_init), METH_FASTCALL, nullptr},
+        {"vm_run", fast(vm_run), METH_FASTCALL, nullptr},
+        {"vm_outputs", vm_outputs, METH_O, nullptr},
         {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_chx_torch_ops", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -24,7 +24,7 @@ IDL_PATH = os.path.join(_HERE, "runtime", "chxvm_ops.idl")
 RUNTIME_EXPORTS = [
     "chxvm_last_error", "chxvm_num_ops", "chxvm_op_name", "chxvm_op_number", "chxvm_proto_roundtrip", "chxvm_free",
     "chxvm_program_create", "chxvm_program_destroy", "chxvm_program_num_instructions", "chxvm_program_num_inputs",
-    "chxvm_program_input_name", "chxvm_program_run", "chxvm_program_run_to_host", "chxvm_outputs_host", "chxvm_outputs_count", "chxvm_outputs_name", "chxvm_outputs_get",
+    "chxvm_program_input_name", "chxvm_program_run", "chxvm_program_run_to_host", "chxvm_outputs_host", "chxvm_outputs_layout", "chxvm_outputs_count", "chxvm_outputs_name", "chxvm_outputs_get",
     "chxvm_outputs_destroy", "chxvm_backend_config_has", "chxvm_backend_config_name", "chxvm_set_option", "chxvm_counter",
     "chxvm_program_set_option", "chxvm_program_counter", "chxvm_program_capture", "chxvm_replay_launch", "chxvm_replay_synchronize",
     "chxvm_replay_outputs", "chxvm_replay_info", "chxvm_replay_destroy",
@@ -99,6 +99,7 @@ def runtime():
         rt.chxvm_replay_info.restype = ctypes.c_int64
         rt.chxvm_replay_destroy.argtypes = [ctypes.c_void_p]
         rt.chxvm_replay_destroy.restype = None
+        rt.chxvm_outputs_layout.argtypes = rt.chxvm_outputs_get.argtypes
         rt.chxvm_backend_config_name.argtypes = [ctypes.c_char_p, ctypes.c_int32, ctypes.c_char_p, ctypes.c_size_t]
         _rt = rt
     return _rt
@@ -334,16 +335,11 @@ _NP_OF_CODE = {1: np.bool_, 2: np.int8, 3: np.int16, 4: np.int32, 5: np.int64, 6
                9: np.float64}
 
 
-def _to_numpy(desc, host=None):
-    """Host copy of the device array a descriptor names, with its shape and element order.  host: where the runtime has
-    the dense elements in host memory already."""
+def _to_numpy(desc):
+    """Host copy of the device array a descriptor names, with its shape and element order."""
     dt = np.dtype(_NP_OF_CODE[desc.dtype])
     nd = desc.ndim
     shape = desc.shape[:nd]
-    if host:
-        a = np.empty(shape, dt)
-        ctypes.memmove(a.ctypes.data, host, a.nbytes)
-        return a
     strides = [desc.strides[i] for i in range(nd)]
     span = dt.itemsize + sum((s - 1) * st for s, st in zip(shape, strides)) if all(shape) else 0
     buf = np.empty(max(span, 1), dtype=np.uint8)
@@ -353,6 +349,36 @@ def _to_numpy(desc, host=None):
     view = np.lib.stride_tricks.as_strided(buf[:dt.itemsize].view(dt), shape=shape, strides=strides) if span else \
         np.empty(shape, dt)
     return np.array(view, order="C")  # a copy that keeps 0-d arrays 0-d (ascontiguousarray would make them 1-d)
+
+
+_machine = None
+
+
+def _native():
+    """The extension module's face of the runtime's runs (binding/torch_ops.cc)."""
+    global _machine
+    if _machine is None:
+        rt, native = runtime(), capi.native()
+        native.vm_init(*[ctypes.cast(getattr(rt, n), ctypes.c_void_p).value for n in (
+            "chxvm_program_run_to_host", "chxvm_outputs_count", "chxvm_outputs_name", "chxvm_outputs_layout", "chxvm_outputs_host",
+            "chxvm_outputs_destroy")])
+        _machine = native
+    return _machine
+
+
+def _arrays(host):
+    """{name: array} from the extension's host copies: [(name, dtype code, shape, bytearray)]."""
+    return {name: np.ndarray(shape, _NP_OF_CODE[code], data) for name, code, shape, data in host}
+
+
+def _fetch(out):
+    """The same by copying the device arrays."""
+    rt, result = runtime(), {}
+    for i in range(rt.chxvm_outputs_count(out)):
+        d = capi.Tensor()
+        _check(rt.chxvm_outputs_get(out, i, ctypes.byref(d)))
+        result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d)
+    return result
 
 
 class Program:
@@ -374,21 +400,15 @@ class Program:
 
     def run(self, inputs, trace_level=0):
         """inputs: {name: torch device tensor}.  Returns {name: numpy array}."""
-        rt = runtime()
-        names = list(inputs)
-        c_names = (ctypes.c_char_p * len(names))(*[n.encode() for n in names])
-        descs = (capi.Tensor * len(names))(*[capi.desc(inputs[n]) for n in names])
-        out = ctypes.c_void_p()
-        _check(rt.chxvm_program_run_to_host(self._h, c_names, descs, len(names), trace_level, ctypes.byref(out)))
+        rc, out, host = _native().vm_run(self._h.value or 0, inputs, trace_level)
+        _check(rc)
+        if host is not None:
+            return _arrays(host)
+        out = ctypes.c_void_p(out)
         try:
-            result = {}
-            for i in range(rt.chxvm_outputs_count(out)):
-                d = capi.Tensor()
-                _check(rt.chxvm_outputs_get(out, i, ctypes.byref(d)))
-                result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d, rt.chxvm_outputs_host(out, i))
-            return result
+            return _fetch(out)
         finally:
-            rt.chxvm_outputs_destroy(out)
+            runtime().chxvm_outputs_destroy(out)
 
     def capture(self, inputs):
         """Records one run on the device buffers of `inputs` ({name: torch device tensor}; keep them alive,
@@ -440,14 +460,9 @@ class Replay:
 
     def outputs(self):
         """{name: numpy array} of the last launch; the device must be done with it (synchronize())."""
-        rt = runtime()
-        out = rt.chxvm_replay_outputs(self._h)
-        result = {}
-        for i in range(rt.chxvm_outputs_count(out)):
-            d = capi.Tensor()
-            _check(rt.chxvm_outputs_get(out, i, ctypes.byref(d)))
-            result[rt.chxvm_outputs_name(out, i).decode()] = _to_numpy(d, rt.chxvm_outputs_host(out, i))
-        return result
+        out = runtime().chxvm_replay_outputs(self._h)
+        host = _native().vm_outputs(out)
+        return _fetch(out) if host is None else _arrays(host)
 
     def info(self, name):
         """"pool_bytes", "pool_blocks", "warm_runs"."""

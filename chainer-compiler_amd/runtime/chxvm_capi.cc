@@ -124,6 +124,7 @@ struct chxvm_outputs {
     std::vector<chainerx::Array> arrays;
     InOuts keep_inputs;
     std::vector<std::vector<char>> host;  // an eager run's host copies, where it made them
+    mutable bool exposed = false;         // the caller knows device addresses
     chxvm_replay* replay = nullptr;       // whose outputs these are
 };
 
@@ -382,6 +383,15 @@ int32_t chxvm_outputs_get(const chxvm_outputs* outputs, int32_t i, chx_hip_tenso
     return Guard([&] {
         CHECK_LT(static_cast<size_t>(i), outputs->arrays.size());
         *out = outputs->arrays[static_cast<size_t>(i)].hip();
+        outputs->exposed = true;
+    });
+}
+
+int32_t chxvm_outputs_layout(const chxvm_outputs* outputs, int32_t i, chx_hip_tensor* out) {
+    return Guard([&] {
+        CHECK_LT(static_cast<size_t>(i), outputs->arrays.size());
+        *out = outputs->arrays[static_cast<size_t>(i)].hip();
+        out->data = nullptr;
     });
 }
 
@@ -403,8 +413,9 @@ const void* chxvm_outputs_host(const chxvm_outputs* outputs, int32_t i) {
 }
 
 void chxvm_outputs_destroy(chxvm_outputs* outputs) {
-    // the arrays' memory is handed out again: nothing may read it any more
-    if (outputs && !outputs->arrays.empty()) (void)chx_hip_device_synchronize();
+    // The arrays' memory is handed out again: nothing may read it any more.  Of a run whose results have arrived on the
+    // host, and whose addresses nobody was given, nothing does (the device is told so 5 us after the host knows).
+    if (outputs && !outputs->arrays.empty() && (outputs->host.empty() || outputs->exposed)) (void)chx_hip_device_synchronize();
     delete outputs;
 }
 

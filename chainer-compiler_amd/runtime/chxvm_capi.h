@@ -57,6 +57,8 @@ int32_t chxvm_outputs_count(const chxvm_outputs* outputs);
 const char* chxvm_outputs_name(const chxvm_outputs* outputs, int32_t i);
 /* Descriptor of output i (device memory owned by `outputs`). */
 int32_t chxvm_outputs_get(const chxvm_outputs* outputs, int32_t i, chx_hip_tensor* out);
+/* The same without the address (data is null): for a caller that takes the host copy and leaves the device's alone. */
+int32_t chxvm_outputs_layout(const chxvm_outputs* outputs, int32_t i, chx_hip_tensor* out);
 /* Output i in host memory, dense, valid as long as `outputs` (a replay's: until its next launch), or null: copy it from
  * the device then.  Of a replay this is the last launch's result; the first call makes later launches send theirs. */
 const void* chxvm_outputs_host(const chxvm_outputs* outputs, int32_t i);
