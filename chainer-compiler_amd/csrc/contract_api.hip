@@ -409,7 +409,7 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
     if (all.size() > 8) all.resize(8);
     if (other) {
         for (Candidate& c : all) c.seen.clear();
-        for (int round = 0; round < 3; ++round) look(1, true);
+        for (int round = 0; round < 5; ++round) look(1, true);
         (void)hipFreeAsync(other, s);
     }
     for (size_t i = 0; i < created; ++i) (void)hipEventDestroy(events[i]);
