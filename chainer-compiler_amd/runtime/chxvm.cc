@@ -567,6 +567,25 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         program_.back()->InitImpl();
     }
+    // the constants that one instruction writes, once, as the only one
+    std::vector<int> writers(num_variables_ > 0 ? num_variables_ : 1, 0);
+    for (const ChxVMInstructionProto& inst : program.instructions)
+        for (int o : inst.outputs)
+            if (o >= 0) ++writers[o];
+    constant_slots_.assign(num_variables_ > 0 ? num_variables_ : 1, nullptr);
+    ChxVMState scratch(ChxVMOptions(), num_variables_, InOuts());
+    for (int i = 0; i < n; ++i) {
+        const ChxVMInstructionProto& inst = program.instructions[i];
+        const bool constant = literal_ops.count(inst.op) && inst.outputs.size() == 1 && inst.outputs[0] >= 0 && writers[inst.outputs[0]] == 1;
+        if (constant && role[i] == 0) {
+            const int slot = inst.outputs[0];
+            program_[i]->Run(&scratch);
+            constants_.emplace_back(new ChxVMVar(*scratch.GetVar(slot)));
+            constant_slots_[slot] = constants_.back().get();
+        } else if (!dynamic_cast<NopOp*>(program_[i].get())) {
+            remaining_.push_back(i);
+        }
+    }
 }
 
 ChxVM::~ChxVM() = default;
@@ -696,6 +715,23 @@ InOuts ChxVM::Run(const InOuts& program_inputs, const ChxVMOptions& options) {
         } else {
             CHECK_EQ(0, type.dtype) << "Input '" << name << "' must be a tensor";
         }
+    }
+    if (options.trace_level == 0 && !options.check_types && !options.check_nans && !options.check_infs && options.dump_memory_usage == 0 &&
+        !options.chrome_tracing && options.dump_outputs_dir.empty()) {
+        ChxVMState state(options, constant_slots_, program_inputs);
+        state.set_minus_128_slots(&minus_128_slots_);
+        for (int pc : remaining_) {
+            ChxVMOp* op = program_[pc].get();
+            state.set_pc(pc);
+            try {
+                op->Run(&state);
+            } catch (...) {
+                std::cerr << "Exception in " << op->name() << " (pc " << pc << ") " << op->debug_info() << std::endl;
+                throw;
+            }
+        }
+        residual_fusions_ += state.residual_fusions();
+        return state.GetOutputs();
     }
     ChxVMState state(options, num_variables_, program_inputs);
     // (a run that checks result types against the program's or writes results to files sees plain codes everywhere)

@@ -82,6 +82,12 @@ private:
     std::vector<ChxVMTypeProto> input_types_;
     int num_variables_ = 0;
     int64_t residual_fusions_ = 0;
+    // For runs that nothing looks into: the constants' variables (null: a slot that instructions write), made once, and the
+    // instructions that remain.  A network of 54 convolutions has 444 constants; setting them took a third of the
+    // interpreter's time.
+    std::vector<std::unique_ptr<ChxVMVar>> constants_;
+    std::vector<ChxVMVar*> constant_slots_;
+    std::vector<int> remaining_;
     std::vector<bool> minus_128_slots_;  // per variable: see ChxVMState::store_minus_128
 };
 

@@ -9,31 +9,44 @@ namespace chainer_compiler {
 namespace runtime {
 
 ChxVMState::ChxVMState(const ChxVMOptions& options, int num_variables, const InOuts& inputs)
-    : variables_(num_variables), inputs_(inputs), options_(options) {
+    : variables_(num_variables), owned_(num_variables), inputs_(inputs), options_(options) {
+}
+
+ChxVMState::ChxVMState(const ChxVMOptions& options, const std::vector<ChxVMVar*>& constants, const InOuts& inputs)
+    : variables_(constants), owned_(constants.size()), inputs_(inputs), options_(options) {
 }
 
 ChxVMVar* ChxVMState::GetVar(int index) {
     CHECK_LE(0, index) << "negative variable id";
     CHECK_GT(static_cast<int>(variables_.size()), index);
-    CHECK(variables_[index].get()) << "variable $" << index << " is read before it is set";
-    return variables_[index].get();
+    CHECK(variables_[index]) << "variable $" << index << " is read before it is set";
+    return variables_[index];
 }
 
 ChxVMVar* ChxVMState::PeekVar(int index) {
     if (index < 0 || index >= static_cast<int>(variables_.size())) return nullptr;
-    return variables_[index].get();
+    return variables_[index];
+}
+
+ChxVMVar* ChxVMState::OwnVar(int index, bool as_it_is) {
+    ChxVMVar* var = GetVar(index);
+    if (as_it_is || owned_[index]) return var;
+    owned_[index].reset(new ChxVMVar(*var));
+    return variables_[index] = owned_[index].get();
 }
 
 void ChxVMState::SetVar(int index, const ChxVMVar& var) {
     CHECK_LE(0, index);
     CHECK_GT(static_cast<int>(variables_.size()), index);
+    if (variables_[index] && !owned_[index]) return;  // the program's constant
     // a slot is written once between two Free's (runtime/chxvm_state.cc:171-176)
-    CHECK(!variables_[index].get()) << "variable $" << index << " is set twice";
-    variables_[index].reset(new ChxVMVar(var));
+    CHECK(!variables_[index]) << "variable $" << index << " is set twice";
+    owned_[index].reset(new ChxVMVar(var));
+    variables_[index] = owned_[index].get();
 }
 
-chainerx::Array ChxVMState::GetArray(int index) {
-    return GetVar(index)->GetArray();
+const chainerx::Array& ChxVMState::GetArray(int index) {
+    return OwnVar(index, GetVar(index)->kind() == ChxVMVar::Kind::kArray)->GetArray();
 }
 
 absl::optional<chainerx::Array> ChxVMState::GetOptionalArray(int index) {
@@ -48,7 +61,8 @@ void ChxVMState::SetArray(int index, const chainerx::Array& value) {
 void ChxVMState::FreeVar(int index) {
     CHECK_LE(0, index);
     CHECK_GT(static_cast<int>(variables_.size()), index);
-    variables_[index].reset();
+    variables_[index] = nullptr;
+    owned_[index].reset();
 }
 
 std::vector<chainerx::Array> ChxVMState::GetArrayList(const std::vector<int>& index) {
@@ -63,7 +77,7 @@ void ChxVMState::SetArrayList(const std::vector<int>& index, const std::vector<c
 }
 
 const chainerx::Shape& ChxVMState::GetShape(int index) {
-    return GetVar(index)->GetShape();
+    return OwnVar(index, GetVar(index)->kind() == ChxVMVar::Kind::kShape)->GetShape();
 }
 
 void ChxVMState::SetShape(int index, chainerx::Shape s) {
@@ -71,7 +85,7 @@ void ChxVMState::SetShape(int index, chainerx::Shape s) {
 }
 
 const StrictScalar& ChxVMState::GetScalar(int index) {
-    return GetVar(index)->GetScalar();
+    return OwnVar(index, GetVar(index)->kind() == ChxVMVar::Kind::kScalar)->GetScalar();
 }
 
 absl::optional<StrictScalar> ChxVMState::GetOptionalScalar(int index) {
@@ -133,7 +147,7 @@ void ChxVMState::CheckInfs(const std::vector<int>& inputs, const std::vector<int
 
 int64_t ChxVMState::GetTotalVariableSize() const {
     std::map<const void*, int64_t> sizes;
-    for (const auto& v : variables_) {
+    for (const ChxVMVar* v : variables_) {
         if (!v || !v->IsArray()) continue;
         const chainerx::Array& a = v->GetArray();
         if (a.IsNullHandle()) continue;

@@ -45,6 +45,9 @@ struct ChxVMOptions {
 class ChxVMState {
 public:
     ChxVMState(const ChxVMOptions& options, int num_variables, const InOuts& inputs);
+    // With the program's constants in their slots already (null: an ordinary slot); an instruction that writes one of
+    // them has no effect.
+    ChxVMState(const ChxVMOptions& options, const std::vector<ChxVMVar*>& constants, const InOuts& inputs);
 
     int pc() const {
         return pc_;
@@ -53,7 +56,8 @@ public:
         pc_ = pc;
     }
 
-    chainerx::Array GetArray(int index);
+    // (valid until the slot is freed)
+    const chainerx::Array& GetArray(int index);
     absl::optional<chainerx::Array> GetOptionalArray(int index);
     void SetArray(int index, const chainerx::Array& value);
     void FreeVar(int index);
@@ -140,7 +144,12 @@ private:
     void CheckNonFinite(const std::vector<int>& inputs, const std::vector<int>& outputs, bool infinities);
 
     int pc_ = 0;
-    std::vector<std::unique_ptr<ChxVMVar>> variables_;
+    // The slots of the run.  A constant's slot points at the program's own variable until somebody asks for it as another
+    // kind: what such a conversion leaves in a variable belongs to this run (its stream, its allocator), so that it is made
+    // on a copy.
+    ChxVMVar* OwnVar(int index, bool as_it_is);
+    std::vector<ChxVMVar*> variables_;
+    std::vector<std::unique_ptr<ChxVMVar>> owned_;
     InOuts inputs_;
     InOuts outputs_;
     ChxVMOptions options_;
