@@ -942,13 +942,15 @@ ConvCall conv_call_from(const QConvChecked& q, const chx_hip_tensor* x, chx_hip_
     return c;
 }
 
-// Runs the depthwise kernel; EUNSUPPORTED when the operand layouts are not channels-last.
+// Runs a depthwise kernel; EUNSUPPORTED when the operands are neither channels-last nor NCHW.
 int run_depthwise(const ConvCall& c, const DepthwiseState& st, hipStream_t s) {
     const chx_hip_tensor& x = *c.x;
     const chx_hip_tensor& y = *c.y;
-    if (!is_depthwise_layout(x) || !is_depthwise_layout(y))
-        CHX_FAIL(CHX_HIP_EUNSUPPORTED, "depthwise kernel needs channels-last 8-bit operands with 16-byte aligned pixels");
-    if (x.strides[3] * x.shape[3] >= (int64_t(1) << 31) || y.strides[3] * y.shape[3] >= (int64_t(1) << 31))
+    const bool channels_last = is_depthwise_layout(x) && is_depthwise_layout(y);
+    const bool planar = !channels_last && is_q8(x.dtype) && is_q8(y.dtype) && (x.strides[3] == 1 || x.shape[3] == 1) && (y.strides[3] == 1 || y.shape[3] == 1);
+    if (!channels_last && !planar)
+        CHX_FAIL(CHX_HIP_EUNSUPPORTED, "depthwise kernel needs channels-last 8-bit operands with 16-byte aligned pixels, or NCHW ones");
+    if (channels_last && (x.strides[3] * x.shape[3] >= (int64_t(1) << 31) || y.strides[3] * y.shape[3] >= (int64_t(1) << 31)))
         CHX_FAIL(CHX_HIP_EUNSUPPORTED, "depthwise kernel: an input or output row spans 2 GiB or more");
     const bool xs = x.dtype == CHX_HIP_INT8;
     const int32_t zp_u = xs ? c.x_zp + 128 : c.x_zp;
@@ -962,6 +964,8 @@ int run_depthwise(const ConvCall& c, const DepthwiseState& st, hipStream_t s) {
     a.y_n_stride = y.strides[0];
     a.y_h_stride = y.strides[2];
     a.y_w_stride = y.strides[3];
+    a.x_c_stride = x.strides[1];
+    a.y_c_stride = y.strides[1];
     a.N = c.cs.N; a.C = c.cs.C; a.H = c.cs.H; a.W = c.cs.W; a.OH = c.cs.OH; a.OW = c.cs.OW;
     a.sh = c.p->stride_h; a.sw = c.p->stride_w; a.ph = c.p->pad_h_begin; a.pw = c.p->pad_w_begin;
     a.x_signed = xs ? 1 : 0;
@@ -978,7 +982,7 @@ int run_depthwise(const ConvCall& c, const DepthwiseState& st, hipStream_t s) {
     a.lo_folded = fold_relu_floor(c.rq.q, c.rq.relu_floor, c.rne);
     a.qp = product_form(c.rq.q, a.lo_folded, c.rne);
     a.y_flip = c.y_minus_128 ? 0x80808080u : 0u;  // (c.y is then the uint8 view of the caller's int8 array)
-    return launch_depthwise3x3(a, c.rne, s);
+    return planar ? launch_depthwise_planar(a, c.rne, s) : launch_depthwise3x3(a, c.rne, s);
 }
 
 }  // namespace

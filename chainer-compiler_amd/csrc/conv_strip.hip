@@ -43,15 +43,6 @@ __device__ __forceinline__ uint32_t divided(uint32_t n, uint32_t mul, uint32_t s
     return (__umulhi(n, mul) + n) >> shift;
 }
 
-// 8 bytes at column `at` of a row of W >= 8, columns outside filled with zp (all of them from W + 8 on)
-__device__ __forceinline__ uint64_t window8(const char* row, int at, int W, uint64_t zp) {
-    typedef uint64_t u64_u __attribute__((aligned(1)));
-    const int from = min(max(at, 0), W - 8), d = at - from, up = min(max(8 * d, 0), 64), down = min(max(-8 * d, 0), 64);
-    // (shifts in two halves: 64 is one of the distances)
-    const uint64_t v = *reinterpret_cast<const u64_u*>(row + from) ^ zp;
-    return ((v >> (up / 2) >> (up - up / 2)) << (down / 2) << (down - down / 2)) ^ zp;
-}
-
 constexpr int kR = 32, kStep = 32, kRegs = 16, kWaves = 8;
 
 // FT: filter tiles of the work-group (64 or 32 filters); its wavefronts split K kWaves / FT ways.

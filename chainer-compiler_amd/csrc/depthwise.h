@@ -10,6 +10,7 @@ struct DepthwiseArgs {
     // activations, channels-last: element (n, c, ih, iw) at x + n*x_n_stride + ih*x_h_stride + iw*x_w_stride + c
     const char* x;
     int64_t x_n_stride, x_h_stride, x_w_stride;
+    int64_t x_c_stride, y_c_stride;  // NCHW arrays only (launch_depthwise_planar)
     char* y;  // same convention
     int64_t y_n_stride, y_h_stride, y_w_stride;
     int32_t N, C, H, W, OH, OW, sh, sw, ph, pw;
@@ -38,5 +39,7 @@ struct DepthwiseArgs {
 
 int pack_depthwise(const chx_hip_tensor& w, int32_t* rows, int32_t* wsum, hipStream_t s);
 int launch_depthwise3x3(DepthwiseArgs a, bool rne, hipStream_t s);
+// NCHW x and y with contiguous rows (depthwise_planar.hip); EUNSUPPORTED, with nothing launched, for strides it does not take
+int launch_depthwise_planar(const DepthwiseArgs& a, bool rne, hipStream_t s);
 
 }  // namespace chx

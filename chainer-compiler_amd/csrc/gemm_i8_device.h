@@ -101,6 +101,15 @@ __device__ __forceinline__ void columns_of(uint32_t (&w)[16], bool ragged, int s
     transpose16x4(w, fb);
 }
 
+// 8 bytes at column `at` of a row of W >= 8, columns outside filled with zp (all of them from W + 8 on)
+__device__ __forceinline__ uint64_t window8(const char* row, int at, int W, uint64_t zp) {
+    typedef uint64_t u64_u __attribute__((aligned(1)));
+    const int from = min(max(at, 0), W - 8), d = at - from, up = min(max(8 * d, 0), 64), down = min(max(-8 * d, 0), 64);
+    // (shifts in two halves: 64 is one of the distances)
+    const uint64_t v = *reinterpret_cast<const u64_u*>(row + from) ^ zp;
+    return ((v >> (up / 2) >> (up - up / 2)) << (down / 2) << (down - down / 2)) ^ zp;
+}
+
 __device__ __forceinline__ int32_t sum_bytes(v4i v, int32_t acc) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_sdot4(v[i], 0x01010101, acc, false);

@@ -1,0 +1,33 @@
+"""QLinearConv plans on NCHW arrays: the planar depthwise kernel (csrc/depthwise_planar.hip) and the layout changes around
+the matrix-core kernel (csrc/layout.hip), at rows shorter than an access, ragged tiles and the last bytes of an array."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_conv_split import codes, g  # noqa: F401 (g is a fixture)
+
+pytestmark = pytest.mark.gpu
+
+# N, C, H, W, OC, k, stride, pad, group
+CASES = [(1, 16, 1, 1, 16, 3, 1, 1, 16), (2, 32, 7, 7, 32, 3, 1, 1, 32), (1, 16, 9, 8, 16, 3, 2, 1, 16), (3, 48, 13, 30, 48, 3, 1, 0, 48), (2, 16, 18, 37, 16, 3, 2, 1, 16),
+         (1, 64, 8, 8, 64, 1, 1, 0, 1), (2, 70, 7, 7, 33, 3, 1, 1, 1), (1, 24, 5, 13, 130, 1, 1, 0, 1), (1, 17, 3, 43, 16, 3, 2, 1, 1)]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_against_the_oracle(g, oracle, case):
+    N, C, H, W, OC, k, st, pad, group = case
+    rng = np.random.default_rng(C + W)
+    for xdt, ydt, xz, yz, rne, relu, bias_mode in [(np.uint8, np.uint8, 0, 0, False, True, 2), (np.uint8, np.uint8, 77, 9, False, True, 1),
+                                                   (np.uint8, np.uint8, 3, 120, False, False, 0), (np.int8, np.int8, -9, 5, True, False, 2)]:
+        x, w = codes(rng, (N, C, H, W), xdt), codes(rng, (OC, C // group, k, k), np.int8)
+        ws, bias = rng.uniform(0.002, 0.02, size=OC).astype(np.float32), rng.integers(-3000, 3000, size=OC).astype(np.int32)
+        ys = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C // group * k * k) / 40)
+        flags = (g.capi.ROUND_ONNX_RNE if rne else 0) | (g.capi.FUSE_RELU if relu else 0) | (g.capi.BIAS_ONNX_INT32 if bias_mode == 2 else 0)
+        plan = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(OC, np.int8)), g.dev(bias) if bias_mode else None, strides=(st, st), pads=(pad, pad), group=group)
+        got = plan.run(g.dev(x), 0.02, xz, ys, yz, zero_point_dtype=torch.uint8 if ydt == np.uint8 else torch.int8, flags=flags)
+        assert got.is_contiguous()
+        okw = dict(bias=bias, bias_mode=oracle.BIAS_ONNX_INT32 if bias_mode == 2 else oracle.BIAS_REFERENCE_FLOAT) if bias_mode else {}
+        want = oracle.qlinear_conv_int(x, 0.02, xz, w, ws, np.zeros(OC, np.int8), ys, yz, ydt, strides=(st, st), pads=(pad, pad), group=group,
+                                       round_mode=oracle.ROUND_ONNX_RNE if rne else oracle.ROUND_REFERENCE, **okw)
+        np.testing.assert_array_equal(g.host(got), np.maximum(want, yz) if relu else want)
+        plan.close()
