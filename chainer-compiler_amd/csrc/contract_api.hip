@@ -308,7 +308,7 @@ public:
         (void)hipGetDevice(&device);
         const int64_t res = a.res.r ? 1 + a.res.affine : 0;
         return {device, a.M, a.H, a.W, a.OH, a.OW, a.KH, a.KW, a.sh, a.sw, a.ph, a.pw, a.C16, a.KP, a.bk, a.OC, a.oc_split, a.x_n_stride,
-                a.x_w_stride, a.y_px_stride, a.y_vec_ok, res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
+                a.x_w_stride, a.y_px_stride, aligned(a.y, 16), res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
     }
     bool find(const Key& k, Configuration* c) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -591,11 +591,16 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         a.x_n_stride = x.strides[0];
         a.x_h_stride = x.strides[2];
         a.x_w_stride = x.strides[3];
-    } else if (is_contiguous(x)) {
+    } else if (is_contiguous(x) || x.strides[1] == 1) {
+        // (channels-last pixels at another pitch, 40 channels packed say, are copied to the pitch of 16 bytes)
         const int64_t HW = (int64_t)cs.H * cs.W;
         CHX_PROPAGATE(acquire_scratch(c.cache, 0, (size_t)cs.N * HW * C16, s, &x_scratch));
-        CHX_PROPAGATE(launch_nchw_to_nhwc_u8(static_cast<const char*>(x.data), static_cast<char*>(x_scratch), cs.N, cs.C,
-                                             HW, C16, s));
+        const int rc_x = is_contiguous(x) ? launch_nchw_to_nhwc_u8(static_cast<const char*>(x.data), static_cast<char*>(x_scratch), cs.N, cs.C, HW, C16, s)
+                                          : launch_pixels_u8(static_cast<const char*>(x.data), x.strides[0], x.strides[2], x.strides[3], static_cast<char*>(x_scratch), cs.N, cs.C, cs.H, cs.W, C16, s);
+        if (rc_x != CHX_HIP_OK) {
+            release_scratch(c.cache, x_scratch, s);
+            return rc_x;
+        }
         a.x = static_cast<const char*>(x_scratch);
         a.x_w_stride = C16;
         a.x_h_stride = (int64_t)cs.W * C16;
@@ -624,7 +629,6 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         release_scratch(c.cache, x_scratch, s);
         CHX_FAIL(CHX_HIP_EUNSUPPORTED, "y layout is neither pixel-major nor NCHW-contiguous 8-bit");
     }
-    a.y_vec_ok = aligned(a.y, 16) && (a.y_px_stride % 16 == 0) ? 1 : 0;
     (void)es;
     if (c.y_minus_128 || c.y2_minus_128) {
         if (stem || y_post || c.out_int32) {
@@ -644,7 +648,6 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         a.oc_split = c.oc_split;
         a.y2 = static_cast<char*>(c.y2->data);
         a.y2_px_stride = y2_px;
-        a.y2_vec_ok = aligned(a.y2, 16) && (y2_px % 16 == 0) ? 1 : 0;
         a.y2_flip = c.y2_minus_128 ? 0x80808080u : 0u;
         a.q2 = c.rq2.q;
         a.inv_y_scale2 = 1.0f / c.rq2.q.scale;
@@ -663,7 +666,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         sa.x_zp = c.x_zp;
         sa.x_unsigned = x.dtype == CHX_HIP_UINT8 ? 1 : 0;
         sa.corr_mult = sa.x_unsigned ? 128 - c.x_zp : -c.x_zp;
-        sa.y = a.y; sa.y_px_stride = a.y_px_stride; sa.y_vec_ok = a.y_vec_ok;
+        sa.y = a.y; sa.y_px_stride = a.y_px_stride;
         sa.w_scale = c.w_scale; sa.w_scale_len = c.w_scale_len; sa.bias = c.bias;
         sa.rq = c.rq;
         sa.inv_y_scale = 1.0f / c.rq.q.scale;

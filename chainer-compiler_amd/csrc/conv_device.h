@@ -8,6 +8,9 @@ namespace chx {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+// the same at any alignment, one instruction all the same (a result's pixels may be of any pitch)
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32_u __attribute__((aligned(1)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 

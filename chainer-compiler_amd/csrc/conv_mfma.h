@@ -69,7 +69,6 @@ struct ConvMfmaArgs {
     // output, pixel-major: element (m, oc) at y + m*y_px_stride + oc*elemsize
     char* y;
     int64_t y_px_stride;
-    int32_t y_vec_ok;     // 16-byte stores allowed (base and pitch aligned)
     uint32_t y_flip;      // 0x80808080: every stored byte is the code minus 128 (CHX_HIP_STORE_MINUS_128), else 0
     // epilogue
     const float* w_scale;
@@ -95,7 +94,6 @@ struct ConvMfmaArgs {
     int32_t oc_split;
     char* y2;
     int64_t y2_px_stride;
-    int32_t y2_vec_ok;
     uint32_t y2_flip;
     QuantParams q2;
     float inv_y_scale2;
@@ -117,7 +115,6 @@ struct ConvStemArgs {
     int32_t corr_mult;    // (128 - x_zp) for uint8 x, (-x_zp) for int8 x
     char* y;              // pixel-major, as for ConvMfmaArgs
     int64_t y_px_stride;
-    int32_t y_vec_ok;
     const float* w_scale;
     int32_t w_scale_len;
     const int32_t* bias;
@@ -207,6 +204,8 @@ int launch_read_through(const void* p, size_t bytes, hipStream_t s);
 
 // [N][C][HW] bytes -> [N][HW][pitch] bytes (lanes c >= C of a pixel are zero filled) and back
 int launch_nchw_to_nhwc_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);
+// pixels of C contiguous bytes at any strides -> [N][H][W][pitch], a multiple of 16, zero filled
+int launch_pixels_u8(const char* src, int64_t n_stride, int64_t h_stride, int64_t w_stride, char* dst, int N, int C, int H, int W, int pitch, hipStream_t s);
 int launch_nhwc_to_nchw_u8(const char* src, char* dst, int N, int C, int64_t HW, int pitch, hipStream_t s);
 
 }  // namespace chx

@@ -481,7 +481,6 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
             if (oc0 >= a.oc_split) {
                 a.y = a.y2 - a.oc_split;
                 a.y_px_stride = a.y2_px_stride;
-                a.y_vec_ok = a.y2_vec_ok;
                 a.y_flip = a.y2_flip;
                 a.rq.q = a.q2;
                 a.inv_y_scale = a.inv_y_scale2;
@@ -507,8 +506,8 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
                         v4i out;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) out[e] = acc[i][j][g * 4 + e];
-                        if (a.y_vec_ok && oc + 4 <= a.OC) {
-                            *reinterpret_cast<v4i*>(yrow + (int64_t)oc * 4) = out;
+                        if (oc + 4 <= a.OC) {
+                            *reinterpret_cast<v4i_u*>(yrow + (int64_t)oc * 4) = out;
                         } else {
 #pragma unroll
                             for (int e = 0; e < 4; ++e)
@@ -600,7 +599,7 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
         // (the operands of this test are the same for the whole work-group); per-lane branches in the loops
         // below cost far more than the instructions they skip.
         // (in 32-bit scalar terms: every pixel tile but the last is full, and the last one is when TN divides M)
-        const bool tile_inside = (px_tile + 1 < a.tiles_px || a.M % TN == 0) && oc0 + TM <= a.OC && a.y_vec_ok && (!kRes || a.res.r_vec_ok);
+        const bool tile_inside = (px_tile + 1 < a.tiles_px || a.M % TN == 0) && oc0 + TM <= a.OC && (!kRes || a.res.r_vec_ok);
         if (kRes && tile_inside) {
 #pragma unroll
             for (int it = 0; it < ITER; ++it) {
@@ -655,7 +654,7 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
                     if constexpr (kMode == 2) val = affine_residual16<true>(val, rres[it], res);
                     if constexpr (kMode == 3) val = add_residual16_any(val, rres[it], res);
                     val ^= store_flip;
-                    *reinterpret_cast<v4i*>(a.y + (m0 + pxl) * a.y_px_stride + oc0 + ch * 16) = val;
+                    *reinterpret_cast<v4i_u*>(a.y + (m0 + pxl) * a.y_px_stride + oc0 + ch * 16) = val;
                 }
             };
             if (!kRes) store_all(std::integral_constant<int, 0>());
@@ -692,13 +691,16 @@ __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(2))) 
                 else val = add_residual16_any(val, rv, a.res);
             }
             val ^= (int)a.y_flip;
-            if (!(a.y_vec_ok && whole)) *reinterpret_cast<v4i*>(src) = val;  // the byte loop below reads LDS
+            if (!whole) *reinterpret_cast<v4i*>(src) = val;  // the loops below read LDS
             char* dst = a.y + m * a.y_px_stride + oc;
-            if (a.y_vec_ok && whole) {
-                *reinterpret_cast<v4i*>(dst) = val;
+            if (whole) {
+                *reinterpret_cast<v4i_u*>(dst) = val;
             } else {
+                int e = 0;
 #pragma nounroll
-                for (int e = 0; e < 16 && oc + e < a.OC; ++e) dst[e] = src[e];
+                for (; oc + e + 4 <= a.OC; e += 4) *reinterpret_cast<u32_u*>(dst + e) = *reinterpret_cast<const uint32_t*>(src + e);
+#pragma nounroll
+                for (; oc + e < a.OC; ++e) dst[e] = src[e];
             }
         }
     };

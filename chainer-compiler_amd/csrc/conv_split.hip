@@ -208,7 +208,6 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
     if (a.oc_split > 0 && oc0 >= a.oc_split) {
         a.y = a.y2 - a.oc_split;
         a.y_px_stride = a.y2_px_stride;
-        a.y_vec_ok = a.y2_vec_ok;
         a.y_flip = a.y2_flip;
         a.rq.q = a.q2;
         a.inv_y_scale = a.inv_y_scale2;
@@ -233,7 +232,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
         }
         word ^= a.y_flip;
         char* dst = a.y + f.m * a.y_px_stride + f.c0;
-        if (a.y_vec_ok && f.c0 + 4 <= OC) *reinterpret_cast<uint32_t*>(dst) = word;
+        if (f.c0 + 4 <= OC) *reinterpret_cast<u32_u*>(dst) = word;
         else
             for (int e = 0; e < 4; ++e)
                 if (f.c0 + e < OC) dst[e] = (char)(word >> (8 * e));

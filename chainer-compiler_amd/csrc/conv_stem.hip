@@ -26,6 +26,7 @@ namespace {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -312,8 +313,8 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
             const char* src = staged(pxl, ch * 16);
             const v4i val = *reinterpret_cast<const v4i*>(src);
             char* dst = a.y + (((int64_t)n * a.OH + oh) * a.OW + ow) * a.y_px_stride + oc;
-            if (a.y_vec_ok && oc + 16 <= a.OC) {
-                *reinterpret_cast<v4i*>(dst) = val;
+            if (oc + 16 <= a.OC) {
+                *reinterpret_cast<v4i_u*>(dst) = val;
             } else {
 #pragma nounroll
                 for (int e = 0; e < 16 && oc + e < a.OC; ++e) dst[e] = src[e];

@@ -1,5 +1,5 @@
-"""QLinearConv plans on NCHW arrays: the planar depthwise kernel (csrc/depthwise_planar.hip) and the layout changes around
-the matrix-core kernel (csrc/layout.hip), at rows shorter than an access, ragged tiles and the last bytes of an array."""
+"""QLinearConv plans on NCHW arrays and on packed channels-last ones: the planar depthwise kernel
+(csrc/depthwise_planar.hip) and the layout changes around the matrix-core kernel (csrc/layout.hip), at rows shorter than an access, ragged tiles and the last bytes of an array."""
 import numpy as np
 import pytest
 import torch
@@ -14,7 +14,8 @@ CASES = [(1, 16, 1, 1, 16, 3, 1, 1, 16), (2, 32, 7, 7, 32, 3, 1, 1, 32), (1, 16,
 
 
 @pytest.mark.parametrize("case", CASES)
-def test_against_the_oracle(g, oracle, case):
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_against_the_oracle(g, oracle, case, channels_last):
     N, C, H, W, OC, k, st, pad, group = case
     rng = np.random.default_rng(C + W)
     for xdt, ydt, xz, yz, rne, relu, bias_mode in [(np.uint8, np.uint8, 0, 0, False, True, 2), (np.uint8, np.uint8, 77, 9, False, True, 1),
@@ -24,8 +25,8 @@ def test_against_the_oracle(g, oracle, case):
         ys = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C // group * k * k) / 40)
         flags = (g.capi.ROUND_ONNX_RNE if rne else 0) | (g.capi.FUSE_RELU if relu else 0) | (g.capi.BIAS_ONNX_INT32 if bias_mode == 2 else 0)
         plan = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(OC, np.int8)), g.dev(bias) if bias_mode else None, strides=(st, st), pads=(pad, pad), group=group)
-        got = plan.run(g.dev(x), 0.02, xz, ys, yz, zero_point_dtype=torch.uint8 if ydt == np.uint8 else torch.int8, flags=flags)
-        assert got.is_contiguous()
+        got = plan.run(g.to_channels_last(g.dev(x)) if channels_last else g.dev(x), 0.02, xz, ys, yz, zero_point_dtype=torch.uint8 if ydt == np.uint8 else torch.int8, flags=flags)
+        assert channels_last or got.is_contiguous()
         okw = dict(bias=bias, bias_mode=oracle.BIAS_ONNX_INT32 if bias_mode == 2 else oracle.BIAS_REFERENCE_FLOAT) if bias_mode else {}
         want = oracle.qlinear_conv_int(x, 0.02, xz, w, ws, np.zeros(OC, np.int8), ys, yz, ydt, strides=(st, st), pads=(pad, pad), group=group,
                                        round_mode=oracle.ROUND_ONNX_RNE if rne else oracle.ROUND_REFERENCE, **okw)
