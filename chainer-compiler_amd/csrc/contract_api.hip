@@ -187,9 +187,11 @@ struct PackedWeights {
     int8_t* wd = nullptr;  // dense only: the same weights in the order of the planar-input kernel (inside wp's allocation)
 };
 
-// Dense packing pays when per-tap padding to 64 channels would at least double the K extent.
+// Dense packing pays when per-tap padding to 64 channels would at least double the K extent, and the channels do not fill
+// 16 bytes: from there on the pixels are read as they are and the zero products cost less than the expanded matrix
+// ([64, 16, 56, 56] with 16 3x3 filters: 45.3 us expanded, 16.9 this way).
 bool prefer_dense(int C, int KH, int KW) {
-    return KH * KW > 1 && round_up(C, 64) * KH * KW >= 2 * round_up(C * KH * KW, 64);
+    return C < 16 && KH * KW > 1 && round_up(C, 64) * KH * KW >= 2 * round_up(C * KH * KW, 64);
 }
 
 size_t packed_bytes(int OC, int C, int KH, int KW, PackedWeights* pw) {
