@@ -11,7 +11,9 @@ namespace {
 constexpr int kThreads = 256;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+// the same for views that start anywhere: one access each all the same
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32_u __attribute__((aligned(1)));
 
 // One 128-bit load and one 32-bit store per lane and step, kUnroll steps per thread at
 // a stride of one block, so that every access instruction of a wavefront covers one
@@ -22,15 +24,16 @@ constexpr int kUnroll = 4;
 // [64, 3, 224, 224]); four steps are 4 % faster on [64, 1024, 1024].
 constexpr int64_t kFewVectors = int64_t(1) << 22;
 
-template <bool kRne, int kSteps = kUnroll>
-__global__ __launch_bounds__(kThreads) void quantize_flat_kernel(
-        const v4f* __restrict__ x, uint32_t* __restrict__ y, int64_t n_vec, QuantParams qp) {
-    const int64_t first = (int64_t)blockIdx.x * (kThreads * kSteps) + threadIdx.x;
+// The up to three elements behind the last vector go with the thread that would have had the next one: a launch of their
+// own took 2 to 3 us of the 7 of a small tensor.
+template <bool kRne, int kSteps>
+__global__ __launch_bounds__(kThreads) void quantize_flat_kernel(const float* __restrict__ x, uint8_t* __restrict__ y, int64_t n, QuantParams qp) {
+    const int64_t first = (int64_t)blockIdx.x * (kThreads * kSteps) + threadIdx.x, n_vec = n / 4;
     v4f v[kSteps];
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
         const int64_t i = first + u * kThreads;
-        if (i < n_vec) v[u] = __builtin_nontemporal_load(x + i);
+        if (i < n_vec) v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4f_u*>(x) + i);
     }
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
@@ -38,18 +41,11 @@ __global__ __launch_bounds__(kThreads) void quantize_flat_kernel(
         if (i < n_vec) {
             const uint32_t out = pack4(quantize_value<kRne>(v[u].x, qp), quantize_value<kRne>(v[u].y, qp),
                                        quantize_value<kRne>(v[u].z, qp), quantize_value<kRne>(v[u].w, qp));
-            __builtin_nontemporal_store(out, y + i);
+            __builtin_nontemporal_store(out, reinterpret_cast<u32_u*>(y) + i);
+        } else if (i == n_vec) {
+            for (int64_t e = 4 * n_vec; e < n; ++e) y[e] = (uint8_t)quantize_value<kRne>(x[e], qp);
         }
     }
-}
-
-// Remainder elements and unaligned buffers: one element per thread.
-template <bool kRne>
-__global__ __launch_bounds__(kThreads) void quantize_scalar_kernel(
-        const float* __restrict__ x, uint8_t* __restrict__ y, int64_t begin, int64_t n, QuantParams qp) {
-    const int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    y[i] = (uint8_t)quantize_value<kRne>(x[i], qp);
 }
 
 __device__ __forceinline__ int64_t strided_offset(int64_t flat, const StridedDesc& d) {
@@ -83,30 +79,25 @@ __device__ __forceinline__ v4f dequant4(uint32_t w, float zpf, float scale) {
     return r;
 }
 
-template <bool kSigned>
-__global__ __launch_bounds__(kThreads) void dequantize_flat_kernel(
-        const uint32_t* __restrict__ x, v4f* __restrict__ y, int64_t n_vec, float zpf, float scale) {
-    const int64_t first = (int64_t)blockIdx.x * (kThreads * kUnroll) + threadIdx.x;
-    uint32_t q[kUnroll];
+template <bool kSigned, int kSteps>
+__global__ __launch_bounds__(kThreads) void dequantize_flat_kernel(const uint8_t* __restrict__ x, float* __restrict__ y, int64_t n, float zpf, float scale) {
+    const int64_t first = (int64_t)blockIdx.x * (kThreads * kSteps) + threadIdx.x, n_vec = n / 4;
+    uint32_t q[kSteps];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < kSteps; ++u) {
         const int64_t i = first + u * kThreads;
-        if (i < n_vec) q[u] = __builtin_nontemporal_load(x + i);
+        if (i < n_vec) q[u] = __builtin_nontemporal_load(reinterpret_cast<const u32_u*>(x) + i);
     }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < kSteps; ++u) {
         const int64_t i = first + u * kThreads;
-        if (i < n_vec) __builtin_nontemporal_store(dequant4<kSigned>(q[u], zpf, scale), y + i);
+        if (i < n_vec) {
+            const v4f v = dequant4<kSigned>(q[u], zpf, scale);
+            __builtin_nontemporal_store(v, reinterpret_cast<v4f_u*>(y) + i);
+        } else if (i == n_vec) {
+            for (int64_t e = 4 * n_vec; e < n; ++e) y[e] = dequantize_value(kSigned ? (int32_t)(int8_t)x[e] : (int32_t)x[e], zpf, scale);
+        }
     }
-}
-
-template <bool kSigned>
-__global__ __launch_bounds__(kThreads) void dequantize_scalar_kernel(
-        const uint8_t* __restrict__ x, float* __restrict__ y, int64_t begin, int64_t n, float zpf, float scale) {
-    const int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const int32_t q = kSigned ? (int32_t)(int8_t)x[i] : (int32_t)x[i];
-    y[i] = dequantize_value(q, zpf, scale);
 }
 
 template <bool kSigned>
@@ -124,8 +115,9 @@ inline unsigned blocks_for(int64_t n) {
     return (unsigned)((n + kThreads - 1) / kThreads);
 }
 
-inline unsigned flat_blocks_for(int64_t n_vec) {
-    return (unsigned)((n_vec + kThreads * kUnroll - 1) / (kThreads * kUnroll));
+inline unsigned flat_blocks_for(int64_t n, int steps) {
+    const int64_t threads = n / 4 + (n % 4 != 0 ? 1 : 0);
+    return (unsigned)((threads + kThreads * steps - 1) / (kThreads * steps));
 }
 
 StridedDesc make_desc(const chx_hip_tensor& t) {
@@ -164,29 +156,16 @@ extern "C" int chx_hip_quantize_linear(
     if (same_dense_layout(*x, *y)) {
         const float* xp = static_cast<const float*>(x->data);
         uint8_t* yp = static_cast<uint8_t*>(y->data);
-        int64_t n_vec = 0;
-        if (aligned(xp, 16) && aligned(yp, 16)) n_vec = n / 4;
-        if (n_vec > 0) {
-            const v4f* xv = reinterpret_cast<const v4f*>(xp);
-            uint32_t* yv = reinterpret_cast<uint32_t*>(yp);
-            if (n_vec <= kFewVectors) {
-                if (rne) quantize_flat_kernel<true, 1><<<blocks_for(n_vec), kThreads, 0, s>>>(xv, yv, n_vec, qp);
-                else quantize_flat_kernel<false, 1><<<blocks_for(n_vec), kThreads, 0, s>>>(xv, yv, n_vec, qp);
-            } else {
-                if (rne) quantize_flat_kernel<true><<<flat_blocks_for(n_vec), kThreads, 0, s>>>(xv, yv, n_vec, qp);
-                else quantize_flat_kernel<false><<<flat_blocks_for(n_vec), kThreads, 0, s>>>(xv, yv, n_vec, qp);
-            }
-            CHX_PROPAGATE(launch_check("quantize_flat_kernel"));
+#define CHX_QUANTIZE(RNE, STEPS) quantize_flat_kernel<RNE, STEPS><<<flat_blocks_for(n, STEPS), kThreads, 0, s>>>(xp, yp, n, qp)
+        if (n / 4 <= kFewVectors) {
+            if (rne) CHX_QUANTIZE(true, 1);
+            else CHX_QUANTIZE(false, 1);
+        } else {
+            if (rne) CHX_QUANTIZE(true, kUnroll);
+            else CHX_QUANTIZE(false, kUnroll);
         }
-        const int64_t done = n_vec * 4;
-        if (done < n) {
-            if (rne)
-                quantize_scalar_kernel<true><<<blocks_for(n - done), kThreads, 0, s>>>(xp, yp, done, n, qp);
-            else
-                quantize_scalar_kernel<false><<<blocks_for(n - done), kThreads, 0, s>>>(xp, yp, done, n, qp);
-            CHX_PROPAGATE(launch_check("quantize_scalar_kernel"));
-        }
-        return CHX_HIP_OK;
+#undef CHX_QUANTIZE
+        return launch_check("quantize_flat_kernel");
     }
     const StridedDesc xd = make_desc(*x), yd = make_desc(*y);
     if (rne)
@@ -215,26 +194,16 @@ extern "C" int chx_hip_dequantize_linear(
     if (same_dense_layout(*x, *y)) {
         const uint8_t* xp = static_cast<const uint8_t*>(x->data);
         float* yp = static_cast<float*>(y->data);
-        int64_t n_vec = 0;
-        if (aligned(xp, 16) && aligned(yp, 16)) n_vec = n / 4;
-        if (n_vec > 0) {
-            if (i8)
-                dequantize_flat_kernel<true><<<flat_blocks_for(n_vec), kThreads, 0, s>>>(
-                        reinterpret_cast<const uint32_t*>(xp), reinterpret_cast<v4f*>(yp), n_vec, zpf, x_scale);
-            else
-                dequantize_flat_kernel<false><<<flat_blocks_for(n_vec), kThreads, 0, s>>>(
-                        reinterpret_cast<const uint32_t*>(xp), reinterpret_cast<v4f*>(yp), n_vec, zpf, x_scale);
-            CHX_PROPAGATE(launch_check("dequantize_flat_kernel"));
+#define CHX_DEQUANTIZE(SIGNED, STEPS) dequantize_flat_kernel<SIGNED, STEPS><<<flat_blocks_for(n, STEPS), kThreads, 0, s>>>(xp, yp, n, zpf, x_scale)
+        if (n / 4 <= kFewVectors) {
+            if (i8) CHX_DEQUANTIZE(true, 1);
+            else CHX_DEQUANTIZE(false, 1);
+        } else {
+            if (i8) CHX_DEQUANTIZE(true, kUnroll);
+            else CHX_DEQUANTIZE(false, kUnroll);
         }
-        const int64_t done = n_vec * 4;
-        if (done < n) {
-            if (i8)
-                dequantize_scalar_kernel<true><<<blocks_for(n - done), kThreads, 0, s>>>(xp, yp, done, n, zpf, x_scale);
-            else
-                dequantize_scalar_kernel<false><<<blocks_for(n - done), kThreads, 0, s>>>(xp, yp, done, n, zpf, x_scale);
-            CHX_PROPAGATE(launch_check("dequantize_scalar_kernel"));
-        }
-        return CHX_HIP_OK;
+#undef CHX_DEQUANTIZE
+        return launch_check("dequantize_flat_kernel");
     }
     const StridedDesc xd = make_desc(*x), yd = make_desc(*y);
     if (i8)
