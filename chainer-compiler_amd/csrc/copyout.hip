@@ -53,7 +53,23 @@ __global__ __launch_bounds__(kThreads) void copy_out_kernel(CopyOutArgs a) {
 }  // namespace
 }  // namespace chx
 
+namespace chx {
+namespace {
+
+// Pinned memory comes in slabs of four blocks: an allocation takes 50 us, which every program that sends results to the
+// host, and every reader of a small array, would pay.
+struct Slab {
+    char* pinned = nullptr;
+    uint32_t* arrived = nullptr;
+    int blocks = 0;  // of it that exist, in use or waiting
+};
+constexpr int kSlabBlocks = 4;
+
+}  // namespace
+}  // namespace chx
+
 struct chx_hip_copyout {
+    chx::Slab* slab = nullptr;
     char* pinned = nullptr;  // the results, and behind them the flag
     uint32_t* arrived = nullptr;
     size_t capacity = 0;
@@ -71,10 +87,30 @@ std::atomic<uint32_t>* flag_of(const chx_hip_copyout* c) {
     return reinterpret_cast<std::atomic<uint32_t>*>(c->pinned + c->capacity);
 }
 
-// Blocks of chx_hip_memcpy_d2h, handed out to one caller at a time; at most kKept stay allocated between calls.
-constexpr size_t kKept = 4;
+// Blocks that nobody uses, at most kKept of them.
+constexpr size_t kKept = 2 * kSlabBlocks, kBlockBytes = kMostBytes + 16 * kMaxRanges + 64;
 std::mutex g_mutex;
 std::vector<chx_hip_copyout*> g_free;
+
+// (g_mutex held)
+void drop(chx_hip_copyout* c) {
+    if (--c->slab->blocks == 0) {
+        if (c->slab->arrived) (void)hipFree(c->slab->arrived);
+        if (c->slab->pinned) (void)hipHostFree(c->slab->pinned);
+        delete c->slab;
+    }
+    delete c;
+}
+
+chx_hip_copyout* take(int device) {
+    for (size_t i = 0; i < g_free.size(); ++i) {
+        if (g_free[i]->device != device) continue;
+        chx_hip_copyout* c = g_free[i];
+        g_free.erase(g_free.begin() + (long)i);
+        return c;
+    }
+    return nullptr;
+}
 
 }  // namespace
 
@@ -82,27 +118,10 @@ std::vector<chx_hip_copyout*> g_free;
 bool small_copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s, int* rc) {
     if (bytes > kMostBytes || stream_is_capturing(s)) return false;
     chx_hip_copyout* c = nullptr;
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return false;
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        for (size_t i = 0; i < g_free.size() && !c; ++i) {
-            if (g_free[i]->device != device) continue;
-            c = g_free[i];
-            g_free.erase(g_free.begin() + (long)i);
-        }
-    }
-    if (!c && chx_hip_copyout_create(kMostBytes, &c) != CHX_HIP_OK) return false;
+    if (chx_hip_copyout_create(kMostBytes, &c) != CHX_HIP_OK) return false;
     *rc = chx_hip_copyout_enqueue(c, &src, &bytes, 1, s);
     if (*rc == CHX_HIP_OK) *rc = chx_hip_copyout_wait(c);
     if (*rc == CHX_HIP_OK) memcpy(dst, chx_hip_copyout_data(c, 0), bytes);
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if (*rc == CHX_HIP_OK && g_free.size() < kKept) {
-            g_free.push_back(c);
-            return true;
-        }
-    }
     chx_hip_copyout_destroy(c);
     return true;
 }
@@ -115,25 +134,36 @@ extern "C" int chx_hip_copyout_create(size_t bytes, chx_hip_copyout** out) {
     CHX_REQUIRE(out != nullptr, "copyout: null output");
     *out = nullptr;
     if (bytes > kMostBytes) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "copyout: %zu bytes are more than the %zu of this path", bytes, kMostBytes);
-    chx_hip_copyout* c = new chx_hip_copyout();
-    c->capacity = (bytes + 16 * kMaxRanges + 63) / 64 * 64;
-    void *p = nullptr, *d = nullptr;
-    hipError_t e = hipGetDevice(&c->device);
-    if (e == hipSuccess) e = hipHostMalloc(&p, c->capacity + 64, hipHostMallocDefault);
-    if (e == hipSuccess) {
-        c->pinned = static_cast<char*>(p);
-        memset(c->pinned + c->capacity, 0, 64);
-        e = hipMalloc(&d, 64);
-    }
-    if (e == hipSuccess) {
-        c->arrived = static_cast<uint32_t*>(d);
-        const uint32_t zero = 0;
-        e = hipMemcpy(d, &zero, sizeof(zero), hipMemcpyHostToDevice);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        chx_hip_copyout_destroy(c);
-        CHX_FAIL(CHX_HIP_ERUNTIME, "copyout: allocation failed: %s", hipGetErrorString(e));
+    int device = 0;
+    CHX_HIP_CALL(hipGetDevice(&device));
+    std::lock_guard<std::mutex> lock(g_mutex);
+    chx_hip_copyout* c = take(device);
+    if (!c) {
+        void *p = nullptr, *d = nullptr;
+        hipError_t e = hipHostMalloc(&p, kSlabBlocks * (kBlockBytes + 64), hipHostMallocDefault);
+        if (e == hipSuccess) e = hipMalloc(&d, kSlabBlocks * 64);
+        if (e == hipSuccess) {
+            const uint32_t zeros[kSlabBlocks * 16] = {};
+            e = hipMemcpy(d, zeros, sizeof(zeros), hipMemcpyHostToDevice);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            if (d) (void)hipFree(d);
+            if (p) (void)hipHostFree(p);
+            CHX_FAIL(CHX_HIP_ERUNTIME, "copyout: allocation failed: %s", hipGetErrorString(e));
+        }
+        Slab* slab = new Slab{static_cast<char*>(p), static_cast<uint32_t*>(d), kSlabBlocks};
+        for (int i = 0; i < kSlabBlocks; ++i) {
+            chx_hip_copyout* b = new chx_hip_copyout();
+            b->slab = slab;
+            b->capacity = kBlockBytes;
+            b->pinned = slab->pinned + i * (kBlockBytes + 64);
+            memset(b->pinned + kBlockBytes, 0, 64);
+            b->arrived = slab->arrived + 16 * i;
+            b->device = device;
+            g_free.push_back(b);
+        }
+        c = take(device);
     }
     *out = c;
     return CHX_HIP_OK;
@@ -192,7 +222,8 @@ extern "C" const void* chx_hip_copyout_data(const chx_hip_copyout* c, int32_t i)
 extern "C" void chx_hip_copyout_destroy(chx_hip_copyout* c) {
     if (!c) return;
     if (c->pending) (void)hipStreamSynchronize(c->stream);
-    if (c->arrived) (void)hipFree(c->arrived);
-    if (c->pinned) (void)hipHostFree(c->pinned);
-    delete c;
+    c->pending = false;
+    std::lock_guard<std::mutex> lock(g_mutex);
+    if (g_free.size() < kKept) g_free.push_back(c);
+    else drop(c);
 }

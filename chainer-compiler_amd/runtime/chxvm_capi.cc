@@ -54,7 +54,13 @@ public:
     HostResults(const HostResults&) = delete;
     HostResults& operator=(const HostResults&) = delete;
     ~HostResults() {
+        Drop();
+    }
+    void Drop() {
         chx_hip_copyout_destroy(copy_);
+        copy_ = nullptr;
+        capacity_ = 0;
+        valid_ = false;
     }
     // false: these results are not for this path
     bool Enqueue(const std::vector<chainerx::Array>& arrays, void* stream) {
@@ -144,6 +150,7 @@ struct chxvm_replay {
         for (chx_hip_qconv_plan* plan : pinned_plans) (void)chx_hip_qconv_plan_pin(plan, -1);
         outputs.arrays.clear();
         outputs.keep_inputs.clear();
+        results.Drop();  // (waits for a copy still on the stream)
         if (stream) (void)chx_hip_stream_destroy(stream);
     }
 };
