@@ -47,7 +47,7 @@ void SetLastError(const std::string& message) {
 namespace {
 
 // Host copies of a run's results, when they are few bytes (chx_hip_copyout): queued behind the run, so that waiting for
-// the run and fetching its results is one wait.
+// the run and fetching its results is one wait.  One run's (or one replay's): not for several threads at once.
 class HostResults {
 public:
     HostResults() = default;
@@ -112,7 +112,6 @@ private:
 struct chxvm_program {
     std::unique_ptr<ChxVM> vm;
     int onnx_int32_bias = -1;  // -1: the process default at the time of a run
-    HostResults results;       // of chxvm_program_run_to_host
 
     chxvm_program() {
         DeviceCache::Get().AddProgram();
@@ -263,11 +262,11 @@ int32_t RunProgram(
         }
         o->keep_inputs = in;
         // the run ends with the device done (tools/run_onnx.cc:462)
-        HostResults* host = to_host ? &program->results : nullptr;
-        if (host && host->Enqueue(o->arrays, nullptr)) {
-            host->Wait();
+        HostResults host;  // this run's: several threads may run one program (the library keeps the blocks of pinned memory)
+        if (to_host && host.Enqueue(o->arrays, nullptr)) {
+            host.Wait();
             for (size_t i = 0; i < o->arrays.size(); ++i) {
-                const char* p = static_cast<const char*>(host->data(static_cast<int32_t>(i)));
+                const char* p = static_cast<const char*>(host.data(static_cast<int32_t>(i)));
                 o->host.emplace_back(p, p + o->arrays[i].GetNBytes());
             }
         } else {

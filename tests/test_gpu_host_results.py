@@ -80,3 +80,24 @@ def test_replay_results_follow_every_launch(g, vm, elements, own_stream):
             out = replay.outputs()
             assert (out["y"] == max(2 * (i - 2.0), 0)).all() and (out["z"] == max(2 * (i - 2.0), 0) + i - 2.0).all()
     replay.close()
+
+
+def test_threads_running_one_program_get_their_own_results(g, vm):
+    import threading
+    prog, wrong = scaling_program(g, vm, (3000,)), []
+
+    def work(k):
+        x = np.full(3000, float(k), np.float32)
+        xd = g.dev(x)
+        torch.cuda.synchronize()
+        for _ in range(200):
+            out = prog.run({"x": xd})
+            if not ((out["y"] == 2 * k).all() and (out["z"] == 3 * k).all()):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(1, 5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

@@ -1,0 +1,74 @@
+"""Results on the host (runtime/chxvm_capi.cc, csrc/copyout.hip) and the memory eager runs reuse, without a GPU."""
+import ctypes
+import os
+import sys
+import threading
+import time
+
+import pytest
+
+import host_hip
+
+
+@pytest.fixture(scope="module")
+def host_so(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host_hip"))
+
+
+@pytest.mark.parametrize("case", ["two_threads_of_one_program"])
+def test_case(host_so, case):
+    host_hip.run_case(host_so, __file__, case)
+
+
+def run_to_host(host, program, inputs):
+    rt = host.chxvm.runtime()
+    out = ctypes.c_void_p()
+    assert rt.chxvm_program_run_to_host(program, *host.names_and(inputs), 0, ctypes.byref(out)) == 0, rt.chxvm_last_error()
+    return out
+
+
+def host_copy(host, out, i, nbytes):
+    p = host.chxvm.runtime().chxvm_outputs_host(out, i)
+    return ctypes.string_at(p, nbytes) if p else None
+
+
+def copying_program(host):
+    b = host.chxvm.ProgramBuilder()
+    b.output("y", b.input("x", "uint8", [64]))
+    return host.program(b)
+
+
+def wait_until(condition):
+    end = time.time() + 20
+    while not condition():
+        assert time.time() < end
+        time.sleep(0.001)
+
+
+def two_threads_of_one_program(host):
+    """One thread's run waits for its results while another thread's run of the same program starts and ends."""
+    program, got = copying_program(host), {}
+
+    def run(name):
+        x = host.tensor("uint8", (64,))
+        host.bytes(x.data, bytes([ord(name)]) * 64)
+        out = run_to_host(host, program, {"x": x})
+        got[name] = host_copy(host, out, 0, 64)
+        host.chxvm.runtime().chxvm_outputs_destroy(out)
+
+    for size in range(3):  # (also with blocks that earlier runs have left)
+        host.hh.hh_hold(1)
+        a = threading.Thread(target=run, args="a")
+        a.start()
+        wait_until(lambda: host.hh.hh_held() >= 1)
+        b = threading.Thread(target=run, args="b")
+        b.start()
+        b.join(20)
+        assert not b.is_alive()
+        host.hh.hh_release()
+        a.join(20)
+        assert got == {"a": b"a" * 64, "b": b"b" * 64}
+
+
+if __name__ == "__main__":
+    host_hip.main(globals())
