@@ -28,7 +28,7 @@ STORE_MINUS_128 = 8
 EINVAL, EUNSUPPORTED, ERUNTIME = 1, 2, 3
 
 EXPORTS = [
-    "chx_hip_init", "chx_hip_last_error", "chx_hip_version", "chx_hip_get_device_props", "chx_hip_malloc",
+    "chx_hip_init", "chx_hip_last_error", "chx_hip_version", "chx_hip_get_device", "chx_hip_get_device_props", "chx_hip_malloc",
     "chx_hip_free", "chx_hip_memcpy_h2d", "chx_hip_memcpy_d2h", "chx_hip_memset", "chx_hip_stream_synchronize", "chx_hip_device_synchronize",
     "chx_hip_copyout_create", "chx_hip_copyout_enqueue", "chx_hip_copyout_wait", "chx_hip_copyout_data", "chx_hip_copyout_destroy",
     "chx_hip_quantize_linear", "chx_hip_dequantize_linear", "chx_hip_qlinear_conv", "chx_hip_qlinear_conv_nd", "chx_hip_conv_integer_nd", "chx_hip_qconv_plan_create",

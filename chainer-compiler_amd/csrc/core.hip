@@ -272,6 +272,14 @@ int chx_hip_init(int device) {
     return prepare_noalloc_scratch();
 }
 
+int chx_hip_get_device(int32_t* device) {
+    CHX_REQUIRE(device != nullptr, "null output");
+    int d = 0;
+    CHX_HIP_CALL(hipGetDevice(&d));
+    *device = d;
+    return CHX_HIP_OK;
+}
+
 int chx_hip_get_device_props(chx_hip_device_props* out) {
     CHX_REQUIRE(out != nullptr, "null output");
     int dev = 0;

@@ -12,6 +12,12 @@ size_t SizeClass(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
+int32_t CurrentDevice() {
+    int32_t device = 0;
+    CHXVM_HIP_CALL(chx_hip_get_device(&device));
+    return device;
+}
+
 }  // namespace
 
 DeviceCache& DeviceCache::Get() {
@@ -21,10 +27,11 @@ DeviceCache& DeviceCache::Get() {
 
 std::shared_ptr<void> DeviceCache::Allocate(size_t bytes) {
     const size_t size = SizeClass(bytes);
+    const int32_t device = CurrentDevice();
     void* p = nullptr;
     {
         std::lock_guard<std::mutex> lock(mu_);
-        auto it = free_.find(size);
+        auto it = free_.find({device, size});
         if (it != free_.end() && !it->second.empty()) {
             p = it->second.back();
             it->second.pop_back();
@@ -35,14 +42,18 @@ std::shared_ptr<void> DeviceCache::Allocate(size_t bytes) {
         Trim();  // what is kept may be what is missing
         CHXVM_HIP_CALL(chx_hip_malloc(&p, size));
     }
-    return std::shared_ptr<void>(p, [this, size](void* q) { Release(q, size); });
+    return std::shared_ptr<void>(p, [this, size, device](void* q) { Release(q, size, device); });
 }
 
-void DeviceCache::Release(void* p, size_t size) {
+void DeviceCache::Release(void* p, size_t size, int32_t device) {
+    // (what is given up while another device is current goes back to the device runtime: the owner has waited for that
+    // other device, hipFree waits for this one)
+    int32_t current = -1;
+    (void)chx_hip_get_device(&current);
     {
         std::lock_guard<std::mutex> lock(mu_);
-        if (programs_ > 0 && size <= kLargestKept && cached_ + size <= kMostCached) {
-            free_[size].push_back(p);
+        if (device == current && programs_ > 0 && size <= kLargestKept && cached_ + size <= kMostCached) {
+            free_[{device, size}].push_back(p);
             cached_ += size;
             return;
         }
@@ -51,7 +62,7 @@ void DeviceCache::Release(void* p, size_t size) {
 }
 
 void DeviceCache::Trim() {
-    std::map<size_t, std::vector<void*>> blocks;
+    std::map<std::pair<int32_t, size_t>, std::vector<void*>> blocks;
     {
         std::lock_guard<std::mutex> lock(mu_);
         blocks.swap(free_);

@@ -1,7 +1,7 @@
 // Device memory of eager runs.  hipFree waits for all work on the device: a run that frees every value after its last
 // reader (as programs do) stopped the host after each instruction, 60 times in a ResNet-50, and the device idled while
 // the host caught up (2.3 ms for a batch of 8 whose kernels take 0.4).  Blocks released by one value are kept for the
-// next request of their size class instead.
+// next request of their size class on the same device instead.
 //
 // All users are eager runs, whose work goes to the null stream: a block handed out again is written only behind the work
 // that still reads it.  Memory that leaves a run (outputs, a program's constants) comes back after the device has been
@@ -10,6 +10,7 @@
 
 #include <map>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "chainerx_lite.h"
@@ -29,13 +30,13 @@ public:
 
 private:
     DeviceCache() = default;
-    void Release(void* p, size_t size);
+    void Release(void* p, size_t size, int32_t device);
 
     static constexpr size_t kMostCached = size_t(1) << 30;    // bytes kept beyond those in use
     static constexpr size_t kLargestKept = size_t(256) << 20;  // larger blocks are not kept
 
     std::mutex mu_;
-    std::map<size_t, std::vector<void*>> free_;  // by size class
+    std::map<std::pair<int32_t, size_t>, std::vector<void*>> free_;  // by device and size class
     size_t cached_ = 0;
     int64_t programs_ = 0;
 };

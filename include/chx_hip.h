@@ -122,6 +122,7 @@ typedef struct chx_hip_device_props {
  * Replaces nothing in the reference (ChainerX owns device selection there,
  * tools/run_onnx.cc:343-357). */
 int chx_hip_init(int device);
+int chx_hip_get_device(int32_t* device); /* the calling thread's */
 const char* chx_hip_last_error(void);
 const char* chx_hip_version(void);
 int chx_hip_get_device_props(chx_hip_device_props* out);

@@ -15,7 +15,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["two_threads_of_one_program"])
+@pytest.mark.parametrize("case", ["two_threads_of_one_program", "memory_of_each_device"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -68,6 +68,30 @@ def two_threads_of_one_program(host):
         host.hh.hh_release()
         a.join(20)
         assert got == {"a": b"a" * 64, "b": b"b" * 64}
+
+
+def memory_of_each_device(host):
+    """Runs on two devices in turn: every array lies on the device of its run, whatever earlier runs have left."""
+    rt, b = host.chxvm.runtime(), host.chxvm.ProgramBuilder()
+    x = b.input("x", "float32", [64])
+    t = b.QuantizeLinear(x, b.scalar(0.5, "float32"), b.scalar(3, "uint8"))
+    b.output("y", b.DequantizeLinear(t, b.scalar(0.25, "float32"), b.scalar(3, "uint8")))
+    b.Free(t)
+    program, held = host.program(b), []
+    for device in (0, 1, 1, 0, 1):
+        host.check(host.lib.chx_hip_init(device))
+        x = host.tensor("float32", (64,))
+        out, y = ctypes.c_void_p(), host.capi.Tensor()
+        assert rt.chxvm_program_run(program, *host.names_and({"x": x}), 0, ctypes.byref(out)) == 0, rt.chxvm_last_error()
+        assert rt.chxvm_outputs_get(out, 0, ctypes.byref(y)) == 0
+        assert host.device_of(y.data) == device
+        held.append((device, out, y.data))
+        if len(held) == 2:
+            # given up while the other device is current: waiting for that one would not do, so the block is not kept
+            device, out, data = held.pop(0)
+            host.check(host.lib.chx_hip_init(1 - device))
+            rt.chxvm_outputs_destroy(out)
+            assert host.device_of(data) == -2
 
 
 if __name__ == "__main__":
