@@ -102,6 +102,29 @@ void drop(chx_hip_copyout* c) {
     delete c;
 }
 
+// Whether a kernel on `device`, the current one, may read p.  Another device's memory, pinned and pageable host memory are
+// hipMemcpy's.
+bool memory_of(int device, const void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == device;
+}
+
+bool stream_of(int device, hipStream_t s) {
+    int current = 0;
+    if (hipGetDevice(&current) != hipSuccess || current != device) return false;
+    if (s == nullptr) return true;
+    hipDevice_t of_stream = 0;
+    if (hipStreamGetDevice(s, &of_stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return of_stream == device;
+}
+
 chx_hip_copyout* take(int device) {
     for (size_t i = 0; i < g_free.size(); ++i) {
         if (g_free[i]->device != device) continue;
@@ -120,6 +143,10 @@ bool small_copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s,
     chx_hip_copyout* c = nullptr;
     if (chx_hip_copyout_create(kMostBytes, &c) != CHX_HIP_OK) return false;
     *rc = chx_hip_copyout_enqueue(c, &src, &bytes, 1, s);
+    if (*rc == CHX_HIP_EUNSUPPORTED) {
+        chx_hip_copyout_destroy(c);
+        return false;
+    }
     if (*rc == CHX_HIP_OK) *rc = chx_hip_copyout_wait(c);
     if (*rc == CHX_HIP_OK) memcpy(dst, chx_hip_copyout_data(c, 0), bytes);
     chx_hip_copyout_destroy(c);
@@ -172,6 +199,9 @@ extern "C" int chx_hip_copyout_create(size_t bytes, chx_hip_copyout** out) {
 extern "C" int chx_hip_copyout_enqueue(chx_hip_copyout* c, const void* const* src, const size_t* bytes, int32_t n, void* stream) {
     CHX_REQUIRE(c != nullptr && n >= 0 && (n == 0 || (src != nullptr && bytes != nullptr)), "copyout: null argument");
     if (n > kMaxRanges) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "copyout: %d ranges, at most %d", n, kMaxRanges);
+    if (!stream_of(c->device, as_stream(stream))) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "copyout: the stream belongs to another device than the block");
+    for (int i = 0; i < n; ++i)
+        if (bytes[i] && !memory_of(c->device, src[i])) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "copyout: range %d is not memory of the block's device", i);
     if (c->pending) CHX_PROPAGATE(chx_hip_copyout_wait(c));
     CopyOutArgs a;
     memset(&a, 0, sizeof(a));

@@ -82,7 +82,9 @@ public:
             if (chx_hip_copyout_create(total, &copy_) != 0) return false;
             capacity_ = total;
         }
-        CHXVM_HIP_CALL(chx_hip_copyout_enqueue(copy_, src, bytes, static_cast<int32_t>(arrays.size()), stream));
+        const int rc = chx_hip_copyout_enqueue(copy_, src, bytes, static_cast<int32_t>(arrays.size()), stream);
+        if (rc == CHX_HIP_EUNSUPPORTED) return false;  // (an input that lies elsewhere and is an output, another device's replay)
+        CHXVM_HIP_CALL(rc);
         valid_ = true;
         return true;
     }

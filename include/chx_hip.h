@@ -137,7 +137,8 @@ int chx_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream); 
 
 /* Small device results for the host: enqueue() queues the copy of up to 8 ranges (512 KB together) behind the work of
  * `stream`, wait() returns when they are in host memory, data() is where range i of the last enqueue lies until the next
- * one.  One object serves one copy at a time. */
+ * one.  One object serves one copy at a time, on the device that was current when it was created: ranges that are not
+ * memory of that device, and other devices' streams, are refused with CHX_HIP_EUNSUPPORTED. */
 typedef struct chx_hip_copyout chx_hip_copyout;
 int chx_hip_copyout_create(size_t bytes, chx_hip_copyout** out);
 int chx_hip_copyout_enqueue(chx_hip_copyout* copyout, const void* const* src, const size_t* bytes, int32_t n, void* stream);

@@ -15,7 +15,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["two_threads_of_one_program", "memory_of_each_device"])
+@pytest.mark.parametrize("case", ["two_threads_of_one_program", "memory_of_each_device", "sources_of_the_result_copy"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -92,6 +92,40 @@ def memory_of_each_device(host):
             host.check(host.lib.chx_hip_init(1 - device))
             rt.chxvm_outputs_destroy(out)
             assert host.device_of(data) == -2
+
+
+def sources_of_the_result_copy(host):
+    """The kernel that copies results reads memory of its own device only: every other source is the runtime's copy, as it
+    was before there was the kernel."""
+    lib, n = host.lib, 1000
+    here = host.malloc(n)
+    host.check(lib.chx_hip_init(1))
+    there, stream_there = host.malloc(n), host.stream()
+    host.check(lib.chx_hip_init(0))
+    pinned, elsewhere = ctypes.c_void_p(), ctypes.create_string_buffer(n)
+    assert host.hh.hipHostMalloc(ctypes.byref(pinned), ctypes.c_size_t(n), 0) == 0
+    pageable = ctypes.addressof(elsewhere)
+    got = ctypes.create_string_buffer(n)
+    for src, stream, kernel in [(here, None, True), (there, None, False), (pinned.value, None, False), (pageable, None, False), (here, stream_there, False),
+                                (there, stream_there, False)]:
+        host.clear()
+        host.bytes(src, bytes(range(250)) * 4)
+        ctypes.memset(got, 0, n)
+        host.check(lib.chx_hip_memcpy_d2h(got, ctypes.c_void_p(src), ctypes.c_size_t(n), stream))
+        assert got.raw == bytes(range(250)) * 4
+        assert any("copy_out_kernel" in k for k in host.launches()) == kernel, (src, stream)
+    # a program whose output is its input, wherever that lies
+    rt, program = host.chxvm.runtime(), copying_program(host)
+    for src in (here, there, pinned.value, pageable):
+        out = run_to_host(host, program, {"x": host.tensor("uint8", (64,), base=src)})
+        assert (host_copy(host, out, 0, 64) is not None) == (src == here)
+        rt.chxvm_outputs_destroy(out)
+    # a block of device 0 does not serve device 1's launches
+    block = ctypes.c_void_p()
+    host.check(lib.chx_hip_copyout_create(ctypes.c_size_t(64), ctypes.byref(block)))
+    host.check(lib.chx_hip_init(1))
+    rc = lib.chx_hip_copyout_enqueue(block, (ctypes.c_void_p * 1)(there), (ctypes.c_size_t * 1)(64), 1, None)
+    assert rc == host.capi.EUNSUPPORTED
 
 
 if __name__ == "__main__":
