@@ -287,6 +287,7 @@ void pick_tile(const LaunchOptions& opt, const ConvMfmaArgs& a, bool out_int32, 
 struct TunedConfig {
     int64_t M;
     int32_t H, W, OH, OW;
+    int64_t x_n_stride, x_h_stride, x_w_stride;  // a kernel may take a dense image only (conv_point_takes)
     int tile_oc, tile_px, max_wgs_per_cu;
     int waves;      // wavefronts per work-group
     bool with_res;  // measured with a fused residual sum (an entry of its own: the epilogue differs)
@@ -304,13 +305,13 @@ struct Configuration {
 // convolutions, and a second program over the same shapes finds all of them measured.
 class MeasuredConfigurations {
 public:
-    using Key = std::array<int64_t, 24>;
+    using Key = std::array<int64_t, 25>;
     static Key key(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne) {
         int device = 0;
         (void)hipGetDevice(&device);
         const int64_t res = a.res.r ? 1 + a.res.affine : 0;
         return {device, a.M, a.H, a.W, a.OH, a.OW, a.KH, a.KW, a.sh, a.sw, a.ph, a.pw, a.C16, a.KP, a.bk, a.OC, a.oc_split, a.x_n_stride,
-                a.x_w_stride, a.y_px_stride, aligned(a.y, 16), res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
+                a.x_h_stride, a.x_w_stride, a.y_px_stride, aligned(a.y, 16), res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
     }
     bool find(const Key& k, Configuration* c) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -734,7 +735,9 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     const TunedConfig* tuned = nullptr;
     if (c.tune) {
         for (const TunedConfig& t : c.tune->entries)
-            if (t.M == a.M && t.H == a.H && t.W == a.W && t.OH == a.OH && t.OW == a.OW && t.with_res == (c.res != nullptr) && t.oc_split == a.oc_split) tuned = &t;
+            if (t.M == a.M && t.H == a.H && t.W == a.W && t.OH == a.OH && t.OW == a.OW && t.x_n_stride == a.x_n_stride && t.x_h_stride == a.x_h_stride &&
+                t.x_w_stride == a.x_w_stride && t.with_res == (c.res != nullptr) && t.oc_split == a.oc_split)
+                tuned = &t;
         if (!tuned && c.opt.autotune && !stream_is_capturing(s)) {
             const MeasuredConfigurations::Key key = MeasuredConfigurations::key(a, xu, c.out_int32, c.rne);
             Configuration best;
@@ -743,7 +746,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
                 if (rc == CHX_HIP_OK) measured_configurations().add(key, best);
             }
             if (rc == CHX_HIP_OK) {
-                c.tune->entries.push_back({a.M, a.H, a.W, a.OH, a.OW, best.tile_oc, best.tile_px, best.max_wgs_per_cu, best.waves, c.res != nullptr, a.oc_split});
+                c.tune->entries.push_back({a.M, a.H, a.W, a.OH, a.OW, a.x_n_stride, a.x_h_stride, a.x_w_stride, best.tile_oc, best.tile_px, best.max_wgs_per_cu, best.waves, c.res != nullptr, a.oc_split});
                 tuned = &c.tune->entries.back();
             }
         }

@@ -38,6 +38,26 @@ def test_plain(g, oracle, case):
         np.testing.assert_array_equal(got[0][-1:, :, -2:], np.maximum(want, yz) if relu else want)
 
 
+@pytest.mark.parametrize("dense_first", [True, False])
+def test_one_plan_on_a_dense_image_and_on_crops(g, oracle, dense_first):
+    """The configuration measured on a dense image is not the crop's (nothing forced)."""
+    rng = np.random.default_rng(7)
+    N, C, H, W, OC = 16, 64, 32, 32, 64
+    big, w = codes(rng, (N, C, 36, 40), np.uint8), codes(rng, (OC, C, 1, 1), np.int8)
+    ws = rng.uniform(0.002, 0.02, size=OC).astype(np.float32)
+    ys = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C) / 40)
+    plan = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(OC, np.int8)), None)
+    bd = g.to_channels_last(g.dev(big))
+    views = [(g.to_channels_last(g.dev(big[:, :, :H, :W])), big[:, :, :H, :W]), (bd[:, :, :H, :W], big[:, :, :H, :W]), (bd[:, :, 4:, 8:], big[:, :, 4:, 8:])]
+    if not dense_first:
+        views.reverse()
+    for xd, x in views + views:
+        got = g.host(plan.run(xd, 0.02, 128, ys, 128))
+        want = oracle.qlinear_conv_int(x[-1:], 0.02, 128, w, ws, np.zeros(OC, np.int8), ys, 128, np.uint8)
+        np.testing.assert_array_equal(got[-1:], want)
+    plan.close()
+
+
 @pytest.mark.parametrize("affine", ["1", "0"])
 @pytest.mark.parametrize("minus_128", [False, True])
 @pytest.mark.parametrize("C,OC", [(48, 40), (200, 72)])
