@@ -560,6 +560,23 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
                       stem_patch_fits(cs.C, cs.KH, cs.KW, sh, sw) && ph < 64 && pw_ < 64 &&
                       (int64_t)cs.C * (x.strides[1] < 0 ? -x.strides[1] : x.strides[1]) < (int64_t(1) << 30) &&
                       x.strides[2] > 0 && (int64_t)cs.H * x.strides[2] < (int64_t(1) << 30) && c.opt.stem_kernel;
+    // Channels-last pixels at another pitch than 16 bytes (40 channels packed, say) are copied to one.  The copy's memory is
+    // this call's and not the plan's: the direct kernel, which has always taken such arrays, lets one plan run on two streams
+    // and inside a recording, pinned or not, and needs none.  A recording keeps that kernel (its memory would have to
+    // outlive the call), and so does a pair, which is refused here.
+    const bool pixels_copied = !stem && !pw.dense && !x_is_mfma_ready(x) && !is_contiguous(x) && x.strides[1] == 1;
+    ScratchCache own;
+    Scratch own_memory;
+    ScratchCache* cache = pixels_copied ? &own : c.cache;
+    if (pixels_copied) {
+        if (c.y2 || stream_is_capturing(s)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv: packed pixels are not copied for a pair or inside a recording");
+        int64_t y_px = 0;
+        own.size[0] = ((size_t)cs.N * cs.H * cs.W * C16 + 255) / 256 * 256;
+        own.size[1] = y_is_pixel_major(y, &y_px) ? 0 : (size_t)cs.N * cs.OH * cs.OW * round_up(cs.OC, 16);
+        CHX_PROPAGATE(own_memory.acquire(own.size[0] + own.size[1], s));
+        own.ptr[0] = own_memory.ptr();
+        own.ptr[1] = static_cast<char*>(own_memory.ptr()) + own.size[0];
+    }
     if (stem && c.res) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "the planar-input kernel has no fused residual sum");
     if (stem) {
         // x is used in place
@@ -567,7 +584,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         // explicit im2col: [M][Kd] bytes, then a 1x1 convolution over Kd channels and M pixels in a row
         const int64_t M = (int64_t)cs.N * cs.OH * cs.OW;
         CHX_REQUIRE(M <= INT32_MAX, "QLinearConv: too many output pixels for the im2col path");
-        CHX_PROPAGATE(acquire_scratch(c.cache, 0, (size_t)M * pw.KP, s, &x_scratch));
+        CHX_PROPAGATE(acquire_scratch(cache, 0, (size_t)M * pw.KP, s, &x_scratch));
         Im2colArgs ia;
         memset(&ia, 0, sizeof(ia));
         ia.x = static_cast<const char*>(x.data);
@@ -580,7 +597,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         ia.col = static_cast<char*>(x_scratch);
         const int rc = launch_im2col_dense(ia, s);
         if (rc != CHX_HIP_OK) {
-            release_scratch(c.cache, x_scratch, s);
+            release_scratch(cache, x_scratch, s);
             return rc;
         }
         a.x = static_cast<const char*>(x_scratch);
@@ -594,14 +611,13 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         a.x_n_stride = x.strides[0];
         a.x_h_stride = x.strides[2];
         a.x_w_stride = x.strides[3];
-    } else if (is_contiguous(x) || x.strides[1] == 1) {
-        // (channels-last pixels at another pitch, 40 channels packed say, are copied to the pitch of 16 bytes)
+    } else if (is_contiguous(x) || pixels_copied) {
         const int64_t HW = (int64_t)cs.H * cs.W;
-        CHX_PROPAGATE(acquire_scratch(c.cache, 0, (size_t)cs.N * HW * C16, s, &x_scratch));
+        CHX_PROPAGATE(acquire_scratch(cache, 0, (size_t)cs.N * HW * C16, s, &x_scratch));
         const int rc_x = is_contiguous(x) ? launch_nchw_to_nhwc_u8(static_cast<const char*>(x.data), static_cast<char*>(x_scratch), cs.N, cs.C, HW, C16, s)
                                           : launch_pixels_u8(static_cast<const char*>(x.data), x.strides[0], x.strides[2], x.strides[3], static_cast<char*>(x_scratch), cs.N, cs.C, cs.H, cs.W, C16, s);
         if (rc_x != CHX_HIP_OK) {
-            release_scratch(c.cache, x_scratch, s);
+            release_scratch(cache, x_scratch, s);
             return rc_x;
         }
         a.x = static_cast<const char*>(x_scratch);
@@ -620,23 +636,23 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     } else if (is_contiguous(y) && !c.out_int32 && !c.res) {
         const int64_t OHW = (int64_t)cs.OH * cs.OW;
         const int pitch = round_up(cs.OC, 16);
-        const int rc_y = acquire_scratch(c.cache, 1, (size_t)cs.N * OHW * pitch, s, &y_scratch);
+        const int rc_y = acquire_scratch(cache, 1, (size_t)cs.N * OHW * pitch, s, &y_scratch);
         if (rc_y != CHX_HIP_OK) {
-            release_scratch(c.cache, x_scratch, s);
+            release_scratch(cache, x_scratch, s);
             return rc_y;
         }
         a.y = static_cast<char*>(y_scratch);
         a.y_px_stride = pitch;
         y_post = true;
     } else {
-        release_scratch(c.cache, x_scratch, s);
+        release_scratch(cache, x_scratch, s);
         CHX_FAIL(CHX_HIP_EUNSUPPORTED, "y layout is neither pixel-major nor NCHW-contiguous 8-bit");
     }
     (void)es;
     if (c.y_minus_128 || c.y2_minus_128) {
         if (stem || y_post || c.out_int32) {
-            release_scratch(c.cache, x_scratch, s);
-            release_scratch(c.cache, y_scratch, s);
+            release_scratch(cache, x_scratch, s);
+            release_scratch(cache, y_scratch, s);
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv: codes minus 128 are stored by the matrix-core kernel into channels-last results only");
         }
         a.y_flip = c.y_minus_128 ? 0x80808080u : 0u;
@@ -644,8 +660,8 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     if (c.y2) {
         int64_t y2_px = 0;
         if (stem || pw.dense || x_scratch || y_post || c.out_int32 || c.res || !y_is_pixel_major(*c.y2, &y2_px)) {
-            release_scratch(c.cache, x_scratch, s);
-            release_scratch(c.cache, y_scratch, s);
+            release_scratch(cache, x_scratch, s);
+            release_scratch(cache, y_scratch, s);
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv pair: needs channels-last x, y1 and y2 and at least 16 input channels");
         }
         a.oc_split = c.oc_split;
@@ -680,7 +696,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
             rc = launch_nhwc_to_nchw_u8(static_cast<const char*>(y_scratch), static_cast<char*>(y.data), cs.N, cs.OC,
                                         (int64_t)cs.OH * cs.OW, (int)a.y_px_stride, s);
         }
-        release_scratch(c.cache, y_scratch, s);
+        release_scratch(cache, y_scratch, s);
         return rc;
     }
     a.C16 = C16eff;
@@ -689,8 +705,8 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         const int64_t n_img = pw.dense ? 1 : cs.N, h_img = pw.dense ? 1 : H, w_img = pw.dense ? (int64_t)cs.N * cs.OH * cs.OW : W;
         const int64_t span = (n_img - 1) * a.x_n_stride + (h_img - 1) * a.x_h_stride + (w_img - 1) * a.x_w_stride + C16eff;
         if (span >= (int64_t(1) << 31) - (int64_t(1) << 24)) {
-            release_scratch(c.cache, x_scratch, s);
-            release_scratch(c.cache, y_scratch, s);
+            release_scratch(cache, x_scratch, s);
+            release_scratch(cache, y_scratch, s);
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv: the activations span 2 GB or more, which the MFMA kernel does not address");
         }
         a.x_bytes = (uint32_t)span;
@@ -762,8 +778,8 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         rc = launch_nhwc_to_nchw_u8(static_cast<const char*>(y_scratch), static_cast<char*>(y.data), cs.N, cs.OC,
                                     (int64_t)cs.OH * cs.OW, (int)a.y_px_stride, s);
     }
-    release_scratch(c.cache, x_scratch, s);
-    release_scratch(c.cache, y_scratch, s);
+    release_scratch(cache, x_scratch, s);
+    release_scratch(cache, y_scratch, s);
     return rc;
 }
 

@@ -32,3 +32,46 @@ def test_against_the_oracle(g, oracle, case, channels_last):
                                        round_mode=oracle.ROUND_ONNX_RNE if rne else oracle.ROUND_REFERENCE, **okw)
         np.testing.assert_array_equal(g.host(got), np.maximum(want, yz) if relu else want)
         plan.close()
+
+
+@pytest.mark.parametrize("result", ["channels_last", "nchw"])
+def test_packed_pixels_on_two_streams_and_in_a_recording(g, oracle, result):
+    """One plan over packed channels-last arrays: on two streams at once, and recorded without a run before."""
+    import ctypes
+    rng, N, C, H, W, OC = np.random.default_rng(2), 8, 24, 28, 28, 40
+    w, ws = codes(rng, (OC, C, 3, 3), np.int8), rng.uniform(0.002, 0.02, size=OC).astype(np.float32)
+    ys = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C * 9) / 40)
+    xs = [codes(rng, (N, C, H, W), np.uint8) for _ in range(2)]
+    wants = [oracle.qlinear_conv_int(x, 0.02, 3, w, ws, np.zeros(OC, np.int8), ys, 120, np.uint8, pads=(1, 1)) for x in xs]
+    lib, like = g.capi.lib(), lambda: torch.empty((N, OC, H, W), dtype=torch.uint8, device="cuda").contiguous(
+        memory_format=torch.channels_last if result == "channels_last" else torch.contiguous_format)
+    x_dev, outs = [g.to_channels_last(g.dev(x)) for x in xs], [like() for _ in xs]
+    plan = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(OC, np.int8)), None, pads=(1, 1))
+    run = lambda i, o: plan.run(x_dev[i], 0.02, 3, ys, 120, out=o)
+    torch.cuda.synchronize()
+    plan._plan_for(x_dev[0])
+    stream, graph = torch.cuda.Stream(), ctypes.c_void_p()
+    recorded = like()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        s = ctypes.c_void_p(stream.cuda_stream)
+        g.capi.check(lib.chx_hip_capture_begin(s))
+        try:
+            run(0, recorded)
+        finally:
+            g.capi.check(lib.chx_hip_capture_end(s, ctypes.byref(graph)))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                for o in outs[i:i + 1] * 3:
+                    o.zero_()
+                    run(i, o)
+        recorded.zero_()
+        torch.cuda.synchronize()
+        g.capi.check(lib.chx_hip_graph_launch(graph, ctypes.c_void_p(stream.cuda_stream)))
+        torch.cuda.synchronize()
+        for got, want in zip(outs + [recorded], wants + wants[:1]):
+            np.testing.assert_array_equal(g.host(got), want)
+    lib.chx_hip_graph_destroy(graph)
+    plan.close()

@@ -11,7 +11,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -37,6 +37,41 @@ def one_plan_on_dense_images_and_crops(host):
     for x in (dense, apart, dense):
         plan = host.plan(64, c, 1)
         host.check(host.plan_run(plan, x, y))
+
+
+def packed_pixels(host):
+    """Channels-last arrays whose pixels are no multiple of 16 bytes: what ran without the plan's scratch memory before there
+    was a copy for them (in a recording, on a pinned plan, on several streams at once) does so still."""
+    n, c, h, w, oc = 2, 24, 14, 14, 40
+    x, y, nchw = host.channels_last("uint8", (n, c, h, w)), host.channels_last("uint8", (n, oc, h, w)), host.tensor("uint8", (n, oc, h, w))
+    larger = host.channels_last("uint8", (2 * n, c, h, w)), host.channels_last("uint8", (2 * n, oc, h, w))
+    streams = [None, host.stream(), host.stream()]
+    memory = lambda: [line for line in host.log() if "alloc" in line.lower() or "Synchronize" in line]
+    # no warm-up: straight into a recording
+    plan, graph = host.plan(oc, c, 1), ctypes.c_void_p()
+    host.check(host.lib.chx_hip_capture_begin(streams[1]))
+    host.clear()
+    host.check(host.plan_run(plan, x, y, stream=streams[1]))
+    assert ["conv_direct" in k for k in host.launches()] == [True] and not memory()
+    host.check(host.lib.chx_hip_capture_end(streams[1], ctypes.byref(graph)))
+    # pinned, and inputs that grow; results channels-last and NCHW
+    host.check(host.lib.chx_hip_qconv_plan_pin(plan, 1))
+    for xd, yd in [(x, y), larger, (x, nchw), larger]:
+        for s in streams:
+            host.check(host.plan_run(plan, xd, yd, stream=s))
+            host.clear()
+            host.check(host.plan_run(plan, xd, yd, stream=s))
+            assert any("pixels" in k for k in host.launches()) and not any("conv_direct" in k for k in host.launches())
+            # memory of the call on a stream of the caller's, the null stream's block otherwise
+            assert [line.startswith("hipMallocAsync") and line.endswith("stream=0x%x" % s.value) for line in memory()] == [True] if s else memory() == []
+    host.check(host.lib.chx_hip_qconv_plan_pin(plan, -1))
+    # two convolutions as one launch: not for these arrays, and nothing is launched
+    both, y2 = host.plan(128, c, 1), host.channels_last("uint8", (n, 64, h, w))
+    y1 = host.channels_last("uint8", (n, 64, h, w))
+    host.clear()
+    rc = host.lib.chx_hip_qconv_plan_run_pair(both, ctypes.byref(x), ctypes.c_float(0.02), 128, 64, ctypes.c_float(0.05), 3, 0, ctypes.byref(y1), ctypes.c_float(0.05), 3, 0,
+                                              ctypes.byref(y2), None)
+    assert rc == host.capi.EUNSUPPORTED and not host.launches()
 
 
 if __name__ == "__main__":
