@@ -2,6 +2,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <unordered_map>
 
 #include "chx_internal.h"
 #include "quant_math.h"
@@ -69,31 +70,51 @@ static QuantProduct product_with(const QuantParams& q, int path, int ulps, int h
     return p;
 }
 
+// The short forms of one quantization (path 0: there is none).
+struct ProductForms {
+    QuantProduct plain, two_fma;
+};
+
+static ProductForms find_forms(const QuantParams& q) {
+    ProductForms f = {};
+    CodeBounds b;
+    if (!find_bounds(q, &b)) return f;
+    const QuantProduct p = product_with(q, 1, 0, 0);
+    if (same_codes(b, p)) f.plain = p;
+    // (99 of 100 scales have one in this range, most within a few steps)
+    for (int i = 0; q.zpf == 0.f && i < 129 * 7 && f.two_fma.path == 0; ++i) {
+        const int ring = (i / 7 + 1) / 2;
+        const QuantProduct t = product_with(q, 3, (i / 7) & 1 ? ring : -ring, i % 7 - 3);
+        if (same_codes(b, t)) f.two_fma = t;
+    }
+    return f;
+}
+
+// Finding them takes about 25 us, for each of a network's layers: the process remembers them by scale and zero point, for
+// every plan, plan-less call and thread.  (A ResNet-50 has 54 pairs; a table of 256 places found by a hash alone had
+// four of them evict each other, 82 us of every interpreted run.)  2000 pairs are some 200 KB; more start over.
+static ProductForms known_forms(const QuantParams& q) {
+    static std::mutex* mutex = new std::mutex;  // (never destroyed: calls may come from other destructors)
+    static auto* known = new std::unordered_map<uint64_t, ProductForms>;
+    uint32_t scale, zp;
+    memcpy(&scale, &q.scale, 4);
+    memcpy(&zp, &q.zpf, 4);
+    const uint64_t key = (uint64_t)scale << 32 | zp;
+    {
+        std::lock_guard<std::mutex> lock(*mutex);
+        const auto it = known->find(key);
+        if (it != known->end()) return it->second;
+    }
+    const ProductForms f = find_forms(q);
+    std::lock_guard<std::mutex> lock(*mutex);
+    if (known->size() >= 2000) known->clear();
+    (*known)[key] = f;
+    return f;
+}
+
 QuantProduct product_form(const QuantParams& q, float lo_folded, bool rne, bool two_fma) {
     if (rne || q.lo != 0.f || q.hi != 255.f) return QuantProduct{};
-    // finding them takes about 25 us: a thread remembers them
-    struct Forms {
-        float scale, zpf;
-        QuantProduct plain, two_fma;  // path 0: there is none
-    };
-    static thread_local Forms seen[256] = {};
-    uint32_t bits;
-    memcpy(&bits, &q.scale, 4);
-    Forms& f = seen[((bits * 2654435761u) >> 24) ^ ((uint32_t)(int)q.zpf & 255u)];
-    if (f.scale != q.scale || f.zpf != q.zpf) {
-        f = Forms{q.scale, q.zpf, {}, {}};
-        CodeBounds b;
-        if (find_bounds(q, &b)) {
-            const QuantProduct p = product_with(q, 1, 0, 0);
-            if (same_codes(b, p)) f.plain = p;
-            // (99 of 100 scales have one in this range, most within a few steps)
-            for (int i = 0; q.zpf == 0.f && i < 129 * 7 && f.two_fma.path == 0; ++i) {
-                const int ring = (i / 7 + 1) / 2;
-                const QuantProduct t = product_with(q, 3, (i / 7) & 1 ? ring : -ring, i % 7 - 3);
-                if (same_codes(b, t)) f.two_fma = t;
-            }
-        }
-    }
+    const ProductForms f = known_forms(q);
     const bool bound = lo_folded > 0.f;
     QuantProduct p = two_fma && !bound && f.two_fma.path != 0 ? f.two_fma : f.plain;
     if (p.path == 1 && bound) p.path = 2;

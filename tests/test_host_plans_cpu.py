@@ -1,5 +1,7 @@
 """Which kernels the entry points of csrc/contract_api.hip launch, and on what memory, without a GPU."""
 import ctypes
+import threading
+import time
 
 import pytest
 
@@ -11,7 +13,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -72,6 +74,27 @@ def packed_pixels(host):
     rc = host.lib.chx_hip_qconv_plan_run_pair(both, ctypes.byref(x), ctypes.c_float(0.02), 128, 64, ctypes.c_float(0.05), 3, 0, ctypes.byref(y1), ctypes.c_float(0.05), 3, 0,
                                               ctypes.byref(y2), None)
     assert rc == host.capi.EUNSUPPORTED and not host.launches()
+
+
+def requantization_forms(host):
+    """The search for a short form (csrc/core.hip, product_form) runs once per scale and zero point, however many there are
+    and whichever thread asks: a network of hundreds of convolutions goes through all of them on every run."""
+    plan, x, y = host.plan(64, 64, 1), host.channels_last("uint8", (1, 64, 7, 7)), host.channels_last("uint8", (1, 64, 7, 7))
+    params = [(0.01 * 1.003 ** i, i % 5 and 100) for i in range(700)]
+
+    def through_all():
+        start = time.perf_counter()
+        for scale, zero_point in params:
+            host.check(host.plan_run(plan, x, y, scale, zero_point))
+        return time.perf_counter() - start
+
+    host.check(host.plan_run(plan, x, y))  # measures
+    first, later = through_all(), []
+    for target in (lambda: later.append(through_all()),) * 3:
+        thread = threading.Thread(target=target)
+        thread.start()
+        thread.join()
+    assert min(later) < first / 3, (first, later)
 
 
 if __name__ == "__main__":
