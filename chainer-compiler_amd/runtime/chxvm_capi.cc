@@ -88,6 +88,10 @@ public:
         valid_ = true;
         return true;
     }
+    // what has been enqueued is no longer the last launch's
+    void Forget() {
+        valid_ = false;
+    }
     // whether the last launch's results are (or will be) in host memory, and the stream they were queued on
     bool valid() const {
         return valid_;
@@ -140,7 +144,8 @@ struct chxvm_replay {
     void* stream = nullptr;
     chx_hip_graph* graph = nullptr;
     chxvm_outputs outputs;
-    // set once the host has asked for a launch's results: every launch then sends them along
+    // The host has asked for the last launch's results: the next launch sends its own along.  One whose results nobody asked
+    // for makes the next one send nothing, so a launch never finds an unread copy on its way that it would have to wait for.
     bool host_reads = false;
     HostResults results;
     int32_t warm_runs = 0;
@@ -350,6 +355,8 @@ int32_t chxvm_replay_launch(chxvm_replay* replay, void* stream) {
         void* on = stream ? stream : replay->stream;
         CHXVM_HIP_CALL(chx_hip_graph_launch(replay->graph, on));
         if (replay->host_reads) (void)replay->results.Enqueue(replay->outputs.arrays, on);
+        else replay->results.Forget();
+        replay->host_reads = false;
     });
 }
 

@@ -60,7 +60,8 @@ int32_t chxvm_outputs_get(const chxvm_outputs* outputs, int32_t i, chx_hip_tenso
 /* The same without the address (data is null): for a caller that takes the host copy and leaves the device's alone. */
 int32_t chxvm_outputs_layout(const chxvm_outputs* outputs, int32_t i, chx_hip_tensor* out);
 /* Output i in host memory, dense, valid as long as `outputs` (a replay's: until its next launch), or null: copy it from
- * the device then.  Of a replay this is the last launch's result; the first call makes later launches send theirs. */
+ * the device then.  Of a replay this is the last launch's result, where that launch sent it
+ * along: one does when the results of the launch before it were asked for with this function. */
 const void* chxvm_outputs_host(const chxvm_outputs* outputs, int32_t i);
 void chxvm_outputs_destroy(chxvm_outputs* outputs);
 

@@ -15,7 +15,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["two_threads_of_one_program", "memory_of_each_device", "sources_of_the_result_copy"])
+@pytest.mark.parametrize("case", ["two_threads_of_one_program", "memory_of_each_device", "sources_of_the_result_copy", "launches_do_not_wait"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -126,6 +126,43 @@ def sources_of_the_result_copy(host):
     host.check(lib.chx_hip_init(1))
     rc = lib.chx_hip_copyout_enqueue(block, (ctypes.c_void_p * 1)(there), (ctypes.c_size_t * 1)(64), 1, None)
     assert rc == host.capi.EUNSUPPORTED
+
+
+def launches_do_not_wait(host):
+    """A replay's launches only enqueue, whatever is still on its way to the host, and those whose results nobody asks for
+    send nothing."""
+    rt, replay, program = host.chxvm.runtime(), ctypes.c_void_p(), copying_program(host)
+    x = host.tensor("uint8", (64,))
+    assert rt.chxvm_program_capture(program, *host.names_and({"x": x}), ctypes.byref(replay)) == 0, rt.chxvm_last_error()
+    rt.chxvm_replay_outputs.restype = ctypes.c_void_p
+    outputs, streams = ctypes.c_void_p(rt.chxvm_replay_outputs(replay)), [None, host.stream(), host.stream()]
+    refill = lambda v: host.bytes(x.data, bytes([v]) * 64)
+
+    def launch(stream=None):
+        rcs = []
+        thread = threading.Thread(target=lambda: rcs.append(rt.chxvm_replay_launch(replay, stream)))
+        host.clear()
+        thread.start()
+        thread.join(10)
+        assert rcs == [0], "a launch waits"
+        return sum("copy_out_kernel" in k for k in host.launches())
+
+    assert launch() == 0 and launch() == 0
+    assert host_copy(host, outputs, 0, 64) is None  # (the caller copies them from the device)
+    for i in range(3):  # read after every launch: every launch sends its results
+        refill(i)
+        assert launch(streams[i]) == 1 and host_copy(host, outputs, 0, 64) == bytes([i]) * 64
+    host.hh.hh_hold(1)
+    assert launch() == 1
+    for s in streams + streams:
+        assert launch(s) == 0
+    host.hh.hh_release()
+    refill(77)
+    assert launch() == 0
+    assert host_copy(host, outputs, 0, 64) is None  # the block holds an older launch's
+    refill(78)
+    assert launch() == 1 and host_copy(host, outputs, 0, 64) == bytes([78]) * 64
+    rt.chxvm_replay_destroy(replay)
 
 
 if __name__ == "__main__":
