@@ -322,7 +322,8 @@ int run_conv_strip(const ConvDirectArgs& d, hipStream_t s) {
     // filling LDS than a launch takes ([2, 128, 28, 28] with 128 3x3, 65 KB: 11.0 / 10.2), and where work-groups follow one
     // another on a compute unit it is filled once too often ([8, 64, 56, 56] with 256 1x1, 896 of them: 20.0 / 12.2).
     // Channels-last arrays cost more to bring in: not for a few work-groups (28 of them: 10.6 / 9.4).
-    if (strip > 48 * 1024 || work_groups > 512 || (!planar && work_groups < 64)) return CHX_HIP_EUNSUPPORTED;
+    // Beside a long table (1024 channels of 3x3: 36 KB) a strip of that size would pass the 64 KB that any launch may ask for.
+    if (strip > 48 * 1024 || bytes > 64 * 1024 || work_groups > 512 || (!planar && work_groups < 64)) return CHX_HIP_EUNSUPPORTED;
     g.table_at = (int32_t)strip;
     g.x = d.x; g.w = d.w; g.y = d.y;
     for (int i = 0; i < 4; ++i) {

@@ -15,7 +15,8 @@ def g():
 # N, C, H, W, OC, k, stride, pad: one output row per strip up to the whole image in one; K ending inside a step (C = 20, 3x3)
 CASES = [(1, 16, 8, 8, 5, 1, 1, 0), (2, 20, 9, 11, 33, 3, 1, 1), (1, 64, 56, 57, 64, 3, 1, 1), (3, 32, 13, 16, 100, 3, 2, 1), (2, 48, 14, 14, 70, 1, 2, 0),
          (1, 17, 10, 120, 32, 3, 1, 0), (1, 128, 7, 9, 40, 3, 1, 2), (1, 24, 5, 8, 65, 3, 2, 0),
-         (16, 20, 12, 40, 33, 3, 1, 1), (40, 32, 15, 13, 70, 3, 2, 1), (33, 64, 7, 9, 130, 1, 1, 0)]  # (enough strips for channels-last arrays)
+         (16, 20, 12, 40, 33, 3, 1, 1), (40, 32, 15, 13, 70, 3, 2, 1), (33, 64, 7, 9, 130, 1, 1, 0),  # (enough strips for channels-last arrays)
+         (8, 900, 3, 3, 512, 3, 1, 0), (8, 1024, 3, 3, 512, 3, 1, 0)]  # the most shared memory a launch takes, and beyond (conv_planar.hip)
 
 
 @pytest.mark.parametrize("case", CASES)

@@ -1,5 +1,6 @@
 """Which kernels the entry points of csrc/contract_api.hip launch, and on what memory, without a GPU."""
 import ctypes
+import random
 import threading
 import time
 
@@ -13,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -95,6 +96,31 @@ def requantization_forms(host):
         thread.start()
         thread.join()
     assert min(later) < first / 3, (first, later)
+
+
+def shared_memory_of_conv_integer(host):
+    """No launch of ConvInteger asks for more than 64 KB of dynamic shared memory, the most that any launch may have without
+    being arranged with the device runtime."""
+    rng, strips = random.Random(3), 0
+    shapes = [(8, 1024, 3, 3, 512, 3, 1, True, 0), (8, 1024, 3, 3, 512, 3, 1, False, 1), (2, 600, 8, 8, 64, 1, 1, False, 0), (1, 48, 9, 8, 64, 3, 2, False, 1)]
+    while len(shapes) < 600:
+        shapes.append((rng.choice([1, 2, 8, 64]), int(2 ** rng.uniform(2, 11)), rng.choice([3, 8, 9, 14, 28, 57]), rng.choice([1, 3, 8, 14, 28, 57, 112]), rng.choice([16, 64, 512]),
+                       rng.choice([1, 3]), rng.choice([1, 2]), rng.random() < 0.5, rng.choice([0, 1])))
+    memory = host.malloc(1 << 28)
+    for n, c, h, w, oc, k, stride, last, pad in shapes:
+        c = c // 4 * 4
+        oh, ow = (h + 2 * pad - k) // stride + 1, (w + 2 * pad - k) // stride + 1
+        if min(h, w) + 2 * pad < k or max(n * c * h * w, n * oc * oh * ow * 4, oc * c * k * k) > 1 << 28:
+            continue
+        x = host.tensor("uint8", (n, c, h, w), [h * w * c, 1, w * c, c] if last else None, base=memory)
+        wt, y = host.tensor("int8", (oc, c, k, k), base=memory), host.tensor("int32", (n, oc, oh, ow), base=memory)
+        params = host.capi.conv_params((stride, stride), (pad, pad), (pad, pad), 1)
+        host.clear()
+        host.check(host.lib.chx_hip_conv_integer(ctypes.byref(x), ctypes.byref(wt), 128, None, ctypes.byref(params), ctypes.byref(y), None))
+        for launch in host.launches():
+            assert int(launch.split("lds=")[1].split()[0]) <= 64 * 1024, ((n, c, h, w, oc, k, stride, last, pad), launch)
+            strips += "conv_strip_kernel" in launch
+    assert strips > 20
 
 
 if __name__ == "__main__":
