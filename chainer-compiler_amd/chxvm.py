@@ -399,7 +399,9 @@ class Program:
         return [rt.chxvm_program_input_name(self._h, i).decode() for i in range(rt.chxvm_program_num_inputs(self._h))]
 
     def run(self, inputs, trace_level=0):
-        """inputs: {name: torch device tensor}.  Returns {name: numpy array}."""
+        """inputs: {name: torch device tensor}, any mapping.  Returns {name: numpy array}."""
+        if type(inputs) is not dict:
+            inputs = {name: inputs[name] for name in inputs}
         rc, out, host = _native().vm_run(self._h.value or 0, inputs, trace_level)
         _check(rc)
         if host is not None:

@@ -470,3 +470,42 @@ def test_loader_marks_the_operands_of_absorbed_residual_sums(chxvm):
         assert marked() == 0
     finally:
         chxvm.set_option("fuse_residual", "on")
+
+
+# ---- Program.run's inputs ---------------------------------------------------------------------
+
+class _Named:  # the least that names inputs: iteration and look-up
+    def __init__(self, items):
+        self.items_ = items
+
+    def __iter__(self):
+        return iter(self.items_)
+
+    def __getitem__(self, name):
+        return self.items_[name]
+
+
+class _Translated(dict):
+    def __getitem__(self, name):
+        return "not what is stored: " + dict.__getitem__(self, name)
+
+
+@pytest.mark.parametrize("kind", ["dict", "mapping", "named", "translated"])
+def test_run_takes_any_mapping(chxvm, monkeypatch, kind):
+    import types
+    items = {"b": "tensor b", "a": "tensor a"}
+    inputs = {"dict": items, "mapping": types.MappingProxyType(items), "named": _Named(items), "translated": _Translated(items)}[kind]
+    seen = []
+
+    class Native:
+        @staticmethod
+        def vm_run(program, given, trace_level):
+            assert type(given) is dict  # the extension walks a dict itself
+            seen.append(list(given.items()))
+            return 0, 0, []
+
+    monkeypatch.setattr(chxvm, "_machine", Native)
+    b = chxvm.ProgramBuilder()
+    b.output("y", b.input("a"))
+    assert chxvm.Program(b.serialize()).run(inputs) == {}
+    assert seen == [[(n, inputs[n]) for n in items]]
