@@ -218,15 +218,6 @@ PyObject* init(PyObject*, PyObject* error) {
     Py_RETURN_NONE;
 }
 
-// describe_at(tensor, address of a chx_hip_tensor)
-PyObject* describe_at(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    return guarded([&]() -> PyObject* {
-        need(n, 2);
-        describe(tensor(a[0]), reinterpret_cast<chx_hip_tensor*>(integer(a[1])));
-        Py_RETURN_NONE;
-    });
-}
-
 // quantize_linear(x, y_scale, y_zero_point, dtype, flags, out or None)
 PyObject* quantize_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
@@ -533,7 +524,6 @@ PyCFunction fast(PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t)) {
 
 PyMethodDef methods[] = {
         {"init", init, METH_O, nullptr},
-        {"describe_at", fast(describe_at), METH_FASTCALL, nullptr},
         {"quantize_linear", fast(quantize_linear), METH_FASTCALL, nullptr},
         {"dequantize_linear", fast(dequantize_linear), METH_FASTCALL, nullptr},
         {"elementwise", fast(elementwise), METH_FASTCALL, nullptr},
