@@ -628,37 +628,45 @@ const char* ctype_of(int32_t dt) {
            : dt == CHX_HIP_INT8 ? "signed char" : "unsigned char";
 }
 
-// What the general kernel is specialised for, beside the program: how each operand is addressed and the number of axes.
-//   F  dense in the order of the result: the flat index      S  one element
-//   C  innermost stride 1      Z  innermost stride 0      X  any strides
+// How the general kernel addresses an operand:
+//   kFlat    dense in the order of the result: the flat index      kOne       one element
+//   kRow     innermost stride 1      kRepeat  innermost stride 0   kStrided   any strides
+enum Addressing : char { kFlat = 'F', kOne = 'S', kRow = 'C', kRepeat = 'Z', kStrided = 'X' };
+
+// What the general kernel is compiled for, beside the program.
 struct GeneralForm {
-    std::string modes;
-    int ndim = 0;         // collapsed axes
-    int vec = 1;          // elements per thread: 16 bytes of the widest operand
-    bool wide = false;    // 2^31 elements or more: 64-bit indices
-    bool short_rows = false;  // the innermost axis is shorter than `vec`
+    std::string modes;  // Addressing, per input
+    int vec = 1;        // elements per thread: 16 bytes of the widest operand (the program's); 1: rows shorter than that
+    int axes = 3;       // collapsed axes: up to three (nearly all calls), or kAxes
+    bool wide = false;  // 2^31 elements or more in the result or in the reach of an operand, or negative strides: 64-bit indices
 };
+constexpr int kAxes = CHX_HIP_MAX_NDIM;
 
 // The general kernel: any strides, types and alignments.  A thread computes `vec` neighbouring elements of the result.
 // Where they lie in one row of the innermost axis (nearly always) each operand is one access of 16 bytes at whatever
-// alignment (F, C), one element (S, Z), or `vec` strided ones (X); a run that crosses the end of a row is read
-// element by element from two positions.  Divisions by the extents are multiplications with their reciprocals.
-// float16 chain over [8, 333, 1001] with two [1001] operands: 15.2 us with one element per thread and 64-bit divisions,
-// 13.4 this way, and 7.5 once its functions cost less (kTanhOfF16).
+// alignment (kFlat, kRow), one element (kOne, kRepeat), or `vec` strided ones; a run that crosses the end of a row is
+// read element by element from two positions.  (Of rows shorter than that a thread computes one element: every run would
+// cross.)  Divisions by the extents are multiplications with their reciprocals.
+// Axes are collapsed ones, the innermost first; those past the last have extent 1, so that the rank of a call is no part of
+// its kernel (a compilation takes 0.3 s of the first call).  The operands' addressing is: as an argument it made the chain
+// below 17 % slower in float32 rows of 1001 (scalar loads behind each branch), which one kernel for all calls would cost.
+// Chain of two operands of [8, 333, 1001] and two of [1001] through Mul, Add, Tanh, Sigmoid, Mul, Add and Relu in float16:
+// 15.2 us with one element per thread and 64-bit divisions, 8.6 with each operand converted beside its load, 6.9 with all
+// loads in flight first.
 void emit_general(const Program& prog, const std::string& name, const GeneralForm& g, const std::string& VT, std::ostringstream& os) {
     const size_t nin = prog.inputs.size(), nout = prog.outputs.size();
-    const int V = g.vec, ND = g.ndim > 0 ? g.ndim : 1;
-    const std::string last = std::to_string(ND - 1);
-    bool placed = false;  // an operand that needs the position of the run
-    for (char m : g.modes) placed = placed || m == 'C' || m == 'Z' || m == 'X';
+    const int V = g.vec;
+    auto placed = [&](size_t i) { return g.modes[i] != kFlat && g.modes[i] != kOne; };  // by the position in the result
+    bool any_placed = false;
+    for (size_t i = 0; i < nin; ++i) any_placed = any_placed || placed(i);
     const char* idx = g.wide ? "unsigned long long" : "unsigned int";
     auto value_type = [&](const Port& p) { return is_float_dtype(p.dtype) ? VT : std::string("int"); };
     auto vec_type = [&](int32_t dt) {
         return std::string("V") + (dt == CHX_HIP_FLOAT32 ? "f" : dt == CHX_HIP_FLOAT16 ? "h" : dt == CHX_HIP_FLOAT64 ? "d" : "b");
     };
-    os << "typedef " << idx << " gidx;\n";
-    os << "struct GenDesc { unsigned int mul[" << CHX_HIP_MAX_NDIM << "], shift[" << CHX_HIP_MAX_NDIM << "]; long long shape[" << CHX_HIP_MAX_NDIM
-       << "]; long long istr[" << nin << "][" << CHX_HIP_MAX_NDIM << "]; };\n";
+    os << "typedef " << idx << " gidx;\ntypedef " << (g.wide ? "long long" : "unsigned int") << " sidx;  // (wide: positions before the operand's first element)\n";
+    os << "struct GenDesc { unsigned int mul[" << kAxes << "], shift[" << kAxes << "]; long long shape[" << kAxes << "]; long long istr[" << nin << "][" << kAxes
+       << "]; };\n";
     os << "typedef float Vf __attribute__((ext_vector_type(" << V << "), aligned(4)));\n";
     os << "typedef _Float16 Vh __attribute__((ext_vector_type(" << V << "), aligned(2)));\n";
     os << "typedef double Vd __attribute__((ext_vector_type(" << V << "), aligned(8)));\n";
@@ -666,14 +674,12 @@ void emit_general(const Program& prog, const std::string& name, const GeneralFor
     os << "__device__ __forceinline__ gidx gdiv(gidx r, const GenDesc& d, int a) {\n";
     if (g.wide) os << "  return r / (gidx)d.shape[a];\n}\n";
     else os << "  return (__umulhi(r, d.mul[a]) + r) >> d.shift[a];\n}\n";
-    // element offsets of every placed operand at flat position r
-    os << "__device__ __forceinline__ void place(gidx r, const GenDesc& d, long long (&off)[" << nin << "], gidx& inner) {\n";
-    os << "  for (int i = 0; i < " << nin << "; ++i) off[i] = 0;\n  inner = 0;\n";
-    os << "#pragma unroll\n  for (int a = " << last << "; a >= 0; --a) {\n";
-    os << "    const gidx q = a ? gdiv(r, d, a) : 0, m = r - q * (gidx)d.shape[a];\n    r = q;\n    if (a == " << last << ") inner = m;\n";
-    for (size_t i = 0; i < nin; ++i)
-        if (g.modes[i] == 'C' || g.modes[i] == 'Z' || g.modes[i] == 'X') os << "    off[" << i << "] += (long long)m * d.istr[" << i << "][a];\n";
-    os << "  }\n}\n";
+    // the position along each axis of flat position r, and an operand's element there
+    os << "__device__ __forceinline__ void place(gidx r, const GenDesc& d, gidx (&at)[" << g.axes << "]) {\n";
+    os << "#pragma unroll\n  for (int a = 0; a < " << g.axes - 1 << "; ++a) {\n    const gidx q = gdiv(r, d, a);\n    at[a] = r - q * (gidx)d.shape[a];\n    r = q;\n  }\n";
+    os << "  at[" << g.axes - 1 << "] = r;\n}\n";
+    os << "__device__ __forceinline__ gidx offset(const long long (&stride)[" << kAxes << "], const gidx (&at)[" << g.axes << "]) {\n  gidx off = 0;\n";
+    os << "#pragma unroll\n  for (int a = 0; a < " << g.axes << "; ++a) off += at[a] * (gidx)stride[a];\n  return off;\n}\n";
 
     os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_gen(unsigned long long total";
     for (size_t i = 0; i < nin; ++i) os << ", const " << ctype_of(prog.inputs[i].dtype) << "* __restrict__ i" << i;
@@ -682,60 +688,62 @@ void emit_general(const Program& prog, const std::string& name, const GeneralFor
     os << "  const gidx n = (gidx)total, base = ((gidx)blockIdx.x * 256u + threadIdx.x) * " << V << "u;\n";
     os << "  if (base >= n) return;\n";
     os << "  const int cnt = n - base < " << V << "u ? (int)(n - base) : " << V << ";\n";
-    os << "  long long off[" << nin << "]; gidx inner = 0;\n";
-    if (placed) {
-        os << "  place(base, d, off, inner);\n";
-        os << "  const gidx left = (gidx)d.shape[" << last << "] - inner;\n";
-        os << "  const bool straight = cnt == " << V << " && left >= " << V << "u;\n";
-    } else {
-        os << "  const bool straight = cnt == " << V << ";\n";
+    // What an operand's elements are as loaded: a vector, and converted behind the last of the loads only (a conversion
+    // beside its load waits for it, one operand after the other).  8-bit codes arrive as words.
+    auto element = [&](size_t i, const std::string& e, const std::string& at) {  // statement: element e of operand i
+        const std::string k = std::to_string(i);
+        if (is_float_dtype(prog.inputs[i].dtype)) return "r" + k + "[" + e + "] = i" + k + "[(sidx)(" + at + ")]; ";
+        return "r" + k + "[" + e + " / 4] |= (unsigned int)(unsigned char)i" + k + "[(sidx)(" + at + ")] << (8 * (" + e + " % 4)); ";
+    };
+    for (size_t i = 0; i < nin; ++i) os << "  " << vec_type(prog.inputs[i].dtype) << " r" << i << " = 0;\n";
+    os << "  const bool whole = cnt == " << V << ";\n";
+    auto whole_access = [&](const Port& p) { return is_float_dtype(p.dtype) || V >= 4; };  // (codes come in words)
+    auto elements = [&](size_t i, const std::string& condition, const std::string& at) {
+        os << "  {\n#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) " << condition << "{ " << element(i, "e", at) << "}\n  }\n";
+    };
+    // (dense operands before the others' addresses are known)
+    for (size_t i = 0; i < nin; ++i) {
+        const std::string k = std::to_string(i), vt = vec_type(prog.inputs[i].dtype);
+        if (g.modes[i] == kOne) elements(i, "", "0");
+        if (g.modes[i] != kFlat) continue;
+        if (whole_access(prog.inputs[i])) os << "  if (whole) r" << k << " = __builtin_nontemporal_load((const " << vt << "*)(i" << k << " + base));\n  else\n";
+        elements(i, "if (e < cnt) ", "base + e");
     }
-    for (size_t i = 0; i < nin; ++i) os << "  " << value_type(prog.inputs[i]) << " x" << i << "[" << V << "];\n";
-    // a vector of 8-bit codes arrives as words
-    auto unpack = [&](size_t i, const std::string& from) {
+    if (any_placed) {
+        os << "  gidx at[" << g.axes << "];\n  place(base, d, at);\n";
+        if (V > 1) os << "  const gidx left = (gidx)d.shape[0] - at[0];\n  if (whole && left >= " << V << "u) {\n";
+        for (size_t i = 0; i < nin; ++i) {
+            if (!placed(i)) continue;
+            const std::string k = std::to_string(i), vt = vec_type(prog.inputs[i].dtype);
+            os << "  { const gidx off = offset(d.istr[" << k << "], at);\n";
+            if (g.modes[i] == kRow && whole_access(prog.inputs[i])) os << "    r" << k << " = *(const " << vt << "*)(i" << k << " + (sidx)off);\n";
+            else elements(i, "", g.modes[i] == kRepeat || V == 1 ? "off" : "off + e * (gidx)d.istr[" + k + "][0]");
+            os << "  }\n";
+        }
+        if (V > 1) {
+            // (`there` is where the elements behind the end of the row would begin if they had all been on the next one)
+            os << "  } else {\n    gidx next[" << g.axes << "];\n    place(base + left < n ? base + left : base, d, next);\n";
+            for (size_t i = 0; i < nin; ++i) {
+                if (!placed(i)) continue;
+                const std::string k = std::to_string(i), step = g.modes[i] == kRow ? "1u" : g.modes[i] == kRepeat ? "0u" : "(gidx)d.istr[" + k + "][0]";
+                os << "  { const gidx here = offset(d.istr[" << k << "], at), there = offset(d.istr[" << k << "], next) - left * " << step << ";\n";
+                elements(i, "if (e < cnt) ", "((gidx)e < left ? here : there) + e * " + step);
+                os << "  }\n";
+            }
+            os << "  }\n";
+        }
+    }
+    for (size_t i = 0; i < nin; ++i) {
+        const std::string k = std::to_string(i);
         const int32_t dt = prog.inputs[i].dtype;
+        os << "  " << value_type(prog.inputs[i]) << " x" << k << "[" << V << "];\n";
         if (is_float_dtype(dt)) {
-            os << "    for (int e = 0; e < " << V << "; ++e) x" << i << "[e] = (" << VT << ")" << from << "[e];\n";
+            os << "  for (int e = 0; e < " << V << "; ++e) x" << k << "[e] = (" << VT << ")r" << k << "[e];\n";
         } else {
             for (int e = 0; e < V; ++e)
-                os << "    x" << i << "[" << e << "] = (int)" << (dt == CHX_HIP_INT8 ? "(signed char)" : "") << "((" << from << "[" << e / 4 << "] >> " << 8 * (e % 4)
-                   << ") & 0xffu);\n";
-        }
-    };
-    os << "  if (straight) {\n";
-    for (size_t i = 0; i < nin; ++i) {
-        const char m = g.modes[i];
-        if ((m == 'F' || m == 'C') && (is_float_dtype(prog.inputs[i].dtype) || V >= 4)) {
-            os << "    { const " << vec_type(prog.inputs[i].dtype) << " t = " << (m == 'F' ? "__builtin_nontemporal_load(" : "*(") << "(const "
-               << vec_type(prog.inputs[i].dtype) << "*)(i" << i << " + " << (m == 'F' ? "base" : "off[" + std::to_string(i) + "]") << "));\n";
-            unpack(i, "t");
-            os << "    }\n";
-        } else {
-            const std::string at = m == 'S' ? "0" : m == 'F' ? "base + e" : m == 'Z' ? "off[" + std::to_string(i) + "]"
-                                   : "off[" + std::to_string(i) + "] + e * d.istr[" + std::to_string(i) + "][" + last + "]";
-            os << "    for (int e = 0; e < " << V << "; ++e) x" << i << "[e] = (" << value_type(prog.inputs[i]) << ")i" << i << "[" << at << "];\n";
+                os << "  x" << k << "[" << e << "] = (int)" << (dt == CHX_HIP_INT8 ? "(signed char)" : "") << "((r" << k << "[" << e / 4 << "] >> " << 8 * (e % 4) << ") & 0xffu);\n";
         }
     }
-    os << "  } else {\n";
-    if (placed && !g.short_rows) {
-        os << "    long long next[" << nin << "]; gidx zero;\n";
-        os << "    place(base + left < n ? base + left : base, d, next, zero);\n";
-    }
-    os << "#pragma unroll\n    for (int e = 0; e < " << V << "; ++e) {\n      if (e < cnt) {\n";
-    if (placed && g.short_rows) os << "        place(base + e, d, off, inner);\n";
-    for (size_t i = 0; i < nin; ++i) {
-        const char m = g.modes[i];
-        const std::string k = std::to_string(i), step = m == 'C' ? "1" : m == 'Z' ? "0" : "d.istr[" + k + "][" + last + "]";
-        os << "        x" << i << "[e] = (" << value_type(prog.inputs[i]) << ")i" << i << "[";
-        if (m == 'S') os << "0";
-        else if (m == 'F') os << "base + e";
-        else if (g.short_rows) os << "off[" << k << "]";
-        else os << "(gidx)e < left ? off[" << k << "] + e * " << step << " : next[" << k << "] + (long long)(e - (int)left) * " << step;
-        os << "];\n";
-    }
-    os << "      } else {\n";
-    for (size_t i = 0; i < nin; ++i) os << "        x" << i << "[e] = 0;\n";
-    os << "      }\n    }\n  }\n";
     for (size_t i = 0; i < nout; ++i) os << "  " << value_type(prog.outputs[i]) << " y" << i << "[" << V << "];\n";
     os << "  bool rare = false;\n";
     for (int fast = 1; fast >= 0; --fast) {
@@ -749,9 +757,13 @@ void emit_general(const Program& prog, const std::string& name, const GeneralFor
     os << "  if (cnt == " << V << ") {\n";
     for (size_t i = 0; i < nout; ++i) {
         const int32_t dt = prog.outputs[i].dtype;
+        if (!whole_access(prog.outputs[i])) {
+            os << "    for (int e = 0; e < " << V << "; ++e) o" << i << "[base + e] = (" << ctype_of(dt) << ")y" << i << "[e];\n";
+            continue;
+        }
         if (is_float_dtype(dt)) {
             os << "    { " << vec_type(dt) << " t; for (int e = 0; e < " << V << "; ++e) t[e] = (" << ctype_of(dt) << ")y" << i << "[e];\n";
-        } else if (V >= 4) {
+        } else {
             os << "    { Vb t;\n";
             for (int w = 0; w < V / 4; ++w) {
                 os << "      t[" << w << "] = ";
@@ -766,15 +778,13 @@ void emit_general(const Program& prog, const std::string& name, const GeneralFor
     os << "    }\n  }\n}\n";
 }
 
-// Source of both kernels for one (program, operand modes) combination.
+// What both kernels of a program begin with: the per-element function and what it needs.  The kernels are sources of their
+// own, compiled when a call first takes one of them:
 //   <name>_vec : V elements per thread through 128-bit accesses; operands are full
 //                (same flat index as the output), scalar, or periodic (index modulo a
-//                period that is a multiple of V).
+//                period that is a multiple of V).  float32 programs.
 //   <name>_gen : emit_general.
-int generate_source(
-        const Program& prog, const std::string& name, const std::string& modes, const std::vector<uint32_t>& periods,
-        int vec, const GeneralForm& gen, bool use_fma, std::string* out) {
-    std::ostringstream os;
+int emit_common(const Program& prog, bool use_fma, std::ostringstream& os) {
     os << "#pragma clang fp contract(off)\n";
     os << "#define FM_FN __device__ __forceinline__\n";
     os << "#define FM_TABLE_QUALIFIER static __device__ const\n";
@@ -789,19 +799,31 @@ int generate_source(
     os << "typedef float v4f __attribute__((ext_vector_type(4)));\n";
     os << "typedef unsigned int v4u __attribute__((ext_vector_type(4)));\n";
     os << "namespace {\n" << body.str() << "}\n";
-    const size_t nin = prog.inputs.size(), nout = prog.outputs.size();
+    return CHX_HIP_OK;
+}
 
-    // ---- vector kernel ----
+const char* value_type_of(const Program& prog) {  // what elem() takes and gives
+    return prog.arith == CHX_HIP_FLOAT64 ? "double" : "float";
+}
+
+int general_source(const Program& prog, const std::string& name, const GeneralForm& form, bool use_fma, std::string* out) {
+    std::ostringstream os;
+    CHX_PROPAGATE(emit_common(prog, use_fma, os));
+    emit_general(prog, name, form, value_type_of(prog), os);
+    *out = os.str();
+    return CHX_HIP_OK;
+}
+
+int vector_source(
+        const Program& prog, const std::string& name, const std::string& modes, const std::vector<uint32_t>& periods, int vec, bool use_fma, std::string* out) {
+    std::ostringstream os;
+    CHX_PROPAGATE(emit_common(prog, use_fma, os));
+    const size_t nin = prog.inputs.size(), nout = prog.outputs.size();
     // `vec` elements per lane and step: 4 when any full-size operand is float32 (float32
     // moves as one 128-bit access per lane, 8-bit codes as one 32-bit access), 16 when all
     // of them are 8-bit (one 128-bit access each).  kSteps steps per thread at a stride of
     // one block keep every access instruction of a wavefront on one contiguous span.
     const int steps = 2;
-    const std::string VT = prog.arith == CHX_HIP_FLOAT64 ? "double" : "float";  // what elem() takes and gives
-    if (prog.arith != CHX_HIP_FLOAT32) {
-        // float16 and float64 programs have the general kernel only; this one is never launched
-        os << "extern \"C\" __global__ void " << name << "_vec(unsigned int n_vec) {}\n";
-    } else {
     os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_vec(unsigned int n_vec";
     for (size_t i = 0; i < nin; ++i) os << ", const " << ctype_of(prog.inputs[i].dtype) << "* __restrict__ i" << i;
     for (size_t i = 0; i < nout; ++i) os << ", " << ctype_of(prog.outputs[i].dtype) << "* __restrict__ o" << i;
@@ -889,22 +911,18 @@ int generate_source(
         }
     }
     os << "  }\n  }\n}\n";
-    }
-
-    // ---- general kernel ----
-    emit_general(prog, name, gen, VT, os);
     *out = os.str();
     return CHX_HIP_OK;
 }
 
-struct CompiledKernels {
+struct CompiledKernel {
     std::vector<char> code;
     hipModule_t module = nullptr;  // loaded lazily, per process (one GPU)
-    hipFunction_t vec = nullptr, gen = nullptr;
+    hipFunction_t function = nullptr;
 };
 
 std::mutex g_cache_mutex;
-std::map<std::string, std::shared_ptr<CompiledKernels>> g_cache;  // key: generated source
+std::map<std::string, std::shared_ptr<CompiledKernel>> g_cache;  // key: generated source
 
 int compile_source(const std::string& src, const std::string& name, std::vector<char>* code) {
     hiprtcProgram p;
@@ -1085,27 +1103,33 @@ int make_plan(
         if (!aligned(outputs[k]->data, 16)) ok = false;
     plan->vector_ok = ok && n >= plan->vec && prog.arith == CHX_HIP_FLOAT32;
     GeneralForm& g = plan->gen;
-    g.ndim = plan->ndim;
     g.vec = any32 ? 4 : prog.arith == CHX_HIP_FLOAT64 ? 2 : prog.arith == CHX_HIP_FLOAT16 ? 8 : 16;
     g.wide = n >= (int64_t(1) << 31) - 4096;  // (indices run past the last element by less than a work-group's share)
-    g.short_rows = plan->ndim > 0 && cshape[plan->ndim - 1] < g.vec;
-    g.modes.assign(n_inputs, 'X');
+    g.axes = plan->ndim > 3 ? kAxes : 3;
+    g.modes.assign(n_inputs, kStrided);
+    bool placed = false;
     for (int i = 0; i < n_inputs; ++i) {
         bool flat = true, one = true;
+        int64_t reach = 0;
         for (int a = 0; a < plan->ndim; ++a) {
             flat = flat && cstr[i][a] == dense[a];
             one = one && cstr[i][a] == 0;
+            reach += (cshape[a] - 1) * cstr[i][a];
+            if (cstr[i][a] < 0) g.wide = true;
         }
-        if (plan->ndim == 0 || one) g.modes[i] = 'S';
-        else if (flat) g.modes[i] = 'F';
-        else if (cstr[i][plan->ndim - 1] == 1) g.modes[i] = 'C';
-        else if (cstr[i][plan->ndim - 1] == 0) g.modes[i] = 'Z';
+        if (reach >= (int64_t(1) << 31) - 4096) g.wide = true;
+        if (plan->ndim == 0 || one) g.modes[i] = kOne;
+        else if (flat) g.modes[i] = kFlat;
+        else if (cstr[i][plan->ndim - 1] == 1) g.modes[i] = kRow;
+        else if (cstr[i][plan->ndim - 1] == 0) g.modes[i] = kRepeat;
+        placed = placed || (g.modes[i] != kOne && g.modes[i] != kFlat);
     }
-    if (!plan->vector_ok) {
-        // the general kernel ignores these modes; use one canonical key
-        plan->modes.assign(n_inputs, kFull);
-        plan->periods.assign(n_inputs, 0);
+    if (placed && cshape[plan->ndim - 1] < g.vec) {
+        g.vec = 1;
+        for (char& m : g.modes)
+            if (m == kRow || m == kRepeat) m = kStrided;  // (the same for one element)
     }
+    if (!placed) g.axes = 3;  // (none is looked at)
     return CHX_HIP_OK;
 }
 
@@ -1125,40 +1149,47 @@ struct ArgPacker {
     }
 };
 
+// Whether a call takes the vector kernel.  (Elements beyond whole vectors would be a launch of their own.)
+bool takes_vector(const Plan& plan) {
+    return plan.vector_ok && plan.n % plan.vec == 0;
+}
+
 int prepare(
         const char* code, int32_t fusion_id, const chx_hip_tensor* const* inputs, int32_t n_inputs,
-        chx_hip_tensor* const* outputs, int32_t n_outputs, Program* prog, Plan* plan, std::string* name,
-        std::string* src) {
+        chx_hip_tensor* const* outputs, int32_t n_outputs, Program* prog, Plan* plan, std::string* name) {
     CHX_REQUIRE(inputs != nullptr && n_inputs > 0, "fusion: no inputs");  // CHECK(!inputs.empty()), nvrtc.cc:93
     CHX_REQUIRE(outputs != nullptr && n_outputs > 0, "fusion: no outputs");
     CHX_PROPAGATE(parse_program(code, prog));
     CHX_PROPAGATE(make_plan(*prog, inputs, n_inputs, outputs, n_outputs, plan));
     *name = "fusion" + std::to_string(fusion_id < 0 ? 0 : fusion_id);
-    CHX_PROPAGATE(generate_source(*prog, *name, plan->modes, plan->periods, plan->vec, plan->gen, host_libm_uses_fma(), src));
     return CHX_HIP_OK;
 }
 
-int get_compiled(const std::string& src, const std::string& name, std::shared_ptr<CompiledKernels>* out) {
+int source_of(const Program& prog, const Plan& plan, const std::string& name, bool vector, std::string* src) {
+    if (vector) return vector_source(prog, name, plan.modes, plan.periods, plan.vec, host_libm_uses_fma(), src);
+    return general_source(prog, name, plan.gen, host_libm_uses_fma(), src);
+}
+
+int get_compiled(const std::string& src, const std::string& name, std::shared_ptr<CompiledKernel>* out) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     auto it = g_cache.find(src);
     if (it != g_cache.end()) {
         *out = it->second;
         return CHX_HIP_OK;
     }
-    auto ck = std::make_shared<CompiledKernels>();
+    auto ck = std::make_shared<CompiledKernel>();
     CHX_PROPAGATE(compile_source(src, name, &ck->code));
     g_cache.emplace(src, ck);
     *out = ck;
     return CHX_HIP_OK;
 }
 
-int load_kernels(CompiledKernels* ck, const std::string& name) {
+int load_kernel(CompiledKernel* ck, const std::string& function) {
     std::lock_guard<std::mutex> lock(g_cache_mutex);
     if (ck->module) return CHX_HIP_OK;
     hipModule_t m;
     CHX_HIP_CALL(hipModuleLoadData(&m, ck->code.data()));
-    CHX_HIP_CALL(hipModuleGetFunction(&ck->vec, m, (name + "_vec").c_str()));
-    CHX_HIP_CALL(hipModuleGetFunction(&ck->gen, m, (name + "_gen").c_str()));
+    CHX_HIP_CALL(hipModuleGetFunction(&ck->function, m, function.c_str()));
     ck->module = m;
     return CHX_HIP_OK;
 }
@@ -1206,13 +1237,19 @@ extern "C" int chx_hip_elementwise_source(
         size_t* needed) {
     Program prog;
     Plan plan;
-    std::string name, src;
-    CHX_PROPAGATE(prepare(code, fusion_id, inputs, n_inputs, outputs, n_outputs, &prog, &plan, &name, &src));
-    if (compile) {
-        std::shared_ptr<CompiledKernels> ck;
-        CHX_PROPAGATE(get_compiled(src, name, &ck));
+    std::string name, text;
+    CHX_PROPAGATE(prepare(code, fusion_id, inputs, n_inputs, outputs, n_outputs, &prog, &plan, &name));
+    // both kernels where the operands are the vector kernel's (a count that is not whole vectors takes the other)
+    for (const bool vector : {true, false}) {
+        if (vector && !plan.vector_ok) continue;
+        std::string src;
+        CHX_PROPAGATE(source_of(prog, plan, name, vector, &src));
+        if (compile && vector == takes_vector(plan)) {
+            std::shared_ptr<CompiledKernel> ck;
+            CHX_PROPAGATE(get_compiled(src, name, &ck));
+        }
+        text += "// modes=" + (plan.vector_ok ? plan.modes + " vector" : std::string((size_t)n_inputs, kFull) + " general") + "\n" + src;
     }
-    std::string text = std::string("// modes=") + plan.modes + (plan.vector_ok ? " vector" : " general") + "\n" + src;
     if (needed) *needed = text.size() + 1;
     if (buffer && buffer_size) {
         const size_t n = text.size() < buffer_size - 1 ? text.size() : buffer_size - 1;
@@ -1228,7 +1265,7 @@ namespace {
 // What a call needs beyond its pointers, kept per (program text, operand layouts): parsing the text, planning and writing
 // out the kernel's source to look the compiled kernel up took 35 us of host time per call.
 struct PreparedCall {
-    std::shared_ptr<CompiledKernels> kernels;
+    std::shared_ptr<CompiledKernel> kernel;
     bool vector = false;
     int vec = 0;
     int64_t n = 0;
@@ -1253,31 +1290,32 @@ int prepare_call(
     Program prog;
     Plan plan;
     std::string name, src;
-    CHX_PROPAGATE(prepare(code, fusion_id, inputs, n_inputs, outputs, n_outputs, &prog, &plan, &name, &src));
+    CHX_PROPAGATE(prepare(code, fusion_id, inputs, n_inputs, outputs, n_outputs, &prog, &plan, &name));
     call->n = plan.n;
     if (plan.n == 0) return CHX_HIP_OK;
     CHX_REQUIRE(plan.n < (int64_t(1) << 39), "fusion: %lld elements is beyond what the general kernel covers", (long long)plan.n);
-    CHX_PROPAGATE(get_compiled(src, name, &call->kernels));
-    CHX_PROPAGATE(load_kernels(call->kernels.get(), name));
-    // (elements beyond whole vectors would be a launch of their own)
-    call->vector = plan.vector_ok && plan.n % plan.vec == 0;
+    call->vector = takes_vector(plan);
     call->vec = plan.vec;
+    CHX_PROPAGATE(source_of(prog, plan, name, call->vector, &src));
+    CHX_PROPAGATE(get_compiled(src, name, &call->kernel));
+    CHX_PROPAGATE(load_kernel(call->kernel.get(), name + (call->vector ? "_vec" : "_gen")));
     if (call->vector) {
         call->grid = (unsigned)((plan.n / plan.vec + 511) / 512);
         return CHX_HIP_OK;
     }
     call->grid = (unsigned)((plan.n + 256 * plan.gen.vec - 1) / (256 * plan.gen.vec));
-    // GenDesc { unsigned mul[MAX], shift[MAX]; long long shape[MAX]; long long istr[nin][MAX]; }
-    const size_t M = CHX_HIP_MAX_NDIM;
+    // GenDesc { unsigned mul[kAxes], shift[kAxes]; long long shape[kAxes], istr[nin][kAxes]; }
+    const size_t M = kAxes;
     call->desc.assign(2 * M * 4 + M * 8 + (size_t)n_inputs * M * 8, 0);
     uint32_t* mul = reinterpret_cast<uint32_t*>(call->desc.data());
     int64_t* shape = reinterpret_cast<int64_t*>(call->desc.data() + 2 * M * 4);
-    for (size_t a = 0; a < M; ++a) {
-        shape[a] = a < (size_t)plan.ndim ? plan.shape[a] : 1;
-        if (!plan.gen.wide) magic_divisor((uint32_t)shape[a], &mul[a], &mul[M + a]);
+    for (size_t k = 0; k < M; ++k) {
+        const bool there = k < (size_t)plan.ndim;
+        const size_t a = (size_t)plan.ndim - 1 - k;  // (the kernel's first axis is the innermost)
+        shape[k] = there ? plan.shape[a] : 1;
+        if (!plan.gen.wide) magic_divisor((uint32_t)shape[k], &mul[k], &mul[M + k]);
+        for (size_t i = 0; there && i < (size_t)n_inputs; ++i) shape[M * (1 + i) + k] = plan.istr[i][a];
     }
-    for (int i = 0; i < n_inputs; ++i)
-        for (int a = 0; a < plan.ndim; ++a) shape[M * (size_t)(1 + i) + (size_t)a] = plan.istr[i][a];
     return CHX_HIP_OK;
 }
 
@@ -1318,7 +1356,7 @@ extern "C" int chx_hip_elementwise(
     for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
     for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
     if (!call->vector) a.push_bytes(call->desc.data(), call->desc.size(), 8);
-    return launch(call->vector ? call->kernels->vec : call->kernels->gen, call->grid, a, as_stream(stream));
+    return launch(call->kernel->function, call->grid, a, as_stream(stream));
 }
 
 extern "C" int chx_hip_elementwise_match_residual_add(const char* code, int32_t* matches, chx_hip_residual_group* group) {

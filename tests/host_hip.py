@@ -77,13 +77,17 @@ class Host:
         self.check(self.lib.chx_hip_stream_create(ctypes.byref(s)))
         return s
 
+    @staticmethod
+    def dense(shape):
+        strides = [1] * len(shape)
+        for i in range(len(shape) - 2, -1, -1):
+            strides[i] = strides[i + 1] * shape[i + 1]
+        return strides
+
     def tensor(self, dtype, shape, strides=None, offset=0, base=None):
         """A descriptor; strides in elements (default dense), base: memory that is there already."""
         size = {"int8": 1, "uint8": 1, "float16": 2, "int32": 4, "float32": 4}[dtype]
-        if strides is None:
-            strides = [1] * len(shape)
-            for i in range(len(shape) - 2, -1, -1):
-                strides[i] = strides[i + 1] * shape[i + 1]
+        strides = self.dense(shape) if strides is None else strides
         span = 1 + sum((n - 1) * s for n, s in zip(shape, strides))
         base = base or self.malloc((span + offset) * size + 64)
         return self.capi.make_desc(base + offset * size, getattr(self.capi, dtype.upper()), shape, [s * size for s in strides])

@@ -15,7 +15,8 @@ def g():
 
 # shapes of the operands of a + b * c: flat, rows repeated (C), inner axis repeated (Z), one element, rows shorter than a vector
 CASES = [((7,), (7,), ()), ((1,), (1,), (1,)), ((3, 5), (5,), (3, 1)), ((4, 3, 2), (3, 1), (2,)), ((9, 1001), (1001,), (9, 1)),
-         ((5, 1, 17), (6, 1), (1, 6, 17)), ((2, 3, 1, 9), (3, 4, 1), (4, 9)), ((33, 8), (8,), (33, 8)), ((2, 257, 3), (257, 1), (3,))]
+         ((5, 1, 17), (6, 1), (1, 6, 17)), ((2, 3, 1, 9), (3, 4, 1), (4, 9)), ((33, 8), (8,), (33, 8)), ((2, 257, 3), (257, 1), (3,)),
+         ((2, 1, 3, 1, 5), (1, 4, 1, 6, 1), (5,)), ((2, 3, 2, 2, 19), (3, 1, 2, 1), (2, 1, 2, 1, 19))]
 
 
 @pytest.mark.parametrize("shapes", CASES)

@@ -1,4 +1,4 @@
-"""Which kernels the entry points of csrc/contract_api.hip launch, and on what memory, without a GPU."""
+"""Which kernels the entry points launch, on what memory, and what they compile at run time, without a GPU."""
 import ctypes
 import random
 import threading
@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer", "kernels_of_a_fused_group"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -121,6 +121,36 @@ def shared_memory_of_conv_integer(host):
             assert int(launch.split("lds=")[1].split()[0]) <= 64 * 1024, ((n, c, h, w, oc, k, stride, last, pad), launch)
             strips += "conv_strip_kernel" in launch
     assert strips > 20
+
+
+def kernels_of_a_fused_group(host):
+    """A call compiles the kernel it takes and no other, and calls that differ in ranks and extents share one: the general
+    kernel is one per way in which the operands are addressed."""
+    def call(program, dtype, shapes, strides=(None, None, None)):
+        ins = [host.tensor(dtype, s, st) for s, st in zip(shapes, strides)]
+        nd = max(len(s) for s in shapes)
+        out = host.tensor(dtype, [max(s[k - nd] if k - nd >= -len(s) else 1 for s in shapes) for k in range(nd)])
+        host.clear()
+        host.check(host.lib.chx_hip_elementwise(program.encode(), 5, host.capi.tensor_array(ins), len(ins), host.capi.tensor_array([out]), 1, None))
+        loads = sum(line == "hipModuleLoadData" for line in host.log())
+        return loads, [k.split()[0] for k in host.launches()]
+
+    text = "chxhip-fusion 1\nin a:%s b:%s c:%s\nm = Mul b c\ny = Add a m\nout y:%s\n"
+    # dense, a row, one per row: one to three axes, one row, a short last vector
+    ranks = [((9, 1001), (1001,), (9, 1)), ((2, 9, 77), (77,), (1, 9, 1)), ((5, 6, 333), (6, 333), (5, 6, 1)), ((3, 2, 19), (3, 1, 19), (2, 1))]
+    short = [((9, 3), (3,), (9, 1)), ((2, 9, 3), (9, 3), (2, 1, 3)), ((7, 2, 3), (1, 2, 1), (3,))]
+    for dtype in ("float16", "float32"):
+        program = text % ((dtype,) * 4)
+        for group in (ranks, short):
+            results = [call(program, dtype, shapes) for shapes in group]
+            assert results == [(1, ["fusion5_gen"])] + [(0, ["fusion5_gen"])] * (len(group) - 1), results
+        strided = [call(program, dtype, [(n, 21)] * 3, [[42, 2]] * 3) for n in (1, 5, 300)]
+        assert strided == [(1, ["fusion5_gen"]), (0, ["fusion5_gen"]), (0, ["fusion5_gen"])]
+    # the vector kernel, and the general one when a call needs it
+    assert call(program, "float32", [(64, 64)] * 3) == (1, ["fusion5_vec"]) and call(program, "float32", [(8, 128)] * 3) == (0, ["fusion5_vec"])
+    assert call(program, "float32", [(3, 7)] * 3) == (1, ["fusion5_gen"]) and call(program, "float32", [(2, 3, 5)] * 3) == (0, ["fusion5_gen"])
+    # which of them a general call needs does not make the vector kernel another
+    assert call(program, "float32", [(64, 64)] * 3) == (0, ["fusion5_vec"]) and call(program, "float32", [(4, 8, 8, 4)] * 3) == (0, ["fusion5_vec"])
 
 
 if __name__ == "__main__":
