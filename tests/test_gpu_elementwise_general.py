@@ -52,3 +52,25 @@ def test_codes_of_every_count(g, oracle, n):
         np.testing.assert_array_equal(g.host(out[0]), oracle.quantize_linear(s, 0.06, 7, np.int8))
         if mixed:
             np.testing.assert_array_equal(g.host(out[1]), s)
+
+
+def test_operands_that_reach_far_or_backwards(g):
+    """64-bit offsets: rows 2^31 elements apart, and strides below zero."""
+    import ctypes
+    rng = np.random.default_rng(4)
+    prog = g.ops.fusion_program([(n, torch.float16) for n in "ab"], [("y", "Sub", "a", "b")], [("y", torch.float16)])
+    far = torch.empty((1 << 31) + 4096, dtype=torch.float16, device="cuda").as_strided((2, 1001), (1 << 31, 1))
+    near = g.dev(rng.standard_normal((2, 1001)).astype(np.float16))
+    far.copy_(g.dev(rng.standard_normal((2, 1001)).astype(np.float16)))
+    row = near[0]
+    for a, b in [(far, near), (row, far), (far, far)]:
+        assert torch.equal(g.ops.ElementWiseNvrtc([a, b], 1, prog, 23)[0], a - b)
+    # descriptors made by hand: torch has no strides below zero
+    src = g.dev(rng.standard_normal((3, 40)).astype(np.float16))
+    out = torch.empty((3, 40), dtype=torch.float16, device="cuda")
+    backwards = g.capi.make_desc(src.data_ptr() + 2 * (3 * 40 - 1), g.capi.FLOAT16, (3, 40), (-80, -2))
+    ins = g.capi.tensor_array([backwards, g.capi.desc(src)])
+    outs = g.capi.tensor_array([g.capi.desc(out)])
+    code = prog.encode() if isinstance(prog, str) else prog
+    g.capi.check(g.capi.lib().chx_hip_elementwise(code, 24, ins, 2, outs, 1, g.capi.stream_ptr()))
+    assert torch.equal(out, src.flip(0, 1) - src)
