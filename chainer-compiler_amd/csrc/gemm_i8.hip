@@ -19,6 +19,7 @@
 //
 // Rows of any length and alignment: a group of 16 k that reaches past K is read as the last 16 bytes of its row and
 // shifted down (zeros move in), and likewise a dword that reaches past N as the last 4 bytes, so no access leaves a row.
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -43,35 +44,107 @@ struct GemmI8Args {
     int32_t tiles_m, tiles, tiles_per_xcd;
     // epilogue
     int32_t requant, rne;
+    int32_t finish;       // Finish
     float b_scale;
     const int32_t* bias;
     RequantParams rq;
+    float inv_y_scale, lo_folded;  // for kFolded*
+    QuantProduct qp;               // for kProduct*
 };
 
-// Four neighbouring results n .. n+3 of one row.
+// How a sum becomes a code.  kProduct + path and the folded forms give the codes of the exact ones (quant_math.h) wherever
+// no intermediate value leaves the range of float32, which the launcher checks; the exact ones divide, about twice the
+// instructions: QLinearMatMul of 8192 x 256 x 8192, whose results are many for its products, 113 us with them and 60 without.
+enum Finish : int32_t { kFolded = 0, kProduct1 = 1, kProduct2 = 2, kProduct3 = 3, kFoldedRne = 4, kExact = 5 };
+
+// Four neighbouring int32 results n .. n+3 of one row.
 __device__ __forceinline__ void store4(const GemmI8Args& g, char* y, int m, int n, v4i acc) {
     if (m >= g.M || n >= g.N) return;
-    char* row = y + (int64_t)m * g.y_row;
-    if (!g.requant) {
-        typedef int v4i_d __attribute__((ext_vector_type(4), aligned(4)));
-        int32_t* p = reinterpret_cast<int32_t*>(row) + n;
-        if (n + 4 <= g.N) __builtin_nontemporal_store(acc, reinterpret_cast<v4i_d*>(p));
-        else
-            for (int i = 0; i < 3; ++i)
-                if (n + i < g.N) p[i] = acc[i];
-        return;
-    }
-    int32_t code[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int32_t bias = g.bias ? g.bias[n + i < g.N ? n + i : g.N - 1] : 0;
-        code[i] = g.rne ? requantize_value<true>(acc[i], g.b_scale, bias, g.rq) : requantize_value<false>(acc[i], g.b_scale, bias, g.rq);
-    }
-    uint8_t* p = reinterpret_cast<uint8_t*>(row) + n;
-    if (n + 4 <= g.N) *reinterpret_cast<u32_u*>(p) = pack4(code[0], code[1], code[2], code[3]);
+    typedef int v4i_d __attribute__((ext_vector_type(4), aligned(4)));
+    int32_t* p = reinterpret_cast<int32_t*>(y + (int64_t)m * g.y_row) + n;
+    if (n + 4 <= g.N) __builtin_nontemporal_store(acc, reinterpret_cast<v4i_d*>(p));
     else
         for (int i = 0; i < 3; ++i)
-            if (n + i < g.N) p[i] = (uint8_t)code[i];
+            if (n + i < g.N) p[i] = acc[i];
+}
+
+// The codes of such results in kRows (1, 2 or 4) rows m[..].
+template <int kFinish, int kRows>
+__device__ __forceinline__ void store_codes(const GemmI8Args& g, char* y, const int (&m)[kRows], int n, const v4i (&acc)[kRows], v4i bias) {
+    uint32_t word[kRows];
+    const float s = g.rq.x_scale * g.b_scale;
+    if constexpr (kFinish == kProduct1 || kFinish == kProduct2 || kFinish == kProduct3) {
+        float pre[4 * kRows];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pre[4 * r + i] = quantize_prefloor_u8<kFinish>((float)(acc[r][i] + bias[i]) * s, g.qp);
+        if constexpr (kRows == 4) floor_sat_u8x16(pre, word);
+        else if constexpr (kRows == 2) floor_sat_u8x8(pre, &word[0], &word[1]);
+        else word[0] = floor_sat_u8x4(pre[0], pre[1], pre[2], pre[3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            int32_t code[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int32_t v = acc[r][i] + bias[i];
+                if constexpr (kFinish == kFolded) code[i] = quantize_value_folded<false>((float)v * s, g.rq.q, g.inv_y_scale, g.lo_folded);
+                else if constexpr (kFinish == kFoldedRne) code[i] = quantize_value_folded<true>((float)v * s, g.rq.q, g.inv_y_scale, g.lo_folded);
+                else code[i] = g.rne ? requantize_value<true>(v, g.b_scale, 0, g.rq) : requantize_value<false>(v, g.b_scale, 0, g.rq);
+            }
+            word[r] = pack4(code[0], code[1], code[2], code[3]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        if (m[r] >= g.M || n >= g.N) continue;
+        uint8_t* p = reinterpret_cast<uint8_t*>(y + (int64_t)m[r] * g.y_row) + n;
+        if (n + 4 <= g.N) *reinterpret_cast<u32_u*>(p) = word[r];
+        else
+            for (int i = 0; i < 3; ++i)
+                if (n + i < g.N) p[i] = (uint8_t)(word[r] >> (8 * i));
+    }
+}
+
+// A lane's results in kCount rows: sum(i) gives the four of row(i), for i < count (the same in every lane).
+template <int kCount, class Row, class Sum>
+__device__ __forceinline__ void store_all(const GemmI8Args& g, char* y, int n, int count, Row row, Sum sum) {
+    if (!g.requant) {
+#pragma unroll
+        for (int i = 0; i < kCount; ++i)
+            if (i < count) store4(g, y, row(i), n, sum(i));
+        return;
+    }
+    v4i bias = {0, 0, 0, 0};  // (the ONNX kind: added to the sum)
+    if (g.bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[i] = g.bias[n + i < g.N ? n + i : g.N - 1];
+    }
+    auto finish = [&](auto how) {
+        constexpr int kRows = kCount % 4 == 0 ? 4 : kCount % 2 == 0 ? 2 : 1;
+#pragma unroll
+        for (int i = 0; i < kCount; i += kRows) {
+            if (i < count) {
+                int m[kRows];
+                v4i acc[kRows];
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) {
+                    m[r] = row(i + r);
+                    acc[r] = sum(i + r);
+                }
+                store_codes<decltype(how)::value, kRows>(g, y, m, n, acc, bias);
+            }
+        }
+    };
+    switch (g.finish) {
+        case kProduct1: return finish(std::integral_constant<int, kProduct1>());
+        case kProduct2: return finish(std::integral_constant<int, kProduct2>());
+        case kProduct3: return finish(std::integral_constant<int, kProduct3>());
+        case kFolded: return finish(std::integral_constant<int, kFolded>());
+        case kFoldedRne: return finish(std::integral_constant<int, kFoldedRne>());
+        default: return finish(std::integral_constant<int, kExact>());
+    }
 }
 
 // Work-groups go round-robin over the 8 XCDs: each XCD takes a contiguous run of tiles, m fastest, so the work-groups
@@ -231,21 +304,19 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_i8_split_kernel(GemmI8Args g) 
         }
     }
     if constexpr (W == 1) {
-#pragma unroll
-        for (int r = 0; r < kRegs; ++r) store4(g, y, m0 + row_of(r), n, v4i{acc[0][r], acc[1][r], acc[2][r], acc[3][r]});
+        store_all<kRegs>(g, y, n, kRegs, [&](int r) { return m0 + row_of(r); }, [&](int r) { return v4i{acc[0][r], acc[1][r], acc[2][r], acc[3][r]}; });
     } else {
 #pragma unroll
         for (int r = 0; r < kRegs; ++r) part[wave][r][lane] = v4i{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
         __syncthreads();
-#pragma unroll
-        for (int r0 = 0; r0 < kRegs; r0 += W) {
-            const int r = r0 + wave;
-            if (r >= kRegs) break;
+        constexpr int kMine = (kRegs + W - 1) / W;  // register r0 = wave, wave + W, ... of every wavefront's
+        store_all<kMine>(g, y, n, kRegs >= W || wave < kRegs ? kMine : 0, [&](int i) { return m0 + row_of(i * W + wave); }, [&](int i) {
+            const int r = i * W + wave;
             v4i sum = part[0][r][lane];
 #pragma unroll
             for (int w = 1; w < W; ++w) sum += part[w][r][lane];
-            store4(g, y, m0 + row_of(r), n, sum);
-        }
+            return sum;
+        });
     }
 }
 
@@ -408,21 +479,21 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(GemmI8Args g) {
                 for (int r = 0; r < 16; ++r) acc[t][i][r] += add;
         }
     }
+    auto row_of = [&](int r) { return (r / 4) * 8 + group * 4 + r % 4; };
+    if (any_cb) {
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int32_t mine = any_cb ? row_sum[t] + __shfl_xor(row_sum[t], 32) + g.K * ca : 0;
+        for (int t = 0; t < MT; ++t) {
+            const int32_t mine = row_sum[t] + __shfl_xor(row_sum[t], 32) + g.K * ca;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = (r / 4) * 8 + group * 4 + r % 4;
-            v4i v = {acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]};
-            if (any_cb) {
-                const int32_t of_row = __shfl(mine, row);
+            for (int r = 0; r < 16; ++r) {
+                const int32_t of_row = __shfl(mine, row_of(r));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] += cb[i] * of_row;
+                for (int i = 0; i < 4; ++i) acc[t][i][r] += cb[i] * of_row;
             }
-            store4(g, y, m0 + 32 * t + row, n, v);
         }
     }
+    store_all<16 * MT>(g, y, n, 16 * MT, [&](int r) { return m0 + 32 * (r / 16) + row_of(r % 16); },
+                       [&](int r) { return v4i{acc[r / 16][0][r % 16], acc[r / 16][1][r % 16], acc[r / 16][2][r % 16], acc[r / 16][3][r % 16]}; });
 }
 
 template <int R, int W>
@@ -457,6 +528,17 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
     g.a_zp = m.a_zp_len ? m.a_zp : nullptr; g.a_zp_signed = m.a_zp_signed; g.a_zp_imm = m.a_zp_imm;
     g.b_zp = m.b_zp_len ? m.b_zp : nullptr; g.b_zp_len = m.b_zp_len; g.b_zp_stride = m.b_zp_stride; g.b_zp_signed = m.b_zp_signed; g.b_zp_imm = m.b_zp_imm;
     g.requant = m.requant; g.rne = rne ? 1 : 0; g.b_scale = m.b_scale; g.bias = m.bias; g.rq = m.rq;
+    if (m.requant) {
+        const QuantParams& q = m.rq.q;
+        const double largest = 0x1p31 * fabs((double)m.rq.x_scale * (double)m.b_scale);  // of the values to be quantized
+        g.finish = kExact;
+        if (q.scale > 1e-20f && q.scale < 1e20f && largest < 1e30 && largest / (double)q.scale < 1e30) {
+            g.inv_y_scale = 1.0f / q.scale;
+            g.lo_folded = fold_relu_floor(q, m.rq.relu_floor, rne);
+            g.qp = product_form(q, g.lo_folded, rne);
+            g.finish = rne ? kFoldedRne : g.qp.path;
+        }
+    }
     auto tiles = [&](int tm, int tn) {
         g.tiles_m = (int32_t)((m.M + tm - 1) / tm);
         const int64_t t = (int64_t)g.tiles_m * ((m.N + tn - 1) / tn);

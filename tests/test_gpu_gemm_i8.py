@@ -80,3 +80,47 @@ def test_views_into_larger_arrays(g):
         np.testing.assert_array_equal(g.host(out), exact(A[3:70, off:off + 201], B[5:206, off:off + 333], 0, 0))
         y[2:69, off:off + 333] = 0
         assert not y.any()
+
+
+# enough tiles of 256 x 128 and K for gemm_i8_tile_kernel, with remainders of each
+LARGE = (4099, 2070, 1037)
+ROWS = sorted({0, 1, 30, 31, 32, 63, 64, 127, 128, 255, 256, 257, 1023, 2047, 4095, 4096, 4097, 4098})
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_large_products(g, oracle, transposed):
+    M, N, K = LARGE
+    rng = np.random.default_rng(1)
+    a, b = codes(rng, (M, K), np.uint8), codes(rng, (K, N), np.int8)
+    bd = g.dev(np.ascontiguousarray(b.T)).t() if transposed else g.dev(b)
+    bz = rng.integers(-9, 9, size=N).astype(np.int8)
+    for az, z in [(128, np.zeros((), np.int8)), (3, bz)]:
+        got = g.ops.MatMulInteger(g.dev(a), bd, g.dev(np.array(az, np.uint8)), g.dev(z))
+        want = np.matmul(a.astype(np.float64) - az, b.astype(np.float64) - z).astype(np.int32)  # (exact: below 2^53)
+        np.testing.assert_array_equal(g.host(got), want)
+    s_y = float(0.02 * 0.005 * 74 * 74 * np.sqrt(K) / 40)
+    for zp, fl, dt in [(0, 0, torch.uint8), (128, g.capi.FUSE_RELU, torch.uint8), (-5, g.capi.ROUND_ONNX_RNE, torch.int8)]:
+        got = g.host(g.ops.QLinearMatMul(g.dev(a), 0.02, 117, bd, 0.005, 4, s_y, zp, None, flags=fl, zero_point_dtype=dt))
+        want = oracle.qlinear_matmul_int(a[ROWS], 0.02, 117, b, 0.005, 4, s_y, zp, y_dtype=np.uint8 if dt == torch.uint8 else np.int8, relu=fl == g.capi.FUSE_RELU,
+                                         round_mode=oracle.ROUND_ONNX_RNE if fl == g.capi.ROUND_ONNX_RNE else oracle.ROUND_REFERENCE)
+        np.testing.assert_array_equal(got[ROWS], want)
+
+
+# shapes by the wavefronts that share a tile's rows out, and ragged columns
+@pytest.mark.parametrize("M,N,K", [(16, 64, 16), (40, 70, 64), (33, 130, 400), (300, 258, 2000), (1030, 515, 40), (2100, 1031, 144)])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -3, 1e-25, 1e25])
+def test_every_form_of_the_requantization(g, oracle, M, N, K, scale):
+    """The short forms, the folded ones and, at scales whose values might leave float32's range on the way, the divisions."""
+    rng = np.random.default_rng(M + K)
+    a, b, bias = codes(rng, (M, K), np.uint8), codes(rng, (K, N), np.int8), rng.integers(-3000, 3000, size=N).astype(np.int32)
+    rows = [r for r in ROWS if r < M - 1] + [M - 1]
+    s_a = 0.02 * scale
+    s_y = float(np.float32(s_a * 0.005 * 74 * 74 * np.sqrt(K) / 45))
+    for zp, relu, rne, dt in [(0, False, False, torch.uint8), (0, True, False, torch.uint8), (128, False, False, torch.uint8), (9, True, False, torch.uint8),
+                              (3, False, False, torch.int8), (-7, True, False, torch.int8), (120, False, True, torch.uint8), (5, True, True, torch.int8)]:
+        fl = (g.capi.ROUND_ONNX_RNE if rne else 0) | (g.capi.FUSE_RELU if relu else 0)
+        for bd, bq in [(g.dev(bias), bias), (None, None)]:
+            got = g.host(g.ops.QLinearMatMul(g.dev(a), s_a, 117, g.dev(b), 0.005, 0, s_y, zp, bd, flags=fl, zero_point_dtype=dt))
+            want = oracle.qlinear_matmul_int(a[rows], s_a, 117, b, 0.005, 0, s_y, zp, bias=bq, y_dtype=np.uint8 if dt == torch.uint8 else np.int8, relu=relu,
+                                             round_mode=oracle.ROUND_ONNX_RNE if rne else oracle.ROUND_REFERENCE)
+            np.testing.assert_array_equal(got[rows], want)
