@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_i8_split_kernel(GemmI8Args g) 
 // wavefront fetches and transposes the columns of one quarter of the step and leaves them in LDS, where all four read
 // them (lane for lane as they were written: no bank conflicts); a's fragments have one reader each and come straight
 // from memory.  Two steps in flight in registers, two LDS stages, one barrier per step.  For large products, where the
-// wavefronts of the split kernel would transpose b once each: 4096 x 4096 x 4096 in 118 us (1160 TOP/s) against 174.
+// wavefronts of the split kernel would transpose b once each: 4096 x 4096 x 4096 in 125 us (1100 TOP/s) against 176.
 template <bool kBT>
 __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(GemmI8Args g) {
     constexpr int MT = 2;  // MFMA tiles along a wavefront's rows
@@ -333,7 +333,10 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(GemmI8Args g) {
     if (tile >= g.tiles || (int)(blockIdx.x >> 3) >= g.tiles_per_xcd) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, group = lane >> 5;
-    const int m0 = ((tile % g.tiles_m) * 4 + wave) * 32 * MT, n0 = (tile / g.tiles_m) * 128;
+    // Tiles go in bands of eight along M, n slowest inside: the 32 that an XCD has at a time read 8 runs of rows and 4 of
+    // columns (with m alone fastest 32 runs of rows, more than its 4 MB of L2 from K = 512 on; 8192 x 1024 x 8192 184 -> 171 us)
+    const int tiles_n = g.tiles / g.tiles_m, band = tile / (8 * tiles_n), in_band = tile - band * 8 * tiles_n, height = min(8, g.tiles_m - 8 * band);
+    const int m0 = ((8 * band + in_band % height) * 4 + wave) * 32 * MT, n0 = (in_band / height) * 128;
     const char* a = g.a + (int64_t)blockIdx.z * g.a_batch;
     const char* b = g.b + (int64_t)blockIdx.z * g.b_batch;
     char* y = g.y + (int64_t)blockIdx.z * g.y_batch;
@@ -548,9 +551,14 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
     };
     if (((m.M + 15) / 16) * ((m.N + 63) / 64) >= (int64_t(1) << 28)) return CHX_HIP_EUNSUPPORTED;
     auto grid = [&]() { return dim3((unsigned)(8 * g.tiles_per_xcd), 1, (unsigned)batch); };
-    // a compute unit for every tile, and K long enough that the loop, not the start and the result, is the time
-    // (2048 x 512 x 4096, 256 tiles: the same 15.7 us on both kernels)
-    if (m.N >= 4 && m.K >= 1024 && tiles(256, 128) * batch >= 256) {
+    // A compute unit for every tile, and K long enough that the loop, not the start and the result, is the time.  us on the
+    // split kernel / on this one, int32 results and codes:
+    //                        K = 256                     512                      768                       1024
+    //    2048 x K x 4096   13.3 / 14.2  12.8 / 13.0   16.6 / 17.1  17.2 / 16.4   21.7 / 20.8  22.9 / 20.1   25.6 / 23.4  26.0 / 22.8
+    //    4096 x K x 4096   20.9 / 27.4  19.3 / 22.5   29.7 / 34.0  30.3 / 29.6   40.9 / 40.6  40.7 / 36.7   49.1 / 45.7  47.8 / 41.8
+    //    8192 x K x 8192   70.0 / 89.8  60.0 / 76.4    105 / 118    101 / 105     151 / 148    142 / 133     181 / 171    171 / 154
+    //   16384 x K x 1024   22.0 / 27.3  20.2 / 22.0   32.2 / 33.7  30.7 / 28.7   45.1 / 41.3  41.1 / 36.0
+    if (m.N >= 4 && m.K >= 768 && tiles(256, 128) * batch >= 256) {
         if (b_transposed) gemm_i8_tile_kernel<true><<<grid(), 256, 0, s>>>(g);
         else gemm_i8_tile_kernel<false><<<grid(), 256, 0, s>>>(g);
         return launch_check("gemm_i8_tile_kernel");
