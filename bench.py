@@ -224,7 +224,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
                         bytes_per_step=model["depthwise_bytes"], kernel_ms_per_step=conv_ms_per_step)
     else:
         achieved = conv_ops / (conv_ms_per_step * 1e-3) / 1e12
-        roofline = dict(bound="mfma", kernel="QLinearConv launches of one step, summed (%d: conv_mfma_kernel, the first layer conv_stem_kernel)" % n_launch,
+        roofline = dict(bound="mfma", kernel="QLinearConv launches of one step, summed (%d)" % n_launch,
                         achieved=achieved, peak=INT8_PEAK_TOPS, unit="TOP/s", frac=achieved / INT8_PEAK_TOPS, traffic=None,
                         ops_per_step=conv_ops, kernel_ms_per_step=conv_ms_per_step)
     # The same launches against BOTH roofs: a launch is priced at the roof that takes longer for its algorithmic
@@ -260,7 +260,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
             pass
     # the launch configurations the plans measured for these launches: tile (output channels x pixels),
     # work-groups per compute unit (0 = as many as fit) and wavefronts per work-group -> number of layers
-    hist, forms = {}, {}
+    hist, forms, kernels = {}, {}, {}
     for rn, _xs in slices:
         for plan in rn.plans.values():
             for line in plan.describe():
@@ -272,7 +272,12 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
                     continue
                 key = "%s/%s/w%s%s" % (f.get("tile"), f.get("wgs_per_cu"), f.get("waves", "4"), "+res" if f.get("res") == "1" else "")
                 hist[key] = hist.get(key, 0) + 1
+                kernels[_kernel_of(f)] = kernels.get(_kernel_of(f), 0) + 1
     roofline["configs"] = hist
+    if not mobilenet:
+        planar = n_launch - sum(kernels.values())
+        roofline["kernel"] = "QLinearConv launches of one step, summed (%d: %s)" % (
+            n_launch, ", ".join("%d %s" % (n, k) for k, n in sorted(kernels.items(), key=lambda kv: -kv[1]) + ([("conv_stem_kernel", planar)] if planar > 0 else [])))
     roofline["configs_source"] = ("plans of the Python runner (ops.py), whose launches the kernel time above is measured on; the "
                                   "plans inside the C++ VM measure their own configurations and may choose differently")
     if forms:
@@ -321,6 +326,14 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
             vm_prog.close()
         timed_runner.close()
     return res, roofline, cpu, runner_close
+
+
+def _kernel_of(config):
+    """The kernel behind a launch configuration of a plan (QLinearConvPlan.describe)."""
+    oc, px = (int(v) for v in config["tile"].split("x"))
+    if (oc, px, config.get("waves")) == (64, 32, "4"):
+        return "conv_point_kernel"
+    return "conv_split_kernel" if oc <= 32 else "conv_mfma_kernel"
 
 
 def _literal_executor(orc):
@@ -388,7 +401,8 @@ def bench_conv3x3(args, torch, pkg):
     torch.cuda.synchronize()
     ms, cnt = ev0.elapsed_time(ev1), args.steps
     achieved = 2.0 * mac / (ms / cnt * 1e-3) / 1e12
-    roofline = dict(bound="mfma", kernel="conv_mfma_kernel", achieved=achieved, peak=INT8_PEAK_TOPS, unit="TOP/s",
+    chosen = dict(kv.split("=") for kv in plan.describe()[0].split() if "=" in kv)
+    roofline = dict(bound="mfma", kernel=_kernel_of(chosen), achieved=achieved, peak=INT8_PEAK_TOPS, unit="TOP/s",
                     frac=achieved / INT8_PEAK_TOPS, traffic=None, ops_per_launch=2.0 * mac, launch_us=ms / cnt * 1e3)
     res = dict(metric="images/sec QLinearConv 3x3 128->128 @28x28 (ResNet-50 stage 3), 1 GPU", value=n / sec,
                unit="images/sec", ms_per_step=sec * 1e3, dtype="int8",
