@@ -92,7 +92,7 @@ static ProductForms find_forms(const QuantParams& q) {
 
 // Finding them takes about 25 us, for each of a network's layers: the process remembers them by scale and zero point, for
 // every plan, plan-less call and thread.  (A ResNet-50 has 54 pairs; a table of 256 places found by a hash alone had
-// four of them evict each other, 82 us of every interpreted run.)  2000 pairs are some 200 KB; more start over.
+// four of them evict each other: a pass through the 54 took 283 us of host time instead of 136.)  2000 pairs are some 200 KB; more start over.
 static ProductForms known_forms(const QuantParams& q) {
     static std::mutex* mutex = new std::mutex;  // (never destroyed: calls may come from other destructors)
     static auto* known = new std::unordered_map<uint64_t, ProductForms>;
