@@ -681,11 +681,11 @@ void emit_general(const Program& prog, const std::string& name, const GeneralFor
     os << "__device__ __forceinline__ gidx offset(const long long (&stride)[" << kAxes << "], const gidx (&at)[" << g.axes << "]) {\n  gidx off = 0;\n";
     os << "#pragma unroll\n  for (int a = 0; a < " << g.axes << "; ++a) off += at[a] * (gidx)stride[a];\n  return off;\n}\n";
 
-    os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_gen(unsigned long long total";
+    os << "extern \"C\" __global__ __launch_bounds__(256) void " << name << "_gen(unsigned long long total, unsigned long long first";
     for (size_t i = 0; i < nin; ++i) os << ", const " << ctype_of(prog.inputs[i].dtype) << "* __restrict__ i" << i;
     for (size_t i = 0; i < nout; ++i) os << ", " << ctype_of(prog.outputs[i].dtype) << "* __restrict__ o" << i;
     os << ", GenDesc d) {\n";
-    os << "  const gidx n = (gidx)total, base = ((gidx)blockIdx.x * 256u + threadIdx.x) * " << V << "u;\n";
+    os << "  const gidx n = (gidx)total, base = (gidx)first + ((gidx)blockIdx.x * 256u + threadIdx.x) * " << V << "u;\n";
     os << "  if (base >= n) return;\n";
     os << "  const int cnt = n - base < " << V << "u ? (int)(n - base) : " << V << ";\n";
     // What an operand's elements are as loaded: a vector, and converted behind the last of the loads only (a conversion
@@ -1269,7 +1269,7 @@ struct PreparedCall {
     bool vector = false;
     int vec = 0;
     int64_t n = 0;
-    unsigned grid = 0;
+    int64_t blocks = 0;
     std::vector<char> desc;  // GenDesc of the general kernel
 };
 constexpr size_t kMostPrepared = 4096;  // (a few hundred bytes each; all are dropped when there are more)
@@ -1300,10 +1300,11 @@ int prepare_call(
     CHX_PROPAGATE(get_compiled(src, name, &call->kernel));
     CHX_PROPAGATE(load_kernel(call->kernel.get(), name + (call->vector ? "_vec" : "_gen")));
     if (call->vector) {
-        call->grid = (unsigned)((plan.n / plan.vec + 511) / 512);
+        call->blocks = (plan.n / plan.vec + 511) / 512;
         return CHX_HIP_OK;
     }
-    call->grid = (unsigned)((plan.n + 256 * plan.gen.vec - 1) / (256 * plan.gen.vec));
+    call->vec = plan.gen.vec;
+    call->blocks = (plan.n + 256 * plan.gen.vec - 1) / (256 * plan.gen.vec);
     // GenDesc { unsigned mul[kAxes], shift[kAxes]; long long shape[kAxes], istr[nin][kAxes]; }
     const size_t M = kAxes;
     call->desc.assign(2 * M * 4 + M * 8 + (size_t)n_inputs * M * 8, 0);
@@ -1350,13 +1351,23 @@ extern "C" int chx_hip_elementwise(
         g_prepared.emplace(std::move(key), call);
     }
     if (call->n == 0) return CHX_HIP_OK;
-    ArgPacker a;
-    if (call->vector) a.push((uint32_t)(call->n / call->vec));
-    else a.push((unsigned long long)call->n);
-    for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
-    for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
-    if (!call->vector) a.push_bytes(call->desc.data(), call->desc.size(), 8);
-    return launch(call->kernel->function, call->grid, a, as_stream(stream));
+    // a launch has fewer than 2^32 threads (fewer than 2^31 elements, and one launch, for the vector kernel)
+    constexpr int64_t kMostBlocks = int64_t(1) << 23;
+    for (int64_t block = 0; block < call->blocks; block += kMostBlocks) {
+        ArgPacker a;
+        if (call->vector) {
+            a.push((uint32_t)(call->n / call->vec));
+        } else {
+            a.push((unsigned long long)call->n);
+            a.push((unsigned long long)(block * 256 * call->vec));
+        }
+        for (int i = 0; i < n_inputs; ++i) a.push(inputs[i]->data);
+        for (int i = 0; i < n_outputs; ++i) a.push(outputs[i]->data);
+        if (!call->vector) a.push_bytes(call->desc.data(), call->desc.size(), 8);
+        const int64_t left = call->blocks - block;
+        CHX_PROPAGATE(launch(call->kernel->function, (unsigned)(left < kMostBlocks ? left : kMostBlocks), a, as_stream(stream)));
+    }
+    return CHX_HIP_OK;
 }
 
 extern "C" int chx_hip_elementwise_match_residual_add(const char* code, int32_t* matches, chx_hip_residual_group* group) {

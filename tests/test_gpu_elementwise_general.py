@@ -74,3 +74,13 @@ def test_operands_that_reach_far_or_backwards(g):
     code = prog.encode() if isinstance(prog, str) else prog
     g.capi.check(g.capi.lib().chx_hip_elementwise(code, 24, ins, 2, outs, 1, g.capi.stream_ptr()))
     assert torch.equal(out, src.flip(0, 1) - src)
+
+
+def test_more_elements_than_one_launch_takes(g):
+    prog = g.ops.fusion_program([(n, torch.float16) for n in "ab"], [("y", "Add", "a", "b")], [("y", torch.float16)])
+    rows = (1 << 30) + 5  # of three: an element per thread, two launches
+    a = torch.arange(rows, device="cuda", dtype=torch.int32).remainder_(997).to(torch.float16).unsqueeze(1)
+    b = torch.tensor([1.0, 2.0, 4.0], device="cuda", dtype=torch.float16)
+    y = g.ops.ElementWiseNvrtc([a, b], 1, prog, 25)[0]
+    for k in range(3):
+        assert torch.equal(y[:, k], a[:, 0] + b[k])

@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer", "kernels_of_a_fused_group"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer", "kernels_of_a_fused_group", "fused_groups_of_many_elements"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -151,6 +151,20 @@ def kernels_of_a_fused_group(host):
     assert call(program, "float32", [(3, 7)] * 3) == (1, ["fusion5_gen"]) and call(program, "float32", [(2, 3, 5)] * 3) == (0, ["fusion5_gen"])
     # which of them a general call needs does not make the vector kernel another
     assert call(program, "float32", [(64, 64)] * 3) == (0, ["fusion5_vec"]) and call(program, "float32", [(4, 8, 8, 4)] * 3) == (0, ["fusion5_vec"])
+
+
+def fused_groups_of_many_elements(host):
+    """A launch has fewer than 2^32 threads; a group of more elements than those of one launch take is several."""
+    memory = host.malloc(64)
+    for dtype, rows, row in [("float32", 1 << 31, 3), ("float32", 5 << 20, 1001), ("float16", 1 << 31, 5), ("float16", 1 << 34, 1)]:
+        text = "chxhip-fusion 1\nin a:%s b:%s\ny = Add a b\nout y:%s\n" % ((dtype,) * 3)
+        wide, one, out = host.tensor(dtype, (rows, row), base=memory), host.tensor(dtype, (rows, 1), base=memory), host.tensor(dtype, (rows, row), base=memory)
+        host.clear()
+        host.check(host.lib.chx_hip_elementwise(text.encode(), 6, host.capi.tensor_array([wide, one]), 2, host.capi.tensor_array([out]), 1, None))
+        grids = [int(k.split("grid=")[1]) for k in host.launches()]
+        assert max(grids) * 256 < 1 << 32 and len(grids) >= 1, grids
+        per_thread = 1 if row in (3, 5) else 8 if dtype == "float16" else 4
+        assert sum(grids) == -(-rows * row // (256 * per_thread)), grids
 
 
 if __name__ == "__main__":
