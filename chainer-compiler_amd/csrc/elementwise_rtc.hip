@@ -648,8 +648,9 @@ constexpr int kAxes = CHX_HIP_MAX_NDIM;
 // read element by element from two positions.  (Of rows shorter than that a thread computes one element: every run would
 // cross.)  Divisions by the extents are multiplications with their reciprocals.
 // Axes are collapsed ones, the innermost first; those past the last have extent 1, so that the rank of a call is no part of
-// its kernel (a compilation takes 0.3 s of the first call); a kernel for each rank ran the chain below in 16.1 us instead of
-// 16.5 in float32 on [16, 333, 1001], and no faster elsewhere.  The operands' addressing is: as an argument it made the chain
+// its kernel (a compilation takes 0.3 s of the first call).  The kernel before, one for each rank and with
+// each operand converted beside its load, took 16.1 us for the chain below in float32 on [16, 333, 1001], this one 16.5; which
+// of the two differences costs it was not measured apart.  The operands' addressing is: as an argument it made the chain
 // below 17 % slower in float32 rows of 1001 (scalar loads behind each branch), which one kernel for all calls would cost.
 // Chain of two operands of [8, 333, 1001] and two of [1001] through Mul, Add, Tanh, Sigmoid, Mul, Add and Relu in float16:
 // 15.2 us with one element per thread and 64-bit divisions, 8.6 with each operand converted beside its load, 6.9 with all
