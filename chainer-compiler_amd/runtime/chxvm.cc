@@ -1,6 +1,7 @@
 #include "chxvm.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <fstream>
 #include <iomanip>
@@ -54,6 +55,91 @@ public:
 
 private:
     int a_, a_scale_, a_zp_, b_, b_scale_, b_zp_, y_scale_, y_zp_, y_;
+};
+
+std::atomic<int64_t> g_matmul_chains{0};
+
+// A chain of such products, with the QuantizeLinear in front of it and the DequantizeLinear behind it where nobody else
+// reads what lies between, as one launch (chx_hip_qlinear_chain).  It stands where the last of its instructions stood; what
+// that kernel does not take runs as the program wrote it.
+class QLinearMatMulChainOp : public ChxVMOp {
+public:
+    struct Layer {
+        int a_scale, a_zp, b_scale, b_zp, y_scale, y_zp;
+        std::shared_ptr<chx_hip_chain_weights> b;
+    };
+    // steps: the instructions that this one replaces and the Free's of their operands between them, in the program's order
+    QLinearMatMulChainOp(const ChxVMInstructionProto& last, const ChxVMInstructionProto* quantize, std::vector<Layer> layers, int64_t columns, int a,
+                         const ChxVMInstructionProto* dequantize, std::vector<ChxVMOp*> steps, std::vector<int> freed)
+        : ChxVMOp(last), quantize_(quantize != nullptr), dequantize_(dequantize != nullptr), x_(quantize ? quantize->inputs[0].array : a),
+          x_scale_(quantize ? quantize->inputs[1].scalar : -1), x_zp_(quantize ? quantize->inputs[2].scalar : -1),
+          y_scale_(dequantize ? dequantize->inputs[1].scalar : -1), y_zp_(dequantize ? dequantize->inputs[2].scalar : -1),
+          y_(last.outputs[0]), columns_(columns), layers_(std::move(layers)), steps_(std::move(steps)), freed_(std::move(freed)) {
+    }
+
+    void Run(ChxVMState* st) override {
+        if (RunAsOne(st)) {
+            for (int slot : freed_) st->FreeVar(slot);
+        } else {
+            for (ChxVMOp* op : steps_) op->Run(st);
+        }
+    }
+
+private:
+    // false: nothing has been written
+    bool RunAsOne(ChxVMState* st) {
+        auto is_null = [&](int slot) { return slot >= 0 && st->GetVar(slot)->IsNull(); };
+        if (is_null(x_) || is_null(x_scale_) || is_null(x_zp_) || is_null(y_scale_) || is_null(y_zp_)) return false;
+        for (const Layer& l : layers_)
+            if (is_null(l.a_scale) || is_null(l.a_zp) || is_null(l.b_scale) || is_null(l.b_zp) || is_null(l.y_scale) || is_null(l.y_zp)) return false;
+        auto zp_of = [&](int slot) -> StrictScalar {
+            absl::optional<StrictScalar> z = st->GetOptionalScalar(slot);
+            return z.has_value() ? *z : StrictScalar(chainerx::Dtype::kUInt8, chainerx::Scalar(0u), false);
+        };
+        auto integer = [](const StrictScalar& z) { return static_cast<int32_t>(static_cast<int64_t>(z)); };
+        const chainerx::Array& x = st->GetArray(x_);
+        if (x.ndim() != 2) return false;
+        const StrictScalar x_zp = zp_of(x_zp_);
+        std::vector<chx_hip_chain_layer> layers(layers_.size());
+        chainerx::Dtype dtype = chainerx::Dtype::kFloat32;
+        for (size_t i = 0; i < layers.size(); ++i) {
+            const Layer& in = layers_[i];
+            chx_hip_chain_layer& l = layers[i];
+            const StrictScalar y_zp = zp_of(in.y_zp);
+            l.b = in.b.get();
+            l.a_scale = static_cast<float>(st->GetScalar(in.a_scale));
+            l.b_scale = static_cast<float>(st->GetScalar(in.b_scale));
+            l.y_scale = static_cast<float>(st->GetScalar(in.y_scale));
+            l.a_zero_point = integer(zp_of(in.a_zp));
+            l.b_zero_point = integer(zp_of(in.b_zp));
+            l.y_zero_point = integer(y_zp);
+            l.y_dtype = static_cast<int32_t>(y_zp.dtype());
+            dtype = y_zp.dtype();
+        }
+        if (dtype != chainerx::Dtype::kUInt8 && dtype != chainerx::Dtype::kInt8) return false;
+        chainerx::Array y = chainerx::Empty(chainerx::Shape{x.shape()[0], columns_}, dequantize_ ? chainerx::Dtype::kFloat32 : dtype);
+        const chx_hip_tensor xt = x.hip();
+        chx_hip_tensor yt = y.hip();
+        const int rc = chx_hip_qlinear_chain(
+                &xt, quantize_ ? static_cast<float>(st->GetScalar(x_scale_)) : 1.f, quantize_ ? integer(x_zp) : 0,
+                static_cast<int32_t>(quantize_ ? x_zp.dtype() : x.dtype()), layers.data(), static_cast<int32_t>(layers.size()), &yt,
+                dequantize_ ? static_cast<float>(st->GetScalar(y_scale_)) : 1.f, dequantize_ ? integer(zp_of(y_zp_)) : 0, chainerx::CurrentStream());
+        // (what it refuses, and operands that are in error, are for the instructions)
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory)  // a recording may outlive the program
+            for (const Layer& l : layers_) st->options().recorded_memory->push_back(l.b);
+        st->SetArray(y_, y);
+        ++g_matmul_chains;
+        return true;
+    }
+
+    bool quantize_, dequantize_;
+    int x_, x_scale_, x_zp_, y_scale_, y_zp_, y_;
+    int64_t columns_;
+    std::vector<Layer> layers_;
+    std::vector<ChxVMOp*> steps_;
+    std::vector<int> freed_;
 };
 
 // DequantizeLinear, MaxPool | AveragePool, QuantizeLinear as one instruction on the 8-bit codes
@@ -583,12 +669,103 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             constants_.emplace_back(new ChxVMVar(*scratch.GetVar(slot)));
             constant_slots_[slot] = constants_.back().get();
         } else if (!dynamic_cast<NopOp*>(program_[i].get())) {
-            remaining_.push_back(i);
+            remaining_.emplace_back(i, program_[i].get());
         }
+    }
+    // Chains of fused products, for the same runs: every value between two links has one reader.  All slots involved are
+    // written once, so that the links may run where the last one stood.
+    std::vector<int> reader(num_variables_ > 0 ? num_variables_ : 1, -1);  // of a value that one instruction reads
+    for (int i = 0; i < n; ++i) {
+        const ChxVMInstructionProto& inst = program.instructions[i];
+        if (inst.op == kDequantize && !inst.inputs.empty() && inst.inputs[0].array >= 0) reader[inst.inputs[0].array] = i;
+    }
+    auto once = [&](int slot) { return slot < 0 || writers[slot] == 1; };
+    auto quantization_once = [&](const ChxVMInstructionProto& inst) {
+        return inst.inputs.size() == 3 && inst.inputs[0].array >= 0 && once(inst.inputs[0].array) && inst.inputs[1].scalar >= 0 &&
+               once(inst.inputs[1].scalar) && once(inst.inputs[2].scalar) && inst.outputs.size() == 1 && once(inst.outputs[0]);
+    };
+    std::map<int, std::shared_ptr<chx_hip_chain_weights>> laid_out;
+    auto link = [&](int q) {  // a fused product that may be part of a chain: its weights are a constant (laid out here, once)
+        if (role[q] != 2 || !quantization_once(program.instructions[q]) || !quantization_once(program.instructions[fused_inputs[q].first]) ||
+            !quantization_once(program.instructions[fused_inputs[q].second]))
+            return false;
+        const ChxVMVar* constant = constant_slots_[program.instructions[fused_inputs[q].second].inputs[0].array];
+        if (!constant || constant->kind() != ChxVMVar::Kind::kArray || laid_out.count(q)) return constant && laid_out.count(q) != 0;
+        const chainerx::Array& b = constant->GetArray();
+        if (b.ndim() != 2 || (b.dtype() != chainerx::Dtype::kUInt8 && b.dtype() != chainerx::Dtype::kInt8)) return false;
+        const chx_hip_tensor bt = b.hip();
+        chx_hip_chain_weights* w = nullptr;
+        const int rc = chx_hip_chain_weights_create(&bt, chainerx::CurrentStream(), &w);
+        if (rc == CHX_HIP_EUNSUPPORTED) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        laid_out[q] = std::shared_ptr<chx_hip_chain_weights>(w, chx_hip_chain_weights_destroy);
+        return true;
+    };
+    auto product_of = [&](int q, int slot) {  // the instruction that the value goes to, when that is as the left operand of a product
+        for (int next = q + 1; next < n; ++next)
+            if (role[next] == 2 && fused_inputs[next].first == reader[slot]) return next;
+        return -1;
+    };
+    constexpr size_t kMostLinks = 6;  // of chx_hip_qlinear_chain
+    std::vector<bool> chained(n, false);
+    for (int q = 0; q < n; ++q) {
+        if (chained[q] || !link(q)) continue;
+        std::vector<int> links = {q};
+        int y = program.instructions[q].outputs[0];
+        for (int next; links.size() < kMostLinks && single_use(y) && reader[y] >= 0 && (next = product_of(links.back(), y)) >= 0 && link(next);) {
+            links.push_back(next);
+            y = program.instructions[next].outputs[0];
+        }
+        const int a = program.instructions[fused_inputs[q].first].inputs[0].array, head = producer[a];
+        const bool quantize = head >= 0 && head < q && program.instructions[head].op == kQuantize && role[head] == 0 && single_use(a) &&
+                              quantization_once(program.instructions[head]);
+        const int tail = reader[y];
+        const bool dequantize = tail > links.back() && single_use(y) && program.instructions[tail].op == kDequantize && role[tail] == 0 &&
+                                quantization_once(program.instructions[tail]);
+        if (links.size() + quantize + dequantize < 2) continue;
+        std::set<int> members(links.begin(), links.end()), slots = {a};
+        if (quantize) members.insert(head);
+        if (dequantize) members.insert(tail);
+        std::vector<QLinearMatMulChainOp::Layer> layers;
+        for (int l : links) {
+            const ChxVMInstructionProto &da = program.instructions[fused_inputs[l].first], &db = program.instructions[fused_inputs[l].second], &qi = program.instructions[l];
+            layers.push_back({da.inputs[1].scalar, da.inputs[2].scalar, db.inputs[1].scalar, db.inputs[2].scalar, qi.inputs[1].scalar, qi.inputs[2].scalar, laid_out[l]});
+            for (int slot : {da.inputs[0].array, da.inputs[1].scalar, da.inputs[2].scalar, db.inputs[0].array, db.inputs[1].scalar, db.inputs[2].scalar, qi.inputs[1].scalar, qi.inputs[2].scalar}) slots.insert(slot);
+        }
+        for (int end : {quantize ? head : -1, dequantize ? tail : -1}) {
+            if (end < 0) continue;
+            const ChxVMInstructionProto& inst = program.instructions[end];
+            for (int slot : {inst.inputs[0].array, inst.inputs[1].scalar, inst.inputs[2].scalar}) slots.insert(slot);
+        }
+        const int64_t columns = constant_slots_[program.instructions[fused_inputs[links.back()].second].inputs[0].array]->GetArray().shape()[1];
+        const int first = *members.begin(), last = *members.rbegin();
+        std::vector<ChxVMOp*> steps;
+        std::vector<int> freed;
+        std::set<int> moved = members;
+        for (int i = first; i <= last; ++i) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            const bool frees = inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array);
+            if (frees) freed.push_back(inst.inputs[0].array);
+            if (frees && !dynamic_cast<NopOp*>(program_[i].get())) moved.insert(i);  // (the others run behind one of the members)
+            if (moved.count(i)) steps.push_back(program_[i].get());
+        }
+        chains_.emplace_back(new QLinearMatMulChainOp(program.instructions[last], quantize ? &program.instructions[head] : nullptr, std::move(layers), columns, a,
+                                                      dequantize ? &program.instructions[tail] : nullptr, std::move(steps), std::move(freed)));
+        for (int m : members) chained[m] = true;
+        std::vector<std::pair<int, ChxVMOp*>> rest;
+        for (const auto& r : remaining_) {
+            if (r.first == last) rest.emplace_back(last, chains_.back().get());
+            else if (!moved.count(r.first)) rest.push_back(r);
+        }
+        remaining_.swap(rest);
     }
 }
 
 ChxVM::~ChxVM() = default;
+
+int64_t MatMulChains() {
+    return g_matmul_chains.load();
+}
 
 void SetFuseResidual(bool on) {
     g_fuse_residual = on;
@@ -720,8 +897,9 @@ InOuts ChxVM::Run(const InOuts& program_inputs, const ChxVMOptions& options) {
         !options.chrome_tracing && options.dump_outputs_dir.empty()) {
         ChxVMState state(options, constant_slots_, program_inputs);
         state.set_minus_128_slots(&minus_128_slots_);
-        for (int pc : remaining_) {
-            ChxVMOp* op = program_[pc].get();
+        for (const auto& instruction : remaining_) {
+            const int pc = instruction.first;
+            ChxVMOp* op = instruction.second;
             state.set_pc(pc);
             try {
                 op->Run(&state);

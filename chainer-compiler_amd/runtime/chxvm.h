@@ -47,6 +47,8 @@ int64_t Minus128Stores();  // results written in that storage so far, process-wi
 // The plain uint8 array of a value held in that storage (chx_hip_codes_minus_128).
 chainerx::Array PlainCodes(const chainerx::Array& minus_128);
 
+int64_t MatMulChains();  // chains of quantized products run as one launch so far, process-wide
+
 class ChxVM {
 public:
     explicit ChxVM(const ChxVMProgramProto& program);
@@ -83,11 +85,12 @@ private:
     int num_variables_ = 0;
     int64_t residual_fusions_ = 0;
     // For runs that nothing looks into: the constants' variables (null: a slot that instructions write), made once, and the
-    // instructions that remain.  A network of 54 convolutions has 444 constants; setting them took a third of the
-    // interpreter's time.
+    // instructions that remain, with the place in the program each of them stands for.  A network of 54 convolutions has 444
+    // constants; setting them took a third of the interpreter's time.
     std::vector<std::unique_ptr<ChxVMVar>> constants_;
     std::vector<ChxVMVar*> constant_slots_;
-    std::vector<int> remaining_;
+    std::vector<std::pair<int, ChxVMOp*>> remaining_;
+    std::vector<std::unique_ptr<ChxVMOp>> chains_;  // what some of them run instead of the program's own
     std::vector<bool> minus_128_slots_;  // per variable: see ChxVMState::store_minus_128
 };
 

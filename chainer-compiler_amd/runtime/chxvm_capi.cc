@@ -150,6 +150,7 @@ struct chxvm_replay {
     HostResults results;
     int32_t warm_runs = 0;
     std::vector<chx_hip_qconv_plan*> pinned_plans;  // whose memory the graph's kernels address
+    std::vector<std::shared_ptr<void>> recorded_memory;
 
     ~chxvm_replay() {
         chx_hip_graph_destroy(graph);
@@ -331,6 +332,7 @@ int32_t chxvm_program_capture(
             chainerx::DeviceContextScope scope(r->stream, r->pool.get());
             ChxVMOptions recorded = options;
             recorded.pinned_plans = &r->pinned_plans;
+            recorded.recorded_memory = &r->recorded_memory;
             result = program->vm->Run(in, recorded);
         } catch (...) {
             chx_hip_graph* dropped = nullptr;
@@ -490,6 +492,7 @@ int64_t chxvm_counter(const char* name) {
     if (n == "qlinearconv_residual_fusions") return QLinearConvResidualFusions();
     if (n == "qlinearconv_pair_fusions") return QLinearConvPairFusions();
     if (n == "minus_128_stores") return Minus128Stores();
+    if (n == "matmul_chains") return MatMulChains();
     return -1;
 }
 

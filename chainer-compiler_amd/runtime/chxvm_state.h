@@ -40,6 +40,8 @@ struct ChxVMOptions {
     // set while a run is being recorded into a device graph: every convolution plan the run uses is pinned and listed
     // here, so that the recording can release them when it is destroyed (chx_hip_qconv_plan_pin)
     std::vector<struct chx_hip_qconv_plan*>* pinned_plans = nullptr;
+    // likewise: what else the recording's kernels address that belongs to the program
+    std::vector<std::shared_ptr<void>>* recorded_memory = nullptr;
 };
 
 class ChxVMState {

@@ -297,6 +297,29 @@ int chx_hip_qlinear_matmul(
         int32_t b_zero_point, float y_scale, int32_t y_zero_point, const chx_hip_tensor* bias, uint32_t flags,
         chx_hip_tensor* y, void* stream);
 
+/* Weights [K, N] of a layer of a chain, laid out for chx_hip_qlinear_chain: uint8 or int8, any strides, at most
+ * 1024 x 512 (CHX_HIP_EUNSUPPORTED beyond).  Waits for the stream; `b` is not needed afterwards. */
+typedef struct chx_hip_chain_weights chx_hip_chain_weights;
+int chx_hip_chain_weights_create(const chx_hip_tensor* b, void* stream, chx_hip_chain_weights** out);
+void chx_hip_chain_weights_destroy(chx_hip_chain_weights* weights);
+
+/* A layer of a chain of products: its weights, and the quantization of its input, of them and of its result. */
+typedef struct chx_hip_chain_layer {
+    const chx_hip_chain_weights* b;
+    float a_scale, b_scale, y_scale;
+    int32_t a_zero_point, b_zero_point, y_zero_point;
+    int32_t y_dtype; /* CHX_HIP_UINT8 or CHX_HIP_INT8 */
+} chx_hip_chain_layer;
+
+/* QuantizeLinear (x float32; left out for x of type x_dtype), n chx_hip_qlinear_matmul without bias, each on the codes
+ * of the one before, and DequantizeLinear (y float32; left out for y of the last layer's type) as one launch, with the
+ * codes of the single calls.  x [M, K] and y [M, N] in rows.  CHX_HIP_EUNSUPPORTED, with nothing launched, for more than
+ * 6 layers, more rows than one launch gains on, and anything that is not in rows or not consistent; the single calls then
+ * say what is wrong with it, if something is. */
+int chx_hip_qlinear_chain(
+        const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, int32_t x_dtype, const chx_hip_chain_layer* layers, int32_t n,
+        chx_hip_tensor* y, float y_scale, int32_t y_zero_point, void* stream);
+
 /* ---- float32 layers around a quantized network ------------------------------------------ */
 
 /* GemmOp::RunImpl, runtime/ops/math.cc:160-177:  r = op(a) . op(b);  r *= alpha when alpha != 1;
