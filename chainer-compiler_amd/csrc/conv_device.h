@@ -78,29 +78,53 @@ constexpr uint32_t kOutOfRange = 0x80000000u;
 // Touch every 64-byte line of the kernel arguments at once.  The argument block of a fresh launch
 // is not in any cache, and the compiler fetches the fields in several dependent batches that
 // each touch new lines: one round trip to memory per batch.  After this, one round trip.
+// (offset of line n, clamped into the block so that nothing outside it is read)
+template <int BYTES>
+constexpr int argument_line(int n) {
+    constexpr int LINES = (BYTES + 63) / 64;
+    static_assert(LINES >= 2 && LINES <= 9, "between two and nine lines are touched");
+    return 64 * (n < LINES ? n : LINES - 1);
+}
+#define CHX_TOUCH_ARGUMENTS                                                                             \
+    "s_load_dword %0, %9, 0x0\n\ts_load_dword %1, %9, 0x40\n\ts_load_dword %2, %9, %10\n\t"              \
+    "s_load_dword %3, %9, %11\n\ts_load_dword %4, %9, %12\n\ts_load_dword %5, %9, %13\n\t"              \
+    "s_load_dword %6, %9, %14\n\ts_load_dword %7, %9, %15\n\ts_load_dword %8, %9, %16\n\ts_waitcnt lgkmcnt(0)"
+#define CHX_ARGUMENT_LINES                                                                               \
+    "n"(argument_line<BYTES>(2)), "n"(argument_line<BYTES>(3)), "n"(argument_line<BYTES>(4)), "n"(argument_line<BYTES>(5)), \
+            "n"(argument_line<BYTES>(6)), "n"(argument_line<BYTES>(7)), "n"(argument_line<BYTES>(8))
 template <int BYTES>
 __device__ __forceinline__ void warm_kernel_arguments() {
     const uint64_t ka = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int LINES = (BYTES + 63) / 64;
-    static_assert(LINES >= 4 && LINES <= 9, "between four and nine lines are touched");
-    // offsets of the last lines, clamped into the block so that nothing outside it is read
-    constexpr int L4 = LINES > 4 ? 0x100 : 0xc0, L5 = LINES > 5 ? 0x140 : L4, L6 = LINES > 6 ? 0x180 : L5, L7 = LINES > 7 ? 0x1c0 : L6, L8 = LINES > 8 ? 0x200 : L7;
     int t0, t1, t2, t3, t4, t5, t6, t7, t8;
-    asm volatile(
-            "s_load_dword %0, %9, 0x0\n\t"
-            "s_load_dword %1, %9, 0x40\n\t"
-            "s_load_dword %2, %9, 0x80\n\t"
-            "s_load_dword %3, %9, 0xc0\n\t"
-            "s_load_dword %4, %9, %10\n\t"
-            "s_load_dword %5, %9, %11\n\t"
-            "s_load_dword %6, %9, %12\n\t"
-            "s_load_dword %7, %9, %13\n\t"
-            "s_load_dword %8, %9, %14\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8)
-            : "s"(ka), "n"(L4), "n"(L5), "n"(L6), "n"(L7), "n"(L8)
-            : "memory");
+    asm volatile(CHX_TOUCH_ARGUMENTS
+                 : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8)
+                 : "s"(ka), CHX_ARGUMENT_LINES
+                 : "memory");
 }
+
+// The arguments (the kernel's only parameter), touched, through a pointer that comes out of the assembly, so that no field
+// is fetched in front of it: the compiler moves loads of a parameter's fields across anything, and the small-tile convolution
+// (conv_split.hip) had a batch of them, one more round trip, in front.  For kernels whose time is their start: with the same
+// treatment of the integer divisions there, ResNet-50 on one image 287 -> 275 us.  The staged convolution
+// (conv_mfma_kernel.h) is 4 % slower on one layer this way (128 -> 128 3x3, 32 images of 28x28: 9.8 and 10.2 us).
+template <class Args>
+__device__ __forceinline__ const Args& kernel_arguments() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int BYTES = sizeof(Args);
+    uint64_t ka = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    int t0, t1, t2, t3, t4, t5, t6, t7, t8;
+    asm volatile(CHX_TOUCH_ARGUMENTS
+                 : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8), "+s"(ka)
+                 : CHX_ARGUMENT_LINES
+                 : "memory");
+    typedef const Args __attribute__((address_space(4))) * ConstantArgs;
+    return *(const Args*)(ConstantArgs)ka;
+#else
+    return *(const Args*)nullptr;  // the host pass only parses the kernel
+#endif
+}
+#undef CHX_TOUCH_ARGUMENTS
+#undef CHX_ARGUMENT_LINES
 
 // Copies Q0 .. Q0+N-1 of a wave's group of up to four asynchronous 16-byte-per-lane copies through a buffer
 // resource into LDS, as one statement so that nothing can touch M0 between them.  Copy q reads byte offset

@@ -56,16 +56,25 @@ __device__ __forceinline__ v4i load_part(const char* src, int n) {
     return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
+struct ConvPointArgs {
+    ConvMfmaArgs conv;
+    uint32_t x_flip;
+    int32_t rne, chunks, chunk_tiles, slots;  // slots: work-groups per chunk
+    uint32_t chunks_mul, chunks_shift;        // magic_divisor(chunks)
+};
+
 // kPath: QuantProduct::path (2 also for a pair of which one is 1; both are 3 or none)
 template <int KS, int kPath, bool kFloatBias, bool kRes>
-__global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs a, uint32_t x_flip_s, int rne, int chunks, int chunk_tiles) {
+__global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvPointArgs) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    warm_kernel_arguments<sizeof(ConvMfmaArgs)>();
+    const ConvPointArgs& args = kernel_arguments<ConvPointArgs>();
+    const ConvMfmaArgs& a = args.conv;
+    const int rne = args.rne, chunks = args.chunks, chunk_tiles = args.chunk_tiles, slots = args.slots;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, group = lane >> 4;
     // the chunks of channels over one run of pixels are neighbours on one XCD: its L2 hands them the pixels
-    const int turn = (int)(blockIdx.x >> 3), chunk = turn % chunks, slot = (turn / chunks) * 8 + (int)(blockIdx.x & 7);
-    const int slots = (int)gridDim.x / chunks;
+    const int turn = (int)(blockIdx.x >> 3), round = (int)fast_div((uint32_t)turn, args.chunks_mul, args.chunks_shift);
+    const int chunk = turn - round * chunks, slot = round * 8 + (int)(blockIdx.x & 7);
     const int tile0 = chunk * chunk_tiles, tiles = min(chunk_tiles, (a.OC + 15) / 16 - tile0);
 
     // ---- this chunk's weights and constants ----
@@ -73,9 +82,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
     int32_t* s_add = reinterpret_cast<int32_t*>(lds + chunk_tiles * KS * 1024);
     float* s_scale = reinterpret_cast<float*>(s_add + chunk_tiles * 16);
     float* s_fbias = s_scale + chunk_tiles * 16;
+    const int bk_shift = a.bk == 128 ? 7 : 6;
     for (int i = tid; i < tiles * KS * 64; i += 64 * kWaves) {
         const int l = i & 63, ts = i >> 6, oc = (tile0 + ts / KS) * 16 + (l & 15), k = (ts % KS) * 64 + (l >> 4) * 16;
-        s_w[i] = *reinterpret_cast<const v4i*>(a.wp + (int64_t)(oc >> 6) * 64 * a.KP + (k / a.bk) * 64 * a.bk + (oc & 63) * a.bk + k % a.bk);
+        s_w[i] = *reinterpret_cast<const v4i*>(a.wp + (int64_t)(oc >> 6) * 64 * a.KP + ((k >> bk_shift) * 64 << bk_shift) + ((oc & 63) << bk_shift) + (k & (a.bk - 1)));
     }
     for (int i = tid; i < tiles * 16; i += 64 * kWaves) {
         const int ch = min(tile0 * 16 + i, a.OC - 1);
@@ -105,7 +115,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_point_kernel(ConvMfmaArgs
     };
     int block = slot * kWaves + wave;
     load(block);
-    const int flip = (int)in_vector_register(x_flip_s);
+    const int flip = (int)in_vector_register(args.x_flip);
     for (; block < blocks; block += step) {
         v4i x[2][KS];
 #pragma unroll
@@ -225,7 +235,15 @@ int launch(const ConvMfmaArgs& a, int max_wgs_per_cu, uint32_t flip, bool rne, h
     int64_t slots = 256 * per_cu / chunks;
     if (slots > wanted) slots = wanted;
     slots = (slots + 7) / 8 * 8;
-    conv_point_kernel<KS, kPath, kFloatBias, kRes><<<(int)(slots * chunks), 64 * kWaves, bytes, s>>>(a, flip, rne ? 1 : 0, chunks, chunk_tiles);
+    ConvPointArgs args;
+    args.conv = a;
+    args.x_flip = flip;
+    args.rne = rne ? 1 : 0;
+    args.chunks = chunks;
+    args.chunk_tiles = chunk_tiles;
+    args.slots = (int)slots;
+    magic_divisor((uint32_t)chunks, &args.chunks_mul, &args.chunks_shift);
+    conv_point_kernel<KS, kPath, kFloatBias, kRes><<<(int)(slots * chunks), 64 * kWaves, bytes, s>>>(args);
     return launch_check("conv_point_kernel");
 }
 

@@ -32,22 +32,30 @@ __device__ __forceinline__ uint32_t affine_residual4(uint32_t c, uint32_t r, con
     return floor_sat_u8x4(t[0], t[1], t[2], t[3]);
 }
 
+struct ConvSplitArgs {
+    ConvMfmaArgs conv;
+    uint32_t x_flip;
+    int32_t rne, tiles_per_xcd;
+    uint32_t tiles_px_mul, tiles_px_shift, c64_mul, c64_shift, kw_mul, kw_shift;  // magic_divisor(tiles_px), (C64), (KW): a division costs some 150 cycles
+};
+
 // (two wavefronts per SIMD promised, so that the sums stay out of the accumulation registers: see conv_stem_kernel)
-template <int R, int PN, int W, bool kPad, int kDepth>
-__global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, uint32_t x_flip, int rne, int tiles_per_xcd) {
+template <int R, int PN, int W, bool kTaps, int kDepth>
+__global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
     constexpr int kGroups = 64 / R, kStep = 16 * kGroups;  // K bytes per MFMA: 32 or 64
     constexpr int kQuads = R * R / 256;                    // groups of four result registers: 4 or 1
     constexpr int kUnits = PN * kQuads;
     using acc_t = typename std::conditional<R == 32, v16i, v4i>::type;
     __shared__ __attribute__((aligned(16))) v4i part[W > 1 ? W : 1][W > 1 ? kUnits : 1][64];
 
-    warm_kernel_arguments<sizeof(ConvMfmaArgs)>();
-    const int idx = (int)(blockIdx.x >> 3), tile = (int)(blockIdx.x & 7) * tiles_per_xcd + idx;
-    if (idx >= tiles_per_xcd || tile >= a.tiles_oc * a.tiles_px) return;
+    const ConvSplitArgs args = kernel_arguments<ConvSplitArgs>();
+    const ConvMfmaArgs& a = args.conv;
+    const int idx = (int)(blockIdx.x >> 3), tile = (int)(blockIdx.x & 7) * args.tiles_per_xcd + idx;
+    if (idx >= args.tiles_per_xcd || tile >= a.tiles_oc * a.tiles_px) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane % R, group = lane / R;
     // an XCD's run of tiles: all pixels of a few channel tiles, so that their weights are fetched into one L2
-    const int oc_tile = tile / a.tiles_px, px_tile = tile - oc_tile * a.tiles_px;
+    const int oc_tile = (int)fast_div((uint32_t)tile, args.tiles_px_mul, args.tiles_px_shift), px_tile = tile - oc_tile * a.tiles_px;
     const int oc0 = oc_tile * R, oc = oc0 + col;
 
     // Every kernel of a network starts with cold caches (what the previous one wrote has to become visible to all XCDs),
@@ -82,7 +90,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
             const uint32_t n = fast_div(r, a.oh_mul, a.oh_shift), oh = r - n * (uint32_t)a.OH;
             const int ih0 = (int)oh * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
             x_off[j] = (int32_t)n * (int32_t)a.x_n_stride + ih0 * (int32_t)a.x_h_stride + iw0 * (int32_t)a.x_w_stride;
-            if (kPad) {
+            if (kTaps) {
                 const int c_lo = min(max(-iw0, 0), a.KW), c_hi = min(max(a.W - iw0, 0), a.KW);
                 const int r_lo = min(max(-ih0, 0), a.KH), r_hi = min(max(a.H - ih0, 0), a.KH);
                 // the column bits repeated in every filter row, the rows outside the image cut off
@@ -96,24 +104,35 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
     const int fill = (int)((uint32_t)(a.x_zp & 0xff) * 0x01010101u);
 
     // the step whose pixels are loaded next: its place in its filter tap, the tap, and the offset into x
-    int k_in, tap, kw, at = lo;
-    uint32_t x_at;
-    {
+    int k_in = 0, tap = 0, kw = 0, at = lo;
+    uint32_t x_at = 0;
+    if constexpr (kTaps) {
         const int k = lo * kStep;
-        tap = k / a.C64;
+        tap = (int)fast_div((uint32_t)k, args.c64_mul, args.c64_shift);
         k_in = k - tap * a.C64;
-        kw = tap % a.KW;
-        x_at = (uint32_t)((tap / a.KW) * (int)a.x_h_stride + kw * (int)a.x_w_stride + k_in);
+        const int kh = (int)fast_div((uint32_t)tap, args.kw_mul, args.kw_shift);
+        kw = tap - kh * a.KW;
+        x_at = (uint32_t)(kh * (int)a.x_h_stride + kw * (int)a.x_w_stride + k_in);
     }
     auto load_x = [&](Step& s) {
+        if constexpr (!kTaps) {  // (channels past C16: as below)
+            const uint32_t k = (uint32_t)(at * kStep);
+            at = min(at + 1, last);
+#pragma unroll
+            for (int j = 0; j < PN; ++j) {
+                const uint32_t off = (int)k + group * 16 < a.C16 ? (uint32_t)x_off[j] + k : 0u;
+                s.x[j] = *reinterpret_cast<const v4i*>(a.x + off);
+            }
+            return;
+        }
         // channels past C16 have zero weights, and a tap outside the image becomes the zero point: both read anything inside x
         const bool channels = k_in + group * 16 < a.C16;
 #pragma unroll
         for (int j = 0; j < PN; ++j) {
-            const bool inside = channels && (!kPad || ((taps[j] >> tap) & 1));
+            const bool inside = channels && (!kTaps || ((taps[j] >> tap) & 1));
             const uint32_t off = inside ? (uint32_t)x_off[j] + x_at : 0u;
             s.x[j] = *reinterpret_cast<const v4i*>(a.x + off);
-            if (kPad) {
+            if (kTaps) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s.x[j][e] = inside ? s.x[j][e] : fill;
             }
@@ -161,6 +180,21 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
                 for (int e = 0; e < 4; ++e)
                     if (f.c0 + e < OC) f.r |= (uint32_t)(uint8_t)src[e] << (8 * e);
         }
+        if (a.w_scale_len > 1 && a.OC % 4 == 0) {
+            typedef int v4i_d __attribute__((ext_vector_type(4), aligned(4)));
+            typedef float v4f_d __attribute__((ext_vector_type(4), aligned(4)));
+            typedef const v4f_d __attribute__((address_space(1))) * Global;  // (which the compiler does not see of a choice of two)
+            const int ch = min(f.c0, a.OC - 4);
+            const v4i_d add = *reinterpret_cast<const v4i_d*>(a.wsum + ch);
+            const v4f_d scale = *reinterpret_cast<const v4f_d*>(a.w_scale + ch), bias = *(Global)(uint64_t)((a.bias ? a.bias : a.wsum) + ch);  // (no branch around a load)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                f.add[e] = add[e];
+                f.scale[e] = scale[e];
+                f.fbias[e] = bias[e];
+            }
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int ch = min(f.c0 + e, a.OC - 1);
@@ -184,7 +218,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
         for (int j = 0; j < PN; ++j) {
             v4i fx = s.x[j];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fx[e] ^= (int)x_flip;
+            for (int e = 0; e < 4; ++e) fx[e] ^= (int)args.x_flip;
             if constexpr (R == 32) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(s.w, fx, acc[j], 0, 0, 0);
             else acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(s.w, fx, acc[j], 0, 0, 0);
         }
@@ -205,14 +239,12 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
     }
 
     // ---- the sums, requantized ----
-    if (a.oc_split > 0 && oc0 >= a.oc_split) {
-        a.y = a.y2 - a.oc_split;
-        a.y_px_stride = a.y2_px_stride;
-        a.y_flip = a.y2_flip;
-        a.rq.q = a.q2;
-        a.inv_y_scale = a.inv_y_scale2;
-        a.lo_folded = a.lo_folded2;
-    }
+    const bool second = a.oc_split > 0 && oc0 >= a.oc_split;
+    char* const y = second ? a.y2 - a.oc_split : a.y;
+    const int64_t y_px_stride = second ? a.y2_px_stride : a.y_px_stride;
+    const uint32_t y_flip = second ? a.y2_flip : a.y_flip;
+    const QuantParams q_out = second ? a.q2 : a.rq.q;
+    const float inv_y_scale = second ? a.inv_y_scale2 : a.inv_y_scale, lo_folded = second ? a.lo_folded2 : a.lo_folded;
     auto finish = [&](const Finish& f, v4i sum) {
         if (f.m >= a.M || f.c0 >= OC) return;
         int32_t code[4];
@@ -223,15 +255,15 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
             if (a.rq.bias_mode == kBiasOnnxInt32) v += bias;
             float x = (float)v * (a.rq.x_scale * f.scale[e]);
             if (a.rq.bias_mode == kBiasReferenceFloat) x = x + (float)bias;
-            code[e] = rne ? quantize_value_folded<true>(x, a.rq.q, a.inv_y_scale, a.lo_folded) : quantize_value_folded<false>(x, a.rq.q, a.inv_y_scale, a.lo_folded);
+            code[e] = args.rne ? quantize_value_folded<true>(x, q_out, inv_y_scale, lo_folded) : quantize_value_folded<false>(x, q_out, inv_y_scale, lo_folded);
         }
         uint32_t word = pack4(code[0], code[1], code[2], code[3]);
         if (a.res.r) {
             if (a.res.affine) word = affine_residual4(word, f.r, a.res);
             else word = (uint32_t)add_residual16_any(v4i{(int)word, 0, 0, 0}, v4i{(int)f.r, 0, 0, 0}, a.res)[0];
         }
-        word ^= a.y_flip;
-        char* dst = a.y + f.m * a.y_px_stride + f.c0;
+        word ^= y_flip;
+        char* dst = y + f.m * y_px_stride + f.c0;
         if (f.c0 + 4 <= OC) *reinterpret_cast<u32_u*>(dst) = word;
         else
             for (int e = 0; e < 4; ++e)
@@ -266,14 +298,22 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvMfmaArgs a, u
 // the largest tile, five with sixteen wavefronts): each round trip less is most of a microsecond.  ResNet-50 on one image
 // 303 -> 294 us.
 template <int R, int PN, int W>
-int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, bool pad, hipStream_t s) {
+int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, bool taps, hipStream_t s) {
     constexpr int kDeep = R * PN == 64 ? 6 : W == 16 && PN == 2 ? 5 : 8, kStep = 1024 / R;
     const int64_t tiles = (int64_t)a.tiles_oc * a.tiles_px;
     const int per_xcd = (int)((tiles + 7) / 8);
     const bool deep = (a.KP / kStep + W - 1) / W > 4;
-#define CHX_SPLIT(PAD, DEPTH) conv_split_kernel<R, PN, W, PAD, DEPTH><<<8 * per_xcd, 64 * W, 0, s>>>(a, flip, rne ? 1 : 0, per_xcd)
-    if (pad && deep) CHX_SPLIT(true, kDeep);
-    else if (pad) CHX_SPLIT(true, 4);
+    ConvSplitArgs args;
+    args.conv = a;
+    args.x_flip = flip;
+    args.rne = rne ? 1 : 0;
+    args.tiles_per_xcd = per_xcd;
+    magic_divisor((uint32_t)a.tiles_px, &args.tiles_px_mul, &args.tiles_px_shift);
+    magic_divisor((uint32_t)a.C64, &args.c64_mul, &args.c64_shift);
+    magic_divisor((uint32_t)a.KW, &args.kw_mul, &args.kw_shift);
+#define CHX_SPLIT(TAPS, DEPTH) conv_split_kernel<R, PN, W, TAPS, DEPTH><<<8 * per_xcd, 64 * W, 0, s>>>(args)
+    if (taps && deep) CHX_SPLIT(true, kDeep);
+    else if (taps) CHX_SPLIT(true, 4);
     else if (deep) CHX_SPLIT(false, kDeep);
     else CHX_SPLIT(false, 4);
 #undef CHX_SPLIT
@@ -289,10 +329,11 @@ bool conv_split_has(int tile_oc, int tile_px, int waves) {
 }
 
 int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s) {
-    const bool pad = a.ph != 0 || a.pw != 0 || (int64_t)(a.OH - 1) * a.sh + a.KH > a.H || (int64_t)(a.OW - 1) * a.sw + a.KW > a.W;
+    // a filter of one tap, inside the image for every pixel, or any filter
+    const bool taps = a.KH * a.KW > 1 || a.ph != 0 || a.pw != 0 || (int64_t)(a.OH - 1) * a.sh + a.KH > a.H || (int64_t)(a.OW - 1) * a.sw + a.KW > a.W;
     const uint32_t flip = x_unsigned ? 0x80808080u : 0u;
 #define CHX_SPLIT(R, PN, W) \
-    if (tile_oc == R && tile_px == R * PN && waves == W) return launch<R, PN, W>(a, flip, rne, pad, s);
+    if (tile_oc == R && tile_px == R * PN && waves == W) return launch<R, PN, W>(a, flip, rne, taps, s);
     CHX_SPLIT(16, 1, 8)
     CHX_SPLIT(16, 1, 16)
     CHX_SPLIT(16, 2, 4)

@@ -34,6 +34,7 @@ struct DepthwiseArgs {
     // that each XCD works through a contiguous run of blocks and the input lines that neighbouring blocks share (the
     // filter's three columns, the halo rows of a strip) are found in that XCD's own L2.  Filled by the launcher.
     uint32_t grid_x, grid_xy, blocks, xcd_chunk;
+    uint32_t grid_x_mul, grid_x_shift, grid_xy_mul, grid_xy_shift, cgs_mul, cgs_shift;  // magic_divisor(grid_x), (grid_xy), (C / 4)
     int64_t total;          // filled by the launcher
 };
 

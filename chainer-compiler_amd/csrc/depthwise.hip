@@ -20,6 +20,8 @@
 #include <type_traits>
 
 #include "contract.h"
+#include "conv_mfma.h"
+#include "conv_device.h"
 #include "depthwise.h"
 
 namespace chx {
@@ -64,19 +66,20 @@ __global__ __launch_bounds__(256) void pack_depthwise_kernel(
 constexpr int rows_per_thread(int step, int strip) { return step == 1 ? (strip == 1 ? 14 : strip == 2 ? 7 : 8) : step == 2 ? 4 : 1; }
 constexpr int kDwThreads = 64;  // small groups: (output columns x channel groups) of a row is rarely a multiple of 256
 template <bool kRne, bool kFloatBias, int kStep, int kPath, int kStrip>
-__global__ __launch_bounds__(kDwThreads) void depthwise3x3_kernel(DepthwiseArgs a) {
+__global__ __launch_bounds__(kDwThreads) void depthwise3x3_kernel(DepthwiseArgs) {
+    const DepthwiseArgs a = kernel_arguments<DepthwiseArgs>();
     constexpr int kRows = rows_per_thread(kStep, kStrip);
     constexpr int kInRows = kStep == 1 ? kRows + 2 : kStep == 2 ? 2 * kRows + 1 : 3;
     // blocks: x over (output column, channel group) of one strip of output rows, then the strips, then the images;
     // which block this work-group takes: see DepthwiseArgs
     const uint32_t block = (blockIdx.x & 7u) * a.xcd_chunk + (blockIdx.x >> 3);
     if (block >= a.blocks) return;
-    const uint32_t bz = block / a.grid_xy, bxy = block - bz * a.grid_xy;
-    const uint32_t by = bxy / a.grid_x, bx = bxy - by * a.grid_x;
+    const uint32_t bz = fast_div(block, a.grid_xy_mul, a.grid_xy_shift), bxy = block - bz * a.grid_xy;
+    const uint32_t by = fast_div(bxy, a.grid_x_mul, a.grid_x_shift), bx = bxy - by * a.grid_x;
     const uint32_t idx = bx * kDwThreads + threadIdx.x;
     const uint32_t cgs = (uint32_t)a.C >> 2;
     if (idx >= (uint32_t)a.OW * cgs) return;
-    const int ow = (int)(idx / cgs);
+    const int ow = (int)fast_div(idx, a.cgs_mul, a.cgs_shift);
     const int cg = (int)(idx - (uint32_t)ow * cgs);
     const int ohb = (int)by;
     const int n = (int)bz;
@@ -232,6 +235,9 @@ int launch_depthwise3x3(DepthwiseArgs a, bool rne, hipStream_t s) {
     a.grid_xy = (uint32_t)(grid_x * a.oh_blocks);
     a.blocks = (uint32_t)all_blocks;
     a.xcd_chunk = (uint32_t)((all_blocks + 7) / 8);
+    magic_divisor(a.grid_x, &a.grid_x_mul, &a.grid_x_shift);
+    magic_divisor(a.grid_xy, &a.grid_xy_mul, &a.grid_xy_shift);
+    magic_divisor((uint32_t)a.C / 4, &a.cgs_mul, &a.cgs_shift);
     const dim3 blocks(a.xcd_chunk * 8u);
     const bool fbias = a.bias != nullptr && a.float_bias != 0;
     const int path = rne ? 0 : a.qp.path;

@@ -8,6 +8,7 @@
 #include "contract.h"
 #include "depthwise.h"
 #include "conv_mfma.h"
+#include "conv_device.h"
 #include "gemm_i8_device.h"
 
 namespace chx {
@@ -27,16 +28,24 @@ __device__ __forceinline__ uint64_t narrow_window(const char* row, int at, int W
     return v;
 }
 
+struct DepthwisePlanarArgs {
+    DepthwiseArgs conv;
+    int32_t rne, G, RB, channels;
+    uint32_t g_mul, g_shift, rb_mul, rb_shift, c_mul, c_shift;
+};
+
 // S: stride.  kPath: QuantProduct::path.
 template <int S, int kPath, bool kFloatBias>
-__global__ __launch_bounds__(256) void depthwise_planar_kernel(DepthwiseArgs a, int rne, int G, int RB, int channels, uint32_t g_mul, uint32_t g_shift, uint32_t rb_mul, uint32_t rb_shift,
-                                                               uint32_t c_mul, uint32_t c_shift) {
+__global__ __launch_bounds__(256) void depthwise_planar_kernel(DepthwisePlanarArgs) {
+    const DepthwisePlanarArgs args = kernel_arguments<DepthwisePlanarArgs>();
+    const DepthwiseArgs& a = args.conv;
+    const int rne = args.rne;
     // (image, channel, run of rows, group of four columns), the last one fastest
     const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t t = (__umulhi(idx, g_mul) + idx) >> g_shift, gc = idx - t * (uint32_t)G;
-    const uint32_t nc = (__umulhi(t, rb_mul) + t) >> rb_shift, rb = t - nc * (uint32_t)RB;
-    if (nc >= (uint32_t)channels) return;
-    const uint32_t n = (__umulhi(nc, c_mul) + nc) >> c_shift, c = nc - n * (uint32_t)a.C;
+    const uint32_t t = fast_div(idx, args.g_mul, args.g_shift), gc = idx - t * (uint32_t)args.G;
+    const uint32_t nc = fast_div(t, args.rb_mul, args.rb_shift), rb = t - nc * (uint32_t)args.RB;
+    if (nc >= (uint32_t)args.channels) return;
+    const uint32_t n = fast_div(nc, args.c_mul, args.c_shift), c = nc - n * (uint32_t)a.C;
     const int oh0 = (int)rb * kRows, ow0 = (int)gc * 4, ih0 = oh0 * S - a.ph, iw0 = ow0 * S - a.pw;
     const char* plane = a.x + (int64_t)n * a.x_n_stride + (int64_t)c * a.x_c_stride;
     const uint64_t flip = a.x_signed ? 0 : 0x8080808080808080ull, zp = (uint64_t)((uint32_t)((a.x_zp_u ^ 0x80) & 0xff) * 0x01010101u) * 0x100000001ull;
@@ -97,14 +106,19 @@ int launch_depthwise_planar(const DepthwiseArgs& a, bool rne, hipStream_t s) {
     const int64_t channels = (int64_t)a.N * a.C, total = channels * RB * G;
     if (total == 0) return CHX_HIP_OK;
     if (total >= (int64_t(1) << 31) - 256) return CHX_HIP_EUNSUPPORTED;
-    uint32_t gm, gs, rm, rs, cm, cs;
-    magic_divisor((uint32_t)G, &gm, &gs);
-    magic_divisor((uint32_t)RB, &rm, &rs);
-    magic_divisor((uint32_t)a.C, &cm, &cs);
+    DepthwisePlanarArgs args;
+    args.conv = a;
+    args.rne = rne ? 1 : 0;
+    args.G = G;
+    args.RB = RB;
+    args.channels = (int32_t)channels;
+    magic_divisor((uint32_t)G, &args.g_mul, &args.g_shift);
+    magic_divisor((uint32_t)RB, &args.rb_mul, &args.rb_shift);
+    magic_divisor((uint32_t)a.C, &args.c_mul, &args.c_shift);
     const bool fb = a.bias != nullptr && a.float_bias != 0;
     const int path = rne ? 0 : a.qp.path;
     const unsigned blocks = (unsigned)((total + 255) / 256);
-#define CHX_DWP(S, P, F) depthwise_planar_kernel<S, P, F><<<blocks, 256, 0, s>>>(a, rne ? 1 : 0, G, RB, (int)channels, gm, gs, rm, rs, cm, cs)
+#define CHX_DWP(S, P, F) depthwise_planar_kernel<S, P, F><<<blocks, 256, 0, s>>>(args)
 #define CHX_DWP_F(S, P)                   \
     do {                                  \
         if (fb) CHX_DWP(S, P, true);      \

@@ -72,10 +72,10 @@ __device__ __forceinline__ int32_t quantize_any(float v, const QuantParams& q, f
     return quantize_value_folded<false>(__builtin_fmaxf(v, -largest), q, inv_scale, q.lo);
 }
 
-__global__ __launch_bounds__(64 * kWaves) void matmul_chain_kernel(ChainArgs g) {
+__global__ __launch_bounds__(64 * kWaves) void matmul_chain_kernel(ChainArgs) {
     __shared__ __attribute__((aligned(16))) char act[kRows * kActRow];    // codes as signed bytes, zeros up to a multiple of 64
     __shared__ __attribute__((aligned(16))) int32_t sum[kRows * kSumRow];  // 0 between layers
-    warm_kernel_arguments<sizeof(ChainArgs)>();
+    const ChainArgs& g = kernel_arguments<ChainArgs>();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, group = lane >> 4;
     const int m0 = (int)blockIdx.x * kRows;

@@ -10,6 +10,8 @@
 #include <cstring>
 
 #include "chx_internal.h"
+#include "conv_mfma.h"
+#include "conv_device.h"
 #include "quant_math.h"
 
 namespace chx {
@@ -25,6 +27,8 @@ struct PoolArgs {
     int32_t N, C, H, W, OH, OW, kh, kw, sh, sw, ph, pw;
     int32_t is_signed;
     int64_t total;
+    uint32_t xcd_chunk;                                                  // see max_pool_cl16_kernel
+    uint32_t cg_mul, cg_shift, ow_mul, ow_shift, oh_mul, oh_shift;  // magic_divisor(channel groups), (OW), (OH), where a kernel says so
 };
 
 __device__ __forceinline__ uint32_t max4_u8(uint32_t a, uint32_t b) {
@@ -56,16 +60,14 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
 // (b % 8) * xcd_chunk + b / 8, so that an XCD works through a contiguous run of output rows and finds the input rows
 // that neighbouring output rows share in its own L2 (the launch is xcd_chunk * 8 work-groups).
 template <bool kSigned>
-__global__ __launch_bounds__(kThreads) void max_pool_cl16_kernel(PoolArgs a, uint32_t xcd_chunk) {
-    const int64_t idx = (int64_t)((blockIdx.x & 7u) * xcd_chunk + (blockIdx.x >> 3)) * kThreads + threadIdx.x;
-    if (idx >= a.total) return;
-    const int cgroups = a.C / 16;
-    const int cg = (int)(idx % cgroups);
-    int64_t r = idx / cgroups;
-    const int ow = (int)(r % a.OW);
-    r /= a.OW;
-    const int oh = (int)(r % a.OH);
-    const int n = (int)(r / a.OH);
+__global__ __launch_bounds__(kThreads) void max_pool_cl16_kernel(PoolArgs) {
+    const PoolArgs a = kernel_arguments<PoolArgs>();
+    // (fewer than 2^31 threads: four divisions of 64 bits were half of the kernel's instructions)
+    const uint32_t idx = ((blockIdx.x & 7u) * a.xcd_chunk + (blockIdx.x >> 3)) * kThreads + threadIdx.x;
+    if (idx >= (uint32_t)a.total) return;
+    const uint32_t q = fast_div(idx, a.cg_mul, a.cg_shift), r = fast_div(q, a.ow_mul, a.ow_shift);
+    const int cg = (int)(idx - q * (uint32_t)(a.C / 16)), ow = (int)(q - r * (uint32_t)a.OW);
+    const int n = (int)fast_div(r, a.oh_mul, a.oh_shift), oh = (int)(r - (uint32_t)n * (uint32_t)a.OH);
     const uint32_t flip = kSigned ? 0x80808080u : 0u;
     const int ih0 = oh * a.sh - a.ph, iw0 = ow * a.sw - a.pw;
     const bool touches = ih0 < a.H && ih0 + a.kh > 0 && iw0 < a.W && iw0 + a.kw > 0;
@@ -239,13 +241,14 @@ __global__ __launch_bounds__(kThreads) void average_pool_cl4_kernel(AvgArgs a) {
 // result is the bytes of the kernels above.
 constexpr int kGlobalPoolTaps = 64;
 template <bool kRne>
-__global__ __launch_bounds__(kThreads) void global_average_pool_cl4_kernel(AvgArgs a) {
+__global__ __launch_bounds__(64) void global_average_pool_cl4_kernel(AvgArgs) {
+    const AvgArgs a = kernel_arguments<AvgArgs>();
     const PoolArgs& p = a.p;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int C4 = p.C >> 2;
-    if (idx >= (p.total >> 2)) return;
-    const int c = (int)(idx % C4) * 4;
-    const int64_t n = idx / C4;
+    const uint32_t idx = blockIdx.x * 64u + threadIdx.x;  // (fewer than 2^31 threads)
+    if (idx >= (uint32_t)(p.total >> 2)) return;
+    const uint32_t image = fast_div(idx, p.cg_mul, p.cg_shift);
+    const int c = (int)(idx - image * (uint32_t)(p.C >> 2)) * 4;
+    const int64_t n = image;
     const uint32_t flip = p.is_signed ? 0x80808080u : 0u;
     const float zpf = a.x_zpf + (p.is_signed ? 128.f : 0.f);
     const int taps = p.H * p.W;
@@ -362,14 +365,15 @@ extern "C" int chx_hip_max_pool_q8(
     hipStream_t s = as_stream(stream);
     int64_t px, py;
     const bool cl16 = a.C % 16 == 0 && is_channels_last(*x, &px) && is_channels_last(*y, &py) && aligned(x->data, 16) &&
-                      aligned(y->data, 16) && px % 16 == 0 && py % 16 == 0;
+                      aligned(y->data, 16) && px % 16 == 0 && py % 16 == 0 && a.total / 16 < (int64_t(1) << 31) - 16 * kThreads;
     if (cl16) {
-        a.total = (int64_t)a.N * a.OH * a.OW * (a.C / 16);
-        const int64_t blocks = (a.total + kThreads - 1) / kThreads;
-        CHX_REQUIRE(blocks < (int64_t(1) << 31) - 8, "MaxPool: 2^31 work-groups or more");
-        const uint32_t xcd_chunk = (uint32_t)((blocks + 7) / 8);
-        if (a.is_signed) max_pool_cl16_kernel<true><<<xcd_chunk * 8, kThreads, 0, s>>>(a, xcd_chunk);
-        else max_pool_cl16_kernel<false><<<xcd_chunk * 8, kThreads, 0, s>>>(a, xcd_chunk);
+        a.total /= 16;
+        a.xcd_chunk = (uint32_t)(((a.total + kThreads - 1) / kThreads + 7) / 8);
+        magic_divisor((uint32_t)(a.C / 16), &a.cg_mul, &a.cg_shift);
+        magic_divisor((uint32_t)a.OW, &a.ow_mul, &a.ow_shift);
+        magic_divisor((uint32_t)a.OH, &a.oh_mul, &a.oh_shift);
+        if (a.is_signed) max_pool_cl16_kernel<true><<<a.xcd_chunk * 8, kThreads, 0, s>>>(a);
+        else max_pool_cl16_kernel<false><<<a.xcd_chunk * 8, kThreads, 0, s>>>(a);
         return launch_check("max_pool_cl16_kernel");
     }
     max_pool_generic_kernel<<<(unsigned)((a.total + kThreads - 1) / kThreads), kThreads, 0, s>>>(a);
@@ -402,8 +406,9 @@ extern "C" int chx_hip_average_pool_q8(
         const PoolArgs& p = a.p;
         // the window is the whole image, stored as one dense run of pixels
         const bool whole_image = p.OH == 1 && p.OW == 1 && p.ph == 0 && p.pw == 0 && p.kh == p.H && p.kw == p.W &&
-                                 (p.H == 1 || p.xs[2] == p.W * p.xs[3]) && p.H * p.W <= kGlobalPoolTaps;
+                                 (p.H == 1 || p.xs[2] == p.W * p.xs[3]) && p.H * p.W <= kGlobalPoolTaps && p.total / 4 < (int64_t(1) << 31) - 64;
         if (whole_image) {
+            magic_divisor((uint32_t)(p.C / 4), &a.p.cg_mul, &a.p.cg_shift);
             if (rne) global_average_pool_cl4_kernel<true><<<blocks4, 64, 0, s>>>(a);
             else global_average_pool_cl4_kernel<false><<<blocks4, 64, 0, s>>>(a);
             return launch_check("global_average_pool_cl4_kernel");

@@ -76,6 +76,23 @@ def pitched(shape, dtype):
 
 
 @pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("C,OC,k,st,scales", [(48, 64, 3, 1, 64), (80, 70, 3, 2, 70), (16, 4, 1, 1, 4), (144, 68, 1, 2, 1)])
+def test_taps_without_padding(g, oracle, tile, C, OC, k, st, scales):
+    """Filters of several taps that no pixel has outside the image, one tap; constants of four channels at once and one by one."""
+    rng = np.random.default_rng(C + OC)
+    x, w = codes(rng, (2, C, 7, 6), np.uint8), codes(rng, (OC, C, k, k), np.int8)
+    ws, bias = rng.uniform(0.002, 0.02, size=scales).astype(np.float32), rng.integers(-3000, 3000, size=OC).astype(np.int32)
+    ys = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C * k * k) / 40)
+    for b in (bias, None):
+        with forced(tile):
+            plan = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(scales, np.int8)), None if b is None else g.dev(b), strides=(st, st), pads=(0, 0))
+            got = plan.run(g.to_channels_last(g.dev(x)), 0.02, 77, ys, 5, zero_point_dtype=torch.uint8, flags=g.capi.BIAS_ONNX_INT32)
+        okw = {} if b is None else dict(bias=b, bias_mode=oracle.BIAS_ONNX_INT32)
+        want = oracle.qlinear_conv_int(x, 0.02, 77, w, np.broadcast_to(ws, (OC,)).copy(), np.zeros(OC, np.int8), ys, 5, np.uint8, strides=(st, st), pads=(0, 0), **okw)
+        np.testing.assert_array_equal(g.host(got), want)
+
+
+@pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("affine", ["1", "0"])
 @pytest.mark.parametrize("minus_128", [False, True])
 def test_residual_pair_and_storage(g, tile, affine, minus_128):
