@@ -9,12 +9,14 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "contract.h"
 #include "conv_mfma.h"
+#include "inverted_residual.h"
 #include "depthwise.h"
 
 namespace chx {
@@ -1012,6 +1014,86 @@ int run_depthwise(const ConvCall& c, const DepthwiseState& st, hipStream_t s) {
 }  // namespace
 }  // namespace chx
 
+namespace chx {
+namespace {
+
+// The residual sums fused behind a convolution so far: each one's parameters, and whether constants were found with which
+// its two-multiply-add form is exact (find_affine_residual); kept so that the search runs once per set of parameters, also
+// for a caller that alternates between a few of them.  Oldest dropped first.
+struct SearchedResidual {
+    ResidualAdd key, found;
+};
+constexpr size_t kMaxSearchedResiduals = 8;
+
+// r: channels-last, r_px bytes from pixel to pixel; out_scale within [2^-60, 2^60]
+int residual_of(const chx_hip_tensor& r, int64_t r_px, float y_scale, int32_t y_zero_point, int32_t y_dtype, float r_scale, int32_t r_zero_point,
+                float out_scale, int32_t out_zero_point, int32_t out_dtype, bool relu, bool wanted, std::vector<SearchedResidual>* searched, hipStream_t s,
+                ResidualAdd* out) {
+    ResidualAdd res;
+    memset(&res, 0, sizeof(res));
+    res.r = static_cast<const char*>(r.data);
+    res.r_px_stride = r_px;
+    res.r_vec_ok = aligned(r.data, 16) && r_px % 16 == 0 ? 1 : 0;
+    res.c_flip = y_dtype == CHX_HIP_INT8 ? 0x80808080u : 0u;
+    res.r_flip = r.dtype == CHX_HIP_INT8 ? 0x80808080u : 0u;
+    res.c_zpf = (float)(y_zero_point + (y_dtype == CHX_HIP_INT8 ? 128 : 0));
+    res.c_scale = y_scale;
+    res.r_zpf = (float)(r_zero_point + (r.dtype == CHX_HIP_INT8 ? 128 : 0));
+    res.r_scale = r_scale;
+    res.relu = relu ? 1 : 0;
+    res.out = make_quant_params(out_scale, out_zero_point, out_dtype == CHX_HIP_INT8);
+    res.inv_out_scale = 1.0f / out_scale;
+    res.big = 0x1p40f * out_scale;
+    // |DQ(y) + DQ(r)| <= 511 * (|y_scale| + |r_scale|): when that is far below `big`, limiting is the identity
+    const double reach = 511.0 * (fabs((double)y_scale) + fabs((double)r_scale));
+    res.guard = (reach == reach && reach < 0.25 * (double)res.big) ? 0 : 1;
+    // (r's zero point in the unsigned range: a uint8 r with zero point 0, or the same codes stored minus 128 as int8)
+    res.lean = out_dtype == CHX_HIP_UINT8 && res.r_zpf == 0.f && out_zero_point == 0 ? 1 : 0;
+    // The cheaper form of the sum, where the search over its constants has shown it exact for these parameters.  The
+    // search runs on the first call with new parameters (it synchronizes the stream and allocates, so not while the
+    // stream is being captured: such a call computes the sum operation by operation).  CHX_HIP_AFFINE_RESIDUAL=0
+    // keeps the operation-by-operation arithmetic everywhere.
+    {
+        ResidualAdd key;
+        memcpy(&key, &res, sizeof(key));  // byte copies: the comparison below is one of bytes, padding included
+        key.r = nullptr;
+        key.r_px_stride = 0;
+        key.r_vec_ok = 0;
+        const ResidualAdd* known = nullptr;
+        for (const SearchedResidual& e : *searched)
+            if (memcmp(&key, &e.key, sizeof(key)) == 0) known = &e.found;
+        if (wanted && known) {
+            res.affine = known->affine;
+            res.kc = known->kc;
+            res.kr = known->kr;
+            res.k0 = known->k0;
+            res.floor_pre = known->floor_pre;
+        } else if (wanted && !stream_is_capturing(s)) {
+            int32_t* counts = nullptr;
+            CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&counts), kAffineCandidates * sizeof(int32_t)));
+            ResidualAdd found;
+            memcpy(&found, &key, sizeof(found));
+            const int rc = find_affine_residual(&found, counts, s);
+            (void)hipFree(counts);
+            CHX_PROPAGATE(rc);
+            if (searched->size() == kMaxSearchedResiduals) searched->erase(searched->begin());
+            searched->emplace_back();
+            memcpy(&searched->back().key, &key, sizeof(key));
+            memcpy(&searched->back().found, &found, sizeof(found));
+            res.affine = found.affine;
+            res.kc = found.kc;
+            res.kr = found.kr;
+            res.k0 = found.k0;
+            res.floor_pre = found.floor_pre;
+        }
+    }
+    memcpy(out, &res, sizeof(res));
+    return CHX_HIP_OK;
+}
+
+}  // namespace
+}  // namespace chx
+
 struct chx_hip_qconv_plan {
     chx_hip_tensor w, w_scale, w_zero_point, bias;
     bool has_bias;
@@ -1022,14 +1104,7 @@ struct chx_hip_qconv_plan {
     chx::PackedWeights pw;
     chx::ScratchCache scratch;  // makes run() unsafe to call concurrently on one plan
     chx::TuneCache tune;
-    // the residual sums fused behind this convolution so far (run_add): each one's parameters, and whether constants
-    // were found with which its two-multiply-add form is exact (find_affine_residual); kept so that the search runs
-    // once per set of parameters, also for a caller that alternates between a few of them.  Oldest dropped first.
-    struct SearchedResidual {
-        chx::ResidualAdd key, found;
-    };
-    static constexpr size_t kMaxSearchedResiduals = 8;
-    std::vector<SearchedResidual> searched;
+    std::vector<chx::SearchedResidual> searched;  // residual sums fused behind this convolution (run_add)
     chx::LaunchOptions opt;  // read once, when the plan is created
     // recorded runs (HIP graphs) that hold addresses of this plan's packed weights and scratch memory
     int pins = 0;
@@ -1389,66 +1464,9 @@ extern "C" int chx_hip_qconv_plan_run_add(
     if (!y_is_pixel_major(*r, &r_px) || !y_is_pixel_major(*out, &o_px))
         CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+Add: r and out must be channels-last");
     ResidualAdd res;
-    memset(&res, 0, sizeof(res));
-    res.r = static_cast<const char*>(r->data);
-    res.r_px_stride = r_px;
-    res.r_vec_ok = aligned(r->data, 16) && r_px % 16 == 0 ? 1 : 0;
-    res.c_flip = y_dtype == CHX_HIP_INT8 ? 0x80808080u : 0u;
-    res.r_flip = r->dtype == CHX_HIP_INT8 ? 0x80808080u : 0u;
-    res.c_zpf = (float)(y_zero_point + (y_dtype == CHX_HIP_INT8 ? 128 : 0));
-    res.c_scale = y_scale;
-    res.r_zpf = (float)(r_zero_point + (r->dtype == CHX_HIP_INT8 ? 128 : 0));
-    res.r_scale = r_scale;
-    res.relu = relu ? 1 : 0;
-    res.out = make_quant_params(out_scale, out_zero_point, out_dtype == CHX_HIP_INT8);
-    res.inv_out_scale = 1.0f / out_scale;
-    res.big = 0x1p40f * out_scale;
-    // |DQ(y) + DQ(r)| <= 511 * (|y_scale| + |r_scale|): when that is far below `big`, limiting is the identity
-    const double reach = 511.0 * (fabs((double)y_scale) + fabs((double)r_scale));
-    res.guard = (reach == reach && reach < 0.25 * (double)res.big) ? 0 : 1;
-    // (r's zero point in the unsigned range: a uint8 r with zero point 0, or the same codes stored minus 128 as int8)
-    res.lean = out_dtype == CHX_HIP_UINT8 && res.r_zpf == 0.f && out_zero_point == 0 ? 1 : 0;
     hipStream_t s = as_stream(stream);
-    // The cheaper form of the sum, where the search over its constants has shown it exact for these parameters.  The
-    // search runs on the first call with new parameters (it synchronizes the stream and allocates, so not while the
-    // stream is being captured: such a call computes the sum operation by operation).  CHX_HIP_AFFINE_RESIDUAL=0
-    // keeps the operation-by-operation arithmetic everywhere.
-    {
-        chx_hip_qconv_plan* mp = const_cast<chx_hip_qconv_plan*>(plan);
-        ResidualAdd key;
-        memcpy(&key, &res, sizeof(key));  // byte copies: the comparison below is one of bytes, padding included
-        key.r = nullptr;
-        key.r_px_stride = 0;
-        key.r_vec_ok = 0;
-        const bool wanted = plan->opt.affine_residual;
-        const ResidualAdd* known = nullptr;
-        for (const chx_hip_qconv_plan::SearchedResidual& e : mp->searched)
-            if (memcmp(&key, &e.key, sizeof(key)) == 0) known = &e.found;
-        if (wanted && known) {
-            res.affine = known->affine;
-            res.kc = known->kc;
-            res.kr = known->kr;
-            res.k0 = known->k0;
-            res.floor_pre = known->floor_pre;
-        } else if (wanted && !stream_is_capturing(s)) {
-            int32_t* counts = nullptr;
-            CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&counts), kAffineCandidates * sizeof(int32_t)));
-            ResidualAdd found;
-            memcpy(&found, &key, sizeof(found));
-            const int rc = find_affine_residual(&found, counts, s);
-            (void)hipFree(counts);
-            CHX_PROPAGATE(rc);
-            if (mp->searched.size() == chx_hip_qconv_plan::kMaxSearchedResiduals) mp->searched.erase(mp->searched.begin());
-            mp->searched.emplace_back();
-            memcpy(&mp->searched.back().key, &key, sizeof(key));
-            memcpy(&mp->searched.back().found, &found, sizeof(found));
-            res.affine = found.affine;
-            res.kc = found.kc;
-            res.kr = found.kr;
-            res.k0 = found.k0;
-            res.floor_pre = found.floor_pre;
-        }
-    }
+    CHX_PROPAGATE(residual_of(*r, r_px, y_scale, y_zero_point, y_dtype, r_scale, r_zero_point, out_scale, out_zero_point, out_dtype, relu != 0,
+                              plan->opt.affine_residual, &const_cast<chx_hip_qconv_plan*>(plan)->searched, s, &res));
     ConvCall call = conv_call_from(q, x, &y, &plan->params, (flags & CHX_HIP_ROUND_ONNX_RNE) != 0, plan->opt);
     call.cache = const_cast<ScratchCache*>(&plan->scratch);
     call.tune = const_cast<TuneCache*>(&plan->tune);
@@ -1622,3 +1640,163 @@ extern "C" int chx_hip_qlinear_matmul(
     return launch_matmul_direct(m, rne, s);
 }
 
+// ---- inverted residual blocks ------------------------------------------------------------------
+
+struct chx_hip_inverted_residual {
+    int32_t channels = 0, expanded = 0, out_channels = 0, stride = 1;
+    bool has_bias = false, affine_residual = true;
+    int tiles = 0, tiles_padded = 0, steps = 0, tiles_oc = 0;
+    char* memory = nullptr;
+    size_t at_w3 = 0, at_t1 = 0, at_t2 = 0, at_t3 = 0;
+    std::mutex mutex;  // of `searched`
+    std::vector<chx::SearchedResidual> searched;
+};
+
+extern "C" void chx_hip_inverted_residual_destroy(chx_hip_inverted_residual* plan) {
+    if (!plan) return;
+    (void)hipFree(plan->memory);
+    delete plan;
+}
+
+extern "C" int chx_hip_inverted_residual_create(const chx_hip_conv_operands* stages, int32_t stride, void* stream, chx_hip_inverted_residual** out) {
+    CHX_REQUIRE(stages != nullptr && out != nullptr, "inverted residual: null argument");
+    *out = nullptr;
+    auto refuse = [](const char* why) {
+        set_error("inverted residual: %s", why);
+        return (int)CHX_HIP_EUNSUPPORTED;
+    };
+    hipStream_t s = as_stream(stream);
+    for (int i = 0; i < 3; ++i) {
+        const chx_hip_conv_operands& c = stages[i];
+        CHX_PROPAGATE(check_tensor(c.w, "inverted residual w"));
+        CHX_PROPAGATE(check_tensor(c.w_scale, "inverted residual w_scale"));
+        CHX_PROPAGATE(check_tensor(c.w_zero_point, "inverted residual w_zero_point"));
+        if (c.w->ndim != 4 || c.w->dtype != CHX_HIP_INT8 || c.w_scale->dtype != CHX_HIP_FLOAT32 || c.w_scale->ndim > 1 || c.w_zero_point->dtype != CHX_HIP_INT8) return refuse("the type of an operand");
+        const int64_t scales = numel(*c.w_scale);
+        if (scales != 1 && scales != c.w->shape[0]) return refuse("the number of scales");
+        if (c.bias) {
+            CHX_PROPAGATE(check_tensor(c.bias, "inverted residual bias"));
+            if (c.bias->dtype != CHX_HIP_INT32 || c.bias->ndim != 1 || c.bias->shape[0] != c.w->shape[0]) return refuse("a bias");
+        }
+        if ((c.bias != nullptr) != (stages[0].bias != nullptr)) return refuse("a bias on some of the convolutions");
+    }
+    const chx_hip_tensor &w1 = *stages[0].w, &w2 = *stages[1].w, &w3 = *stages[2].w;
+    const int64_t hid = w1.shape[0];
+    if (w1.shape[2] != 1 || w1.shape[3] != 1 || w3.shape[2] != 1 || w3.shape[3] != 1 || w2.shape[2] != 3 || w2.shape[3] != 3 || w2.shape[1] != 1 || w2.shape[0] != hid ||
+        w3.shape[1] != hid || (stride != 1 && stride != 2))
+        return refuse("not 1x1, depthwise 3x3, 1x1");
+    if (w1.shape[1] < 1 || w1.shape[1] > kInvertedMaxIn || hid < 1 || hid > 4096 || w3.shape[0] < 1 || w3.shape[0] > kInvertedMaxOut) return refuse("the number of channels");
+    for (int i = 0; i < 3; ++i) {
+        std::vector<uint8_t> zp;
+        CHX_PROPAGATE(read_back(*stages[i].w_zero_point, &zp, s));
+        if (!all_zero(zp)) return refuse("zero points of the weights");
+    }
+    std::unique_ptr<chx_hip_inverted_residual, void (*)(chx_hip_inverted_residual*)> p(new chx_hip_inverted_residual(), chx_hip_inverted_residual_destroy);
+    p->channels = (int32_t)w1.shape[1];
+    p->expanded = (int32_t)hid;
+    p->out_channels = (int32_t)w3.shape[0];
+    p->stride = stride;
+    p->has_bias = stages[0].bias != nullptr;
+    p->affine_residual = read_launch_options().affine_residual;
+    p->tiles = (int)((hid + 31) / 32);
+    p->tiles_padded = (p->tiles + 7) / 8 * 8;  // (the kernel takes up to eight at a time)
+    p->steps = p->channels <= 32 ? 1 : p->channels <= 96 ? 3 : 5;
+    p->tiles_oc = (p->out_channels + 31) / 32;
+    p->at_w3 = (size_t)p->tiles_padded * p->steps * 1024;
+    p->at_t1 = p->at_w3 + (size_t)p->tiles_padded * p->tiles_oc * 1024;
+    p->at_t2 = p->at_t1 + (size_t)p->tiles_padded * 32 * 16;
+    p->at_t3 = p->at_t2 + (size_t)p->tiles_padded * 32 * 32;
+    CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&p->memory), p->at_t3 + (size_t)p->tiles_oc * 32 * 16));
+    auto table = [&](size_t at) { return reinterpret_cast<int32_t*>(p->memory + at); };
+    CHX_PROPAGATE(pack_inverted_point(w1, *stages[0].w_scale, stages[0].bias, false, p->tiles_padded, p->steps, p->memory, table(p->at_t1), s));
+    CHX_PROPAGATE(pack_inverted_depthwise(w2, *stages[1].w_scale, stages[1].bias, p->tiles_padded, table(p->at_t2), s));
+    CHX_PROPAGATE(pack_inverted_point(w3, *stages[2].w_scale, stages[2].bias, true, p->tiles_oc, p->tiles_padded, p->memory + p->at_w3, table(p->at_t3), s));
+    // (later calls may come on any stream)
+    CHX_HIP_CALL(hipStreamSynchronize(s));
+    *out = p.release();
+    return CHX_HIP_OK;
+}
+
+extern "C" int chx_hip_inverted_residual_run(
+        chx_hip_inverted_residual* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points,
+        int32_t y_dtype, uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu,
+        chx_hip_tensor* out, void* stream) {
+    CHX_REQUIRE(plan != nullptr && y_scales != nullptr && y_zero_points != nullptr, "inverted residual: null argument");
+    CHX_PROPAGATE(check_tensor(x, "inverted residual x"));
+    chx_hip_tensor outv;
+    bool out_minus_128 = false;
+    CHX_PROPAGATE(result_view(out, flags, "inverted residual out", &outv, &out_minus_128));
+    auto refuse = [](const char* why) {
+        set_error("inverted residual: %s", why);
+        return (int)CHX_HIP_EUNSUPPORTED;
+    };
+    auto in_range = [](int32_t zp, int32_t dt) { return dt == CHX_HIP_INT8 ? zp >= -128 && zp <= 127 : zp >= 0 && zp <= 255; };
+    if (x->ndim != 4 || out->ndim != 4 || !is_q8(x->dtype) || x->shape[1] != plan->channels || !in_range(x_zero_point, x->dtype)) return refuse("x");
+    if ((flags & (CHX_HIP_ROUND_ONNX_RNE | CHX_HIP_FUSE_RELU)) != 0 || (plan->has_bias && !(flags & CHX_HIP_BIAS_ONNX_INT32))) return refuse("the flags");
+    const int32_t out_dtype = r ? outv.dtype : y_dtype;
+    if (y_dtype != CHX_HIP_UINT8 || outv.dtype != CHX_HIP_UINT8) return refuse("the type of a result");
+    const int64_t N = x->shape[0], H = x->shape[2], W = x->shape[3], OH = (H - 1) / plan->stride + 1, OW = (W - 1) / plan->stride + 1;
+    if (N < 1 || H < 1 || W < 1 || out->shape[0] != N || out->shape[1] != plan->out_channels || out->shape[2] != OH || out->shape[3] != OW) return refuse("the shape of the result");
+    int64_t x_px = 0, o_px = 0, r_px = 0;
+    if (!y_is_pixel_major(*x, &x_px) || !y_is_pixel_major(outv, &o_px)) return refuse("x or out is not channels-last");
+    const int64_t chunks = (plan->channels + 15) / 16;
+    if (!aligned(x->data, 16) || x_px % 16 != 0 || x_px < 16 * chunks || !aligned(out->data, 16) || o_px % 16 != 0 || o_px < plan->out_channels) return refuse("pixels that are not whole 16-byte chunks");
+    if (H * W * x_px >= (int64_t(1) << 31) || N >= (int64_t(1) << 24)) return refuse("an image of 2 GB");
+    if (byte_ranges_overlap(outv, *x)) return refuse("out overlaps x");
+    InvertedResidualArgs a;
+    memset(&a, 0, sizeof(a));
+    for (int i = 0; i < 3; ++i) {
+        if (!in_range(y_zero_points[i], CHX_HIP_UINT8)) return refuse("a zero point");
+    }
+    auto product = [&](int i, bool two_fma) {
+        const QuantParams q = make_quant_params(y_scales[i], y_zero_points[i], false);
+        return product_form(q, q.lo, false, two_fma);
+    };
+    a.q1 = product(0, true);
+    a.q2 = product(1, true);
+    if (a.q1.path != a.q2.path) {
+        a.q1 = product(0, false);
+        a.q2 = product(1, false);
+    }
+    a.q3 = product(2, true);
+    if (a.q1.path != a.q2.path || (a.q1.path != 1 && a.q1.path != 3) || a.q3.path == 0) return refuse("a requantization without a product form");
+    hipStream_t s = as_stream(stream);
+    if (r) {
+        CHX_PROPAGATE(check_tensor(r, "inverted residual r"));
+        for (int i = 0; i < 4; ++i)
+            if (r->ndim != 4 || r->shape[i] != out->shape[i]) return refuse("the shape of r");
+        if (!is_q8(r->dtype) || !in_range(r_zero_point, r->dtype) || !in_range(out_zero_point, out_dtype) || !(out_scale >= 0x1p-60f && out_scale <= 0x1p60f)) return refuse("the quantization of the sum");
+        if (!y_is_pixel_major(*r, &r_px) || !aligned(r->data, 16) || r_px % 16 != 0 || r_px < plan->out_channels) return refuse("r is not channels-last in whole chunks");
+        if (byte_ranges_overlap(outv, *r)) return refuse("out overlaps r");
+        std::lock_guard<std::mutex> lock(plan->mutex);
+        CHX_PROPAGATE(residual_of(*r, r_px, y_scales[2], y_zero_points[2], y_dtype, r_scale, r_zero_point, out_scale, out_zero_point, out_dtype, relu != 0,
+                                  plan->affine_residual, &plan->searched, s, &a.res));
+    }
+    a.x = static_cast<const char*>(x->data);
+    a.y = static_cast<char*>(out->data);
+    a.x_px = x_px;
+    a.x_n = H * W * x_px;
+    a.y_px = o_px;
+    a.y_n = OH * OW * o_px;
+    a.w1 = plan->memory;
+    a.w3 = plan->memory + plan->at_w3;
+    a.t1 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t1);
+    a.t2 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t2);
+    a.t3 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t3);
+    a.N = (int32_t)N; a.H = (int32_t)H; a.W = (int32_t)W; a.OH = (int32_t)OH; a.OW = (int32_t)OW;
+    a.OC = plan->out_channels;
+    a.hid_tiles = plan->tiles;
+    a.hid_tiles_padded = plan->tiles_padded;
+    a.x_chunks = (int32_t)chunks;
+    a.KS = plan->steps;
+    a.x_flip = x->dtype == CHX_HIP_UINT8 ? 0x80808080u : 0u;
+    a.y_flip = out_minus_128 ? 0x80808080u : 0u;
+    a.corr1 = (x->dtype == CHX_HIP_UINT8 ? 128 : 0) - x_zero_point;
+    a.corr2 = 128 - y_zero_points[0];
+    a.corr3 = 128 - y_zero_points[1];
+    a.s1 = x_scale;
+    a.s2 = y_scales[0];
+    a.s3 = y_scales[1];
+    a.fill = (int32_t)(((uint32_t)y_zero_points[0] ^ 0x80u) * 0x01010101u);
+    return launch_inverted_residual(a, plan->stride, s);
+}

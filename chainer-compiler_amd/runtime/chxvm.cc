@@ -336,6 +336,119 @@ private:
     std::shared_ptr<ResidualFusionState> state_;
 };
 
+std::atomic<int64_t> g_inverted_residuals{0};
+
+// The three convolutions of an inverted residual block (1x1 expansion, depthwise 3x3, 1x1 projection whose results in between
+// nobody else reads), and the residual sum behind them where the projection may compute it, as one launch
+// (chx_hip_inverted_residual_run).  It stands where the projection stood; what that kernel does not take runs as the program
+// wrote it.  The operands are constants of the program, laid out when it is loaded.
+class InvertedResidualOp : public ChxVMOp {
+public:
+    struct Quantization {  // the variable slots of a convolution
+        int x_scale, x_zp, y_scale, y_zp;
+    };
+    struct Sum {
+        chx_hip_residual_group group;
+        int conv_operand = 0, other = -1, out = -1;
+        std::shared_ptr<ResidualFusionState> state;  // null: no sum
+    };
+    InvertedResidualOp(const ChxVMInstructionProto& projection, std::shared_ptr<chx_hip_inverted_residual> block, int x, int between, const std::vector<Quantization>& convs,
+                       int64_t out_channels, int stride, bool has_bias, Sum sum, std::vector<ChxVMOp*> steps, std::vector<int> freed)
+        : ChxVMOp(projection), block_(std::move(block)), x_(x), between_(between), y_(projection.outputs[0]), convs_(convs), out_channels_(out_channels), stride_(stride),
+          has_bias_(has_bias), sum_(std::move(sum)), steps_(std::move(steps)), freed_(std::move(freed)) {
+    }
+
+    void Run(ChxVMState* st) override {
+        if (RunAsOne(st)) {
+            for (int slot : freed_) st->FreeVar(slot);
+        } else {
+            for (ChxVMOp* op : steps_) op->Run(st);
+        }
+    }
+
+private:
+    static int32_t Integer(const StrictScalar& z) {
+        return static_cast<int32_t>(static_cast<int64_t>(z));
+    }
+
+    // false: nothing has been written
+    bool RunAsOne(ChxVMState* st) {
+        if (st->GetVar(x_)->IsNull() || (has_bias_ && !st->options().qlinearconv_onnx_int32_bias)) return false;
+        float scales[3];
+        int32_t zero_points[3];
+        for (int i = 0; i < 3; ++i) {
+            for (int slot : {convs_[i].x_scale, convs_[i].x_zp, convs_[i].y_scale, convs_[i].y_zp})
+                if (st->GetVar(slot)->IsNull()) return false;
+            const StrictScalar& zp = st->GetScalar(convs_[i].y_zp);
+            if (zp.dtype() != chainerx::Dtype::kUInt8) return false;
+            scales[i] = static_cast<float>(st->GetScalar(convs_[i].y_scale));
+            zero_points[i] = Integer(zp);
+            // each reads its input the way the one before wrote it
+            if (i > 0 && (static_cast<float>(st->GetScalar(convs_[i].x_scale)) != scales[i - 1] || Integer(st->GetScalar(convs_[i].x_zp)) != zero_points[i - 1] ||
+                          st->GetScalar(convs_[i].x_zp).dtype() != chainerx::Dtype::kUInt8))
+                return false;
+        }
+        const chainerx::Array x = st->GetArray(x_);
+        if (x.ndim() != 4) return false;
+        const StrictScalar& x_zp = st->GetScalar(convs_[0].x_zp);
+        // a value kept as code - 128 is an int8 tensor with the zero point 128 lower
+        auto minus_128 = [&](int slot, const chainerx::Array& a, chainerx::Dtype type_in_program) {
+            return st->store_minus_128(slot) && a.dtype() == chainerx::Dtype::kInt8 && type_in_program == chainerx::Dtype::kUInt8;
+        };
+        const int out_slot = sum_.state ? sum_.out : y_;
+        const bool signed_storage = st->store_minus_128(out_slot);
+        const chainerx::Shape shape{x.shape()[0], out_channels_, (x.shape()[2] - 1) / stride_ + 1, (x.shape()[3] - 1) / stride_ + 1};
+        chainerx::Array r;
+        int32_t r_zp = 0;
+        if (sum_.state) {
+            const chx_hip_residual_group& g = sum_.group;
+            const int k = sum_.conv_operand;
+            if (st->GetVar(sum_.other)->IsNull() || g.in_scale[k] != scales[2] || g.in_zero_point[k] != zero_points[2] ||
+                static_cast<chainerx::Dtype>(g.in_dtype[k]) != chainerx::Dtype::kUInt8 || static_cast<chainerx::Dtype>(g.out_dtype) != chainerx::Dtype::kUInt8)
+                return false;
+            r = st->GetArray(sum_.other);
+            const chainerx::Dtype r_type = static_cast<chainerx::Dtype>(g.in_dtype[1 - k]);
+            const bool lowered = minus_128(sum_.other, r, r_type);
+            if ((r.dtype() != r_type && !lowered) || r.shape() != shape) return false;
+            r_zp = g.in_zero_point[1 - k] - (lowered ? 128 : 0);
+        }
+        chainerx::Array out = chainerx::EmptyChannelsLastPadded(shape, signed_storage ? chainerx::Dtype::kInt8 : chainerx::Dtype::kUInt8);
+        const chx_hip_tensor xt = x.hip();
+        chx_hip_tensor ot = out.hip(), rt;
+        if (sum_.state) rt = r.hip();
+        const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT) |
+                               (signed_storage ? CHX_HIP_STORE_MINUS_128 : 0u);
+        const int rc = chx_hip_inverted_residual_run(
+                block_.get(), &xt, static_cast<float>(st->GetScalar(convs_[0].x_scale)), Integer(x_zp) - (minus_128(x_, x, x_zp.dtype()) ? 128 : 0), scales, zero_points,
+                static_cast<int32_t>(chainerx::Dtype::kUInt8), flags, sum_.state ? &rt : nullptr, sum_.group.in_scale[1 - sum_.conv_operand], r_zp, sum_.group.out_scale,
+                sum_.group.out_zero_point, sum_.group.relu, &ot, chainerx::CurrentStream());
+        // (what it refuses, and operands that are in error, are for the instructions)
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(block_);  // a recording may outlive the program
+        // (the depthwise result is code - 128 on its way to the projection)
+        CountMinus128Stores((signed_storage ? 1 : 0) + (st->store_minus_128(between_) ? 1 : 0));
+        if (sum_.state) {
+            sum_.state->fused = true;
+            CountResidualFusion();
+            st->count_residual_fusion();
+        }
+        st->SetArray(out_slot, out);
+        ++g_inverted_residuals;
+        return true;
+    }
+
+    std::shared_ptr<chx_hip_inverted_residual> block_;
+    int x_, between_, y_;
+    std::vector<Quantization> convs_;
+    int64_t out_channels_;
+    int stride_;
+    bool has_bias_;
+    Sum sum_;
+    std::vector<ChxVMOp*> steps_;
+    std::vector<int> freed_;
+};
+
 // A fused op followed by the Free instructions of its operands that the program had placed
 // between the instructions it replaces.
 class SequenceOp : public ChxVMOp {
@@ -759,9 +872,102 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         remaining_.swap(rest);
     }
+    // Inverted residual blocks, for the same runs: three convolutions whose results in between have one reader, over constants.
+    auto constant_array = [&](int slot) -> const chainerx::Array* {
+        return slot >= 0 && constant_slots_[slot] && constant_slots_[slot]->kind() == ChxVMVar::Kind::kArray ? &constant_slots_[slot]->GetArray() : nullptr;
+    };
+    auto all_are = [](const std::vector<int64_t>& v, int64_t value) { return std::all_of(v.begin(), v.end(), [&](int64_t e) { return e == value; }); };
+    auto convolution = [&](int i, bool last) {  // one that may be part of a block
+        if (i < 0) return false;
+        const ChxVMInstructionProto& inst = program.instructions[i];
+        if (inst.op != kQLinearConv || inst.inputs.size() != 13 || inst.outputs.size() != 1 || !(role[i] == 0 || (last && role[i] == 4)) || chained[i]) return false;
+        if (!(inst.inputs[12].s.empty() || inst.inputs[12].s == "NOTSET")) return false;
+        for (int k : {0, 3, 4, 5, 8})
+            if (!once(inst.inputs[k].array) || (k != 8 && inst.inputs[k].array < 0)) return false;
+        for (int k : {1, 2, 6, 7})
+            if (inst.inputs[k].scalar < 0 || !once(inst.inputs[k].scalar)) return false;
+        for (int k : {3, 4, 5})
+            if (!constant_array(inst.inputs[k].array)) return false;
+        return once(inst.outputs[0]) && (inst.inputs[8].array < 0 || constant_array(inst.inputs[8].array));
+    };
+    std::vector<int> conv_reader(num_variables_ > 0 ? num_variables_ : 1, -1);
+    for (int i = 0; i < n; ++i)
+        if (program.instructions[i].op == kQLinearConv && !program.instructions[i].inputs.empty() && program.instructions[i].inputs[0].array >= 0)
+            conv_reader[program.instructions[i].inputs[0].array] = i;
+    for (int e = 0; e < n; ++e) {
+        if (!convolution(e, false)) continue;
+        const int h1 = program.instructions[e].outputs[0], d = conv_reader[h1];
+        if (d <= e || !single_use(h1) || !convolution(d, false)) continue;
+        const int h2 = program.instructions[d].outputs[0], p = conv_reader[h2];
+        if (p <= d || !single_use(h2) || !convolution(p, true)) continue;
+        const int members[3] = {e, d, p};
+        const ChxVMInstructionProto& di = program.instructions[d];
+        const int64_t stride = di.inputs[9].ints.empty() ? 1 : di.inputs[9].ints[0];
+        bool fits = all_are(di.inputs[9].ints, stride) && !di.inputs[10].ints.empty() && all_are(di.inputs[10].ints, 1) && di.inputs[11].i > 1;
+        for (int m : {e, p}) {
+            const ChxVMInstructionProto& inst = program.instructions[m];
+            fits = fits && all_are(inst.inputs[9].ints, 1) && all_are(inst.inputs[10].ints, 0) && inst.inputs[11].i == 1;
+        }
+        if (!fits) continue;
+        chx_hip_conv_operands stages[3];
+        chx_hip_tensor tensors[3][4];
+        std::vector<InvertedResidualOp::Quantization> convs;
+        std::set<int> slots = {h1, h2, program.instructions[e].inputs[0].array};
+        for (int m = 0; m < 3; ++m) {
+            const ChxVMInstructionProto& inst = program.instructions[members[m]];
+            const int operand[4] = {inst.inputs[3].array, inst.inputs[4].array, inst.inputs[5].array, inst.inputs[8].array};
+            for (int k = 0; k < 4; ++k)
+                if (operand[k] >= 0) {
+                    tensors[m][k] = constant_array(operand[k])->hip();
+                    slots.insert(operand[k]);
+                }
+            stages[m] = {&tensors[m][0], &tensors[m][1], &tensors[m][2], operand[3] >= 0 ? &tensors[m][3] : nullptr};
+            convs.push_back({inst.inputs[1].scalar, inst.inputs[2].scalar, inst.inputs[6].scalar, inst.inputs[7].scalar});
+            for (int k : {1, 2, 6, 7}) slots.insert(inst.inputs[k].scalar);
+        }
+        if (tensors[1][0].shape[0] != di.inputs[11].i) continue;  // (as many groups as channels)
+        chx_hip_inverted_residual* block = nullptr;
+        const int rc = chx_hip_inverted_residual_create(stages, static_cast<int32_t>(stride), chainerx::CurrentStream(), &block);
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        InvertedResidualOp::Sum sum = {};
+        if (role[p] == 4) {
+            const ChxVMInstructionProto& group = program.instructions[partner[p]];
+            sum.group = groups[p];
+            sum.conv_operand = conv_operand[p];
+            sum.other = group.inputs[0].array_list[1 - conv_operand[p]];
+            sum.out = group.outputs[0];
+            sum.state = fusion_state[p];
+        }
+        std::set<int> moved(members, members + 3);
+        std::vector<ChxVMOp*> steps;
+        std::vector<int> freed;
+        for (int i = e; i <= p; ++i) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
+                freed.push_back(inst.inputs[0].array);
+                moved.insert(i);
+            }
+            if (moved.count(i)) steps.push_back(program_[i].get());
+        }
+        chains_.emplace_back(new InvertedResidualOp(program.instructions[p], std::shared_ptr<chx_hip_inverted_residual>(block, chx_hip_inverted_residual_destroy),
+                                                    program.instructions[e].inputs[0].array, h2, convs, tensors[2][0].shape[0], static_cast<int>(stride),
+                                                    stages[0].bias != nullptr, sum, std::move(steps), std::move(freed)));
+        for (int m : members) chained[m] = true;
+        std::vector<std::pair<int, ChxVMOp*>> rest;
+        for (const auto& r : remaining_) {
+            if (r.first == p) rest.emplace_back(p, chains_.back().get());
+            else if (!moved.count(r.first)) rest.push_back(r);
+        }
+        remaining_.swap(rest);
+    }
 }
 
 ChxVM::~ChxVM() = default;
+
+int64_t InvertedResiduals() {
+    return g_inverted_residuals.load();
+}
 
 int64_t MatMulChains() {
     return g_matmul_chains.load();

@@ -47,6 +47,10 @@ int64_t Minus128Stores();  // results written in that storage so far, process-wi
 // The plain uint8 array of a value held in that storage (chx_hip_codes_minus_128).
 chainerx::Array PlainCodes(const chainerx::Array& minus_128);
 
+// for ops outside ops/quantize.cc that do the same
+void CountResidualFusion();
+void CountMinus128Stores(int64_t n);
+int64_t InvertedResiduals();  // inverted residual blocks run as one launch so far, process-wide
 int64_t MatMulChains();  // chains of quantized products run as one launch so far, process-wide
 
 class ChxVM {

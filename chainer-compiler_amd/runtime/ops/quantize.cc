@@ -47,6 +47,14 @@ int64_t Minus128Stores() {
     return g_minus_128_stores.load();
 }
 
+void CountResidualFusion() {
+    ++g_residual_fusions;
+}
+
+void CountMinus128Stores(int64_t n) {
+    g_minus_128_stores += n;
+}
+
 chainerx::Array PlainCodes(const chainerx::Array& minus_128) {
     CHECK(minus_128.dtype() == chainerx::Dtype::kInt8);
     const bool channels_last = minus_128.ndim() == 4 && !minus_128.IsContiguous() && minus_128.strides()[1] == minus_128.GetItemSize();

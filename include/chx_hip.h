@@ -279,6 +279,26 @@ int chx_hip_conv_integer(
         const chx_hip_tensor* x, const chx_hip_tensor* w, int32_t x_zero_point, const chx_hip_tensor* w_zero_point,
         const chx_hip_conv_params* params, chx_hip_tensor* y, void* stream);
 
+/* An inverted residual block: 1x1 convolution, depthwise 3x3 with padding 1 and stride 1 or 2, 1x1 convolution, and
+ * optionally the residual sum of chx_hip_qconv_plan_run_add, as one launch, with the codes of the single calls.
+ * stages: the three convolutions' int8 weights (zero points 0), scales, zero points and int32 biases (all or none NULL);
+ * they are laid out when the block is created, which waits for the stream, and not needed afterwards. */
+typedef struct chx_hip_conv_operands {
+    const chx_hip_tensor *w, *w_scale, *w_zero_point, *bias;
+} chx_hip_conv_operands;
+typedef struct chx_hip_inverted_residual chx_hip_inverted_residual;
+int chx_hip_inverted_residual_create(const chx_hip_conv_operands* stages, int32_t stride, void* stream, chx_hip_inverted_residual** out);
+void chx_hip_inverted_residual_destroy(chx_hip_inverted_residual* plan);
+/* y_scales, y_zero_points: of the three convolutions' results, all of type y_dtype.  r NULL: `out` is the third one's;
+ * else the sum of it and r (arguments as for chx_hip_qconv_plan_run_add).  CHX_HIP_EUNSUPPORTED, with nothing launched, for
+ * what the kernel does not take (anything but channels-last arrays in whole 16-byte chunks, uint8 results, the reference's
+ * rounding, an int32 bias of the ONNX kind, rows that fit LDS) or is not the faster one for; the single calls then say
+ * what is wrong with the operands, if something is. */
+int chx_hip_inverted_residual_run(
+        chx_hip_inverted_residual* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points,
+        int32_t y_dtype, uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu,
+        chx_hip_tensor* out, void* stream);
+
 /* MatMulIntegerOp::RunImpl, runtime/ops/quantize.cc:96-114 with NumpyMatMul,
  * runtime/chainerx_util.cc:210-230.  a [..,M,K], b [..,K,N] with equal leading
  * dims, y int32 [..,M,N].  Zero points: NULL, or arrays of ndim <= 1 subtracted by

@@ -224,6 +224,9 @@ hipError_t hipGetLastError() {
 hipError_t hipGetSymbolAddress(void** p, const void*) {
     return allocate(p, 1 << 16, t_device);
 }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) {
+    return hipSuccess;
+}
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
     *n = 2;
     return hipSuccess;
