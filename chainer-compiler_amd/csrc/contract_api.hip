@@ -223,7 +223,8 @@ bool weights_fit_mfma(const chx_hip_tensor& w, int group) {
 // How a convolution is launched, beyond what its operands decide.  The defaults are what a host wants; the
 // environment variables are overrides for tuning and for tests (which reach every launch configuration through them),
 // read when a plan is created or a one-shot entry point is called, never on the path of a plan's runs.
-//   CHX_HIP_TILE=<oc>,<px>[,<work-groups per compute unit>[,<wavefronts: 4 or 8>]]  forces a launch configuration
+//   CHX_HIP_TILE=<oc>,<px>[,<work-groups per compute unit>[,<wavefronts: 4 or 8>]]  forces a launch configuration (with the
+//                               small tiles, in place of the work-groups: 1 for pixels from LDS, where that fits)
 //   CHX_HIP_AUTOTUNE=0          keeps the heuristic tile choice instead of timing the configurations
 //   CHX_HIP_NO_STEM=1           keeps few-channel first layers off the planar-input kernel
 //   CHX_HIP_AFFINE_RESIDUAL=0   keeps fused residual sums on the operation-by-operation arithmetic
@@ -368,8 +369,10 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
     // read their operands from L2 once per tile
     if (!out_int32 && conv_split_takes(a) && (int64_t)((a.OC + 63) / 64) * ((a.M + 63) / 64) <= 2048)
         for (const ConvSplitTile& t : kConvSplitTiles)
-            if (t.waves * 512 / t.oc <= a.KP)  // (half a step and more for every wavefront)
+            if (t.waves * 512 / t.oc <= a.KP) {  // (half a step and more for every wavefront)
                 all.push_back({{t.oc, t.px, 0, t.waves}, {}});
+                if (conv_split_patch_takes(a, t.oc, t.px, t.waves)) all.push_back({{t.oc, t.px, kConvSplitPatch, t.waves}, {}});
+            }
 
     if (!out_int32 && conv_point_takes(a))
         for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, {}});

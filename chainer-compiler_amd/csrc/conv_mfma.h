@@ -184,7 +184,10 @@ struct ConvSplitTile {
 constexpr ConvSplitTile kConvSplitTiles[] = {{16, 16, 8}, {16, 16, 16}, {16, 32, 4}, {16, 32, 8}, {16, 32, 16}, {32, 32, 2}, {32, 32, 4}, {32, 32, 8}, {32, 64, 4}, {32, 64, 8}};
 bool conv_split_has(int tile_oc, int tile_px, int waves);
 inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
-int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s);
+// `patch`: several taps over an image whose results have its own size, its pixels from LDS (else, and for what that does not take, from memory)
+constexpr int kConvSplitPatch = 1;  // ... as a launch configuration: in the place of the work-groups per compute unit
+bool conv_split_patch_takes(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves);
+int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool patch, bool x_unsigned, bool rne, hipStream_t s);
 
 // 1x1, stride 1, no padding over a dense image: input pixel m is at x + m * x_w_stride
 inline bool conv_px_linear(const ConvMfmaArgs& a) {

@@ -406,7 +406,7 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     }
     if (tile_oc <= 32) {
         if (out_int32) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the %dx%d tile has 8-bit results only", tile_oc, tile_px);
-        return launch_conv_split(a, tile_oc, tile_px, waves, x_unsigned, rne, s);
+        return launch_conv_split(a, tile_oc, tile_px, waves, max_wgs_per_cu == kConvSplitPatch, x_unsigned, rne, s);
     }
     if (waves == 8) {
         // eight wavefronts: the pixels of the tile are split four ways

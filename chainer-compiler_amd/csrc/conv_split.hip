@@ -11,6 +11,15 @@
 //
 // Arguments, requantization, residual sums, pairs and storage are those of conv_mfma_kernel; filter taps outside the
 // image are replaced by the zero point on the fragment.
+//
+// With several taps a tile's pixels are gathered once per tap, 32 or 64 bytes from a pixel at a time: nine times 32 x 256
+// bytes for what lies in 62 x 256.  Where the results have the image's own size those taps fall on one run of pixels of the
+// dense image, and kPatch brings that run into LDS, once, while the weights of up to nine steps are on their way; a step then
+// is weights from memory and a 16-byte LDS read per lane, pixels an odd number of 16 bytes apart (no bank conflicts), taps
+// outside the image read 64 bytes of zero point.  In us, best tile with the pixels from memory and from LDS, launches
+// back to back with weights of their own, 3x3 filters: one image, 512 channels at 7x7 8.5 and 5.9, 256 at 14x14 5.4 and 4.6,
+// 128 at 28x28 4.8 and 4.3, 64 at 56x56 3.9 and 4.4; eight images, 11.9 and 7.9, 9.8 and 6.8, 7.1 (staged tiles) and 8.2,
+// 6.9 (staged tiles) and 8.9.  So both are measured per shape.
 #include <type_traits>
 
 #include "conv_mfma.h"
@@ -37,16 +46,23 @@ struct ConvSplitArgs {
     uint32_t x_flip;
     int32_t rne, tiles_per_xcd;
     uint32_t tiles_px_mul, tiles_px_shift, c64_mul, c64_shift, kw_mul, kw_shift;  // magic_divisor(tiles_px), (C64), (KW): a division costs some 150 cycles
+    int32_t patch_chunks, patch_pitch;       // kPatch: 16-byte chunks of the patch, bytes from a pixel to the next in LDS
+    uint32_t chunks_mul, chunks_shift;       // magic_divisor(chunks per pixel)
 };
 
+// Where the pixels come from: one filter tap, from memory; several taps, from memory; several taps over an image whose
+// results have its own size, from LDS.
+enum Form { kPoint, kTaps, kPatch };
+
 // (two wavefronts per SIMD promised, so that the sums stay out of the accumulation registers: see conv_stem_kernel)
-template <int R, int PN, int W, bool kTaps, int kDepth>
+template <int R, int PN, int W, Form kForm, int kDepth>
 __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
     constexpr int kGroups = 64 / R, kStep = 16 * kGroups;  // K bytes per MFMA: 32 or 64
     constexpr int kQuads = R * R / 256;                    // groups of four result registers: 4 or 1
     constexpr int kUnits = PN * kQuads;
     using acc_t = typename std::conditional<R == 32, v16i, v4i>::type;
     __shared__ __attribute__((aligned(16))) v4i part[W > 1 ? W : 1][W > 1 ? kUnits : 1][64];
+    extern __shared__ __attribute__((aligned(16))) char patch[];  // kPatch: 64 bytes of the zero point, then the pixels
 
     const ConvSplitArgs args = kernel_arguments<ConvSplitArgs>();
     const ConvMfmaArgs& a = args.conv;
@@ -62,7 +78,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
     // so a round trip to memory costs more than a microsecond here and the kernel is a chain of them.  The weights of the
     // first steps are requested before the pixels' addresses are known, and the operands of the epilogue before the loop.
     struct Step {
-        v4i w, x[PN];
+        v4i w, x[kForm == kPatch ? 1 : PN];
     };
     const int steps = a.KP / kStep, per = (steps + W - 1) / W, lo = wave * per, hi = min(steps, lo + per), last = hi - 1;
     const uint32_t w_off = (uint32_t)(oc >> 6) * (uint32_t)(64 * a.KP) + (uint32_t)((oc & 63) * a.bk + group * 16);
@@ -72,6 +88,33 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
         const uint32_t k = (uint32_t)(min(step, last) * kStep);
         s.w = *reinterpret_cast<const v4i*>(a.wp + (((k >> bk_shift) * 64u) << bk_shift) + (k & (uint32_t)(a.bk - 1)) + w_off);
     };
+    const int fill = (int)((uint32_t)(a.x_zp & 0xff) * 0x01010101u);
+    // The patch: the pixels that the taps of the tile's pixels fall on are one run of the dense image.  (Pixels outside x are
+    // replaced by others: only taps outside the image look at them.)
+    constexpr int kBatch = W >= 8 ? 4 : 8, kThreads = 64 * W;
+    const int patch_px0 = px_tile * PN * R - a.ph * a.W - a.pw;
+    auto load_patch = [&](int base, v4i* v) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const uint32_t i = (uint32_t)min(base + b * kThreads + (int)threadIdx.x, args.patch_chunks - 1);
+            const uint32_t px = fast_div(i, args.chunks_mul, args.chunks_shift), chunk = i - px * (uint32_t)(a.C16 >> 4);
+            const int m = min(max(patch_px0 + (int)px, 0), (int)a.M - 1);
+            v[b] = *reinterpret_cast<const v4i*>(a.x + ((uint32_t)m * (uint32_t)a.x_w_stride + chunk * 16));
+        }
+    };
+    auto store_patch = [&](int base, const v4i* v) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const uint32_t i = (uint32_t)min(base + b * kThreads + (int)threadIdx.x, args.patch_chunks - 1);
+            const uint32_t px = fast_div(i, args.chunks_mul, args.chunks_shift), chunk = i - px * (uint32_t)(a.C16 >> 4);
+            v4i flipped = v[b];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) flipped[e] ^= (int)args.x_flip;
+            *reinterpret_cast<v4i*>(patch + 64 + px * (uint32_t)args.patch_pitch + chunk * 16) = flipped;
+        }
+    };
+    v4i batch[kForm == kPatch ? kBatch : 1];
+    if constexpr (kForm == kPatch) load_patch(0, batch);
     Step ring[kDepth];
     if (lo < hi) {
 #pragma unroll
@@ -90,7 +133,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
             const uint32_t n = fast_div(r, a.oh_mul, a.oh_shift), oh = r - n * (uint32_t)a.OH;
             const int ih0 = (int)oh * a.sh - a.ph, iw0 = (int)ow * a.sw - a.pw;
             x_off[j] = (int32_t)n * (int32_t)a.x_n_stride + ih0 * (int32_t)a.x_h_stride + iw0 * (int32_t)a.x_w_stride;
-            if (kTaps) {
+            if (kForm != kPoint) {
                 const int c_lo = min(max(-iw0, 0), a.KW), c_hi = min(max(a.W - iw0, 0), a.KW);
                 const int r_lo = min(max(-ih0, 0), a.KH), r_hi = min(max(a.H - ih0, 0), a.KH);
                 // the column bits repeated in every filter row, the rows outside the image cut off
@@ -99,23 +142,41 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
                 taps[j] = (cols * a.row_unit) & rows;
             }
         }
+        if constexpr (kForm == kPatch) x_off[j] = 64 + (j * R + col) * args.patch_pitch;
         x_off[j] += group * 16;
     }
-    const int fill = (int)((uint32_t)(a.x_zp & 0xff) * 0x01010101u);
 
     // the step whose pixels are loaded next: its place in its filter tap, the tap, and the offset into x
     int k_in = 0, tap = 0, kw = 0, at = lo;
     uint32_t x_at = 0;
-    if constexpr (kTaps) {
+    if constexpr (kForm != kPoint) {
         const int k = lo * kStep;
         tap = (int)fast_div((uint32_t)k, args.c64_mul, args.c64_shift);
         k_in = k - tap * a.C64;
         const int kh = (int)fast_div((uint32_t)tap, args.kw_mul, args.kw_shift);
         kw = tap - kh * a.KW;
-        x_at = (uint32_t)(kh * (int)a.x_h_stride + kw * (int)a.x_w_stride + k_in);
+        x_at = kForm == kPatch ? (uint32_t)((kh * a.W + kw) * args.patch_pitch + k_in) : (uint32_t)(kh * (int)a.x_h_stride + kw * (int)a.x_w_stride + k_in);
     }
+    const uint32_t row_step = kForm == kPatch ? (uint32_t)((a.W - a.KW + 1) * args.patch_pitch) : (uint32_t)a.x_h_stride - (uint32_t)((a.KW - 1) * (int)a.x_w_stride);
+    const uint32_t column_step = kForm == kPatch ? (uint32_t)args.patch_pitch : (uint32_t)a.x_w_stride;
+    auto next_step = [&]() {
+        if (at < last) {
+            ++at;
+            k_in += kStep;
+            x_at += kStep;
+            if (k_in == a.C64) {
+                x_at -= (uint32_t)a.C64;
+                k_in = 0;
+                ++tap;
+                ++kw;
+                const bool row = kw == a.KW;
+                kw = row ? 0 : kw;
+                x_at += row ? row_step : column_step;
+            }
+        }
+    };
     auto load_x = [&](Step& s) {
-        if constexpr (!kTaps) {  // (channels past C16: as below)
+        if constexpr (kForm == kPoint) {  // (channels past C16: as below)
             const uint32_t k = (uint32_t)(at * kStep);
             at = min(at + 1, last);
 #pragma unroll
@@ -129,32 +190,19 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
         const bool channels = k_in + group * 16 < a.C16;
 #pragma unroll
         for (int j = 0; j < PN; ++j) {
-            const bool inside = channels && (!kTaps || ((taps[j] >> tap) & 1));
+            const bool inside = channels && ((taps[j] >> tap) & 1);
             const uint32_t off = inside ? (uint32_t)x_off[j] + x_at : 0u;
             s.x[j] = *reinterpret_cast<const v4i*>(a.x + off);
-            if (kTaps) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s.x[j][e] = inside ? s.x[j][e] : fill;
-            }
+            for (int e = 0; e < 4; ++e) s.x[j][e] = inside ? s.x[j][e] : fill;
         }
-        if (at < last) {
-            ++at;
-            k_in += kStep;
-            x_at += kStep;
-            if (k_in == a.C64) {
-                x_at -= (uint32_t)a.C64;
-                k_in = 0;
-                ++tap;
-                ++kw;
-                const bool row = kw == a.KW;
-                kw = row ? 0 : kw;
-                x_at += row ? (uint32_t)a.x_h_stride - (uint32_t)((a.KW - 1) * (int)a.x_w_stride) : (uint32_t)a.x_w_stride;
-            }
-        }
+        next_step();
     };
-    if (lo < hi) {
+    if constexpr (kForm != kPatch) {
+        if (lo < hi) {
 #pragma unroll
-        for (int d = 0; d < kDepth; ++d) load_x(ring[d]);
+            for (int d = 0; d < kDepth; ++d) load_x(ring[d]);
+        }
     }
     // unit u of the result: four channels of one pixel per lane (u / kQuads: block of R pixels, u % kQuads: of 8 channels);
     // this wavefront finishes units wave, wave + W, ...
@@ -213,15 +261,33 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
     for (int j = 0; j < PN; ++j)
 #pragma unroll
         for (int r = 0; r < 4 * kQuads; ++r) acc[j][r] = 0;
+    if constexpr (kForm == kPatch) {
+        if (threadIdx.x < 16) reinterpret_cast<int*>(patch)[threadIdx.x] = fill ^ (int)args.x_flip;
+        store_patch(0, batch);
+        for (int base = kBatch * kThreads; base < args.patch_chunks; base += kBatch * kThreads) {
+            load_patch(base, batch);
+            store_patch(base, batch);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
     auto multiply = [&](const Step& s) {
 #pragma unroll
         for (int j = 0; j < PN; ++j) {
-            v4i fx = s.x[j];
+            v4i fx;
+            if constexpr (kForm == kPatch) {  // (channels past C16 have zero weights: what follows a pixel's channels is some other's)
+                const uint32_t off = (taps[j] >> tap) & 1 ? (uint32_t)x_off[j] + x_at : (uint32_t)(group * 16);
+                fx = *reinterpret_cast<const v4i*>(patch + off);
+            } else {
+                fx = s.x[j];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fx[e] ^= (int)args.x_flip;
+                for (int e = 0; e < 4; ++e) fx[e] ^= (int)args.x_flip;
+            }
             if constexpr (R == 32) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(s.w, fx, acc[j], 0, 0, 0);
             else acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(s.w, fx, acc[j], 0, 0, 0);
         }
+        if constexpr (kForm == kPatch) next_step();
     };
     if (lo < hi) {
         int step = lo;
@@ -230,7 +296,7 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
             for (int d = 0; d < kDepth; ++d) {
                 multiply(ring[d]);
                 load_w(step + d + kDepth, ring[d]);
-                load_x(ring[d]);
+                if constexpr (kForm != kPatch) load_x(ring[d]);
             }
         }
 #pragma unroll
@@ -294,15 +360,33 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
     }
 }
 
+constexpr int kLdsOfUnit = 160 * 1024;
+
+constexpr int partial_bytes(int R, int PN, int W) {
+    return W > 1 ? W * PN * (R * R / 256) * 1024 : 0;
+}
+
+int patch_pitch(const ConvMfmaArgs& a) {  // an odd number of 16 bytes: no bank conflicts
+    return a.C16 % 32 == 0 ? a.C16 + 16 : a.C16;
+}
+
+int patch_pixels(const ConvMfmaArgs& a, int tile_px) {
+    return tile_px + (a.KH - 1) * a.W + a.KW - 1;
+}
+
+int patch_bytes(const ConvMfmaArgs& a, int tile_px) {
+    return 64 + patch_pixels(a, tile_px) * patch_pitch(a) + 64;  // (a pixel's channels are read up to C64)
+}
+
 // kDepth: steps in flight.  All of a wavefront's steps when they are no more than eight (as far as registers allow: six of
 // the largest tile, five with sixteen wavefronts): each round trip less is most of a microsecond.  ResNet-50 on one image
 // 303 -> 294 us.
 template <int R, int PN, int W>
-int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, bool taps, hipStream_t s) {
+int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, Form form, hipStream_t s) {
     constexpr int kDeep = R * PN == 64 ? 6 : W == 16 && PN == 2 ? 5 : 8, kStep = 1024 / R;
     const int64_t tiles = (int64_t)a.tiles_oc * a.tiles_px;
     const int per_xcd = (int)((tiles + 7) / 8);
-    const bool deep = (a.KP / kStep + W - 1) / W > 4;
+    const int steps = (a.KP / kStep + W - 1) / W;
     ConvSplitArgs args;
     args.conv = a;
     args.x_flip = flip;
@@ -311,11 +395,23 @@ int launch(const ConvMfmaArgs& a, uint32_t flip, bool rne, bool taps, hipStream_
     magic_divisor((uint32_t)a.tiles_px, &args.tiles_px_mul, &args.tiles_px_shift);
     magic_divisor((uint32_t)a.C64, &args.c64_mul, &args.c64_shift);
     magic_divisor((uint32_t)a.KW, &args.kw_mul, &args.kw_shift);
-#define CHX_SPLIT(TAPS, DEPTH) conv_split_kernel<R, PN, W, TAPS, DEPTH><<<8 * per_xcd, 64 * W, 0, s>>>(args)
-    if (taps && deep) CHX_SPLIT(true, kDeep);
-    else if (taps) CHX_SPLIT(true, 4);
-    else if (deep) CHX_SPLIT(false, kDeep);
-    else CHX_SPLIT(false, 4);
+    magic_divisor((uint32_t)(a.C16 / 16), &args.chunks_mul, &args.chunks_shift);
+    args.patch_pitch = patch_pitch(a);
+    args.patch_chunks = patch_pixels(a, R * PN) * (a.C16 / 16);
+    const int lds = form == kPatch ? patch_bytes(a, R * PN) : 0;
+#define CHX_SPLIT(FORM, DEPTH)                                                                                                                             \
+    do {                                                                                                                                                   \
+        if (lds + partial_bytes(R, PN, W) > 64 * 1024) /* (has to be asked for, on every device) */                                                        \
+            CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_split_kernel<R, PN, W, FORM, DEPTH>), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                             kLdsOfUnit - partial_bytes(R, PN, W)));                                                                       \
+        conv_split_kernel<R, PN, W, FORM, DEPTH><<<8 * per_xcd, 64 * W, lds, s>>>(args);                                                                   \
+    } while (0)
+    if (form == kPatch && steps > 5) CHX_SPLIT(kPatch, 9);  // (a step in flight is four registers: 4.5 or 9 for the layers of ResNet-50)
+    else if (form == kPatch) CHX_SPLIT(kPatch, 5);
+    else if (form == kTaps && steps > 4) CHX_SPLIT(kTaps, kDeep);
+    else if (form == kTaps) CHX_SPLIT(kTaps, 4);
+    else if (steps > 4) CHX_SPLIT(kPoint, kDeep);
+    else CHX_SPLIT(kPoint, 4);
 #undef CHX_SPLIT
     return launch_check("conv_split_kernel");
 }
@@ -328,12 +424,22 @@ bool conv_split_has(int tile_oc, int tile_px, int waves) {
     return false;
 }
 
-int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, bool rne, hipStream_t s) {
+// Stride 1, the results' image of the input's size, its pixels dense: a tap is a distance in pixels.  The run has to fit LDS
+// beside the partial sums, and its indices 32 bits.
+bool conv_split_patch_takes(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves) {
+    return a.KH * a.KW > 1 && a.KH * a.KW <= 32 && a.sh == 1 && a.sw == 1 && a.OH == a.H && a.OW == a.W && a.ph < a.KH && a.pw < a.KW &&
+           a.x_h_stride == (int64_t)a.W * a.x_w_stride && (a.x_n_stride == (int64_t)a.H * a.x_h_stride || a.M == (int64_t)a.OH * a.OW) &&
+           a.x_w_stride >= a.C16 && (a.KH - 1) * (int64_t)a.W < 8192 && a.C16 <= 8192 &&
+           (int64_t)patch_pixels(a, tile_px) * patch_pitch(a) + 128 + partial_bytes(tile_oc, tile_px / tile_oc, waves) <= kLdsOfUnit;
+}
+
+int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool patch, bool x_unsigned, bool rne, hipStream_t s) {
     // a filter of one tap, inside the image for every pixel, or any filter
     const bool taps = a.KH * a.KW > 1 || a.ph != 0 || a.pw != 0 || (int64_t)(a.OH - 1) * a.sh + a.KH > a.H || (int64_t)(a.OW - 1) * a.sw + a.KW > a.W;
+    const Form form = patch && conv_split_patch_takes(a, tile_oc, tile_px, waves) ? kPatch : taps ? kTaps : kPoint;
     const uint32_t flip = x_unsigned ? 0x80808080u : 0u;
 #define CHX_SPLIT(R, PN, W) \
-    if (tile_oc == R && tile_px == R * PN && waves == W) return launch<R, PN, W>(a, flip, rne, taps, s);
+    if (tile_oc == R && tile_px == R * PN && waves == W) return launch<R, PN, W>(a, flip, rne, form, s);
     CHX_SPLIT(16, 1, 8)
     CHX_SPLIT(16, 1, 16)
     CHX_SPLIT(16, 2, 4)
