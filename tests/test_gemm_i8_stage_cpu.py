@@ -1,0 +1,56 @@
+"""Which kernel an integer product runs on (csrc/gemm_i8.hip), without a GPU: the tiles that tests/test_gpu_gemm_i8_stage.py
+means to reach, and the forms that the staged kernel does not take."""
+import ctypes
+
+import pytest
+
+import host_hip
+
+
+@pytest.fixture(scope="module")
+def host_so(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host_hip"))
+
+
+@pytest.mark.parametrize("case", ["tiles", "other_forms"])
+def test_case(host_so, case):
+    from test_gpu_gemm_i8_stage import SHAPES
+    host_hip.run_case(host_so, __file__, case, SHAPES=repr(SHAPES))
+
+
+def kernel(host, a, b, y):
+    host.clear()
+    host.check(host.lib.chx_hip_matmul_integer(ctypes.byref(a), ctypes.byref(b), None, None, ctypes.byref(y), None))
+    names = host.launches()
+    assert len(names) == 1
+    return names[0]
+
+
+def product(host, M, K, N, transposed=False, a_strides=None, b_strides=None):
+    a, y = host.tensor("uint8", (M, K), a_strides), host.tensor("int32", (M, N))
+    b = host.tensor("int8", (K, N), [1, K] if transposed else b_strides)
+    return kernel(host, a, b, y)
+
+
+def tiles(host):
+    import os
+    for M, K, N, tile, tile_transposed in eval(os.environ["SHAPES"]):
+        for transposed, want in ((False, tile), (True, tile_transposed)):
+            name = product(host, M, K, N, transposed)
+            if want is None:
+                assert "gemm_i8_split_kernel" in name, (M, K, N, name)
+            else:
+                assert "gemm_i8_stage_kernel<%s, %s>" % ("true" if transposed else "false", want) in name, (M, K, N, transposed, name)
+
+
+def other_forms(host):
+    assert "stage" in product(host, 1024, 1024, 4096)
+    assert "stage" in product(host, 1024, 1024, 4096, a_strides=[1100, 1])
+    assert "stage" not in product(host, 1024, 1024, 4096, a_strides=[1 << 24, 1])  # offsets in a tile beyond 32 bits
+    assert "stage" not in product(host, 4096, 4096, 15)  # a row shorter than a read
+    assert "stage" not in product(host, 4096, 176, 4096)  # one stage and a part
+    assert "stage" not in product(host, 32, 512, 512)
+
+
+if __name__ == "__main__":
+    host_hip.main(globals())
