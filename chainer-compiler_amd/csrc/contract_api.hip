@@ -186,6 +186,7 @@ struct PackedWeights {
     int C64 = 0, OCpad = 0, KP = 0;
     int BK = 64;         // K bytes per kernel step; the packed layout depends on it
     bool dense = false;  // taps packed densely; activations go through an explicit im2col
+    int8_t* wf = nullptr;  // of a plan: the weights in the order of the small tiles (inside wp's allocation)
     int8_t* wd = nullptr;  // dense only: the same weights in the order of the planar-input kernel (inside wp's allocation)
 };
 
@@ -727,6 +728,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     a.bk = pw.BK;
     a.nk = pw.KP / pw.BK;
     a.wp = pw.wp;
+    a.wf = pw.wf;
     a.wsum = pw.wsum;
     a.padsum = pw.padsum;
     a.padsum_stride = pw.OCpad;
@@ -824,7 +826,7 @@ int make_packed(const chx_hip_tensor& w, bool persistent, hipStream_t s, PackedW
     const bool stem = pw->dense && stem_shape_fits((int)w.shape[1], (int)w.shape[2], (int)w.shape[3]);
     const size_t stem_bytes =
             stem ? (size_t)(pw->OCpad / 64) * stem_k_blocks((int)w.shape[1], (int)w.shape[2], (int)w.shape[3]) * 2048 : 0;
-    const size_t bytes = mfma_bytes + stem_bytes;
+    const size_t bytes = mfma_bytes + stem_bytes + (persistent ? mfma_bytes : 0);  // (a call's own weights are read once: not worth another pass)
     // the per-channel sums, and behind them the sixteen classes of border sums
     // (between 2 and 32 taps: the kernel's tap masks hold 32, and a single tap that can lie outside is rare enough for
     // the flat-address padding)
@@ -850,8 +852,10 @@ int make_packed(const chx_hip_tensor& w, bool persistent, hipStream_t s, PackedW
     pw->padsum = border_sums ? pw->wsum + pw->OCpad : nullptr;
     pw->wd = stem ? pw->wp + mfma_bytes : nullptr;
     if (stem) CHX_PROPAGATE(pack_weights_stem(w, pw->OCpad, pw->wd, s));
-    if (pw->dense) return pack_weights_dense(w, pw->KP, pw->BK, pw->OCpad, pw->wp, pw->wsum, s);
-    return pack_weights(w, pw->C64, pw->BK, pw->OCpad, pw->wp, pw->wsum, pw->padsum, s);
+    pw->wf = persistent ? pw->wp + mfma_bytes + stem_bytes : nullptr;
+    if (pw->dense) CHX_PROPAGATE(pack_weights_dense(w, pw->KP, pw->BK, pw->OCpad, pw->wp, pw->wsum, s));
+    else CHX_PROPAGATE(pack_weights(w, pw->C64, pw->BK, pw->OCpad, pw->wp, pw->wsum, pw->padsum, s));
+    return pw->wf ? fragment_weights(pw->wp, pw->KP, pw->BK, pw->OCpad, pw->wf, s) : (int)CHX_HIP_OK;
 }
 
 void release_packed(PackedWeights* pw, bool persistent, hipStream_t s) {
@@ -866,6 +870,7 @@ void release_packed(PackedWeights* pw, bool persistent, hipStream_t s) {
     pw->wsum = nullptr;
     pw->padsum = nullptr;
     pw->wd = nullptr;
+    pw->wf = nullptr;
 }
 
 // Depthwise 3x3 on int8 weights with zero weight zero points: packed filter rows and per-channel sums.

@@ -55,6 +55,7 @@ struct ConvMfmaArgs {
     int32_t nk;   // K steps: KP / bk
     int32_t KP;   // packed row length: KH * KW * C64
     const int8_t* wp;     // [OCpad / 64][nk][64][bk]
+    const int8_t* wf;     // the same in the order of the small tiles' fragments (fragment_weights); null: not for those
     const int32_t* wsum;  // [OCpad]
     // [16][OCpad]: the sum of a filter's weights over the taps of its first row (class bit 3), last row (bit 2), first
     // column (bit 1) and last column (bit 0), each tap once: what a pixel whose window leaves the image on those sides
@@ -147,6 +148,8 @@ inline void magic_divisor(uint32_t d, uint32_t* mul, uint32_t* shift) {
 }
 
 int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int32_t* wsum, hipStream_t s);
+// [OCpad / 32][KP / 64][2 halves of 64 k][2 x 16 channels][2 x 16 k][16 channels][16 k]: a step's fragment is 1 KB in one or two places
+int fragment_weights(const int8_t* wp, int KP, int BK, int OCpad, int8_t* wf, hipStream_t s);
 int launch_im2col_dense(const Im2colArgs& a, hipStream_t s);
 int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int32_t* wsum, int32_t* padsum, hipStream_t s);
 // the stem kernel: weights [C][KH][KW] with C*KH <= 32 and KW <= 8; patch = LDS bytes of a tile's input rows
@@ -183,7 +186,7 @@ struct ConvSplitTile {
 };
 constexpr ConvSplitTile kConvSplitTiles[] = {{16, 16, 8}, {16, 16, 16}, {16, 32, 4}, {16, 32, 8}, {16, 32, 16}, {32, 32, 2}, {32, 32, 4}, {32, 32, 8}, {32, 64, 4}, {32, 64, 8}};
 bool conv_split_has(int tile_oc, int tile_px, int waves);
-inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
+inline bool conv_split_takes(const ConvMfmaArgs& a) { return a.wf != nullptr && a.KH * a.KW <= 32; }  // (a mask bit per filter tap)
 // `patch`: several taps over an image whose results have its own size, its pixels from LDS (else, and for what that does not take, from memory)
 constexpr int kConvSplitPatch = 1;  // ... as a launch configuration: in the place of the work-groups per compute unit
 bool conv_split_patch_takes(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves);

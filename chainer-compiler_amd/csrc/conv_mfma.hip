@@ -100,6 +100,16 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
     }
 }
 
+// One thread per 16 bytes of wf.
+__global__ __launch_bounds__(256) void fragment_weights_kernel(const int8_t* __restrict__ wp, int KP, int BK, int64_t chunks, int8_t* __restrict__ wf) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= chunks) return;
+    const int64_t block = i >> 7;  // 32 channels x 64 k
+    const int in = (int)i & 127, half = in >> 6, sixteen = in >> 5 & 1, group = in >> 4 & 1;
+    const int oc = (int)(block / (KP / 64)) * 32 + sixteen * 16 + (in & 15), k = (int)(block % (KP / 64)) * 64 + half * 32 + group * 16;
+    reinterpret_cast<uint4*>(wf)[i] = *reinterpret_cast<const uint4*>(wp + packed_offset(oc, k, KP, BK));
+}
+
 // Few input channels (the 3-channel stem): padding each filter tap to 64 K-bytes would waste
 // most of the matrix-core work, so the taps are packed densely instead.  The weights become
 // [OCpad][Kd] with k = (kh*KW + kw)*C + c, Kd = KH*KW*C rounded up to 64, and the activations
@@ -249,6 +259,12 @@ int pack_weights(
             static_cast<const char*>(w.data), w.strides[0], w.strides[1], w.strides[2], w.strides[3], (int)w.shape[0],
             (int)w.shape[1], (int)w.shape[2], (int)w.shape[3], C64, BK, wp, wsum, padsum);
     return launch_check("pack_weights_kernel");
+}
+
+int fragment_weights(const int8_t* wp, int KP, int BK, int OCpad, int8_t* wf, hipStream_t s) {
+    const int64_t chunks = (int64_t)OCpad * (KP / 16);
+    fragment_weights_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, s>>>(wp, KP, BK, chunks, wf);
+    return launch_check("fragment_weights_kernel");
 }
 
 int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int32_t* wsum, hipStream_t s) {

@@ -8,6 +8,8 @@
 // steps in flight, no barrier until the W partial sums meet in LDS.  Weights are read once per pixel tile and pixels once
 // per channel tile, from L2, so this is for launches bound by latency; which configuration runs is measured per shape
 // (tune_conv_mfma).  ResNet-50 on one image, all 55 launches replayed: 370 us with the staged tiles alone, 308 with these.
+// The weights have a layout of their own (ConvMfmaArgs::wf), in which a step's fragment is in one or two places: from the staged
+// tiles' one ResNet-50 takes 258 us on one image and 372 on eight, from this 240 and 360.
 //
 // Arguments, requantization, residual sums, pairs and storage are those of conv_mfma_kernel; filter taps outside the
 // image are replaced by the zero point on the fragment.
@@ -81,12 +83,12 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
         v4i w, x[kForm == kPatch ? 1 : PN];
     };
     const int steps = a.KP / kStep, per = (steps + W - 1) / W, lo = wave * per, hi = min(steps, lo + per), last = hi - 1;
-    const uint32_t w_off = (uint32_t)(oc >> 6) * (uint32_t)(64 * a.KP) + (uint32_t)((oc & 63) * a.bk + group * 16);
-    const uint32_t bk_shift = a.bk == 128 ? 7 : 6;
+    // (a fragment in one or two places: 8 lines of 128 bytes for a load of 1 KB; in the staged tiles' layout it is 16 or 32)
+    const uint32_t w_off = (uint32_t)(oc >> 5) * (uint32_t)(32 * a.KP) + (uint32_t)((oc & 31) >> 4 << 9) + (uint32_t)((group >> 1 << 10) + ((group & 1) << 8) + (oc & 15) * 16);
     auto load_w = [&](int step, Step& s) {
         // (past the wavefront's last step: that step again, see gemm_i8.hip)
         const uint32_t k = (uint32_t)(min(step, last) * kStep);
-        s.w = *reinterpret_cast<const v4i*>(a.wp + (((k >> bk_shift) * 64u) << bk_shift) + (k & (uint32_t)(a.bk - 1)) + w_off);
+        s.w = *reinterpret_cast<const v4i*>(a.wf + (k * 32 + w_off));
     };
     const int fill = (int)((uint32_t)(a.x_zp & 0xff) * 0x01010101u);
     // The patch: the pixels that the taps of the tile's pixels fall on are one run of the dense image.  (Pixels outside x are
