@@ -1524,6 +1524,63 @@ extern "C" void chx_hip_qconv_plan_destroy(chx_hip_qconv_plan* plan) {
     delete plan;
 }
 
+namespace chx {
+namespace {
+// A ConvInteger with 1x1 filters as the product that it is, on gemm_i8.hip: pixels by filters where x and y are channels-last and
+// dense, filters by pixels for every image where both are planar (one zero point for all filters: there it is that of the
+// rows).  EUNSUPPORTED, with nothing launched, for anything else.  The other kernels bring channels-last pixels into planes
+// first and keep strips of few filters; us there and here: 5 x 80 -> 24 channels at 11x11, channels-last 9.0 and 6.2, 36 x 96 -> 56 at
+// 32x32 17.2 and 7.5; planar 37 x 48 -> 224 at 16x16 11.4 and 6.4, 56 x 168 -> 32 at 39x39 28.9 and 9.3, with few of both the same (3 x
+// 48 -> 24 at 55x55 6.3 and 6.3).  Of sixty such layers one was slower (42 x 184 -> 40 at 23x23, planar: 9.5 and 10.4).
+int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_t x_zero_point, const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, const chx_hip_tensor& y, hipStream_t s) {
+    if (cs.KH != 1 || cs.KW != 1 || p.group != 1 || p.stride_h != 1 || p.stride_w != 1 || cs.OH != cs.H || cs.OW != cs.W || p.pad_h_begin != 0 || p.pad_w_begin != 0) return CHX_HIP_EUNSUPPORTED;
+    const int64_t C = x.shape[1], OC = cs.OC, HW = (int64_t)cs.OH * cs.OW;
+    if ((C != 1 && w.strides[1] != 1) || a.total == 0) return CHX_HIP_EUNSUPPORTED;
+    MatMulDirectArgs m;
+    memset(&m, 0, sizeof(m));
+    int64_t x_px = 0, y_px = 0;
+    m.y = static_cast<char*>(y.data);
+    m.total = a.total;
+    m.K = C;
+    if (y_is_pixel_major(x, &x_px) && y_is_pixel_major(y, &y_px)) {
+        m.a = static_cast<const char*>(x.data);
+        m.b = static_cast<const char*>(w.data);
+        m.M = cs.N * HW;
+        m.N = OC;
+        m.a_row = x_px; m.a_col = 1;
+        m.b_row = 1; m.b_col = w.strides[0];
+        m.y_row = y_px; m.y_col = 4;
+        m.a_signed = x.dtype == CHX_HIP_INT8;
+        m.b_signed = w.dtype == CHX_HIP_INT8;
+        m.a_zp_imm = x_zero_point;
+        m.b_zp = a.w_zp;
+        m.b_zp_len = a.w_zp_len;
+        m.b_zp_stride = a.w_zp_stride;
+        m.b_zp_signed = m.b_signed;
+        return launch_matmul_i8(m, false, s);
+    }
+    const bool planar = (cs.OW == 1 || (x.strides[3] == 1 && y.strides[3] == 4)) && (cs.OH == 1 || (x.strides[2] == x.shape[3] && y.strides[2] == 4 * x.shape[3]));
+    if (planar && a.w_zp_len <= 1) {
+        m.a = static_cast<const char*>(w.data);
+        m.b = static_cast<const char*>(x.data);
+        m.M = OC;
+        m.N = HW;
+        m.a_row = w.strides[0]; m.a_col = 1;
+        m.b_batch = x.strides[0]; m.b_row = x.strides[1]; m.b_col = 1;
+        m.y_batch = y.strides[0]; m.y_row = y.strides[1]; m.y_col = 4;
+        m.a_signed = w.dtype == CHX_HIP_INT8;
+        m.b_signed = x.dtype == CHX_HIP_INT8;
+        m.a_zp = a.w_zp;
+        m.a_zp_len = a.w_zp_len;
+        m.a_zp_signed = m.a_signed;
+        m.b_zp_imm = x_zero_point;
+        return launch_matmul_i8(m, false, s);
+    }
+    return CHX_HIP_EUNSUPPORTED;
+}
+}  // namespace
+}  // namespace chx
+
 extern "C" int chx_hip_conv_integer(
         const chx_hip_tensor* x, const chx_hip_tensor* w, int32_t x_zero_point, const chx_hip_tensor* w_zero_point,
         const chx_hip_conv_params* params, chx_hip_tensor* y, void* stream) {
@@ -1547,6 +1604,10 @@ extern "C" int chx_hip_conv_integer(
         a.w_zp_stride = stride;
     }
     hipStream_t s = as_stream(stream);
+    {
+        const int rc = run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, s);
+        if (rc != CHX_HIP_EUNSUPPORTED) return rc;
+    }
     // (a recorded run takes the kernel without scratch memory: the weights of this entry point arrive with the call)
     const bool capturing = stream_is_capturing(s);
     // The packed kernel multiplies faster but costs some 70 us of host time per call (read-back of the zero points,

@@ -1,0 +1,51 @@
+"""Which ConvInteger calls are products (csrc/contract_api.hip, run_conv_as_product), without a GPU."""
+import ctypes
+
+import pytest
+
+import host_hip
+
+
+@pytest.fixture(scope="module")
+def host_so(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host_hip"))
+
+
+@pytest.mark.parametrize("case", ["products", "other_forms"])
+def test_case(host_so, case):
+    host_hip.run_case(host_so, __file__, case)
+
+
+def is_product(host, n=3, c=40, h=9, w=7, oc=24, k=1, strides=(1, 1), pads=(0, 0), group=1, channels_last=False, pitch=None, y_channels_last=None, zero_points=0, w_strides=None):
+    oh, ow = (h + 2 * pads[0] - k) // strides[0] + 1, (w + 2 * pads[1] - k) // strides[1] + 1
+    x = host.channels_last("uint8", (n, c, h, w), pitch) if channels_last else host.tensor("uint8", (n, c, h, w), pitch and [c * h * pitch, h * pitch, pitch, 1])
+    y = (host.channels_last if (channels_last if y_channels_last is None else y_channels_last) else host.tensor)("int32", (n, oc, oh, ow))
+    f = host.tensor("int8", (oc, c // group, k, k), w_strides)
+    zp = host.tensor("int8", (zero_points,)) if zero_points else None
+    params = host.capi.conv_params(strides, pads, pads, group)
+    host.clear()
+    host.check(host.lib.chx_hip_conv_integer(ctypes.byref(x), ctypes.byref(f), 5, ctypes.byref(zp) if zp else None, ctypes.byref(params), ctypes.byref(y), None))
+    return any("gemm_i8" in name for name in host.launches())
+
+
+def products(host):
+    for channels_last in (False, True):
+        assert is_product(host, channels_last=channels_last)
+        assert is_product(host, channels_last=channels_last, zero_points=1)
+        assert is_product(host, channels_last=channels_last, h=1, w=1)
+        assert is_product(host, channels_last=channels_last, n=1, w=1)
+    assert is_product(host, channels_last=True, zero_points=24) and not is_product(host, zero_points=24)
+    assert is_product(host, channels_last=True, pitch=57)
+    assert is_product(host, n=64, c=200, h=56, w=56, oc=200) and is_product(host, n=64, c=200, h=56, w=56, oc=200, channels_last=True)
+
+
+def other_forms(host):
+    assert not is_product(host, k=3, pads=(1, 1)) and not is_product(host, strides=(2, 2), channels_last=True) and not is_product(host, pads=(1, 1))
+    assert not is_product(host, group=2) and not is_product(host, c=15)
+    assert not is_product(host, pitch=9)  # rows apart
+    assert not is_product(host, channels_last=True, y_channels_last=False) and not is_product(host, y_channels_last=True)
+    assert not is_product(host, w_strides=[1, 24, 1, 1])  # filters across
+
+
+if __name__ == "__main__":
+    host_hip.main(globals())
