@@ -1527,13 +1527,16 @@ extern "C" void chx_hip_qconv_plan_destroy(chx_hip_qconv_plan* plan) {
 namespace chx {
 namespace {
 // A ConvInteger with 1x1 filters as the product that it is, on gemm_i8.hip: pixels by filters where x and y are channels-last and
-// dense, filters by pixels for every image where both are planar (one zero point for all filters: there it is that of the
+// dense (with strides above 1 a product for every row of results), filters by pixels for every image where both are planar (one zero point for all filters: there it is that of the
 // rows).  EUNSUPPORTED, with nothing launched, for anything else.  The other kernels bring channels-last pixels into planes
 // first and keep strips of few filters; us there and here: 5 x 80 -> 24 channels at 11x11, channels-last 9.0 and 6.2, 36 x 96 -> 56 at
 // 32x32 17.2 and 7.5; planar 37 x 48 -> 224 at 16x16 11.4 and 6.4, 56 x 168 -> 32 at 39x39 28.9 and 9.3, with few of both the same (3 x
 // 48 -> 24 at 55x55 6.3 and 6.3).  Of sixty such layers one was slower (42 x 184 -> 40 at 23x23, planar: 9.5 and 10.4).
+// Stride 2, channels-last: 9 x 48 -> 40 at 8x8 8.8 and 6.3, 40 x 40 -> 152 at 24x24 9.7 and 6.4, 37 x 64 -> 128 at 46x46 16.5 and 16.9.
 int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_t x_zero_point, const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, const chx_hip_tensor& y, hipStream_t s) {
-    if (cs.KH != 1 || cs.KW != 1 || p.group != 1 || p.stride_h != 1 || p.stride_w != 1 || cs.OH != cs.H || cs.OW != cs.W || p.pad_h_begin != 0 || p.pad_w_begin != 0) return CHX_HIP_EUNSUPPORTED;
+    // (pads at the ends with stride 1 would show in OH and OW; with larger strides the last window has to lie inside)
+    if (cs.KH != 1 || cs.KW != 1 || p.group != 1 || p.pad_h_begin != 0 || p.pad_w_begin != 0 || (cs.OH - 1) * p.stride_h >= cs.H || (cs.OW - 1) * p.stride_w >= cs.W) return CHX_HIP_EUNSUPPORTED;
+    const bool dense = p.stride_h == 1 && p.stride_w == 1;
     const int64_t C = x.shape[1], OC = cs.OC, HW = (int64_t)cs.OH * cs.OW;
     if ((C != 1 && w.strides[1] != 1) || a.total == 0) return CHX_HIP_EUNSUPPORTED;
     MatMulDirectArgs m;
@@ -1548,6 +1551,13 @@ int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_
         m.M = cs.N * HW;
         m.N = OC;
         m.a_row = x_px; m.a_col = 1;
+        if (!dense) {  // a product for every row of results, whose first pixels have to be equally far apart
+            if (cs.N > 1 && cs.H != cs.OH * p.stride_h) return CHX_HIP_EUNSUPPORTED;
+            m.M = cs.OW;
+            m.a_row = p.stride_w * x_px;
+            m.a_batch = (int64_t)p.stride_h * cs.W * x_px;
+            m.y_batch = cs.OW * y_px;
+        }
         m.b_row = 1; m.b_col = w.strides[0];
         m.y_row = y_px; m.y_col = 4;
         m.a_signed = x.dtype == CHX_HIP_INT8;
@@ -1559,7 +1569,7 @@ int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_
         m.b_zp_signed = m.b_signed;
         return launch_matmul_i8(m, false, s);
     }
-    const bool planar = (cs.OW == 1 || (x.strides[3] == 1 && y.strides[3] == 4)) && (cs.OH == 1 || (x.strides[2] == x.shape[3] && y.strides[2] == 4 * x.shape[3]));
+    const bool planar = dense && (cs.OW == 1 || (x.strides[3] == 1 && y.strides[3] == 4)) && (cs.OH == 1 || (x.strides[2] == x.shape[3] && y.strides[2] == 4 * x.shape[3]));
     if (planar && a.w_zp_len <= 1) {
         m.a = static_cast<const char*>(w.data);
         m.b = static_cast<const char*>(x.data);

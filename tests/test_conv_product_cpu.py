@@ -36,11 +36,14 @@ def products(host):
         assert is_product(host, channels_last=channels_last, n=1, w=1)
     assert is_product(host, channels_last=True, zero_points=24) and not is_product(host, zero_points=24)
     assert is_product(host, channels_last=True, pitch=57)
+    # strides: rows of results equally far apart, or one image
+    assert is_product(host, strides=(2, 2), channels_last=True, h=8) and is_product(host, strides=(2, 1), channels_last=True, h=8) and is_product(host, strides=(1, 3), channels_last=True)
+    assert is_product(host, strides=(2, 2), channels_last=True, n=1) and not is_product(host, strides=(2, 2), channels_last=True, h=9) and not is_product(host, strides=(2, 2))
     assert is_product(host, n=64, c=200, h=56, w=56, oc=200) and is_product(host, n=64, c=200, h=56, w=56, oc=200, channels_last=True)
 
 
 def other_forms(host):
-    assert not is_product(host, k=3, pads=(1, 1)) and not is_product(host, strides=(2, 2), channels_last=True) and not is_product(host, pads=(1, 1))
+    assert not is_product(host, k=3, pads=(1, 1)) and not is_product(host, pads=(1, 1)) and not is_product(host, pads=(1, 1), channels_last=True)
     assert not is_product(host, group=2) and not is_product(host, c=15)
     assert not is_product(host, pitch=9)  # rows apart
     assert not is_product(host, channels_last=True, y_channels_last=False) and not is_product(host, y_channels_last=True)

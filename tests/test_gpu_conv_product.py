@@ -48,8 +48,10 @@ def test_layouts(g, N, C, H, W, OC, dts):
 
 def test_other_geometries(g, oracle):
     rng = np.random.default_rng(1)
-    x, w = codes(rng, (2, 32, 9, 8), np.uint8), codes(rng, (24, 32, 1, 1), np.int8)
-    for strides, pads in [((2, 2), (0, 0)), ((1, 2), (0, 0)), ((1, 1), (1, 1))]:
-        want = oracle.conv_integer(x, w, 5, np.zeros(24, np.int8), strides=strides, pads=pads)
-        for xd in (g.dev(x), g.to_channels_last(g.dev(x))):
-            np.testing.assert_array_equal(g.host(g.ops.ConvInteger(xd, g.dev(w), 5, None, strides=strides, pads=pads)), want)
+    w = codes(rng, (24, 32, 1, 1), np.int8)
+    for N, H, W in [(2, 9, 8), (3, 8, 7), (1, 7, 5)]:
+        x = codes(rng, (N, 32, H, W), np.uint8)
+        for strides, pads in [((2, 2), (0, 0)), ((1, 2), (0, 0)), ((2, 1), (0, 0)), ((3, 3), (0, 0)), ((1, 1), (1, 1))]:
+            want = oracle.conv_integer(x, w, 5, np.zeros(24, np.int8), strides=strides, pads=pads)
+            for xd in layouts(g, x):
+                np.testing.assert_array_equal(g.host(g.ops.ConvInteger(xd, g.dev(w), 5, None, strides=strides, pads=pads)), want)
