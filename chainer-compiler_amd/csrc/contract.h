@@ -47,6 +47,7 @@ struct MatMulDirectArgs {
     int32_t a_zp_signed, b_zp_signed;
     int32_t a_zp_imm, b_zp_imm;  // host-side scalar zero points, subtracted as well
     int32_t requant;
+    int32_t lds_64k;  // no kernel with more than 64 KB of LDS
     float b_scale;
     const int32_t* bias;
     RequantParams rq;

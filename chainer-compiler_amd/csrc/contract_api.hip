@@ -1545,6 +1545,7 @@ int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_
     m.y = static_cast<char*>(y.data);
     m.total = a.total;
     m.K = C;
+    m.lds_64k = 1;  // (a ConvInteger asks for no more than any launch may: the split kernel only)
     if (y_is_pixel_major(x, &x_px) && y_is_pixel_major(y, &y_px)) {
         m.a = static_cast<const char*>(x.data);
         m.b = static_cast<const char*>(w.data);

@@ -694,7 +694,7 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
     // than three steps for a wavefront, which the split kernel has in flight at once, none).  A row's 16 bytes are read in one
     // place, offsets in a tile are 32 bits wide, and one stage is no loop.  (Below 2^26 products the start is the time on either.)
     const int64_t steps_each = (steps + w - 1) / w;
-    if (steps_each > 2 && m.N >= 16 && m.K >= 192 && (double)(m.M * m.N) * (double)(m.K * batch) >= 0x1p26 && m.a_row >= 0 && m.a_row < (int64_t(1) << 24) && b_ld < (int64_t(1) << 24)) {
+    if (!m.lds_64k && steps_each > 2 && m.N >= 16 && m.K >= 192 && (double)(m.M * m.N) * (double)(m.K * batch) >= 0x1p26 && m.a_row >= 0 && m.a_row < (int64_t(1) << 24) && b_ld < (int64_t(1) << 24)) {
         const bool a_odd = m.K % 4 != 0, b_odd = m.N % 4 != 0;
         const int64_t along_m[3] = {128, 64, 64}, along_n[3] = {128, 128, 64};
         double least = 0.9 * split_time(kSplitCosts[b_transposed], (double)steps_each, (double)(work_groups * w) / 1024.0, a_odd, b_odd,

@@ -25,6 +25,7 @@ def is_product(host, n=3, c=40, h=9, w=7, oc=24, k=1, strides=(1, 1), pads=(0, 0
     params = host.capi.conv_params(strides, pads, pads, group)
     host.clear()
     host.check(host.lib.chx_hip_conv_integer(ctypes.byref(x), ctypes.byref(f), 5, ctypes.byref(zp) if zp else None, ctypes.byref(params), ctypes.byref(y), None))
+    assert not any("gemm_i8_stage" in name for name in host.launches())  # (more than 64 KB of LDS)
     return any("gemm_i8" in name for name in host.launches())
 
 
