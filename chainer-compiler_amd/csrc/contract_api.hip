@@ -1615,15 +1615,22 @@ extern "C" int chx_hip_conv_integer(
         a.w_zp_stride = stride;
     }
     hipStream_t s = as_stream(stream);
-    {
-        const int rc = run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, s);
-        if (rc != CHX_HIP_EUNSUPPORTED) return rc;
-    }
-    // (a recorded run takes the kernel without scratch memory: the weights of this entry point arrive with the call)
+    // (a recorded run takes a kernel without scratch memory: the weights of this entry point arrive with the call)
     const bool capturing = stream_is_capturing(s);
     // The packed kernel multiplies faster but costs some 70 us of host time per call (read-back of the zero points,
     // allocations, packing): the two meet at 8 G multiply-adds, and it takes channels-last results only.
-    const bool packed = weights_fit_mfma(*w, params->group) && (double)a.total * cs.Cg * cs.KH * cs.KW >= 0x1p33 && x_is_mfma_ready(*x);
+    const double macs = (double)a.total * cs.Cg * cs.KH * cs.KW;
+    const bool packed = weights_fit_mfma(*w, params->group) && macs >= 0x1p33 && x_is_mfma_ready(*x);
+    // A product (1x1 filters) needs none of that and meets it later, the later the fewer channels there are to multiply for each
+    // result: us packed and as a product, 256 channels 266 and 212 at 39 G, 329 and 277 at 53 G, 384 109 and 121 at 20 G and 208 and 232 at 39 G, 512 83 and 75 at 11 G
+    // and 97 and 108 at 20 G, 1024 79 and 72 at 10 G, between 77 and 72 and 88 and 93 at 13 G and 117 and 192 at 39 G, 2048 212 and 498 at 79 G.  With few pixels to a filter
+    // its packing is what counts (64 images of 7x7, 2048 -> 3072: 145 and 101).
+    const bool product_first = cs.KH * cs.KW == 1 && (capturing || !packed || macs < 14e9 || macs * cs.Cg < 0x1p43 || cs.Cg < 320 || (int64_t)cs.N * cs.OH * cs.OW < 8192);
+    auto product = [&]() { return run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, s); };
+    if (product_first) {
+        const int rc = product();
+        if (rc != CHX_HIP_EUNSUPPORTED) return rc;
+    }
     if (!capturing && !packed) {
         int rc = run_conv_strip(a, s);
         if (rc == CHX_HIP_EUNSUPPORTED) rc = run_conv_planar(a, s);
@@ -1653,6 +1660,8 @@ extern "C" int chx_hip_conv_integer(
             if (rc != CHX_HIP_EUNSUPPORTED) return rc;
         }
     }
+    const int rc = product();  // (zero points of the filters that are not 0)
+    if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     return launch_conv_direct(a, false, s);
 }
 

@@ -11,7 +11,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["products", "other_forms"])
+@pytest.mark.parametrize("case", ["products", "other_forms", "packed_weights"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -49,6 +49,33 @@ def other_forms(host):
     assert not is_product(host, pitch=9)  # rows apart
     assert not is_product(host, channels_last=True, y_channels_last=False) and not is_product(host, y_channels_last=True)
     assert not is_product(host, w_strides=[1, 24, 1, 1])  # filters across
+
+
+def packed_weights(host):
+    """Large channels-last layers multiply on the packed kernel, which reads the filters' zero points back and packs them on every
+    call; where a product is faster, in a recording, and with zero points that are not 0 they are a product."""
+    def kernels(n, c, hw, oc, zero_point=0, stride=1, stream=None):
+        o = (hw - 1) // stride + 1
+        x, y = host.channels_last("uint8", (n, c, hw, hw)), host.channels_last("int32", (n, oc, o, o))
+        f, zp = host.tensor("int8", (oc, c, 1, 1)), host.tensor("int8", ())
+        host.bytes(zp.data, bytes([zero_point]))
+        params = host.capi.conv_params((stride, stride), (0, 0), (0, 0), 1)
+        host.clear()
+        host.check(host.lib.chx_hip_conv_integer(ctypes.byref(x), ctypes.byref(f), 5, ctypes.byref(zp), ctypes.byref(params), ctypes.byref(y), stream))
+        for a in (x, y, f):
+            host.check(host.lib.chx_hip_free(ctypes.c_void_p(a.data)))
+        return ["packed" if "conv_mfma" in k else "product" if "gemm_i8" in k else "other" for k in host.launches() if "pack_weights" not in k]
+
+    assert kernels(64, 1024, 28, 1024) == ["packed"] and kernels(64, 512, 56, 512) == ["packed"]
+    assert kernels(64, 1024, 28, 1024, zero_point=3) == ["product"]
+    assert kernels(32, 1024, 56, 1024, stride=2) == ["packed"]
+    assert kernels(64, 256, 56, 384) == ["product"] and kernels(64, 512, 28, 320) == ["product"]  # (few channels, 8 G multiply-adds)
+    assert kernels(64, 1024, 14, 1024) == ["product"] and kernels(32, 256, 112, 512) == ["product"]
+    assert kernels(64, 2048, 7, 3072) == ["product"]  # 3136 pixels, 6 MB of filters
+    s, graph = host.stream(), ctypes.c_void_p()
+    host.check(host.lib.chx_hip_capture_begin(s))
+    assert kernels(64, 1024, 28, 1024, stream=s) == ["product"]
+    host.check(host.lib.chx_hip_capture_end(s, ctypes.byref(graph)))
 
 
 if __name__ == "__main__":

@@ -55,3 +55,15 @@ def test_other_geometries(g, oracle):
             want = oracle.conv_integer(x, w, 5, np.zeros(24, np.int8), strides=strides, pads=pads)
             for xd in layouts(g, x):
                 np.testing.assert_array_equal(g.host(g.ops.ConvInteger(xd, g.dev(w), 5, None, strides=strides, pads=pads)), want)
+
+
+# 15 G multiply-adds: the packed kernel; with zero points of the filters that are not 0, and at 13 G, the product
+@pytest.mark.parametrize("OC", [1160, 1024])
+@pytest.mark.parametrize("wz", [0, 3])
+def test_large_layers(g, OC, wz):
+    rng = np.random.default_rng(OC + wz)
+    x, w = codes(rng, (64, 14, 14, 1024), np.uint8), codes(rng, (OC, 1024, 1, 1), np.int8)
+    got = g.host(g.ops.ConvInteger(g.dev(x).permute(0, 3, 1, 2), g.dev(w), 5, g.dev(np.asarray(wz, np.int8)))).transpose(0, 2, 3, 1).reshape(-1, OC)
+    pixels = sorted({0, 1, 127, 128, len(got) // 2, len(got) - 129, len(got) - 1} | set(range(77, len(got), 997)))
+    want = (x.reshape(-1, 1024)[pixels].astype(np.float64) - 5) @ (w[:, :, 0, 0].astype(np.float64) - wz).T  # (exact: below 2^53)
+    np.testing.assert_array_equal(got[pixels], want.astype(np.int32))
