@@ -60,6 +60,7 @@ int launch_matmul_direct(const MatMulDirectArgs& a, bool rne, hipStream_t s);
 int run_conv_planar(const ConvDirectArgs& a, hipStream_t s);
 // The same in one launch for convolutions whose strips of input fit LDS (conv_strip.hip).
 int run_conv_strip(const ConvDirectArgs& a, hipStream_t s);
+bool conv_strip_takes(const ConvDirectArgs& a);
 // The same product on the matrix cores (gemm_i8.hip); EUNSUPPORTED, with nothing launched, for layouts it does not take.
 int launch_matmul_i8(const MatMulDirectArgs& a, bool rne, hipStream_t s);
 

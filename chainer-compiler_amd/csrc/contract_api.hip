@@ -1526,14 +1526,38 @@ extern "C" void chx_hip_qconv_plan_destroy(chx_hip_qconv_plan* plan) {
 
 namespace chx {
 namespace {
+// Whether a ConvInteger with 1x1 filters that could be a product is one of those for which another kernel is faster, as far as
+// that kernel takes it.  Measured on 1,380 calls drawn from 8 to 2048 channels in and out, images of 4 to 112, 2^23 to 2^36
+// multiply-adds, in us, there and as a product:
+//  * planar, fewer columns than three quarters of a tile of 128 and enough tiles that this counts (in steps of 32 channels): 51 x 216
+//    -> 1336 channels at 7x7 15.8 and 21.4, 64 x 512 -> 2048 30.6 and 43.3; few tiles (8 x 1016 -> 664) 13.3 and 10.7, 11x11 19.8 and 8.5;
+//  * planar, few channels in, many results, rows that do not start at lines of 128 bytes, whose parts two tiles then write: 246 x
+//    32 -> 200 at 35x35 55.7 and 87.4, 10 x 32 -> 728 at 97x97 55.4 and 93.2; at 56x56 (whole lines) 84.4 and 54.9 for 230 x 32 -> 104;
+//  * channels-last with strides, fewer filters than 0.3 of the channels and one launch (conv_strip.hip): 21 x 176 -> 16 at 34x34 8.7 and 11.5, 55 x 672 -> 80
+//    at 5x5 11.2 and 19.2; more filters (10 x 136 -> 320 at 24x24, 11.6 and 8.4) gain by the product, by 14 % on average;
+//  * channels-last with strides and rows of no more than half a tile of 16, by what the two kernels' work comes to: 64 x 1024 -> 2048
+//    at 7x7 84 and 130, 62 x 544 -> 1312 at 4x4 22.1 and 32.6; 135 x 552 -> 304 at 7x7 61.3 and 27.6.
+bool faster_than_product(const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, bool channels_last) {
+    const int64_t C = a.C, OC = cs.OC, columns = (int64_t)cs.OH * cs.OW;
+    if (!channels_last) {
+        if (columns <= 96) return (int64_t)cs.N * ((OC + 31) / 32) * ((C + 31) / 32) > 9000;
+        return C <= 112 && OC >= 200 && columns % 32 != 0 && (int64_t)a.total > 16000000;
+    }
+    if ((p.stride_h == 1 && p.stride_w == 1) || p.stride_h != p.stride_w || p.stride_h > 2) return false;
+    if (conv_strip_takes(a)) return 10 * OC <= 3 * C;
+    if (cs.OW > 8) return false;
+    const double steps = (double)cs.N * cs.OH * ((OC + 63) / 64) * ((C + 63) / 64);
+    const double planes = 12.0 + 2.5e-6 * (double)cs.N * (double)C * (double)cs.H * (double)cs.W + 4e-9 * (double)a.total * (double)C + 2e-6 * (double)a.total;
+    return planes < 0.9 * (7.0 + 0.45e-3 * steps);
+}
+
 // A ConvInteger with 1x1 filters as the product that it is, on gemm_i8.hip: pixels by filters where x and y are channels-last and
 // dense (with strides above 1 a product for every row of results), filters by pixels for every image where both are planar (one zero point for all filters: there it is that of the
-// rows).  EUNSUPPORTED, with nothing launched, for anything else.  The other kernels bring channels-last pixels into planes
+// rows).  EUNSUPPORTED, with nothing launched, for anything else and, unless `any`, for what faster_than_product() names.  The other kernels bring channels-last pixels into planes
 // first and keep strips of few filters; us there and here: 5 x 80 -> 24 channels at 11x11, channels-last 9.0 and 6.2, 36 x 96 -> 56 at
 // 32x32 17.2 and 7.5; planar 37 x 48 -> 224 at 16x16 11.4 and 6.4, 56 x 168 -> 32 at 39x39 28.9 and 9.3, with few of both the same (3 x
-// 48 -> 24 at 55x55 6.3 and 6.3).  Of sixty such layers one was slower (42 x 184 -> 40 at 23x23, planar: 9.5 and 10.4).
-// Stride 2, channels-last: 9 x 48 -> 40 at 8x8 8.8 and 6.3, 40 x 40 -> 152 at 24x24 9.7 and 6.4, 37 x 64 -> 128 at 46x46 16.5 and 16.9.
-int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_t x_zero_point, const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, const chx_hip_tensor& y, hipStream_t s) {
+// 48 -> 24 at 55x55 6.3 and 6.3).  Stride 2, channels-last: 9 x 48 -> 40 at 8x8 8.8 and 6.3, 40 x 40 -> 152 at 24x24 9.7 and 6.4.
+int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_t x_zero_point, const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, const chx_hip_tensor& y, bool any, hipStream_t s) {
     // (pads at the ends with stride 1 would show in OH and OW; with larger strides the last window has to lie inside)
     if (cs.KH != 1 || cs.KW != 1 || p.group != 1 || p.pad_h_begin != 0 || p.pad_w_begin != 0 || (cs.OH - 1) * p.stride_h >= cs.H || (cs.OW - 1) * p.stride_w >= cs.W) return CHX_HIP_EUNSUPPORTED;
     const bool dense = p.stride_h == 1 && p.stride_w == 1;
@@ -1547,6 +1571,7 @@ int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_
     m.K = C;
     m.lds_64k = 1;  // (a ConvInteger asks for no more than any launch may: the split kernel only)
     if (y_is_pixel_major(x, &x_px) && y_is_pixel_major(y, &y_px)) {
+        if (!any && faster_than_product(p, cs, a, true)) return CHX_HIP_EUNSUPPORTED;
         m.a = static_cast<const char*>(x.data);
         m.b = static_cast<const char*>(w.data);
         m.M = cs.N * HW;
@@ -1572,6 +1597,7 @@ int run_conv_as_product(const chx_hip_tensor& x, const chx_hip_tensor& w, int32_
     }
     const bool planar = dense && (cs.OW == 1 || (x.strides[3] == 1 && y.strides[3] == 4)) && (cs.OH == 1 || (x.strides[2] == x.shape[3] && y.strides[2] == 4 * x.shape[3]));
     if (planar && a.w_zp_len <= 1) {
+        if (!any && faster_than_product(p, cs, a, false)) return CHX_HIP_EUNSUPPORTED;
         m.a = static_cast<const char*>(w.data);
         m.b = static_cast<const char*>(x.data);
         m.M = OC;
@@ -1624,16 +1650,18 @@ extern "C" int chx_hip_conv_integer(
     // A product (1x1 filters) needs none of that and meets it later, the later the fewer channels there are to multiply for each
     // result: us packed and as a product, 256 channels 266 and 212 at 39 G, 329 and 277 at 53 G, 384 109 and 121 at 20 G and 208 and 232 at 39 G, 512 83 and 75 at 11 G
     // and 97 and 108 at 20 G, 1024 79 and 72 at 10 G, between 77 and 72 and 88 and 93 at 13 G and 117 and 192 at 39 G, 2048 212 and 498 at 79 G.  With few pixels to a filter
-    // its packing is what counts (64 images of 7x7, 2048 -> 3072: 145 and 101).
-    const bool product_first = cs.KH * cs.KW == 1 && (capturing || !packed || macs < 14e9 || macs * cs.Cg < 0x1p43 || cs.Cg < 320 || (int64_t)cs.N * cs.OH * cs.OW < 8192);
-    auto product = [&]() { return run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, s); };
+    // its packing is what counts (64 images of 7x7, 2048 -> 3072: 145 and 101); with strides the product's tiles are rows of results (138 x 2000 -> 376 at
+    // 11x11, 12.6 G: 75 and 162).
+    const bool product_first = cs.KH * cs.KW == 1 && (capturing || !packed || macs < (params->stride_w == 1 ? 14e9 : 0x1p33) || macs * cs.Cg < 0x1p43 || cs.Cg < 320 || (int64_t)cs.N * cs.OH * cs.OW < 8192);
+    auto product = [&](bool any) { return run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, any, s); };
     if (product_first) {
-        const int rc = product();
+        const int rc = product(capturing);
         if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     }
     if (!capturing && !packed) {
         int rc = run_conv_strip(a, s);
         if (rc == CHX_HIP_EUNSUPPORTED) rc = run_conv_planar(a, s);
+        if (rc == CHX_HIP_EUNSUPPORTED) rc = product(true);
         if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     }
     if (weights_fit_mfma(*w, params->group) && !capturing) {
@@ -1660,7 +1688,7 @@ extern "C" int chx_hip_conv_integer(
             if (rc != CHX_HIP_EUNSUPPORTED) return rc;
         }
     }
-    const int rc = product();  // (zero points of the filters that are not 0)
+    const int rc = product(true);  // (zero points of the filters that are not 0)
     if (rc != CHX_HIP_EUNSUPPORTED) return rc;
     return launch_conv_direct(a, false, s);
 }

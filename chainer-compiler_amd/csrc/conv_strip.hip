@@ -296,22 +296,20 @@ void launch(const StripArgs& g, size_t bytes, hipStream_t s) {
     else conv_strip_kernel<S, KW, kChannelsLast, 1><<<dim3(strips, 1), 64 * kWaves, bytes, s>>>(g);
 }
 
-}  // namespace
-
-int run_conv_strip(const ConvDirectArgs& d, hipStream_t s) {
-    if (d.total == 0) return CHX_HIP_OK;
+// The strips of a call that the kernel takes, its LDS bytes, and whether x is read along its rows; false for any other call.
+bool cut_strips(const ConvDirectArgs& d, StripArgs* strips, int64_t* lds, bool* along_rows) {
     const int64_t K = (int64_t)d.Cg * d.KH * d.KW;
     const bool w_dense = (d.KW == 1 || d.ws[3] == 1) && (d.KH == 1 || d.ws[2] == d.KW) && (d.Cg == 1 || d.ws[1] == d.KH * d.KW);
-    if (d.requant || d.D != 1 || d.KD != 1 || d.OD != 1 || !w_dense || K < 16 || d.group != 1) return CHX_HIP_EUNSUPPORTED;
-    if (d.sh != d.sw || d.sh > 2 || (d.KW != 1 && d.KW != 3)) return CHX_HIP_EUNSUPPORTED;
-    if (d.x_signed ? (d.x_zp < -128 || d.x_zp > 127) : (d.x_zp < 0 || d.x_zp > 255)) return CHX_HIP_EUNSUPPORTED;
+    if (d.requant || d.D != 1 || d.KD != 1 || d.OD != 1 || !w_dense || K < 16 || d.group != 1) return false;
+    if (d.sh != d.sw || d.sh > 2 || (d.KW != 1 && d.KW != 3)) return false;
+    if (d.x_signed ? (d.x_zp < -128 || d.x_zp > 127) : (d.x_zp < 0 || d.x_zp > 255)) return false;
     const bool channels_last = d.xs[1] == 1 && d.C > 1 && d.C % 4 == 0, planar = d.xs[3] == 1 && d.W >= 8;
-    if (!channels_last && !planar) return CHX_HIP_EUNSUPPORTED;
-    StripArgs g;
+    if (!channels_last && !planar) return false;
+    StripArgs& g = *strips;
     memset(&g, 0, sizeof(g));
     // a strip is as many rows as the 32 lanes of a tile have groups of four columns for
     g.G = (d.OW + 3) / 4;
-    if (g.G > 32 || d.KH > 64) return CHX_HIP_EUNSUPPORTED;
+    if (g.G > 32 || d.KH > 64) return false;
     g.TR = 32 / g.G < d.OH ? 32 / g.G : d.OH;
     g.RI = (g.TR - 1) * d.sh + d.KH;
     g.strips = (d.OH + g.TR - 1) / g.TR;
@@ -323,8 +321,28 @@ int run_conv_strip(const ConvDirectArgs& d, hipStream_t s) {
     // another on a compute unit it is filled once too often ([8, 64, 56, 56] with 256 1x1, 896 of them: 20.0 / 12.2).
     // Channels-last arrays cost more to bring in: not for a few work-groups (28 of them: 10.6 / 9.4).
     // Beside a long table (1024 channels of 3x3: 36 KB) a strip of that size would pass the 64 KB that any launch may ask for.
-    if (strip > 48 * 1024 || bytes > 64 * 1024 || work_groups > 512 || (!planar && work_groups < 64)) return CHX_HIP_EUNSUPPORTED;
+    if (strip > 48 * 1024 || bytes > 64 * 1024 || work_groups > 512 || (!planar && work_groups < 64)) return false;
     g.table_at = (int32_t)strip;
+    *lds = bytes;
+    *along_rows = planar;
+    return true;
+}
+
+}  // namespace
+
+bool conv_strip_takes(const ConvDirectArgs& d) {
+    StripArgs g;
+    int64_t bytes;
+    bool planar;
+    return cut_strips(d, &g, &bytes, &planar);
+}
+
+int run_conv_strip(const ConvDirectArgs& d, hipStream_t s) {
+    if (d.total == 0) return CHX_HIP_OK;
+    StripArgs g;
+    int64_t bytes;
+    bool planar;
+    if (!cut_strips(d, &g, &bytes, &planar)) return CHX_HIP_EUNSUPPORTED;
     g.x = d.x; g.w = d.w; g.y = d.y;
     for (int i = 0; i < 4; ++i) {
         g.xs[i] = d.xs[i];
@@ -335,7 +353,7 @@ int run_conv_strip(const ConvDirectArgs& d, hipStream_t s) {
     g.w_flip = d.w_signed ? 0u : 0x80808080u;
     g.zp = (((uint32_t)d.x_zp & 0xffu) * 0x01010101u) ^ g.x_flip;
     g.cx = (d.x_signed ? 0 : 128) - d.x_zp;
-    g.w_row = d.ws[0]; g.M = d.OC; g.K = (int32_t)K;
+    g.w_row = d.ws[0]; g.M = d.OC; g.K = (int32_t)((int64_t)d.Cg * d.KH * d.KW);
     g.w_zp = d.w_zp_len ? d.w_zp : nullptr; g.w_zp_len = d.w_zp_len; g.w_zp_stride = d.w_zp_stride; g.w_zp_signed = d.w_signed;
     magic_divisor((uint32_t)(d.KH * d.KW), &g.taps_mul, &g.taps_shift);
     magic_divisor((uint32_t)d.KW, &g.kw_mul, &g.kw_shift);

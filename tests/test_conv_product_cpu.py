@@ -11,7 +11,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["products", "other_forms", "packed_weights"])
+@pytest.mark.parametrize("case", ["products", "other_forms", "packed_weights", "short_and_parted_rows"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -68,7 +68,7 @@ def packed_weights(host):
 
     assert kernels(64, 1024, 28, 1024) == ["packed"] and kernels(64, 512, 56, 512) == ["packed"]
     assert kernels(64, 1024, 28, 1024, zero_point=3) == ["product"]
-    assert kernels(32, 1024, 56, 1024, stride=2) == ["packed"]
+    assert kernels(32, 1024, 56, 1024, stride=2) == ["packed"] and kernels(64, 2000, 28, 400, stride=2) == ["packed"]
     assert kernels(64, 256, 56, 384) == ["product"] and kernels(64, 512, 28, 320) == ["product"]  # (few channels, 8 G multiply-adds)
     assert kernels(64, 1024, 14, 1024) == ["product"] and kernels(32, 256, 112, 512) == ["product"]
     assert kernels(64, 2048, 7, 3072) == ["product"]  # 3136 pixels, 6 MB of filters
@@ -76,6 +76,19 @@ def packed_weights(host):
     host.check(host.lib.chx_hip_capture_begin(s))
     assert kernels(64, 1024, 28, 1024, stream=s) == ["product"]
     host.check(host.lib.chx_hip_capture_end(s, ctypes.byref(graph)))
+
+
+def short_and_parted_rows(host):
+    """Products that would be mostly padding, or write parts of lines, are for the other kernels, but in a recording."""
+    assert not is_product(host, n=51, c=216, h=7, w=7, oc=1336) and is_product(host, n=8, c=1016, h=7, w=7, oc=664)  # 49 columns, many and few tiles
+    assert is_product(host, n=125, c=160, h=11, w=11, oc=128)
+    assert not is_product(host, n=246, c=32, h=35, w=35, oc=200) and is_product(host, n=230, c=32, h=56, w=56, oc=104)
+    assert not is_product(host, n=55, c=672, h=10, w=10, oc=80, strides=(2, 2), channels_last=True)  # strips
+    assert is_product(host, n=10, c=136, h=48, w=48, oc=320, strides=(2, 2), channels_last=True)
+    assert not is_product(host, n=62, c=544, h=8, w=8, oc=1312, strides=(2, 2), channels_last=True)  # planes
+    assert is_product(host, n=135, c=552, h=14, w=14, oc=304, strides=(2, 2), channels_last=True)
+    # what the others do not take: rows of results that are strided differently, a stride of 3
+    assert is_product(host, n=62, c=544, h=8, w=8, oc=1312, strides=(2, 1), channels_last=True) and is_product(host, n=62, c=544, h=12, w=12, oc=1312, strides=(3, 3), channels_last=True)
 
 
 if __name__ == "__main__":

@@ -67,3 +67,15 @@ def test_large_layers(g, OC, wz):
     pixels = sorted({0, 1, 127, 128, len(got) // 2, len(got) - 129, len(got) - 1} | set(range(77, len(got), 997)))
     want = (x.reshape(-1, 1024)[pixels].astype(np.float64) - 5) @ (w[:, :, 0, 0].astype(np.float64) - wz).T  # (exact: below 2^53)
     np.testing.assert_array_equal(got[pixels], want.astype(np.int32))
+
+
+# where the product would be mostly padding or write parts of lines, and the calls beside those that stay products
+@pytest.mark.parametrize("N,C,H,OC,stride", [(51, 216, 7, 1336, 1), (8, 1016, 7, 664, 1), (246, 32, 35, 200, 1), (55, 672, 10, 80, 2), (62, 544, 8, 1312, 2), (135, 552, 14, 304, 2)])
+def test_short_and_parted_rows(g, N, C, H, OC, stride):
+    rng = np.random.default_rng(N + C)
+    x, w = codes(rng, (N, C, H, H), np.uint8), codes(rng, (OC, C, 1, 1), np.int8)
+    xd = g.dev(x) if stride == 1 else g.to_channels_last(g.dev(x))
+    got = g.host(g.ops.ConvInteger(xd, g.dev(w), 5, None, strides=(stride, stride)))
+    for n in {0, 1, N // 2, N - 1}:
+        want = np.tensordot(w[:, :, 0, 0].astype(np.float64), x[n, :, ::stride, ::stride].astype(np.float64) - 5, 1)  # (exact: below 2^53)
+        np.testing.assert_array_equal(got[n], want.astype(np.int32))
