@@ -693,8 +693,15 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
     // the split kernel's, whose fit is the coarser one (then one product in 200 gets slower by more than 3 %, and with less
     // than three steps for a wavefront, which the split kernel has in flight at once, none).  A row's 16 bytes are read in one
     // place, offsets in a tile are 32 bits wide, and one stage is no loop.  (Below 2^26 products the start is the time on either.)
+    // The fits end at 4096 rows and take codes and int32 for one.  With b as it lies, K of 192 (to codes also 256 and 320) and rows of y in
+    // whole lines that counts: two or three stages are no pipeline, and the split kernel's results leave sooner, codes most of all.  Split and
+    // stage in us: 8192 x 192 x 4096 to codes 29.4 and 33.9, 18612 x 192 x 2944 51 and 58, 32768 x 256 x 4096 112 and 117; to int32 100352 x 192 x 256 28.6 and
+    // 31.8, but 65180 x 256 x 128 13.6 and 11.6; from K 352 on stage is faster (8192 x 384 x 1024 6 % and 12 %).  The fits hold where the split
+    // kernel has a rest of K (26288 x 252 x 2944 to codes 85 and 75) and for rows that do not begin lines, of which its tiles write parts
+    // (49490 x 240 x 2712 152 and 129).
+    const bool short_k = !b_transposed && m.K % 64 == 0 && m.K <= (m.requant ? 320 : 192) && m.y_row % 128 == 0;
     const int64_t steps_each = (steps + w - 1) / w;
-    if (!m.lds_64k && steps_each > 2 && m.N >= 16 && m.K >= 192 && (double)(m.M * m.N) * (double)(m.K * batch) >= 0x1p26 && m.a_row >= 0 && m.a_row < (int64_t(1) << 24) && b_ld < (int64_t(1) << 24)) {
+    if (!m.lds_64k && !short_k && steps_each > 2 && m.N >= 16 && m.K >= 192 && (double)(m.M * m.N) * (double)(m.K * batch) >= 0x1p26 && m.a_row >= 0 && m.a_row < (int64_t(1) << 24) && b_ld < (int64_t(1) << 24)) {
         const bool a_odd = m.K % 4 != 0, b_odd = m.N % 4 != 0;
         const int64_t along_m[3] = {128, 64, 64}, along_n[3] = {128, 128, 64};
         double least = 0.9 * split_time(kSplitCosts[b_transposed], (double)steps_each, (double)(work_groups * w) / 1024.0, a_odd, b_odd,

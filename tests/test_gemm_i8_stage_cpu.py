@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["tiles", "other_forms"])
+@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k"])
 def test_case(host_so, case):
     from test_gpu_gemm_i8_stage import SHAPES
     host_hip.run_case(host_so, __file__, case, SHAPES=repr(SHAPES))
@@ -50,6 +50,22 @@ def other_forms(host):
     assert "stage" not in product(host, 4096, 4096, 15)  # a row shorter than a read
     assert "stage" not in product(host, 4096, 176, 4096)  # one stage and a part
     assert "stage" not in product(host, 32, 512, 512)
+
+
+def short_k(host):
+    """Two or three whole stages of K: the split kernel, but for b transposed, rows of y that are no whole lines, and int32 from K 256 on."""
+    def codes(M, K, N):
+        a, b, y = host.tensor("uint8", (M, K)), host.tensor("int8", (K, N)), host.tensor("uint8", (M, N))
+        host.clear()
+        scale = ctypes.c_float
+        host.check(host.lib.chx_hip_qlinear_matmul(ctypes.byref(a), scale(0.02), 128, ctypes.byref(b), scale(0.005), 0, scale(0.04), 128, None, 0, ctypes.byref(y), None))
+        return host.launches()[0]
+
+    assert "split" in codes(8192, 192, 4096) and "split" in codes(32768, 256, 4096) and "split" in codes(8192, 320, 1024)
+    assert "stage" in codes(8192, 384, 1024) and "stage" in codes(26288, 252, 2944) and "stage" in codes(8192, 256, 2712)
+    assert "split" in product(host, 100352, 192, 256) and "split" in product(host, 8192, 192, 8192)
+    assert "stage" in product(host, 8192, 384, 1024) and "stage" in product(host, 33449, 192, 1044)
+    assert "stage" in product(host, 8192, 256, 1024) and "stage" in product(host, 8192, 192, 8192, transposed=True)
 
 
 if __name__ == "__main__":
