@@ -851,7 +851,10 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             for (int slot : {inst.inputs[0].array, inst.inputs[1].scalar, inst.inputs[2].scalar}) slots.insert(slot);
         }
         const int64_t columns = constant_slots_[program.instructions[fused_inputs[links.back()].second].inputs[0].array]->GetArray().shape()[1];
-        const int first = *members.begin(), last = *members.rbegin();
+        // (from the links' dropped instructions on: the Free of a link's operand, which waits for the link, stands behind those)
+        int first = *members.begin();
+        for (int l : links) first = std::min({first, fused_inputs[l].first, fused_inputs[l].second});
+        const int last = *members.rbegin();
         std::vector<ChxVMOp*> steps;
         std::vector<int> freed;
         std::set<int> moved = members;

@@ -14,12 +14,12 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "refused_forms", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "frees_in_front", "refused_forms", "instruction_by_instruction"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
 
-def program(host, dims=(96, 64, 32), rows=8, quantize=True, dequantize=True, free=False, extra=None, x_shape=None):
+def program(host, dims=(96, 64, 32), rows=8, quantize=True, dequantize=True, free=False, extra=None, x_shape=None, quantized_again=False):
     import numpy as np
     b = host.chxvm.ProgramBuilder()
     h = b.input("x", "float32" if quantize else "uint8", x_shape or [rows, dims[0]])
@@ -51,6 +51,9 @@ def program(host, dims=(96, 64, 32), rows=8, quantize=True, dequantize=True, fre
         d = b.DequantizeLinear(h, scale, zp)
         free_of(h, scale, zp)
         h = d
+    if quantized_again:
+        h = b.QuantizeLinear(d, b.scalar(0.7, "float32"), b.scalar(1, "uint8"))
+        free_of(d)
     b.output("y", h)
     return host.program(b)
 
@@ -86,6 +89,14 @@ def frees_between(host):
         assert kernels(host, p, (8, 96)) == [CHAIN]
         # also where the instructions run one by one: every other column of an array
         assert kernels(host, p, (8, 96), strides=[192, 2]) == ["quantize_strided_kernel", PRODUCT, PRODUCT, PRODUCT, DEQUANTIZE]
+
+
+def frees_in_front(host):
+    """A chain without a QuantizeLinear in front gives back its input: the Free of it stands in front of the chain's first instruction."""
+    # six layers, two layers, and a QuantizeLinear whose result (1 MB) takes the place of what lies between the two chains
+    p = program(host, (64,) * 9, rows=16384, free=True, quantized_again=True)
+    assert kernels(host, p, (16384, 64)) == [CHAIN, CHAIN, QUANTIZE]
+    assert host.log().count("hipMalloc %d" % (16384 * 64)) == 1
 
 
 def refused_forms(host):
