@@ -57,6 +57,16 @@ private:
     int a_, a_scale_, a_zp_, b_, b_scale_, b_zp_, y_scale_, y_zp_, y_;
 };
 
+// Instructions of a program, with their places in it.
+typedef std::vector<std::pair<int, ChxVMOp*>> ChxVMSteps;
+
+void RunSteps(const ChxVMSteps& steps, ChxVMState* st) {
+    for (const auto& step : steps) {
+        st->set_pc(step.first);  // (what an error is reported with)
+        step.second->Run(st);
+    }
+}
+
 std::atomic<int64_t> g_matmul_chains{0};
 
 // A chain of such products, with the QuantizeLinear in front of it and the DequantizeLinear behind it where nobody else
@@ -70,7 +80,7 @@ public:
     };
     // steps: the instructions that this one replaces and the Free's of their operands between them, in the program's order
     QLinearMatMulChainOp(const ChxVMInstructionProto& last, const ChxVMInstructionProto* quantize, std::vector<Layer> layers, int64_t columns, int a,
-                         const ChxVMInstructionProto* dequantize, std::vector<ChxVMOp*> steps, std::vector<int> freed)
+                         const ChxVMInstructionProto* dequantize, ChxVMSteps steps, std::vector<int> freed)
         : ChxVMOp(last), quantize_(quantize != nullptr), dequantize_(dequantize != nullptr), x_(quantize ? quantize->inputs[0].array : a),
           x_scale_(quantize ? quantize->inputs[1].scalar : -1), x_zp_(quantize ? quantize->inputs[2].scalar : -1),
           y_scale_(dequantize ? dequantize->inputs[1].scalar : -1), y_zp_(dequantize ? dequantize->inputs[2].scalar : -1),
@@ -81,7 +91,7 @@ public:
         if (RunAsOne(st)) {
             for (int slot : freed_) st->FreeVar(slot);
         } else {
-            for (ChxVMOp* op : steps_) op->Run(st);
+            RunSteps(steps_, st);
         }
     }
 
@@ -138,7 +148,7 @@ private:
     int x_, x_scale_, x_zp_, y_scale_, y_zp_, y_;
     int64_t columns_;
     std::vector<Layer> layers_;
-    std::vector<ChxVMOp*> steps_;
+    ChxVMSteps steps_;
     std::vector<int> freed_;
 };
 
@@ -353,7 +363,7 @@ public:
         std::shared_ptr<ResidualFusionState> state;  // null: no sum
     };
     InvertedResidualOp(const ChxVMInstructionProto& projection, std::shared_ptr<chx_hip_inverted_residual> block, int x, int between, const std::vector<Quantization>& convs,
-                       int64_t out_channels, int stride, bool has_bias, Sum sum, std::vector<ChxVMOp*> steps, std::vector<int> freed)
+                       int64_t out_channels, int stride, bool has_bias, Sum sum, ChxVMSteps steps, std::vector<int> freed)
         : ChxVMOp(projection), block_(std::move(block)), x_(x), between_(between), y_(projection.outputs[0]), convs_(convs), out_channels_(out_channels), stride_(stride),
           has_bias_(has_bias), sum_(std::move(sum)), steps_(std::move(steps)), freed_(std::move(freed)) {
     }
@@ -362,7 +372,7 @@ public:
         if (RunAsOne(st)) {
             for (int slot : freed_) st->FreeVar(slot);
         } else {
-            for (ChxVMOp* op : steps_) op->Run(st);
+            RunSteps(steps_, st);
         }
     }
 
@@ -445,7 +455,7 @@ private:
     int stride_;
     bool has_bias_;
     Sum sum_;
-    std::vector<ChxVMOp*> steps_;
+    ChxVMSteps steps_;
     std::vector<int> freed_;
 };
 
@@ -855,7 +865,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         int first = *members.begin();
         for (int l : links) first = std::min({first, fused_inputs[l].first, fused_inputs[l].second});
         const int last = *members.rbegin();
-        std::vector<ChxVMOp*> steps;
+        ChxVMSteps steps;
         std::vector<int> freed;
         std::set<int> moved = members;
         for (int i = first; i <= last; ++i) {
@@ -863,7 +873,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             const bool frees = inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array);
             if (frees) freed.push_back(inst.inputs[0].array);
             if (frees && !dynamic_cast<NopOp*>(program_[i].get())) moved.insert(i);  // (the others run behind one of the members)
-            if (moved.count(i)) steps.push_back(program_[i].get());
+            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
         }
         chains_.emplace_back(new QLinearMatMulChainOp(program.instructions[last], quantize ? &program.instructions[head] : nullptr, std::move(layers), columns, a,
                                                       dequantize ? &program.instructions[tail] : nullptr, std::move(steps), std::move(freed)));
@@ -943,7 +953,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             sum.state = fusion_state[p];
         }
         std::set<int> moved(members, members + 3);
-        std::vector<ChxVMOp*> steps;
+        ChxVMSteps steps;
         std::vector<int> freed;
         for (int i = e; i <= p; ++i) {
             const ChxVMInstructionProto& inst = program.instructions[i];
@@ -951,7 +961,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
                 freed.push_back(inst.inputs[0].array);
                 moved.insert(i);
             }
-            if (moved.count(i)) steps.push_back(program_[i].get());
+            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
         }
         chains_.emplace_back(new InvertedResidualOp(program.instructions[p], std::shared_ptr<chx_hip_inverted_residual>(block, chx_hip_inverted_residual_destroy),
                                                     program.instructions[e].inputs[0].array, h2, convs, tensors[2][0].shape[0], static_cast<int>(stride),
@@ -1107,13 +1117,12 @@ InOuts ChxVM::Run(const InOuts& program_inputs, const ChxVMOptions& options) {
         ChxVMState state(options, constant_slots_, program_inputs);
         state.set_minus_128_slots(&minus_128_slots_);
         for (const auto& instruction : remaining_) {
-            const int pc = instruction.first;
-            ChxVMOp* op = instruction.second;
-            state.set_pc(pc);
+            state.set_pc(instruction.first);
             try {
-                op->Run(&state);
+                instruction.second->Run(&state);
             } catch (...) {
-                std::cerr << "Exception in " << op->name() << " (pc " << pc << ") " << op->debug_info() << std::endl;
+                const ChxVMOp* op = program_[state.pc()].get();  // (one of those that a chain stands for, where it runs them)
+                std::cerr << "Exception in " << op->name() << " (pc " << state.pc() << ") " << op->debug_info() << std::endl;
                 throw;
             }
         }

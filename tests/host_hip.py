@@ -5,6 +5,7 @@ import importlib
 import os
 import subprocess
 import sys
+import tempfile
 import types
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -112,6 +113,21 @@ class Host:
         rt = self.chxvm.runtime()
         assert rt.chxvm_program_create(data, len(data), ctypes.byref(h)) == 0, rt.chxvm_last_error()
         return h
+
+    def run_fails(self, program, inputs):
+        """What the runtime writes to stderr about a run that does not succeed."""
+        rt, out = self.chxvm.runtime(), ctypes.c_void_p()
+        with tempfile.TemporaryFile() as f:
+            kept = os.dup(2)
+            os.dup2(f.fileno(), 2)
+            try:
+                rc = rt.chxvm_program_run(program, *self.names_and(inputs), 0, ctypes.byref(out))
+            finally:
+                os.dup2(kept, 2)
+                os.close(kept)
+            assert rc != 0
+            f.seek(0)
+            return f.read().decode()
 
     def names_and(self, inputs):
         """{name: descriptor} as the C ABI takes it."""

@@ -25,7 +25,7 @@ def sum_code():
     return pkg.workloads.add_program(pkg.ops, (0.3, 128), (0.1, 7), (0.4, 120))
 
 
-@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "errors", "instruction_by_instruction"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -138,6 +138,13 @@ def few_rows(host):
     """More than 256 channels out and fewer than 512 rows."""
     for channels, n, blocks in (((160, 960, 320), 64, 0), ((160, 960, 320), 74, 1), ((160, 960, 256), 1, 1), ((160, 960, 257), 1, 0)):
         assert one(host, program(host, channels, image=7), (n, channels[0], 7, 7)) == blocks
+
+
+def errors(host):
+    """An error names the convolution that it is of: the expansion."""
+    x = host.channels_last("uint8", (2, 32, 8, 8))  # (twice the channels)
+    said = host.run_fails(program(host), {"x": x})
+    assert "Exception in QLinearConv (pc 9)" in said, said
 
 
 def instruction_by_instruction(host):
