@@ -1762,6 +1762,7 @@ extern "C" int chx_hip_qlinear_matmul(
 struct chx_hip_inverted_residual {
     int32_t channels = 0, expanded = 0, out_channels = 0, stride = 1;
     bool has_bias = false, affine_residual = true;
+    int device = 0;  // whose memory the operands are laid out in
     int tiles = 0, tiles_padded = 0, steps = 0, tiles_oc = 0;
     char* memory = nullptr;
     size_t at_w3 = 0, at_t1 = 0, at_t2 = 0, at_t3 = 0;
@@ -1809,6 +1810,7 @@ extern "C" int chx_hip_inverted_residual_create(const chx_hip_conv_operands* sta
         if (!all_zero(zp)) return refuse("zero points of the weights");
     }
     std::unique_ptr<chx_hip_inverted_residual, void (*)(chx_hip_inverted_residual*)> p(new chx_hip_inverted_residual(), chx_hip_inverted_residual_destroy);
+    CHX_HIP_CALL(hipGetDevice(&p->device));
     p->channels = (int32_t)w1.shape[1];
     p->expanded = (int32_t)hid;
     p->out_channels = (int32_t)w3.shape[0];
@@ -1847,6 +1849,9 @@ extern "C" int chx_hip_inverted_residual_run(
         set_error("inverted residual: %s", why);
         return (int)CHX_HIP_EUNSUPPORTED;
     };
+    int device = 0;
+    CHX_HIP_CALL(hipGetDevice(&device));
+    if (device != plan->device) return refuse("another device than the one that it was created on");
     auto in_range = [](int32_t zp, int32_t dt) { return dt == CHX_HIP_INT8 ? zp >= -128 && zp <= 127 : zp >= 0 && zp <= 255; };
     if (x->ndim != 4 || out->ndim != 4 || !is_q8(x->dtype) || x->shape[1] != plan->channels || !in_range(x_zero_point, x->dtype)) return refuse("x");
     if ((flags & (CHX_HIP_ROUND_ONNX_RNE | CHX_HIP_FUSE_RELU)) != 0 || (plan->has_bias && !(flags & CHX_HIP_BIAS_ONNX_INT32))) return refuse("the flags");

@@ -313,6 +313,8 @@ extern "C" int chx_hip_qlinear_chain(
     //    1024 -> 512                        9.7 / 10.9      9.9 / 11.1    13.5 / 21.0    45.5 / 46.7
     //    six layers of 512                 22.7 / 30.8     22.9 / 32.6    26.8 / 53.4    92.9 / 115
     if (x->shape[0] > 16384) return refuse("too many rows");
+    int device = 0;
+    CHX_HIP_CALL(hipGetDevice(&device));
     ChainArgs g;
     memset(&g, 0, sizeof(g));
     g.x_is_float = x->dtype == CHX_HIP_FLOAT32;
@@ -331,7 +333,7 @@ extern "C" int chx_hip_qlinear_chain(
     for (int i = 0; i < n; ++i) {
         const chx_hip_chain_layer& in = layers[i];
         ChainLayer& L = g.layer[i];
-        if (in.b == nullptr) return refuse("a layer's weights");
+        if (in.b == nullptr || in.b->device != device) return refuse("a layer's weights");
         if (in.b->K != k || (i > 0 && k > kMaxN)) return refuse("a layer's size");
         if (!is_q8(in.y_dtype) || !zero_point_fits(in.a_zero_point, dtype) || !zero_point_fits(in.b_zero_point, in.b->is_signed ? CHX_HIP_INT8 : CHX_HIP_UINT8) || !zero_point_fits(in.y_zero_point, in.y_dtype))
             return refuse("a layer's quantization");

@@ -292,7 +292,7 @@ void chx_hip_inverted_residual_destroy(chx_hip_inverted_residual* plan);
 /* y_scales, y_zero_points: of the three convolutions' results, all of type y_dtype.  r NULL: `out` is the third one's;
  * else the sum of it and r (arguments as for chx_hip_qconv_plan_run_add).  CHX_HIP_EUNSUPPORTED, with nothing launched, for
  * what the kernel does not take (anything but channels-last arrays in whole 16-byte chunks, uint8 results, the reference's
- * rounding, an int32 bias of the ONNX kind, rows that fit LDS) or is not the faster one for; the single calls then say
+ * rounding, an int32 bias of the ONNX kind, rows that fit LDS, the device that the block was created on) or is not the faster one for; the single calls then say
  * what is wrong with the operands, if something is. */
 int chx_hip_inverted_residual_run(
         chx_hip_inverted_residual* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points,
@@ -334,7 +334,7 @@ typedef struct chx_hip_chain_layer {
 /* QuantizeLinear (x float32; left out for x of type x_dtype), n chx_hip_qlinear_matmul without bias, each on the codes
  * of the one before, and DequantizeLinear (y float32; left out for y of the last layer's type) as one launch, with the
  * codes of the single calls.  x [M, K] and y [M, N] in rows.  CHX_HIP_EUNSUPPORTED, with nothing launched, for more than
- * 6 layers, more rows than one launch gains on, and anything that is not in rows or not consistent; the single calls then
+ * 6 layers, more rows than one launch gains on, weights laid out on another device than the current one, and anything that is not in rows or not consistent; the single calls then
  * say what is wrong with it, if something is. */
 int chx_hip_qlinear_chain(
         const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, int32_t x_dtype, const chx_hip_chain_layer* layers, int32_t n,

@@ -25,7 +25,7 @@ def sum_code():
     return pkg.workloads.add_program(pkg.ops, (0.3, 128), (0.1, 7), (0.4, 120))
 
 
-@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "errors", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "errors", "another_device", "instruction_by_instruction"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -145,6 +145,15 @@ def errors(host):
     x = host.channels_last("uint8", (2, 32, 8, 8))  # (twice the channels)
     said = host.run_fails(program(host), {"x": x})
     assert "Exception in QLinearConv (pc 9)" in said, said
+
+
+def another_device(host):
+    """The operands are laid out in one device's memory: on another one the convolutions run."""
+    p = program(host)
+    host.check(host.lib.chx_hip_init(1))
+    assert one(host, p) == 0
+    host.check(host.lib.chx_hip_init(0))
+    assert one(host, p) == 1
 
 
 def instruction_by_instruction(host):

@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "frees_in_front", "refused_forms", "errors", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "frees_in_front", "refused_forms", "errors", "another_device", "instruction_by_instruction"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -110,6 +110,15 @@ def errors(host):
     """An error names the instruction that it is of, not the one that the chain stands in the place of."""
     # x has a column too many for the first product, the 12th instruction
     assert "Exception in QuantizeLinear (pc 12)" in host.run_fails(program(host), {"x": host.tensor("float32", (8, 97))})
+
+
+def another_device(host):
+    """The weights are laid out in one device's memory: on another one the instructions run."""
+    p = program(host)
+    host.check(host.lib.chx_hip_init(1))
+    assert kernels(host, p, (8, 96)) == [QUANTIZE, PRODUCT, PRODUCT, DEQUANTIZE]
+    host.check(host.lib.chx_hip_init(0))
+    assert kernels(host, p, (8, 96)) == [CHAIN]
 
 
 def instruction_by_instruction(host):
