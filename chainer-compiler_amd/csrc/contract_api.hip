@@ -180,14 +180,15 @@ inline int round_up(int v, int m) {
 
 // Packed weights for the MFMA kernel (see conv_mfma.hip).
 struct PackedWeights {
-    int8_t* wp = nullptr;
+    int8_t* wp = nullptr;       // and in the same allocation the others, but for
+    int8_t* wf_apart = nullptr;  // wf, where that has one of its own
     int32_t* wsum = nullptr;
-    int32_t* padsum = nullptr;  // ConvMfmaArgs::padsum (inside wsum's allocation), null for dense packing and for more than 32 taps
+    int32_t* padsum = nullptr;  // ConvMfmaArgs::padsum, null for dense packing and for more than 32 taps
     int C64 = 0, OCpad = 0, KP = 0;
     int BK = 64;         // K bytes per kernel step; the packed layout depends on it
     bool dense = false;  // taps packed densely; activations go through an explicit im2col
-    int8_t* wf = nullptr;  // of a plan: the weights in the order of the small tiles (inside wp's allocation)
-    int8_t* wd = nullptr;  // dense only: the same weights in the order of the planar-input kernel (inside wp's allocation)
+    int8_t* wf = nullptr;  // of a plan with at most 32 taps: the weights in the order of the small tiles
+    int8_t* wd = nullptr;  // dense only: the same weights in the order of the planar-input kernel
 };
 
 // Dense packing pays when per-tap padding to 64 channels would at least double the K extent, and the channels do not fill
@@ -826,51 +827,42 @@ int make_packed(const chx_hip_tensor& w, bool persistent, hipStream_t s, PackedW
     const bool stem = pw->dense && stem_shape_fits((int)w.shape[1], (int)w.shape[2], (int)w.shape[3]);
     const size_t stem_bytes =
             stem ? (size_t)(pw->OCpad / 64) * stem_k_blocks((int)w.shape[1], (int)w.shape[2], (int)w.shape[3]) * 2048 : 0;
-    const size_t bytes = mfma_bytes + stem_bytes + (persistent ? mfma_bytes : 0);  // (a call's own weights are read once: not worth another pass)
+    // (a call's own weights are read once: not worth another pass; the small tiles take up to 32 taps)
+    const size_t fragment_bytes = persistent && (pw->dense || w.shape[2] * w.shape[3] <= 32) ? mfma_bytes : 0;
     // the per-channel sums, and behind them the sixteen classes of border sums
     // (between 2 and 32 taps: the kernel's tap masks hold 32, and a single tap that can lie outside is rare enough for
     // the flat-address padding)
     const bool border_sums = !pw->dense && w.shape[2] * w.shape[3] <= 32 && w.shape[2] * w.shape[3] > 1;
-    const size_t sums_bytes = sizeof(int32_t) * pw->OCpad * (border_sums ? 17 : 1);
-    void* p0 = nullptr;
-    void* p1 = nullptr;
-    if (persistent) {
-        CHX_HIP_CALL(hipMalloc(&p0, bytes));
-        if (hipMalloc(&p1, sums_bytes) != hipSuccess) {
-            (void)hipFree(p0);
-            CHX_FAIL(CHX_HIP_ERUNTIME, "hipMalloc failed for the per-channel weight sums");
-        }
-    } else {
-        CHX_PROPAGATE(scratch_alloc(&p0, bytes, s));
-        if (scratch_alloc(&p1, sums_bytes, s) != CHX_HIP_OK) {
-            scratch_free(p0, s);
-            return CHX_HIP_ERUNTIME;
-        }
+    const size_t sums_bytes = sizeof(int32_t) * pw->OCpad * (border_sums ? 17 : 1), others = mfma_bytes + stem_bytes + sums_bytes;
+    // An allocation above 2 MB takes the device runtime 20 us more than one below, and two small ones 1 us more than one: 512 ->
+    // 2048 channels in one 57 us for the plan, apart 37.
+    const bool apart = fragment_bytes > 0 && others + fragment_bytes > (size_t(2) << 20) && others <= (size_t(2) << 20);
+    void* p = nullptr;
+    void* p_apart = nullptr;
+    if (persistent) CHX_HIP_CALL(hipMalloc(&p, others + (apart ? 0 : fragment_bytes)));
+    else CHX_PROPAGATE(scratch_alloc(&p, others, s));
+    if (apart && hipMalloc(&p_apart, fragment_bytes) != hipSuccess) {
+        (void)hipFree(p);
+        CHX_FAIL(CHX_HIP_ERUNTIME, "hipMalloc failed for the small tiles' weights");
     }
-    pw->wp = static_cast<int8_t*>(p0);
-    pw->wsum = static_cast<int32_t*>(p1);
-    pw->padsum = border_sums ? pw->wsum + pw->OCpad : nullptr;
+    // (weights, and what is made of them, are multiples of 2048 bytes)
+    pw->wp = static_cast<int8_t*>(p);
     pw->wd = stem ? pw->wp + mfma_bytes : nullptr;
+    pw->wf_apart = static_cast<int8_t*>(p_apart);
+    pw->wf = apart ? pw->wf_apart : fragment_bytes ? pw->wp + mfma_bytes + stem_bytes : nullptr;
+    pw->wsum = reinterpret_cast<int32_t*>(pw->wp + mfma_bytes + stem_bytes + (apart ? 0 : fragment_bytes));
+    pw->padsum = border_sums ? pw->wsum + pw->OCpad : nullptr;
     if (stem) CHX_PROPAGATE(pack_weights_stem(w, pw->OCpad, pw->wd, s));
-    pw->wf = persistent ? pw->wp + mfma_bytes + stem_bytes : nullptr;
-    if (pw->dense) CHX_PROPAGATE(pack_weights_dense(w, pw->KP, pw->BK, pw->OCpad, pw->wp, pw->wsum, s));
-    else CHX_PROPAGATE(pack_weights(w, pw->C64, pw->BK, pw->OCpad, pw->wp, pw->wsum, pw->padsum, s));
-    return pw->wf ? fragment_weights(pw->wp, pw->KP, pw->BK, pw->OCpad, pw->wf, s) : (int)CHX_HIP_OK;
+    if (pw->dense) return pack_weights_dense(w, pw->KP, pw->BK, pw->OCpad, pw->wp, pw->wf, pw->wsum, s);
+    return pack_weights(w, pw->C64, pw->BK, pw->OCpad, pw->wp, pw->wf, pw->wsum, pw->padsum, s);
 }
 
 void release_packed(PackedWeights* pw, bool persistent, hipStream_t s) {
-    if (persistent) {
-        if (pw->wp) (void)hipFree(pw->wp);
-        if (pw->wsum) (void)hipFree(pw->wsum);
-    } else {
-        scratch_free(pw->wp, s);
-        scratch_free(pw->wsum, s);
-    }
-    pw->wp = nullptr;
-    pw->wsum = nullptr;
-    pw->padsum = nullptr;
-    pw->wd = nullptr;
-    pw->wf = nullptr;
+    if (!persistent) scratch_free(pw->wp, s);
+    else if (pw->wp) (void)hipFree(pw->wp);
+    if (pw->wf_apart) (void)hipFree(pw->wf_apart);
+    pw->wp = pw->wf = pw->wf_apart = pw->wd = nullptr;
+    pw->wsum = pw->padsum = nullptr;
 }
 
 // Depthwise 3x3 on int8 weights with zero weight zero points: packed filter rows and per-channel sums.

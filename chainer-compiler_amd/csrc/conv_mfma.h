@@ -55,7 +55,7 @@ struct ConvMfmaArgs {
     int32_t nk;   // K steps: KP / bk
     int32_t KP;   // packed row length: KH * KW * C64
     const int8_t* wp;     // [OCpad / 64][nk][64][bk]
-    const int8_t* wf;     // the same in the order of the small tiles' fragments (fragment_weights); null: not for those
+    const int8_t* wf;     // the same in the order of the small tiles' fragments (fragment_offset in conv_mfma.hip); null: not for those
     const int32_t* wsum;  // [OCpad]
     // [16][OCpad]: the sum of a filter's weights over the taps of its first row (class bit 3), last row (bit 2), first
     // column (bit 1) and last column (bit 0), each tap once: what a pixel whose window leaves the image on those sides
@@ -147,11 +147,9 @@ inline void magic_divisor(uint32_t d, uint32_t* mul, uint32_t* shift) {
     *shift = l;
 }
 
-int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int32_t* wsum, hipStream_t s);
-// [OCpad / 32][KP / 64][2 halves of 64 k][2 x 16 channels][2 x 16 k][16 channels][16 k]: a step's fragment is 1 KB in one or two places
-int fragment_weights(const int8_t* wp, int KP, int BK, int OCpad, int8_t* wf, hipStream_t s);
+int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, hipStream_t s);
 int launch_im2col_dense(const Im2colArgs& a, hipStream_t s);
-int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int32_t* wsum, int32_t* padsum, hipStream_t s);
+int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, int32_t* padsum, hipStream_t s);
 // the stem kernel: weights [C][KH][KW] with C*KH <= 32 and KW <= 8; patch = LDS bytes of a tile's input rows
 bool stem_shape_fits(int C, int KH, int KW);
 bool stem_patch_fits(int C, int KH, int KW, int sh, int sw);

@@ -45,14 +45,21 @@ __host__ __device__ __forceinline__ int64_t packed_offset(int oc, int k, int KP,
     return ((int64_t)(oc >> 6) * (KP / BK) + k / BK) * (64 * BK) + (oc & 63) * BK + k % BK;
 }
 
+// The same weights as the small tiles read them (ConvMfmaArgs::wf): [OCpad / 32][KP / 64][2 halves of 64 k][2 x 16 channels]
+// [2 x 16 k][16 channels][16 k], so that a step's fragment is 1 KB in one or two places.
+__device__ __forceinline__ int64_t fragment_offset(int oc, int k, int KP) {
+    return ((int64_t)(oc >> 5) * (KP / 64) + (k >> 6)) * 2048 + (k >> 5 & 1) * 1024 + (oc >> 4 & 1) * 512 + (k >> 4 & 1) * 256 + (oc & 15) * 16 + (k & 15);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Weight repacking: w [OC][C][KH][KW] (any strides) -> Wp, K index k = (kh*KW + kw)*C64 + c with
 // C64 = C rounded up to 64 (zero filled), and wsum[oc] = sum of the row.  One work-group per
 // output channel.  padsum (when not null; at most 32 taps): [16][gridDim.x] sums of the row over the taps of the
-// filter's border rows and columns that the class names (ConvMfmaArgs::padsum).
+// filter's border rows and columns that the class names (ConvMfmaArgs::padsum).  wf (when not null): the weights in that order
+// as well (a kernel of its own for them cost a plan 3 us more).
 __global__ __launch_bounds__(256) void pack_weights_kernel(
         const char* __restrict__ w, int64_t s_oc, int64_t s_c, int64_t s_kh, int64_t s_kw, int OC, int C, int KH, int KW,
-        int C64, int BK, int8_t* __restrict__ wp, int32_t* __restrict__ wsum, int32_t* __restrict__ padsum) {
+        int C64, int BK, int8_t* __restrict__ wp, int8_t* __restrict__ wf, int32_t* __restrict__ wsum, int32_t* __restrict__ padsum) {
     const int oc = blockIdx.x;
     const int KP = KH * KW * C64;
     __shared__ int32_t tap_sum[32];
@@ -69,6 +76,7 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
             v = *reinterpret_cast<const int8_t*>(w + oc * s_oc + c * s_c + kh * s_kh + kw * s_kw);
         }
         wp[packed_offset(oc, k, KP, BK)] = v;
+        if (wf) wf[fragment_offset(oc, k, KP)] = v;
         local += v;
         if (padsum) {
             if (pos != run_pos) {
@@ -100,16 +108,6 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
     }
 }
 
-// One thread per 16 bytes of wf.
-__global__ __launch_bounds__(256) void fragment_weights_kernel(const int8_t* __restrict__ wp, int KP, int BK, int64_t chunks, int8_t* __restrict__ wf) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= chunks) return;
-    const int64_t block = i >> 7;  // 32 channels x 64 k
-    const int in = (int)i & 127, half = in >> 6, sixteen = in >> 5 & 1, group = in >> 4 & 1;
-    const int oc = (int)(block / (KP / 64)) * 32 + sixteen * 16 + (in & 15), k = (int)(block % (KP / 64)) * 64 + half * 32 + group * 16;
-    reinterpret_cast<uint4*>(wf)[i] = *reinterpret_cast<const uint4*>(wp + packed_offset(oc, k, KP, BK));
-}
-
 // Few input channels (the 3-channel stem): padding each filter tap to 64 K-bytes would waste
 // most of the matrix-core work, so the taps are packed densely instead.  The weights become
 // [OCpad][Kd] with k = (kh*KW + kw)*C + c, Kd = KH*KW*C rounded up to 64, and the activations
@@ -118,7 +116,7 @@ __global__ __launch_bounds__(256) void fragment_weights_kernel(const int8_t* __r
 // holds anything (its weights are zero).
 __global__ __launch_bounds__(256) void pack_weights_dense_kernel(
         const char* __restrict__ w, int64_t s_oc, int64_t s_c, int64_t s_kh, int64_t s_kw, int OC, int C, int KH, int KW,
-        int Kd, int BK, int8_t* __restrict__ wp, int32_t* __restrict__ wsum) {
+        int Kd, int BK, int8_t* __restrict__ wp, int8_t* __restrict__ wf, int32_t* __restrict__ wsum) {
     const int oc = blockIdx.x;
     const int K = KH * KW * C;
     int32_t local = 0;
@@ -131,6 +129,7 @@ __global__ __launch_bounds__(256) void pack_weights_dense_kernel(
             v = *reinterpret_cast<const int8_t*>(w + oc * s_oc + c * s_c + kh * s_kh + kw * s_kw);
         }
         wp[packed_offset(oc, k, Kd, BK)] = v;
+        if (wf) wf[fragment_offset(oc, k, Kd)] = v;
         local += v;
     }
     __shared__ int32_t red[256];
@@ -254,23 +253,17 @@ __global__ __launch_bounds__(256) void im2col_dense_lds_kernel(Im2colArgs a, int
 }  // namespace
 
 int pack_weights(
-        const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int32_t* wsum, int32_t* padsum, hipStream_t s) {
+        const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, int32_t* padsum, hipStream_t s) {
     pack_weights_kernel<<<OCpad, 256, 0, s>>>(
             static_cast<const char*>(w.data), w.strides[0], w.strides[1], w.strides[2], w.strides[3], (int)w.shape[0],
-            (int)w.shape[1], (int)w.shape[2], (int)w.shape[3], C64, BK, wp, wsum, padsum);
+            (int)w.shape[1], (int)w.shape[2], (int)w.shape[3], C64, BK, wp, wf, wsum, padsum);
     return launch_check("pack_weights_kernel");
 }
 
-int fragment_weights(const int8_t* wp, int KP, int BK, int OCpad, int8_t* wf, hipStream_t s) {
-    const int64_t chunks = (int64_t)OCpad * (KP / 16);
-    fragment_weights_kernel<<<(unsigned)((chunks + 255) / 256), 256, 0, s>>>(wp, KP, BK, chunks, wf);
-    return launch_check("fragment_weights_kernel");
-}
-
-int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int32_t* wsum, hipStream_t s) {
+int pack_weights_dense(const chx_hip_tensor& w, int Kd, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, hipStream_t s) {
     pack_weights_dense_kernel<<<OCpad, 256, 0, s>>>(
             static_cast<const char*>(w.data), w.strides[0], w.strides[1], w.strides[2], w.strides[3], (int)w.shape[0],
-            (int)w.shape[1], (int)w.shape[2], (int)w.shape[3], Kd, BK, wp, wsum);
+            (int)w.shape[1], (int)w.shape[2], (int)w.shape[3], Kd, BK, wp, wf, wsum);
     return launch_check("pack_weights_dense_kernel");
 }
 

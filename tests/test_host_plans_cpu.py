@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer", "kernels_of_a_fused_group", "fused_groups_of_many_elements"])
+@pytest.mark.parametrize("case", ["one_plan_on_dense_images_and_crops", "packed_pixels", "requantization_forms", "shared_memory_of_conv_integer", "kernels_of_a_fused_group", "what_a_plan_costs", "fused_groups_of_many_elements"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -75,6 +75,22 @@ def packed_pixels(host):
     rc = host.lib.chx_hip_qconv_plan_run_pair(both, ctypes.byref(x), ctypes.c_float(0.02), 128, 64, ctypes.c_float(0.05), 3, 0, ctypes.byref(y1), ctypes.c_float(0.05), 3, 0,
                                               ctypes.byref(y2), None)
     assert rc == host.capi.EUNSUPPORTED and not host.launches()
+
+
+def what_a_plan_costs(host):
+    """One launch and one allocation (two where one would pass 2 MB).  The weights are there twice, in the order of the staged and
+    of the small tiles, but for filters that the small tiles do not take."""
+    for oc, c, k, copies, apart in ((128, 64, 1, 2, False), (128, 256, 3, 2, False), (128, 64, 5, 2, False), (128, 64, 7, 1, False), (2048, 512, 1, 2, True), (512, 512, 3, 2, False)):
+        host.clear()
+        plan = host.plan(oc, c, k)
+        weights, sums = oc * k * k * c, oc * 4 * (17 if 1 < k < 6 else 1)
+        sizes = [weights + sums, weights] if apart else [weights * copies + sums]
+        assert len(host.launches()) == 1
+        # (behind those of the filters, scales, zero points that host.plan makes)
+        assert [line for line in host.log() if "hipMalloc" in line][3:] == ["hipMalloc %d" % n for n in sizes]
+        host.clear()
+        host.lib.chx_hip_qconv_plan_destroy(plan)
+        assert host.log().count("hipFree") == len(sizes)
 
 
 def requantization_forms(host):
