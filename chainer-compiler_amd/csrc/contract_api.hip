@@ -1882,6 +1882,15 @@ extern "C" int chx_hip_inverted_residual_run(
         if (!is_q8(r->dtype) || !in_range(r_zero_point, r->dtype) || !in_range(out_zero_point, out_dtype) || !(out_scale >= 0x1p-60f && out_scale <= 0x1p60f)) return refuse("the quantization of the sum");
         if (!y_is_pixel_major(*r, &r_px) || !aligned(r->data, 16) || r_px % 16 != 0 || r_px < plan->out_channels) return refuse("r is not channels-last in whole chunks");
         if (byte_ranges_overlap(outv, *r)) return refuse("out overlaps r");
+    }
+    a.N = (int32_t)N; a.H = (int32_t)H; a.W = (int32_t)W; a.OH = (int32_t)OH; a.OW = (int32_t)OW;
+    a.OC = plan->out_channels;
+    a.hid_tiles = plan->tiles;
+    a.hid_tiles_padded = plan->tiles_padded;
+    a.x_chunks = (int32_t)chunks;
+    a.KS = plan->steps;
+    CHX_PROPAGATE(plan_inverted_residual(&a, plan->stride));
+    if (r) {  // (the first call with a sum's parameters launches a search: nothing is refused behind it)
         std::lock_guard<std::mutex> lock(plan->mutex);
         CHX_PROPAGATE(residual_of(*r, r_px, y_scales[2], y_zero_points[2], y_dtype, r_scale, r_zero_point, out_scale, out_zero_point, out_dtype, relu != 0,
                                   plan->affine_residual, &plan->searched, s, &a.res));
@@ -1897,12 +1906,6 @@ extern "C" int chx_hip_inverted_residual_run(
     a.t1 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t1);
     a.t2 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t2);
     a.t3 = reinterpret_cast<const int32_t*>(plan->memory + plan->at_t3);
-    a.N = (int32_t)N; a.H = (int32_t)H; a.W = (int32_t)W; a.OH = (int32_t)OH; a.OW = (int32_t)OW;
-    a.OC = plan->out_channels;
-    a.hid_tiles = plan->tiles;
-    a.hid_tiles_padded = plan->tiles_padded;
-    a.x_chunks = (int32_t)chunks;
-    a.KS = plan->steps;
     a.x_flip = x->dtype == CHX_HIP_UINT8 ? 0x80808080u : 0u;
     a.y_flip = out_minus_128 ? 0x80808080u : 0u;
     a.corr1 = (x->dtype == CHX_HIP_UINT8 ? 128 : 0) - x_zero_point;

@@ -24,14 +24,16 @@ struct InvertedResidualArgs {
     QuantProduct q1, q2, q3;
     int32_t fill;                 // the zero point of the expansion's result in the signed range, four times
     ResidualAdd res;              // res.r null: none
-    // the launch (filled by launch_inverted_residual)
+    // the launch (filled by plan_inverted_residual)
+    int32_t G, lds;  // tiles of 32 expanded channels per interval; bytes of LDS
     int32_t R, rows, pitch, pixels, px_bytes, pitch_o, items, tiles_px, tiles_oc, cs, cs2, intervals;
     int32_t at_mask, at_hid, at_dw, at_t3, blocks, strips, xcd_chunk;
     uint32_t strips_mul, strips_shift, pitch_mul, pitch_shift, pitch_o_mul, pitch_o_shift, w_mul, w_shift, chunks_mul, chunks_shift, oct_mul, oct_shift, blk_mul, blk_shift;
 };
 
-// EUNSUPPORTED, with nothing launched, where the block does not fit (LDS, channels) or single launches are faster.
-int launch_inverted_residual(InvertedResidualArgs a, int stride, hipStream_t s);
+// From the sizes above; EUNSUPPORTED where the block does not fit (LDS, channels) or single launches are faster.
+int plan_inverted_residual(InvertedResidualArgs* a, int stride);
+int launch_inverted_residual(const InvertedResidualArgs& a, int stride, hipStream_t s);
 // Weights of a 1x1 convolution [rows, K] (int8, zero points 0) as MFMA fragments, with their tables; `projection`: rows are
 // output channels in the order that leaves a lane sixteen neighbouring ones.
 int pack_inverted_point(const chx_hip_tensor& w, const chx_hip_tensor& scale, const chx_hip_tensor* bias, bool projection, int row_tiles, int k_tiles,

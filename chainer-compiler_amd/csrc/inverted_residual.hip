@@ -404,7 +404,8 @@ int launch_steps(const InvertedResidualArgs& a, int stride, int bytes, hipStream
 
 }  // namespace
 
-int launch_inverted_residual(InvertedResidualArgs a, int stride, hipStream_t s) {
+int plan_inverted_residual(InvertedResidualArgs* launch, int stride) {
+    InvertedResidualArgs& a = *launch;
     // Rows per strip, and tiles of channels per interval.  A strip expands the rows of its halo again, so few rows cost work;
     // many leave compute units idle, or LDS for one work-group only; many channels per interval mean few barriers, each
     // wavefront on channels of its own, and little left to share out where the strip is large.  The least of rounds x
@@ -438,7 +439,8 @@ int launch_inverted_residual(InvertedResidualArgs a, int stride, hipStream_t s) 
         }
     }
     if (best == 0) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: a row does not fit");
-    const int bytes = lay_out(a, stride, best, best_g), tiles = a.tiles_px * a.tiles_oc;
+    a.G = best_g;
+    a.lds = lay_out(a, stride, best, best_g);
     const int64_t blocks = (int64_t)a.strips * a.N;
     if (blocks >= (int64_t(1) << 28)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: 2^28 strips or more");
     a.blocks = (int32_t)blocks;
@@ -450,16 +452,20 @@ int launch_inverted_residual(InvertedResidualArgs a, int stride, hipStream_t s) 
     magic_divisor((uint32_t)a.x_chunks, &a.chunks_mul, &a.chunks_shift);
     magic_divisor((uint32_t)a.tiles_oc, &a.oct_mul, &a.oct_shift);
     magic_divisor((uint32_t)(a.pitch_o / 8), &a.blk_mul, &a.blk_shift);
-    const int per_wave = (tiles + kWaves - 1) / kWaves;
+    return CHX_HIP_OK;
+}
+
+int launch_inverted_residual(const InvertedResidualArgs& a, int stride, hipStream_t s) {
+    const int bytes = a.lds, per_wave = (a.tiles_px * a.tiles_oc + kWaves - 1) / kWaves;
     if (per_wave == 1) {
-        switch (best_g) {
+        switch (a.G) {
             case 1: return launch_steps<1, 1>(a, stride, bytes, s);
             case 2: return launch_steps<1, 2>(a, stride, bytes, s);
             case 4: return launch_steps<1, 4>(a, stride, bytes, s);
             default: return launch_steps<1, 8>(a, stride, bytes, s);
         }
     }
-    switch (best_g) {
+    switch (a.G) {
         case 1: return launch_steps<kMostTiles, 1>(a, stride, bytes, s);
         case 2: return launch_steps<kMostTiles, 2>(a, stride, bytes, s);
         case 4: return launch_steps<kMostTiles, 4>(a, stride, bytes, s);

@@ -25,7 +25,7 @@ def sum_code():
     return pkg.workloads.add_program(pkg.ops, (0.3, 128), (0.1, 7), (0.4, 120))
 
 
-@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "errors", "another_device", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "nothing_launched", "errors", "another_device", "instruction_by_instruction"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -138,6 +138,30 @@ def few_rows(host):
     """More than 256 channels out and fewer than 512 rows."""
     for channels, n, blocks in (((160, 960, 320), 64, 0), ((160, 960, 320), 74, 1), ((160, 960, 256), 1, 1), ((160, 960, 257), 1, 0)):
         assert one(host, program(host, channels, image=7), (n, channels[0], 7, 7)) == blocks
+
+
+def nothing_launched(host):
+    """What is refused has launched nothing: not the search for a sum's short form either."""
+    lib, capi, ref = host.lib, host.capi, ctypes.byref
+    keep, operands = [], []
+    for shape in ((96, 16, 1, 1), (96, 1, 3, 3), (257, 96, 1, 1)):
+        tensors = host.tensor("int8", shape), host.tensor("float32", shape[:1]), host.tensor("int8", shape[:1])
+        keep.append(tensors)
+        operands += [ctypes.addressof(t) for t in tensors] + [None]
+    block = ctypes.c_void_p()
+    host.check(lib.chx_hip_inverted_residual_create((ctypes.c_void_p * 12)(*operands), 1, None, ref(block)))
+    scales, zeros = (ctypes.c_float * 3)(0.2, 0.25, 0.3), (ctypes.c_int32 * 3)(0, 0, 128)
+
+    def run(n):
+        x, r, y = host.channels_last("uint8", (n, 16, 8, 8)), host.channels_last("uint8", (n, 257, 8, 8), 272), host.channels_last("uint8", (n, 257, 8, 8), 272)
+        host.clear()
+        rc = lib.chx_hip_inverted_residual_run(block, ref(x), ctypes.c_float(0.1), 7, scales, zeros, capi.UINT8, 0, ref(r), ctypes.c_float(0.15), 3,
+                                               ctypes.c_float(0.4), 120, 0, ref(y), None)
+        return rc, len(host.launches())
+
+    assert run(2) == (2, 0)  # CHX_HIP_EUNSUPPORTED: 16 rows for more than 256 channels
+    assert run(64) == (0, 2)  # the search and the block
+    assert run(64) == (0, 1)
 
 
 def errors(host):
