@@ -1752,7 +1752,7 @@ extern "C" int chx_hip_qlinear_matmul(
 // ---- inverted residual blocks ------------------------------------------------------------------
 
 struct chx_hip_inverted_residual {
-    int32_t channels = 0, expanded = 0, out_channels = 0, stride = 1;
+    int32_t channels = 0, out_channels = 0, stride = 1;
     bool has_bias = false, affine_residual = true;
     int device = 0;  // whose memory the operands are laid out in
     int tiles = 0, tiles_padded = 0, steps = 0, tiles_oc = 0;
@@ -1804,7 +1804,6 @@ extern "C" int chx_hip_inverted_residual_create(const chx_hip_conv_operands* sta
     std::unique_ptr<chx_hip_inverted_residual, void (*)(chx_hip_inverted_residual*)> p(new chx_hip_inverted_residual(), chx_hip_inverted_residual_destroy);
     CHX_HIP_CALL(hipGetDevice(&p->device));
     p->channels = (int32_t)w1.shape[1];
-    p->expanded = (int32_t)hid;
     p->out_channels = (int32_t)w3.shape[0];
     p->stride = stride;
     p->has_bias = stages[0].bias != nullptr;

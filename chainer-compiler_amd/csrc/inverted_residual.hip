@@ -293,13 +293,7 @@ __global__ __launch_bounds__(64 * kWaves, kTiles == 1 && kG <= 2 ? 4 : 2) void i
         float pre[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) pre[r] = (float)(acc[t][r] + s_add[oc + r]) * s_scale[oc + r];
-        const QuantProduct q = in_vector_registers(a.q3);
-        if (q.path == 2) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) pre[r] = quantize_prefloor_u8<2>(pre[r], q);
-        } else {
-            prefloor(pre, q);
-        }
+        prefloor(pre, in_vector_registers(a.q3));
         uint32_t word[4];
         floor_sat_u8x16(pre, word);
         v4i val = {(int)word[0], (int)word[1], (int)word[2], (int)word[3]};

@@ -55,7 +55,7 @@ struct ChainArgs {
     float x_inv_scale, x_largest;  // 1 / scale; 2^40 scale
     char* y;
     int64_t y_row;
-    int32_t y_is_float, y_signed;
+    int32_t y_is_float;
     float y_zpf, y_scale;
     int32_t M, layers;
 };
@@ -363,7 +363,6 @@ extern "C" int chx_hip_qlinear_chain(
     if (!g.y_is_float && y->dtype != dtype) return refuse("the type of y");
     g.y = static_cast<char*>(y->data);
     g.y_row = y->strides[0];
-    g.y_signed = dtype == CHX_HIP_INT8;
     g.y_zpf = (float)y_zero_point;
     g.y_scale = y_scale;
     matmul_chain_kernel<<<(unsigned)((g.M + kRows - 1) / kRows), 64 * kWaves, 0, as_stream(stream)>>>(g);
