@@ -1,5 +1,6 @@
 """Inverted residual blocks as one launch (csrc/inverted_residual.hip): whole networks, every block's output bit for bit
-against the oracle's convolutions and sums."""
+against the oracle's convolutions and sums; and single blocks with quantizations that no network here has."""
+import ctypes
 import importlib
 
 import numpy as np
@@ -54,10 +55,11 @@ def check(g, vm, oracle, model, keep, blocks):
 
 
 def block_outputs(model):
-    """The last value of every block: a sum, or the result of a projection that no sum reads."""
+    """The last value of every block: a sum, or the result of a projection that no sum follows."""
     program = model["program"]
-    read_by_sum = {v for ins in program if ins[0] in ("Add", "AddRelu") for v in ins[2:4]}
-    names = [ins[1] for ins in program if ins[0] == "Add"]
+    summed = {ins[2] for ins in program if ins[0] == "Add"}  # (the other operand is an earlier block's value)
+    names = [ins[1] for ins in program if ins[0] == "Add" or (ins[0] == "QLinearConv" and ins[3].endswith("_project") and ins[1] not in summed)]
+    assert len(names) == sum(ins[0] == "QLinearConv" and ins[3].endswith("_project") for ins in program)
     return names
 
 
@@ -94,3 +96,62 @@ def test_full_size(g, vm, oracle, batch):
     for name in got:
         np.testing.assert_array_equal(got[name][picks], ref[name], err_msg=name)
     prog.close()
+
+
+# N, channels (in, expanded, out), H, W, stride, x's type and zero point, the three results' zero points, scales per tensor, bias, sum
+# (0 none, 1, 2 with Relu), result stored as code - 128.  Odd images, padding with another zero point than 0, one pixel, several
+# tiles of channels out for a wavefront.
+BLOCKS = [
+    (2, (16, 96, 24), 9, 7, 1, np.uint8, 77, (13, 200, 128), False, True, 0, False),
+    (2, (16, 96, 24), 9, 7, 2, np.int8, -9, (13, 0, 5), True, False, 0, True),
+    (3, (40, 130, 33), 8, 11, 2, np.uint8, 0, (0, 255, 0), True, True, 0, False),
+    (1, (24, 72, 40), 5, 5, 1, np.int8, 100, (255, 9, 117), False, False, 1, False),
+    (2, (17, 33, 17), 6, 13, 1, np.uint8, 255, (128, 128, 3), True, False, 2, True),
+    (3, (64, 64, 64), 1, 1, 2, np.uint8, 4, (60, 61, 62), True, True, 1, False),
+    (75, (160, 96, 320), 7, 7, 1, np.uint8, 131, (31, 7, 90), True, True, 2, False),
+    (2, (96, 384, 256), 3, 50, 1, np.int8, 0, (0, 0, 128), False, True, 1, True),
+]
+
+
+@pytest.mark.parametrize("case", range(len(BLOCKS)))
+def test_single_blocks(g, oracle, case):
+    N, (cin, hid, cout), H, W, stride, x_type, x_zp, zero_points, per_tensor, bias, with_sum, minus_128 = BLOCKS[case]
+    from test_gpu_conv_split import codes, pitched
+    rng = np.random.default_rng(case)
+    lib, capi = g.capi.lib(), g.capi
+    x = codes(rng, (N, cin, H, W), x_type)
+    h, scale, zp = x, 0.02, x_zp
+    operands, kept, scales = [], [], []
+    for i, (shape, group, step, pad) in enumerate((((hid, cin, 1, 1), 1, 1, 0), ((hid, 1, 3, 3), hid, stride, 1), ((cout, hid, 1, 1), 1, 1, 0))):
+        w, n = codes(rng, shape, np.int8), 1 if per_tensor else shape[0]
+        ws, b = rng.uniform(0.002, 0.02, size=n).astype(np.float32), rng.integers(-3000, 3000, size=shape[0]).astype(np.int32) if bias else None
+        y_scale = np.float32(scale * ws.mean() * 74 * 74 * np.sqrt(np.prod(shape[1:])) / 60)
+        okw = dict(bias=b, bias_mode=oracle.BIAS_ONNX_INT32) if bias else {}
+        h = oracle.qlinear_conv_int(h, scale, zp, w, np.broadcast_to(ws, shape[:1]).copy(), np.zeros(shape[0], np.int8), y_scale, zero_points[i], np.uint8,
+                                    strides=(step, step), pads=(pad, pad), group=group, **okw)
+        assert len(np.unique(h)) > 20
+        kept += [g.dev(w), g.dev(ws), g.dev(np.zeros(n, np.int8))] + ([g.dev(b)] if bias else [])
+        descs = [capi.desc(t) for t in kept[-(4 if bias else 3):]]
+        kept += descs
+        operands += [ctypes.addressof(d) for d in descs] + ([] if bias else [None])
+        scales.append(y_scale)
+        scale, zp = y_scale, zero_points[i]
+    block = ctypes.c_void_p()
+    capi.check(lib.chx_hip_inverted_residual_create((ctypes.c_void_p * 12)(*operands), stride, capi.stream_ptr(), ctypes.byref(block)))
+    xd = pitched(x.shape, torch.uint8 if x_type == np.uint8 else torch.int8)
+    xd.copy_(g.dev(x))
+    y, rd = pitched(h.shape, torch.int8 if minus_128 else torch.uint8), None
+    r_scale, out_scale, out_zp, r_zp = np.float32(0.7 * scale), np.float32(1.6 * scale), 40, 21
+    if with_sum:
+        r = codes(rng, h.shape, np.uint8)
+        rd = pitched(h.shape, torch.uint8)
+        rd.copy_(g.dev(r))
+        total = oracle.binary(oracle.ADD, oracle.dequantize_linear(h, scale, zp), oracle.dequantize_linear(r, r_scale, r_zp))
+        h = oracle.quantize_linear(oracle.relu(total) if with_sum == 2 else total, out_scale, out_zp, np.uint8)
+    flags = (capi.BIAS_ONNX_INT32 if bias else 0) | (capi.STORE_MINUS_128 if minus_128 else 0)
+    capi.check(lib.chx_hip_inverted_residual_run(
+        block, capi.ref(xd), ctypes.c_float(0.02), x_zp, (ctypes.c_float * 3)(*scales), (ctypes.c_int32 * 3)(*zero_points), capi.UINT8, flags,
+        capi.ref(rd) if with_sum else None, ctypes.c_float(r_scale), r_zp, ctypes.c_float(out_scale), out_zp, int(with_sum == 2), capi.ref(y), capi.stream_ptr()))
+    got = g.host(y)
+    np.testing.assert_array_equal(got.view(np.uint8) ^ 0x80 if minus_128 else got, h)
+    lib.chx_hip_inverted_residual_destroy(block)
