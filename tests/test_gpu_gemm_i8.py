@@ -82,7 +82,7 @@ def test_views_into_larger_arrays(g):
         assert not y.any()
 
 
-# tiles of 128 x 128 of gemm_i8_stage_kernel, many and with remainders of each
+# tiles of 64 x 128 of gemm_i8_stage_kernel, many and with remainders of each
 LARGE = (4099, 2070, 1037)
 ROWS = sorted({0, 1, 30, 31, 32, 63, 64, 127, 128, 255, 256, 257, 1023, 2047, 4095, 4096, 4097, 4098})
 
