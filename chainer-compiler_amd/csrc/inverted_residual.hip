@@ -396,6 +396,34 @@ int launch_steps(const InvertedResidualArgs& a, int stride, int bytes, hipStream
     return a.KS == 1 ? launch<2, kTiles, kG, 1>(a, bytes, s) : a.KS == 3 ? launch<2, kTiles, kG, 3>(a, bytes, s) : launch<2, kTiles, kG, 5>(a, bytes, s);
 }
 
+// The two sides of whether the block is one launch, in us, fitted to 1,059 blocks of 8 to 160 channels, expanded 1 to 6 times, to 8 to
+// 320, on 1 to 128 images of 4 to 150, each measured both ways inside a recording (within 8 and 7 %).  A strip expands its halo
+// again: where LDS holds a row or two of a wide image at a time, or many channels leave, that costs more than the expanded
+// activations' way through memory.  us as three launches and as one: 54 x 8 -> 48 -> 80 at 86x86 46 and 83, 60 x 128 -> 768 -> 208 at 51x51
+// 161 and 290, 70 x 24 -> 144 -> 104 at 104x104 155 and 340; 126 x 16 -> 48 -> 8 at 99x99 75 and 129.  All as one launch were 0.92 of
+// the time of three on average, one in seven more than 5 % slower (up to 2.1 times); by this choice 0.89, nine of them, by up
+// to 20 %; of 400 others, six by up to 14 %.  All blocks of a MobileNetV2 on 1 to 128 images are one launch, but for what the refusal below names.
+double time_of_launches(const InvertedResidualArgs& a) {
+    auto pad = [](int64_t n, int64_t by) { return (double)((n + by - 1) / by * by); };
+    const int64_t channels = (int64_t)a.x_chunks * 16, hid = (int64_t)a.hid_tiles * 32;
+    const double in = 1e-6 * (double)a.N * a.H * a.W, out = 1e-6 * (double)a.N * a.OH * a.OW, h = (double)hid, oc = pad(a.OC, 16);
+    const double expansion = std::max(2.4e-3 * in * pad(channels, 64) * pad(hid, 64), 0.28 * in * h), projection = std::max(2.4e-3 * out * pad(hid, 64) * pad(a.OC, 64), 0.28 * out * oc);
+    return 11.6 + expansion + projection + in * (3.8 + 0.104 * h) + 0.50 * out * h;
+}
+
+double time_of_block(const InvertedResidualArgs& a, int64_t blocks) {
+    auto shares = [](int n, int by) { return (double)((n + by - 1) / by); };
+    const int per = kWaves / a.G, tiles = a.tiles_px * a.tiles_oc;
+    const double runs = shares(a.pixels / 32, per), items = shares((a.items + 1) / 2, per), mine = shares(tiles, kWaves), rows = (double)a.rows * a.W * a.x_chunks / 512.0;
+    const bool two = 2 * a.lds <= kLdsOfUnit && tiles <= kWaves && a.G <= 2 && blocks > 256;
+    const double rounds = two ? 1.2 * (blocks > 2048 ? blocks / 512.0 : (double)((blocks + 511) / 512)) : (double)((blocks + 255) / 256);
+    const double filled = 2.05 + 1e-3 * rounds * ((a.intervals + 2) * (944.0 + runs * (109.0 + 46.0 * a.KS) + 300.0 * items + 54.0 * mine * a.G) + 23.0 * rows + 92.0 * (mine + 1));
+    if (blocks > 256) return filled;
+    // one round: the start is most of it
+    const double start = 6.7 + 1e-3 * ((a.intervals + 2) * (76.0 + 58.0 * runs * a.KS + 349.0 * items) + 348.0 * (mine + 1));
+    return start > 13.0 && filled > start ? 0.65 * start + 0.35 * filled : start;
+}
+
 }  // namespace
 
 int plan_inverted_residual(InvertedResidualArgs* launch, int stride) {
@@ -437,6 +465,8 @@ int plan_inverted_residual(InvertedResidualArgs* launch, int stride) {
     a.lds = lay_out(a, stride, best, best_g);
     const int64_t blocks = (int64_t)a.strips * a.N;
     if (blocks >= (int64_t(1) << 28)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: 2^28 strips or more");
+    const double launches = time_of_launches(a);  // (up to 16 us most of it is that they are three)
+    if (time_of_block(a, blocks) > (launches < 16.0 ? launches + 2.3 : 0.93 * launches + 1.0)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: slower than its convolutions");
     a.blocks = (int32_t)blocks;
     a.xcd_chunk = (int32_t)((blocks + 7) / 8);
     magic_divisor((uint32_t)a.strips, &a.strips_mul, &a.strips_shift);

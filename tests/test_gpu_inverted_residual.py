@@ -109,7 +109,7 @@ BLOCKS = [
     (2, (17, 33, 17), 6, 13, 1, np.uint8, 255, (128, 128, 3), True, False, 2, True),
     (3, (64, 64, 64), 1, 1, 2, np.uint8, 4, (60, 61, 62), True, True, 1, False),
     (75, (160, 96, 320), 7, 7, 1, np.uint8, 131, (31, 7, 90), True, True, 2, False),
-    (2, (96, 384, 256), 3, 50, 1, np.int8, 0, (0, 0, 128), False, True, 1, True),
+    (2, (96, 384, 256), 5, 9, 1, np.int8, 0, (0, 0, 128), False, True, 1, True),
 ]
 
 

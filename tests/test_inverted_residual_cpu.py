@@ -25,7 +25,7 @@ def sum_code():
     return pkg.workloads.add_program(pkg.ops, (0.3, 128), (0.1, 7), (0.4, 120))
 
 
-@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "nothing_launched", "errors", "another_device", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_blocks", "sums", "values_read_twice", "frees_between", "refused_forms", "few_rows", "slower_blocks", "nothing_launched", "errors", "another_device", "instruction_by_instruction"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -138,6 +138,14 @@ def few_rows(host):
     """More than 256 channels out and fewer than 512 rows."""
     for channels, n, blocks in (((160, 960, 320), 64, 0), ((160, 960, 320), 74, 1), ((160, 960, 256), 1, 1), ((160, 960, 257), 1, 0)):
         assert one(host, program(host, channels, image=7), (n, channels[0], 7, 7)) == blocks
+
+
+def slower_blocks(host):
+    """Blocks whose strips are a row or two of a wide image, or whose halo costs more than it saves, run as three launches."""
+    for n, channels, image, stride, blocks in ((70, (24, 144, 104), 104, 1, 0), (54, (8, 48, 80), 86, 1, 0), (60, (128, 768, 208), 51, 1, 0), (126, (16, 48, 8), 99, 1, 0),
+                                               (1, (152, 912, 208), 64, 2, 0), (10, (160, 960, 160), 56, 1, 0), (128, (16, 96, 24), 112, 2, 1), (128, (24, 144, 24), 56, 1, 1),
+                                               (32, (24, 144, 32), 56, 2, 1), (128, (96, 576, 160), 14, 2, 1), (1, (160, 960, 160), 7, 1, 1)):
+        assert one(host, program(host, channels, stride=stride, image=image, batch=n), (n, channels[0], image, image)) == blocks, (n, channels, image)
 
 
 def nothing_launched(host):
