@@ -30,6 +30,7 @@ namespace chx {
 namespace {
 
 constexpr int kWaves = 16, kRows = 16;
+// (the codes and sums of a work-group then are 49.7 KB, below the 64 KB that a kernel has without asking; 1024 columns would be 82 KB)
 constexpr int kMaxLayers = 6, kMaxK = 1024, kMaxN = 512;
 constexpr int kActRow = kMaxK + 16, kSumRow = kMaxN + 4;  // (off a multiple of the LDS banks)
 constexpr int kDepth = 8;                                 // fragments of weights in flight per wavefront
@@ -252,6 +253,24 @@ bool is_rows(const chx_hip_tensor& t) {
     return t.ndim == 2 && (t.shape[1] == 1 || t.strides[1] == es) && t.strides[0] >= 0 && t.strides[0] % es == 0 && aligned(t.data, (size_t)es);
 }
 
+// Above 8192 rows every compute unit has a third work-group to begin with, and narrow layers are faster as launches that fill the
+// chip at once.  Both times in us, fitted to 305 networks of one to six layers, 8 to 512 columns and 4,096 to 16,384 rows, measured both ways inside
+// a recording (within 5 and 12 %).  All of them as chains were 0.82 of the time of single calls on average, but 28 slower by more than 5 %
+// (15797 x 1005 -> 32 -> 107 codes 23.2 and 34.6 us, 16033 x 148 -> 44 -> 44 20.4 and 25.2); by this choice 0.84, and by at most 5 %.
+bool slower_in_rounds(const ChainArgs& g) {
+    if (g.M <= 8192) return false;
+    const double rounds = (double)((g.M + 256 * kRows - 1) / (256 * kRows)), million_rows = 1e-6 * g.M;
+    const int32_t K = g.layer[0].K, N = g.layer[g.layers - 1].N;
+    double chain = 0.47 + (g.x_is_float ? 0.615 * ((K + 255) / 256) : 0.149 * ((K + 63) / 64));
+    double single = (g.x_is_float + g.y_is_float) * 2.82 + million_rows * (0.49 * K + (g.x_is_float ? 0.80 * K : 0.0) + (g.y_is_float ? 0.12 * N : 0.0));
+    for (int i = 0; i < g.layers; ++i) {
+        const ChainLayer& L = g.layer[i];
+        chain += 0.342 + 0.085 * (L.slices > 1 ? L.per : L.per * L.steps) + 0.943 * ((L.N + 255) / 256);
+        single += 4.45 + million_rows * (3.68e-3 * L.K * L.N + 1.69 * L.N);
+    }
+    return 3.44 + rounds * chain + 0.308 * million_rows * N * (g.y_is_float ? 4 : 1) > 0.9 * single;
+}
+
 }  // namespace
 }  // namespace chx
 
@@ -306,12 +325,13 @@ extern "C" int chx_hip_qlinear_chain(
     };
     if (n > kMaxLayers) return refuse("too many layers");
     if (!is_rows(*x) || !is_rows(*y) || x->shape[0] < 1) return refuse("operands that are not rows");
-    // One work-group a compute unit up to 4096 rows.  us for the whole network on this kernel / as single calls, by rows:
-    //                                         32             256            4096           16384
+    // One work-group a compute unit up to 4096 rows; one after the other beyond.  us for the whole network on this kernel / as single
+    // calls, by rows:                         32             256            4096           16384
     //    784 -> 100 -> 100 -> 10            8.9 / 17.0      9.0 / 17.8     9.3 / 22.8    33.0 / 37.2
     //    1024 -> 512 -> 512 -> 100         13.5 / 17.8     13.7 / 18.9    16.3 / 34.1    57.2 / 65.4
     //    1024 -> 512                        9.7 / 10.9      9.9 / 11.1    13.5 / 21.0    45.5 / 46.7
     //    six layers of 512                 22.7 / 30.8     22.9 / 32.6    26.8 / 53.4    92.9 / 115
+    // (and see slower_in_rounds)
     if (x->shape[0] > 16384) return refuse("too many rows");
     int device = 0;
     CHX_HIP_CALL(hipGetDevice(&device));
@@ -365,6 +385,7 @@ extern "C" int chx_hip_qlinear_chain(
     g.y_row = y->strides[0];
     g.y_zpf = (float)y_zero_point;
     g.y_scale = y_scale;
+    if (slower_in_rounds(g)) return refuse("slower than its layers for so many rows");
     matmul_chain_kernel<<<(unsigned)((g.M + kRows - 1) / kRows), 64 * kWaves, 0, as_stream(stream)>>>(g);
     return launch_check("matmul_chain_kernel");
 }

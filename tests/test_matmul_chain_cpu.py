@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "frees_in_front", "refused_forms", "errors", "another_device", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["whole_networks", "values_read_twice", "frees_between", "frees_in_front", "refused_forms", "many_rows", "errors", "another_device", "instruction_by_instruction"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -93,10 +93,10 @@ def frees_between(host):
 
 def frees_in_front(host):
     """A chain without a QuantizeLinear in front gives back its input: the Free of it stands in front of the chain's first instruction."""
-    # six layers, two layers, and a QuantizeLinear whose result (1 MB) takes the place of what lies between the two chains
-    p = program(host, (64,) * 9, rows=16384, free=True, quantized_again=True)
-    assert kernels(host, p, (16384, 64)) == [CHAIN, CHAIN, QUANTIZE]
-    assert host.log().count("hipMalloc %d" % (16384 * 64)) == 1
+    # six layers, two layers, and a QuantizeLinear whose result (512 KB) takes the place of what lies between the two chains
+    p = program(host, (64,) * 9, rows=8192, free=True, quantized_again=True)
+    assert kernels(host, p, (8192, 64)) == [CHAIN, CHAIN, QUANTIZE]
+    assert host.log().count("hipMalloc %d" % (8192 * 64)) == 1
 
 
 def refused_forms(host):
@@ -104,6 +104,15 @@ def refused_forms(host):
     assert kernels(host, program(host, (1025, 64, 32)), (8, 1025)) == [QUANTIZE, PRODUCT, CHAIN]
     assert kernels(host, program(host, (96, 513, 32)), (8, 96)) == [QUANTIZE, PRODUCT, CHAIN]
     assert kernels(host, program(host, (96, 64, 513)), (8, 96)) == [CHAIN, PRODUCT, DEQUANTIZE]
+
+
+def many_rows(host):
+    """Above 8192 rows narrow layers are launches of their own."""
+    for dims, rows, chain in (((1005, 32, 107), 15797, False), ((1005, 32, 107), 8192, True), ((784, 100, 100, 10), 16384, True), ((1024, 512, 512, 100), 16384, True),
+                              ((512,) * 7, 16384, True), ((64, 512, 16), 16385, False)):
+        codes = dims[0] == 1005
+        p = program(host, dims, rows=rows, quantize=not codes, dequantize=not codes)
+        assert (CHAIN in kernels(host, p, (rows, dims[0]), "uint8" if codes else "float32")) == chain, (dims, rows)
 
 
 def errors(host):
