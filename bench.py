@@ -137,6 +137,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
     # The timed region replays the whole program as one HIP graph (about 125 launches per step
     # would otherwise be bound by the host); --no-graph launches every op from the host instead.
     vm_prog = vm_replay = None
+    fused_blocks = 0  # of the timed recording: inverted residual blocks as one launch
     use_vm = args.runner == "chxvm" and args.parts <= 1 and fuse
     if use_vm:
         # the drop-in itself: the network as one serialized program in the C++ VM
@@ -151,6 +152,9 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
                 vm_prog.run({"x": x})
             sec = timed_steps(torch, step, args.steps, args.warmup)
         else:
+            fused_blocks = vm.counter("inverted_residuals")
+            vm_prog.run({"x": x})
+            fused_blocks = vm.counter("inverted_residuals") - fused_blocks
             vm_replay = vm_prog.capture({"x": x})
             stream = capi.stream_ptr()
             sec = timed_steps(torch, lambda _t: vm_replay.launch(stream), args.steps, args.warmup)
@@ -162,7 +166,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
 
     # Launch duration of the dominant kernel: event pairs cannot be recorded inside a graph
     # replay, and around single 10-60 us launches they mostly measure submission gaps.  So the
-    # QLinearConv instructions of the program (for MobileNetV2: the depthwise ones) are recorded,
+    # QLinearConv instructions of the program (for MobileNetV2: the depthwise ones; see the label) are recorded,
     # in program order and on the buffers of the step just timed, into a graph of their own;
     # that graph is replayed REP times between one event pair on the launch stream.  Every layer
     # then finds its input where the timed step leaves it (written many launches earlier, not
@@ -219,7 +223,8 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
     layer_graphs.append(idle)
     if mobilenet:
         achieved = model["depthwise_bytes"] / (conv_ms_per_step * 1e-3) / 1e9
-        roofline = dict(bound="hbm", kernel="depthwise3x3_kernel (%d launches per step, summed)" % n_launch,
+        roofline = dict(bound="hbm", kernel="depthwise3x3_kernel (%d launches of the runner that launches op by op, summed; the timed recording has %d of the blocks "
+                        "as one inverted_residual_kernel each)" % (n_launch, fused_blocks),
                         achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS, traffic=None,
                         bytes_per_step=model["depthwise_bytes"], kernel_ms_per_step=conv_ms_per_step)
     else:

@@ -17,7 +17,7 @@
 // With several taps a tile's pixels are gathered once per tap, 32 or 64 bytes from a pixel at a time: nine times 32 x 256
 // bytes for what lies in 62 x 256.  Where the results have the image's own size those taps fall on one run of pixels of the
 // dense image, and kPatch brings that run into LDS, once, while the weights of up to nine steps are on their way; a step then
-// is weights from memory and a 16-byte LDS read per lane, pixels an odd number of 16 bytes apart (no bank conflicts), taps
+// is weights from memory and a 16-byte LDS read per lane, pixels an odd number of 16 bytes apart, taps
 // outside the image read 64 bytes of zero point.  In us, best tile with the pixels from memory and from LDS, launches
 // back to back with weights of their own, 3x3 filters: one image, 512 channels at 7x7 8.5 and 5.9, 256 at 14x14 5.4 and 4.6,
 // 128 at 28x28 4.8 and 4.3, 64 at 56x56 3.9 and 4.4; eight images, 11.9 and 7.9, 9.8 and 6.8, 7.1 (staged tiles) and 8.2,
@@ -368,7 +368,7 @@ constexpr int partial_bytes(int R, int PN, int W) {
     return W > 1 ? W * PN * (R * R / 256) * 1024 : 0;
 }
 
-int patch_pitch(const ConvMfmaArgs& a) {  // an odd number of 16 bytes: no bank conflicts
+int patch_pitch(const ConvMfmaArgs& a) {  // an odd number of 16 bytes: neighbouring pixels on different banks (1.5 to 2 conflict cycles per LDS instruction are left)
     return a.C16 % 32 == 0 ? a.C16 + 16 : a.C16;
 }
 

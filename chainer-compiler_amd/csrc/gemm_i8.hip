@@ -342,7 +342,7 @@ __device__ __forceinline__ v2i transposed8(const char* p) {
 // Tile of 64 kRW rows x 64 kCW columns per work-group of eight wavefronts; kKW of them share out the K of a stage (128, or 256
 // with eight).  Every thread brings 16 bytes of a row of a and 16 of a row of b at a time, coalesced and once per work-group,
 // into one of two stages in LDS, one barrier per stage.  A fragment of a is a 16-byte read (rows an odd number of 16
-// bytes apart: no bank conflicts); one of b, whose rows run along n, comes out of ds_read_b64_tr_b8 transposed, without a vector
+// bytes apart; 0.1 to 0.4 conflict cycles per LDS instruction in all); one of b, whose rows run along n, comes out of ds_read_b64_tr_b8 transposed, without a vector
 // instruction (b transposed: like a).  b is the first operand of the MFMA, so that a lane ends with four
 // neighbouring results of a row.
 //

@@ -10,7 +10,8 @@
 // 28x28 14.2 and 7.2, 18.0 and 10.8, 37.4 and 20.4; 64 -> 384 -> 64 at 14x14 14.0 and 7.8, 17.0 and 9.1, 24.5 and 16.9;
 // 160 -> 960 -> 160 at 7x7 13.9 and 12.7, 15.7 and 13.7, 30.3 and 17.1.
 //
-// What bounds it is vector instructions: 5 per requantized value (conversion, scale, two multiply-adds, conversion), 4.5
+// What bounds it is vector instructions (their pipeline is 0.8 full on 128 images of 112x112 and 56x56; 0.4 at 7x7, where a work-group has the compute unit
+// alone and waits at its barriers): 5 per requantized value (conversion, scale, two multiply-adds, conversion), 4.5
 // dot products and shifts per depthwise result, so the layouts are chosen to need none for moving data:
 //  * Expansion: the pixels are the rows of the MFMA, so that a lane holds one channel, its scale and its zero point's
 //    share for the whole interval, and, with the pixels in the order of pixel_of(), sixteen neighbouring pixels: one
@@ -20,8 +21,8 @@
 //    results two read an aligned dword (against the filter row, or the filter row moved up by a byte), two a shifted one.
 //  * Projection: its operand is wanted [pixel][channel]: ds_read_b64_tr_b8 transposes 8 x 16 bytes on the way from LDS.
 //  * The projection's filters are permuted so that a lane ends with sixteen neighbouring channels of a pixel: one store.
-// The input strip lies in LDS with pixels an odd number of 16 bytes apart, channels of the other buffers likewise (no bank
-// conflicts).  All results are those of the three convolutions and the sum, bit for bit: exact int32 sums, the same
+// The input strip lies in LDS with pixels an odd number of 16 bytes apart, channels of the other buffers likewise, so that 16-byte accesses keep
+// off each other's banks (the depthwise part's dwords share a fourth of them: 3.5 to 6.7 conflict cycles per LDS instruction in all).  All results are those of the three convolutions and the sum, bit for bit: exact int32 sums, the same
 // requantization (quant_math.h) and the same sum of codes (conv_device.h).
 #include <algorithm>
 #include <cstring>
