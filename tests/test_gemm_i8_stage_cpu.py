@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k"])
+@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k", "large"])
 def test_case(host_so, case):
     from test_gpu_gemm_i8_stage import SHAPES
     host_hip.run_case(host_so, __file__, case, SHAPES=repr(SHAPES))
@@ -66,6 +66,19 @@ def short_k(host):
     assert "split" in product(host, 100352, 192, 256) and "split" in product(host, 8192, 192, 8192)
     assert "stage" in product(host, 8192, 384, 1024) and "stage" in product(host, 33449, 192, 1044)
     assert "stage" in product(host, 8192, 256, 1024) and "stage" in product(host, 8192, 192, 8192, transposed=True)
+
+
+def large(host):
+    """Operands that leave the caches, for which the times behind the choice would name the split kernel."""
+    def codes(M, K, N):
+        a, b, y = host.tensor("uint8", (M, K)), host.tensor("int8", (K, N)), host.tensor("uint8", (M, N))
+        host.clear()
+        scale = ctypes.c_float
+        host.check(host.lib.chx_hip_qlinear_matmul(ctypes.byref(a), scale(0.02), 128, ctypes.byref(b), scale(0.005), 0, scale(0.04), 128, None, 0, ctypes.byref(y), None))
+        return host.launches()[0]
+
+    for shape in ((27015, 4416, 3968), (13507, 5184, 6528), (12686, 3152, 6208), (65536, 768, 128)):
+        assert "gemm_i8_stage_kernel" in codes(*shape) and "gemm_i8_stage_kernel" in product(host, *shape), shape
 
 
 if __name__ == "__main__":
