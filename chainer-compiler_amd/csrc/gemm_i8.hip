@@ -365,9 +365,10 @@ struct StageShape {
     static constexpr int kLds = 2 * kStage > kParts + (kKW + 1) * (kRows + kCols) * 4 ? 2 * kStage : kParts + (kKW + 1) * (kRows + kCols) * 4;
 };
 
-// (launch bounds: 128 registers)
-template <bool kBT, int kRW, int kCW, int kKW>
-__global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(GemmI8Args g) {
+// kShort: rows of b of 4 to 15 bytes (b not transposed).  The 16 bytes that are read of a row reach into the rows behind it, whose share of the result is
+// stored nowhere; the last rows are read as the last 16 bytes of b and shifted.
+template <bool kBT, int kRW, int kCW, int kKW, bool kShort>
+__device__ __forceinline__ void stage_product(const GemmI8Args& g) {
     using S = StageShape<kBT, kRW, kCW, kKW>;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tile = tile_of_block(g);
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
     uint32_t a_off[S::kAChunks], b_off[S::kBChunks];  // (the launcher has seen that they fit)
 #pragma unroll
     for (int c = 0; c < S::kAChunks; ++c) a_off[c] = (uint32_t)min((tid + c * S::kThreads) / kAPerRow, g.M - 1 - m0) * (uint32_t)g.a_row + tid % kAPerRow * 16;
-    const int b_n = n0 + tid % kBPerRow * 16, b_from = min(b_n, g.N - 16);
+    const int b_n = n0 + tid % kBPerRow * 16, b_from = kShort ? 0 : min(b_n, g.N - 16);
     // the bytes by which a chunk that reaches past the end of its row is read too early (16 and more: it is past the end whole)
     const int b_shift = kBT ? 0 : b_n - b_from;
 #pragma unroll
@@ -398,7 +399,10 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
         const int i = (tid + c * S::kThreads) / kBPerRow;
         b_off[c] = kBT ? (uint32_t)min(i, g.N - 1 - n0) * (uint32_t)g.b_ld + tid % kBPerRow * 16 : (uint32_t)i * (uint32_t)g.b_ld + b_from;
     }
-    const bool ragged = !kBT && n0 + S::kCols > g.N;
+    const bool ragged = !kBT && !kShort && n0 + S::kCols > g.N;
+    // the bytes by which the 16 of row k would pass the end of b
+    const int64_t b_bytes = (int64_t)(g.K - 1) * g.b_ld + g.N;
+    auto past_b = [&](int k) { return (int)max(min(k, g.K - 1) * g.b_ld + 16 - b_bytes, (int64_t)0); };
     const int a_k = tid % kAPerRow * 16, b_k = kBT ? tid % kBPerRow * 16 : tid / kBPerRow;
 
     struct Stage {
@@ -416,6 +420,7 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
             const char* p = from_b + b_off[c];
             if (kTail && kBT && k + 16 > g.K) p -= k + 16 - g.K;
             if (kTail && !kBT && k >= g.K) p -= (k + 1 - g.K) * g.b_ld;
+            if (kShort) p -= past_b(k);
             s.b[c] = *reinterpret_cast<const v4i_u*>(p);
         }
 #pragma unroll
@@ -439,6 +444,10 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
                 *reinterpret_cast<v4i*>(sb + i / kBPerRow * S::kBPitch + b_k) = v;
             } else {
                 if (ragged && b_shift > 0 && b_shift < 16) v = shift_down(v, b_shift);
+                if (kShort) {
+                    const int past = past_b(k0 + i / kBPerRow);
+                    if (past > 0) v = shift_down(v, past);
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = kTail && k0 + i / kBPerRow >= g.K ? 0 : v[e] ^ (int)g.b_flip;
                 *reinterpret_cast<v4i*>(sb + i / kBPerRow * S::kBPitch + i % kBPerRow * 16) = v;
@@ -513,12 +522,12 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
     if (full > 0) {
         load(no_tail(), 0, held);
         for (int s = 0; s + 1 < full; ++s) {
-            share(no_tail(), 0, s & 1, held);
+            share(no_tail(), s, s & 1, held);
             load(no_tail(), s + 1, held);
             __syncthreads();
             multiply(s & 1);
         }
-        share(no_tail(), 0, (full - 1) & 1, held);
+        share(no_tail(), full - 1, (full - 1) & 1, held);
         if (rest) load(tail(), full, held);
         else load_columns();
         __syncthreads();
@@ -593,6 +602,17 @@ __global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(
     finish(std::integral_constant<int, 1>());
 }
 
+// (launch bounds: 128 registers)
+template <bool kBT, int kRW, int kCW, int kKW>
+__global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_kernel(GemmI8Args g) {
+    stage_product<kBT, kRW, kCW, kKW, false>(g);
+}
+
+template <int kRW, int kCW, int kKW>
+__global__ __launch_bounds__(64 * kRW * kCW * kKW, 4) void gemm_i8_stage_short_kernel(GemmI8Args g) {
+    stage_product<false, kRW, kCW, kKW, true>(g);
+}
+
 template <bool kBT, int kRW, int kCW, int kKW>
 int launch_stage(const GemmI8Args& g, dim3 grid, hipStream_t s) {
     using S = StageShape<kBT, kRW, kCW, kKW>;
@@ -600,6 +620,14 @@ int launch_stage(const GemmI8Args& g, dim3 grid, hipStream_t s) {
         CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_i8_stage_kernel<kBT, kRW, kCW, kKW>), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds));
     gemm_i8_stage_kernel<kBT, kRW, kCW, kKW><<<grid, S::kThreads, S::kLds, s>>>(g);
     return launch_check("gemm_i8_stage_kernel");
+}
+
+template <int kRW, int kCW, int kKW>
+int launch_stage_short(const GemmI8Args& g, dim3 grid, hipStream_t s) {
+    using S = StageShape<false, kRW, kCW, kKW>;
+    CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_i8_stage_short_kernel<kRW, kCW, kKW>), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds));
+    gemm_i8_stage_short_kernel<kRW, kCW, kKW><<<grid, S::kThreads, S::kLds, s>>>(g);
+    return launch_check("gemm_i8_stage_short_kernel");
 }
 
 template <int R, int W>
@@ -723,6 +751,13 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
             return b_transposed ? launch_stage<true, 1, 1, 8>(g, grid(), s) : launch_stage<false, 1, 1, 8>(g, grid(), s);
         }
         (void)tiles(small ? 16 : 32, small ? 64 : 128);
+    }
+    // Fewer than 16 columns, which the choice above leaves out, and a compute unit for every 256 rows: the split kernel reads (and transposes) b for every 32
+    // rows of a.  us there and in tiles of 128 x 64: 110767 x 3583 x 15 404 and 117, 181346 x 907 x 15 129 and 44, 304796 x 2322 x 6 to codes 517 and 166; with b transposed
+    // 229322 x 1723 x 8 to codes 310 and 105, 359525 x 2641 x 4 739 and 253.
+    if (!m.lds_64k && m.N >= 4 && m.N < 16 && m.K >= 768 && ((m.M + 255) / 256) * batch >= 256 && m.a_row >= 0 && m.a_row < (int64_t(1) << 24) && (b_transposed ? b_ld < (int64_t(1) << 24) : b_ld >= m.N)) {
+        (void)tiles(128, 64);
+        return b_transposed ? launch_stage<true, 2, 1, 4>(g, grid(), s) : launch_stage_short<2, 1, 4>(g, grid(), s);
     }
     if (small) {
         if (w == 1) launch_split<16, 1>(g, b_transposed, grid(), s);

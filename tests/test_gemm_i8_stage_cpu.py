@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k", "large"])
+@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k", "large", "few_columns"])
 def test_case(host_so, case):
     from test_gpu_gemm_i8_stage import SHAPES
     host_hip.run_case(host_so, __file__, case, SHAPES=repr(SHAPES))
@@ -79,6 +79,12 @@ def large(host):
 
     for shape in ((27015, 4416, 3968), (13507, 5184, 6528), (12686, 3152, 6208), (65536, 768, 128)):
         assert "gemm_i8_stage_kernel" in codes(*shape) and "gemm_i8_stage_kernel" in product(host, *shape), shape
+
+
+def few_columns(host):
+    assert "stage_short" in product(host, 65281, 768, 15) and "stage_short" in product(host, 65281, 768, 4) and "stage_short" in product(host, 65281, 1000, 8, b_strides=[20, 1])
+    assert "split" in product(host, 65280, 768, 15) and "split" in product(host, 65281, 767, 15) and "split" in product(host, 65281, 768, 3)
+    assert "gemm_i8_stage_kernel<true, 2, 1, 4>" in product(host, 65281, 768, 8, transposed=True) and "split" in product(host, 65281, 768, 8, b_strides=[7, 1])  # (rows that overlap)
 
 
 if __name__ == "__main__":

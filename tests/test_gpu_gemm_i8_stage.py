@@ -71,3 +71,25 @@ def test_batches(g):
     got = g.host(g.ops.MatMulInteger(g.dev(a), g.dev(b), g.dev(np.array(9, np.uint8)), g.dev(np.array(-5, np.int8))))
     want = np.matmul(a[:, ::37].astype(np.float64) - 9, b.astype(np.float64) + 5).astype(np.int32)
     np.testing.assert_array_equal(got[:, ::37], want)
+
+
+# rows of b of 4 to 15 bytes, whole stages of 128 and a rest; rows next to each other, 9 bytes apart, b transposed (1)
+@pytest.mark.parametrize("M,K,N", [(65300, 768, 4), (65281, 1023, 15), (65408, 1280, 10), (65285, 897, 7)])
+@pytest.mark.parametrize("apart", [0, 1, 9])
+def test_few_columns(g, oracle, M, K, N, apart):
+    rng = np.random.default_rng(K + N + apart)
+    a, b = codes(rng, (M, K), np.uint8), codes(rng, (K, N), np.int8)
+    rows = rows_of(M)
+    bd = torch.zeros(K * (N + apart) - apart, dtype=torch.int8, device="cuda").as_strided((K, N), (N + apart, 1))  # ends with its last element
+    bd.copy_(g.dev(b))
+    if apart == 1:
+        bd = g.dev(np.ascontiguousarray(b.T)).t()
+    for az, bz in [(128, np.asarray(0)), (7, rng.integers(-90, 90, size=N))]:
+        got = g.ops.MatMulInteger(g.dev(a), bd, g.dev(np.asarray(az, np.uint8)), g.dev(bz.astype(np.int8)))
+        want = np.matmul(a[rows].astype(np.float64) - az, b.astype(np.float64) - bz).astype(np.int64).astype(np.int32)  # (exact: below 2^53)
+        np.testing.assert_array_equal(g.host(got)[rows], want)
+        flip = g.ops.MatMulInteger(g.dev(np.ascontiguousarray(a[::-1])), bd, g.dev(np.asarray(az, np.uint8)), g.dev(bz.astype(np.int8)))
+        assert torch.equal(flip.flip(0), got)
+    bias, s_y = rng.integers(-3000, 3000, size=N).astype(np.int32), float(0.02 * 0.005 * 74 * 74 * np.sqrt(K) / 32)
+    got = g.host(g.ops.QLinearMatMul(g.dev(a), 0.02, 117, bd, 0.005, 4, s_y, 128, g.dev(bias)))
+    np.testing.assert_array_equal(got[rows], oracle.qlinear_matmul_int(a[rows], 0.02, 117, b, 0.005, 4, s_y, 128, bias=bias))
