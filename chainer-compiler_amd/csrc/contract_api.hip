@@ -1518,22 +1518,28 @@ extern "C" void chx_hip_qconv_plan_destroy(chx_hip_qconv_plan* plan) {
 
 namespace chx {
 namespace {
+double padded(int64_t n, int64_t by) {
+    return (double)((n + by - 1) / by * by);
+}
+
 // Whether a ConvInteger with 1x1 filters that could be a product is one of those for which another kernel is faster, as far as
-// that kernel takes it.  Measured on 1,380 calls drawn from 8 to 2048 channels in and out, images of 4 to 112, 2^23 to 2^36
-// multiply-adds, in us, there and as a product:
-//  * planar, fewer columns than three quarters of a tile of 128 and enough tiles that this counts (in steps of 32 channels): 51 x 216
-//    -> 1336 channels at 7x7 15.8 and 21.4, 64 x 512 -> 2048 30.6 and 43.3; few tiles (8 x 1016 -> 664) 13.3 and 10.7, 11x11 19.8 and 8.5;
-//  * planar, few channels in, many results, rows that do not start at lines of 128 bytes, whose parts two tiles then write: 246 x
-//    32 -> 200 at 35x35 55.7 and 87.4, 10 x 32 -> 728 at 97x97 55.4 and 93.2; at 56x56 (whole lines) 84.4 and 54.9 for 230 x 32 -> 104;
-//  * channels-last with strides, fewer filters than 0.3 of the channels and one launch (conv_strip.hip): 21 x 176 -> 16 at 34x34 8.7 and 11.5, 55 x 672 -> 80
-//    at 5x5 11.2 and 19.2; more filters (10 x 136 -> 320 at 24x24, 11.6 and 8.4) gain by the product, by 14 % on average;
-//  * channels-last with strides and rows of no more than half a tile of 16, by what the two kernels' work comes to: 64 x 1024 -> 2048
+// that kernel takes it.
+//  * Planar: a product is padded to tiles of 128 columns of an image and of 32 filters, and where rows do not start at lines of 128 bytes two tiles
+//    write parts of one.  Both times in us, fitted to 346 calls of 16 to 2048 channels in, 8 to 2048 out and images of 4 to 80, measured both ways (within
+//    20 and 15 %).  All as products were 0.67 of the others' time on average and 46 slower by more than 5 % (up to 3.1 times: 73 x 1640 -> 960 at 5x5 26
+//    and 80); by this choice 0.65, six of them, by up to 10 % (of 600 others, planar and not, one, 70 x 672 -> 72 at 5x5: 10.3 and 14.0).
+//  * Channels-last with strides, fewer filters than 0.3 of the channels and one launch (conv_strip.hip), in us there and as a product: 21 x 176 -> 16 at 34x34 8.7 and
+//    11.5, 55 x 672 -> 80 at 5x5 11.2 and 19.2; more filters (10 x 136 -> 320 at 24x24, 11.6 and 8.4) gain by the product, by 14 % on average.
+//  * Channels-last with strides and rows of no more than half a tile of 16, by what the two kernels' work comes to: 64 x 1024 -> 2048
 //    at 7x7 84 and 130, 62 x 544 -> 1312 at 4x4 22.1 and 32.6; 135 x 552 -> 304 at 7x7 61.3 and 27.6.
 bool faster_than_product(const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a, bool channels_last) {
     const int64_t C = a.C, OC = cs.OC, columns = (int64_t)cs.OH * cs.OW;
     if (!channels_last) {
-        if (columns <= 96) return (int64_t)cs.N * ((OC + 31) / 32) * ((C + 31) / 32) > 9000;
-        return C <= 112 && OC >= 200 && columns % 32 != 0 && (int64_t)a.total > 16000000;
+        const double N = cs.N, pixels = N * columns, filters = padded(OC, 32), channels = padded(C, 32), results = 4e-6 * (double)a.total;
+        const double product = 4.7 + N * padded(columns, 128) * filters * (3.41e-9 * channels + 0.165e-6) + (columns % 32 == 0 ? 0.044 : 0.121) * results;
+        const double other = 6.9 + pixels * (0.737e-9 * filters * channels + 0.432e-6 * C) + 0.126 * results + 0.541e-6 * N * C * padded(columns, 64) + 2.7e-6 * OC * C +
+                             0.313e-6 * N * ((cs.OW + 3) / 4) * cs.OH * filters * ((C + 31) / 32);
+        return product > 0.88 * other;
     }
     if ((p.stride_h == 1 && p.stride_w == 1) || p.stride_h != p.stride_w || p.stride_h > 2) return false;
     if (conv_strip_takes(a)) return 10 * OC <= 3 * C;
@@ -1541,6 +1547,22 @@ bool faster_than_product(const chx_hip_conv_params& p, const ConvShape& cs, cons
     const double steps = (double)cs.N * cs.OH * ((OC + 63) / 64) * ((C + 63) / 64);
     const double planes = 12.0 + 2.5e-6 * (double)cs.N * (double)C * (double)cs.H * (double)cs.W + 4e-9 * (double)a.total * (double)C + 2e-6 * (double)a.total;
     return planes < 0.9 * (7.0 + 0.45e-3 * steps);
+}
+
+// Whether a channels-last ConvInteger with 1x1 filters that the packed kernel takes is faster there.  That reads the filters' zero points back and packs
+// them, 73 us whatever the size; a product needs none of it, but its kernel is the slower one, and its tiles are of 128 filters.  Both times in us, fitted to 182
+// calls of 5 to 30 G multiply-adds, measured both ways (within 8 and 15 %): by this choice 0.95 of the packed kernel's time on average, none slower
+// by more than 6 % (of 350 others one, by 11 %).  64 x 512 -> 512 channels at 56x56 221 packed and 276 as a product, 64 x 1024 -> 1024 at 28x28 164 and 250; 20 x 512 -> 280 at 72x72 81
+// and 111, with few filters beside a tile; 256 -> 384 channels at 39 G 208 and 166.  With few pixels to a filter its packing is what counts (64 images of 7x7, 2048 -> 3072: 145
+// and 101), and with strides the product's tiles are rows of results (138 x 2000 -> 376 at 11x11, 12.6 G: 75 and 162; of 40 such calls from 8 G on, 13 slower, by up to 4.3 times).
+bool faster_packed(const chx_hip_conv_params& p, const ConvShape& cs, const ConvDirectArgs& a) {
+    if (p.stride_h != 1 || p.stride_w != 1) return true;
+    const int64_t pixels = (int64_t)cs.N * cs.OH * cs.OW;
+    if (pixels < 8192) return false;
+    const double results = 4e-6 * (double)a.total;
+    const double product = 7.6 + 4.37e-9 * (double)pixels * padded(cs.OC, 128) * padded(a.C, 32) + 0.069 * results;
+    const double packed = 8.7 + (double)pixels * (1.7e-9 * padded(cs.OC, 64) * padded(a.C, 64) + 0.155e-6 * a.C + 17.5e-6) + 0.305 * results;
+    return product > 0.95 * std::max(73.0, packed);
 }
 
 // A ConvInteger with 1x1 filters as the product that it is, on gemm_i8.hip: pixels by filters where x and y are channels-last and
@@ -1639,12 +1661,7 @@ extern "C" int chx_hip_conv_integer(
     // allocations, packing): the two meet at 8 G multiply-adds, and it takes channels-last results only.
     const double macs = (double)a.total * cs.Cg * cs.KH * cs.KW;
     const bool packed = weights_fit_mfma(*w, params->group) && macs >= 0x1p33 && x_is_mfma_ready(*x);
-    // A product (1x1 filters) needs none of that and meets it later, the later the fewer channels there are to multiply for each
-    // result: us packed and as a product, 256 channels 266 and 212 at 39 G, 329 and 277 at 53 G, 384 109 and 121 at 20 G and 208 and 232 at 39 G, 512 83 and 75 at 11 G
-    // and 97 and 108 at 20 G, 1024 79 and 72 at 10 G, between 77 and 72 and 88 and 93 at 13 G and 117 and 192 at 39 G, 2048 212 and 498 at 79 G.  With few pixels to a filter
-    // its packing is what counts (64 images of 7x7, 2048 -> 3072: 145 and 101); with strides the product's tiles are rows of results (138 x 2000 -> 376 at
-    // 11x11, 12.6 G: 75 and 162).
-    const bool product_first = cs.KH * cs.KW == 1 && (capturing || !packed || macs < (params->stride_w == 1 ? 14e9 : 0x1p33) || macs * cs.Cg < 0x1p43 || cs.Cg < 320 || (int64_t)cs.N * cs.OH * cs.OW < 8192);
+    const bool product_first = cs.KH * cs.KW == 1 && (capturing || !packed || !faster_packed(*params, cs, a));
     auto product = [&](bool any) { return run_conv_as_product(*x, *w, x_zero_point, *params, cs, a, *y, any, s); };
     if (product_first) {
         const int rc = product(capturing);

@@ -72,6 +72,9 @@ def packed_weights(host):
     assert kernels(64, 256, 56, 384) == ["product"] and kernels(64, 512, 28, 320) == ["product"]  # (few channels, 8 G multiply-adds)
     assert kernels(64, 1024, 14, 1024) == ["product"] and kernels(32, 256, 112, 512) == ["product"]
     assert kernels(64, 2048, 7, 3072) == ["product"]  # 3136 pixels, 6 MB of filters
+    # few filters beside a tile of 128, and as many as fill it; rows of results with strides
+    assert kernels(20, 512, 72, 280) == ["packed"] and kernels(48, 1696, 30, 152) == ["packed"] and kernels(48, 1696, 30, 120) == ["product"]
+    assert kernels(59, 400, 37, 1872, stride=2) == ["packed"] and kernels(20, 400, 38, 1872, stride=2) == ["product"]
     s, graph = host.stream(), ctypes.c_void_p()
     host.check(host.lib.chx_hip_capture_begin(s))
     assert kernels(64, 1024, 28, 1024, stream=s) == ["product"]
@@ -82,6 +85,8 @@ def short_and_parted_rows(host):
     """Products that would be mostly padding, or write parts of lines, are for the other kernels, but in a recording."""
     assert not is_product(host, n=51, c=216, h=7, w=7, oc=1336) and is_product(host, n=8, c=1016, h=7, w=7, oc=664)  # 49 columns, many and few tiles
     assert is_product(host, n=125, c=160, h=11, w=11, oc=128)
+    assert not is_product(host, n=73, c=1640, h=5, w=5, oc=960) and not is_product(host, n=247, c=120, h=5, w=5, oc=200)  # 25 columns
+    assert not is_product(host, n=36, c=16, h=38, w=38, oc=1168) and not is_product(host, n=16, c=120, h=29, w=29, oc=1936)  # parts of lines
     assert not is_product(host, n=246, c=32, h=35, w=35, oc=200) and is_product(host, n=230, c=32, h=56, w=56, oc=104)
     assert not is_product(host, n=55, c=672, h=10, w=10, oc=80, strides=(2, 2), channels_last=True)  # strips
     assert is_product(host, n=10, c=136, h=48, w=48, oc=320, strides=(2, 2), channels_last=True)
