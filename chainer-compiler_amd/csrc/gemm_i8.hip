@@ -759,6 +759,9 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
         (void)tiles(128, 64);
         return b_transposed ? launch_stage<true, 2, 1, 4>(g, grid(), s) : launch_stage_short<2, 1, 4>(g, grid(), s);
     }
+    // (few products of one tile start sooner on one XCD, which has two wavefronts per SIMD for 256: 63 x 4 x 100 x 11 3.7 us and 4.2 on all, 219 x
+    // 10 x 23 x 11 4.6 and 4.9, 258 wavefronts of 129 x 29 x 83 x 45 0.7 of the time on all)
+    if (g.tiles == 1 && batch * w <= 256) g.turn = 0;
     if (small) {
         if (w == 1) launch_split<16, 1>(g, b_transposed, grid(), s);
         else if (w == 2) launch_split<16, 2>(g, b_transposed, grid(), s);
