@@ -744,6 +744,10 @@ int launch_matmul_i8(const MatMulDirectArgs& m, bool rne, hipStream_t s) {
                 best = i;
             }
         }
+        // (the fits are of single products.  In batches with a K of two or three stages, a round or two of tiles that are mostly padding have little beside their start: 17 x 638 x 295 x 146
+        // 10.3 us split and 13.7, 454 x 68 x 259 x 21 32 and 41; of 37 drawn batches of such K nine were slower by more than 3 %, seven of them these;
+        // of 289 others by this choice nine, by up to 22 %, and 0.71 of the time on average)
+        if (best == 0 && batch > 1 && !b_transposed && m.K < 400 && tiles(128, 128) * batch <= 512 && 1.6 * (double)(m.M * m.N) < 16384.0 * (double)g.tiles) best = -1;
         if (best >= 0) {
             (void)tiles((int)along_m[best], (int)along_n[best]);
             if (best == 0) return b_transposed ? launch_stage<true, 2, 2, 2>(g, grid(), s) : launch_stage<false, 2, 2, 2>(g, grid(), s);

@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k", "large", "few_columns"])
+@pytest.mark.parametrize("case", ["tiles", "other_forms", "short_k", "batches", "large", "few_columns"])
 def test_case(host_so, case):
     from test_gpu_gemm_i8_stage import SHAPES
     host_hip.run_case(host_so, __file__, case, SHAPES=repr(SHAPES))
@@ -66,6 +66,16 @@ def short_k(host):
     assert "split" in product(host, 100352, 192, 256) and "split" in product(host, 8192, 192, 8192)
     assert "stage" in product(host, 8192, 384, 1024) and "stage" in product(host, 33449, 192, 1044)
     assert "stage" in product(host, 8192, 256, 1024) and "stage" in product(host, 8192, 192, 8192, transposed=True)
+
+
+def batches(host):
+    """Two or three stages of K in batches whose tiles are mostly padding: the split kernel."""
+    def kernel_of(batch, M, K, N):
+        a, b, y = host.tensor("uint8", (batch, M, K)), host.tensor("int8", (batch, K, N)), host.tensor("int32", (batch, M, N))
+        return kernel(host, a, b, y)
+
+    assert "split" in kernel_of(17, 638, 295, 146) and "split" in kernel_of(454, 68, 259, 21)
+    assert "stage" in kernel_of(7, 704, 213, 634) and "stage" in kernel_of(331, 304, 302, 79) and "stage" in kernel_of(17, 638, 400, 146)
 
 
 def large(host):
