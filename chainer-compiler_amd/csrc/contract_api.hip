@@ -17,6 +17,7 @@
 #include "contract.h"
 #include "conv_mfma.h"
 #include "inverted_residual.h"
+#include "bottleneck.h"
 #include "depthwise.h"
 
 namespace chx {
@@ -1766,6 +1767,32 @@ extern "C" int chx_hip_qlinear_matmul(
     return launch_matmul_direct(m, rne, s);
 }
 
+// ---- blocks of convolutions as one launch ------------------------------------------------------
+
+namespace chx {
+namespace {
+// The operands of a convolution of a block: int8 weights, one scale or one per filter, an int32 bias on all of the block's or on none.
+int check_block_operands(const chx_hip_conv_operands& c, bool biased, const char* what) {
+    auto refuse = [&](const char* why) {
+        set_error("%s: %s", what, why);
+        return (int)CHX_HIP_EUNSUPPORTED;
+    };
+    CHX_PROPAGATE(check_tensor(c.w, what));
+    CHX_PROPAGATE(check_tensor(c.w_scale, what));
+    CHX_PROPAGATE(check_tensor(c.w_zero_point, what));
+    if (c.w->ndim != 4 || c.w->dtype != CHX_HIP_INT8 || c.w_scale->dtype != CHX_HIP_FLOAT32 || c.w_scale->ndim > 1 || c.w_zero_point->dtype != CHX_HIP_INT8) return refuse("the type of an operand");
+    const int64_t scales = numel(*c.w_scale);
+    if (scales != 1 && scales != c.w->shape[0]) return refuse("the number of scales");
+    if (c.bias) {
+        CHX_PROPAGATE(check_tensor(c.bias, what));
+        if (c.bias->dtype != CHX_HIP_INT32 || c.bias->ndim != 1 || c.bias->shape[0] != c.w->shape[0]) return refuse("a bias");
+    }
+    if ((c.bias != nullptr) != biased) return refuse("a bias on some of the convolutions");
+    return CHX_HIP_OK;
+}
+}  // namespace
+}  // namespace chx
+
 // ---- inverted residual blocks ------------------------------------------------------------------
 
 struct chx_hip_inverted_residual {
@@ -1793,20 +1820,7 @@ extern "C" int chx_hip_inverted_residual_create(const chx_hip_conv_operands* sta
         return (int)CHX_HIP_EUNSUPPORTED;
     };
     hipStream_t s = as_stream(stream);
-    for (int i = 0; i < 3; ++i) {
-        const chx_hip_conv_operands& c = stages[i];
-        CHX_PROPAGATE(check_tensor(c.w, "inverted residual w"));
-        CHX_PROPAGATE(check_tensor(c.w_scale, "inverted residual w_scale"));
-        CHX_PROPAGATE(check_tensor(c.w_zero_point, "inverted residual w_zero_point"));
-        if (c.w->ndim != 4 || c.w->dtype != CHX_HIP_INT8 || c.w_scale->dtype != CHX_HIP_FLOAT32 || c.w_scale->ndim > 1 || c.w_zero_point->dtype != CHX_HIP_INT8) return refuse("the type of an operand");
-        const int64_t scales = numel(*c.w_scale);
-        if (scales != 1 && scales != c.w->shape[0]) return refuse("the number of scales");
-        if (c.bias) {
-            CHX_PROPAGATE(check_tensor(c.bias, "inverted residual bias"));
-            if (c.bias->dtype != CHX_HIP_INT32 || c.bias->ndim != 1 || c.bias->shape[0] != c.w->shape[0]) return refuse("a bias");
-        }
-        if ((c.bias != nullptr) != (stages[0].bias != nullptr)) return refuse("a bias on some of the convolutions");
-    }
+    for (int i = 0; i < 3; ++i) CHX_PROPAGATE(check_block_operands(stages[i], stages[0].bias != nullptr, "inverted residual"));
     const chx_hip_tensor &w1 = *stages[0].w, &w2 = *stages[1].w, &w3 = *stages[2].w;
     const int64_t hid = w1.shape[0];
     if (w1.shape[2] != 1 || w1.shape[3] != 1 || w3.shape[2] != 1 || w3.shape[3] != 1 || w2.shape[2] != 3 || w2.shape[3] != 3 || w2.shape[1] != 1 || w2.shape[0] != hid ||
@@ -1932,4 +1946,152 @@ extern "C" int chx_hip_inverted_residual_run(
     a.s3 = y_scales[1];
     a.fill = (int32_t)(((uint32_t)y_zero_points[0] ^ 0x80u) * 0x01010101u);
     return launch_inverted_residual(a, plan->stride, s);
+}
+
+// ---- bottleneck blocks -------------------------------------------------------------------------
+
+struct chx_hip_bottleneck {
+    int32_t mid = 0, wide = 0, next = 0;
+    bool has_bias = false, affine_residual = true;
+    int device = 0;  // whose memory the operands are laid out in
+    char* memory = nullptr;
+    size_t at[3] = {0, 0, 0}, at_table = 0;
+    std::mutex mutex;  // of `searched`
+    std::vector<chx::SearchedResidual> searched;
+};
+
+extern "C" void chx_hip_bottleneck_destroy(chx_hip_bottleneck* plan) {
+    if (!plan) return;
+    (void)hipFree(plan->memory);
+    delete plan;
+}
+
+extern "C" int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, int32_t count, void* stream, chx_hip_bottleneck** out) {
+    CHX_REQUIRE(stages != nullptr && out != nullptr && (count == 2 || count == 3), "bottleneck: null argument");
+    *out = nullptr;
+    auto refuse = [](const char* why) {
+        set_error("bottleneck: %s", why);
+        return (int)CHX_HIP_EUNSUPPORTED;
+    };
+    hipStream_t s = as_stream(stream);
+    int64_t channels = 0;
+    for (int i = 0; i < count; ++i) {
+        CHX_PROPAGATE(check_block_operands(stages[i], stages[0].bias != nullptr, "bottleneck"));
+        const chx_hip_tensor& w = *stages[i].w;
+        const int64_t k = i == 0 ? 3 : 1;
+        if (w.shape[2] != k || w.shape[3] != k || (i > 0 && w.shape[1] != channels)) return refuse("not 3x3, 1x1, 1x1");
+        channels = w.shape[0];
+    }
+    const int64_t mid = stages[0].w->shape[0], wide = stages[1].w->shape[0], next = count == 3 ? channels : 0;
+    if (stages[0].w->shape[1] != mid || !bottleneck_mid(mid) || wide < 256 || wide > 2048 || (wide & (wide - 1)) != 0 || next % 32 != 0 || next > 1024) return refuse("the number of channels");
+    for (int i = 0; i < count; ++i) {
+        std::vector<uint8_t> zp;
+        CHX_PROPAGATE(read_back(*stages[i].w_zero_point, &zp, s));
+        if (!all_zero(zp)) return refuse("zero points of the weights");
+    }
+    std::unique_ptr<chx_hip_bottleneck, void (*)(chx_hip_bottleneck*)> p(new chx_hip_bottleneck(), chx_hip_bottleneck_destroy);
+    CHX_HIP_CALL(hipGetDevice(&p->device));
+    p->mid = (int32_t)mid;
+    p->wide = (int32_t)wide;
+    p->next = (int32_t)next;
+    p->has_bias = stages[0].bias != nullptr;
+    p->affine_residual = read_launch_options().affine_residual;
+    p->at[1] = (size_t)(9 * mid * mid);
+    p->at[2] = p->at[1] + (size_t)(mid * wide);
+    p->at_table = p->at[2] + (size_t)(wide * next);
+    CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&p->memory), p->at_table + (size_t)round_up(mid + wide + next, 64) * 16));  // (the kernel reads 64 rows at a time)
+    int32_t* table = reinterpret_cast<int32_t*>(p->memory + p->at_table);
+    for (int i = 0; i < count; ++i) {
+        CHX_PROPAGATE(pack_bottleneck(*stages[i].w, *stages[i].w_scale, stages[i].bias, p->memory + p->at[i], table, s));
+        table += 4 * stages[i].w->shape[0];
+    }
+    // (later calls may come on any stream)
+    CHX_HIP_CALL(hipStreamSynchronize(s));
+    *out = p.release();
+    return CHX_HIP_OK;
+}
+
+extern "C" int chx_hip_bottleneck_run(
+        chx_hip_bottleneck* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points, int32_t y_dtype,
+        uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu, uint32_t out_flags, chx_hip_tensor* out,
+        uint32_t next_flags, chx_hip_tensor* next, void* stream) {
+    CHX_REQUIRE(plan != nullptr && y_scales != nullptr && y_zero_points != nullptr && (next != nullptr) == (plan->next != 0), "bottleneck: null argument");
+    CHX_PROPAGATE(check_tensor(x, "bottleneck x"));
+    CHX_PROPAGATE(check_tensor(r, "bottleneck r"));
+    chx_hip_tensor views[2];
+    chx_hip_tensor* const results[2] = {out, next};
+    bool minus_128[2] = {false, false};
+    CHX_PROPAGATE(result_view(out, out_flags, "bottleneck out", &views[0], &minus_128[0]));
+    if (next) CHX_PROPAGATE(result_view(next, next_flags, "bottleneck next", &views[1], &minus_128[1]));
+    auto refuse = [](const char* why) {
+        set_error("bottleneck: %s", why);
+        return (int)CHX_HIP_EUNSUPPORTED;
+    };
+    int device = 0;
+    CHX_HIP_CALL(hipGetDevice(&device));
+    if (device != plan->device) return refuse("another device than the one that it was created on");
+    auto in_range = [](int32_t zp, int32_t dt) { return dt == CHX_HIP_INT8 ? zp >= -128 && zp <= 127 : zp >= 0 && zp <= 255; };
+    if (x->ndim != 4 || !is_q8(x->dtype) || x->shape[1] != plan->mid || !in_range(x_zero_point, x->dtype)) return refuse("x");
+    if ((flags & (CHX_HIP_ROUND_ONNX_RNE | CHX_HIP_FUSE_RELU)) != 0 || (plan->has_bias && !(flags & CHX_HIP_BIAS_ONNX_INT32))) return refuse("the flags");
+    if (y_dtype != CHX_HIP_UINT8) return refuse("the type of a result");
+    const int64_t N = x->shape[0], H = x->shape[2], W = x->shape[3];
+    if (N < 1 || H < 1 || W < 1 || N * H * W >= (int64_t(1) << 30)) return refuse("the number of pixels");
+    const int64_t most_px = int64_t(1) << 24;  // (bytes from a pixel to the next: 24-bit products)
+    int64_t x_px = 0, px[2] = {0, 0}, r_px = 0;
+    if (!y_is_pixel_major(*x, &x_px) || !aligned(x->data, 16) || x_px % 16 != 0 || x_px >= most_px) return refuse("x is not channels-last in whole chunks");
+    for (int i = 0; i < (next ? 2 : 1); ++i) {
+        const chx_hip_tensor& t = *results[i];
+        if (t.ndim != 4 || t.shape[0] != N || t.shape[1] != (i ? plan->next : plan->wide) || t.shape[2] != H || t.shape[3] != W) return refuse("the shape of a result");
+        if (views[i].dtype != CHX_HIP_UINT8) return refuse("the type of a result");
+        if (!y_is_pixel_major(views[i], &px[i]) || !aligned(t.data, 16) || px[i] % 16 != 0 || px[i] >= most_px) return refuse("a result is not channels-last in whole chunks");
+        if (byte_ranges_overlap(views[i], *x) || byte_ranges_overlap(views[i], *r)) return refuse("a result overlaps an operand");
+    }
+    if (next && byte_ranges_overlap(views[0], views[1])) return refuse("the results overlap");
+    for (int i = 0; i < 4; ++i)
+        if (r->ndim != 4 || r->shape[i] != out->shape[i]) return refuse("the shape of r");
+    if (!is_q8(r->dtype) || !in_range(r_zero_point, r->dtype) || !in_range(out_zero_point, CHX_HIP_UINT8) || !(out_scale >= 0x1p-60f && out_scale <= 0x1p60f)) return refuse("the quantization of the sum");
+    if (!y_is_pixel_major(*r, &r_px) || !aligned(r->data, 16) || r_px % 16 != 0 || r_px >= most_px) return refuse("r is not channels-last in whole chunks");
+    BottleneckArgs a;
+    memset(&a, 0, sizeof(a));
+    QuantProduct* const products[3] = {&a.q1, &a.q2, &a.q3};
+    for (int i = 0; i < (next ? 3 : 2); ++i) {
+        if (!in_range(y_zero_points[i], CHX_HIP_UINT8)) return refuse("a zero point");
+        const QuantParams q = make_quant_params(y_scales[i], y_zero_points[i], false);
+        *products[i] = product_form(q, q.lo, false, true);
+        if (products[i]->path != 1 && products[i]->path != 3) return refuse("a requantization without a product form");
+    }
+    a.pixels = (int32_t)(N * H * W);
+    a.H = (int32_t)H;
+    a.W = (int32_t)W;
+    a.mid = plan->mid;
+    a.wide = plan->wide;
+    a.next = plan->next;
+    CHX_PROPAGATE(plan_bottleneck(&a));
+    hipStream_t s = as_stream(stream);
+    {  // (the first call with a sum's parameters launches a search: nothing is refused behind it)
+        std::lock_guard<std::mutex> lock(plan->mutex);
+        CHX_PROPAGATE(residual_of(*r, r_px, y_scales[1], y_zero_points[1], y_dtype, r_scale, r_zero_point, out_scale, out_zero_point, CHX_HIP_UINT8, relu != 0, plan->affine_residual,
+                                  &plan->searched, s, &a.res));
+    }
+    a.x = static_cast<const char*>(x->data);
+    a.y = static_cast<char*>(out->data);
+    a.z = next ? static_cast<char*>(next->data) : nullptr;
+    a.x_px = x_px;
+    a.y_px = px[0];
+    a.z_px = px[1];
+    a.w1 = plan->memory;
+    a.w2 = plan->memory + plan->at[1];
+    a.w3 = plan->memory + plan->at[2];
+    a.table = reinterpret_cast<const int32_t*>(plan->memory + plan->at_table);
+    a.x_flip = x->dtype == CHX_HIP_UINT8 ? 0x80808080u : 0u;
+    a.y_flip = minus_128[0] ? 0x80808080u : 0u;
+    a.z_flip = minus_128[1] ? 0x80808080u : 0u;
+    a.corr1 = (x->dtype == CHX_HIP_UINT8 ? 128 : 0) - x_zero_point;
+    a.corr2 = 128 - y_zero_points[0];
+    a.corr3 = 128 - out_zero_point;
+    a.s1 = x_scale;
+    a.s2 = y_scales[0];
+    a.s3 = out_scale;
+    a.fill = (int32_t)(((uint32_t)x_zero_point ^ (x->dtype == CHX_HIP_UINT8 ? 0x80u : 0u)) & 0xffu) * 0x01010101;
+    return launch_bottleneck(a, s);
 }

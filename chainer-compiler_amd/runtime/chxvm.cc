@@ -459,6 +459,114 @@ private:
     std::vector<int> freed_;
 };
 
+std::atomic<int64_t> g_bottlenecks{0};
+
+// The 3x3 convolution of a bottleneck block, the 1x1 convolution behind it with the residual sum, and the 1x1 convolution that
+// reads the sum in the next block (where there is one) as one launch (chx_hip_bottleneck_run).  It stands where the last of them
+// stood; what that kernel does not take runs as the program wrote it.  The operands are constants of the program, laid out when it
+// is loaded.
+class BottleneckOp : public ChxVMOp {
+public:
+    struct Quantization {  // the variable slots of a convolution
+        int x_scale, x_zp, y_scale, y_zp;
+    };
+    struct Sum {
+        chx_hip_residual_group group;
+        int conv_operand, other, out;
+        std::shared_ptr<ResidualFusionState> state;
+    };
+    BottleneckOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_bottleneck> block, int x, int between, int next, const std::vector<Quantization>& convs,
+                 int64_t wide_channels, int64_t next_channels, bool has_bias, Sum sum, ChxVMSteps steps, std::vector<int> freed)
+        : ChxVMOp(last), block_(std::move(block)), x_(x), between_(between), next_(next), convs_(convs), wide_channels_(wide_channels), next_channels_(next_channels),
+          has_bias_(has_bias), sum_(std::move(sum)), steps_(std::move(steps)), freed_(std::move(freed)) {
+    }
+
+    void Run(ChxVMState* st) override {
+        if (RunAsOne(st)) {
+            for (int slot : freed_) st->FreeVar(slot);
+        } else {
+            RunSteps(steps_, st);
+        }
+    }
+
+private:
+    static int32_t Integer(const StrictScalar& z) {
+        return static_cast<int32_t>(static_cast<int64_t>(z));
+    }
+
+    // false: nothing has been written
+    bool RunAsOne(ChxVMState* st) {
+        if (st->GetVar(x_)->IsNull() || st->GetVar(sum_.other)->IsNull() || (has_bias_ && !st->options().qlinearconv_onnx_int32_bias)) return false;
+        float scales[3] = {1.f, 1.f, 1.f};
+        int32_t zero_points[3] = {0, 0, 0};
+        const chx_hip_residual_group& g = sum_.group;
+        const int k = sum_.conv_operand;
+        for (size_t i = 0; i < convs_.size(); ++i) {
+            for (int slot : {convs_[i].x_scale, convs_[i].x_zp, convs_[i].y_scale, convs_[i].y_zp})
+                if (st->GetVar(slot)->IsNull()) return false;
+            const StrictScalar& zp = st->GetScalar(convs_[i].y_zp);
+            if (zp.dtype() != chainerx::Dtype::kUInt8) return false;
+            scales[i] = static_cast<float>(st->GetScalar(convs_[i].y_scale));
+            zero_points[i] = Integer(zp);
+            // each reads its input the way it was written: the second the first's result, the third the sum
+            const float scale = i == 1 ? scales[0] : g.out_scale;
+            const int32_t zero_point = i == 1 ? zero_points[0] : g.out_zero_point;
+            if (i > 0 && (static_cast<float>(st->GetScalar(convs_[i].x_scale)) != scale || Integer(st->GetScalar(convs_[i].x_zp)) != zero_point ||
+                          st->GetScalar(convs_[i].x_zp).dtype() != chainerx::Dtype::kUInt8))
+                return false;
+        }
+        if (g.in_scale[k] != scales[1] || g.in_zero_point[k] != zero_points[1] || static_cast<chainerx::Dtype>(g.in_dtype[k]) != chainerx::Dtype::kUInt8 ||
+            static_cast<chainerx::Dtype>(g.out_dtype) != chainerx::Dtype::kUInt8)
+            return false;
+        const chainerx::Array x = st->GetArray(x_), r = st->GetArray(sum_.other);
+        if (x.ndim() != 4) return false;
+        const StrictScalar& x_zp = st->GetScalar(convs_[0].x_zp);
+        // a value kept as code - 128 is an int8 tensor with the zero point 128 lower
+        auto minus_128 = [&](int slot, const chainerx::Array& a, chainerx::Dtype type_in_program) {
+            return st->store_minus_128(slot) && a.dtype() == chainerx::Dtype::kInt8 && type_in_program == chainerx::Dtype::kUInt8;
+        };
+        const chainerx::Shape shape{x.shape()[0], wide_channels_, x.shape()[2], x.shape()[3]};
+        const chainerx::Dtype r_type = static_cast<chainerx::Dtype>(g.in_dtype[1 - k]);
+        const bool lowered = minus_128(sum_.other, r, r_type);
+        if ((r.dtype() != r_type && !lowered) || r.shape() != shape) return false;
+        const int32_t r_zp = g.in_zero_point[1 - k] - (lowered ? 128 : 0);
+        const bool out_signed = st->store_minus_128(sum_.out), next_signed = next_ >= 0 && st->store_minus_128(next_);
+        chainerx::Array out = chainerx::EmptyChannelsLastPadded(shape, out_signed ? chainerx::Dtype::kInt8 : chainerx::Dtype::kUInt8), next;
+        if (next_ >= 0)
+            next = chainerx::EmptyChannelsLastPadded(chainerx::Shape{x.shape()[0], next_channels_, x.shape()[2], x.shape()[3]}, next_signed ? chainerx::Dtype::kInt8 : chainerx::Dtype::kUInt8);
+        const chx_hip_tensor xt = x.hip(), rt = r.hip();
+        chx_hip_tensor ot = out.hip(), nt;
+        if (next_ >= 0) nt = next.hip();
+        const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
+        const int rc = chx_hip_bottleneck_run(
+                block_.get(), &xt, static_cast<float>(st->GetScalar(convs_[0].x_scale)), Integer(x_zp) - (minus_128(x_, x, x_zp.dtype()) ? 128 : 0), scales, zero_points,
+                static_cast<int32_t>(chainerx::Dtype::kUInt8), flags, &rt, g.in_scale[1 - k], r_zp, g.out_scale, g.out_zero_point, g.relu,
+                out_signed ? CHX_HIP_STORE_MINUS_128 : 0u, &ot, next_signed ? CHX_HIP_STORE_MINUS_128 : 0u, next_ >= 0 ? &nt : nullptr, chainerx::CurrentStream());
+        // (what it refuses, and operands that are in error, are for the instructions)
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(block_);  // a recording may outlive the program
+        // (the 3x3 convolution's result is code - 128 on its way to the next)
+        CountMinus128Stores((out_signed ? 1 : 0) + (next_signed ? 1 : 0) + (st->store_minus_128(between_) ? 1 : 0));
+        sum_.state->fused = true;
+        CountResidualFusion();
+        st->count_residual_fusion();
+        st->SetArray(sum_.out, out);
+        if (next_ >= 0) st->SetArray(next_, next);
+        ++g_bottlenecks;
+        return true;
+    }
+
+    std::shared_ptr<chx_hip_bottleneck> block_;
+    int x_, between_, next_;
+    std::vector<Quantization> convs_;
+    int64_t wide_channels_, next_channels_;
+    bool has_bias_;
+    Sum sum_;
+    ChxVMSteps steps_;
+    std::vector<int> freed_;
+};
+
 // A fused op followed by the Free instructions of its operands that the program had placed
 // between the instructions it replaces.
 class SequenceOp : public ChxVMOp {
@@ -974,9 +1082,98 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         remaining_.swap(rest);
     }
+    // Bottleneck blocks, likewise: a 3x3 convolution, the 1x1 convolution behind it that computes the residual sum, and the 1x1
+    // convolution that reads the sum, where nothing but constants and Free instructions stands in between.
+    for (int d = 0; d < n; ++d) {
+        if (!convolution(d, false)) continue;
+        const int h = program.instructions[d].outputs[0], p = conv_reader[h];
+        if (p <= d || !single_use(h) || role[p] != 4 || !convolution(p, true) || partner[p] <= p) continue;
+        const int e = partner[p];
+        const ChxVMInstructionProto& group = program.instructions[e];
+        const int out = group.outputs[0], other = group.inputs[0].array_list[1 - conv_operand[p]];
+        if (!once(out) || !once(other)) continue;
+        auto form = [&](int i, int64_t kernel, int64_t pad) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            const chainerx::Array& w = *constant_array(inst.inputs[3].array);
+            return all_are(inst.inputs[9].ints, 1) && (pad == 0 || !inst.inputs[10].ints.empty()) && all_are(inst.inputs[10].ints, pad) && inst.inputs[11].i == 1 && w.ndim() == 4 &&
+                   w.shape()[2] == kernel && w.shape()[3] == kernel;
+        };
+        if (!form(d, 3, 1) || !form(p, 1, 0)) continue;
+        auto nothing_between = [&](int from, int to) {
+            for (int i = from + 1; i < to; ++i) {
+                const ChxVMInstructionProto& inst = program.instructions[i];
+                const bool constant = inst.outputs.size() == 1 && inst.outputs[0] >= 0 && constant_slots_[inst.outputs[0]] != nullptr;
+                if (i != p && i != e && inst.op != kFree && !constant && !dynamic_cast<NopOp*>(program_[i].get())) return false;
+            }
+            return true;
+        };
+        if (!nothing_between(d, e)) continue;
+        std::vector<int> convs = {d, p};
+        for (int c = e + 1; c < n; ++c) {
+            const ChxVMInstructionProto& inst = program.instructions[c];
+            if (inst.op != kQLinearConv || inst.inputs.empty() || inst.inputs[0].array != out) continue;
+            if (convolution(c, false) && form(c, 1, 0) && nothing_between(e, c)) convs.push_back(c);
+            break;
+        }
+        int last = convs.back() > e ? convs.back() : e;
+        chx_hip_conv_operands stages[3];
+        chx_hip_tensor tensors[3][4];
+        std::vector<BottleneckOp::Quantization> quantizations;
+        std::set<int> slots = {h, program.instructions[d].inputs[0].array, program.instructions[p].outputs[0], other, out};
+        auto take = [&](size_t m) {
+            const ChxVMInstructionProto& inst = program.instructions[convs[m]];
+            const int operand[4] = {inst.inputs[3].array, inst.inputs[4].array, inst.inputs[5].array, inst.inputs[8].array};
+            for (int k = 0; k < 4; ++k)
+                if (operand[k] >= 0) {
+                    tensors[m][k] = constant_array(operand[k])->hip();
+                    slots.insert(operand[k]);
+                }
+            stages[m] = {&tensors[m][0], &tensors[m][1], &tensors[m][2], operand[3] >= 0 ? &tensors[m][3] : nullptr};
+            quantizations.push_back({inst.inputs[1].scalar, inst.inputs[2].scalar, inst.inputs[6].scalar, inst.inputs[7].scalar});
+            for (int k : {1, 2, 6, 7}) slots.insert(inst.inputs[k].scalar);
+        };
+        for (size_t m = 0; m < convs.size(); ++m) take(m);
+        chx_hip_bottleneck* block = nullptr;
+        int rc = chx_hip_bottleneck_create(stages, static_cast<int32_t>(convs.size()), chainerx::CurrentStream(), &block);
+        if (rc == CHX_HIP_EUNSUPPORTED && convs.size() == 3) {  // perhaps without the third
+            convs.pop_back();
+            quantizations.pop_back();
+            last = e;
+            rc = chx_hip_bottleneck_create(stages, 2, chainerx::CurrentStream(), &block);
+        }
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        std::set<int> moved(convs.begin(), convs.end());
+        moved.insert(e);
+        ChxVMSteps steps;
+        std::vector<int> freed;
+        for (int i = d; i <= last; ++i) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
+                freed.push_back(inst.inputs[0].array);
+                moved.insert(i);
+            }
+            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
+        }
+        const bool reduced = convs.size() == 3;
+        chains_.emplace_back(new BottleneckOp(program.instructions[last], std::shared_ptr<chx_hip_bottleneck>(block, chx_hip_bottleneck_destroy), program.instructions[d].inputs[0].array, h,
+                                              reduced ? program.instructions[convs[2]].outputs[0] : -1, quantizations, tensors[1][0].shape[0], reduced ? tensors[2][0].shape[0] : 0,
+                                              stages[0].bias != nullptr, {groups[p], conv_operand[p], other, out, fusion_state[p]}, std::move(steps), std::move(freed)));
+        for (int m : convs) chained[m] = true;
+        std::vector<std::pair<int, ChxVMOp*>> rest;
+        for (const auto& r : remaining_) {
+            if (r.first == last) rest.emplace_back(last, chains_.back().get());
+            else if (!moved.count(r.first)) rest.push_back(r);
+        }
+        remaining_.swap(rest);
+    }
 }
 
 ChxVM::~ChxVM() = default;
+
+int64_t Bottlenecks() {
+    return g_bottlenecks.load();
+}
 
 int64_t InvertedResiduals() {
     return g_inverted_residuals.load();

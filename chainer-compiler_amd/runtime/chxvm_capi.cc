@@ -493,6 +493,7 @@ int64_t chxvm_counter(const char* name) {
     if (n == "qlinearconv_pair_fusions") return QLinearConvPairFusions();
     if (n == "minus_128_stores") return Minus128Stores();
     if (n == "matmul_chains") return MatMulChains();
+    if (n == "bottlenecks") return Bottlenecks();
     if (n == "inverted_residuals") return InvertedResiduals();
     return -1;
 }

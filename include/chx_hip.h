@@ -299,6 +299,21 @@ int chx_hip_inverted_residual_run(
         int32_t y_dtype, uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu,
         chx_hip_tensor* out, void* stream);
 
+/* The tail of a bottleneck block: 3x3 convolution with padding 1, 1x1 convolution and the residual sum of
+ * chx_hip_qconv_plan_run_add; with three stages, the 1x1 convolution of the sum as well (the next block's first), as one launch,
+ * with the codes of the single calls.  stages: as for chx_hip_inverted_residual_create, strides 1; 64, 128 or 256 channels in
+ * between, a multiple of 256 behind the sum, of 32 behind the third. */
+typedef struct chx_hip_bottleneck chx_hip_bottleneck;
+int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, int32_t count, void* stream, chx_hip_bottleneck** out);
+void chx_hip_bottleneck_destroy(chx_hip_bottleneck* plan);
+/* y_scales, y_zero_points: of the convolutions' results, all of type y_dtype.  out: the sum; next: the third convolution's result
+ * (NULL with two stages).  out_flags, next_flags: 0 or CHX_HIP_STORE_MINUS_128.  CHX_HIP_EUNSUPPORTED, with nothing launched, as
+ * for chx_hip_inverted_residual_run. */
+int chx_hip_bottleneck_run(
+        chx_hip_bottleneck* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points,
+        int32_t y_dtype, uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu,
+        uint32_t out_flags, chx_hip_tensor* out, uint32_t next_flags, chx_hip_tensor* next, void* stream);
+
 /* MatMulIntegerOp::RunImpl, runtime/ops/quantize.cc:96-114 with NumpyMatMul,
  * runtime/chainerx_util.cc:210-230.  a [..,M,K], b [..,K,N] with equal leading
  * dims, y int32 [..,M,N].  Zero points: NULL, or arrays of ndim <= 1 subtracted by
