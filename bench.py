@@ -338,6 +338,8 @@ def _kernel_of(config):
     oc, px = (int(v) for v in config["tile"].split("x"))
     if (oc, px, config.get("waves")) == (64, 32, "4"):
         return "conv_point_kernel"
+    if config.get("wgs_per_cu") == "100":
+        return "conv_same_kernel"
     return "conv_split_kernel" if oc <= 32 else "conv_mfma_kernel"
 
 

@@ -227,7 +227,8 @@ bool weights_fit_mfma(const chx_hip_tensor& w, int group) {
 // environment variables are overrides for tuning and for tests (which reach every launch configuration through them),
 // read when a plan is created or a one-shot entry point is called, never on the path of a plan's runs.
 //   CHX_HIP_TILE=<oc>,<px>[,<work-groups per compute unit>[,<wavefronts: 4 or 8>]]  forces a launch configuration (with the
-//                               small tiles, in place of the work-groups: 1 for pixels from LDS, where that fits)
+//                               small tiles, in place of the work-groups: 1 for pixels from LDS, where that fits; 100 for the tiles
+//                               of conv_same_kernel)
 //   CHX_HIP_AUTOTUNE=0          keeps the heuristic tile choice instead of timing the configurations
 //   CHX_HIP_NO_STEM=1           keeps few-channel first layers off the planar-input kernel
 //   CHX_HIP_AFFINE_RESIDUAL=0   keeps fused residual sums on the operation-by-operation arithmetic
@@ -264,9 +265,10 @@ void pick_tile(const LaunchOptions& opt, const ConvMfmaArgs& a, bool out_int32, 
     *waves = 4;
     if (opt.forced_tile) {
         const int toc = opt.tile_oc, tpx = opt.tile_px, wv = opt.waves;
+        const bool same = opt.max_wgs_per_cu == kConvSame;
         const bool four = wv == 4 && (toc == 64 || toc == 128) && (tpx == 64 || tpx == 128);
         const bool eight = wv == 8 && ((toc == 128 && tpx == 128) || (a.bk == 128 && ((toc == 128 && tpx == 256) || (toc == 64 && tpx == 128))));
-        if (four || eight || (conv_split_has(toc, tpx, wv) && conv_split_takes(a) && !out_int32) ||
+        if (same ? conv_same_has(toc, tpx, wv) && conv_same_takes(a, tpx) && !out_int32 : four || eight || (conv_split_has(toc, tpx, wv) && conv_split_takes(a) && !out_int32) ||
             (toc == kConvPointTile.oc && tpx == kConvPointTile.px && wv == kConvPointTile.waves && conv_point_takes(a) && !out_int32)) {
             *tile_oc = toc;
             *tile_px = tpx;
@@ -377,6 +379,9 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
                 if (conv_split_patch_takes(a, t.oc, t.px, t.waves)) all.push_back({{t.oc, t.px, kConvSplitPatch, t.waves}, {}});
             }
 
+    if (!out_int32 && !rne)
+        for (const ConvSplitTile& t : kConvSameTiles)
+            if (conv_same_takes(a, t.px) && (a.OC > 64 || t.oc == 64)) all.push_back({{t.oc, t.px, kConvSame, t.waves}, {}});
     if (!out_int32 && conv_point_takes(a))
         for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, {}});
 

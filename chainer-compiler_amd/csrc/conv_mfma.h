@@ -190,6 +190,13 @@ constexpr int kConvSplitPatch = 1;  // ... as a launch configuration: in the pla
 bool conv_split_patch_takes(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves);
 int launch_conv_split(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool patch, bool x_unsigned, bool rne, hipStream_t s);
 
+// The kernel for 3x3 filters over an image whose results have its size (conv_same.hip): output channels x pixels, wavefronts.
+constexpr ConvSplitTile kConvSameTiles[] = {{64, 64, 4}, {64, 128, 4}, {128, 64, 4}, {128, 128, 8}};
+constexpr int kConvSame = 100;  // as a launch configuration: in the place of the work-groups per compute unit
+bool conv_same_has(int tile_oc, int tile_px, int waves);
+bool conv_same_takes(const ConvMfmaArgs& a, int tile_px);
+int launch_conv_same(const ConvMfmaArgs& a, int tile_oc, int tile_px, int waves, bool x_unsigned, hipStream_t s);
+
 // 1x1, stride 1, no padding over a dense image: input pixel m is at x + m * x_w_stride
 inline bool conv_px_linear(const ConvMfmaArgs& a) {
     return a.KH == 1 && a.KW == 1 && a.sh == 1 && a.sw == 1 && a.ph == 0 && a.pw == 0 && a.OH == a.H && a.OW == a.W &&

@@ -409,6 +409,10 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     a.row_unit = 0;
     if (a.KH * a.KW <= 32)
         for (int i = 0; i < a.KH; ++i) a.row_unit |= 1u << (i * a.KW);
+    if (max_wgs_per_cu == kConvSame) {
+        if (out_int32 || rne || !conv_same_takes(a, tile_px)) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the kernel with the pixels in LDS does not take this convolution");
+        return launch_conv_same(a, tile_oc, tile_px, waves, x_unsigned, s);
+    }
     if (tile_oc == kConvPointTile.oc && tile_px == kConvPointTile.px && waves == kConvPointTile.waves) {
         if (out_int32 || !conv_point_takes(a)) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the pixel-streaming kernel does not take this convolution");
         return launch_conv_point(a, max_wgs_per_cu, x_unsigned, rne, s);
