@@ -296,6 +296,7 @@ struct TunedConfig {
     int64_t M;
     int32_t H, W, OH, OW;
     int64_t x_n_stride, x_h_stride, x_w_stride;  // a kernel may take a dense image only (conv_point_takes)
+    bool short_form;                             // ... or a requantization in a short form only (conv_same_takes)
     int tile_oc, tile_px, max_wgs_per_cu;
     int waves;      // wavefronts per work-group
     bool with_res;  // measured with a fused residual sum (an entry of its own: the epilogue differs)
@@ -319,7 +320,7 @@ public:
         (void)hipGetDevice(&device);
         const int64_t res = a.res.r ? 1 + a.res.affine : 0;
         return {device, a.M, a.H, a.W, a.OH, a.OW, a.KH, a.KW, a.sh, a.sw, a.ph, a.pw, a.C16, a.KP, a.bk, a.OC, a.oc_split, a.x_n_stride,
-                a.x_h_stride, a.x_w_stride, a.y_px_stride, aligned(a.y, 16), res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0)};
+                a.x_h_stride, a.x_w_stride, a.y_px_stride, aligned(a.y, 16), res, (a.x_zp & 0xff) != 0, (xu ? 1 : 0) | (out_int32 ? 2 : 0) | (rne ? 4 : 0) | (a.qp.path != 0 ? 8 : 0)};
     }
     bool find(const Key& k, Configuration* c) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -766,7 +767,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     if (c.tune) {
         for (const TunedConfig& t : c.tune->entries)
             if (t.M == a.M && t.H == a.H && t.W == a.W && t.OH == a.OH && t.OW == a.OW && t.x_n_stride == a.x_n_stride && t.x_h_stride == a.x_h_stride &&
-                t.x_w_stride == a.x_w_stride && t.with_res == (c.res != nullptr) && t.oc_split == a.oc_split)
+                t.x_w_stride == a.x_w_stride && t.short_form == (a.qp.path != 0) && t.with_res == (c.res != nullptr) && t.oc_split == a.oc_split)
                 tuned = &t;
         if (!tuned && c.opt.autotune && !stream_is_capturing(s)) {
             const MeasuredConfigurations::Key key = MeasuredConfigurations::key(a, xu, c.out_int32, c.rne);
@@ -776,7 +777,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
                 if (rc == CHX_HIP_OK) measured_configurations().add(key, best);
             }
             if (rc == CHX_HIP_OK) {
-                c.tune->entries.push_back({a.M, a.H, a.W, a.OH, a.OW, a.x_n_stride, a.x_h_stride, a.x_w_stride, best.tile_oc, best.tile_px, best.max_wgs_per_cu, best.waves, c.res != nullptr, a.oc_split});
+                c.tune->entries.push_back({a.M, a.H, a.W, a.OH, a.OW, a.x_n_stride, a.x_h_stride, a.x_w_stride, a.qp.path != 0, best.tile_oc, best.tile_px, best.max_wgs_per_cu, best.waves, c.res != nullptr, a.oc_split});
                 tuned = &c.tune->entries.back();
             }
         }

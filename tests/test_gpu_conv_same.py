@@ -53,3 +53,18 @@ def test_plain(g, oracle, tile):  # noqa: F811
             got = g.host(out)
             np.testing.assert_array_equal(got.view(np.uint8) ^ 0x80 if minus_128 else got, want, err_msg="case %d %s" % (i, (N, C, H, W, OC, xdt, xz)))
             plan.close()
+
+
+# (the plan's measured configuration may be this kernel, which has no code for int8 results or rounding to nearest even)
+@pytest.mark.parametrize("N,C,HW,OC", [(8, 512, 7, 512), (2, 64, 12, 96)])
+def test_one_plan_with_other_quantizations(g, oracle, N, C, HW, OC):  # noqa: F811
+    rng = np.random.default_rng(C)
+    x, w, ws = codes(rng, (N, C, HW, HW), np.uint8), codes(rng, (OC, C, 3, 3), np.int8), rng.uniform(0.002, 0.02, size=OC).astype(np.float32)
+    y_scale = float(0.02 * 0.01 * 74 * 74 * np.sqrt(C * 9) / 40)
+    plan, xd = g.ops.QLinearConvPlan(g.dev(w), g.dev(ws), g.dev(np.zeros(OC, np.int8)), None, strides=(1, 1), pads=(1, 1)), g.to_channels_last(g.dev(x))
+    for dtype, zero_point, rne in [(np.uint8, 128, False), (np.int8, -5, False), (np.uint8, 128, True), (np.uint8, 0, False), (np.int8, 0, True)]:
+        got = plan.run(xd, 0.02, 77, y_scale, zero_point, torch.uint8 if dtype == np.uint8 else torch.int8, flags=g.capi.ROUND_ONNX_RNE if rne else 0)
+        want = oracle.qlinear_conv_int(x, 0.02, 77, w, ws, np.zeros(OC, np.int8), y_scale, zero_point, dtype, pads=(1, 1),
+                                       round_mode=oracle.ROUND_ONNX_RNE if rne else oracle.ROUND_REFERENCE)
+        np.testing.assert_array_equal(g.host(got), want)
+    plan.close()
