@@ -529,6 +529,9 @@ struct ConvCall {
     RequantParams rq2;
     // CHX_HIP_STORE_MINUS_128 for y / y2: the stored byte is the uint8 code minus 128
     bool y_minus_128 = false, y2_minus_128 = false;
+    // x's values before their QuantizeLinear, which the kernel does on the way (x then only describes the codes)
+    const chx_hip_tensor* x_float = nullptr;
+    QuantProduct xq = {};
 };
 
 // Runs the MFMA kernel on packed weights.  x may be channels-last (used in place) or
@@ -571,9 +574,13 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         pw_ = c.p->pad_w_begin, C16eff = C16;
     // few channels read from planar rows: the direct kernel, no expanded matrix
     const bool stem = pw.dense && pw.wd && !c.out_int32 && x.strides[3] == 1 &&
-                      stem_patch_fits(cs.C, cs.KH, cs.KW, sh, sw) && ph < 64 && pw_ < 64 &&
+                      stem_patch_fits(cs.C, cs.KH, cs.KW, sh, sw, pw_) && ph < 64 && pw_ < 64 && cs.W >= 4 &&
                       (int64_t)cs.C * (x.strides[1] < 0 ? -x.strides[1] : x.strides[1]) < (int64_t(1) << 30) &&
                       x.strides[2] > 0 && (int64_t)cs.H * x.strides[2] < (int64_t(1) << 30) && c.opt.stem_kernel;
+    if (c.x_float) {
+        if (!stem || c.rne || !stem_patch_is_small(cs.C, cs.KH, cs.KW, sh, sw, pw_))
+            CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: few channels in planar rows and small filters only");
+    }
     // Channels-last pixels at another pitch than 16 bytes (40 channels packed, say) are copied to one.  The copy's memory is
     // this call's and not the plan's: the direct kernel, which has always taken such arrays, lets one plan run on two streams
     // and inside a recording, pinned or not, and needs none.  A recording keeps that kernel (its memory would have to
@@ -689,8 +696,11 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     if (stem) {
         ConvStemArgs sa;
         memset(&sa, 0, sizeof(sa));
-        sa.x = static_cast<const char*>(x.data);
-        sa.x_n_stride = x.strides[0]; sa.x_c_stride = x.strides[1]; sa.x_h_stride = x.strides[2];
+        const chx_hip_tensor& values = c.x_float ? *c.x_float : x;
+        sa.x = static_cast<const char*>(values.data);
+        sa.x_n_stride = values.strides[0]; sa.x_c_stride = values.strides[1]; sa.x_h_stride = values.strides[2];
+        sa.x_float = c.x_float != nullptr;
+        sa.xq = c.xq;
         sa.N = cs.N; sa.C = cs.C; sa.H = cs.H; sa.W = cs.W; sa.OH = cs.OH; sa.OW = cs.OW; sa.KH = cs.KH; sa.KW = cs.KW;
         sa.sh = sh; sa.sw = sw; sa.ph = ph; sa.pw = pw_;
         sa.OC = cs.OC;
@@ -1390,6 +1400,38 @@ extern "C" int chx_hip_qconv_plan_run(
     }
     if (minus_128) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv: codes minus 128 are stored by the matrix-core and the depthwise kernel only");
     return launch_conv_direct(q.direct, rne, s);
+}
+
+extern "C" int chx_hip_qconv_plan_run_quantize(
+        const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float q_scale, int32_t q_zero_point, float x_scale, int32_t x_zero_point,
+        float y_scale, int32_t y_zero_point, uint32_t flags, chx_hip_tensor* y, void* stream) {
+    CHX_REQUIRE(plan != nullptr, "QuantizeLinear+QLinearConv: null plan");
+    CHX_PROPAGATE(check_tensor(x, "QuantizeLinear+QLinearConv x"));
+    CHX_PROPAGATE(check_tensor(y, "QuantizeLinear+QLinearConv y"));
+    CHX_REQUIRE(x->dtype == CHX_HIP_FLOAT32, "QuantizeLinear+QLinearConv: x must be float32, got %s", dtype_name(x->dtype));
+    CHX_REQUIRE(q_zero_point >= 0 && q_zero_point <= 255, "QuantizeLinear+QLinearConv: zero point %d outside the range of uint8", q_zero_point);
+    if (flags & (CHX_HIP_STORE_MINUS_128 | CHX_HIP_ROUND_ONNX_RNE))
+        CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear+QLinearConv: the reference's rounding and plain codes only");
+    // the codes as they would lie, were there an array of them
+    chx_hip_tensor codes = *x;
+    codes.dtype = CHX_HIP_UINT8;
+    for (int i = 0; i < x->ndim; ++i) {
+        if (x->strides[i] % 4 != 0) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear+QLinearConv: floats at any byte");
+        codes.strides[i] /= 4;
+    }
+    if (reinterpret_cast<uintptr_t>(x->data) % 4 != 0) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear+QLinearConv: floats at any byte");
+    QConvChecked q;
+    CHX_PROPAGATE(check_qconv(&codes, x_scale, x_zero_point, &plan->w, &plan->w_scale, &plan->w_zero_point, y_scale, y_zero_point,
+                              plan->has_bias ? &plan->bias : nullptr, &plan->params, flags, y, &q));
+    if (byte_ranges_overlap(*y, *x)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear+QLinearConv: x and y overlap in memory");
+    const QuantProduct xq = product_form_of_any_value(make_quant_params(q_scale, q_zero_point, false));
+    if (!plan->mfma || xq.path == 0) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear+QLinearConv: no short form of this quantization, or weights for another kernel");
+    ConvCall call = conv_call_from(q, &codes, y, &plan->params, false, plan->opt);
+    call.cache = const_cast<ScratchCache*>(&plan->scratch);
+    call.tune = const_cast<TuneCache*>(&plan->tune);
+    call.x_float = x;
+    call.xq = xq;
+    return run_conv_mfma(call, plan->pw, as_stream(stream));
 }
 
 extern "C" int chx_hip_qconv_plan_run_pair(

@@ -104,8 +104,11 @@ struct ConvMfmaArgs {
 
 // Direct convolution over planar activations with few channels (conv_stem.hip).
 struct ConvStemArgs {
-    // activations, rows contiguous: element (n, c, ih, iw) at x + n*x_n_stride + c*x_c_stride + ih*x_h_stride + iw
+    // activations, rows contiguous: element (n, c, ih, iw) at x + n*x_n_stride + c*x_c_stride + ih*x_h_stride + iw, the strides
+    // in bytes; or (x_float) floats that become uint8 codes by xq on the way into LDS
     const char* x;
+    int32_t x_float;
+    QuantProduct xq;
     int64_t x_n_stride, x_c_stride, x_h_stride;
     int32_t N, C, H, W, OH, OW, KH, KW, sh, sw, ph, pw;
     int32_t OC;
@@ -152,7 +155,8 @@ int launch_im2col_dense(const Im2colArgs& a, hipStream_t s);
 int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, int32_t* padsum, hipStream_t s);
 // the stem kernel: weights [C][KH][KW] with C*KH <= 32 and KW <= 8; patch = LDS bytes of a tile's input rows
 bool stem_shape_fits(int C, int KH, int KW);
-bool stem_patch_fits(int C, int KH, int KW, int sh, int sw);
+bool stem_patch_fits(int C, int KH, int KW, int sh, int sw, int pw);
+bool stem_patch_is_small(int C, int KH, int KW, int sh, int sw, int pw);  // as float32 rows need it
 int stem_k_blocks(int C, int KH, int KW);
 int pack_weights_stem(const chx_hip_tensor& w, int OCpad64, int8_t* wd, hipStream_t s);
 int launch_conv_stem(ConvStemArgs a, bool rne, hipStream_t s);

@@ -70,9 +70,18 @@ static QuantProduct product_with(const QuantParams& q, int path, int ulps, int h
     return p;
 }
 
+// Path 1 for values that may be infinite: inv below the reciprocal and inv_low above 0, so that the two products of an
+// infinity have one sign.
+static QuantProduct product_below(const QuantParams& q) {
+    QuantProduct p = product_with(q, 1, 0, 0);
+    if (p.inv_low < 0.f) p = product_with(q, 1, -1, 0);
+    if (p.inv_low == 0.f) p.inv_low = p.inv * 0x1p-60f;
+    return p;
+}
+
 // The short forms of one quantization (path 0: there is none).
 struct ProductForms {
-    QuantProduct plain, two_fma;
+    QuantProduct plain, two_fma, any_value;
 };
 
 static ProductForms find_forms(const QuantParams& q) {
@@ -81,6 +90,8 @@ static ProductForms find_forms(const QuantParams& q) {
     if (!find_bounds(q, &b)) return f;
     const QuantProduct p = product_with(q, 1, 0, 0);
     if (same_codes(b, p)) f.plain = p;
+    const QuantProduct below = product_below(q);
+    if (below.inv_low > 0.f && same_codes(b, below)) f.any_value = below;
     // (99 of 100 scales have one in this range, most within a few steps)
     for (int i = 0; q.zpf == 0.f && i < 129 * 7 && f.two_fma.path == 0; ++i) {
         const int ring = (i / 7 + 1) / 2;
@@ -120,6 +131,10 @@ QuantProduct product_form(const QuantParams& q, float lo_folded, bool rne, bool 
     if (p.path == 1 && bound) p.path = 2;
     p.floor_half = lo_folded + 0.5f;
     return p;
+}
+
+QuantProduct product_form_of_any_value(const QuantParams& q) {
+    return q.lo != 0.f || q.hi != 255.f ? QuantProduct{} : known_forms(q).any_value;
 }
 
 static thread_local std::string g_last_error;

@@ -243,6 +243,9 @@ struct QuantProduct {
 
 // two_fma: path 3 may be chosen
 QuantProduct product_form(const QuantParams& q, float lo_folded, bool rne, bool two_fma = true);  // core.hip
+// Path 1 (or 0) for a caller's floats, infinities included: t is infinite with their sign.  Only what is not a number is not
+// the reference's (its comparison with the largest code takes it as that).
+QuantProduct product_form_of_any_value(const QuantParams& q);
 
 template <int kPath>
 __device__ __forceinline__ float quantize_prefloor_u8(float v, const QuantProduct& p) {

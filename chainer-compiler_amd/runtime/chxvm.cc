@@ -12,6 +12,7 @@
 
 #include <iostream>
 
+#include "chainerx_util.h"
 #include "chrome_tracing.h"
 
 namespace chainer_compiler {
@@ -563,6 +564,76 @@ private:
     int64_t wide_channels_, next_channels_;
     bool has_bias_;
     Sum sum_;
+    ChxVMSteps steps_;
+    std::vector<int> freed_;
+};
+
+std::atomic<int64_t> g_quantized_convolutions{0};
+
+// A QuantizeLinear and the convolution over few channels that reads its result as one launch (chx_hip_qconv_plan_run_quantize).
+// It stands where the convolution stood; what that kernel does not take runs as the program wrote it.  The operands are
+// constants of the program, laid out when it is loaded.
+class QuantizedConvolutionOp : public ChxVMOp {
+public:
+    struct Quantization {  // variable slots
+        int scale, zp;
+    };
+    // quantize: of the QuantizeLinear (a zero point of -1: none); in, out: of the convolution
+    QuantizedConvolutionOp(const ChxVMInstructionProto& conv, std::shared_ptr<chx_hip_qconv_plan> plan, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
+                           Quantization quantize, Quantization in, Quantization out, ChxVMSteps steps, std::vector<int> freed)
+        : ChxVMOp(conv), plan_(std::move(plan)), params_(params), w_(w), x_(x), y_(conv.outputs[0]), quantize_(quantize), in_(in), out_(out), steps_(std::move(steps)),
+          freed_(std::move(freed)) {
+    }
+
+    void Run(ChxVMState* st) override {
+        if (RunAsOne(st)) {
+            for (int slot : freed_) st->FreeVar(slot);
+        } else {
+            RunSteps(steps_, st);
+        }
+    }
+
+private:
+    static int32_t Integer(const StrictScalar& z) {
+        return static_cast<int32_t>(static_cast<int64_t>(z));
+    }
+
+    // false: nothing has been written
+    bool RunAsOne(ChxVMState* st) {
+        for (int slot : {x_, quantize_.scale, in_.scale, in_.zp, out_.scale, out_.zp})
+            if (st->GetVar(slot)->IsNull()) return false;
+        if (quantize_.zp >= 0 && st->GetVar(quantize_.zp)->IsNull()) return false;
+        const chainerx::Array x = st->GetArray(x_);
+        const absl::optional<StrictScalar> q_zp = st->GetOptionalScalar(quantize_.zp);  // (none: uint8 0)
+        const StrictScalar &x_zp = st->GetScalar(in_.zp), &y_zp = st->GetScalar(out_.zp);
+        auto is_q8 = [](chainerx::Dtype t) { return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8; };
+        if (x.ndim() != 4 || x.dtype() != chainerx::Dtype::kFloat32 || x.shape()[1] != w_.shape()[1] || (q_zp.has_value() && q_zp->dtype() != chainerx::Dtype::kUInt8) ||
+            x_zp.dtype() != chainerx::Dtype::kUInt8 || !is_q8(y_zp.dtype()))
+            return false;
+        const chainerx::Shape y_shape = ConvOutputShape(x, w_, params_);
+        for (int64_t extent : y_shape)
+            if (extent <= 0) return false;
+        chainerx::Array y = chainerx::EmptyChannelsLastPadded(y_shape, y_zp.dtype());
+        const chx_hip_tensor xt = x.hip();
+        chx_hip_tensor yt = y.hip();
+        const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
+        const int rc = chx_hip_qconv_plan_run_quantize(
+                plan_.get(), &xt, static_cast<float>(st->GetScalar(quantize_.scale)), q_zp.has_value() ? Integer(*q_zp) : 0, static_cast<float>(st->GetScalar(in_.scale)),
+                Integer(x_zp), static_cast<float>(st->GetScalar(out_.scale)), Integer(y_zp), flags, &yt, chainerx::CurrentStream());
+        // (what it refuses, and operands that are in error, are for the instructions)
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        st->SetArray(y_, y);
+        ++g_quantized_convolutions;
+        return true;
+    }
+
+    std::shared_ptr<chx_hip_qconv_plan> plan_;
+    chx_hip_conv_params params_;
+    chainerx::Array w_;
+    int x_, y_;
+    Quantization quantize_, in_, out_;
     ChxVMSteps steps_;
     std::vector<int> freed_;
 };
@@ -1167,9 +1238,60 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         remaining_.swap(rest);
     }
+    // QuantizeLinear in front of a convolution over few channels, likewise.
+    for (int q = 0; q < n; ++q) {
+        const ChxVMInstructionProto& qi = program.instructions[q];
+        if (qi.op != kQuantize || role[q] != 0 || chained[q] || !quantization_once(qi)) continue;
+        const int codes = qi.outputs[0], c = codes >= 0 ? conv_reader[codes] : -1;
+        if (c <= q || !single_use(codes) || !convolution(c, false)) continue;
+        const ChxVMInstructionProto& ci = program.instructions[c];
+        const chainerx::Array& w = *constant_array(ci.inputs[3].array);
+        // (the kernel's K axis is channels by filter rows)
+        if (w.ndim() != 4 || w.shape()[1] * w.shape()[2] > 32 || ci.inputs[11].i != 1) continue;
+        const std::vector<int64_t>&strides = ci.inputs[9].ints, &pads = ci.inputs[10].ints;
+        if ((!strides.empty() && strides.size() != 2) || (!pads.empty() && pads.size() != 2 && pads.size() != 4)) continue;
+        auto of = [](const std::vector<int64_t>& v, size_t k, int64_t none) { return static_cast<int32_t>(v.empty() ? none : v[k]); };
+        const chx_hip_conv_params params = {of(strides, 0, 1), of(strides, 1, 1), of(pads, 0, 0), of(pads, 1, 0), of(pads, pads.size() == 4 ? 2 : 0, 0), of(pads, pads.size() == 4 ? 3 : 1, 0), 1};
+        const int bias = ci.inputs[8].array;
+        const chx_hip_tensor wt = w.hip(), scale = constant_array(ci.inputs[4].array)->hip(), zp = constant_array(ci.inputs[5].array)->hip();
+        chx_hip_tensor bt;
+        if (bias >= 0) bt = constant_array(bias)->hip();
+        chx_hip_qconv_plan* plan = nullptr;
+        const int rc = chx_hip_qconv_plan_create(&wt, &scale, &zp, bias >= 0 ? &bt : nullptr, &params, chainerx::CurrentStream(), &plan);
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        std::set<int> slots = {codes, qi.inputs[0].array, qi.inputs[1].scalar, qi.inputs[2].scalar};
+        for (int k : {3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
+        for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
+        std::set<int> moved = {q, c};
+        ChxVMSteps steps;
+        std::vector<int> freed;
+        for (int i = q; i <= c; ++i) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
+                freed.push_back(inst.inputs[0].array);
+                moved.insert(i);
+            }
+            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
+        }
+        chains_.emplace_back(new QuantizedConvolutionOp(ci, std::shared_ptr<chx_hip_qconv_plan>(plan, chx_hip_qconv_plan_destroy), params, w, qi.inputs[0].array,
+                                                        {qi.inputs[1].scalar, qi.inputs[2].scalar}, {ci.inputs[1].scalar, ci.inputs[2].scalar},
+                                                        {ci.inputs[6].scalar, ci.inputs[7].scalar}, std::move(steps), std::move(freed)));
+        chained[q] = chained[c] = true;
+        std::vector<std::pair<int, ChxVMOp*>> rest;
+        for (const auto& r : remaining_) {
+            if (r.first == c) rest.emplace_back(c, chains_.back().get());
+            else if (!moved.count(r.first)) rest.push_back(r);
+        }
+        remaining_.swap(rest);
+    }
 }
 
 ChxVM::~ChxVM() = default;
+
+int64_t QuantizedConvolutions() {
+    return g_quantized_convolutions.load();
+}
 
 int64_t Bottlenecks() {
     return g_bottlenecks.load();

@@ -494,6 +494,7 @@ int64_t chxvm_counter(const char* name) {
     if (n == "minus_128_stores") return Minus128Stores();
     if (n == "matmul_chains") return MatMulChains();
     if (n == "bottlenecks") return Bottlenecks();
+    if (n == "quantized_convolutions") return QuantizedConvolutions();
     if (n == "inverted_residuals") return InvertedResiduals();
     return -1;
 }

@@ -224,6 +224,13 @@ int chx_hip_qconv_plan_create(
 int chx_hip_qconv_plan_run(
         const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, float y_scale,
         int32_t y_zero_point, uint32_t flags, chx_hip_tensor* y, void* stream);
+/* A QuantizeLinear to uint8 (QuantizeLinearOp::RunImpl, runtime/ops/quantize.cc:48-53) and the QLinearConv that is the only reader of its
+ * result, as one launch: the codes of x (float32, any value) by q_scale and q_zero_point are made on the way into the
+ * convolution and never written; y has the bytes that the two ops give.  For the first convolution of an image network: few
+ * channels in planar rows.  CHX_HIP_EUNSUPPORTED for everything else, and when x and y overlap: the caller then runs the two ops. */
+int chx_hip_qconv_plan_run_quantize(
+        const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float q_scale, int32_t q_zero_point, float x_scale, int32_t x_zero_point,
+        float y_scale, int32_t y_zero_point, uint32_t flags, chx_hip_tensor* y, void* stream);
 /* The launch configurations the plan has measured so far, as text into buf (truncated to buf_size - 1
  * characters): one "M=<output pixels> <OH>x<OW> res=<0|1> tile=<oc>x<px> wgs_per_cu=<n, 0 = as many as fit>"
  * per line (followed by "waves=<4|8>", the wavefronts per work-group), and after a chx_hip_qconv_plan_run_add a line
