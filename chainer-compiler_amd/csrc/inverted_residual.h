@@ -26,9 +26,10 @@ struct InvertedResidualArgs {
     ResidualAdd res;              // res.r null: none
     // the launch (filled by plan_inverted_residual)
     int32_t G, lds;  // tiles of 32 expanded channels per interval; bytes of LDS
+    int32_t buffers;  // of expanded and of convolved channels: 2, the three parts for three chunks at a time, or 1
     int32_t R, rows, pitch, pixels, px_bytes, pitch_o, items, tiles_px, tiles_oc, cs, cs2, intervals;
     int32_t at_mask, at_hid, at_dw, at_t3, blocks, strips, xcd_chunk;
-    uint32_t strips_mul, strips_shift, pitch_mul, pitch_shift, pitch_o_mul, pitch_o_shift, w_mul, w_shift, chunks_mul, chunks_shift, oct_mul, oct_shift, blk_mul, blk_shift;
+    uint32_t strips_mul, strips_shift, pitch_mul, pitch_shift, pitch_o_mul, pitch_o_shift, row_mul, row_shift, chunks_mul, chunks_shift, oct_mul, oct_shift, blk_mul, blk_shift;
 };
 
 // From the sizes above; EUNSUPPORTED where the block does not fit (LDS, channels) or single launches are faster.

@@ -5,9 +5,11 @@
 // boundary each.  Here a work-group takes a strip of R output rows of an image, whole width, and walks through the expanded
 // channels in chunks of 32 or 64.  In one interval its eight wavefronts do three things, each for another chunk, with one
 // barrier at the end: expand chunk i into LDS, convolve chunk i - 1 depthwise from LDS into LDS, and multiply chunk i - 2
-// into the projection's sums, which stay in registers.  In us, as three launches inside a graph and as one, over 1, 32 and
-// 128 images: 16 -> 96 -> 24 channels, 112x112 to 56x56, 14.1 and 8.1, 34.8 and 25.1, 97.1 and 71.4; 32 -> 192 -> 32 at
-// 28x28 14.2 and 7.2, 18.0 and 10.8, 37.4 and 20.4; 64 -> 384 -> 64 at 14x14 14.0 and 7.8, 17.0 and 9.1, 24.5 and 16.9;
+// into the projection's sums, which stay in registers.  Wide images take one buffer each for the expanded and the convolved chunk
+// instead of two, which leaves room for more rows: then an interval is the expansion of chunk i and the projection of chunk i - 1,
+// a barrier, the depthwise part of chunk i, a barrier.  In us, as three launches inside a graph and as one, over 1, 32 and
+// 128 images: 16 -> 96 -> 24 channels, 112x112 to 56x56, 14.1 and 8.1, 34.8 and 20.0, 97.1 and 66.8; 32 -> 192 -> 32 at
+// 28x28 14.2 and 7.2, 18.0 and 10.8, 37.4 and 20.2; 64 -> 384 -> 64 at 14x14 14.0 and 7.8, 17.0 and 9.1, 24.5 and 16.9;
 // 160 -> 960 -> 160 at 7x7 13.9 and 12.7, 15.7 and 13.7, 30.3 and 17.1.
 //
 // What bounds it is vector instructions (their pipeline is 0.8 full on 128 images of 112x112 and 56x56; 0.4 at 7x7, where a work-group has the compute unit
@@ -68,9 +70,9 @@ __device__ __forceinline__ void store_first(char* dst, v4i v, int n) {
 }
 
 // kTiles: 32 x 32 tiles of the projection per wavefront, at most; kG: tiles of 32 expanded channels per interval; kKS: K steps
-// of the expansion.
-template <int kStride, int kTiles, int kG, int kKS>
-__global__ __launch_bounds__(64 * kWaves, kTiles == 1 && kG <= 2 ? 4 : 2) void inverted_residual_kernel(InvertedResidualArgs) {
+// of the expansion; kBuffers: of the expanded and of the convolved channels.
+template <int kStride, int kTiles, int kG, int kKS, int kBuffers>
+__global__ __launch_bounds__(64 * kWaves, (kTiles == 1 || (kTiles == 2 && kBuffers == 1)) && kG <= 2 ? 4 : 2) void inverted_residual_kernel(InvertedResidualArgs) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const InvertedResidualArgs& a = kernel_arguments<InvertedResidualArgs>();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -112,29 +114,36 @@ __global__ __launch_bounds__(64 * kWaves, kTiles == 1 && kG <= 2 ? 4 : 2) void i
 
     // ---- the input strip, and what the other buffers need once ----
     {
-        constexpr int kBatch = 4;  // chunks requested before the first is stored
+        // A strip's rows lie behind each other, so that a chunk's place in memory is its number but for what lies between two
+        // pixels' chunks; in LDS there is room behind each pixel and each row.  Rows outside the image are masked later: what is read for them is
+        // the nearest chunk inside.  (Divisions for each chunk's row and pixel, four chunks at a time, were 110 of a wavefront's 1,380 vector
+        // instructions for 16 -> 96 -> 24 at 112x112: 77.8 us for 75.8.)
+        constexpr int kBatch = 2;  // chunks requested before the first is stored
+        const int per_row = a.W * a.x_chunks, total = a.rows * per_row, first = ih0 * per_row, most = a.H * per_row - 1;
+        const int px_room = a.px_bytes - 16 * a.x_chunks, x_room = (int)a.x_px - 16 * a.x_chunks, row_room = (a.pitch - a.W) * a.px_bytes;
         const char* x = a.x + (int64_t)n * a.x_n;
-        const int total = a.rows * a.W * a.x_chunks;
         for (int i0 = tid; i0 < total; i0 += kBatch * 64 * kWaves) {
             v4i v[kBatch];
             int at[kBatch];
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) {
                 const int i = min(i0 + b * 64 * kWaves, total - 1);
-                const int px = (int)fast_div((uint32_t)i, a.chunks_mul, a.chunks_shift), c = i - px * a.x_chunks;
-                const int row = (int)fast_div((uint32_t)px, a.w_mul, a.w_shift), xx = px - row * a.W;
-                const int ih = min(max(ih0 + row, 0), a.H - 1);  // (rows outside the image are masked later)
-                v[b] = *reinterpret_cast<const v4i*>(x + (int64_t)(ih * a.W + xx) * a.x_px + c * 16);
-                at[b] = (row * a.pitch + xx) * a.px_bytes + c * 16;
+                const int chunk = min(max(first + i, 0), most);
+                uint32_t from = (uint32_t)chunk * 16;
+                if (x_room != 0) from += fast_div((uint32_t)chunk, a.chunks_mul, a.chunks_shift) * (uint32_t)x_room;
+                v[b] = *reinterpret_cast<const v4i*>(x + from);
+                at[b] = i * 16 + (int)fast_div((uint32_t)i, a.row_mul, a.row_shift) * row_room;
+                if (px_room != 0) at[b] += (int)fast_div((uint32_t)i, a.chunks_mul, a.chunks_shift) * px_room;
             }
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) *reinterpret_cast<v4i*>(xs + at[b]) = v[b] ^ (int)a.x_flip;
         }
-        for (int p = tid; p < a.pixels; p += 64 * kWaves) {
+        for (int p = tid * 4; p < a.pixels; p += 4 * 64 * kWaves) {  // (a row's pitch is a multiple of 4)
             const int row = (int)fast_div((uint32_t)p, a.pitch_mul, a.pitch_shift), xx = p - row * a.pitch, ih = ih0 + row;
-            mask[p] = ih >= 0 && ih < a.H && xx < a.W ? (char)0xff : (char)0;
+            const int left = ih >= 0 && ih < a.H ? min(max(a.W - xx, 0), 4) : 0;
+            *reinterpret_cast<uint32_t*>(mask + p) = left == 0 ? 0u : 0xffffffffu >> (32 - 8 * left);
         }
-        for (int i = tid; i < 2 * kG * 32; i += 64 * kWaves) *reinterpret_cast<v4i*>(hid + i * a.cs) = v4i{a.fill, a.fill, a.fill, a.fill};
+        for (int i = tid; i < kBuffers * kG * 32; i += 64 * kWaves) *reinterpret_cast<v4i*>(hid + i * a.cs) = v4i{a.fill, a.fill, a.fill, a.fill};
         for (int i = tid; i < 32 * a.tiles_oc; i += 64 * kWaves) {
             const v4i t = *reinterpret_cast<const v4i*>(a.t3 + i * 4);
             s_scale[i] = a.s3 * __int_as_float(t[0]);
@@ -163,114 +172,141 @@ __global__ __launch_bounds__(64 * kWaves, kTiles == 1 && kG <= 2 ? 4 : 2) void i
     // lanes of a group of 16 read 8 channels of 16 pixels, two to a channel, and hold 8 channels of a pixel
     const int in = lane & 15, quarter = lane >> 4;
     const uint32_t dw_from = (uint32_t)(uintptr_t)dw + (uint32_t)((16 * (quarter >> 1) + (in >> 1)) * cs2 + 16 * (quarter & 1) + 8 * (in & 1));
-    for (int i = 0; i < intervals + 2; ++i) {
-        // Memory is read without a branch around it (at the ends: some chunk again), or the compiler waits for everything
-        // where the branches meet.  The fragments of this interval's expansion are there first; the filters of its second and
-        // third part are requested then, and the next expansion's behind this one.
+    auto expand = [&](char* to) __attribute__((always_inline)) {
+        const float scale = s1 * __int_as_float(c1[0]);
+        const int32_t add = c1[1] + corr1 * c1[2];
+        to += 16 + 16 * half;
+        for (int run = share; run < runs; run += kShare) {
+            const char* px = px0 + run * 32 * px_bytes;
+            v4i x[kKS];
 #pragma unroll
-        for (int k = 0; k < kKS; ++k) asm volatile("" : "+v"(w1[k]));
-        asm volatile("" : "+v"(c1));
-        const int32_t* t2 = t2_base + min(max(i - 1, 0), intervals - 1) * kG * 256;
-        const v4i d0 = *reinterpret_cast<const v4i*>(t2);
-        const v2i d1 = *reinterpret_cast<const v2i*>(t2 + 4);
-        const int project = min(max(i - 2, 0), intervals - 1) * kG;
-        v4i w3[kTiles][kG];
+            for (int k = 0; k < kKS; ++k) x[k] = *reinterpret_cast<const v4i*>(px + min(k * 32 + 16 * half, last_chunk));
+            const v4i m = *reinterpret_cast<const v4i*>(mask + run * 32 + 16 * half);
+            v16i sum;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = add;
+#pragma unroll
+            for (int k = 0; k < kKS; ++k) sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[k], w1[k], sum, 0, 0, 0);
+            float pre[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pre[r] = (float)sum[r] * scale;
+            prefloor(pre, q1);
+            uint32_t word[4];
+            floor_sat_u8x16(pre, word);
+            v4i out;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = ((int)(word[e] ^ 0x80808080u) & m[e]) | (fill & ~m[e]);
+            *reinterpret_cast<v4i*>(to + run * 32) = out;
+        }
+    };
+    auto depthwise = [&](v4i d0, v2i d1, const char* from, char* to) __attribute__((always_inline)) {
+        const float scale = s2 * __int_as_float(d0[3]);
+        const int32_t add = d1[0] + corr2 * d1[1];
+        from += 12;  // the dword in front of the first pixel
+        const int w[3] = {d0[0], d0[1], d0[2]}, wu[3] = {d0[0] << 8, d0[1] << 8, d0[2] << 8};
+        for (int item0 = share * 2; item0 < items; item0 += kShare * 2) {
+            const int item = min(item0 + half, items - 1);
+            const int r = (int)fast_div((uint32_t)item, blk_mul, blk_shift), xb = item - r * blocks;
+            const char* src = from + r * kStride * pitch + xb * 8 * kStride;
+            int32_t sum[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = add;
+#pragma unroll
+            for (int f = 0; f < 3; ++f) {
+                const uint32_t* row = reinterpret_cast<const uint32_t*>(src + f * pitch);
+                auto dot = [&](int e, uint32_t v, int weights) __attribute__((always_inline)) { sum[e] = __builtin_amdgcn_sdot4((int)v, weights, sum[e], false); };
+                if constexpr (kStride == 1) {
+                    const uint32_t b = row[0], p = row[1], q1 = row[2], nx = row[3];
+                    dot(0, __builtin_amdgcn_alignbyte(p, b, 3), w[f]);
+                    dot(1, p, w[f]);
+                    dot(2, p, wu[f]);
+                    dot(3, __builtin_amdgcn_alignbyte(q1, p, 2), w[f]);
+                    dot(4, __builtin_amdgcn_alignbyte(q1, p, 3), w[f]);
+                    dot(5, q1, w[f]);
+                    dot(6, q1, wu[f]);
+                    dot(7, __builtin_amdgcn_alignbyte(nx, q1, 2), w[f]);
+                } else {
+                    uint32_t v[5];
+#pragma unroll
+                    for (int e = 0; e < 5; ++e) v[e] = row[e];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        dot(2 * e, __builtin_amdgcn_alignbyte(v[e + 1], v[e], 3), w[f]);
+                        dot(2 * e + 1, v[e + 1], wu[f]);
+                    }
+                }
+            }
+            float pre[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pre[e] = (float)sum[e] * scale;
+            prefloor(pre, q2);
+            uint32_t lo, hi;
+            floor_sat_u8x8(pre, &lo, &hi);
+            *reinterpret_cast<v2i*>(to + r * pitch_o + xb * 8) = v2i{(int)(lo ^ 0x80808080u), (int)(hi ^ 0x80808080u)};
+        }
+    };
+    v4i w3[kTiles][kG];  // the projection's filters for a chunk
+    auto fetch3 = [&](int chunk) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-            for (int k = 0; k < kG; ++k) w3[t][k] = *reinterpret_cast<const v4i*>(w3_at[t] + (project + k) * 1024);
-        if (i < intervals) {
-            const float scale = s1 * __int_as_float(c1[0]);
-            const int32_t add = c1[1] + corr1 * c1[2];
-            char* to = hid_lane + (i & 1) * cs_chunk + 16 + 16 * half;
-            for (int run = share; run < runs; run += kShare) {
-                const char* px = px0 + run * 32 * px_bytes;
-                v4i x[kKS];
+            for (int k = 0; k < kG; ++k) w3[t][k] = *reinterpret_cast<const v4i*>(w3_at[t] + (chunk * kG + k) * 1024);
+    };
+    auto project = [&](uint32_t from) __attribute__((always_inline)) {
 #pragma unroll
-                for (int k = 0; k < kKS; ++k) x[k] = *reinterpret_cast<const v4i*>(px + min(k * 32 + 16 * half, last_chunk));
-                const v4i m = *reinterpret_cast<const v4i*>(mask + run * 32 + 16 * half);
-                v16i sum;
+        for (int t = 0; t < kTiles; ++t) {
+            if (wave + kWaves * t >= tiles) break;
+            v2i lo[kG], hi[kG];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sum[r] = add;
-#pragma unroll
-                for (int k = 0; k < kKS; ++k) sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[k], w1[k], sum, 0, 0, 0);
-                float pre[16];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) pre[r] = (float)sum[r] * scale;
-                prefloor(pre, q1);
-                uint32_t word[4];
-                floor_sat_u8x16(pre, word);
-                v4i out;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) out[e] = ((int)(word[e] ^ 0x80808080u) & m[e]) | (fill & ~m[e]);
-                *reinterpret_cast<v4i*>(to + run * 32) = out;
+            for (int k = 0; k < kG; ++k) {
+                const uint32_t at = from + (uint32_t)(k * 32 * cs2 + tile_px[t] * 32);
+                lo[k] = transposed8(at);
+                hi[k] = transposed8(at + 8 * (uint32_t)cs2);
             }
+#pragma unroll
+            for (int k = 0; k < kG; ++k) acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w3[t][k], v4i{lo[k][0], lo[k][1], hi[k][0], hi[k][1]}, acc[t], 0, 0, 0);
         }
-        fetch1(min(i + 1, intervals - 1));
-        if (i >= 1 && i <= intervals) {
-            const float scale = s2 * __int_as_float(d0[3]);
-            const int32_t add = d1[0] + corr2 * d1[1];
-            const char* from = hid_lane + ((i - 1) & 1) * cs_chunk + 12;  // the dword in front of the first pixel
-            char* to = dw_lane + ((i - 1) & 1) * cs2_chunk;
-            const int w[3] = {d0[0], d0[1], d0[2]}, wu[3] = {d0[0] << 8, d0[1] << 8, d0[2] << 8};
-            for (int item0 = share * 2; item0 < items; item0 += kShare * 2) {
-                const int item = min(item0 + half, items - 1);
-                const int r = (int)fast_div((uint32_t)item, blk_mul, blk_shift), xb = item - r * blocks;
-                const char* src = from + r * kStride * pitch + xb * 8 * kStride;
-                int32_t sum[8];
+    };
+    auto fetch2 = [&](int chunk, v4i* d0, v2i* d1) __attribute__((always_inline)) {
+        const int32_t* t2 = t2_base + chunk * kG * 256;
+        *d0 = *reinterpret_cast<const v4i*>(t2);
+        *d1 = *reinterpret_cast<const v2i*>(t2 + 4);
+    };
+    // Memory is read without a branch around it (at the ends: some chunk again), or the compiler waits for everything
+    // where the branches meet.  The fragments of this interval's expansion are there first; the filters of its second and
+    // third part are requested then, and the next expansion's behind this one.
+    auto expansion_is_there = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) sum[e] = add;
-#pragma unroll
-                for (int f = 0; f < 3; ++f) {
-                    const uint32_t* row = reinterpret_cast<const uint32_t*>(src + f * pitch);
-                    auto dot = [&](int e, uint32_t v, int weights) __attribute__((always_inline)) { sum[e] = __builtin_amdgcn_sdot4((int)v, weights, sum[e], false); };
-                    if constexpr (kStride == 1) {
-                        const uint32_t b = row[0], p = row[1], q1 = row[2], nx = row[3];
-                        dot(0, __builtin_amdgcn_alignbyte(p, b, 3), w[f]);
-                        dot(1, p, w[f]);
-                        dot(2, p, wu[f]);
-                        dot(3, __builtin_amdgcn_alignbyte(q1, p, 2), w[f]);
-                        dot(4, __builtin_amdgcn_alignbyte(q1, p, 3), w[f]);
-                        dot(5, q1, w[f]);
-                        dot(6, q1, wu[f]);
-                        dot(7, __builtin_amdgcn_alignbyte(nx, q1, 2), w[f]);
-                    } else {
-                        uint32_t v[5];
-#pragma unroll
-                        for (int e = 0; e < 5; ++e) v[e] = row[e];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            dot(2 * e, __builtin_amdgcn_alignbyte(v[e + 1], v[e], 3), w[f]);
-                            dot(2 * e + 1, v[e + 1], wu[f]);
-                        }
-                    }
-                }
-                float pre[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) pre[e] = (float)sum[e] * scale;
-                prefloor(pre, q2);
-                uint32_t lo, hi;
-                floor_sat_u8x8(pre, &lo, &hi);
-                *reinterpret_cast<v2i*>(to + r * pitch_o + xb * 8) = v2i{(int)(lo ^ 0x80808080u), (int)(hi ^ 0x80808080u)};
-            }
+        for (int k = 0; k < kKS; ++k) asm volatile("" : "+v"(w1[k]));
+        asm volatile("" : "+v"(c1));
+    };
+    v4i d0;
+    v2i d1;
+    if constexpr (kBuffers == 2) {
+        for (int i = 0; i < intervals + 2; ++i) {
+            expansion_is_there();
+            fetch2(min(max(i - 1, 0), intervals - 1), &d0, &d1);
+            fetch3(min(max(i - 2, 0), intervals - 1));
+            if (i < intervals) expand(hid_lane + (i & 1) * cs_chunk);
+            fetch1(min(i + 1, intervals - 1));
+            if (i >= 1 && i <= intervals) depthwise(d0, d1, hid_lane + ((i - 1) & 1) * cs_chunk, dw_lane + ((i - 1) & 1) * cs2_chunk);
+            if (i >= 2) project(dw_from + (uint32_t)((i & 1) * cs2_chunk));
+            __syncthreads();
         }
-        if (i >= 2) {
-            const uint32_t from = dw_from + (uint32_t)((i & 1) * cs2_chunk);
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t) {
-                if (wave + kWaves * t >= tiles) break;
-                v2i lo[kG], hi[kG];
-#pragma unroll
-                for (int k = 0; k < kG; ++k) {
-                    const uint32_t at = from + (uint32_t)(k * 32 * cs2 + tile_px[t] * 32);
-                    lo[k] = transposed8(at);
-                    hi[k] = transposed8(at + 8 * (uint32_t)cs2);
-                }
-#pragma unroll
-                for (int k = 0; k < kG; ++k) acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w3[t][k], v4i{lo[k][0], lo[k][1], hi[k][0], hi[k][1]}, acc[t], 0, 0, 0);
-            }
+    } else {
+        for (int i = 0;; ++i) {
+            expansion_is_there();
+            if (kTiles == 1) fetch3(max(i - 1, 0));
+            if (i < intervals) expand(hid_lane);
+            if (kTiles != 1) fetch3(max(i - 1, 0));  // (in front of the expansion they are registers too many)
+            fetch2(min(i, intervals - 1), &d0, &d1);
+            fetch1(min(i + 1, intervals - 1));
+            if (i >= 1) project(dw_from);
+            if (i == intervals) break;
+            __syncthreads();
+            depthwise(d0, d1, hid_lane, dw_lane);
+            __syncthreads();
         }
-        __syncthreads();
     }
 
     // ---- the projection's sums ----
@@ -358,8 +394,9 @@ int odd16(int bytes) {  // an odd number of 16 bytes
 }
 
 // What a work-group of R output rows needs: fills the launch's fields, returns its LDS bytes.
-int lay_out(InvertedResidualArgs& a, int stride, int R, int G) {
+int lay_out(InvertedResidualArgs& a, int stride, int R, int G, int buffers) {
     a.R = R;
+    a.buffers = buffers;
     a.rows = (R - 1) * stride + 3;
     a.pitch = (a.W + 1 + 3) / 4 * 4;
     a.pixels = (a.rows * a.pitch + 31) / 32 * 32;
@@ -375,26 +412,29 @@ int lay_out(InvertedResidualArgs& a, int stride, int R, int G) {
     a.strips = (a.OH + R - 1) / R;
     a.at_mask = a.pixels * a.px_bytes;
     a.at_hid = a.at_mask + a.pixels;
-    a.at_dw = a.at_hid + 2 * G * 32 * a.cs;
-    a.at_t3 = a.at_dw + 2 * G * 32 * a.cs2;
+    a.at_dw = a.at_hid + buffers * G * 32 * a.cs;
+    a.at_t3 = a.at_dw + buffers * G * 32 * a.cs2;
     return a.at_t3 + 32 * a.tiles_oc * 8;
 }
 
 constexpr int kLdsOfUnit = 160 * 1024;
 
-template <int kStride, int kTiles, int kG, int kKS>
+template <int kStride, int kTiles, int kG, int kKS, int kBuffers>
 int launch(const InvertedResidualArgs& a, int bytes, hipStream_t s) {
     // (more than 64 KB has to be asked for, on every device)
     if (bytes > 64 * 1024)
-        CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&inverted_residual_kernel<kStride, kTiles, kG, kKS>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfUnit));
-    inverted_residual_kernel<kStride, kTiles, kG, kKS><<<8 * a.xcd_chunk, 64 * kWaves, bytes, s>>>(a);
+        CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&inverted_residual_kernel<kStride, kTiles, kG, kKS, kBuffers>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfUnit));
+    inverted_residual_kernel<kStride, kTiles, kG, kKS, kBuffers><<<8 * a.xcd_chunk, 64 * kWaves, bytes, s>>>(a);
     return launch_check("inverted_residual_kernel");
 }
 
-template <int kTiles, int kG>
+template <int kTiles, int kG, int kBuffers>
 int launch_steps(const InvertedResidualArgs& a, int stride, int bytes, hipStream_t s) {
-    if (stride == 1) return a.KS == 1 ? launch<1, kTiles, kG, 1>(a, bytes, s) : a.KS == 3 ? launch<1, kTiles, kG, 3>(a, bytes, s) : launch<1, kTiles, kG, 5>(a, bytes, s);
-    return a.KS == 1 ? launch<2, kTiles, kG, 1>(a, bytes, s) : a.KS == 3 ? launch<2, kTiles, kG, 3>(a, bytes, s) : launch<2, kTiles, kG, 5>(a, bytes, s);
+    if constexpr (kBuffers == 2) {
+        if (a.KS == 5) return stride == 1 ? launch<1, kTiles, kG, 5, kBuffers>(a, bytes, s) : launch<2, kTiles, kG, 5, kBuffers>(a, bytes, s);
+    }
+    if (stride == 1) return a.KS == 1 ? launch<1, kTiles, kG, 1, kBuffers>(a, bytes, s) : launch<1, kTiles, kG, 3, kBuffers>(a, bytes, s);
+    return a.KS == 1 ? launch<2, kTiles, kG, 1, kBuffers>(a, bytes, s) : launch<2, kTiles, kG, 3, kBuffers>(a, bytes, s);
 }
 
 // The two sides of whether the block is one launch, in us, fitted to 1,059 blocks of 8 to 160 channels, expanded 1 to 6 times, to 8 to
@@ -440,40 +480,64 @@ int plan_inverted_residual(InvertedResidualArgs* launch, int stride) {
     // projection's own launch has its channels spread over the chip: 160 -> 960 -> 320 at 7x7 takes, as three launches and as
     // one, 14.1 and 16.9 us on 1 image, 15.6 and 19.2 on 32, 19.0 and 19.2 on 64 (448 rows), 28.5 and 23.7 on 128 (896 rows).
     if ((a.OC + 31) / 32 > kWaves && (int64_t)a.N * a.OH < 512) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: too few rows for so many channels");
-    int best = 0, best_g = 1;
+    //
+    // With one buffer of each kind (the kernel's kBuffers) LDS holds about twice the rows: 16 -> 96 -> 24 at 112x112 takes four per strip
+    // for two, and expands nine rows where it expanded ten; the price is a second barrier per interval.  In us with two and with one, 128
+    // images: 77.5 and 63.2 (16 -> 96 -> 24 at 112x112), 68.1 and 63.1 (24 -> 144 -> 24 at 56x56), 23.7 and 21.4 (32 -> 192 -> 32 at 28x28);
+    // 64 images 48.9 and 37.5, 39.1 and 33.6, 15.5 and 15.2; 14x14 and 7x7, where a strip is most of an image anyway, 18.4
+    // and 19.0.  The constants are those of 182 blocks on 1 to 128 images, each with all rows and tiles measured: of 31 that take one
+    // buffer none was slower, the most 0.60 of the time.  Where one round does not fill the chip a second barrier is all it is.
+    // (160 input channels, and two tiles of the projection with other than 16 or 32 input channels, do not fit the registers.)
+    int best = 0, best_g = 1, best_buffers = 2, rows_of_two = 0, tiles_of_two = 1;
     double least = 0;
-    for (int G = 1; G <= 8; G *= 2) {
-        if (G > 1 && G / 2 >= a.hid_tiles) break;
-        for (int R = 1; R <= a.OH && R <= 16; ++R) {
-            const int bytes = lay_out(a, stride, R, G), tiles = a.tiles_px * a.tiles_oc;
-            if (bytes > kLdsOfUnit || tiles > kMostTiles * kWaves || (G == 8 && tiles > 2 * kWaves)) continue;
-            const int64_t blocks = (int64_t)a.strips * a.N;
-            const int per = kWaves / G;  // wavefronts that share the runs and items of a tile of channels
-            auto shares = [](int n, int by) { return (double)((n + by - 1) / by); };
-            const double interval = shares(a.pixels / 32, per) * (120.0 + 14.0 * a.KS) + shares((a.items + 1) / 2, per) * 132.0 + shares(tiles, kWaves) * 13.0 * G + 190.0;
-            const double work = (a.intervals + 2) * interval + 850.0 + a.rows * a.W * a.x_chunks / 512 * 25.0;
-            const bool two = 2 * bytes <= kLdsOfUnit && tiles <= kWaves && G <= 2 && blocks > 256;  // work-groups on a compute unit at once
-            const double cost = two ? (blocks > 2048 ? blocks / 512.0 : (double)((blocks + 511) / 512)) * 1.232 * work : (double)((blocks + 255) / 256) * work;
-            if (best == 0 || cost < least) {
-                least = cost;
-                best = R;
-                best_g = G;
+    for (int buffers = 2; buffers >= 1; --buffers) {
+        for (int G = 1; G <= (buffers == 1 ? 2 : 8); G *= 2) {
+            if (G > 1 && G / 2 >= a.hid_tiles) break;
+            for (int R = 1; R <= a.OH && R <= 16; ++R) {
+                const int bytes = lay_out(a, stride, R, G, buffers), tiles = a.tiles_px * a.tiles_oc;
+                const int64_t blocks = (int64_t)a.strips * a.N;
+                if (bytes > kLdsOfUnit || tiles > kMostTiles * kWaves || (G == 8 && tiles > 2 * kWaves)) continue;
+                if (buffers == 1 && (blocks <= 256 || a.KS == 5 || tiles > (G == 1 && a.KS == 1 ? 2 : 1) * kWaves)) continue;
+                const int per = kWaves / G;  // wavefronts that share the runs and items of a tile of channels
+                auto shares = [](int n, int by) { return (double)((n + by - 1) / by); };
+                const double interval = shares(a.pixels / 32, per) * (120.0 + 14.0 * a.KS) + shares((a.items + 1) / 2, per) * 132.0 + shares(tiles, kWaves) * 13.0 * G + (buffers == 2 ? 190.0 : 300.0);
+                const double work = (a.intervals + (buffers == 2 ? 2.0 : 0.5)) * interval + (buffers == 2 ? 850.0 : 1300.0) + a.rows * a.W * a.x_chunks / 512 * 25.0;
+                const bool two = 2 * bytes <= kLdsOfUnit && (buffers == 1 || (tiles <= kWaves && G <= 2)) && blocks > 256;  // work-groups on a compute unit at once
+                const double cost = two ? (blocks > 2048 ? blocks / 512.0 : (double)((blocks + 511) / 512)) * (buffers == 2 ? 1.232 : 1.3) * work : (double)((blocks + 255) / 256) * work;
+                if (best == 0 || cost < least) {
+                    least = cost;
+                    best = R;
+                    best_g = G;
+                    best_buffers = buffers;
+                }
             }
+        }
+        if (buffers == 2) {
+            rows_of_two = best;
+            tiles_of_two = best_g;
         }
     }
     if (best == 0) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: a row does not fit");
+    // (the estimate for one buffer is within 14 %: what two would be refused for has to be that much better)
+    double here = best_buffers == 1 ? 1.15 * (0.7 + 2.35e-3 * least) : 0.0;
+    if (rows_of_two != 0) {
+        a.G = tiles_of_two;
+        a.lds = lay_out(a, stride, rows_of_two, tiles_of_two, 2);
+        const double two = time_of_block(a, (int64_t)a.strips * a.N);
+        here = best_buffers == 1 ? std::min(here, two) : two;
+    }
+    const double launches = time_of_launches(a);  // (up to 16 us most of it is that they are three)
+    if (here > (launches < 16.0 ? launches + 2.3 : 0.93 * launches + 1.0)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: slower than its convolutions");
     a.G = best_g;
-    a.lds = lay_out(a, stride, best, best_g);
+    a.lds = lay_out(a, stride, best, best_g, best_buffers);
     const int64_t blocks = (int64_t)a.strips * a.N;
     if (blocks >= (int64_t(1) << 28)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: 2^28 strips or more");
-    const double launches = time_of_launches(a);  // (up to 16 us most of it is that they are three)
-    if (time_of_block(a, blocks) > (launches < 16.0 ? launches + 2.3 : 0.93 * launches + 1.0)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "inverted residual: slower than its convolutions");
     a.blocks = (int32_t)blocks;
     a.xcd_chunk = (int32_t)((blocks + 7) / 8);
     magic_divisor((uint32_t)a.strips, &a.strips_mul, &a.strips_shift);
     magic_divisor((uint32_t)a.pitch, &a.pitch_mul, &a.pitch_shift);
     magic_divisor((uint32_t)a.pitch_o, &a.pitch_o_mul, &a.pitch_o_shift);
-    magic_divisor((uint32_t)a.W, &a.w_mul, &a.w_shift);
+    magic_divisor((uint32_t)(a.W * a.x_chunks), &a.row_mul, &a.row_shift);
     magic_divisor((uint32_t)a.x_chunks, &a.chunks_mul, &a.chunks_shift);
     magic_divisor((uint32_t)a.tiles_oc, &a.oct_mul, &a.oct_shift);
     magic_divisor((uint32_t)(a.pitch_o / 8), &a.blk_mul, &a.blk_shift);
@@ -482,19 +546,23 @@ int plan_inverted_residual(InvertedResidualArgs* launch, int stride) {
 
 int launch_inverted_residual(const InvertedResidualArgs& a, int stride, hipStream_t s) {
     const int bytes = a.lds, per_wave = (a.tiles_px * a.tiles_oc + kWaves - 1) / kWaves;
+    if (a.buffers == 1) {
+        if (per_wave == 2) return stride == 1 ? launch<1, 2, 1, 1, 1>(a, bytes, s) : launch<2, 2, 1, 1, 1>(a, bytes, s);
+        return a.G == 1 ? launch_steps<1, 1, 1>(a, stride, bytes, s) : launch_steps<1, 2, 1>(a, stride, bytes, s);
+    }
     if (per_wave == 1) {
         switch (a.G) {
-            case 1: return launch_steps<1, 1>(a, stride, bytes, s);
-            case 2: return launch_steps<1, 2>(a, stride, bytes, s);
-            case 4: return launch_steps<1, 4>(a, stride, bytes, s);
-            default: return launch_steps<1, 8>(a, stride, bytes, s);
+            case 1: return launch_steps<1, 1, 2>(a, stride, bytes, s);
+            case 2: return launch_steps<1, 2, 2>(a, stride, bytes, s);
+            case 4: return launch_steps<1, 4, 2>(a, stride, bytes, s);
+            default: return launch_steps<1, 8, 2>(a, stride, bytes, s);
         }
     }
     switch (a.G) {
-        case 1: return launch_steps<kMostTiles, 1>(a, stride, bytes, s);
-        case 2: return launch_steps<kMostTiles, 2>(a, stride, bytes, s);
-        case 4: return launch_steps<kMostTiles, 4>(a, stride, bytes, s);
-        default: return launch_steps<2, 8>(a, stride, bytes, s);  // (the filters of three tiles do not fit the registers)
+        case 1: return launch_steps<kMostTiles, 1, 2>(a, stride, bytes, s);
+        case 2: return launch_steps<kMostTiles, 2, 2>(a, stride, bytes, s);
+        case 4: return launch_steps<kMostTiles, 4, 2>(a, stride, bytes, s);
+        default: return launch_steps<2, 8, 2>(a, stride, bytes, s);  // (the filters of three tiles do not fit the registers)
     }
 }
 
