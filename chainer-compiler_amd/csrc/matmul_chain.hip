@@ -6,7 +6,7 @@
 // own 3.5 to 4 us with the hand-over from the kernel before it, and its host side another 2.5.  Here a work-group takes
 // 16 rows through all layers: the codes between them stay in LDS, and the weights of a layer are requested before the sums of
 // the layer before it are requantized, so that only the first layer waits for memory.  784 -> 100 -> 100 -> 10 over 32 rows
-// 17.0 -> 8.9 us, Program.run of it, with the result on the host, 27-31 -> 19.6.
+// 17.0 -> 8.5 us, Program.run of it, with the result on the host, 27-31 -> 19.5.
 //
 // The weights are laid out once, as fragments of v_mfma_i32_16x16x64_i8 (1 KB for 64 k of 16 columns, a lane's 16 bytes
 // together), zeros where a matrix ends, and behind them the sum of each column: read as they lie, a step took 100
@@ -153,6 +153,12 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_chain_kernel(ChainArgs) {
 
     for (int l = 0; l < g.layers; ++l) {
         const ChainLayer& L = g.layer[l];
+        // the columns' sums that this thread's codes take, before anything is waited for (asked for where they are used, behind the barrier,
+        // they are a memory latency per layer: 8.9 us for 8.5 at 784 -> 100 -> 100 -> 10 over 32 rows)
+        const v4i* columns = reinterpret_cast<const v4i*>(L.b + (int64_t)L.tiles * L.steps * 1024);
+        v4i of_column[kMaxN / 256];
+#pragma unroll
+        for (int i = 0; i < kMaxN / 256; ++i) of_column[i] = columns[min(lane + 64 * i, L.tiles * 4 - 1)];
         if (p.count > 0) {
             v4i acc = {0, 0, 0, 0};
             int step = p.first, tile = p.tile;
@@ -190,17 +196,19 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_chain_kernel(ChainArgs) {
             for (int d = 1; d < 64; d *= 2) s += __shfl_xor(s, d);
             of_row = L.cb * (s + L.K * L.ca);
         }
-        const v4i* columns = reinterpret_cast<const v4i*>(L.b + (int64_t)L.tiles * L.steps * 1024);
         if (!last) {
             p = part_of(g.layer[l + 1]);
             load_first();
         }
         __syncthreads();
         const int padded = last ? L.tiles * 16 : (L.tiles + 3) / 4 * 64;
-        for (int n = 4 * lane; n < padded; n += 256) {
+#pragma unroll
+        for (int i = 0; i < kMaxN / 256; ++i) {
+            const int n = 4 * lane + 256 * i;
+            if (n >= padded) break;
             v4i* at = reinterpret_cast<v4i*>(&sum[wave * kSumRow + n]);
             v4i v = *at + of_row;
-            if (L.ca != 0 && n < L.N) v += L.ca * columns[n / 4];
+            if (n < L.N) v += L.ca * of_column[i];
             int32_t code[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) code[e] = quantize_value_folded<false>((float)v[e] * L.scale, L.q, L.inv_scale, L.q.lo);
