@@ -133,7 +133,7 @@ def sizes(host):
 
 
 SIZES = [((64, 256, 64), 1, 56, True), ((64, 256, 64), 64, 56, True), ((128, 512, 128), 1, 28, True), ((128, 512, 128), 64, 28, True), ((256, 1024, 256), 64, 14, True),
-         ((256, 1024, 256), 1, 14, False), ((64, 1024, 64), 8, 7, False)]
+         ((256, 1024, 256), 1, 14, False), ((256, 1024, 256), 8, 14, True), ((256, 1024, 512), 8, 14, False), ((64, 1024, 64), 8, 7, False)]
 
 
 def nothing_launched(host):
