@@ -363,7 +363,7 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
     std::vector<Candidate> all;
     for (const auto& t : tiles) {
         if (a.OC <= 64 && t[0] > 64) continue;
-        if (a.oc_split % t[0] != 0) continue;  // two outputs: a tile belongs to one of them whole
+        if (a.oc_split % t[0] != 0) continue;  // two outputs: a tile belongs to one of them whole (floats: none of these)
         if (t[2] == 8 && (t[0] == 64 || t[1] == 256) && a.bk != 128) continue;
         const int64_t tiles_all = (int64_t)((a.OC + t[0] - 1) / t[0]) * ((a.M + t[1] - 1) / t[1]);
         all.push_back({{t[0], t[1], 0, t[2]}, {}});
@@ -383,7 +383,7 @@ int tune_conv_mfma(const ConvMfmaArgs& a, bool xu, bool out_int32, bool rne, hip
     if (!out_int32 && !rne)
         for (const ConvSplitTile& t : kConvSameTiles)
             if (conv_same_takes(a, t.px) && (a.OC > 64 || t.oc == 64)) all.push_back({{t.oc, t.px, kConvSame, t.waves}, {}});
-    if (!out_int32 && conv_point_takes(a))
+    if (!out_int32 && a.oc_split != kFloatResults && conv_point_takes(a))
         for (int per_cu : {2, 4, 6}) all.push_back({{kConvPointTile.oc, kConvPointTile.px, per_cu, kConvPointTile.waves}, {}});
 
     std::vector<hipEvent_t> events(2 * all.size());
@@ -532,6 +532,10 @@ struct ConvCall {
     // x's values before their QuantizeLinear, which the kernel does on the way (x then only describes the codes)
     const chx_hip_tensor* x_float = nullptr;
     QuantProduct xq = {};
+    // where the result goes as floats (y then only describes its codes)
+    float* dq = nullptr;
+    int64_t dq_px = 0;
+    float dq_zpf = 0.f, dq_scale = 0.f;
 };
 
 // Runs the MFMA kernel on packed weights.  x may be channels-last (used in place) or
@@ -598,6 +602,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         own.ptr[0] = own_memory.ptr();
         own.ptr[1] = static_cast<char*>(own_memory.ptr()) + own.size[0];
     }
+    if (c.dq && (stem || pixels_copied || c.out_int32 || c.res || c.y2)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: channels-last arrays of at least 16 channels only");
     if (stem && c.res) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "the planar-input kernel has no fused residual sum");
     if (stem) {
         // x is used in place
@@ -769,9 +774,22 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     }
     if (c.res) a.res = *c.res;
     CHX_REQUIRE(a.M < (int64_t(1) << 31), "QLinearConv: too many output pixels for the MFMA kernel");
+    if (c.dq) {
+        a.oc_split = kFloatResults;
+        a.y2 = reinterpret_cast<char*>(c.dq);
+        a.y2_px_stride = c.dq_px;
+        a.inv_y_scale2 = c.dq_zpf;
+        a.lo_folded2 = c.dq_scale;
+    }
     int toc = 64, tpx = 64, cap = 0, waves = 4;
     pick_tile(c.opt, a, c.out_int32, &toc, &tpx, &cap, &waves);
-    if (a.oc_split % toc != 0) toc = 64, waves = 4, tpx = tpx > 128 ? 128 : tpx;  // (the split is a multiple of 64)
+    if (a.oc_split == kFloatResults) {
+        if (!conv_split_takes(a) || (int64_t)((a.OC + 63) / 64) * ((a.M + 63) / 64) > 2048) {
+            release_scratch(cache, x_scratch, s);
+            CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: not one for the small tiles");
+        }
+        if (!conv_split_has(toc, tpx, waves)) toc = 32, tpx = 32, cap = 0, waves = 2;
+    } else if (a.oc_split % toc != 0) toc = 64, waves = 4, tpx = tpx > 128 ? 128 : tpx;  // (the split is a multiple of 64)
     int rc = CHX_HIP_OK;
     const TunedConfig* tuned = nullptr;
     if (c.tune) {
@@ -1357,6 +1375,10 @@ extern "C" int chx_hip_qconv_plan_create(
 
 namespace chx {
 namespace {
+// Results that chx_hip_qconv_plan_run_dequantize takes.  Two launches and one inside a recording, us: 8 x 2048 -> 1000 7.3 and 5.3, 128 x 1280
+// -> 1000 8.5 and 5.9, 512 x 2048 -> 1000 14.8 and 8.5, 100 x 4096 -> 4096 15.1 and 12.8; beyond, the small tiles read their operands too often:
+// 4 x 2048 -> 256 at 32x32 (a million results) 12.4 and 16.0, 8 x 1024 -> 512 at 28x28 14.2 and 24.3.
+constexpr int64_t kMostFloats = 1 << 19;
 // CHX_HIP_STORE_MINUS_128: the array is int8, its quantization is that of the uint8 array it stands for.  *view is what
 // the checks and the requantization parameters are derived from.
 int result_view(const chx_hip_tensor* y, uint32_t flags, const char* op, chx_hip_tensor* view, bool* minus_128) {
@@ -1431,6 +1453,40 @@ extern "C" int chx_hip_qconv_plan_run_quantize(
     call.tune = const_cast<TuneCache*>(&plan->tune);
     call.x_float = x;
     call.xq = xq;
+    return run_conv_mfma(call, plan->pw, as_stream(stream));
+}
+
+extern "C" int chx_hip_qconv_plan_run_dequantize(
+        const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, float y_scale, int32_t y_zero_point, int32_t y_dtype,
+        uint32_t flags, float dq_scale, int32_t dq_zero_point, chx_hip_tensor* y, void* stream) {
+    CHX_REQUIRE(plan != nullptr, "QLinearConv+DequantizeLinear: null plan");
+    CHX_PROPAGATE(check_tensor(x, "QLinearConv+DequantizeLinear x"));
+    CHX_PROPAGATE(check_tensor(y, "QLinearConv+DequantizeLinear y"));
+    CHX_REQUIRE(y->dtype == CHX_HIP_FLOAT32, "QLinearConv+DequantizeLinear: y must be float32, got %s", dtype_name(y->dtype));
+    CHX_REQUIRE(is_q8(y_dtype), "QLinearConv+DequantizeLinear: the codes must be uint8 or int8");
+    if (flags & CHX_HIP_STORE_MINUS_128) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: plain codes only");
+    // the codes as they would lie, were there an array of them
+    chx_hip_tensor codes = *y;
+    codes.dtype = y_dtype;
+    bool whole = reinterpret_cast<uintptr_t>(y->data) % 4 == 0;
+    for (int i = 0; i < y->ndim; ++i) {
+        whole = whole && y->strides[i] % 4 == 0;
+        codes.strides[i] /= 4;
+    }
+    QConvChecked q;
+    CHX_PROPAGATE(check_qconv(x, x_scale, x_zero_point, &plan->w, &plan->w_scale, &plan->w_zero_point, y_scale, y_zero_point,
+                              plan->has_bias ? &plan->bias : nullptr, &plan->params, flags, &codes, &q));
+    int64_t px = 0;
+    if (!plan->mfma || !whole || !y_is_pixel_major(codes, &px) || plan->w.shape[2] != 1 || plan->w.shape[3] != 1 || numel(codes) > kMostFloats || byte_ranges_overlap(*y, *x) ||
+        (plan->opt.forced_tile && !conv_split_has(plan->opt.tile_oc, plan->opt.tile_px, plan->opt.waves)))
+        CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: 1x1 filters, few channels-last results that do not overlap x");
+    ConvCall call = conv_call_from(q, x, &codes, &plan->params, (flags & CHX_HIP_ROUND_ONNX_RNE) != 0, plan->opt);
+    call.cache = const_cast<ScratchCache*>(&plan->scratch);
+    call.tune = const_cast<TuneCache*>(&plan->tune);
+    call.dq = static_cast<float*>(y->data);
+    call.dq_px = px;
+    call.dq_zpf = (float)dq_zero_point;
+    call.dq_scale = dq_scale;
     return run_conv_mfma(call, plan->pw, as_stream(stream));
 }
 

@@ -101,6 +101,9 @@ struct ConvMfmaArgs {
     float lo_folded2;
     QuantProduct qp2;
 };
+// As ConvMfmaArgs::oc_split: no second result, but the codes as floats in place of y, (code - zero point) * scale (the small tiles only): y2 is where,
+// y2_px_stride floats from one pixel to the next, inv_y_scale2 the zero point, lo_folded2 the scale.
+constexpr int kFloatResults = -1;
 
 // Direct convolution over planar activations with few channels (conv_stem.hip).
 struct ConvStemArgs {

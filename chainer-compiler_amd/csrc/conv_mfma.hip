@@ -391,7 +391,7 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     a.tiles_oc = (a.OC + tile_oc - 1) / tile_oc;
     a.tiles_px = (int)((a.M + tile_px - 1) / tile_px);
     if (a.M == 0 || a.OC == 0) return CHX_HIP_OK;
-    if (a.oc_split != 0 && (a.oc_split < 0 || a.oc_split >= a.OC || a.oc_split % tile_oc != 0 || out_int32 || a.res.r))
+    if (a.oc_split != 0 && a.oc_split != kFloatResults && (a.oc_split < 0 || a.oc_split >= a.OC || a.oc_split % tile_oc != 0 || out_int32 || a.res.r))
         CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: two outputs split at channel %d do not fit tiles of %d output channels", a.oc_split, tile_oc);
     // 32-bit offsets into x: the bias keeps the offset of a tap in the padding of the first image non-negative
     // (and leaves room for the immediates the copies subtract); a tap that is fetched lies inside x
@@ -409,6 +409,7 @@ int launch_conv_mfma(ConvMfmaArgs a, int tile_oc, int tile_px, int max_wgs_per_c
     a.row_unit = 0;
     if (a.KH * a.KW <= 32)
         for (int i = 0; i < a.KH; ++i) a.row_unit |= 1u << (i * a.KW);
+    if (a.oc_split == kFloatResults && (!conv_split_has(tile_oc, tile_px, waves) || out_int32 || a.res.r)) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: floats leave the small tiles only");
     if (max_wgs_per_cu == kConvSame) {
         if (out_int32 || rne || !conv_same_takes(a, tile_px)) CHX_FAIL(CHX_HIP_EINVAL, "conv_mfma: the kernel with the pixels in LDS does not take this convolution");
         return launch_conv_same(a, tile_oc, tile_px, waves, x_unsigned, s);

@@ -43,6 +43,8 @@ __device__ __forceinline__ uint32_t affine_residual4(uint32_t c, uint32_t r, con
     return floor_sat_u8x4(t[0], t[1], t[2], t[3]);
 }
 
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+
 struct ConvSplitArgs {
     ConvMfmaArgs conv;
     uint32_t x_flip;
@@ -324,6 +326,17 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
             float x = (float)v * (a.rq.x_scale * f.scale[e]);
             if (a.rq.bias_mode == kBiasReferenceFloat) x = x + (float)bias;
             code[e] = args.rne ? quantize_value_folded<true>(x, q_out, inv_y_scale, lo_folded) : quantize_value_folded<false>(x, q_out, inv_y_scale, lo_folded);
+        }
+        if (a.oc_split == kFloatResults) {  // a DequantizeLinear behind the convolution
+            float* dst = reinterpret_cast<float*>(a.y2) + f.m * a.y2_px_stride + f.c0;
+            v4f out;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = dequantize_value(code[e], a.inv_y_scale2, a.lo_folded2);
+            if (f.c0 + 4 <= OC) *reinterpret_cast<v4f_u*>(dst) = out;
+            else
+                for (int e = 0; e < 4; ++e)
+                    if (f.c0 + e < OC) dst[e] = out[e];
+            return;
         }
         uint32_t word = pack4(code[0], code[1], code[2], code[3]);
         if (a.res.r) {

@@ -638,6 +638,76 @@ private:
     std::vector<int> freed_;
 };
 
+std::atomic<int64_t> g_dequantized_convolutions{0};
+
+// A convolution with 1x1 filters and the DequantizeLinear that reads its result, likewise (chx_hip_qconv_plan_run_dequantize): it
+// stands where the DequantizeLinear stood.
+class DequantizedConvolutionOp : public ChxVMOp {
+public:
+    typedef QuantizedConvolutionOp::Quantization Quantization;
+    // in, out: of the convolution; dequantize: of the DequantizeLinear (a zero point of -1: none)
+    DequantizedConvolutionOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_qconv_plan> plan, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
+                             Quantization in, Quantization out, Quantization dequantize, ChxVMSteps steps, std::vector<int> freed)
+        : ChxVMOp(last), plan_(std::move(plan)), params_(params), w_(w), x_(x), y_(last.outputs[0]), in_(in), out_(out), dequantize_(dequantize), steps_(std::move(steps)),
+          freed_(std::move(freed)) {
+    }
+
+    void Run(ChxVMState* st) override {
+        if (RunAsOne(st)) {
+            for (int slot : freed_) st->FreeVar(slot);
+        } else {
+            RunSteps(steps_, st);
+        }
+    }
+
+private:
+    static int32_t Integer(const StrictScalar& z) {
+        return static_cast<int32_t>(static_cast<int64_t>(z));
+    }
+
+    // false: nothing has been written
+    bool RunAsOne(ChxVMState* st) {
+        for (int slot : {x_, in_.scale, in_.zp, out_.scale, out_.zp, dequantize_.scale})
+            if (st->GetVar(slot)->IsNull()) return false;
+        if (dequantize_.zp >= 0 && st->GetVar(dequantize_.zp)->IsNull()) return false;
+        const chainerx::Array x = st->GetArray(x_);
+        const absl::optional<StrictScalar> dq_zp = st->GetOptionalScalar(dequantize_.zp);  // (none: uint8 0)
+        const StrictScalar &x_zp = st->GetScalar(in_.zp), &y_zp = st->GetScalar(out_.zp);
+        auto is_q8 = [](chainerx::Dtype t) { return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8; };
+        if (x.ndim() != 4 || !is_q8(x.dtype()) || x.shape()[1] != w_.shape()[1] || !is_q8(y_zp.dtype()) || (dq_zp.has_value() && !is_q8(dq_zp->dtype()))) return false;
+        const chainerx::Shape shape = ConvOutputShape(x, w_, params_);
+        for (int64_t extent : shape)
+            if (extent <= 0) return false;
+        // (an input kept as code - 128 is an int8 tensor with the zero point 128 lower)
+        const bool lowered = st->store_minus_128(x_) && x.dtype() == chainerx::Dtype::kInt8 && x_zp.dtype() == chainerx::Dtype::kUInt8;
+        // laid out as the DequantizeLinear does: like the convolution's result, which is channels-last with whole 16 bytes per pixel
+        const bool contiguous = shape[2] == 1 && shape[3] == 1 && (shape[1] % 16 == 0 || shape[0] == 1);
+        chainerx::Array y = contiguous ? chainerx::Empty(shape, chainerx::Dtype::kFloat32) : chainerx::EmptyChannelsLast(shape, chainerx::Dtype::kFloat32);
+        const chx_hip_tensor xt = x.hip();
+        chx_hip_tensor yt = y.hip();
+        const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
+        const int rc = chx_hip_qconv_plan_run_dequantize(
+                plan_.get(), &xt, static_cast<float>(st->GetScalar(in_.scale)), Integer(x_zp) - (lowered ? 128 : 0), static_cast<float>(st->GetScalar(out_.scale)), Integer(y_zp),
+                static_cast<int32_t>(y_zp.dtype()), flags, static_cast<float>(st->GetScalar(dequantize_.scale)), dq_zp.has_value() ? Integer(*dq_zp) : 0, &yt,
+                chainerx::CurrentStream());
+        // (what it refuses, and operands that are in error, are for the instructions)
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        st->SetArray(y_, y);
+        ++g_dequantized_convolutions;
+        return true;
+    }
+
+    std::shared_ptr<chx_hip_qconv_plan> plan_;
+    chx_hip_conv_params params_;
+    chainerx::Array w_;
+    int x_, y_;
+    Quantization in_, out_, dequantize_;
+    ChxVMSteps steps_;
+    std::vector<int> freed_;
+};
+
 // A fused op followed by the Free instructions of its operands that the program had placed
 // between the instructions it replaces.
 class SequenceOp : public ChxVMOp {
@@ -1238,16 +1308,19 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         remaining_.swap(rest);
     }
-    // QuantizeLinear in front of a convolution over few channels, likewise.
-    for (int q = 0; q < n; ++q) {
-        const ChxVMInstructionProto& qi = program.instructions[q];
-        if (qi.op != kQuantize || role[q] != 0 || chained[q] || !quantization_once(qi)) continue;
-        const int codes = qi.outputs[0], c = codes >= 0 ? conv_reader[codes] : -1;
-        if (c <= q || !single_use(codes) || !convolution(c, false)) continue;
+    // QuantizeLinear in front of a convolution over few channels, and DequantizeLinear behind one with 1x1 filters, likewise.
+    for (int i = 0; i < n; ++i) {
+        const ChxVMInstructionProto& other = program.instructions[i];
+        const bool in_front = other.op == kQuantize;
+        if ((!in_front && other.op != kDequantize) || role[i] != 0 || chained[i] || !quantization_once(other)) continue;
+        const int codes = in_front ? other.outputs[0] : other.inputs[0].array;
+        const int c = codes < 0 ? -1 : in_front ? conv_reader[codes] : producer[codes];
+        if (c < 0 || (in_front ? c <= i : c >= i) || !single_use(codes) || !convolution(c, false)) continue;
         const ChxVMInstructionProto& ci = program.instructions[c];
         const chainerx::Array& w = *constant_array(ci.inputs[3].array);
-        // (the kernel's K axis is channels by filter rows)
-        if (w.ndim() != 4 || w.shape()[1] * w.shape()[2] > 32 || ci.inputs[11].i != 1) continue;
+        if (w.ndim() != 4 || ci.inputs[11].i != 1) continue;
+        // (the first kernel's K axis is channels by filter rows)
+        if (in_front ? w.shape()[1] * w.shape()[2] > 32 : w.shape()[2] != 1 || w.shape()[3] != 1) continue;
         const std::vector<int64_t>&strides = ci.inputs[9].ints, &pads = ci.inputs[10].ints;
         if ((!strides.empty() && strides.size() != 2) || (!pads.empty() && pads.size() != 2 && pads.size() != 4)) continue;
         auto of = [](const std::vector<int64_t>& v, size_t k, int64_t none) { return static_cast<int32_t>(v.empty() ? none : v[k]); };
@@ -1260,27 +1333,30 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         const int rc = chx_hip_qconv_plan_create(&wt, &scale, &zp, bias >= 0 ? &bt : nullptr, &params, chainerx::CurrentStream(), &plan);
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        std::set<int> slots = {codes, qi.inputs[0].array, qi.inputs[1].scalar, qi.inputs[2].scalar};
-        for (int k : {3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
+        std::shared_ptr<chx_hip_qconv_plan> kept(plan, chx_hip_qconv_plan_destroy);
+        std::set<int> slots = {codes, other.inputs[0].array, other.inputs[1].scalar, other.inputs[2].scalar};
+        for (int k : {0, 3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
         for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
-        std::set<int> moved = {q, c};
+        const int first = std::min(i, c), last = std::max(i, c);
+        std::set<int> moved = {i, c};
         ChxVMSteps steps;
         std::vector<int> freed;
-        for (int i = q; i <= c; ++i) {
-            const ChxVMInstructionProto& inst = program.instructions[i];
+        for (int m = first; m <= last; ++m) {
+            const ChxVMInstructionProto& inst = program.instructions[m];
             if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
                 freed.push_back(inst.inputs[0].array);
-                moved.insert(i);
+                moved.insert(m);
             }
-            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
+            if (moved.count(m)) steps.emplace_back(m, program_[m].get());
         }
-        chains_.emplace_back(new QuantizedConvolutionOp(ci, std::shared_ptr<chx_hip_qconv_plan>(plan, chx_hip_qconv_plan_destroy), params, w, qi.inputs[0].array,
-                                                        {qi.inputs[1].scalar, qi.inputs[2].scalar}, {ci.inputs[1].scalar, ci.inputs[2].scalar},
-                                                        {ci.inputs[6].scalar, ci.inputs[7].scalar}, std::move(steps), std::move(freed)));
-        chained[q] = chained[c] = true;
+        typedef QuantizedConvolutionOp::Quantization Quantization;
+        const Quantization in = {ci.inputs[1].scalar, ci.inputs[2].scalar}, out = {ci.inputs[6].scalar, ci.inputs[7].scalar}, own = {other.inputs[1].scalar, other.inputs[2].scalar};
+        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, params, w, other.inputs[0].array, own, in, out, std::move(steps), std::move(freed)));
+        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, params, w, ci.inputs[0].array, in, out, own, std::move(steps), std::move(freed)));
+        chained[i] = chained[c] = true;
         std::vector<std::pair<int, ChxVMOp*>> rest;
         for (const auto& r : remaining_) {
-            if (r.first == c) rest.emplace_back(c, chains_.back().get());
+            if (r.first == last) rest.emplace_back(last, chains_.back().get());
             else if (!moved.count(r.first)) rest.push_back(r);
         }
         remaining_.swap(rest);
@@ -1288,6 +1364,10 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
 }
 
 ChxVM::~ChxVM() = default;
+
+int64_t DequantizedConvolutions() {
+    return g_dequantized_convolutions.load();
+}
 
 int64_t QuantizedConvolutions() {
     return g_quantized_convolutions.load();

@@ -50,6 +50,7 @@ chainerx::Array PlainCodes(const chainerx::Array& minus_128);
 // for ops outside ops/quantize.cc that do the same
 void CountResidualFusion();
 void CountMinus128Stores(int64_t n);
+int64_t DequantizedConvolutions();  // likewise, with the DequantizeLinear behind them
 int64_t QuantizedConvolutions();  // convolutions run with the QuantizeLinear in front of them as one launch so far, process-wide
 int64_t Bottlenecks();        // tails of bottleneck blocks run as one launch so far, process-wide
 int64_t InvertedResiduals();  // inverted residual blocks run as one launch so far, process-wide

@@ -495,6 +495,7 @@ int64_t chxvm_counter(const char* name) {
     if (n == "matmul_chains") return MatMulChains();
     if (n == "bottlenecks") return Bottlenecks();
     if (n == "quantized_convolutions") return QuantizedConvolutions();
+    if (n == "dequantized_convolutions") return DequantizedConvolutions();
     if (n == "inverted_residuals") return InvertedResiduals();
     return -1;
 }
