@@ -602,7 +602,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         own.ptr[0] = own_memory.ptr();
         own.ptr[1] = static_cast<char*>(own_memory.ptr()) + own.size[0];
     }
-    if (c.dq && (stem || pixels_copied || c.out_int32 || c.res || c.y2)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: channels-last arrays of at least 16 channels only");
+    if (c.dq && (stem || pw.dense || !x_is_mfma_ready(x) || c.out_int32 || c.res || c.y2)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: channels-last arrays of at least 16 channels only");
     if (stem && c.res) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "the planar-input kernel has no fused residual sum");
     if (stem) {
         // x is used in place

@@ -579,9 +579,9 @@ public:
         int scale, zp;
     };
     // quantize: of the QuantizeLinear (a zero point of -1: none); in, out: of the convolution
-    QuantizedConvolutionOp(const ChxVMInstructionProto& conv, std::shared_ptr<chx_hip_qconv_plan> plan, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
+    QuantizedConvolutionOp(const ChxVMInstructionProto& conv, std::shared_ptr<chx_hip_qconv_plan> plan, int32_t device, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
                            Quantization quantize, Quantization in, Quantization out, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(conv), plan_(std::move(plan)), params_(params), w_(w), x_(x), y_(conv.outputs[0]), quantize_(quantize), in_(in), out_(out), steps_(std::move(steps)),
+        : ChxVMOp(conv), plan_(std::move(plan)), device_(device), params_(params), w_(w), x_(x), y_(conv.outputs[0]), quantize_(quantize), in_(in), out_(out), steps_(std::move(steps)),
           freed_(std::move(freed)) {
     }
 
@@ -600,6 +600,8 @@ private:
 
     // false: nothing has been written
     bool RunAsOne(ChxVMState* st) {
+        int32_t device = 0;
+        if (chx_hip_get_device(&device) != CHX_HIP_OK || device != device_) return false;
         for (int slot : {x_, quantize_.scale, in_.scale, in_.zp, out_.scale, out_.zp})
             if (st->GetVar(slot)->IsNull()) return false;
         if (quantize_.zp >= 0 && st->GetVar(quantize_.zp)->IsNull()) return false;
@@ -630,6 +632,7 @@ private:
     }
 
     std::shared_ptr<chx_hip_qconv_plan> plan_;
+    int32_t device_;  // that it was made on
     chx_hip_conv_params params_;
     chainerx::Array w_;
     int x_, y_;
@@ -646,9 +649,9 @@ class DequantizedConvolutionOp : public ChxVMOp {
 public:
     typedef QuantizedConvolutionOp::Quantization Quantization;
     // in, out: of the convolution; dequantize: of the DequantizeLinear (a zero point of -1: none)
-    DequantizedConvolutionOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_qconv_plan> plan, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
+    DequantizedConvolutionOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_qconv_plan> plan, int32_t device, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
                              Quantization in, Quantization out, Quantization dequantize, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(last), plan_(std::move(plan)), params_(params), w_(w), x_(x), y_(last.outputs[0]), in_(in), out_(out), dequantize_(dequantize), steps_(std::move(steps)),
+        : ChxVMOp(last), plan_(std::move(plan)), device_(device), params_(params), w_(w), x_(x), y_(last.outputs[0]), in_(in), out_(out), dequantize_(dequantize), steps_(std::move(steps)),
           freed_(std::move(freed)) {
     }
 
@@ -667,6 +670,8 @@ private:
 
     // false: nothing has been written
     bool RunAsOne(ChxVMState* st) {
+        int32_t device = 0;
+        if (chx_hip_get_device(&device) != CHX_HIP_OK || device != device_) return false;
         for (int slot : {x_, in_.scale, in_.zp, out_.scale, out_.zp, dequantize_.scale})
             if (st->GetVar(slot)->IsNull()) return false;
         if (dequantize_.zp >= 0 && st->GetVar(dequantize_.zp)->IsNull()) return false;
@@ -700,6 +705,7 @@ private:
     }
 
     std::shared_ptr<chx_hip_qconv_plan> plan_;
+    int32_t device_;  // that it was made on
     chx_hip_conv_params params_;
     chainerx::Array w_;
     int x_, y_;
@@ -1334,6 +1340,8 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
         std::shared_ptr<chx_hip_qconv_plan> kept(plan, chx_hip_qconv_plan_destroy);
+        int32_t device = 0;
+        CHXVM_HIP_CALL(chx_hip_get_device(&device));
         std::set<int> slots = {codes, other.inputs[0].array, other.inputs[1].scalar, other.inputs[2].scalar};
         for (int k : {0, 3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
         for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
@@ -1351,8 +1359,8 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         typedef QuantizedConvolutionOp::Quantization Quantization;
         const Quantization in = {ci.inputs[1].scalar, ci.inputs[2].scalar}, out = {ci.inputs[6].scalar, ci.inputs[7].scalar}, own = {other.inputs[1].scalar, other.inputs[2].scalar};
-        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, params, w, other.inputs[0].array, own, in, out, std::move(steps), std::move(freed)));
-        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, params, w, ci.inputs[0].array, in, out, own, std::move(steps), std::move(freed)));
+        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, device, params, w, other.inputs[0].array, own, in, out, std::move(steps), std::move(freed)));
+        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, device, params, w, ci.inputs[0].array, in, out, own, std::move(steps), std::move(freed)));
         chained[i] = chained[c] = true;
         std::vector<std::pair<int, ChxVMOp*>> rest;
         for (const auto& r : remaining_) {

@@ -44,7 +44,7 @@ def test_floats(g, oracle, case):  # noqa: F811
         plan.close()
 
 
-@pytest.mark.parametrize("N,C,H,OC,kernel,fused", [(3, 64, 1, 100, 1, True), (2, 48, 5, 32, 1, True), (1, 32, 1, 17, 1, True), (2, 64, 6, 32, 3, False), (2, 3, 4, 32, 1, True), (60, 64, 20, 64, 1, False)])
+@pytest.mark.parametrize("N,C,H,OC,kernel,fused", [(3, 64, 1, 100, 1, True), (2, 48, 5, 32, 1, True), (1, 32, 1, 17, 1, True), (2, 64, 6, 32, 3, False), (2, 3, 4, 32, 1, False), (60, 64, 20, 64, 1, False)])
 def test_programs(g, oracle, N, C, H, OC, kernel, fused):  # noqa: F811
     """One launch where the kernel takes them, the two instructions otherwise, with the same arrays; eagerly, recorded, and with the codes as an
     output, which keeps the two apart."""
