@@ -582,6 +582,9 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
                       (int64_t)cs.C * (x.strides[1] < 0 ? -x.strides[1] : x.strides[1]) < (int64_t(1) << 30) &&
                       x.strides[2] > 0 && (int64_t)cs.H * x.strides[2] < (int64_t(1) << 30) && c.opt.stem_kernel;
     if (c.x_float) {
+        // (the kernel's offsets inside an image are 32 bits, those of floats four times the codes')
+        const int64_t channels = (int64_t)cs.C * c.x_float->strides[1], rows = (int64_t)cs.H * c.x_float->strides[2], most = int64_t(1) << 30;
+        if (channels <= -most || channels >= most || rows >= most) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: an image of 1 GB");
         if (!stem || c.rne || !stem_patch_is_small(cs.C, cs.KH, cs.KW, sh, sw, pw_))
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: few channels in planar rows and small filters only");
     }

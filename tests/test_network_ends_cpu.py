@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["one_launch_each", "frees_between", "refused_forms", "larger_results", "another_device", "instruction_by_instruction"])
+@pytest.mark.parametrize("case", ["one_launch_each", "frees_between", "refused_forms", "larger_results", "far_apart", "another_device", "instruction_by_instruction"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -87,6 +87,22 @@ def larger_results(host):
     for batch, one in ((8, True), (9, False)):  # (2^19 results and more)
         at = dict(channels=(3, 32, 64), image=32, batch=batch)
         assert ends(host, program(host, **at), **at) == (True, one), batch
+
+
+def far_apart(host):
+    """Rows and channels of floats whose distances do not fit the kernel's 32 bits, one short of it and at it."""
+    w, ws, zp = host.tensor("int8", (32, 3, 3, 3)), host.tensor("float32", (32,)), host.tensor("int8", (32,))
+    params, plan = host.capi.conv_params((1, 1), (1, 1), (1, 1), 1), ctypes.c_void_p()
+    host.check(host.lib.chx_hip_qconv_plan_create(ctypes.byref(w), ctypes.byref(ws), ctypes.byref(zp), None, ctypes.byref(params), None, ctypes.byref(plan)))
+    y = host.channels_last("uint8", (1, 32, 8, 8))
+    for row, channel, taken in ((32, 256, True), ((1 << 27) - 4, 256, True), (1 << 27, 256, False), (32, (1 << 30) // 3 // 4 * 4, True), (32, (1 << 30) // 3 // 4 * 4 + 4, False),
+                                (32, -((1 << 30) // 3 // 4 * 4 + 4), False), (1 << 28, 1 << 28, False)):
+        x = host.tensor("float32", (1, 3, 8, 8))
+        x.strides[1], x.strides[2] = channel, row
+        host.clear()
+        rc = host.lib.chx_hip_qconv_plan_run_quantize(plan, ctypes.byref(x), ctypes.c_float(0.1), 7, ctypes.c_float(0.1), 7, ctypes.c_float(0.2), 0, 0, ctypes.byref(y), None)
+        assert (rc == 0, len(host.launches())) == ((True, 1) if taken else (False, 0)), (row, channel, rc)
+        assert taken or rc == host.capi.EUNSUPPORTED
 
 
 def another_device(host):
