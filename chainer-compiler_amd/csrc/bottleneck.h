@@ -21,7 +21,7 @@ struct BottleneckArgs {
     QuantProduct q1, q2, q3;
     ResidualAdd res;
     // the launch (filled by plan_bottleneck)
-    int32_t px_tiles, px_waves, lds;  // tiles of 32 pixels of a work-group, wavefronts that share them, bytes of LDS
+    int32_t px_tiles, px_waves, groups, lds;  // tiles of 32 pixels of a work-group, wavefronts that share them, groups of wavefronts, bytes of LDS
     int32_t patch_rows, at_mid, at_wide, at_table, tiles, xcd_chunk, quads_log2;  // log2(wide / 256)
     uint32_t w_mul, w_shift, h_mul, h_shift;
 };

@@ -5,8 +5,8 @@
 // by the next sum, the 3x3 convolution's result is written and read, and on few images each launch is 4 to 5 us of start and
 // end.  From the 3x3 convolution on nothing but a pixel's own values is needed, so a work-group takes 32 or 64 pixels in a row
 // through all of it, and no pixel is computed twice.  us inside a recording, three launches and one, over 1, 8 and 64 images:
-// 64 -> 256 -> 64 channels at 56x56 11.3 and 7.4, 19.8 and 10.5, 64.7 and 55.2; 128 -> 512 -> 128 at 28x28 12.4 and 8.4, 18.4
-// and 9.5, 43.6 and 37.4; 256 -> 1024 -> 256 at 14x14 11.1 and 17.7 (not taken), 17.1 and 17.1, 35.6 and 25.3.
+// 64 -> 256 -> 64 channels at 56x56 12.6 and 6.5, 17.7 and 10.2, 62.5 and 55.3; 128 -> 512 -> 128 at 28x28 12.1 and 7.5, 16.1
+// and 8.6, 41.8 and 37.1; 256 -> 1024 -> 256 at 14x14 11.1 and 17.7 (not taken), 17.1 and 17.1, 35.6 and 25.3.
 //
 // The pixels that the taps fall on are one run of the dense image, which goes into LDS once (pixels an odd number of 16 bytes apart;
 // taps outside the image read a pixel of zero points).  Weights are not shared between wavefronts: each has 32 channels of its own, for all of
@@ -79,15 +79,16 @@ __device__ __forceinline__ v16i seeds16(const int32_t* add) {
 constexpr int kSigned = (int)0x80808080u;
 
 // kMid: channels of the 3x3 convolution; kPT: tiles of 32 pixels; kWP: wavefronts that share them (kMid / 32 share the channels);
+// kGroups: groups of kMid / 32 * kWP wavefronts, of which the first has the 3x3 convolution and each a share of the channels of the 1x1;
 // kAffine: the sum has its short form, without a lower bound (ResidualAdd::affine is 1).
-template <int kMid, int kPT, int kWP, bool kAffine>
-__global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(BottleneckArgs) {
-    constexpr int kWO = kMid / 32, kWaves = kWO * kWP, kThreads = 64 * kWaves, kXT = kPT / kWP, kPx = 32 * kPT;
+template <int kMid, int kPT, int kWP, int kGroups, bool kAffine>
+__global__ __launch_bounds__(kMid * 2 * kWP * kGroups, 2) void bottleneck_kernel(BottleneckArgs) {
+    constexpr int kWO = kMid / 32, kFirst = kWO * kWP, kWaves = kFirst * kGroups, kThreads = 64 * kWaves, kXT = kPT / kWP, kPx = 32 * kPT;
     constexpr int kSteps = kMid / 32, kTaps = kMid == 256 ? 1 : 3, kRing = kSteps * kTaps, kPitch = kMid + 16;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const BottleneckArgs& a = kernel_arguments<BottleneckArgs>();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = lane & 31, half = lane >> 5, wo = wave % kWO, wp = wave / kWO;
+    const int col = lane & 31, half = lane >> 5, wo = wave % kWO, wp = wave / kWO % kWP, group = wave / kFirst;
     const int tile = (int)(blockIdx.x & 7) * a.xcd_chunk + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= a.xcd_chunk || tile >= a.tiles) return;
     const int m0 = tile * kPx, wide = a.wide, last_px = a.pixels - 1;
@@ -134,8 +135,10 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
                 if (b0 + b < batches) *reinterpret_cast<v4i*>(to + (b0 + b) * kRows * kPitch) = v[b] ^ (int)a.x_flip;
         };
         load(0);
+        if (kGroups == 1 || group == 0) {
 #pragma unroll
-        for (int i = 0; i < kRing; ++i) ring[i] = fragment(w1, i);
+            for (int i = 0; i < kRing; ++i) ring[i] = fragment(w1, i);
+        }
         // (64 rows of the tables are one convolution's)
         for (int i0 = wave * 64; i0 < rows; i0 += kThreads) {
             const bool one = i0 < kMid, two = i0 < kMid + wide;
@@ -178,13 +181,12 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
     // The loops are in the order that they are written in (sched_barrier): left alone, the compiler moves a fragment's load in front of
     // its use.
     v16i acc[kPT];
-    {
+    v4i expand[kSteps];
+    const int first_wide = min(wave, (wide >> 5) - 1) * kSteps;
+    if (kGroups == 1 || group == 0) {
         const v16i seed = seeds16(s_add + wo * 32 + 16 * half);
 #pragma unroll
         for (int j = 0; j < kXT; ++j) acc[j] = seed;
-    }
-    v4i expand[kSteps];
-    {
         constexpr int kAhead = kMid == 256 ? 3 : 2, kRows = kAhead + 1;  // steps that the pixels are read ahead
         static_assert(kRing % kRows == 0 && kAhead <= kSteps, "");
         int tap = 0, tap_off = 0, kw = 0, off[kXT], off_next[kXT];
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
 #pragma unroll
                     for (int j = 0; j < kXT; ++j) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[i], px[i % kRows][j], acc[j], 0, 0, 0);
                     if constexpr (decltype(last)::value) {
-                        if (t == 0) expand[k] = fragment(a.w2, wave * kSteps + k);
+                        if (t == 0) expand[k] = fragment(a.w2, first_wide + k);
                     } else {
                         ring[i] = fragment(next, i);
                     }
@@ -231,19 +233,22 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
 #pragma unroll 1
         for (int done = 0; done < 9 - kTaps; done += kTaps) taps_of(std::false_type(), done);
         taps_of(std::true_type(), 9 - kTaps);
-    }
-    const QuantProduct q1 = in_vector_registers(a.q1);
+        const QuantProduct q1 = in_vector_registers(a.q1);
 #pragma unroll
-    for (int j = 0; j < kXT; ++j) {
-        const v4i codes = codes16(acc[j], s_scale + wo * 32 + 16 * half, q1);
-        *reinterpret_cast<v4i*>(mids + ((wp * kXT + j) * 32 + col) * kPitch + wo * 32 + 16 * half) = codes ^ kSigned;
+        for (int j = 0; j < kXT; ++j) {
+            const v4i codes = codes16(acc[j], s_scale + wo * 32 + 16 * half, q1);
+            *reinterpret_cast<v4i*>(mids + ((wp * kXT + j) * 32 + col) * kPitch + wo * 32 + 16 * half) = codes ^ kSigned;
+        }
+    } else {  // (the second group only brings what the first needs, until the expansion)
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) expand[k] = fragment(a.w2, first_wide + k);
     }
     wait_vmcnt<0>();  // (the residual is there, too)
     lds_barrier();
 
     // ---- 1x1 expansion and the sum: every wavefront has all pixels, and channels of its own ----
     const int wide_tiles = wide >> 5, reduce_steps = wide >> 5;
-    const char* const w3 = a.w3 + (uint32_t)(min(wo, max((a.next >> 5) - 1, 0)) * reduce_steps) * 1024u;
+    const char* const w3 = a.w3 + (uint32_t)(min(wo + kWO * group, max((a.next >> 5) - 1, 0)) * reduce_steps) * 1024u;
     v4i reduce[8];
     {
         const QuantProduct q2 = in_vector_registers(a.q2);
@@ -308,7 +313,7 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
         const uint32_t z_lane = __umul24((uint32_t)col, (uint32_t)z_px) + 16u * (uint32_t)half;
         const char* const from = wides + (wp * kXT * 32 + col) * wide;
 #pragma unroll 1
-        for (int t = wo; t < a.next >> 5; t += kWO) {
+        for (int t = wo + kWO * group; t < a.next >> 5; t += kWO * kGroups) {
             {
                 const v16i seed = seeds16(s_add + kMid + wide + t * 32 + 16 * half);
 #pragma unroll
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(kMid * 2 * kWP, 2) void bottleneck_kernel(Bottlenec
 #pragma unroll 1
             for (int s = 0; s < reduce_steps; s += 8) {
                 // (behind the tile's last steps: the next tile's first, or some again)
-                const int ahead = s + 8 < reduce_steps ? s + 8 : t + kWO < a.next >> 5 ? kWO * reduce_steps : 0;
+                const int ahead = s + 8 < reduce_steps ? s + 8 : t + kWO * kGroups < a.next >> 5 ? kWO * kGroups * reduce_steps : 0;
                 const char *const row = from + s * 32, *const row_next = from + (s + 8 < reduce_steps ? s + 8 : 0) * 32;
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
@@ -376,11 +381,12 @@ __global__ __launch_bounds__(64) void pack_bottleneck_table_kernel(const int8_t*
 
 constexpr int kLdsOfUnit = 160 * 1024;
 
-int lay_out(BottleneckArgs& a, int px_tiles, int px_waves) {
+int lay_out(BottleneckArgs& a, int px_tiles, int px_waves, int groups) {
     const int px = 32 * px_tiles;
     a.px_tiles = px_tiles;
     a.px_waves = px_waves;
-    const int rows = 64 * (a.mid / 32 * px_waves) / (a.mid / 16);  // that a work-group brings at a time
+    a.groups = groups;
+    const int rows = 64 * (a.mid / 32 * px_waves * groups) / (a.mid / 16);  // that a work-group brings at a time
     a.patch_rows = (px + 2 * a.W + 2 + rows - 1) / rows * rows;
     a.at_mid = a.mid + a.patch_rows * (a.mid + 16);
     a.at_wide = a.at_mid + px * (a.mid + 16);
@@ -388,11 +394,11 @@ int lay_out(BottleneckArgs& a, int px_tiles, int px_waves) {
     return a.at_table + (a.mid + a.wide + a.next + 63) / 64 * 64 * 8;
 }
 
-template <int kMid, int kPT, int kWP, bool kAffine>
+template <int kMid, int kPT, int kWP, int kGroups, bool kAffine>
 int launch(const BottleneckArgs& a, hipStream_t s) {
     if (a.lds > 64 * 1024)  // (has to be asked for, on every device)
-        CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&bottleneck_kernel<kMid, kPT, kWP, kAffine>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfUnit));
-    bottleneck_kernel<kMid, kPT, kWP, kAffine><<<8 * a.xcd_chunk, kMid * 2 * kWP, a.lds, s>>>(a);
+        CHX_HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void*>(&bottleneck_kernel<kMid, kPT, kWP, kGroups, kAffine>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsOfUnit));
+    bottleneck_kernel<kMid, kPT, kWP, kGroups, kAffine><<<8 * a.xcd_chunk, kMid * 2 * kWP * kGroups, a.lds, s>>>(a);
     return launch_check("bottleneck_kernel");
 }
 
@@ -405,14 +411,20 @@ int plan_bottleneck(BottleneckArgs* launch) {
     // work-group reads all weights for its tile.  More than four times as many channels behind the expansion as in front of it, and
     // 256 channels on few pixels, are faster as single launches (up to 2.0 and 1.4 times).  With 256 a tile takes 16 to 17 us however few
     // there are, which the three launches of 256 -> 1024 -> 256 reach at 1,500 pixels (17.3 us inside a recording at 1,568,
-    // 19.0 at 2,304; run by run, where a launch costs more, a ResNet-50 on 8 images takes 305 us with them as three and 280 as one),
+    // 19.0 at 2,304; run by run, where a launch costs more, a ResNet-50 on 8 images takes 25 us less with them as one),
     // two launches without a reduction, and three with one to more than 256 channels, at 2,500.
     const int per = a.wide / a.mid, fewest = a.next == 0 || a.next > 256 ? 2500 : 1500;
     if (per > 4 || (a.mid == 256 && (a.pixels < fewest || a.pixels > 60000))) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: slower than its convolutions");
     const int pt = a.mid == 64 ? 2 : a.mid == 128 ? (a.pixels < 24000 ? 1 : 2) : a.pixels < 9000 ? 1 : 2, wp = a.mid == 64 ? 2 : 1;
-    a.lds = lay_out(a, pt, wp);
+    // A second group of wavefronts: where a compute unit has at most two tiles, one group leaves its four SIMDs waiting for weights in
+    // the 1x1 convolutions.  Inside a recording, with one group and with two: 64 channels 8.2 and 7.5 us at 245 tiles, 10.8 and 10.5
+    // at 490, 13.3 and 15.3 at 588; 128 channels 9.5 and 8.5 at 245, 13.7 and 13.6 at 490 (without a reduction 11.9 and 11.3), 17.7
+    // and 19.1 at 588.  Four groups of 128 channels are no faster than two (8.8 and 8.6 at 196 tiles), and with 256 channels, where
+    // a group has eight wavefronts, two are slower at every size (17.7 and 16.7 at 49 tiles, 34.5 and 31.7 at 392).
+    a.tiles = (a.pixels + 32 * pt - 1) / (32 * pt);
+    a.lds = lay_out(a, pt, wp, a.mid < 256 && pt == wp && a.tiles <= 512 ? 2 : 1);
+    if (a.groups == 2 && a.lds * (a.tiles > 256 ? 2 : 1) > kLdsOfUnit) a.lds = lay_out(a, pt, wp, 1);  // (its patch may be larger)
     if (a.lds > kLdsOfUnit) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: the rows do not fit");
-    a.tiles = (a.pixels + 32 * a.px_tiles - 1) / (32 * a.px_tiles);
     a.xcd_chunk = (a.tiles + 7) / 8;
     magic_divisor((uint32_t)a.W, &a.w_mul, &a.w_shift);
     magic_divisor((uint32_t)a.H, &a.h_mul, &a.h_shift);
@@ -422,13 +434,16 @@ int plan_bottleneck(BottleneckArgs* launch) {
 }
 
 int launch_bottleneck(const BottleneckArgs& a, hipStream_t s) {
-#define CHX_SPLIT(MID, PT, WP) \
-    if (a.mid == MID && a.px_tiles == PT && a.px_waves == WP) return a.res.affine == 1 ? launch<MID, PT, WP, true>(a, s) : launch<MID, PT, WP, false>(a, s);
-    CHX_SPLIT(64, 2, 2)
-    CHX_SPLIT(128, 1, 1)
-    CHX_SPLIT(128, 2, 1)
-    CHX_SPLIT(256, 1, 1)
-    CHX_SPLIT(256, 2, 1)
+#define CHX_SPLIT(MID, PT, WP, GROUPS)                                                                                   \
+    if (a.mid == MID && a.px_tiles == PT && a.px_waves == WP && a.groups == GROUPS)                                         \
+        return a.res.affine == 1 ? launch<MID, PT, WP, GROUPS, true>(a, s) : launch<MID, PT, WP, GROUPS, false>(a, s);
+    CHX_SPLIT(64, 2, 2, 1)
+    CHX_SPLIT(64, 2, 2, 2)
+    CHX_SPLIT(128, 1, 1, 1)
+    CHX_SPLIT(128, 1, 1, 2)
+    CHX_SPLIT(128, 2, 1, 1)
+    CHX_SPLIT(256, 1, 1, 1)
+    CHX_SPLIT(256, 2, 1, 1)
 #undef CHX_SPLIT
     CHX_FAIL(CHX_HIP_EINVAL, "bottleneck: no kernel for %d channels and %d tiles of pixels", a.mid, a.px_tiles);
 }

@@ -73,6 +73,13 @@ BLOCKS = [
     ((256, 1024, 256), 13, 14, 15, np.int8, -128, (0, 131, 0), 0, False, True, True, True),
     ((256, 1024, 64), 51, 14, 14, np.uint8, 33, (7, 99, 201), 13, False, True, False, False),
     ((256, 512, 0), 60, 7, 21, np.int8, 5, (0, 0, 0), 0, True, True, True, True),
+    # more tiles than two groups of wavefronts are for (512), and as many; rows whose pixels fit for one group only
+    ((64, 256, 64), 11, 55, 55, np.int8, -128, (0, 117, 0), 0, False, True, True, True),
+    ((64, 256, 0), 32, 32, 32, np.uint8, 9, (5, 77, 0), 30, False, True, True, False),
+    ((128, 512, 128), 20, 29, 29, np.uint8, 50, (0, 131, 0), 0, True, True, True, False),
+    ((128, 512, 96), 16, 32, 32, np.int8, -128, (0, 131, 9), 11, False, False, False, True),
+    ((64, 256, 64), 1, 2, 831, np.uint8, 3, (0, 128, 0), 0, False, True, True, True),
+    ((128, 512, 128), 2, 1, 447, np.int8, -128, (1, 130, 2), 5, False, True, False, False),
 ]
 
 
