@@ -967,7 +967,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
     // Free of such an operand between the two (the compiler frees a value right after its last
     // reader) moves behind the fused op.
     std::vector<std::vector<int>> deferred_frees(n);
-    std::vector<bool> deferred(n, false);
+    std::vector<int> deferred(n, -1);  // the fused op that runs the Free
     for (int q = 0; q < n; ++q) {
         if (role[q] != 2 && role[q] != 3) continue;
         std::vector<int> dropped = {fused_inputs[q].first, fused_inputs[q].second};
@@ -984,7 +984,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         for (int i = first; i < q; ++i) {
             const ChxVMInstructionProto& fi = program.instructions[i];
             if (fi.op == kFree && fi.inputs.size() == 1 && fi.inputs[0].array >= 0 && operands.count(fi.inputs[0].array)) {
-                deferred[i] = true;
+                deferred[i] = q;
                 deferred_frees[q].push_back(i);
             }
         }
@@ -998,7 +998,7 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
     for (int i = 0; i < n; ++i) {
         const ChxVMInstructionProto& inst = program.instructions[i];
         const bool frees_dead = inst.op == kFree && inst.inputs.size() == 1 && inst.inputs[0].array >= 0 && dead[inst.inputs[0].array];
-        if (role[i] == 1 || role[i] == 7 || frees_dead || deferred[i]) {
+        if (role[i] == 1 || role[i] == 7 || frees_dead || deferred[i] >= 0) {
             program_.emplace_back(new NopOp(inst));
         } else if (role[i] == 6) {
             std::vector<std::unique_ptr<ChxVMOp>> seq;
@@ -1050,6 +1050,37 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             remaining_.emplace_back(i, program_[i].get());
         }
     }
+    // A group of instructions that runs as one launch stands where its last one stood: the Free's of its operands in front of that
+    // wait for it.  Only one of two groups (or of a group and a fused op) can have a Free, so the other is not formed: it would
+    // run behind the Free of what it reads.
+    struct Group {
+        std::set<int> moved;  // the members and their Free's
+        ChxVMSteps steps;     // these, in the program's order
+        std::vector<int> freed;
+    };
+    std::vector<bool> taken(n, false);  // Free's that a group runs
+    auto gather = [&](const std::set<int>& members, int first, const std::set<int>& slots, Group* group) {
+        group->moved = members;
+        for (int i = first; i <= *members.rbegin(); ++i) {
+            const ChxVMInstructionProto& inst = program.instructions[i];
+            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
+                if (taken[i] || (deferred[i] >= 0 && !members.count(deferred[i]))) return false;
+                group->freed.push_back(inst.inputs[0].array);
+                if (deferred[i] < 0) group->moved.insert(i);  // (the others run behind one of the members)
+            }
+            if (group->moved.count(i)) group->steps.emplace_back(i, program_[i].get());
+        }
+        return true;
+    };
+    auto install = [&](const Group& group, int last, ChxVMOp* op) {
+        for (int i : group.moved) taken[i] = true;
+        std::vector<std::pair<int, ChxVMOp*>> rest;
+        for (const auto& r : remaining_) {
+            if (r.first == last) rest.emplace_back(last, op);
+            else if (!group.moved.count(r.first)) rest.push_back(r);
+        }
+        remaining_.swap(rest);
+    };
     // Chains of fused products, for the same runs: every value between two links has one reader.  All slots involved are
     // written once, so that the links may run where the last one stood.
     std::vector<int> reader(num_variables_ > 0 ? num_variables_ : 1, -1);  // of a value that one instruction reads
@@ -1120,25 +1151,12 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         int first = *members.begin();
         for (int l : links) first = std::min({first, fused_inputs[l].first, fused_inputs[l].second});
         const int last = *members.rbegin();
-        ChxVMSteps steps;
-        std::vector<int> freed;
-        std::set<int> moved = members;
-        for (int i = first; i <= last; ++i) {
-            const ChxVMInstructionProto& inst = program.instructions[i];
-            const bool frees = inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array);
-            if (frees) freed.push_back(inst.inputs[0].array);
-            if (frees && !dynamic_cast<NopOp*>(program_[i].get())) moved.insert(i);  // (the others run behind one of the members)
-            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
-        }
+        Group group;
+        if (!gather(members, first, slots, &group)) continue;
         chains_.emplace_back(new QLinearMatMulChainOp(program.instructions[last], quantize ? &program.instructions[head] : nullptr, std::move(layers), columns, a,
-                                                      dequantize ? &program.instructions[tail] : nullptr, std::move(steps), std::move(freed)));
+                                                      dequantize ? &program.instructions[tail] : nullptr, group.steps, group.freed));
         for (int m : members) chained[m] = true;
-        std::vector<std::pair<int, ChxVMOp*>> rest;
-        for (const auto& r : remaining_) {
-            if (r.first == last) rest.emplace_back(last, chains_.back().get());
-            else if (!moved.count(r.first)) rest.push_back(r);
-        }
-        remaining_.swap(rest);
+        install(group, last, chains_.back().get());
     }
     // Inverted residual blocks, for the same runs: three convolutions whose results in between have one reader, over constants.
     auto constant_array = [&](int slot) -> const chainerx::Array* {
@@ -1194,40 +1212,26 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
             for (int k : {1, 2, 6, 7}) slots.insert(inst.inputs[k].scalar);
         }
         if (tensors[1][0].shape[0] != di.inputs[11].i) continue;  // (as many groups as channels)
+        Group group;
+        if (!gather(std::set<int>(members, members + 3), e, slots, &group)) continue;
         chx_hip_inverted_residual* block = nullptr;
         const int rc = chx_hip_inverted_residual_create(stages, static_cast<int32_t>(stride), chainerx::CurrentStream(), &block);
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
         InvertedResidualOp::Sum sum = {};
         if (role[p] == 4) {
-            const ChxVMInstructionProto& group = program.instructions[partner[p]];
+            const ChxVMInstructionProto& add = program.instructions[partner[p]];
             sum.group = groups[p];
             sum.conv_operand = conv_operand[p];
-            sum.other = group.inputs[0].array_list[1 - conv_operand[p]];
-            sum.out = group.outputs[0];
+            sum.other = add.inputs[0].array_list[1 - conv_operand[p]];
+            sum.out = add.outputs[0];
             sum.state = fusion_state[p];
-        }
-        std::set<int> moved(members, members + 3);
-        ChxVMSteps steps;
-        std::vector<int> freed;
-        for (int i = e; i <= p; ++i) {
-            const ChxVMInstructionProto& inst = program.instructions[i];
-            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
-                freed.push_back(inst.inputs[0].array);
-                moved.insert(i);
-            }
-            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
         }
         chains_.emplace_back(new InvertedResidualOp(program.instructions[p], std::shared_ptr<chx_hip_inverted_residual>(block, chx_hip_inverted_residual_destroy),
                                                     program.instructions[e].inputs[0].array, h2, convs, tensors[2][0].shape[0], static_cast<int>(stride),
-                                                    stages[0].bias != nullptr, sum, std::move(steps), std::move(freed)));
+                                                    stages[0].bias != nullptr, sum, group.steps, group.freed));
         for (int m : members) chained[m] = true;
-        std::vector<std::pair<int, ChxVMOp*>> rest;
-        for (const auto& r : remaining_) {
-            if (r.first == p) rest.emplace_back(p, chains_.back().get());
-            else if (!moved.count(r.first)) rest.push_back(r);
-        }
-        remaining_.swap(rest);
+        install(group, p, chains_.back().get());
     }
     // Bottleneck blocks, likewise: a 3x3 convolution, the 1x1 convolution behind it that computes the residual sum, and the 1x1
     // convolution that reads the sum, where nothing but constants and Free instructions stands in between.
@@ -1236,8 +1240,8 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         const int h = program.instructions[d].outputs[0], p = conv_reader[h];
         if (p <= d || !single_use(h) || role[p] != 4 || !convolution(p, true) || partner[p] <= p) continue;
         const int e = partner[p];
-        const ChxVMInstructionProto& group = program.instructions[e];
-        const int out = group.outputs[0], other = group.inputs[0].array_list[1 - conv_operand[p]];
+        const ChxVMInstructionProto& add = program.instructions[e];
+        const int out = add.outputs[0], other = add.inputs[0].array_list[1 - conv_operand[p]];
         if (!once(out) || !once(other)) continue;
         auto form = [&](int i, int64_t kernel, int64_t pad) {
             const ChxVMInstructionProto& inst = program.instructions[i];
@@ -1290,29 +1294,17 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         }
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        std::set<int> moved(convs.begin(), convs.end());
-        moved.insert(e);
-        ChxVMSteps steps;
-        std::vector<int> freed;
-        for (int i = d; i <= last; ++i) {
-            const ChxVMInstructionProto& inst = program.instructions[i];
-            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
-                freed.push_back(inst.inputs[0].array);
-                moved.insert(i);
-            }
-            if (moved.count(i)) steps.emplace_back(i, program_[i].get());
-        }
+        std::shared_ptr<chx_hip_bottleneck> kept(block, chx_hip_bottleneck_destroy);
+        std::set<int> members(convs.begin(), convs.end());
+        members.insert(e);
+        Group group;
+        if (!gather(members, d, slots, &group)) continue;
         const bool reduced = convs.size() == 3;
-        chains_.emplace_back(new BottleneckOp(program.instructions[last], std::shared_ptr<chx_hip_bottleneck>(block, chx_hip_bottleneck_destroy), program.instructions[d].inputs[0].array, h,
+        chains_.emplace_back(new BottleneckOp(program.instructions[last], kept, program.instructions[d].inputs[0].array, h,
                                               reduced ? program.instructions[convs[2]].outputs[0] : -1, quantizations, tensors[1][0].shape[0], reduced ? tensors[2][0].shape[0] : 0,
-                                              stages[0].bias != nullptr, {groups[p], conv_operand[p], other, out, fusion_state[p]}, std::move(steps), std::move(freed)));
+                                              stages[0].bias != nullptr, {groups[p], conv_operand[p], other, out, fusion_state[p]}, group.steps, group.freed));
         for (int m : convs) chained[m] = true;
-        std::vector<std::pair<int, ChxVMOp*>> rest;
-        for (const auto& r : remaining_) {
-            if (r.first == last) rest.emplace_back(last, chains_.back().get());
-            else if (!moved.count(r.first)) rest.push_back(r);
-        }
-        remaining_.swap(rest);
+        install(group, last, chains_.back().get());
     }
     // QuantizeLinear in front of a convolution over few channels, and DequantizeLinear behind one with 1x1 filters, likewise.
     for (int i = 0; i < n; ++i) {
@@ -1331,6 +1323,11 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         if ((!strides.empty() && strides.size() != 2) || (!pads.empty() && pads.size() != 2 && pads.size() != 4)) continue;
         auto of = [](const std::vector<int64_t>& v, size_t k, int64_t none) { return static_cast<int32_t>(v.empty() ? none : v[k]); };
         const chx_hip_conv_params params = {of(strides, 0, 1), of(strides, 1, 1), of(pads, 0, 0), of(pads, 1, 0), of(pads, pads.size() == 4 ? 2 : 0, 0), of(pads, pads.size() == 4 ? 3 : 1, 0), 1};
+        std::set<int> slots = {codes, other.inputs[0].array, other.inputs[1].scalar, other.inputs[2].scalar};
+        for (int k : {0, 3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
+        for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
+        Group group;
+        if (!gather({i, c}, std::min(i, c), slots, &group)) continue;
         const int bias = ci.inputs[8].array;
         const chx_hip_tensor wt = w.hip(), scale = constant_array(ci.inputs[4].array)->hip(), zp = constant_array(ci.inputs[5].array)->hip();
         chx_hip_tensor bt;
@@ -1342,32 +1339,12 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         std::shared_ptr<chx_hip_qconv_plan> kept(plan, chx_hip_qconv_plan_destroy);
         int32_t device = 0;
         CHXVM_HIP_CALL(chx_hip_get_device(&device));
-        std::set<int> slots = {codes, other.inputs[0].array, other.inputs[1].scalar, other.inputs[2].scalar};
-        for (int k : {0, 3, 4, 5, 8}) slots.insert(ci.inputs[k].array);
-        for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
-        const int first = std::min(i, c), last = std::max(i, c);
-        std::set<int> moved = {i, c};
-        ChxVMSteps steps;
-        std::vector<int> freed;
-        for (int m = first; m <= last; ++m) {
-            const ChxVMInstructionProto& inst = program.instructions[m];
-            if (inst.op == kFree && inst.inputs.size() == 1 && slots.count(inst.inputs[0].array)) {
-                freed.push_back(inst.inputs[0].array);
-                moved.insert(m);
-            }
-            if (moved.count(m)) steps.emplace_back(m, program_[m].get());
-        }
         typedef QuantizedConvolutionOp::Quantization Quantization;
         const Quantization in = {ci.inputs[1].scalar, ci.inputs[2].scalar}, out = {ci.inputs[6].scalar, ci.inputs[7].scalar}, own = {other.inputs[1].scalar, other.inputs[2].scalar};
-        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, device, params, w, other.inputs[0].array, own, in, out, std::move(steps), std::move(freed)));
-        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, device, params, w, ci.inputs[0].array, in, out, own, std::move(steps), std::move(freed)));
+        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, device, params, w, other.inputs[0].array, own, in, out, group.steps, group.freed));
+        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, device, params, w, ci.inputs[0].array, in, out, own, group.steps, group.freed));
         chained[i] = chained[c] = true;
-        std::vector<std::pair<int, ChxVMOp*>> rest;
-        for (const auto& r : remaining_) {
-            if (r.first == last) rest.emplace_back(last, chains_.back().get());
-            else if (!moved.count(r.first)) rest.push_back(r);
-        }
-        remaining_.swap(rest);
+        install(group, std::max(i, c), chains_.back().get());
     }
 }
 
