@@ -414,6 +414,7 @@ int plan_bottleneck(BottleneckArgs* launch) {
     // 19.0 at 2,304; run by run, where a launch costs more, a ResNet-50 on 8 images takes 25 us less with them as one),
     // two launches without a reduction, and three with one to more than 256 channels, at 2,500.
     const int per = a.wide / a.mid, fewest = a.next == 0 || a.next > 256 ? 2500 : 1500;
+    if (a.W >= 8192) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: the rows do not fit");  // (some 950 pixels of 64 channels do; what follows counts bytes in 32 bits)
     if (per > 4 || (a.mid == 256 && (a.pixels < fewest || a.pixels > 60000))) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: slower than its convolutions");
     const int pt = a.mid == 64 ? 2 : a.mid == 128 ? (a.pixels < 24000 ? 1 : 2) : a.pixels < 9000 ? 1 : 2, wp = a.mid == 64 ? 2 : 1;
     // A second group of wavefronts: where a compute unit has at most two tiles, one group leaves its four SIMDs waiting for weights in

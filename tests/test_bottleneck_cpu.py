@@ -26,7 +26,7 @@ def sum_code():
 
 
 @pytest.mark.parametrize("case", ["whole_blocks", "without_reduction", "values_read_elsewhere", "frees_between", "refused_forms", "sizes", "nothing_launched", "errors", "another_device",
-                                  "instruction_by_instruction"])
+                                  "instruction_by_instruction", "long_rows"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -159,6 +159,29 @@ def nothing_launched(host):
     assert run(64, 512) == (2, 0)
     assert run(64) == (0, 2)  # the search and the block
     assert run(64) == (0, 1)
+
+
+def long_rows(host):
+    """Rows that do not fit LDS are refused, however long: 31 and 32 bits of bytes are reached at some 13 and 27 million pixels."""
+    lib, capi, ref = host.lib, host.capi, ctypes.byref
+    keep, operands = [], []
+    for shape in ((64, 64, 3, 3), (256, 64, 1, 1)):
+        tensors = host.tensor("int8", shape), host.tensor("float32", shape[:1]), host.tensor("int8", shape[:1])
+        keep.append(tensors)
+        operands += [ctypes.addressof(t) for t in tensors] + [None]
+    block, small = ctypes.c_void_p(), host.channels_last("uint8", (1, 256, 1, 1))
+    host.check(lib.chx_hip_bottleneck_create((ctypes.c_void_p * 8)(*operands), 2, None, ref(block)))
+
+    def run(w):  # (nothing is read or written)
+        x, r, y = (capi.make_desc(small.data + (i << 40), capi.UINT8, (1, c, 1, w), (w * c, 1, w * c, c)) for i, c in enumerate((64, 256, 256)))
+        host.clear()
+        rc = lib.chx_hip_bottleneck_run(block, ref(x), ctypes.c_float(0.1), 7, (ctypes.c_float * 2)(0.2, 0.25), (ctypes.c_int32 * 2)(0, 0), capi.UINT8, 0, ref(r), ctypes.c_float(0.15), 3,
+                                        ctypes.c_float(0.4), 120, 0, 0, ref(y), 0, None, None)
+        return rc, sum(BLOCK in line for line in host.launches())
+
+    assert run(800) == (0, 1)
+    for w in (1000, 8191, 8192, 13_000_000, 13_500_000, 14_000_000, 20_000_000, 26_843_400, 26_843_540, 40_265_000, 100_000_000, (1 << 30) - 1):
+        assert run(w) == (capi.EUNSUPPORTED, 0), w
 
 
 def errors(host):
