@@ -584,9 +584,16 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     if (c.x_float) {
         // (the kernel's offsets inside an image are 32 bits, those of floats four times the codes')
         const int64_t channels = (int64_t)cs.C * c.x_float->strides[1], rows = (int64_t)cs.H * c.x_float->strides[2], most = int64_t(1) << 30;
-        if (channels <= -most || channels >= most || rows >= most) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: an image of 1 GB");
+        if (channels <= -most || channels >= most || rows >= most || cs.W >= most / 4) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: an image of 1 GB");
         if (!stem || c.rne || !stem_patch_is_small(cs.C, cs.KH, cs.KW, sh, sw, pw_))
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: few channels in planar rows and small filters only");
+    }
+    // ... from the first row of a tile's to the last, also of those outside the image; a distance between rows that a single one does not have is not
+    // counted (launch below).  What lies further apart is left to the direct kernel, which needs no scratch memory either.
+    if (stem && cs.H > 1) {
+        const chx_hip_tensor& values = c.x_float ? *c.x_float : x;
+        const int64_t channels = (int64_t)cs.C * (values.strides[1] < 0 ? -values.strides[1] : values.strides[1]);
+        if (stem_patch_rows(cs.KH, sh) * values.strides[2] + channels >= (int64_t(1) << 32)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "the planar-input kernel: rows too far apart");
     }
     // Channels-last pixels at another pitch than 16 bytes (40 channels packed, say) are copied to one.  The copy's memory is
     // this call's and not the plan's: the direct kernel, which has always taken such arrays, lets one plan run on two streams
@@ -706,7 +713,7 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         memset(&sa, 0, sizeof(sa));
         const chx_hip_tensor& values = c.x_float ? *c.x_float : x;
         sa.x = static_cast<const char*>(values.data);
-        sa.x_n_stride = values.strides[0]; sa.x_c_stride = values.strides[1]; sa.x_h_stride = values.strides[2];
+        sa.x_n_stride = values.strides[0]; sa.x_c_stride = values.strides[1]; sa.x_h_stride = cs.H > 1 ? values.strides[2] : 0;
         sa.x_float = c.x_float != nullptr;
         sa.xq = c.xq;
         sa.N = cs.N; sa.C = cs.C; sa.H = cs.H; sa.W = cs.W; sa.OH = cs.OH; sa.OW = cs.OW; sa.KH = cs.KH; sa.KW = cs.KW;

@@ -159,6 +159,7 @@ int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp
 // the stem kernel: weights [C][KH][KW] with C*KH <= 32 and KW <= 8; patch = LDS bytes of a tile's input rows
 bool stem_shape_fits(int C, int KH, int KW);
 bool stem_patch_fits(int C, int KH, int KW, int sh, int sw, int pw);
+int stem_patch_rows(int KH, int sh);  // of a tile's input rows, those outside the image among them
 bool stem_patch_is_small(int C, int KH, int KW, int sh, int sw, int pw);  // as float32 rows need it
 int stem_k_blocks(int C, int KH, int KW);
 int pack_weights_stem(const chx_hip_tensor& w, int OCpad64, int8_t* wd, hipStream_t s);

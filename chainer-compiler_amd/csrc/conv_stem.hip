@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
 
     // the patch dwords this thread fills: the same places for every tile
     int pd_rc[kPD] = {};        // row << 16 | column
-    uint32_t pd_off[kPD] = {};  // bytes from the place of the first of all channels in memory (their stride may be negative)
+    uint32_t pd_off[kPD] = {};  // bytes from the place of the first of all channels in memory (their stride may be negative): run_conv_mfma sees to it that they fit
     const int c_turn = a.x_c_stride < 0 ? a.C - 1 : 0;
     const uint32_t c_step = (uint32_t)(a.x_c_stride < 0 ? -a.x_c_stride : a.x_c_stride);
 #pragma unroll
@@ -378,11 +378,14 @@ int stem_k_blocks(int C, int KH, int KW) {
     return (C * KH * kwp + 31) / 32;
 }
 
+int stem_patch_rows(int KH, int sh) {
+    return (kTileH - 1) * sh + KH;
+}
+
 size_t stem_patch_bytes(int C, int KH, int KW, int sh, int sw, int pw) {
     const int kwp = KW <= 4 ? 4 : 8;
-    const int PH = (kTileH - 1) * sh + KH;
     const int PP = ((-pw & 3) + (kTileW - 1) * sw + kwp + 3) & ~3;
-    return (size_t)C * PH * PP;
+    return (size_t)C * stem_patch_rows(KH, sh) * PP;
 }
 
 bool stem_shape_fits(int C, int KH, int KW) {
@@ -396,7 +399,7 @@ bool stem_patch_is_small(int C, int KH, int KW, int sh, int sw, int pw) {
 bool stem_patch_fits(int C, int KH, int KW, int sh, int sw, int pw) {
     const int kwp = KW <= 4 ? 4 : 8;
     // the small_div ranges: rows per channel and dwords per row below 64
-    return stem_patch_bytes(C, KH, KW, sh, sw, pw) <= (size_t)256 * kMaxPatchDwords * 4 && (kTileH - 1) * sh + KH < 64 &&
+    return stem_patch_bytes(C, KH, KW, sh, sw, pw) <= (size_t)256 * kMaxPatchDwords * 4 && stem_patch_rows(KH, sh) < 64 &&
            (-pw & 3) + (kTileW - 1) * sw + kwp < 252;
 }
 
@@ -447,7 +450,7 @@ int launch_conv_stem(ConvStemArgs a, bool rne, hipStream_t s) {
     magic_divisor((uint32_t)a.tiles_w, &a.tw_mul, &a.tw_shift);
     a.KB = stem_k_blocks(a.C, a.KH, a.KW);
     const bool kwp4 = a.KW <= 4;
-    const uint32_t ppw = (uint32_t)((((-a.pw & 3) + (kTileW - 1) * a.sw + (kwp4 ? 4 : 8) + 3) & ~3) >> 2), ph_rows = (uint32_t)((kTileH - 1) * a.sh + a.KH);
+    const uint32_t ppw = (uint32_t)((((-a.pw & 3) + (kTileW - 1) * a.sw + (kwp4 ? 4 : 8) + 3) & ~3) >> 2), ph_rows = (uint32_t)stem_patch_rows(a.KH, a.sh);
     a.m_ppw = ((1u << 20) + ppw - 1) / ppw;
     a.m_ph = ((1u << 20) + ph_rows - 1) / ph_rows;
     a.m_kh = ((1u << 20) + (uint32_t)a.KH - 1) / (uint32_t)a.KH;

@@ -90,6 +90,36 @@ def test_floats(g, oracle, case):  # noqa: F811
         plan.close()
 
 
+# H, kernel, stride, bytes between rows: more than 2^32 from a tile's first row to its last, most of which the image does not have; just less
+@pytest.mark.parametrize("H,kernel,stride,row", [(1, 7, 2, 1 << 28), (1, 3, 1, (1 << 30) - 4), (4, 7, 2, 215 << 20), (4, 7, 2, 195 << 20)])
+def test_rows_far_apart(g, oracle, H, kernel, stride, row):  # noqa: F811
+    case = (1, 3, H, 21, 32, kernel, kernel, stride, kernel // 2)
+    for floats in (False, True):
+        row = row // 4 if floats else row
+        if floats:
+            x = (np.random.default_rng(H).normal(size=case[:4]) * 1.2).astype(np.float32)
+            q = oracle.quantize_linear(x, np.float32(0.02), 31, np.uint8)
+        else:
+            x = q = codes(np.random.default_rng(H), case[:4], np.uint8)
+        # (the channels lie side by side in each row)
+        xd = torch.empty(row * (H - 1) + 64, dtype=torch.float32 if floats else torch.uint8, device="cuda").as_strided(case[:4], (row, 21, row, 1))
+        xd.copy_(torch.from_numpy(x))
+        w, ws, bias, y_scale, want = operands(oracle, q, case, FORMS[0], (0.02, 31))
+        plan, out = plan_of(g, w, ws, bias, case), pitched(want.shape, torch.uint8)
+        if floats:
+            rc = g.capi.lib().chx_hip_qconv_plan_run_quantize(
+                plan._plan_of(g.capi.ConvParams(stride, stride, *(kernel // 2,) * 4, 1)), g.capi.ref(xd), ctypes.c_float(0.02), 31, ctypes.c_float(0.02), 31, ctypes.c_float(y_scale), 0,
+                ctypes.c_uint32(flags_of(g, FORMS[0])), g.capi.ref(out), g.capi.stream_ptr())
+            assert rc == (g.capi.EUNSUPPORTED if row * 4 == 215 << 20 else 0)
+            if rc != 0:
+                plan.close()
+                continue
+        else:
+            plan.run(xd, 0.02, 31, y_scale, 0, flags=flags_of(g, FORMS[0]), out=out)
+        np.testing.assert_array_equal(g.host(out), want)
+        plan.close()
+
+
 @pytest.mark.parametrize("channels,image,kernel,fused", [(3, 40, 7, True), (3, 33, 3, True), (3, 3, 3, False), (32, 12, 1, False)])
 def test_programs(g, oracle, channels, image, kernel, fused):  # noqa: F811
     """QuantizeLinear and the convolution behind it in a program: one launch where the kernel takes them, the two instructions otherwise; eagerly,
