@@ -578,14 +578,14 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
         pw_ = c.p->pad_w_begin, C16eff = C16;
     // few channels read from planar rows: the direct kernel, no expanded matrix
     const bool stem = pw.dense && pw.wd && !c.out_int32 && x.strides[3] == 1 &&
-                      stem_patch_fits(cs.C, cs.KH, cs.KW, sh, sw, pw_) && ph < 64 && pw_ < 64 && cs.W >= 4 &&
+                      stem_patch_fits(cs.C, cs.KH, cs.KW, sh, sw) && ph < 64 && pw_ < 64 &&
                       (int64_t)cs.C * (x.strides[1] < 0 ? -x.strides[1] : x.strides[1]) < (int64_t(1) << 30) &&
                       x.strides[2] > 0 && (int64_t)cs.H * x.strides[2] < (int64_t(1) << 30) && c.opt.stem_kernel;
     if (c.x_float) {
         // (the kernel's offsets inside an image are 32 bits, those of floats four times the codes')
         const int64_t channels = (int64_t)cs.C * c.x_float->strides[1], rows = (int64_t)cs.H * c.x_float->strides[2], most = int64_t(1) << 30;
         if (channels <= -most || channels >= most || rows >= most || cs.W >= most / 4) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: an image of 1 GB");
-        if (!stem || c.rne || !stem_patch_is_small(cs.C, cs.KH, cs.KW, sh, sw, pw_))
+        if (!stem || c.rne || cs.W < 4 || !stem_patch_is_small(cs.C, cs.KH, cs.KW, sh, sw, pw_))
             CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QuantizeLinear and QLinearConv as one launch: few channels in planar rows and small filters only");
     }
     // ... from the first row of a tile's to the last, also of those outside the image; a distance between rows that a single one does not have is not

@@ -158,7 +158,7 @@ int launch_im2col_dense(const Im2colArgs& a, hipStream_t s);
 int pack_weights(const chx_hip_tensor& w, int C64, int BK, int OCpad, int8_t* wp, int8_t* wf, int32_t* wsum, int32_t* padsum, hipStream_t s);
 // the stem kernel: weights [C][KH][KW] with C*KH <= 32 and KW <= 8; patch = LDS bytes of a tile's input rows
 bool stem_shape_fits(int C, int KH, int KW);
-bool stem_patch_fits(int C, int KH, int KW, int sh, int sw, int pw);
+bool stem_patch_fits(int C, int KH, int KW, int sh, int sw);
 int stem_patch_rows(int KH, int sh);  // of a tile's input rows, those outside the image among them
 bool stem_patch_is_small(int C, int KH, int KW, int sh, int sw, int pw);  // as float32 rows need it
 int stem_k_blocks(int C, int KH, int KW);

@@ -44,7 +44,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kTileH = 8;    // output rows per work-group: two per wavefront
 constexpr int kTileW = 16;   // output columns
 constexpr int kMaxKB = 8;    // 32-byte K blocks
-constexpr int kMaxPatchDwords = 8;  // per thread: the input patch holds at most 256 * 8 dwords
+constexpr int kMaxPatchDwords = 8;  // per thread: the input patch holds at most 256 * 8 dwords, counted without the columns in front (head)
+constexpr int kAnyPatchDwords = 10;  // with them
 constexpr size_t kFewPatchBytes = 256 * 3 * 4;
 
 struct __attribute__((packed, aligned(1))) Unaligned4 {
@@ -85,7 +86,7 @@ __device__ __forceinline__ uint32_t magic_div(uint32_t n, uint32_t mul, uint32_t
     return (__umulhi(n, mul) + n) >> shift;
 }
 
-// n / d for n < 2048 and d < 64 with m = ceil(2^20 / d)
+// n / d for n < 2^14 and d <= 64 with m = ceil(2^20 / d)
 __device__ __forceinline__ int small_div(int n, uint32_t m) {
     return (int)(((uint32_t)n * m) >> 20);
 }
@@ -105,7 +106,7 @@ enum StemRounding { kStemReference, kStemRne, kStemTwoFma };
 
 // kKB: 32-byte K blocks held in registers, at least a.KB (the others multiply zeros: with a branch around each block its reads
 // from LDS cannot run ahead of the MFMAs in front of it: 39.8 us for 35.9 at 3 -> 64 channels, 7x7, 64 images);
-// kPD: patch dwords per thread; kPG: groups of 32 pixels per wavefront: 1 for up to 32 output channels, or 2, the other two
+// kPD: patch dwords per thread (kAnyPatchDwords: also images of fewer than 4 columns); kPG: groups of 32 pixels per wavefront: 1 for up to 32 output channels, or 2, the other two
 // wavefronts with the other 32 channels (one group and 64 channels each: 199 registers, two work-groups on a unit, 42 us for 39.8).
 template <int KWP, int kKB, int kPD, int kPG, StemRounding kRounding, bool kFloat>
 __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
@@ -154,6 +155,7 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
     int n = 0, oh0 = 0, ow0 = 0;  // of the tile fetched last
     int ih0 = 0, iw0 = 0;
     bool inside = false;
+    const bool narrow = kPD == kAnyPatchDwords && a.W < 4;
     auto fetch_patch = [&](int t) {
         n = (int)magic_div((uint32_t)t, a.tpi_mul, a.tpi_shift);
         const int r = t - n * tiles_per_image;
@@ -170,6 +172,17 @@ __global__ __launch_bounds__(256, 2) void conv_stem_kernel(ConvStemArgs a) {
             for (int j = 0; j < kPD; ++j) {
                 if (j >= npd) break;
                 pv[j] = reinterpret_cast<const Fetched*>(from + pd_off[j])->v;
+            }
+        } else if (narrow) {  // (there are no 4 bytes to read: the row's, as the last of a dword)
+            if constexpr (kPD == kAnyPatchDwords) {
+#pragma unroll
+                for (int j = 0; j < kPD; ++j) {
+                    if (j >= npd) break;
+                    const int ih = ih0 + (pd_rc[j] >> 16), iw = iw0 + (pd_rc[j] & 0xffff);
+                    const char* src = from + ((int64_t)pd_off[j] + (int64_t)(min(max(ih, 0), a.H - 1) - ih) * a.x_h_stride - iw);
+                    pv[j] = 0;
+                    for (int e = 0; e < a.W; ++e) pv[j] |= (uint32_t)(uint8_t)src[e] << (8 * (4 - a.W + e));
+                }
             }
         } else {
 #pragma unroll
@@ -396,11 +409,10 @@ bool stem_patch_is_small(int C, int KH, int KW, int sh, int sw, int pw) {
     return stem_patch_bytes(C, KH, KW, sh, sw, pw) <= kFewPatchBytes;
 }
 
-bool stem_patch_fits(int C, int KH, int KW, int sh, int sw, int pw) {
+bool stem_patch_fits(int C, int KH, int KW, int sh, int sw) {
     const int kwp = KW <= 4 ? 4 : 8;
-    // the small_div ranges: rows per channel and dwords per row below 64
-    return stem_patch_bytes(C, KH, KW, sh, sw, pw) <= (size_t)256 * kMaxPatchDwords * 4 && stem_patch_rows(KH, sh) < 64 &&
-           (-pw & 3) + (kTileW - 1) * sw + kwp < 252;
+    // the small_div ranges: rows per channel below 64, dwords per row at most 64
+    return stem_patch_bytes(C, KH, KW, sh, sw, 0) <= (size_t)256 * kMaxPatchDwords * 4 && stem_patch_rows(KH, sh) < 64 && (kTileW - 1) * sw + kwp < 252;
 }
 
 int pack_weights_stem(const chx_hip_tensor& w, int OCpad64, int8_t* wd, hipStream_t s) {
@@ -461,8 +473,12 @@ int launch_conv_stem(ConvStemArgs a, bool rne, hipStream_t s) {
     (two ? launch_stem<KWP, KB, PD, 2, ROUNDING, FLOAT>(a, patch, s) : launch_stem<KWP, KB, PD, 1, ROUNDING, FLOAT>(a, patch, s))
 #define CHX_STEM(KWP, KB, PD, FLOAT) \
     (rounding == kStemTwoFma && PD == 3 ? CHX_STEM_OF(KWP, KB, 3, kStemTwoFma, FLOAT) : CHX_STEM_OF(KWP, KB, PD, kStemReference, FLOAT))
+    CHX_REQUIRE(!a.x_float || (patch <= kFewPatchBytes && a.W >= 4), "QLinearConv: the input rows of a tile are too many, or too short, to be quantized on the way");
+    if (patch > (size_t)256 * kMaxPatchDwords * 4 || a.W < 4) {
+        if (rne) return kwp4 ? CHX_STEM_OF(4, 4, kAnyPatchDwords, kStemRne, false) : CHX_STEM_OF(8, 8, kAnyPatchDwords, kStemRne, false);
+        return kwp4 ? CHX_STEM(4, 4, kAnyPatchDwords, false) : CHX_STEM(8, 8, kAnyPatchDwords, false);
+    }
     if (patch > kFewPatchBytes) {
-        CHX_REQUIRE(!a.x_float, "QLinearConv: the input rows of a tile are too many to be quantized on the way");
         if (rne) return kwp4 ? CHX_STEM_OF(4, 4, 8, kStemRne, false) : CHX_STEM_OF(8, 8, 8, kStemRne, false);
         return kwp4 ? CHX_STEM(4, 4, 8, false) : CHX_STEM(8, 8, 8, false);
     }

@@ -12,7 +12,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["rows_far_apart"])
+@pytest.mark.parametrize("case", ["rows_far_apart", "small_images_and_large_tiles"])
 def test_case(host_so, case):
     host_hip.run_case(host_so, __file__, case)
 
@@ -49,6 +49,13 @@ def rows_far_apart(host):
                         assert kernel(host, dtype, (1, 3, H, 21), k, stride, k // 2, row=row, channel=256) == ("conv_stem_kernel" if taken else other), (dtype, k, H, row)
             # one row has no distance to another
             assert kernel(host, dtype, (1, 3, 1, 21), k, stride, k // 2, row=(1 << 30) - 4, channel=256) == "conv_stem_kernel"
+
+
+def small_images_and_large_tiles(host):
+    """Images of fewer than four columns, and tiles whose rows only fit without the columns in front of them, need no scratch memory; floats are for the others."""
+    for shape, k, stride, pad in (((2, 3, 9, 1), 3, 1, 1), ((2, 3, 9, 3), 3, 1, 1), ((1, 3, 2, 2), 7, 2, 3), ((2, 4, 56, 56), 3, 4, 0), ((2, 4, 56, 56), 3, 4, 1), ((1, 4, 56, 57), 3, 4, 3)):
+        assert kernel(host, "uint8", shape, k, stride, pad) == "conv_stem_kernel", (shape, pad)
+        assert kernel(host, "float32", shape, k, stride, pad) is None, (shape, pad)
 
 
 if __name__ == "__main__":

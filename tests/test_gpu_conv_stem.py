@@ -41,7 +41,12 @@ def flags_of(g, form):  # noqa: F811
     return (0, g.capi.BIAS_REFERENCE_FLOAT, g.capi.BIAS_ONNX_INT32)[form[2]] | (g.capi.FUSE_RELU if form[1] else 0)
 
 
-@pytest.mark.parametrize("case", CASES + [(2, 3, 9, 3, 7, 3, 3, 1, 1)])  # (rows of fewer than 4 bytes: another kernel)
+# rows of fewer than 4 bytes; tiles whose rows only fit without the columns in front of them (up to 10 dwords per thread)
+NARROW = [(2, 3, 9, 3, 7, 3, 3, 1, 1), (3, 3, 5, 1, 40, 3, 3, 1, 1), (2, 1, 18, 2, 64, 7, 7, 2, 3), (1, 2, 3, 3, 33, 4, 4, 1, 3)]
+LARGE = [(2, 4, 57, 61, 64, 3, 3, 4, 1), (1, 4, 30, 33, 20, 3, 3, 4, 3)]
+
+
+@pytest.mark.parametrize("case", CASES + NARROW + LARGE)
 def test_codes(g, oracle, case):  # noqa: F811
     for i, form in enumerate(FORMS):
         x = codes(np.random.default_rng(i), case[:4], np.int8 if i % 2 else np.uint8)
