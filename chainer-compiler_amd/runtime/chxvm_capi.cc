@@ -116,18 +116,8 @@ private:
 }  // namespace
 
 struct chxvm_program {
-    std::unique_ptr<ChxVM> vm;
-    int onnx_int32_bias = -1;  // -1: the process default at the time of a run
-
-    chxvm_program() {
-        DeviceCache::Get().AddProgram();
-    }
-    ~chxvm_program() {
-        // constants may be read by work of any stream still (a replay's)
-        (void)chx_hip_device_synchronize();
-        vm.reset();
-        DeviceCache::Get().RemoveProgram();
-    }
+    std::shared_ptr<ChxVM> vm;  // and its recordings', whose kernels address its constants
+    int onnx_int32_bias = -1;   // -1: the process default at the time of a run
 };
 
 struct chxvm_outputs {
@@ -140,6 +130,7 @@ struct chxvm_outputs {
 };
 
 struct chxvm_replay {
+    std::shared_ptr<ChxVM> vm;  // (given up last)
     std::shared_ptr<PoolAllocator> pool;
     void* stream = nullptr;
     chx_hip_graph* graph = nullptr;
@@ -163,6 +154,24 @@ struct chxvm_replay {
 };
 
 namespace {
+
+std::shared_ptr<ChxVM> LoadProgram(const ChxVMProgramProto& program) {
+    struct Loaded {
+        std::unique_ptr<ChxVM> vm;
+        Loaded() {
+            DeviceCache::Get().AddProgram();
+        }
+        ~Loaded() {
+            // constants may be read by work of any stream still (a replay's)
+            (void)chx_hip_device_synchronize();
+            vm.reset();
+            DeviceCache::Get().RemoveProgram();
+        }
+    };
+    const auto loaded = std::make_shared<Loaded>();
+    loaded->vm.reset(new ChxVM(program));
+    return std::shared_ptr<ChxVM>(loaded, loaded->vm.get());
+}
 
 InOuts BorrowInputs(const char* const* input_names, const chx_hip_tensor* inputs, int32_t num_inputs) {
     InOuts in;
@@ -218,7 +227,7 @@ int32_t chxvm_program_create(const void* bytes, size_t size, chxvm_program** out
     return Guard([&] {
         const ChxVMProgramProto program = ChxVMProgramProto::ParseFromString(std::string(static_cast<const char*>(bytes), size));
         std::unique_ptr<chxvm_program> p(new chxvm_program());
-        p->vm.reset(new ChxVM(program));
+        p->vm = LoadProgram(program);
         *out = p.release();
     });
 }
@@ -309,6 +318,7 @@ int32_t chxvm_program_capture(
         ChxVMOptions options;  // no tracing, checking or dumping: all of them read results back
         options.qlinearconv_onnx_int32_bias = program->onnx_int32_bias >= 0 ? program->onnx_int32_bias != 0 : g_onnx_int32_bias;
         std::unique_ptr<chxvm_replay> r(new chxvm_replay());
+        r->vm = program->vm;
         r->pool = std::make_shared<PoolAllocator>();
         CHXVM_HIP_CALL(chx_hip_stream_create(&r->stream));
         // Eager runs on the stream until one of them finds every block it asks for in the pool: plans are

@@ -81,7 +81,8 @@ void chxvm_outputs_destroy(chxvm_outputs* outputs);
  * expansion scratch), which eager runs of the same program share.  The plans a recording has used are therefore
  * pinned until the replay is destroyed: an eager run of the program on larger inputs, which would have to move
  * that scratch memory, fails with an error instead (run the largest inputs before capture()), and a plan that
- * the program gives up (other weight operands) is released only with the replay.  Eager runs and launches of a
+ * the program gives up (other weight operands) is released only with the replay.  The kernels address the program's constants
+ * too: what a program that is destroyed before its replays holds on the device is released with the last of them.  Eager runs and launches of a
  * replay of one program must not overlap in time: both write that scratch memory. */
 typedef struct chxvm_replay chxvm_replay;
 int32_t chxvm_program_capture(
