@@ -408,14 +408,13 @@ int plan_bottleneck(BottleneckArgs* launch) {
     BottleneckArgs& a = *launch;
     // Pixels of a work-group, and whether the block is one launch: by 400 drawn blocks measured both ways inside a recording, three
     // with weights of their own in turn.  Few pixels leave compute units idle when they are shared out in tiles of 64, and each
-    // work-group reads all weights for its tile.  More than four times as many channels behind the expansion as in front of it, and
-    // 256 channels on few pixels, are faster as single launches (up to 2.0 and 1.4 times).  With 256 a tile takes 16 to 17 us however few
+    // work-group reads all weights for its tile.  256 channels on few pixels are faster as single launches (up to 1.4 times).  With 256 a tile takes 16 to 17 us however few
     // there are, which the three launches of 256 -> 1024 -> 256 reach at 1,500 pixels (17.3 us inside a recording at 1,568,
     // 19.0 at 2,304; run by run, where a launch costs more, a ResNet-50 on 8 images takes 25 us less with them as one),
     // two launches without a reduction, and three with one to more than 256 channels, at 2,500.
-    const int per = a.wide / a.mid, fewest = a.next == 0 || a.next > 256 ? 2500 : 1500;
+    const int fewest = a.next == 0 || a.next > 256 ? 2500 : 1500;
     if (a.W >= 8192) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: the rows do not fit");  // (some 950 pixels of 64 channels do; what follows counts bytes in 32 bits)
-    if (per > 4 || (a.mid == 256 && (a.pixels < fewest || a.pixels > 60000))) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: slower than its convolutions");
+    if (a.mid == 256 && (a.pixels < fewest || a.pixels > 60000)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: slower than its convolutions");
     const int pt = a.mid == 64 ? 2 : a.mid == 128 ? (a.pixels < 24000 ? 1 : 2) : a.pixels < 9000 ? 1 : 2, wp = a.mid == 64 ? 2 : 1;
     // A second group of wavefronts: where a compute unit has at most two tiles, one group leaves its four SIMDs waiting for weights in
     // the 1x1 convolutions.  Inside a recording, with one group and with two: 64 channels 8.2 and 7.5 us at 245 tiles, 10.8 and 10.5

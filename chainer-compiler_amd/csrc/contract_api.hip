@@ -2097,7 +2097,7 @@ extern "C" int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, in
         channels = w.shape[0];
     }
     const int64_t mid = stages[0].w->shape[0], wide = stages[1].w->shape[0], next = count == 3 ? channels : 0;
-    if (stages[0].w->shape[1] != mid || !bottleneck_mid(mid) || wide < 256 || wide > 2048 || (wide & (wide - 1)) != 0 || next % 32 != 0 || next > 1024) return refuse("the number of channels");
+    if (stages[0].w->shape[1] != mid || !bottleneck_takes_channels(mid, wide, next)) return refuse("the number of channels");
     for (int i = 0; i < count; ++i) {
         std::vector<uint8_t> zp;
         CHX_PROPAGATE(read_back(*stages[i].w_zero_point, &zp, s));

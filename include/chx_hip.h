@@ -315,7 +315,7 @@ int chx_hip_inverted_residual_run(
 /* The tail of a bottleneck block: 3x3 convolution with padding 1, 1x1 convolution and the residual sum of
  * chx_hip_qconv_plan_run_add; with three stages, the 1x1 convolution of the sum as well (the next block's first), as one launch,
  * with the codes of the single calls.  stages: as for chx_hip_inverted_residual_create, strides 1; 64, 128 or 256 channels in
- * between, a multiple of 256 behind the sum, of 32 behind the third. */
+ * between, 256, 512 or 1024 behind the sum but no more than four times as many, a multiple of 32 up to 1024 behind the third. */
 typedef struct chx_hip_bottleneck chx_hip_bottleneck;
 int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, int32_t count, void* stream, chx_hip_bottleneck** out);
 void chx_hip_bottleneck_destroy(chx_hip_bottleneck* plan);

@@ -26,7 +26,7 @@ def sum_code():
 
 
 @pytest.mark.parametrize("case", ["whole_blocks", "without_reduction", "values_read_elsewhere", "frees_between", "refused_forms", "sizes", "nothing_launched", "errors", "another_device",
-                                  "instruction_by_instruction", "long_rows"])
+                                  "instruction_by_instruction", "long_rows", "channels_that_never_run"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -182,6 +182,21 @@ def long_rows(host):
     assert run(800) == (0, 1)
     for w in (1000, 8191, 8192, 13_000_000, 13_500_000, 14_000_000, 20_000_000, 26_843_400, 26_843_540, 40_265_000, 100_000_000, (1 << 30) - 1):
         assert run(w) == (capi.EUNSUPPORTED, 0), w
+
+
+def channels_that_never_run(host):
+    """Channels that the kernel takes for no number of pixels are refused when the block is created, before anything is laid out."""
+    lib, ref = host.lib, ctypes.byref
+    for mid, wide, nxt, taken in ((64, 256, 64, True), (64, 512, 64, False), (128, 512, 1024, True), (128, 1024, 0, False), (256, 1024, 256, True), (256, 2048, 256, False), (256, 512, 1056, False)):
+        keep, operands = [], []
+        for shape in ((mid, mid, 3, 3), (wide, mid, 1, 1)) + (((nxt, wide, 1, 1),) if nxt else ()):
+            tensors = host.tensor("int8", shape), host.tensor("float32", shape[:1]), host.tensor("int8", shape[:1])
+            keep.append(tensors)
+            operands += [ctypes.addressof(t) for t in tensors] + [None]
+        block = ctypes.c_void_p()
+        host.clear()
+        rc = lib.chx_hip_bottleneck_create((ctypes.c_void_p * len(operands))(*operands), len(keep), None, ref(block))
+        assert (rc == 0) == taken and (taken or (rc == host.capi.EUNSUPPORTED and not host.log())), (mid, wide, nxt, host.log())
 
 
 def errors(host):
