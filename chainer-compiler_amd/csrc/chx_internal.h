@@ -148,6 +148,9 @@ int prepare_noalloc_scratch();
 bool small_copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s, int* rc);
 // whether work submitted to s is being recorded into a graph instead of executed
 bool stream_is_capturing(hipStream_t s);
+// Memory for operands in a second order, without which the caller goes another way: CHX_HIP_EUNSUPPORTED where there is none, and no error is left
+// for the next launch to report.
+int spare_memory(void** p, size_t bytes, const char* what);
 int scratch_alloc(void** p, size_t bytes, hipStream_t s);
 void scratch_free(void* p, hipStream_t s);
 

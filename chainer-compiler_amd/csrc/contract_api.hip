@@ -1961,7 +1961,7 @@ extern "C" int chx_hip_inverted_residual_create(const chx_hip_conv_operands* sta
     p->at_t1 = p->at_w3 + (size_t)p->tiles_padded * p->tiles_oc * 1024;
     p->at_t2 = p->at_t1 + (size_t)p->tiles_padded * 32 * 16;
     p->at_t3 = p->at_t2 + (size_t)p->tiles_padded * 32 * 32;
-    CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&p->memory), p->at_t3 + (size_t)p->tiles_oc * 32 * 16));
+    CHX_PROPAGATE(spare_memory(reinterpret_cast<void**>(&p->memory), p->at_t3 + (size_t)p->tiles_oc * 32 * 16, "inverted residual"));
     auto table = [&](size_t at) { return reinterpret_cast<int32_t*>(p->memory + at); };
     CHX_PROPAGATE(pack_inverted_point(w1, *stages[0].w_scale, stages[0].bias, false, p->tiles_padded, p->steps, p->memory, table(p->at_t1), s));
     CHX_PROPAGATE(pack_inverted_depthwise(w2, *stages[1].w_scale, stages[1].bias, p->tiles_padded, table(p->at_t2), s));
@@ -2113,7 +2113,7 @@ extern "C" int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, in
     p->at[1] = (size_t)(9 * mid * mid);
     p->at[2] = p->at[1] + (size_t)(mid * wide);
     p->at_table = p->at[2] + (size_t)(wide * next);
-    CHX_HIP_CALL(hipMalloc(reinterpret_cast<void**>(&p->memory), p->at_table + (size_t)round_up(mid + wide + next, 64) * 16));  // (the kernel reads 64 rows at a time)
+    CHX_PROPAGATE(spare_memory(reinterpret_cast<void**>(&p->memory), p->at_table + (size_t)round_up(mid + wide + next, 64) * 16, "bottleneck"));  // (the kernel reads 64 rows at a time)
     int32_t* table = reinterpret_cast<int32_t*>(p->memory + p->at_table);
     for (int i = 0; i < count; ++i) {
         CHX_PROPAGATE(pack_bottleneck(*stages[i].w, *stages[i].w_scale, stages[i].bias, p->memory + p->at[i], table, s));

@@ -210,6 +210,14 @@ int launch_check(const char* kernel) {
     return CHX_HIP_OK;
 }
 
+int spare_memory(void** p, size_t bytes, const char* what) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return CHX_HIP_OK;
+    *p = nullptr;
+    (void)hipGetLastError();
+    CHX_FAIL(e == hipErrorOutOfMemory ? CHX_HIP_EUNSUPPORTED : CHX_HIP_ERUNTIME, "%s: hipMalloc of %zu bytes failed: %s", what, bytes, hipGetErrorString(e));
+}
+
 bool stream_is_capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess) {

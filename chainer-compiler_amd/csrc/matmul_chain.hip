@@ -294,7 +294,7 @@ extern "C" int chx_hip_chain_weights_create(const chx_hip_tensor* b, void* strea
     chx_hip_chain_weights w;
     CHX_HIP_CALL(hipGetDevice(&w.device));
     void* p = nullptr;
-    CHX_HIP_CALL(hipMalloc(&p, (size_t)(tiles * steps * 1024 + tiles * 64)));
+    CHX_PROPAGATE(spare_memory(&p, (size_t)(tiles * steps * 1024 + tiles * 64), "chain weights"));
     w.fragments = static_cast<char*>(p);
     w.K = (int32_t)b->shape[0];
     w.N = (int32_t)b->shape[1];

@@ -295,7 +295,8 @@ int chx_hip_conv_integer(
 /* An inverted residual block: 1x1 convolution, depthwise 3x3 with padding 1 and stride 1 or 2, 1x1 convolution, and
  * optionally the residual sum of chx_hip_qconv_plan_run_add, as one launch, with the codes of the single calls.
  * stages: the three convolutions' int8 weights (zero points 0), scales, zero points and int32 biases (all or none NULL);
- * they are laid out when the block is created, which waits for the stream, and not needed afterwards. */
+ * they are laid out when the block is created, which waits for the stream, and not needed afterwards (CHX_HIP_EUNSUPPORTED where there is
+ * no memory for that). */
 typedef struct chx_hip_conv_operands {
     const chx_hip_tensor *w, *w_scale, *w_zero_point, *bias;
 } chx_hip_conv_operands;
@@ -346,7 +347,7 @@ int chx_hip_qlinear_matmul(
         chx_hip_tensor* y, void* stream);
 
 /* Weights [K, N] of a layer of a chain, laid out for chx_hip_qlinear_chain: uint8 or int8, any strides, at most
- * 1024 x 512 (CHX_HIP_EUNSUPPORTED beyond).  Waits for the stream; `b` is not needed afterwards. */
+ * 1024 x 512 (CHX_HIP_EUNSUPPORTED beyond, and where there is no memory for them).  Waits for the stream; `b` is not needed afterwards. */
 typedef struct chx_hip_chain_weights chx_hip_chain_weights;
 int chx_hip_chain_weights_create(const chx_hip_tensor* b, void* stream, chx_hip_chain_weights** out);
 void chx_hip_chain_weights_destroy(chx_hip_chain_weights* weights);

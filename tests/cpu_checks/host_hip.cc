@@ -4,6 +4,7 @@
 //   hh_log / hh_clear         what happened since hh_clear, a line each
 //   hh_device_of(p)           the device whose memory p is, -1: none
 //   hh_prefer(text)           event pairs around launches of kernels with this in their name measure a tenth of the others
+//   hh_no_memory(n)           there is none for requests of exactly n bytes (0: for all)
 //   hh_hold(1), hh_held(), hh_release()
 //                             copies to the host stay queued, and the first caller of hipStreamSynchronize stays in it,
 //                             until the release; later callers let all queued copies happen, as a device would
@@ -55,10 +56,12 @@ std::string& g_prefer = *new std::string;
 bool g_hold = false;
 int g_held = 0;
 int g_preferred_launches = 0;
+size_t g_no_memory = 0;
 thread_local int t_device = 0;
 thread_local dim3 t_grid, t_block;
 thread_local size_t t_lds;
 thread_local hipStream_t t_stream;
+thread_local hipError_t t_error = hipSuccess;
 
 typedef std::lock_guard<std::recursive_mutex> Lock;
 
@@ -69,6 +72,7 @@ void note(const std::string& line) {
 
 hipError_t allocate(void** p, size_t n, int device) {
     Lock lock(g_mutex);
+    if (n != 0 && n == g_no_memory) return t_error = hipErrorOutOfMemory;
     char* q = static_cast<char*>(calloc(1, n ? n : 1));
     if (!q) return hipErrorOutOfMemory;
     g_blocks[q] = Block{n, device};
@@ -137,6 +141,10 @@ int hh_device_of(const void* p) {
 void hh_prefer(const char* text) {
     Lock lock(g_mutex);
     g_prefer = text;
+}
+void hh_no_memory(size_t n) {
+    Lock lock(g_mutex);
+    g_no_memory = n;
 }
 void hh_hold(int on) {
     Lock lock(g_mutex);
@@ -219,7 +227,9 @@ const char* hipGetErrorString(hipError_t) {
     return "an error of the stand-in device runtime";
 }
 hipError_t hipGetLastError() {
-    return hipSuccess;
+    const hipError_t e = t_error;
+    t_error = hipSuccess;
+    return e;
 }
 hipError_t hipGetSymbolAddress(void** p, const void*) {
     return allocate(p, 1 << 16, t_device);
