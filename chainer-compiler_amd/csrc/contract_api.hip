@@ -884,11 +884,11 @@ int make_packed(const chx_hip_tensor& w, bool persistent, hipStream_t s, PackedW
     const bool apart = fragment_bytes > 0 && others + fragment_bytes > (size_t(2) << 20) && others <= (size_t(2) << 20);
     void* p = nullptr;
     void* p_apart = nullptr;
-    if (persistent) CHX_HIP_CALL(hipMalloc(&p, others + (apart ? 0 : fragment_bytes)));
-    else CHX_PROPAGATE(scratch_alloc(&p, others, s));
-    if (apart && hipMalloc(&p_apart, fragment_bytes) != hipSuccess) {
+    if (!persistent) CHX_PROPAGATE(scratch_alloc(&p, others, s));
+    else if (spare_memory(&p, others + (apart ? 0 : fragment_bytes), "weights of a convolution") != CHX_HIP_OK) return CHX_HIP_ERUNTIME;
+    if (apart && spare_memory(&p_apart, fragment_bytes, "weights of a convolution") != CHX_HIP_OK) {
         (void)hipFree(p);
-        CHX_FAIL(CHX_HIP_ERUNTIME, "hipMalloc failed for the small tiles' weights");
+        return CHX_HIP_ERUNTIME;
     }
     // (weights, and what is made of them, are multiples of 2048 bytes)
     pw->wp = static_cast<int8_t*>(p);
@@ -1385,10 +1385,6 @@ extern "C" int chx_hip_qconv_plan_create(
 
 namespace chx {
 namespace {
-// Results that chx_hip_qconv_plan_run_dequantize takes.  Two launches and one inside a recording, us: 8 x 2048 -> 1000 7.3 and 5.3, 128 x 1280
-// -> 1000 8.5 and 5.9, 512 x 2048 -> 1000 14.8 and 8.5, 100 x 4096 -> 4096 15.1 and 12.8; beyond, the small tiles read their operands too often:
-// 4 x 2048 -> 256 at 32x32 (a million results) 12.4 and 16.0, 8 x 1024 -> 512 at 28x28 14.2 and 24.3.
-constexpr int64_t kMostFloats = 1 << 19;
 // CHX_HIP_STORE_MINUS_128: the array is int8, its quantization is that of the uint8 array it stands for.  *view is what
 // the checks and the requantization parameters are derived from.
 int result_view(const chx_hip_tensor* y, uint32_t flags, const char* op, chx_hip_tensor* view, bool* minus_128) {
@@ -1466,6 +1462,9 @@ extern "C" int chx_hip_qconv_plan_run_quantize(
     return run_conv_mfma(call, plan->pw, as_stream(stream));
 }
 
+// CHX_HIP_MOST_DEQUANTIZED: two launches and one inside a recording, us: 8 x 2048 -> 1000 7.3 and 5.3, 128 x 1280
+// -> 1000 8.5 and 5.9, 512 x 2048 -> 1000 14.8 and 8.5, 100 x 4096 -> 4096 15.1 and 12.8; beyond, the small tiles read their operands too often:
+// 4 x 2048 -> 256 at 32x32 (a million results) 12.4 and 16.0, 8 x 1024 -> 512 at 28x28 14.2 and 24.3.
 extern "C" int chx_hip_qconv_plan_run_dequantize(
         const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, float y_scale, int32_t y_zero_point, int32_t y_dtype,
         uint32_t flags, float dq_scale, int32_t dq_zero_point, chx_hip_tensor* y, void* stream) {
@@ -1487,7 +1486,7 @@ extern "C" int chx_hip_qconv_plan_run_dequantize(
     CHX_PROPAGATE(check_qconv(x, x_scale, x_zero_point, &plan->w, &plan->w_scale, &plan->w_zero_point, y_scale, y_zero_point,
                               plan->has_bias ? &plan->bias : nullptr, &plan->params, flags, &codes, &q));
     int64_t px = 0;
-    if (!plan->mfma || !whole || !y_is_pixel_major(codes, &px) || plan->w.shape[2] != 1 || plan->w.shape[3] != 1 || numel(codes) > kMostFloats || byte_ranges_overlap(*y, *x) ||
+    if (!plan->mfma || !whole || !y_is_pixel_major(codes, &px) || plan->w.shape[2] != 1 || plan->w.shape[3] != 1 || numel(codes) > CHX_HIP_MOST_DEQUANTIZED || byte_ranges_overlap(*y, *x) ||
         (plan->opt.forced_tile && !conv_split_has(plan->opt.tile_oc, plan->opt.tile_px, plan->opt.waves)))
         CHX_FAIL(CHX_HIP_EUNSUPPORTED, "QLinearConv+DequantizeLinear: 1x1 filters, few channels-last results that do not overlap x");
     ConvCall call = conv_call_from(q, x, &codes, &plan->params, (flags & CHX_HIP_ROUND_ONNX_RNE) != 0, plan->opt);

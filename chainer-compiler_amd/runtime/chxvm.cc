@@ -6,6 +6,7 @@
 #include <fstream>
 #include <iomanip>
 #include <map>
+#include <mutex>
 #include <sstream>
 
 #include <set>
@@ -568,21 +569,22 @@ private:
     std::vector<int> freed_;
 };
 
-std::atomic<int64_t> g_quantized_convolutions{0};
-
-// A QuantizeLinear and the convolution over few channels that reads its result as one launch (chx_hip_qconv_plan_run_quantize).
-// It stands where the convolution stood; what that kernel does not take runs as the program wrote it.  The operands are
-// constants of the program, laid out when it is loaded.
-class QuantizedConvolutionOp : public ChxVMOp {
+// A QLinearConv over constants and the instruction in front of it or behind it as one launch.  It has a plan of its own, made
+// by the first run that may take it: most programs then have one plan of the convolution, this or the instruction's.
+class ConvolutionEndOp : public ChxVMOp {
 public:
     struct Quantization {  // variable slots
         int scale, zp;
     };
-    // quantize: of the QuantizeLinear (a zero point of -1: none); in, out: of the convolution
-    QuantizedConvolutionOp(const ChxVMInstructionProto& conv, std::shared_ptr<chx_hip_qconv_plan> plan, int32_t device, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
-                           Quantization quantize, Quantization in, Quantization out, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(conv), plan_(std::move(plan)), device_(device), params_(params), w_(w), x_(x), y_(conv.outputs[0]), quantize_(quantize), in_(in), out_(out), steps_(std::move(steps)),
-          freed_(std::move(freed)) {
+    struct Convolution {
+        chainerx::Array w, w_scale, w_zp, bias;  // (bias: perhaps none)
+        chx_hip_conv_params params;
+        int32_t device;  // that these are on
+        int x;
+        Quantization in, out;
+    };
+    ConvolutionEndOp(const ChxVMInstructionProto& last, Convolution conv, ChxVMSteps steps, std::vector<int> freed)
+        : ChxVMOp(last), conv_(std::move(conv)), y_(last.outputs[0]), steps_(std::move(steps)), freed_(std::move(freed)) {
     }
 
     void Run(ChxVMState* st) override {
@@ -593,125 +595,143 @@ public:
         }
     }
 
-private:
+protected:
+    // false: nothing has been written
+    virtual bool RunAsOne(ChxVMState* st) = 0;
+
     static int32_t Integer(const StrictScalar& z) {
         return static_cast<int32_t>(static_cast<int64_t>(z));
     }
-
-    // false: nothing has been written
-    bool RunAsOne(ChxVMState* st) {
+    static bool IsQ8(chainerx::Dtype t) {
+        return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8;
+    }
+    // The plan's memory is on one device: on another one the instructions run.
+    bool OnDevice() const {
         int32_t device = 0;
-        if (chx_hip_get_device(&device) != CHX_HIP_OK || device != device_) return false;
-        for (int slot : {x_, quantize_.scale, in_.scale, in_.zp, out_.scale, out_.zp})
+        return chx_hip_get_device(&device) == CHX_HIP_OK && device == conv_.device;
+    }
+    // null where there is none (no memory for it, say: the instruction's own plan has yet to be refused it)
+    chx_hip_qconv_plan* Plan() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (!plan_) {
+            const chx_hip_tensor w = conv_.w.hip(), scale = conv_.w_scale.hip(), zp = conv_.w_zp.hip();
+            chx_hip_tensor bias;
+            if (!conv_.bias.IsNullHandle()) bias = conv_.bias.hip();
+            chx_hip_qconv_plan* plan = nullptr;
+            if (chx_hip_qconv_plan_create(&w, &scale, &zp, conv_.bias.IsNullHandle() ? nullptr : &bias, &conv_.params, nullptr, &plan) != CHX_HIP_OK) return nullptr;
+            plan_.reset(plan, chx_hip_qconv_plan_destroy);
+        }
+        return plan_.get();
+    }
+    // rc: of the launch.  false: the instructions run (what it refuses, and operands that are in error, are for them)
+    bool Launched(ChxVMState* st, int rc) {
+        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
+        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        return true;
+    }
+
+    Convolution conv_;
+    int y_;
+
+private:
+    std::mutex mutex_;  // of plan_
+    std::shared_ptr<chx_hip_qconv_plan> plan_;
+    ChxVMSteps steps_;
+    std::vector<int> freed_;
+};
+
+std::atomic<int64_t> g_quantized_convolutions{0};
+
+// A QuantizeLinear and the convolution over few channels that reads its result (chx_hip_qconv_plan_run_quantize).  It stands
+// where the convolution stood; what that kernel does not take runs as the program wrote it.
+class QuantizedConvolutionOp : public ConvolutionEndOp {
+public:
+    // x, quantize: of the QuantizeLinear (a zero point of -1: none)
+    QuantizedConvolutionOp(const ChxVMInstructionProto& conv, Convolution operands, int x, Quantization quantize, ChxVMSteps steps, std::vector<int> freed)
+        : ConvolutionEndOp(conv, std::move(operands), std::move(steps), std::move(freed)), x_(x), quantize_(quantize) {
+    }
+
+private:
+    bool RunAsOne(ChxVMState* st) override {
+        if (!OnDevice()) return false;
+        for (int slot : {x_, quantize_.scale, conv_.in.scale, conv_.in.zp, conv_.out.scale, conv_.out.zp})
             if (st->GetVar(slot)->IsNull()) return false;
         if (quantize_.zp >= 0 && st->GetVar(quantize_.zp)->IsNull()) return false;
         const chainerx::Array x = st->GetArray(x_);
         const absl::optional<StrictScalar> q_zp = st->GetOptionalScalar(quantize_.zp);  // (none: uint8 0)
-        const StrictScalar &x_zp = st->GetScalar(in_.zp), &y_zp = st->GetScalar(out_.zp);
-        auto is_q8 = [](chainerx::Dtype t) { return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8; };
-        if (x.ndim() != 4 || x.dtype() != chainerx::Dtype::kFloat32 || x.shape()[1] != w_.shape()[1] || (q_zp.has_value() && q_zp->dtype() != chainerx::Dtype::kUInt8) ||
-            x_zp.dtype() != chainerx::Dtype::kUInt8 || !is_q8(y_zp.dtype()))
+        const StrictScalar &x_zp = st->GetScalar(conv_.in.zp), &y_zp = st->GetScalar(conv_.out.zp);
+        if (x.ndim() != 4 || x.dtype() != chainerx::Dtype::kFloat32 || x.shape()[1] != conv_.w.shape()[1] || (q_zp.has_value() && q_zp->dtype() != chainerx::Dtype::kUInt8) ||
+            x_zp.dtype() != chainerx::Dtype::kUInt8 || !IsQ8(y_zp.dtype()))
             return false;
-        const chainerx::Shape y_shape = ConvOutputShape(x, w_, params_);
+        const chainerx::Shape y_shape = ConvOutputShape(x, conv_.w, conv_.params);
         for (int64_t extent : y_shape)
             if (extent <= 0) return false;
+        chx_hip_qconv_plan* const plan = Plan();
+        if (!plan) return false;
         chainerx::Array y = chainerx::EmptyChannelsLastPadded(y_shape, y_zp.dtype());
         const chx_hip_tensor xt = x.hip();
         chx_hip_tensor yt = y.hip();
         const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
-        const int rc = chx_hip_qconv_plan_run_quantize(
-                plan_.get(), &xt, static_cast<float>(st->GetScalar(quantize_.scale)), q_zp.has_value() ? Integer(*q_zp) : 0, static_cast<float>(st->GetScalar(in_.scale)),
-                Integer(x_zp), static_cast<float>(st->GetScalar(out_.scale)), Integer(y_zp), flags, &yt, chainerx::CurrentStream());
-        // (what it refuses, and operands that are in error, are for the instructions)
-        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
-        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        if (!Launched(st, chx_hip_qconv_plan_run_quantize(
+                                  plan, &xt, static_cast<float>(st->GetScalar(quantize_.scale)), q_zp.has_value() ? Integer(*q_zp) : 0, static_cast<float>(st->GetScalar(conv_.in.scale)),
+                                  Integer(x_zp), static_cast<float>(st->GetScalar(conv_.out.scale)), Integer(y_zp), flags, &yt, chainerx::CurrentStream())))
+            return false;
         st->SetArray(y_, y);
         ++g_quantized_convolutions;
         return true;
     }
 
-    std::shared_ptr<chx_hip_qconv_plan> plan_;
-    int32_t device_;  // that it was made on
-    chx_hip_conv_params params_;
-    chainerx::Array w_;
-    int x_, y_;
-    Quantization quantize_, in_, out_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
+    int x_;
+    Quantization quantize_;
 };
 
 std::atomic<int64_t> g_dequantized_convolutions{0};
 
 // A convolution with 1x1 filters and the DequantizeLinear that reads its result, likewise (chx_hip_qconv_plan_run_dequantize): it
 // stands where the DequantizeLinear stood.
-class DequantizedConvolutionOp : public ChxVMOp {
+class DequantizedConvolutionOp : public ConvolutionEndOp {
 public:
-    typedef QuantizedConvolutionOp::Quantization Quantization;
-    // in, out: of the convolution; dequantize: of the DequantizeLinear (a zero point of -1: none)
-    DequantizedConvolutionOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_qconv_plan> plan, int32_t device, const chx_hip_conv_params& params, const chainerx::Array& w, int x,
-                             Quantization in, Quantization out, Quantization dequantize, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(last), plan_(std::move(plan)), device_(device), params_(params), w_(w), x_(x), y_(last.outputs[0]), in_(in), out_(out), dequantize_(dequantize), steps_(std::move(steps)),
-          freed_(std::move(freed)) {
-    }
-
-    void Run(ChxVMState* st) override {
-        if (RunAsOne(st)) {
-            for (int slot : freed_) st->FreeVar(slot);
-        } else {
-            RunSteps(steps_, st);
-        }
+    // dequantize: of the DequantizeLinear (a zero point of -1: none)
+    DequantizedConvolutionOp(const ChxVMInstructionProto& last, Convolution operands, Quantization dequantize, ChxVMSteps steps, std::vector<int> freed)
+        : ConvolutionEndOp(last, std::move(operands), std::move(steps), std::move(freed)), dequantize_(dequantize) {
     }
 
 private:
-    static int32_t Integer(const StrictScalar& z) {
-        return static_cast<int32_t>(static_cast<int64_t>(z));
-    }
-
-    // false: nothing has been written
-    bool RunAsOne(ChxVMState* st) {
-        int32_t device = 0;
-        if (chx_hip_get_device(&device) != CHX_HIP_OK || device != device_) return false;
-        for (int slot : {x_, in_.scale, in_.zp, out_.scale, out_.zp, dequantize_.scale})
+    bool RunAsOne(ChxVMState* st) override {
+        if (!OnDevice()) return false;
+        for (int slot : {conv_.x, conv_.in.scale, conv_.in.zp, conv_.out.scale, conv_.out.zp, dequantize_.scale})
             if (st->GetVar(slot)->IsNull()) return false;
         if (dequantize_.zp >= 0 && st->GetVar(dequantize_.zp)->IsNull()) return false;
-        const chainerx::Array x = st->GetArray(x_);
+        const chainerx::Array x = st->GetArray(conv_.x);
         const absl::optional<StrictScalar> dq_zp = st->GetOptionalScalar(dequantize_.zp);  // (none: uint8 0)
-        const StrictScalar &x_zp = st->GetScalar(in_.zp), &y_zp = st->GetScalar(out_.zp);
-        auto is_q8 = [](chainerx::Dtype t) { return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8; };
-        if (x.ndim() != 4 || !is_q8(x.dtype()) || x.shape()[1] != w_.shape()[1] || !is_q8(y_zp.dtype()) || (dq_zp.has_value() && !is_q8(dq_zp->dtype()))) return false;
-        const chainerx::Shape shape = ConvOutputShape(x, w_, params_);
+        const StrictScalar &x_zp = st->GetScalar(conv_.in.zp), &y_zp = st->GetScalar(conv_.out.zp);
+        if (x.ndim() != 4 || !IsQ8(x.dtype()) || x.shape()[1] != conv_.w.shape()[1] || !IsQ8(y_zp.dtype()) || (dq_zp.has_value() && !IsQ8(dq_zp->dtype()))) return false;
+        const chainerx::Shape shape = ConvOutputShape(x, conv_.w, conv_.params);
         for (int64_t extent : shape)
             if (extent <= 0) return false;
+        if (shape[0] * shape[1] * shape[2] * shape[3] > CHX_HIP_MOST_DEQUANTIZED) return false;
+        chx_hip_qconv_plan* const plan = Plan();
+        if (!plan) return false;
         // (an input kept as code - 128 is an int8 tensor with the zero point 128 lower)
-        const bool lowered = st->store_minus_128(x_) && x.dtype() == chainerx::Dtype::kInt8 && x_zp.dtype() == chainerx::Dtype::kUInt8;
+        const bool lowered = st->store_minus_128(conv_.x) && x.dtype() == chainerx::Dtype::kInt8 && x_zp.dtype() == chainerx::Dtype::kUInt8;
         // laid out as the DequantizeLinear does: like the convolution's result, which is channels-last with whole 16 bytes per pixel
         const bool contiguous = shape[2] == 1 && shape[3] == 1 && (shape[1] % 16 == 0 || shape[0] == 1);
         chainerx::Array y = contiguous ? chainerx::Empty(shape, chainerx::Dtype::kFloat32) : chainerx::EmptyChannelsLast(shape, chainerx::Dtype::kFloat32);
         const chx_hip_tensor xt = x.hip();
         chx_hip_tensor yt = y.hip();
         const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
-        const int rc = chx_hip_qconv_plan_run_dequantize(
-                plan_.get(), &xt, static_cast<float>(st->GetScalar(in_.scale)), Integer(x_zp) - (lowered ? 128 : 0), static_cast<float>(st->GetScalar(out_.scale)), Integer(y_zp),
-                static_cast<int32_t>(y_zp.dtype()), flags, static_cast<float>(st->GetScalar(dequantize_.scale)), dq_zp.has_value() ? Integer(*dq_zp) : 0, &yt,
-                chainerx::CurrentStream());
-        // (what it refuses, and operands that are in error, are for the instructions)
-        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
-        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        if (!Launched(st, chx_hip_qconv_plan_run_dequantize(
+                                  plan, &xt, static_cast<float>(st->GetScalar(conv_.in.scale)), Integer(x_zp) - (lowered ? 128 : 0), static_cast<float>(st->GetScalar(conv_.out.scale)),
+                                  Integer(y_zp), static_cast<int32_t>(y_zp.dtype()), flags, static_cast<float>(st->GetScalar(dequantize_.scale)), dq_zp.has_value() ? Integer(*dq_zp) : 0, &yt,
+                                  chainerx::CurrentStream())))
+            return false;
         st->SetArray(y_, y);
         ++g_dequantized_convolutions;
         return true;
     }
 
-    std::shared_ptr<chx_hip_qconv_plan> plan_;
-    int32_t device_;  // that it was made on
-    chx_hip_conv_params params_;
-    chainerx::Array w_;
-    int x_, y_;
-    Quantization in_, out_, dequantize_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
+    Quantization dequantize_;
 };
 
 // A fused op followed by the Free instructions of its operands that the program had placed
@@ -1328,21 +1348,19 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
         Group group;
         if (!gather({i, c}, std::min(i, c), slots, &group)) continue;
-        const int bias = ci.inputs[8].array;
-        const chx_hip_tensor wt = w.hip(), scale = constant_array(ci.inputs[4].array)->hip(), zp = constant_array(ci.inputs[5].array)->hip();
-        chx_hip_tensor bt;
-        if (bias >= 0) bt = constant_array(bias)->hip();
-        chx_hip_qconv_plan* plan = nullptr;
-        const int rc = chx_hip_qconv_plan_create(&wt, &scale, &zp, bias >= 0 ? &bt : nullptr, &params, chainerx::CurrentStream(), &plan);
-        if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) continue;
-        CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        std::shared_ptr<chx_hip_qconv_plan> kept(plan, chx_hip_qconv_plan_destroy);
-        int32_t device = 0;
-        CHXVM_HIP_CALL(chx_hip_get_device(&device));
-        typedef QuantizedConvolutionOp::Quantization Quantization;
-        const Quantization in = {ci.inputs[1].scalar, ci.inputs[2].scalar}, out = {ci.inputs[6].scalar, ci.inputs[7].scalar}, own = {other.inputs[1].scalar, other.inputs[2].scalar};
-        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, kept, device, params, w, other.inputs[0].array, own, in, out, group.steps, group.freed));
-        else chains_.emplace_back(new DequantizedConvolutionOp(other, kept, device, params, w, ci.inputs[0].array, in, out, own, group.steps, group.freed));
+        ConvolutionEndOp::Convolution conv;
+        conv.w = w;
+        conv.w_scale = *constant_array(ci.inputs[4].array);
+        conv.w_zp = *constant_array(ci.inputs[5].array);
+        if (ci.inputs[8].array >= 0) conv.bias = *constant_array(ci.inputs[8].array);
+        conv.params = params;
+        CHXVM_HIP_CALL(chx_hip_get_device(&conv.device));
+        conv.x = ci.inputs[0].array;
+        conv.in = {ci.inputs[1].scalar, ci.inputs[2].scalar};
+        conv.out = {ci.inputs[6].scalar, ci.inputs[7].scalar};
+        const ConvolutionEndOp::Quantization own = {other.inputs[1].scalar, other.inputs[2].scalar};
+        if (in_front) chains_.emplace_back(new QuantizedConvolutionOp(ci, std::move(conv), other.inputs[0].array, own, group.steps, group.freed));
+        else chains_.emplace_back(new DequantizedConvolutionOp(other, std::move(conv), own, group.steps, group.freed));
         chained[i] = chained[c] = true;
         install(group, std::max(i, c), chains_.back().get());
     }

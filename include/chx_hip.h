@@ -232,8 +232,9 @@ int chx_hip_qconv_plan_run_quantize(
         const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float q_scale, int32_t q_zero_point, float x_scale, int32_t x_zero_point,
         float y_scale, int32_t y_zero_point, uint32_t flags, chx_hip_tensor* y, void* stream);
 /* A QLinearConv with 1x1 filters and the DequantizeLinear (DequantizeLinearOp::RunImpl, runtime/ops/quantize.cc:55-60) that is the only reader
- * of its result, as one launch: y float32, the codes (of type y_dtype) are never written.  For a network's last layer: few
- * results, channels-last.  CHX_HIP_EUNSUPPORTED for everything else, and when x and y overlap: the caller then runs the two ops. */
+ * of its result, as one launch: y float32, the codes (of type y_dtype) are never written.  For a network's last layer: at most
+ * CHX_HIP_MOST_DEQUANTIZED results, channels-last.  CHX_HIP_EUNSUPPORTED for everything else, and when x and y overlap: the caller then runs the two ops. */
+#define CHX_HIP_MOST_DEQUANTIZED (1 << 19)
 int chx_hip_qconv_plan_run_dequantize(
         const chx_hip_qconv_plan* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, float y_scale, int32_t y_zero_point, int32_t y_dtype,
         uint32_t flags, float dq_scale, int32_t dq_zero_point, chx_hip_tensor* y, void* stream);

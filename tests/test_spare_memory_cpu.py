@@ -14,7 +14,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["bottleneck", "inverted_residual", "chain"])
+@pytest.mark.parametrize("case", ["bottleneck", "inverted_residual", "chain", "plans_of_the_ends"])
 def test_case(host_so, sum_code, case):  # noqa: F811
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -79,6 +79,30 @@ def chain(host):
         return p.b
 
     without_memory(host, build, {"x": host.tensor("float32", (32, 64))}, "matmul_chain_kernel", "chain_weights_kernel")
+
+
+def plans_of_the_ends(host):
+    """A convolution has one plan, made when it first runs: of the launch with its quantization in front or behind, or its instruction's where that launch
+    does not take it."""
+    rt = host.chxvm.runtime()
+    assert rt.chxvm_set_option(b"qlinearconv_bias", b"onnx_int32") == 0
+    for batch, one in ((8, True), (9, False)):  # (the last layer's results: 2^19 and more)
+        p = Program(host)
+        scale, mid = p.b.scales(0.1, 7), p.b.scales(0.2, 0)
+        x = p.b.input("x", "float32", [batch, 3, 32, 32])
+        h = p.convolution(p.convolution(p.b.QuantizeLinear(x, *scale), scale, (32, 3, 3, 3), mid), mid, (64, 32, 1, 1), mid)
+        p.b.output("y", p.b.DequantizeLinear(h, *mid))
+        host.clear()
+        program = host.program(p.b)
+        assert not host.launches()
+        for _ in range(3):
+            out = ctypes.c_void_p()
+            assert rt.chxvm_program_run(program, *host.names_and({"x": host.tensor("float32", (batch, 3, 32, 32))}), 0, ctypes.byref(out)) == 0, rt.chxvm_last_error()
+            rt.chxvm_outputs_destroy(out)
+        names = " ".join(host.launches())
+        # (the first layer's weights are laid out in two orders by a launch each)
+        assert (names.count("pack_weights_stem_kernel"), names.count("pack_weights_dense_kernel"), names.count("pack_weights_kernel")) == (1, 1, 1), names
+        assert ("dequantize" in names) != one
 
 
 if __name__ == "__main__":
