@@ -2124,6 +2124,30 @@ extern "C" int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, in
     return CHX_HIP_OK;
 }
 
+namespace chx {
+namespace {
+// The launch of a block over so many pixels.
+int plan_bottleneck_of(const chx_hip_bottleneck& plan, int64_t N, int64_t H, int64_t W, BottleneckArgs* a) {
+    if (N < 1 || H < 1 || W < 1 || N > INT32_MAX || H > INT32_MAX || W > INT32_MAX || N * H >= (int64_t(1) << 30) || N * H * W >= (int64_t(1) << 30))
+        CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: the number of pixels");
+    memset(a, 0, sizeof(*a));
+    a->pixels = (int32_t)(N * H * W);
+    a->H = (int32_t)H;
+    a->W = (int32_t)W;
+    a->mid = plan.mid;
+    a->wide = plan.wide;
+    a->next = plan.next;
+    return plan_bottleneck(a);
+}
+}  // namespace
+}  // namespace chx
+
+extern "C" int chx_hip_bottleneck_takes(const chx_hip_bottleneck* plan, int64_t n, int64_t h, int64_t w) {
+    CHX_REQUIRE(plan != nullptr, "bottleneck: null plan");
+    BottleneckArgs a;
+    return plan_bottleneck_of(*plan, n, h, w, &a);
+}
+
 extern "C" int chx_hip_bottleneck_run(
         chx_hip_bottleneck* plan, const chx_hip_tensor* x, float x_scale, int32_t x_zero_point, const float* y_scales, const int32_t* y_zero_points, int32_t y_dtype,
         uint32_t flags, const chx_hip_tensor* r, float r_scale, int32_t r_zero_point, float out_scale, int32_t out_zero_point, int32_t relu, uint32_t out_flags, chx_hip_tensor* out,
@@ -2148,7 +2172,8 @@ extern "C" int chx_hip_bottleneck_run(
     if ((flags & (CHX_HIP_ROUND_ONNX_RNE | CHX_HIP_FUSE_RELU)) != 0 || (plan->has_bias && !(flags & CHX_HIP_BIAS_ONNX_INT32))) return refuse("the flags");
     if (y_dtype != CHX_HIP_UINT8) return refuse("the type of a result");
     const int64_t N = x->shape[0], H = x->shape[2], W = x->shape[3];
-    if (N < 1 || H < 1 || W < 1 || N * H * W >= (int64_t(1) << 30)) return refuse("the number of pixels");
+    BottleneckArgs a;
+    CHX_PROPAGATE(plan_bottleneck_of(*plan, N, H, W, &a));
     const int64_t most_px = int64_t(1) << 24;  // (bytes from a pixel to the next: 24-bit products)
     int64_t x_px = 0, px[2] = {0, 0}, r_px = 0;
     if (!y_is_pixel_major(*x, &x_px) || !aligned(x->data, 16) || x_px % 16 != 0 || x_px >= most_px) return refuse("x is not channels-last in whole chunks");
@@ -2164,8 +2189,6 @@ extern "C" int chx_hip_bottleneck_run(
         if (r->ndim != 4 || r->shape[i] != out->shape[i]) return refuse("the shape of r");
     if (!is_q8(r->dtype) || !in_range(r_zero_point, r->dtype) || !in_range(out_zero_point, CHX_HIP_UINT8) || !(out_scale >= 0x1p-60f && out_scale <= 0x1p60f)) return refuse("the quantization of the sum");
     if (!y_is_pixel_major(*r, &r_px) || !aligned(r->data, 16) || r_px % 16 != 0 || r_px >= most_px) return refuse("r is not channels-last in whole chunks");
-    BottleneckArgs a;
-    memset(&a, 0, sizeof(a));
     QuantProduct* const products[3] = {&a.q1, &a.q2, &a.q3};
     for (int i = 0; i < (next ? 3 : 2); ++i) {
         if (!in_range(y_zero_points[i], CHX_HIP_UINT8)) return refuse("a zero point");
@@ -2173,13 +2196,6 @@ extern "C" int chx_hip_bottleneck_run(
         *products[i] = product_form(q, q.lo, false, true);
         if (products[i]->path != 1 && products[i]->path != 3) return refuse("a requantization without a product form");
     }
-    a.pixels = (int32_t)(N * H * W);
-    a.H = (int32_t)H;
-    a.W = (int32_t)W;
-    a.mid = plan->mid;
-    a.wide = plan->wide;
-    a.next = plan->next;
-    CHX_PROPAGATE(plan_bottleneck(&a));
     hipStream_t s = as_stream(stream);
     {  // (the first call with a sum's parameters launches a search: nothing is refused behind it)
         std::lock_guard<std::mutex> lock(plan->mutex);

@@ -531,6 +531,8 @@ private:
         const chainerx::Dtype r_type = static_cast<chainerx::Dtype>(g.in_dtype[1 - k]);
         const bool lowered = minus_128(sum_.other, r, r_type);
         if ((r.dtype() != r_type && !lowered) || r.shape() != shape) return false;
+        // (asked before there is memory for the results: on few images most blocks may be faster as their instructions)
+        if (chx_hip_bottleneck_takes(block_.get(), x.shape()[0], x.shape()[2], x.shape()[3]) != CHX_HIP_OK) return false;
         const int32_t r_zp = g.in_zero_point[1 - k] - (lowered ? 128 : 0);
         const bool out_signed = st->store_minus_128(sum_.out), next_signed = next_ >= 0 && st->store_minus_128(next_);
         chainerx::Array out = chainerx::EmptyChannelsLastPadded(shape, out_signed ? chainerx::Dtype::kInt8 : chainerx::Dtype::kUInt8), next;

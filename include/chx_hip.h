@@ -321,6 +321,8 @@ int chx_hip_inverted_residual_run(
 typedef struct chx_hip_bottleneck chx_hip_bottleneck;
 int chx_hip_bottleneck_create(const chx_hip_conv_operands* stages, int32_t count, void* stream, chx_hip_bottleneck** out);
 void chx_hip_bottleneck_destroy(chx_hip_bottleneck* plan);
+/* Whether chx_hip_bottleneck_run takes n images of h x w pixels: CHX_HIP_EUNSUPPORTED where they do not fit, or the single calls are faster. */
+int chx_hip_bottleneck_takes(const chx_hip_bottleneck* plan, int64_t n, int64_t h, int64_t w);
 /* y_scales, y_zero_points: of the convolutions' results, all of type y_dtype.  out: the sum; next: the third convolution's result
  * (NULL with two stages).  out_flags, next_flags: 0 or CHX_HIP_STORE_MINUS_128.  CHX_HIP_EUNSUPPORTED, with nothing launched, as
  * for chx_hip_inverted_residual_run. */

@@ -26,7 +26,7 @@ def sum_code():
 
 
 @pytest.mark.parametrize("case", ["whole_blocks", "without_reduction", "values_read_elsewhere", "frees_between", "refused_forms", "sizes", "nothing_launched", "errors", "another_device",
-                                  "instruction_by_instruction", "long_rows", "channels_that_never_run"])
+                                  "instruction_by_instruction", "long_rows", "channels_that_never_run", "asked_first"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -197,6 +197,30 @@ def channels_that_never_run(host):
         host.clear()
         rc = lib.chx_hip_bottleneck_create((ctypes.c_void_p * len(operands))(*operands), len(keep), None, ref(block))
         assert (rc == 0) == taken and (taken or (rc == host.capi.EUNSUPPORTED and not host.log())), (mid, wide, nxt, host.log())
+
+
+def asked_first(host):
+    """chx_hip_bottleneck_takes says what chx_hip_bottleneck_run does."""
+    lib, capi, ref = host.lib, host.capi, ctypes.byref
+    for mid, wide, nxt in ((64, 256, 64), (128, 512, 0), (256, 1024, 256), (256, 512, 0)):
+        keep, operands = [], []
+        for shape in ((mid, mid, 3, 3), (wide, mid, 1, 1)) + (((nxt, wide, 1, 1),) if nxt else ()):
+            tensors = host.tensor("int8", shape), host.tensor("float32", shape[:1]), host.tensor("int8", shape[:1])
+            keep.append(tensors)
+            operands += [ctypes.addressof(t) for t in tensors] + [None]
+        block = ctypes.c_void_p()
+        host.check(lib.chx_hip_bottleneck_create((ctypes.c_void_p * len(operands))(*operands), len(keep), None, ref(block)))
+        takes = lambda *s: lib.chx_hip_bottleneck_takes(block, *[ctypes.c_int64(v) for v in s])
+        seen = set()
+        for n, h, w in ((1, 1, 1), (1, 14, 14), (8, 14, 14), (13, 14, 14), (400, 14, 14), (1, 3, 300), (1, 3, 1200), (70000, 14, 14), (1, 1, 14_000_000)):
+            x, r, y, z = (capi.make_desc((i + 1) << 44, capi.UINT8, (n, c, h, w), (h * w * c, 1, w * c, c)) for i, c in enumerate((mid, wide, wide, nxt or 1)))
+            rc = lib.chx_hip_bottleneck_run(block, ref(x), ctypes.c_float(0.1), 7, (ctypes.c_float * 3)(0.2, 0.25, 0.3), (ctypes.c_int32 * 3)(0, 0, 0), capi.UINT8, 0, ref(r),
+                                            ctypes.c_float(0.15), 3, ctypes.c_float(0.4), 120, 0, 0, ref(y), 0, ref(z) if nxt else None, None)
+            assert takes(n, h, w) == rc, (mid, wide, nxt, n, h, w)
+            seen.add(rc)
+        assert seen == {0, capi.EUNSUPPORTED}
+        for s in ((0, 1, 1), (1, -1, -1), (1 << 40, 1 << 40, 1 << 40), (1 << 62, 4, 1)):
+            assert takes(*s) == capi.EUNSUPPORTED
 
 
 def errors(host):
