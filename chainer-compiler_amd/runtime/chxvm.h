@@ -43,7 +43,7 @@ void SetPairConvolutions(bool on);
 // stored as code - 128 in int8 arrays (CHX_HIP_STORE_MINUS_128 of the device library): the reading kernel then
 // needs no sign flips in its inner loop.  Whether programs loaded from now on do so at all (default: yes).
 void SetStoreMinus128(bool on);
-int64_t Minus128Stores();  // results written in that storage so far, process-wide
+int64_t Minus128Stores();  // results kept in that storage so far, process-wide, those between the convolutions of a block included, which are never written
 // The plain uint8 array of a value held in that storage (chx_hip_codes_minus_128).
 chainerx::Array PlainCodes(const chainerx::Array& minus_128);
 

@@ -121,7 +121,8 @@ int64_t chxvm_program_counter(const chxvm_program* program, const char* name);
 int32_t chxvm_set_option(const char* name, const char* value);
 /* Process-wide event counts.  name "qlinearconv_residual_fusions": runs of a QLinearConv that
  * computed the residual-sum group behind it inside its kernel; "qlinearconv_pair_fusions": pairs of
- * QLinearConv that ran as one launch; "minus_128_stores": results written as code - 128; "matmul_chains": chains of
+ * QLinearConv that ran as one launch; "minus_128_stores": convolutions' results kept as code - 128, those included that a
+ * block computes and never writes; "matmul_chains": chains of
  * quantized products that ran as one launch; "inverted_residuals" and "bottlenecks": blocks of convolutions that did;
  * "quantized_convolutions" and "dequantized_convolutions": convolutions that ran with the QuantizeLinear in front of them, or the DequantizeLinear behind them, as one launch.  Unknown names give -1. */
 int64_t chxvm_counter(const char* name);
