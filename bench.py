@@ -275,7 +275,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
                     # found exact on all code pairs ("affine"), or the operation-by-operation arithmetic ("exact")
                     forms[f["residual"]] = forms.get(f["residual"], 0) + 1
                     continue
-                key = "%s/%s/w%s%s" % (f.get("tile"), f.get("wgs_per_cu"), f.get("waves", "4"), "+res" if f.get("res") == "1" else "")
+                key = "%s/%s/w%s%s%s" % (f.get("tile"), f.get("wgs_per_cu"), f.get("waves", "4"), "+lds" if f.get("pixels") == "lds" else "", "+res" if f.get("res") == "1" else "")
                 hist[key] = hist.get(key, 0) + 1
                 kernels[_kernel_of(f)] = kernels.get(_kernel_of(f), 0) + 1
     roofline["configs"] = hist
@@ -338,9 +338,9 @@ def _kernel_of(config):
     oc, px = (int(v) for v in config["tile"].split("x"))
     if (oc, px, config.get("waves")) == (64, 32, "4"):
         return "conv_point_kernel"
-    if config.get("wgs_per_cu") == "100":
-        return "conv_same_kernel"
-    return "conv_split_kernel" if oc <= 32 else "conv_mfma_kernel"
+    if oc <= 32:
+        return "conv_split_kernel"
+    return "conv_same_kernel" if config.get("pixels") == "lds" else "conv_mfma_kernel"
 
 
 def _literal_executor(orc):

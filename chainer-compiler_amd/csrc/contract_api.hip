@@ -786,10 +786,10 @@ int run_conv_mfma(const ConvCall& c, const PackedWeights& pw, hipStream_t s) {
     CHX_REQUIRE(a.M < (int64_t(1) << 31), "QLinearConv: too many output pixels for the MFMA kernel");
     if (c.dq) {
         a.oc_split = kFloatResults;
-        a.y2 = reinterpret_cast<char*>(c.dq);
-        a.y2_px_stride = c.dq_px;
-        a.inv_y_scale2 = c.dq_zpf;
-        a.lo_folded2 = c.dq_scale;
+        a.floats = c.dq;
+        a.floats_px_stride = c.dq_px;
+        a.floats_zp = c.dq_zpf;
+        a.floats_scale = c.dq_scale;
     }
     int toc = 64, tpx = 64, cap = 0, waves = 4;
     pick_tile(c.opt, a, c.out_int32, &toc, &tpx, &cap, &waves);
@@ -1593,9 +1593,10 @@ extern "C" int chx_hip_qconv_plan_describe(const chx_hip_qconv_plan* plan, char*
     CHX_REQUIRE(plan != nullptr && buf != nullptr && buf_size > 0, "QLinearConv plan: null argument");
     std::string text;
     for (const TunedConfig& t : plan->tune.entries) {
+        const bool lds = t.max_wgs_per_cu == kConvSame || (t.max_wgs_per_cu == kConvSplitPatch && conv_split_has(t.tile_oc, t.tile_px, t.waves));
         char line[160];
-        snprintf(line, sizeof(line), "M=%lld %dx%d res=%d tile=%dx%d wgs_per_cu=%d waves=%d\n", (long long)t.M, t.OH, t.OW, t.with_res ? 1 : 0,
-                 t.tile_oc, t.tile_px, t.max_wgs_per_cu, t.waves);
+        snprintf(line, sizeof(line), "M=%lld %dx%d res=%d tile=%dx%d wgs_per_cu=%d waves=%d%s\n", (long long)t.M, t.OH, t.OW, t.with_res ? 1 : 0,
+                 t.tile_oc, t.tile_px, lds ? 0 : t.max_wgs_per_cu, t.waves, lds ? " pixels=lds" : "");
         text += line;
     }
     if (!plan->searched.empty()) text += plan->searched.back().found.affine ? "residual=affine\n" : "residual=exact\n";

@@ -92,17 +92,25 @@ struct ConvMfmaArgs {
     // other; output channels [0, oc_split) are the first convolution's and go to y with rq.q / inv_y_scale /
     // lo_folded, channels [oc_split, OC) are the second's and go to y2 (its channel oc - oc_split) with the set below.
     // oc_split is a multiple of the tile's output channels, so a tile belongs to one of the two whole.
+    // Or (oc_split is kFloatResults, the small tiles only) the codes as floats in place of y, (code - zero point) * scale.
     int32_t oc_split;
-    char* y2;
-    int64_t y2_px_stride;
-    uint32_t y2_flip;
-    QuantParams q2;
-    float inv_y_scale2;
-    float lo_folded2;
-    QuantProduct qp2;
+    union {
+        struct {
+            char* y2;
+            int64_t y2_px_stride;
+            uint32_t y2_flip;
+            QuantParams q2;
+            float inv_y_scale2;
+            float lo_folded2;
+            QuantProduct qp2;
+        };
+        struct {
+            float* floats;
+            int64_t floats_px_stride;  // in floats
+            float floats_zp, floats_scale;
+        };
+    };
 };
-// As ConvMfmaArgs::oc_split: no second result, but the codes as floats in place of y, (code - zero point) * scale (the small tiles only): y2 is where,
-// y2_px_stride floats from one pixel to the next, inv_y_scale2 the zero point, lo_folded2 the scale.
 constexpr int kFloatResults = -1;
 
 // Direct convolution over planar activations with few channels (conv_stem.hip).

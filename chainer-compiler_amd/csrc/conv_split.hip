@@ -328,10 +328,10 @@ __global__ __launch_bounds__(64 * W, 2) void conv_split_kernel(ConvSplitArgs) {
             code[e] = args.rne ? quantize_value_folded<true>(x, q_out, inv_y_scale, lo_folded) : quantize_value_folded<false>(x, q_out, inv_y_scale, lo_folded);
         }
         if (a.oc_split == kFloatResults) {  // a DequantizeLinear behind the convolution
-            float* dst = reinterpret_cast<float*>(a.y2) + f.m * a.y2_px_stride + f.c0;
+            float* dst = a.floats + f.m * a.floats_px_stride + f.c0;
             v4f out;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) out[e] = dequantize_value(code[e], a.inv_y_scale2, a.lo_folded2);
+            for (int e = 0; e < 4; ++e) out[e] = dequantize_value(code[e], a.floats_zp, a.floats_scale);
             if (f.c0 + 4 <= OC) *reinterpret_cast<v4f_u*>(dst) = out;
             else
                 for (int e = 0; e < 4; ++e)

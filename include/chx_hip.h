@@ -240,7 +240,8 @@ int chx_hip_qconv_plan_run_dequantize(
         uint32_t flags, float dq_scale, int32_t dq_zero_point, chx_hip_tensor* y, void* stream);
 /* The launch configurations the plan has measured so far, as text into buf (truncated to buf_size - 1
  * characters): one "M=<output pixels> <OH>x<OW> res=<0|1> tile=<oc>x<px> wgs_per_cu=<n, 0 = as many as fit>"
- * per line (followed by "waves=<4|8>", the wavefronts per work-group), and after a chx_hip_qconv_plan_run_add a line
+ * per line (followed by "waves=<n>", the wavefronts per work-group, and "pixels=lds" for the kernels that bring a tile's
+ * pixels there once), and after a chx_hip_qconv_plan_run_add a line
  * "residual=affine" or "residual=exact" (which arithmetic the fused sum uses, see there); empty for a plan that
  * does not run on the matrix-core kernel or has not run eagerly yet.  No counterpart in the reference; benchmarks
  * report it next to their timings. */

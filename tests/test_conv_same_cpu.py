@@ -13,7 +13,7 @@ def host_so(tmp_path_factory):
     return host_hip.build(tmp_path_factory.mktemp("host_hip"))
 
 
-@pytest.mark.parametrize("case", ["cases", "limits"])
+@pytest.mark.parametrize("case", ["cases", "limits", "described"])
 def test_case(host_so, case):
     from test_gpu_conv_same import CASES, TILES
     host_hip.run_case(host_so, __file__, case, CASES=repr(CASES), TILES=repr(TILES))
@@ -52,6 +52,19 @@ def limits(host):
     assert not taken(host, tile, 1, 320, 5, 5, 32)  # ten K steps to a tap
     # (64 + 2 W + 2) pixels of 272 bytes in 160 KB less the tables
     assert taken(host, tile, 1, 256, 3, 260, 16) and not taken(host, tile, 1, 256, 3, 270, 16)
+
+
+def described(host):
+    """A configuration that brings the pixels into LDS once names no number of work-groups."""
+    os.environ.pop("CHX_HIP_TILE", None)
+    for n, kernel, lds in ((8, "conv_same_kernel", True), (9, "conv_mfma_kernel", False)):  # (what was measured is shared between plans)
+        x, y = host.channels_last("uint8", (n, 64, 28, 28)), host.channels_last("uint8", (n, 64, 28, 28))
+        host.hh.hh_prefer(kernel.encode())
+        plan, buf = host.plan(64, 64, 3, pads=(1, 1)), ctypes.create_string_buffer(1024)
+        host.check(host.plan_run(plan, x, y))
+        host.check(host.lib.chx_hip_qconv_plan_describe(plan, buf, ctypes.c_size_t(len(buf))))
+        fields = dict(f.split("=") for f in buf.value.decode().split() if "=" in f)
+        assert (fields.get("pixels") == "lds") == lds and int(fields["wgs_per_cu"]) <= 4, (kernel, buf.value)
 
 
 if __name__ == "__main__":
