@@ -26,7 +26,7 @@ def sum_code():
 
 
 @pytest.mark.parametrize("case", ["whole_blocks", "without_reduction", "values_read_elsewhere", "frees_between", "refused_forms", "sizes", "nothing_launched", "errors", "another_device",
-                                  "instruction_by_instruction", "long_rows", "channels_that_never_run", "asked_first"])
+                                  "instruction_by_instruction", "long_rows", "channels_that_never_run", "asked_first", "sums"])
 def test_case(host_so, sum_code, case):
     host_hip.run_case(host_so, __file__, case, SUM_CODE=sum_code)
 
@@ -221,6 +221,19 @@ def asked_first(host):
         assert seen == {0, capi.EUNSUPPORTED}
         for s in ((0, 1, 1), (1, -1, -1), (1 << 40, 1 << 40, 1 << 40), (1 << 62, 4, 1)):
             assert takes(*s) == capi.EUNSUPPORTED
+
+
+def sums(host):
+    """The kernel's form for the sum's short form, and the one for all others."""
+    def forms(p):
+        kernels(host, p)
+        return re.findall(r"bottleneck_kernel<.*(true|false)>", "\n".join(host.launches())), any(SEARCH in line for line in host.launches())
+
+    p = program(host)
+    os.environ["CHX_HIP_AFFINE_RESIDUAL"] = "0"
+    without = program(host)
+    assert forms(without) == (["false"], False)
+    assert forms(p)[1]  # (the stand-in's search finds what it finds)
 
 
 def errors(host):

@@ -131,3 +131,40 @@ def test_single_blocks(g, oracle, case):
         assert len(np.unique(ref)) > 20
         np.testing.assert_array_equal(got.view(np.uint8) ^ 0x80 if minus_128 else got, ref)
     lib.chx_hip_bottleneck_destroy(block)
+
+
+@pytest.mark.parametrize("mid,H,W,relu,r_zp", [(64, 5, 13, True, -17), (128, 3, 31, False, 90), (256, 57, 28, True, -128)])
+@pytest.mark.parametrize("affine", [True, False])
+def test_sums(g, oracle, monkeypatch, affine, mid, H, W, relu, r_zp):
+    """Both ways of the sum, its short form and operation by operation, with a residual of int8."""
+    from test_gpu_conv_split import codes, pitched
+    if not affine:
+        monkeypatch.setenv("CHX_HIP_AFFINE_RESIDUAL", "0")
+    rng, lib, capi, wide = np.random.default_rng(mid + W), g.capi.lib(), g.capi, 4 * mid
+    x, r = codes(rng, (2, mid, H, W), np.uint8), codes(rng, (2, wide, H, W), np.int8)
+    operands, kept, h, scales = [], [], x, [np.float32(0.02)]
+    oracle.set_threads(16)
+    try:
+        for shape, zp, y_zp in (((mid, mid, 3, 3), 33, 0), ((wide, mid, 1, 1), 0, 117)):
+            w, ws = codes(rng, shape, np.int8), rng.uniform(0.002, 0.02, size=shape[0]).astype(np.float32)
+            scales.append(np.float32(scales[-1] * ws.mean() * 74 * 74 * np.sqrt(np.prod(shape[1:])) / 60))
+            h = oracle.qlinear_conv_int(h, scales[-2], zp, w, ws, np.zeros(shape[0], np.int8), scales[-1], y_zp, np.uint8, pads=(shape[2] // 2,) * 2)
+            tensors = [g.dev(w), g.dev(ws), g.dev(np.zeros(shape[0], np.int8))]
+            kept += [tensors, [capi.desc(t) for t in tensors]]
+            operands += [ctypes.addressof(d) for d in kept[-1]] + [None]
+        r_scale, out_scale = np.float32(0.71 * scales[2]), np.float32(1.57 * scales[2])
+        want = oracle.binary(oracle.ADD, oracle.dequantize_linear(h, scales[2], 117), oracle.dequantize_linear(r, r_scale, r_zp))
+        want = oracle.quantize_linear(oracle.relu(want) if relu else want, out_scale, 40, np.uint8)
+    finally:
+        oracle.set_threads(1)
+    block = ctypes.c_void_p()
+    capi.check(lib.chx_hip_bottleneck_create((ctypes.c_void_p * 8)(*operands), 2, capi.stream_ptr(), ctypes.byref(block)))
+    xd, rd, out = pitched(x.shape, torch.uint8), pitched(r.shape, torch.int8), pitched(want.shape, torch.uint8)
+    xd.copy_(g.dev(x))
+    rd.copy_(g.dev(r))
+    capi.check(lib.chx_hip_bottleneck_run(
+        block, capi.ref(xd), ctypes.c_float(0.02), 33, (ctypes.c_float * 2)(*scales[1:]), (ctypes.c_int32 * 2)(0, 117), capi.UINT8, 0, capi.ref(rd), ctypes.c_float(r_scale), r_zp,
+        ctypes.c_float(out_scale), 40, int(relu), 0, capi.ref(out), 0, None, capi.stream_ptr()))
+    assert len(np.unique(want)) > 20
+    np.testing.assert_array_equal(g.host(out), want)
+    lib.chx_hip_bottleneck_destroy(block)
