@@ -27,18 +27,6 @@
 namespace chx {
 namespace {
 
-// The channel of a tile of 32 that row m of an MFMA takes: register r of lane half h is row 8 (r / 4) + 4 h + r % 4, and
-// should be channel 16 h + r, so that a lane holds sixteen neighbouring channels of a pixel.
-__host__ __device__ __forceinline__ int channel_of(int m) {
-    return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-}
-
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // async_copy16 from 32-bit offsets
 __device__ __forceinline__ void async_copy16_at(const char* base, uint32_t offset, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_addr) : "memory", "m0");

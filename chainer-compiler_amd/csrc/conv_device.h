@@ -35,6 +35,19 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, uint32_t mul, uint32_t 
     return (__umulhi(n, mul) + n) >> shift;
 }
 
+// The channel of a tile of 32 that row m of an MFMA takes: register r of lane half h is row 8 (r / 4) + 4 h + r % 4, and
+// should be channel 16 h + r, so that a lane holds sixteen neighbouring channels of a pixel.
+__device__ __forceinline__ int channel_of(int m) {
+    return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
+}
+
+// A barrier of the work-group that waits for LDS alone: loads and stores stay under way.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Asynchronous copy of 16 bytes per lane from global memory straight into LDS: lane i of the
 // wavefront writes LDS bytes [lds_addr + 16*i, lds_addr + 16*i + 16).  lds_addr must be the
 // same for all lanes (it travels in M0).  Completion is tracked by the wave's vector-memory

@@ -26,17 +26,6 @@ struct ConvSameArgs {
     uint32_t tiles_px_mul, tiles_px_shift, chunks_mul, chunks_shift;
 };
 
-// Sixteen neighbouring channels of a pixel for a lane: register r of lane half h is row 8 (r / 4) + 4 h + r % 4 of a tile of 32.
-__device__ __forceinline__ int channel_of(int m) {
-    return 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-}
-
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // kU: steps of 32 K bytes in a segment; kT: segments of an iteration, whose weights are requested one iteration ahead.  kXT: tiles of
 // 32 pixels of a wavefront; kWO, kWP: wavefronts along the channels and along the pixels.
 template <int kU, int kT, int kXT, int kWO, int kWP>

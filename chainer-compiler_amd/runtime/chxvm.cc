@@ -62,44 +62,58 @@ private:
 // Instructions of a program, with their places in it.
 typedef std::vector<std::pair<int, ChxVMOp*>> ChxVMSteps;
 
-void RunSteps(const ChxVMSteps& steps, ChxVMState* st) {
-    for (const auto& step : steps) {
-        st->set_pc(step.first);  // (what an error is reported with)
-        step.second->Run(st);
-    }
-}
-
-std::atomic<int64_t> g_matmul_chains{0};
-
-// A chain of such products, with the QuantizeLinear in front of it and the DequantizeLinear behind it where nobody else
-// reads what lies between, as one launch (chx_hip_qlinear_chain).  It stands where the last of its instructions stood; what
-// that kernel does not take runs as the program wrote it.
-class QLinearMatMulChainOp : public ChxVMOp {
+// Several instructions as one launch.  It stands where the last of them stood; what its kernel does not take runs as the program
+// wrote it.  Operands that are constants of the program are laid out when it is loaded.
+class GroupOp : public ChxVMOp {
 public:
-    struct Layer {
-        int a_scale, a_zp, b_scale, b_zp, y_scale, y_zp;
-        std::shared_ptr<chx_hip_chain_weights> b;
-    };
     // steps: the instructions that this one replaces and the Free's of their operands between them, in the program's order
-    QLinearMatMulChainOp(const ChxVMInstructionProto& last, const ChxVMInstructionProto* quantize, std::vector<Layer> layers, int64_t columns, int a,
-                         const ChxVMInstructionProto* dequantize, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(last), quantize_(quantize != nullptr), dequantize_(dequantize != nullptr), x_(quantize ? quantize->inputs[0].array : a),
-          x_scale_(quantize ? quantize->inputs[1].scalar : -1), x_zp_(quantize ? quantize->inputs[2].scalar : -1),
-          y_scale_(dequantize ? dequantize->inputs[1].scalar : -1), y_zp_(dequantize ? dequantize->inputs[2].scalar : -1),
-          y_(last.outputs[0]), columns_(columns), layers_(std::move(layers)), steps_(std::move(steps)), freed_(std::move(freed)) {
+    GroupOp(const ChxVMInstructionProto& last, ChxVMSteps steps, std::vector<int> freed) : ChxVMOp(last), steps_(std::move(steps)), freed_(std::move(freed)) {
     }
 
     void Run(ChxVMState* st) override {
         if (RunAsOne(st)) {
             for (int slot : freed_) st->FreeVar(slot);
-        } else {
-            RunSteps(steps_, st);
+            return;
+        }
+        for (const auto& step : steps_) {
+            st->set_pc(step.first);  // (what an error is reported with)
+            step.second->Run(st);
         }
     }
 
-private:
+protected:
     // false: nothing has been written
-    bool RunAsOne(ChxVMState* st) {
+    virtual bool RunAsOne(ChxVMState* st) = 0;
+
+    static int32_t Integer(const StrictScalar& z) {
+        return static_cast<int32_t>(static_cast<int64_t>(z));
+    }
+
+private:
+    ChxVMSteps steps_;
+    std::vector<int> freed_;
+};
+
+std::atomic<int64_t> g_matmul_chains{0};
+
+// A chain of such products, with the QuantizeLinear in front of it and the DequantizeLinear behind it where nobody else
+// reads what lies between, as one launch (chx_hip_qlinear_chain).
+class QLinearMatMulChainOp : public GroupOp {
+public:
+    struct Layer {
+        int a_scale, a_zp, b_scale, b_zp, y_scale, y_zp;
+        std::shared_ptr<chx_hip_chain_weights> b;
+    };
+    QLinearMatMulChainOp(const ChxVMInstructionProto& last, const ChxVMInstructionProto* quantize, std::vector<Layer> layers, int64_t columns, int a,
+                         const ChxVMInstructionProto* dequantize, ChxVMSteps steps, std::vector<int> freed)
+        : GroupOp(last, std::move(steps), std::move(freed)), quantize_(quantize != nullptr), dequantize_(dequantize != nullptr), x_(quantize ? quantize->inputs[0].array : a),
+          x_scale_(quantize ? quantize->inputs[1].scalar : -1), x_zp_(quantize ? quantize->inputs[2].scalar : -1),
+          y_scale_(dequantize ? dequantize->inputs[1].scalar : -1), y_zp_(dequantize ? dequantize->inputs[2].scalar : -1),
+          y_(last.outputs[0]), columns_(columns), layers_(std::move(layers)) {
+    }
+
+private:
+    bool RunAsOne(ChxVMState* st) override {
         auto is_null = [&](int slot) { return slot >= 0 && st->GetVar(slot)->IsNull(); };
         if (is_null(x_) || is_null(x_scale_) || is_null(x_zp_) || is_null(y_scale_) || is_null(y_zp_)) return false;
         for (const Layer& l : layers_)
@@ -108,7 +122,6 @@ private:
             absl::optional<StrictScalar> z = st->GetOptionalScalar(slot);
             return z.has_value() ? *z : StrictScalar(chainerx::Dtype::kUInt8, chainerx::Scalar(0u), false);
         };
-        auto integer = [](const StrictScalar& z) { return static_cast<int32_t>(static_cast<int64_t>(z)); };
         const chainerx::Array& x = st->GetArray(x_);
         if (x.ndim() != 2) return false;
         const StrictScalar x_zp = zp_of(x_zp_);
@@ -122,9 +135,9 @@ private:
             l.a_scale = static_cast<float>(st->GetScalar(in.a_scale));
             l.b_scale = static_cast<float>(st->GetScalar(in.b_scale));
             l.y_scale = static_cast<float>(st->GetScalar(in.y_scale));
-            l.a_zero_point = integer(zp_of(in.a_zp));
-            l.b_zero_point = integer(zp_of(in.b_zp));
-            l.y_zero_point = integer(y_zp);
+            l.a_zero_point = Integer(zp_of(in.a_zp));
+            l.b_zero_point = Integer(zp_of(in.b_zp));
+            l.y_zero_point = Integer(y_zp);
             l.y_dtype = static_cast<int32_t>(y_zp.dtype());
             dtype = y_zp.dtype();
         }
@@ -133,9 +146,9 @@ private:
         const chx_hip_tensor xt = x.hip();
         chx_hip_tensor yt = y.hip();
         const int rc = chx_hip_qlinear_chain(
-                &xt, quantize_ ? static_cast<float>(st->GetScalar(x_scale_)) : 1.f, quantize_ ? integer(x_zp) : 0,
+                &xt, quantize_ ? static_cast<float>(st->GetScalar(x_scale_)) : 1.f, quantize_ ? Integer(x_zp) : 0,
                 static_cast<int32_t>(quantize_ ? x_zp.dtype() : x.dtype()), layers.data(), static_cast<int32_t>(layers.size()), &yt,
-                dequantize_ ? static_cast<float>(st->GetScalar(y_scale_)) : 1.f, dequantize_ ? integer(zp_of(y_zp_)) : 0, chainerx::CurrentStream());
+                dequantize_ ? static_cast<float>(st->GetScalar(y_scale_)) : 1.f, dequantize_ ? Integer(zp_of(y_zp_)) : 0, chainerx::CurrentStream());
         // (what it refuses, and operands that are in error, are for the instructions)
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
@@ -150,8 +163,6 @@ private:
     int x_, x_scale_, x_zp_, y_scale_, y_zp_, y_;
     int64_t columns_;
     std::vector<Layer> layers_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
 };
 
 // DequantizeLinear, MaxPool | AveragePool, QuantizeLinear as one instruction on the 8-bit codes
@@ -352,9 +363,8 @@ std::atomic<int64_t> g_inverted_residuals{0};
 
 // The three convolutions of an inverted residual block (1x1 expansion, depthwise 3x3, 1x1 projection whose results in between
 // nobody else reads), and the residual sum behind them where the projection may compute it, as one launch
-// (chx_hip_inverted_residual_run).  It stands where the projection stood; what that kernel does not take runs as the program
-// wrote it.  The operands are constants of the program, laid out when it is loaded.
-class InvertedResidualOp : public ChxVMOp {
+// (chx_hip_inverted_residual_run).
+class InvertedResidualOp : public GroupOp {
 public:
     struct Quantization {  // the variable slots of a convolution
         int x_scale, x_zp, y_scale, y_zp;
@@ -366,25 +376,12 @@ public:
     };
     InvertedResidualOp(const ChxVMInstructionProto& projection, std::shared_ptr<chx_hip_inverted_residual> block, int x, int between, const std::vector<Quantization>& convs,
                        int64_t out_channels, int stride, bool has_bias, Sum sum, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(projection), block_(std::move(block)), x_(x), between_(between), y_(projection.outputs[0]), convs_(convs), out_channels_(out_channels), stride_(stride),
-          has_bias_(has_bias), sum_(std::move(sum)), steps_(std::move(steps)), freed_(std::move(freed)) {
-    }
-
-    void Run(ChxVMState* st) override {
-        if (RunAsOne(st)) {
-            for (int slot : freed_) st->FreeVar(slot);
-        } else {
-            RunSteps(steps_, st);
-        }
+        : GroupOp(projection, std::move(steps), std::move(freed)), block_(std::move(block)), x_(x), between_(between), y_(projection.outputs[0]), convs_(convs), out_channels_(out_channels), stride_(stride),
+          has_bias_(has_bias), sum_(std::move(sum)) {
     }
 
 private:
-    static int32_t Integer(const StrictScalar& z) {
-        return static_cast<int32_t>(static_cast<int64_t>(z));
-    }
-
-    // false: nothing has been written
-    bool RunAsOne(ChxVMState* st) {
+    bool RunAsOne(ChxVMState* st) override {
         if (st->GetVar(x_)->IsNull() || (has_bias_ && !st->options().qlinearconv_onnx_int32_bias)) return false;
         float scales[3];
         int32_t zero_points[3];
@@ -457,17 +454,13 @@ private:
     int stride_;
     bool has_bias_;
     Sum sum_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
 };
 
 std::atomic<int64_t> g_bottlenecks{0};
 
 // The 3x3 convolution of a bottleneck block, the 1x1 convolution behind it with the residual sum, and the 1x1 convolution that
-// reads the sum in the next block (where there is one) as one launch (chx_hip_bottleneck_run).  It stands where the last of them
-// stood; what that kernel does not take runs as the program wrote it.  The operands are constants of the program, laid out when it
-// is loaded.
-class BottleneckOp : public ChxVMOp {
+// reads the sum in the next block (where there is one) as one launch (chx_hip_bottleneck_run).
+class BottleneckOp : public GroupOp {
 public:
     struct Quantization {  // the variable slots of a convolution
         int x_scale, x_zp, y_scale, y_zp;
@@ -479,25 +472,12 @@ public:
     };
     BottleneckOp(const ChxVMInstructionProto& last, std::shared_ptr<chx_hip_bottleneck> block, int x, int between, int next, const std::vector<Quantization>& convs,
                  int64_t wide_channels, int64_t next_channels, bool has_bias, Sum sum, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(last), block_(std::move(block)), x_(x), between_(between), next_(next), convs_(convs), wide_channels_(wide_channels), next_channels_(next_channels),
-          has_bias_(has_bias), sum_(std::move(sum)), steps_(std::move(steps)), freed_(std::move(freed)) {
-    }
-
-    void Run(ChxVMState* st) override {
-        if (RunAsOne(st)) {
-            for (int slot : freed_) st->FreeVar(slot);
-        } else {
-            RunSteps(steps_, st);
-        }
+        : GroupOp(last, std::move(steps), std::move(freed)), block_(std::move(block)), x_(x), between_(between), next_(next), convs_(convs), wide_channels_(wide_channels), next_channels_(next_channels),
+          has_bias_(has_bias), sum_(std::move(sum)) {
     }
 
 private:
-    static int32_t Integer(const StrictScalar& z) {
-        return static_cast<int32_t>(static_cast<int64_t>(z));
-    }
-
-    // false: nothing has been written
-    bool RunAsOne(ChxVMState* st) {
+    bool RunAsOne(ChxVMState* st) override {
         if (st->GetVar(x_)->IsNull() || st->GetVar(sum_.other)->IsNull() || (has_bias_ && !st->options().qlinearconv_onnx_int32_bias)) return false;
         float scales[3] = {1.f, 1.f, 1.f};
         int32_t zero_points[3] = {0, 0, 0};
@@ -567,13 +547,11 @@ private:
     int64_t wide_channels_, next_channels_;
     bool has_bias_;
     Sum sum_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
 };
 
 // A QLinearConv over constants and the instruction in front of it or behind it as one launch.  It has a plan of its own, made
 // by the first run that may take it: most programs then have one plan of the convolution, this or the instruction's.
-class ConvolutionEndOp : public ChxVMOp {
+class ConvolutionEndOp : public GroupOp {
 public:
     struct Quantization {  // variable slots
         int scale, zp;
@@ -586,24 +564,10 @@ public:
         Quantization in, out;
     };
     ConvolutionEndOp(const ChxVMInstructionProto& last, Convolution conv, ChxVMSteps steps, std::vector<int> freed)
-        : ChxVMOp(last), conv_(std::move(conv)), y_(last.outputs[0]), steps_(std::move(steps)), freed_(std::move(freed)) {
-    }
-
-    void Run(ChxVMState* st) override {
-        if (RunAsOne(st)) {
-            for (int slot : freed_) st->FreeVar(slot);
-        } else {
-            RunSteps(steps_, st);
-        }
+        : GroupOp(last, std::move(steps), std::move(freed)), conv_(std::move(conv)), y_(last.outputs[0]) {
     }
 
 protected:
-    // false: nothing has been written
-    virtual bool RunAsOne(ChxVMState* st) = 0;
-
-    static int32_t Integer(const StrictScalar& z) {
-        return static_cast<int32_t>(static_cast<int64_t>(z));
-    }
     static bool IsQ8(chainerx::Dtype t) {
         return t == chainerx::Dtype::kUInt8 || t == chainerx::Dtype::kInt8;
     }
@@ -639,14 +603,11 @@ protected:
 private:
     std::mutex mutex_;  // of plan_
     std::shared_ptr<chx_hip_qconv_plan> plan_;
-    ChxVMSteps steps_;
-    std::vector<int> freed_;
 };
 
 std::atomic<int64_t> g_quantized_convolutions{0};
 
-// A QuantizeLinear and the convolution over few channels that reads its result (chx_hip_qconv_plan_run_quantize).  It stands
-// where the convolution stood; what that kernel does not take runs as the program wrote it.
+// A QuantizeLinear and the convolution over few channels that reads its result (chx_hip_qconv_plan_run_quantize).
 class QuantizedConvolutionOp : public ConvolutionEndOp {
 public:
     // x, quantize: of the QuantizeLinear (a zero point of -1: none)
@@ -690,8 +651,7 @@ private:
 
 std::atomic<int64_t> g_dequantized_convolutions{0};
 
-// A convolution with 1x1 filters and the DequantizeLinear that reads its result, likewise (chx_hip_qconv_plan_run_dequantize): it
-// stands where the DequantizeLinear stood.
+// A convolution with 1x1 filters and the DequantizeLinear that reads its result (chx_hip_qconv_plan_run_dequantize).
 class DequantizedConvolutionOp : public ConvolutionEndOp {
 public:
     // dequantize: of the DequantizeLinear (a zero point of -1: none)
