@@ -6,7 +6,6 @@
 #include <fstream>
 #include <iomanip>
 #include <map>
-#include <mutex>
 #include <sstream>
 
 #include <set>
@@ -75,15 +74,19 @@ public:
             for (int slot : freed_) st->FreeVar(slot);
             return;
         }
-        for (const auto& step : steps_) {
-            st->set_pc(step.first);  // (what an error is reported with)
-            step.second->Run(st);
-        }
+        RunSteps(st);
     }
 
 protected:
     // false: nothing has been written
     virtual bool RunAsOne(ChxVMState* st) = 0;
+
+    virtual void RunSteps(ChxVMState* st) {
+        for (const auto& step : steps_) {
+            st->set_pc(step.first);  // (what an error is reported with)
+            step.second->Run(st);
+        }
+    }
 
     static int32_t Integer(const StrictScalar& z) {
         return static_cast<int32_t>(static_cast<int64_t>(z));
@@ -549,17 +552,17 @@ private:
     Sum sum_;
 };
 
-// A QLinearConv over constants and the instruction in front of it or behind it as one launch.  It has a plan of its own, made
-// by the first run that may take it: most programs then have one plan of the convolution, this or the instruction's.
+// A QLinearConv over constants and the instruction in front of it or behind it as one launch.  The convolution's plan is made when
+// the program is loaded, and is the instruction's too where the launch is not taken.
 class ConvolutionEndOp : public GroupOp {
 public:
     struct Quantization {  // variable slots
         int scale, zp;
     };
     struct Convolution {
-        chainerx::Array w, w_scale, w_zp, bias;  // (bias: perhaps none)
-        chx_hip_conv_params params;
-        int32_t device;  // that these are on
+        ChxVMState::OfferedPlan plan;
+        int32_t device;  // that it is on
+        chainerx::Array w;
         int x;
         Quantization in, out;
     };
@@ -576,33 +579,21 @@ protected:
         int32_t device = 0;
         return chx_hip_get_device(&device) == CHX_HIP_OK && device == conv_.device;
     }
-    // null where there is none (no memory for it, say: the instruction's own plan has yet to be refused it)
-    chx_hip_qconv_plan* Plan() {
-        std::lock_guard<std::mutex> lock(mutex_);
-        if (!plan_) {
-            const chx_hip_tensor w = conv_.w.hip(), scale = conv_.w_scale.hip(), zp = conv_.w_zp.hip();
-            chx_hip_tensor bias;
-            if (!conv_.bias.IsNullHandle()) bias = conv_.bias.hip();
-            chx_hip_qconv_plan* plan = nullptr;
-            if (chx_hip_qconv_plan_create(&w, &scale, &zp, conv_.bias.IsNullHandle() ? nullptr : &bias, &conv_.params, nullptr, &plan) != CHX_HIP_OK) return nullptr;
-            plan_.reset(plan, chx_hip_qconv_plan_destroy);
-        }
-        return plan_.get();
+    void RunSteps(ChxVMState* st) override {
+        if (OnDevice()) st->set_offered_plan(&conv_.plan);
+        GroupOp::RunSteps(st);
+        st->set_offered_plan(nullptr);
     }
     // rc: of the launch.  false: the instructions run (what it refuses, and operands that are in error, are for them)
     bool Launched(ChxVMState* st, int rc) {
         if (rc == CHX_HIP_EUNSUPPORTED || rc == CHX_HIP_EINVAL) return false;
         CHECK_EQ(CHX_HIP_OK, rc) << chx_hip_last_error();
-        if (st->options().recorded_memory) st->options().recorded_memory->push_back(plan_);  // a recording may outlive the program
+        if (st->options().recorded_memory) st->options().recorded_memory->push_back(conv_.plan.plan);  // a recording may outlive the program
         return true;
     }
 
     Convolution conv_;
     int y_;
-
-private:
-    std::mutex mutex_;  // of plan_
-    std::shared_ptr<chx_hip_qconv_plan> plan_;
 };
 
 std::atomic<int64_t> g_quantized_convolutions{0};
@@ -627,17 +618,15 @@ private:
         if (x.ndim() != 4 || x.dtype() != chainerx::Dtype::kFloat32 || x.shape()[1] != conv_.w.shape()[1] || (q_zp.has_value() && q_zp->dtype() != chainerx::Dtype::kUInt8) ||
             x_zp.dtype() != chainerx::Dtype::kUInt8 || !IsQ8(y_zp.dtype()))
             return false;
-        const chainerx::Shape y_shape = ConvOutputShape(x, conv_.w, conv_.params);
+        const chainerx::Shape y_shape = ConvOutputShape(x, conv_.w, conv_.plan.params);
         for (int64_t extent : y_shape)
             if (extent <= 0) return false;
-        chx_hip_qconv_plan* const plan = Plan();
-        if (!plan) return false;
         chainerx::Array y = chainerx::EmptyChannelsLastPadded(y_shape, y_zp.dtype());
         const chx_hip_tensor xt = x.hip();
         chx_hip_tensor yt = y.hip();
         const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
         if (!Launched(st, chx_hip_qconv_plan_run_quantize(
-                                  plan, &xt, static_cast<float>(st->GetScalar(quantize_.scale)), q_zp.has_value() ? Integer(*q_zp) : 0, static_cast<float>(st->GetScalar(conv_.in.scale)),
+                                  conv_.plan.plan.get(), &xt, static_cast<float>(st->GetScalar(quantize_.scale)), q_zp.has_value() ? Integer(*q_zp) : 0, static_cast<float>(st->GetScalar(conv_.in.scale)),
                                   Integer(x_zp), static_cast<float>(st->GetScalar(conv_.out.scale)), Integer(y_zp), flags, &yt, chainerx::CurrentStream())))
             return false;
         st->SetArray(y_, y);
@@ -669,12 +658,10 @@ private:
         const absl::optional<StrictScalar> dq_zp = st->GetOptionalScalar(dequantize_.zp);  // (none: uint8 0)
         const StrictScalar &x_zp = st->GetScalar(conv_.in.zp), &y_zp = st->GetScalar(conv_.out.zp);
         if (x.ndim() != 4 || !IsQ8(x.dtype()) || x.shape()[1] != conv_.w.shape()[1] || !IsQ8(y_zp.dtype()) || (dq_zp.has_value() && !IsQ8(dq_zp->dtype()))) return false;
-        const chainerx::Shape shape = ConvOutputShape(x, conv_.w, conv_.params);
+        const chainerx::Shape shape = ConvOutputShape(x, conv_.w, conv_.plan.params);
         for (int64_t extent : shape)
             if (extent <= 0) return false;
         if (shape[0] * shape[1] * shape[2] * shape[3] > CHX_HIP_MOST_DEQUANTIZED) return false;
-        chx_hip_qconv_plan* const plan = Plan();
-        if (!plan) return false;
         // (an input kept as code - 128 is an int8 tensor with the zero point 128 lower)
         const bool lowered = st->store_minus_128(conv_.x) && x.dtype() == chainerx::Dtype::kInt8 && x_zp.dtype() == chainerx::Dtype::kUInt8;
         // laid out as the DequantizeLinear does: like the convolution's result, which is channels-last with whole 16 bytes per pixel
@@ -684,7 +671,7 @@ private:
         chx_hip_tensor yt = y.hip();
         const uint32_t flags = CHX_HIP_ROUND_REFERENCE | (st->options().qlinearconv_onnx_int32_bias ? CHX_HIP_BIAS_ONNX_INT32 : CHX_HIP_BIAS_REFERENCE_FLOAT);
         if (!Launched(st, chx_hip_qconv_plan_run_dequantize(
-                                  plan, &xt, static_cast<float>(st->GetScalar(conv_.in.scale)), Integer(x_zp) - (lowered ? 128 : 0), static_cast<float>(st->GetScalar(conv_.out.scale)),
+                                  conv_.plan.plan.get(), &xt, static_cast<float>(st->GetScalar(conv_.in.scale)), Integer(x_zp) - (lowered ? 128 : 0), static_cast<float>(st->GetScalar(conv_.out.scale)),
                                   Integer(y_zp), static_cast<int32_t>(y_zp.dtype()), flags, static_cast<float>(st->GetScalar(dequantize_.scale)), dq_zp.has_value() ? Integer(*dq_zp) : 0, &yt,
                                   chainerx::CurrentStream())))
             return false;
@@ -1310,13 +1297,17 @@ ChxVM::ChxVM(const ChxVMProgramProto& program) : input_names_(program.input_name
         for (int k : {1, 2, 6, 7}) slots.insert(ci.inputs[k].scalar);
         Group group;
         if (!gather({i, c}, std::min(i, c), slots, &group)) continue;
+        const int bias = ci.inputs[8].array;
+        const chx_hip_tensor wt = w.hip(), scale = constant_array(ci.inputs[4].array)->hip(), zp = constant_array(ci.inputs[5].array)->hip();
+        chx_hip_tensor bt;
+        if (bias >= 0) bt = constant_array(bias)->hip();
+        chx_hip_qconv_plan* plan = nullptr;
+        // (operands that are in error, and no memory, are for the instruction)
+        if (chx_hip_qconv_plan_create(&wt, &scale, &zp, bias >= 0 ? &bt : nullptr, &params, chainerx::CurrentStream(), &plan) != CHX_HIP_OK) continue;
         ConvolutionEndOp::Convolution conv;
-        conv.w = w;
-        conv.w_scale = *constant_array(ci.inputs[4].array);
-        conv.w_zp = *constant_array(ci.inputs[5].array);
-        if (ci.inputs[8].array >= 0) conv.bias = *constant_array(ci.inputs[8].array);
-        conv.params = params;
+        conv.plan = {std::shared_ptr<chx_hip_qconv_plan>(plan, chx_hip_qconv_plan_destroy), params};
         CHXVM_HIP_CALL(chx_hip_get_device(&conv.device));
+        conv.w = w;
         conv.x = ci.inputs[0].array;
         conv.in = {ci.inputs[1].scalar, ci.inputs[2].scalar};
         conv.out = {ci.inputs[6].scalar, ci.inputs[7].scalar};

@@ -124,6 +124,17 @@ public:
     void set_residual_request(QLinearConvResidualRequest* request) {
         residual_request_ = request;
     }
+    // A plan over a convolution's constant operands that the next QLinearConvOp::RunImpl of this run takes where it has none yet.
+    struct OfferedPlan {
+        std::shared_ptr<chx_hip_qconv_plan> plan;
+        chx_hip_conv_params params;
+    };
+    const OfferedPlan* offered_plan() const {
+        return offered_plan_;
+    }
+    void set_offered_plan(const OfferedPlan* offered) {
+        offered_plan_ = offered;
+    }
     // residual sums computed inside a convolution during this run
     int64_t residual_fusions() const {
         return residual_fusions_;
@@ -156,6 +167,7 @@ private:
     InOuts outputs_;
     ChxVMOptions options_;
     QLinearConvResidualRequest* residual_request_ = nullptr;
+    const OfferedPlan* offered_plan_ = nullptr;
     int64_t residual_fusions_ = 0;
     const std::vector<bool>* minus_128_slots_ = nullptr;
 };

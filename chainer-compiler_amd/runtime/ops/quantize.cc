@@ -97,6 +97,7 @@ chainerx::Array DequantizeLinearOp::RunImpl(
 class QLinearConvOp::QLinearConvImpl {
 public:
     chx_hip_qconv_plan* plan = nullptr;
+    std::shared_ptr<chx_hip_qconv_plan> shared;  // the same, where it has another owner too (ChxVMState::OfferedPlan)
     chx_hip_conv_params params;
     chainerx::Array w, w_scale, w_zero_point, bias;  // what the plan was built from
     bool minus_128_refused = false;  // the kernel that runs this plan does not write the minus-128 storage
@@ -112,8 +113,12 @@ public:
         if (b.has_value() && !same(bias, *b)) return false;
         return memcmp(&params, &p, sizeof(p)) == 0;
     }
+    ~QLinearConvImpl() {
+        Drop();
+    }
     void Drop() {
-        chx_hip_qconv_plan_destroy(plan);
+        if (!shared) chx_hip_qconv_plan_destroy(plan);
+        shared.reset();
         plan = nullptr;
         w = w_scale = w_zero_point = bias = chainerx::Array();
         minus_128_refused = false;
@@ -125,7 +130,6 @@ void QLinearConvOp::InitImpl() {
 }
 
 QLinearConvOp::~QLinearConvOp() {
-    if (impl_) chx_hip_qconv_plan_destroy(impl_->plan);
     delete impl_;
 }
 
@@ -183,7 +187,13 @@ chainerx::Array QLinearConvOp::RunImpl(
     if (!impl_->plan) {
         chx_hip_tensor wt = q_w.hip(), st2 = w_scale.hip(), zt = w_zero_point.hip(), bt;
         if (b.has_value()) bt = b->hip();
-        CHXVM_HIP_CALL(chx_hip_qconv_plan_create(&wt, &st2, &zt, b.has_value() ? &bt : nullptr, &p, nullptr, &impl_->plan));
+        const ChxVMState::OfferedPlan* offered = st->offered_plan();
+        if (offered && memcmp(&offered->params, &p, sizeof(p)) == 0) {
+            impl_->shared = offered->plan;
+            impl_->plan = impl_->shared.get();
+        } else {
+            CHXVM_HIP_CALL(chx_hip_qconv_plan_create(&wt, &st2, &zt, b.has_value() ? &bt : nullptr, &p, nullptr, &impl_->plan));
+        }
         impl_->params = p;
         impl_->w = q_w;
         impl_->w_scale = w_scale;

@@ -82,27 +82,47 @@ def chain(host):
 
 
 def plans_of_the_ends(host):
-    """A convolution has one plan, made when it first runs: of the launch with its quantization in front or behind, or its instruction's where that launch
-    does not take it."""
+    """A convolution has one plan, of the launch with its quantization in front or behind and of its instruction where that launch does not take it; one
+    that there is no memory for is missed by the instruction first."""
+    host.hh.hh_no_memory.argtypes = [ctypes.c_size_t]
     rt = host.chxvm.runtime()
     assert rt.chxvm_set_option(b"qlinearconv_bias", b"onnx_int32") == 0
-    for batch, one in ((8, True), (9, False)):  # (the last layer's results: 2^19 and more)
+
+    def build():
         p = Program(host)
         scale, mid = p.b.scales(0.1, 7), p.b.scales(0.2, 0)
-        x = p.b.input("x", "float32", [batch, 3, 32, 32])
-        h = p.convolution(p.convolution(p.b.QuantizeLinear(x, *scale), scale, (32, 3, 3, 3), mid), mid, (64, 32, 1, 1), mid)
+        h = p.convolution(p.convolution(p.b.QuantizeLinear(p.b.input("x", "float32", [8, 3, 32, 32]), *scale), scale, (32, 3, 3, 3), mid), mid, (64, 32, 1, 1), mid)
         p.b.output("y", p.b.DequantizeLinear(h, *mid))
+        return p.b
+
+    def run(program, batch):
+        out = ctypes.c_void_p()
+        rc = rt.chxvm_program_run(program, *host.names_and({"x": host.tensor("float32", (batch, 3, 32, 32))}), 0, ctypes.byref(out))
+        rt.chxvm_outputs_destroy(out)
+        return rc
+
+    for batches in ((8, 9, 8), (9, 8, 9)):  # (the last layer's results: 2^19 and more)
         host.clear()
-        program = host.program(p.b)
-        assert not host.launches()
-        for _ in range(3):
-            out = ctypes.c_void_p()
-            assert rt.chxvm_program_run(program, *host.names_and({"x": host.tensor("float32", (batch, 3, 32, 32))}), 0, ctypes.byref(out)) == 0, rt.chxvm_last_error()
-            rt.chxvm_outputs_destroy(out)
+        program = host.program(build())
+        for n in batches:
+            at = len(host.launches())
+            assert run(program, n) == 0, rt.chxvm_last_error()
+            assert any("dequantize" in k for k in host.launches()[at:]) == (n == 9)
         names = " ".join(host.launches())
         # (the first layer's weights are laid out in two orders by a launch each)
         assert (names.count("pack_weights_stem_kernel"), names.count("pack_weights_dense_kernel"), names.count("pack_weights_kernel")) == (1, 1, 1), names
-        assert ("dequantize" in names) != one
+        graph = ctypes.c_void_p()  # the plan of a recording outlives the program
+        assert rt.chxvm_program_capture(program, *host.names_and({"x": host.tensor("float32", (batches[0], 3, 32, 32))}), ctypes.byref(graph)) == 0, rt.chxvm_last_error()
+        rt.chxvm_program_destroy(program)
+        assert rt.chxvm_replay_launch(graph, None) == 0
+        rt.chxvm_replay_destroy(graph)
+    log = host.log()
+    at = next(i for i, line in enumerate(log) if "pack_weights_kernel" in line)
+    host.hh.hh_no_memory(int(next(line for line in reversed(log[:at]) if line.startswith("hipMalloc ")).split()[1]))
+    program = host.program(build())
+    assert run(program, 8) != 0 and b"hipMalloc" in rt.chxvm_last_error()
+    host.hh.hh_no_memory(0)
+    assert run(program, 8) == 0, rt.chxvm_last_error()
 
 
 if __name__ == "__main__":
