@@ -137,7 +137,7 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
     # The timed region replays the whole program as one HIP graph (about 125 launches per step
     # would otherwise be bound by the host); --no-graph launches every op from the host instead.
     vm_prog = vm_replay = None
-    fused_blocks = 0  # of the timed recording: inverted residual blocks as one launch
+    fused_blocks = 0  # of the timed recording: blocks as one launch
     use_vm = args.runner == "chxvm" and args.parts <= 1 and fuse
     if use_vm:
         # the drop-in itself: the network as one serialized program in the C++ VM
@@ -152,9 +152,10 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
                 vm_prog.run({"x": x})
             sec = timed_steps(torch, step, args.steps, args.warmup)
         else:
-            fused_blocks = vm.counter("inverted_residuals")
+            blocks = "inverted_residuals" if mobilenet else "bottlenecks"
+            fused_blocks = vm.counter(blocks)
             vm_prog.run({"x": x})
-            fused_blocks = vm.counter("inverted_residuals") - fused_blocks
+            fused_blocks = vm.counter(blocks) - fused_blocks
             vm_replay = vm_prog.capture({"x": x})
             stream = capi.stream_ptr()
             sec = timed_steps(torch, lambda _t: vm_replay.launch(stream), args.steps, args.warmup)
@@ -232,6 +233,8 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
         roofline = dict(bound="mfma", kernel="QLinearConv launches of one step, summed (%d)" % n_launch,
                         achieved=achieved, peak=INT8_PEAK_TOPS, unit="TOP/s", frac=achieved / INT8_PEAK_TOPS, traffic=None,
                         ops_per_step=conv_ops, kernel_ms_per_step=conv_ms_per_step)
+        # the operations of the convolutions over the whole timed step, whose launches are other ones (fused blocks)
+        roofline["frac_of_timed_step"] = conv_ops / sec / 1e12 / INT8_PEAK_TOPS
     # The same launches against BOTH roofs: a launch is priced at the roof that takes longer for its algorithmic
     # operations and bytes (input pixels it needs, weights, output, residual operand; workloads.conv_layer_table);
     # most 1x1 layers of these networks are below the ridge of 625 op/byte and belong to the HBM roof.  For
@@ -281,8 +284,8 @@ def bench_resnet50(args, torch, pkg, mobilenet=False):
     roofline["configs"] = hist
     if not mobilenet:
         planar = n_launch - sum(kernels.values())
-        roofline["kernel"] = "QLinearConv launches of one step, summed (%d: %s)" % (
-            n_launch, ", ".join("%d %s" % (n, k) for k, n in sorted(kernels.items(), key=lambda kv: -kv[1]) + ([("conv_stem_kernel", planar)] if planar > 0 else [])))
+        roofline["kernel"] = "QLinearConv launches of the runner that launches op by op, summed (%d: %s); the timed recording has %d of the blocks' tails as one bottleneck_kernel each" % (
+            n_launch, ", ".join("%d %s" % (n, k) for k, n in sorted(kernels.items(), key=lambda kv: -kv[1]) + ([("conv_stem_kernel", planar)] if planar > 0 else [])), fused_blocks)
     roofline["configs_source"] = ("plans of the Python runner (ops.py), whose launches the kernel time above is measured on; the "
                                   "plans inside the C++ VM measure their own configurations and may choose differently")
     if forms:

@@ -396,10 +396,12 @@ int plan_bottleneck(BottleneckArgs* launch) {
     BottleneckArgs& a = *launch;
     // Pixels of a work-group, and whether the block is one launch: by 400 drawn blocks measured both ways inside a recording, three
     // with weights of their own in turn.  Few pixels leave compute units idle when they are shared out in tiles of 64, and each
-    // work-group reads all weights for its tile.  256 channels on few pixels are faster as single launches (up to 1.4 times).  With 256 a tile takes 16 to 17 us however few
-    // there are, which the three launches of 256 -> 1024 -> 256 reach at 1,500 pixels (17.3 us inside a recording at 1,568,
-    // 19.0 at 2,304; run by run, where a launch costs more, a ResNet-50 on 8 images takes 25 us less with them as one),
-    // two launches without a reduction, and three with one to more than 256 channels, at 2,500.
+    // work-group reads all weights for its tile.  256 channels on few pixels are faster as single launches (up to 1.4 times).  With 256 a tile takes 16 to 18 us however few
+    // there are.  256 -> 1024 -> 256, six in a row, one launch and three: inside a recording 18.3 and 16.7 us at 980 pixels, 18.3 and 17.9 at 1,176 and
+    // 1,372, 18.2 and 18.2 at 1,568, 18.2 and 18.8 at 1,960, 18.3 and 20.3 at 2,352; run by run, where a launch costs more, 24.5 and 22.8 at 588, 24.5 and
+    // 26.3 at 784, 25.5 and 29.4 at 1,372.  The line is that of recordings, which are what is run again and again; run by run
+    // 2 to 4 us a block are left between 700 pixels and it.  Two launches without a reduction, and three with one to more than 256
+    // channels, meet the one at 2,500.
     const int fewest = a.next == 0 || a.next > 256 ? 2500 : 1500;
     if (a.W >= 8192) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: the rows do not fit");  // (some 950 pixels of 64 channels do; what follows counts bytes in 32 bits)
     if (a.mid == 256 && (a.pixels < fewest || a.pixels > 60000)) CHX_FAIL(CHX_HIP_EUNSUPPORTED, "bottleneck: slower than its convolutions");
